@@ -112,6 +112,18 @@ int ktx_linear_forward_fused(ktx_linear_t h, const int32_t* d_bsz, int T, const 
                              const ktx_linear_fusion* fusion, ktx_stream_t stream);
 int ktx_linear_decode_eligible(ktx_linear_t h, int T);
 
+/* ktx_linear_forward_fused with scratch memory, for calls above the decode kernel's rows: batches and short prompts then run on tiles
+ * that cut K over workgroups (fp32 chunk sums in d_ws, added in chunk order) instead of one strip per wavefront over all of K.
+ * ktx_linear_workspace_bytes says how much d_ws such a call of T rows needs; 0: none (d_ws may be NULL).  plain: 1 for a call without
+ * d_bsz, addends and GLU (long bf16 prompts then need none).  d_ws: device memory, 16-byte
+ * aligned, used by this call alone until its work on `stream` is done.  Calls that the tiles don't cover (no or too little d_ws,
+ * in_features % 128 != 0, rows that are not 16-byte aligned, decode-sized T) run as ktx_linear_forward_fused.  `fusion` may be NULL.
+ * prompt (T > 32): 1 takes a prompt's arithmetic — FP8: a 128-block in one K = 128 MFMA instead of four of K = 32 (the order of
+ * ktx_linear_forward); W4: the rounded multiplicand bf16((q - 8) * s) of ktx_linear_dequant_bf16 instead of exact integers. */
+size_t ktx_linear_workspace_bytes(ktx_linear_t h, int T, int plain);
+int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T, const void* d_x, void* d_y, const ktx_linear_fusion* fusion,
+                          int prompt, void* d_ws, size_t ws_bytes, ktx_stream_t stream);
+
 /* ktx_linear_forward_fused with the MoE router riding in the same launch (decode steps, T <= 4).  For the MoE block of a
  * decoder layer (KDeepseekV3MoE.forward, archive/ktransformers/operators/experts.py:974-1012: router, routed experts and the
  * shared experts all read the same post-attention hidden row): `h` is the shared experts' merged gate|up linear, `fusion`
@@ -178,7 +190,8 @@ int ktx_linear_dequant_bf16(ktx_linear_t h, void* d_out, int64_t ld_out, ktx_str
  *                        amax(x[t][128 kb .. 128 kb + 127]) / 448 (block-major, so a tile's scales of one k-step are contiguous);
  *   ktx_linear_gemm_fp8 — y bf16 [T][ldy] = fp8_gemm(d_q, scales, W, scale_inv) (+ bias): 128 x 128 output tiles, k-step = one
  *                        128-block, accumulator += dot * a_s * b_s (fp8gemm.py:156).  s_ld >= ceil(T / 128) * 128, a multiple of 4.
- * Same arithmetic as ktx_linear_forward on the same handle (bit for bit); the decode layout of the weights is read in place. */
+ * Same products and scalings as ktx_linear_forward on the same handle; the decode layout of the weights is read in place.  Columns
+ * [T, min(s_ld, ceil(T / 128) * 128)) of d_scales_t are set to zero. */
 int ktx_fp8_act_quant(const void* d_x, int64_t ldx, int T, int K, void* d_q, float* d_scales_t, int64_t s_ld, ktx_stream_t stream);
 int ktx_linear_gemm_fp8(ktx_linear_t h, const void* d_q, const float* d_scales_t, int64_t s_ld, int T, void* d_y, int64_t ldy,
                         ktx_stream_t stream);

@@ -134,6 +134,10 @@ def _load() -> C.CDLL:
                                                     C.c_void_p, C.c_void_p, C.c_void_p, C.c_float, C.c_void_p]
     lib.ktx_linear_forward_fused.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.POINTER(_LinearFusion),
                                              C.c_void_p]
+    lib.ktx_linear_workspace_bytes.argtypes = [C.c_void_p, C.c_int, C.c_int]
+    lib.ktx_linear_workspace_bytes.restype = C.c_size_t
+    lib.ktx_linear_forward_ws.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.POINTER(_LinearFusion), C.c_int, C.c_void_p,
+                                          C.c_size_t, C.c_void_p]
     lib.ktx_linear_decode_eligible.argtypes = [C.c_void_p, C.c_int]
     lib.ktx_linear_dequant_bf16.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p]
     lib.ktx_fp8_act_quant.argtypes = [C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p]
@@ -201,7 +205,7 @@ def _load() -> C.CDLL:
 STREAM_CALLS = frozenset((
     "ktx_moe_forward", "ktx_moe_forward_ex", "ktx_moe_combine", "ktx_gate_logits", "ktx_gate_select", "ktx_gate_forward",
     "ktx_gate_forward_norm", "ktx_mla_decode", "ktx_mla_decode_append", "ktx_mla_cache_append", "ktx_mla_prefill", "ktx_linear_forward",
-    "ktx_linear_forward_batched", "ktx_linear_forward_batched_prep", "ktx_linear_forward_fused", "ktx_rmsnorm", "ktx_fused_add_rmsnorm", "ktx_silu_mul",
+    "ktx_linear_forward_batched", "ktx_linear_forward_batched_prep", "ktx_linear_forward_fused", "ktx_linear_forward_ws", "ktx_rmsnorm", "ktx_fused_add_rmsnorm", "ktx_silu_mul",
     "ktx_mla_prep", "ktx_argmax", "ktx_gemm_bf16_nt", "ktx_attn_decode", "ktx_fp8_act_quant", "ktx_linear_gemm_fp8"))   # (not ktx_ep_*: a gather replayed without its reduce would desynchronise the call tags)
 TRACE: list | None = None
 HANDLES: dict = {}      # native handle address -> weakref to the owning MoEHandle / LinearHandle (labels for traced calls)
@@ -673,7 +677,12 @@ class LinearHandle:
 
     # ---- prompt-sized W4 calls: de-quantise once (Marlin's rounding), then the library's own BF16 GEMM (csrc/ktx_gemm.hip;
     # KTX_VENDOR_GEMM=1 sends the product to torch's F.linear instead — the A/B switch of scripts/gemm_bench.py) ------------
-    PROMPT_MIN_T = 512          # below this the hand-written W4 GEMM (no scratch pass) is faster
+    PROMPT_MIN_T = 512          # below this exact integer weights (ktx_linear_forward_ws); from here Marlin's rounded multiplicand
+    # up to this many rows a product of few 256 x 256 tiles cuts K on ktx_linear_forward_ws instead of expanding the weights for a GEMM that
+    # leaves most of the chip idle (512 rows, us, expansion / tiles: 16384 -> 7168 321 / 177, 7168 -> 2112 87 / 51; 1536 -> 24576, 192 tiles:
+    # 55 / 76; 700 rows of 7168 -> 4096: 91 / 100)
+    W4_CHUNKED_MAX_T = 640
+    PROMPT_MIN_TILES = 192
     _DEQ_SCRATCH: dict = {}
 
     def dequant_bf16(self, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -709,12 +718,15 @@ class LinearHandle:
     # ---- prompt-sized FP8 calls: act_quant once per call + the block-scaled fp8 GEMM on the handle's own tiles
     # (csrc/ktx_linear_fp8gemm.inc; bit-identical to ktx_linear_forward; KTX_FP8_PROMPT_KERNEL=1 keeps the strip kernel for A/B) ----
     FP8_PROMPT_MIN_T = 128
+    FP8_CHUNKED_MAX_T = 1024    # up to here a call with K > 2048 cuts K (ktx_linear_forward_ws): 300 rows of 7168 -> 2112 93 us here, 28 there;
+                                # where K stays whole the 128 x 128 tiles of this path give the same bits, and win on large products
+    FP8_GEMM_MIN_OUT = 4 << 20  # (256 rows of 1536 -> 24576: 31 us against 37; 1000 rows of 2048 -> 576: 36 against 20)
 
     def _prompt_forward_fp8(self, x2: torch.Tensor, out, add1, add2, glu: bool) -> torch.Tensor:
         T = x2.shape[0]
         tp = (T + 127) // 128 * 128
         q = torch.empty((T, self.K), dtype=torch.uint8, device=self.device)
-        st = torch.zeros((self.K // 128, tp), dtype=torch.float32, device=self.device)   # (act_quant writes T columns: the pad rows' scales are 0, not garbage)
+        st = torch.empty((self.K // 128, tp), dtype=torch.float32, device=self.device)
         y = torch.empty((T, self.N), dtype=torch.bfloat16, device=self.device)
         sp = _stream_ptr(self.device)
         check(lib.ktx_fp8_act_quant(x2.data_ptr(), x2.stride(0), T, self.K, q.data_ptr(), st.data_ptr(), tp, sp))
@@ -799,11 +811,12 @@ class LinearHandle:
         # kernels, which take any out_features)
         gemm_ok = (self.batch == 1 and bsz_tensor is None and self.N % 8 == 0 and self.K % 64 == 0 and x2.data_ptr() % 16 == 0
                    and (x2.stride(0) * 2) % 16 == 0 and not torch.cuda.is_current_stream_capturing())
-        if (self.fmt == "W4" and gemm_ok and T >= self.PROMPT_MIN_T and not os.environ.get("KTX_W4_PROMPT_KERNEL")):
+        if (self.fmt == "W4" and gemm_ok and T >= self.PROMPT_MIN_T
+                and (T > self.W4_CHUNKED_MAX_T or -(-T // 256) * -(-self.N // 256) >= self.PROMPT_MIN_TILES) and not os.environ.get("KTX_W4_PROMPT_KERNEL")):
             if norm is not None:
                 x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)
             return self._prompt_forward(x2, out, add1, add2, glu).reshape(*x.shape[:-1], n_out)
-        if (self.fmt == "FP8" and gemm_ok and T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")):
+        if (self.fmt == "FP8" and gemm_ok and T >= self.FP8_PROMPT_MIN_T and (T > self.FP8_CHUNKED_MAX_T or self.K <= 2048) and T * self.N >= self.FP8_GEMM_MIN_OUT and not os.environ.get("KTX_FP8_PROMPT_KERNEL")):
             if norm is not None:
                 x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)
             return self._prompt_forward_fp8(x2, out, add1, add2, glu).reshape(*x.shape[:-1], n_out)
@@ -816,7 +829,10 @@ class LinearHandle:
                 raise KtxError("forward: bsz_tensor must be int32 on the handle's device")
             bsz = bsz_tensor.data_ptr()
         if norm is None and add1 is None and add2 is None and not strided and not glu:
-            check(lib.ktx_linear_forward(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), _stream_ptr(self.device)))
+            if T > 8:
+                self._forward_ws(bsz, T, x2, out, None)
+            else:
+                check(lib.ktx_linear_forward(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), _stream_ptr(self.device)))
             return out.reshape(*x.shape[:-1], self.N)
         fu = _LinearFusion(None, 0.0, None, 0, None, 0, x2.stride(0) if strided else 0, 0, 1 if glu else 0)
         keep = []
@@ -836,8 +852,20 @@ class LinearHandle:
                 setattr(fu, name, a2.data_ptr())
                 setattr(fu, name + "_ld", a2.stride(0))
                 keep.append(a2)
-        check(lib.ktx_linear_forward_fused(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), C.byref(fu), _stream_ptr(self.device)))
+        if T > 8:
+            self._forward_ws(bsz, T, x2, out, C.byref(fu))
+        else:
+            check(lib.ktx_linear_forward_fused(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), C.byref(fu), _stream_ptr(self.device)))
         return out.reshape(*x.shape[:-1], n_out)
+
+    def _forward_ws(self, bsz, T: int, x2: torch.Tensor, out: torch.Tensor, fu) -> None:
+        """ktx_linear_forward_ws with its scratch from torch's allocator (freed to the stream's pool behind the launches)."""
+        need = int(lib.ktx_linear_workspace_bytes(self._h, T, 1 if bsz is None and fu is None else 0))
+        ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
+        prompt = (T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")) if self.fmt == "FP8" else \
+            (T >= self.PROMPT_MIN_T and not os.environ.get("KTX_W4_PROMPT_KERNEL"))
+        check(lib.ktx_linear_forward_ws(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), fu, 1 if prompt else 0, ws.data_ptr() if need else None, need,
+                                        _stream_ptr(self.device)))
 
     def _forward_glu_in(self, x, bsz_tensor, out, norm, add1, add2, glu):
         if norm is not None or glu:

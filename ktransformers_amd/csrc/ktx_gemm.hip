@@ -236,7 +236,9 @@ __device__ __forceinline__ void gemm_dma_off(const void* base, uint32_t off_lane
                : "memory");
 }
 
-template <bool F32OUT>
+// BTILES: B is a dense linear's weights in the decode layout of ktx_linear.hip (16-feature strips x k-steps of 128, p.ldb = k-steps): a
+// 16-byte piece of a row is a 16-byte piece of a tile, so only the DMA's source addresses differ.
+template <bool F32OUT, bool BTILES = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm256_bf16_nt_kernel(GemmParams p) {
   using C = Gemm256;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2 stages][A_a0 | A_a1 | B_b0 | B_b1]
@@ -283,7 +285,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const int grow = min(row0 + (L >> 6) * 128 + h * 64 + (L & 63), p.M - 1);
       const int gcol = min(col0 + (L >> 5) * 64 + h * 32 + (L & 31), p.N - 1);
       offA[h][i] = (uint32_t)(((size_t)grow * p.lda) * 2 + piece * 16);
-      offB[h][i] = (uint32_t)(((size_t)gcol * p.ldb) * 2 + piece * 16);
+      offB[h][i] = BTILES ? (uint32_t)(((size_t)(gcol >> 4) * p.ldb * 4 + (piece & 3)) * 1024 + ((piece >> 2) * 16 + (gcol & 15)) * 16)
+                          : (uint32_t)(((size_t)gcol * p.ldb) * 2 + piece * 16);
     }
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(const __attribute__((address_space(3))) void*)smem) + wave * 2048;
   // half-tile slots of a stage: 0 = A_a0, 1 = A_a1, 2 = B_b0, 3 = B_b1
@@ -293,8 +296,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       gemm_dma_off(A + (size_t)kt * C::BK, offA[slot][0], dst);
       gemm_dma_off(A + (size_t)kt * C::BK, offA[slot][1], dst + 1024);
     } else {
-      gemm_dma_off(B + (size_t)kt * C::BK, offB[slot - 2][0], dst);
-      gemm_dma_off(B + (size_t)kt * C::BK, offB[slot - 2][1], dst + 1024);
+      const bf16_t* b = B + (BTILES ? (size_t)(kt >> 1) * 2048 + (kt & 1) * 256 : (size_t)kt * C::BK);
+      gemm_dma_off(b, offB[slot - 2][0], dst);
+      gemm_dma_off(b, offB[slot - 2][1], dst + 1024);
     }
   };
 
@@ -416,9 +420,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-template <bool F32OUT>
+template <bool F32OUT, bool BTILES = false>
 int launch_gemm256(GemmParams p, int batch, hipStream_t st) {
-  auto kern = gemm256_bf16_nt_kernel<F32OUT>;
+  auto kern = gemm256_bf16_nt_kernel<F32OUT, BTILES>;
   constexpr int lds = 2 * Gemm256::STAGE;
   p.tm = (p.M + 255) / 256;
   p.tn = (p.N + 255) / 256;
@@ -520,6 +524,23 @@ extern "C" int ktx_gemm_bf16_nt(const ktx_gemm_args* a, ktx_stream_t stream) {
     case 3: return f ? launch_gemm<GemmCfg<256, 128, 32, 2>, true>(p, a->batch, st) : launch_gemm<GemmCfg<256, 128, 32, 2>, false>(p, a->batch, st);
     default: return f ? launch_gemm<GemmCfg<256, 128, 64, 1>, true>(p, a->batch, st) : launch_gemm<GemmCfg<256, 128, 64, 1>, false>(p, a->batch, st);
   }
+}
+
+// ktx_internal.h: a linear's tiles as B; nsplit > 1: equal parts of K side by side, part s to Y + s * y_bs (fp32)
+int ktx_gemm256_tiles(int M, int N, int K, int nsplit, const bf16_t* A, long lda, const uint8_t* tiles, int nks, void* Y, long ldy, long y_bs,
+                      bool out_f32, hipStream_t st) {
+  KTX_REQUIRE(K % 128 == 0 && nsplit > 0 && (K / 128) % nsplit == 0 && lda % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)Y % 16 == 0 &&
+                  N % (out_f32 ? 4 : 8) == 0 && ldy % (out_f32 ? 4 : 8) == 0 && y_bs % 4 == 0 && (out_f32 || nsplit == 1) &&
+                  (size_t)M * lda * 2 < ((size_t)1 << 32) && (size_t)(N + 15) / 16 * nks * 4096 < ((size_t)1 << 32),
+              "ktx_gemm256_tiles: unsupported operands");
+  GemmParams p{};
+  p.M = M; p.N = N; p.K = K / nsplit;
+  p.A = A; p.lda = lda; p.a_bs = p.K;
+  p.B = reinterpret_cast<const bf16_t*>(tiles); p.ldb = nks; p.b_bs = (long)(p.K / 128) * 2048;
+  p.Y = Y; p.ldy = ldy; p.y_bs = y_bs;
+  KTX_TIMED(st, (double)nks * ((N + 15) / 16) * 4096.0 + (double)M * K * 2.0 + (double)M * N * nsplit * (out_f32 ? 4 : 2),
+            "gemm256_bf16_nt_kernel<%s,tiles> %dx%dx%d splits %d", out_f32 ? "f32" : "bf16", M, N, K, nsplit);
+  return out_f32 ? launch_gemm256<true, true>(p, nsplit, st) : launch_gemm256<false, true>(p, nsplit, st);
 }
 
 extern "C" int ktx_split_f32_bf16x3(const float* w, int64_t n, void* planes, ktx_stream_t stream) {

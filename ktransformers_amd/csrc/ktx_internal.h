@@ -22,4 +22,9 @@ int ktx_linear_raw(ktx_linear_t h, KtxLinearRaw* out);
 struct ktx_mla_config;
 extern "C" int ktx_mla_decode_nsplit(const ktx_mla_config* cfg, int total_q_tokens, size_t workspace_bytes);
 
+
+// Y = A . W^T on the 256 x 256 tiles of ktx_gemm.hip with a BF16 linear's decode tiles as W (no row-major copy of the weights);
+// nsplit > 1 writes that many fp32 parts of K.
+int ktx_gemm256_tiles(int M, int N, int K, int nsplit, const bf16_t* A, long lda, const uint8_t* tiles, int nks, void* Y, long ldy, long y_bs,
+                      bool out_f32, hipStream_t st);
 #endif

@@ -26,6 +26,7 @@
 // mapping, so the order inside the hardware dot product is irrelevant.
 #include "ktx_common.h"
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -1231,6 +1232,8 @@ __global__ __launch_bounds__(256) void lin_gemm_w4n_kernel(LinParams p) {
   }
 }
 
+#include "ktx_linear_tile.inc"
+
 // =====================================================================================================
 // Load-time kernels: one wavefront per W tile; lane l = kc*16 + n owns feature strip*16+n.
 // =====================================================================================================
@@ -2130,6 +2133,93 @@ extern "C" int ktx_linear_forward_fused(ktx_linear_t h, const int32_t* d_bsz, in
   const long ldx = fusion && fusion->x_ld ? (long)fusion->x_ld : (long)h->cfg.in_features * (fusion && fusion->glu_in ? 2 : 1);
   const long ldy = fusion && fusion->y_ld ? (long)fusion->y_ld : (long)(fusion && fusion->glu ? h->cfg.out_features / 2 : h->cfg.out_features);
   return linear_forward_impl(h, d_bsz, T, d_x, ldx, 0, d_y, ldy, 0, stream, fusion);
+}
+
+// 9 rows and more with a workspace: ktx_linear_tile.inc.  (dev knob 12, the strips per wavefront of the strip kernels, keeps those)
+static bool tile_eligible(const ktx_linear_s* h, int T) { return T <= h->cfg.max_len && !dec_eligible(h, T) && !ktx_debug_get(12) && !g_lin_force_gemm; }
+static bool tile_plan(const ktx_linear_s* h, int T, LinTilePlan* o) {
+  return lin_tile_plan(h->cfg.format, 128 / std::max(h->cfg.group_size, 1), h->cfg.out_features, h->cfg.in_features, h->NKS, h->batch, T, o);
+}
+static int gemm_parts(const ktx_linear_s* h, int T) {
+  return h->cfg.format == KTX_LIN_BF16 ? lin_gemm_parts(h->cfg.out_features, h->cfg.in_features, h->NKS, h->batch, T) : 0;
+}
+// the GEMM's own epilogue writes y (no row count on the device, no bias, adds or GLU; whole 16-byte pieces)
+static bool gemm_direct(const ktx_linear_s* h, int parts, int plain) { return parts == 1 && plain && !h->d_bias && h->cfg.out_features % 8 == 0; }
+static size_t gemm_ws(const ktx_linear_s* h, int T, int parts) { return (size_t)parts * T * h->nstrips * 16 * sizeof(float); }
+
+extern "C" size_t ktx_linear_workspace_bytes(ktx_linear_t h, int T, int plain) {
+  LinTilePlan o;
+  if (!h || !tile_eligible(h, T)) return 0;
+  if (const int parts = gemm_parts(h, T)) return gemm_direct(h, parts, plain) ? 0 : gemm_ws(h, T, parts);
+  return tile_plan(h, T, &o) ? o.part_bytes + o.sT_bytes + o.xq_bytes : 0;
+}
+
+extern "C" int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T, const void* d_x, void* d_y, const ktx_linear_fusion* fu,
+                                     int prompt, void* d_ws, size_t ws_bytes, ktx_stream_t stream) {
+  KTX_REQUIRE(h && d_x && d_y, "ktx_linear_forward_ws: null argument");
+  KTX_REQUIRE(h->loaded, "ktx_linear_forward_ws: weights not loaded");
+  KTX_REQUIRE(h->batch == 1, "ktx_linear_forward_ws: batched handle (use ktx_linear_forward_batched)");
+  KTX_REQUIRE(T >= 0 && T <= h->cfg.max_len, "ktx_linear_forward_ws: T exceeds max_len");
+  const long ldx = fu && fu->x_ld ? (long)fu->x_ld : (long)h->cfg.in_features;
+  // (16-byte LDS-DMA pieces of the activation rows: other alignments stay on the strip kernels' plain loads)
+  const bool ok = tile_eligible(h, T) && (uintptr_t)d_x % 16 == 0 && ldx % 8 == 0 && !(fu && (fu->norm_weight || fu->glu_in));
+  auto ws_fits = [&](size_t need) { return need == 0 || (d_ws && (uintptr_t)d_ws % 16 == 0 && ws_bytes >= need); };
+  LinTilePlan o;
+  int parts = ok && (size_t)T * ldx * 2 < ((size_t)1 << 32) ? gemm_parts(h, T) : 0;
+  const bool direct = gemm_direct(h, parts, !d_bsz && (!fu || (!fu->add1 && !fu->add2 && !fu->glu))) && (uintptr_t)d_y % 16 == 0 && (!fu || fu->y_ld % 8 == 0);
+  if (!direct && parts && !ws_fits(gemm_ws(h, T, parts))) parts = 0;
+  if (!parts && !(ok && tile_plan(h, T, &o) && ws_fits(o.part_bytes + o.sT_bytes + o.xq_bytes)))
+    return ktx_linear_forward_fused(h, d_bsz, T, d_x, d_y, fu, stream);
+  LinTileParams q{};
+  LinParams& p = q.p;
+  p.w = h->d_w; p.sc = h->d_sc; p.bias = h->d_bias;
+  p.x = (const bf16_t*)d_x; p.y = (bf16_t*)d_y; p.d_bsz = d_bsz;
+  p.T = T; p.N = h->cfg.out_features; p.Kx = h->cfg.in_features; p.NKS = h->NKS; p.nstrips = h->nstrips;
+  p.ldx = ldx;
+  p.ldy = fu && fu->y_ld ? (long)fu->y_ld : (long)(fu && fu->glu ? h->cfg.out_features / 2 : h->cfg.out_features);
+  if (fu) {
+    p.add1 = (const bf16_t*)fu->add1; p.ld1 = fu->add1_ld ? fu->add1_ld : h->cfg.out_features;
+    p.add2 = (const bf16_t*)fu->add2; p.ld2 = fu->add2_ld ? fu->add2_ld : h->cfg.out_features;
+    p.glu = fu->glu ? 1 : 0;
+    KTX_REQUIRE(!p.glu || (h->cfg.out_features % 16 == 0 && !h->d_bias && !p.add1 && !p.add2),
+                "ktx_linear_forward_ws: glu needs out_features % 16 == 0 and no bias / addends");
+  }
+  hipStream_t st = (hipStream_t)stream;
+  uint8_t* ws = (uint8_t*)d_ws;
+  if (direct) return ktx_gemm256_tiles(T, p.N, p.Kx, 1, p.x, ldx, h->d_w, h->NKS, d_y, p.ldy, 0, false, st);
+  if (parts) {
+    q.part = (float*)ws; q.npad = (long)h->nstrips * 16; q.nch = parts;
+    const int rc = ktx_gemm256_tiles(T, (int)q.npad, p.Kx, parts, p.x, ldx, h->d_w, h->NKS, ws, q.npad, (long)T * q.npad, true, st);
+    return rc ? rc : launch_tile_reduce(q, st);
+  }
+  q.part = o.split ? (float*)ws : nullptr;
+  q.npad = (long)h->nstrips * 16;
+  q.chk = o.chk; q.nch = o.nch; q.nft = o.nft; q.ntt = o.ntt;
+  q.s_ld = (T + 127) / 128 * 128;
+  q.sT = (const float*)(ws + o.part_bytes);
+  q.xq = ws + o.part_bytes + o.sT_bytes;
+  if (h->cfg.format == KTX_LIN_FP8) {
+    const int rc = ktx_fp8_act_quant(d_x, ldx, T, p.Kx, (void*)q.xq, (float*)q.sT, q.s_ld, stream);
+    if (rc) return rc;
+    return prompt && o.mt >= 4 ? forward_tile<F_FP8, 128, true>(o, q, st) : forward_tile<F_FP8, 128>(o, q, st);
+  }
+  const int g = h->cfg.group_size;
+  const bool alt = prompt && h->cfg.format == KTX_LIN_W4 && o.mt >= 4;
+  if (o.sT_bytes && !alt) {
+    const dim3 grid((unsigned)((q.s_ld * (p.Kx / 8) + 255) / 256));
+    KTX_TIMED(st, (double)T * p.Kx * 2.0, "lin_tile_sums_kernel T=%d K=%d", T, p.Kx);
+    if (g == 32) hipLaunchKernelGGL(lin_tile_sums_kernel<32>, grid, dim3(256), 0, st, p.x, ldx, T, p.Kx, (float*)q.sT, q.s_ld);
+    else if (g == 64) hipLaunchKernelGGL(lin_tile_sums_kernel<64>, grid, dim3(256), 0, st, p.x, ldx, T, p.Kx, (float*)q.sT, q.s_ld);
+    else hipLaunchKernelGGL(lin_tile_sums_kernel<128>, grid, dim3(256), 0, st, p.x, ldx, T, p.Kx, (float*)q.sT, q.s_ld);
+    KTX_HIP(hipGetLastError());
+  }
+  switch (h->cfg.format) {
+    case KTX_LIN_BF16: return forward_tile<F_BF16, 128>(o, q, st);
+    case KTX_LIN_W8: return g == 32 ? forward_tile<F_W8, 32>(o, q, st) : g == 64 ? forward_tile<F_W8, 64>(o, q, st) : forward_tile<F_W8, 128>(o, q, st);
+    default:
+      if (alt) return g == 32 ? forward_tile<F_W4, 32, true>(o, q, st) : g == 64 ? forward_tile<F_W4, 64, true>(o, q, st) : forward_tile<F_W4, 128, true>(o, q, st);
+      return g == 32 ? forward_tile<F_W4, 32>(o, q, st) : g == 64 ? forward_tile<F_W4, 64>(o, q, st) : forward_tile<F_W4, 128>(o, q, st);
+  }
 }
 
 extern "C" int ktx_linear_decode_eligible(ktx_linear_t h, int T) { return h && dec_eligible(h, T) ? 1 : 0; }

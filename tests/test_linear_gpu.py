@@ -693,3 +693,54 @@ def test_five_to_eight_rows_run_as_four_row_passes_of_the_decode_kernel(fmt, K, 
         n.check(n.lib.ktx_debug_set(3, 0))
     for a, b in zip(fast, slow):
         close(a, b.cpu())
+
+
+@pytest.mark.parametrize("fmt", ["W4", "FP8", "BF16"])
+@pytest.mark.parametrize("K,N,T", [(128, 17, 9), (384, 200, 33), (2176, 577, 16), (7168, 2112, 65), (2176, 1040, 130), (2048, 4104, 300),
+                                   (7168, 1536, 513), (2048, 12288, 520)])
+def test_batches_and_short_prompts_on_tiles(fmt, K, N, T):
+    """ktx_linear_forward_ws (ktx_linear_tile.inc; BF16 from 512 rows the GEMM's 256 x 256 tiles): ragged rows, features and last k-chunk,
+    split and whole K, bias, addends, GLU, strided and misaligned rows, a device-side row count — against the oracle at the file's bound;
+    and an operator's rows do not depend on what else is in the matrix (K is cut by K and T alone)."""
+    n = native()
+    torch.manual_seed(K + N + T)
+    w = (torch.randn(N, K) / 10).to(torch.bfloat16)
+    x = (torch.randn(T, K) / 10).to(torch.bfloat16)
+    bias = (torch.randn(N) / 10).to(torch.bfloat16)
+    w8, sc = (torch.randn(N, K) / 4).to(torch.float8_e4m3fn), (torch.rand((N + 127) // 128, K // 128) + 0.5) / 32
+
+    def handle(rows, b):
+        h = n.LinearHandle(K, rows, fmt, {"W4": 64, "FP8": 128, "BF16": 0}[fmt], 1024)
+        bb = bias[:rows].cuda() if b else None
+        if fmt == "FP8":
+            h.load_fp8(w8[:rows].cuda(), sc[: (rows + 127) // 128].cuda(), bb)
+        else:
+            h.load_bf16(w[:rows].cuda(), bb)
+        return h
+
+    ref = (linear_fp8_ref(x, w8, sc) if fmt == "FP8" else linear_bf16_ref(x, w) if fmt == "BF16" else
+           linear_w4_ref(x, *quantize_weights_ref(w.T.contiguous(), 64), 64, round_weights=T >= 512)).float()
+
+    h, hb, xc = handle(N, False), handle(N, True), x.cuda()
+    y = h.forward(xc)
+    close(y, ref, rel=2e-3)
+    # the bias is added to the rounded sum (or, in the W4 GEMM, to the sum): a half ulp of either, on top of the half ulp that y carries
+    want = y.float() + bias.cuda().float()
+    assert bool(((hb.forward(xc).float() - want).abs() <= 2.0 ** -8 * (y.float().abs() + want.abs())).all()), "bias"
+    a1, a2 = (torch.randn(T, N).to(torch.bfloat16).cuda() for _ in range(2))
+    assert torch.equal(h.forward(xc, add1=a1, add2=a2), a2 + (a1 + y))
+    wide = torch.zeros(T, K + 64, dtype=torch.bfloat16, device="cuda")
+    wide[:, 8:K + 8] = xc
+    assert torch.equal(h.forward(wide[:, 8:K + 8]), y), "strided rows"
+    wide[:, 3:K + 3] = xc
+    close(h.forward(wide[:, 3:K + 3]), ref, rel=2e-3)
+    got = h.forward(xc, bsz_tensor=torch.tensor([T - 3], dtype=torch.int32, device="cuda"))
+    if fmt == "FP8" or T < 512:      # (a bf16 or 4-bit prompt with a device-side row count takes another path)
+        close(got[: T - 3], y[: T - 3].float().cpu())
+    assert not bool(got[T - 3:].any())
+    if N % 16 == 0:
+        g = y.float().view(T, N // 16, 2, 8)
+        s = (g[:, :, 0] / (1 + torch.exp(-g[:, :, 0]))).to(torch.bfloat16).float()
+        close(h.forward(xc, glu=True), (s * g[:, :, 1]).reshape(T, N // 2).cpu(), rel=5e-3)
+    if N > 256 and T < 512:
+        assert torch.equal(handle(256, False).forward(xc), y[:, :256]), "a merged operator's rows"
