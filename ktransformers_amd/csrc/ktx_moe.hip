@@ -1754,8 +1754,14 @@ struct RawGemmParams {
   bf16_t* out;                 // [sorted rows][N]
 };
 
-template <int NT, bool GATE_UP>
-__global__ __launch_bounds__(256) void moe_rawint4_gemm_kernel(RawGemmParams p) {
+// Bound by the weights' bytes while an expert sees a token or two (a decode batch: 16 tokens over 384 experts) and by the VALU from about four
+// on: a scale product, a conversion and an fma per (token, weight row, 4 k).  So the work per (weight row, 4 k) follows the tile's rows
+// (1, 2 or up to 4: a v_dot4 per token, from 3 on one 4x4x4 MFMA for all of them: the same integers), and D = 2 512-k steps of weights stay
+// requested per wavefront, two workgroups per CU (4 steps spill).  The kernel before it did four tokens' work for every tile and kept 408 registers (one
+// wavefront per SIMD, one step in flight): 16 tokens at Kimi-K2's sizes, gate|up + down: 489 + 150 us -> 262 + 133 (2.1 GB of weights and scales: 390 us at the
+// rate a large read reaches).
+template <int D, bool GATE_UP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATE_UP ? 2 : 4, 4))) void moe_rawint4_rows_kernel(RawGemmParams p) {
   constexpr int NMAT = GATE_UP ? 2 : 1;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int KP = p.K + 32;                                        // padded activation row (bank spread of the 4 tokens)
@@ -1773,6 +1779,30 @@ __global__ __launch_bounds__(256) void moe_rawint4_gemm_kernel(RawGemmParams p) 
   const int NS = p.K / 512, G = p.K / 32;
   const int L = lane >> 2, j = lane & 3, hsel = L >> 3;
 
+  // (step, matrix) pairs in turns through a ring of D slots; the launcher picks D so that it divides their number
+  struct Slot { uint4 w[4], s[4]; };
+  const uint8_t* wb[NMAT];
+  const bf16_t* sb[NMAT];
+  const int ls = strip_ok ? strip : 0;
+  wb[0] = p.w0 + (size_t)tile.expert * p.expert_stride + (size_t)(ls * 4) * NS * 1024 + lane * 16;
+  sb[0] = p.s0 + (size_t)tile.expert * p.scale_stride + (size_t)(ls * 4) * NS * 64 + (j * 2 + hsel) * 8;
+  if constexpr (GATE_UP) {
+    wb[1] = p.w1 + (size_t)tile.expert * p.expert_stride + (size_t)(ls * 4) * NS * 1024 + lane * 16;
+    sb[1] = p.s1 + (size_t)tile.expert * p.scale_stride + (size_t)(ls * 4) * NS * 64 + (j * 2 + hsel) * 8;
+  }
+  const int total = NS * NMAT;
+  auto load_slot = [&](Slot& d, auto mc, int idx) {
+    constexpr int m = decltype(mc)::value;
+    const int st = min(idx, total - 1) / NMAT;      // (past the end: the last step again, from the caches)
+#pragma unroll
+    for (int rg = 0; rg < 4; rg++) {
+      d.w[rg] = *reinterpret_cast<const uint4*>(wb[m] + ((size_t)rg * NS + st) * 1024);
+      d.s[rg] = *reinterpret_cast<const uint4*>(sb[m] + ((size_t)rg * NS + st) * 64);
+    }
+  };
+  Slot ring[D];
+  static_for<D>([&](auto dc) { load_slot(ring[decltype(dc)::value], std::integral_constant<int, decltype(dc)::value % NMAT>{}, decltype(dc)::value); });
+
   if (tid < 4) s_src[tid] = tid < tile.nrows ? (p.row_src ? p.row_src[tile.row0 + tid] : tile.row0 + tid) : -1;
   __syncthreads();
   for (int u = tid; u < 4 * (p.K / 16); u += 256) {
@@ -1788,140 +1818,133 @@ __global__ __launch_bounds__(256) void moe_rawint4_gemm_kernel(RawGemmParams p) 
   __syncthreads();
   if (!strip_ok) return;
 
-  float acc[NMAT][4][NT];
+  auto body = [&](auto ntc) __attribute__((always_inline)) {
+    constexpr int NT = decltype(ntc)::value;
+    float acc[NMAT][4][NT];
 #pragma unroll
-  for (int m = 0; m < NMAT; m++)
+    for (int m = 0; m < NMAT; m++)
 #pragma unroll
-    for (int rg = 0; rg < 4; rg++)
+      for (int rg = 0; rg < 4; rg++)
 #pragma unroll
-      for (int r = 0; r < NT; r++) acc[m][rg][r] = 0.0f;
-
-  const uint8_t* wb[NMAT];
-  const bf16_t* sb[NMAT];
-  wb[0] = p.w0 + (size_t)tile.expert * p.expert_stride + (size_t)(strip * 4) * NS * 1024 + lane * 16;
-  sb[0] = p.s0 + (size_t)tile.expert * p.scale_stride + (size_t)(strip * 4) * NS * 64 + (j * 2 + hsel) * 8;
-  if constexpr (GATE_UP) {
-    wb[1] = p.w1 + (size_t)tile.expert * p.expert_stride + (size_t)(strip * 4) * NS * 1024 + lane * 16;
-    sb[1] = p.s1 + (size_t)tile.expert * p.scale_stride + (size_t)(strip * 4) * NS * 64 + (j * 2 + hsel) * 8;
-  }
-  const int8_t* xa = xq + j * KP + 4 * L;   // A operand: lane (L, i = j) supplies token i's 4 int8 of AVX lane L
-
-  // Double buffer over (512-k step, matrix) pairs, ONE matrix per buffer: gate and up of a step take turns (the activation
-  // fragments are re-read from LDS for the second).  Round 2 kept both matrices of the current AND the next step in
-  // registers (128 VGPRs of operands beside 32 accumulators): the 4-token gate|up variant spilled 100 B per lane to scratch.
-  // Every accumulator still receives its blocks in the same order: results unchanged.
-  uint4 wcur[4], scur[4], wnxt[4], snxt[4];
-  auto load_step = [&](auto mc, uint4(&w)[4], uint4(&sc)[4], int st) {
-    constexpr int m = decltype(mc)::value;
+        for (int r = 0; r < NT; r++) acc[m][rg][r] = 0.0f;
+    const int8_t* xa = NT < 4 ? xq + 4 * L : xq + j * KP + 4 * L;   // MFMA A operand: lane (L, i = j) supplies token i's 4 int8 of AVX lane L
+    auto compute = [&](const Slot& sl, float (&ac)[4][NT], int st) __attribute__((always_inline)) {
 #pragma unroll
-    for (int rg = 0; rg < 4; rg++) {
-      w[rg] = *reinterpret_cast<const uint4*>(wb[m] + ((size_t)rg * NS + st) * 1024);
-      sc[rg] = *reinterpret_cast<const uint4*>(sb[m] + ((size_t)rg * NS + st) * 64);
-    }
-  };
-  auto compute_step = [&](auto mc, uint4(&w)[4], uint4(&sc)[4], int st) {
-    constexpr int m = decltype(mc)::value;
+      for (int kb8 = 0; kb8 < 8; kb8++) {
+        const int kb = st * 8 + kb8;
+        int a_op[NT < 4 ? NT : 1];
+        float asv[NT];
 #pragma unroll
-    for (int kb8 = 0; kb8 < 8; kb8++) {
-      const int kb = st * 8 + kb8;
-      const int a_op = *reinterpret_cast<const int*>(xa + 64 * kb);
-      const float4 as4 = *reinterpret_cast<const float4*>(as_l + (2 * kb + hsel) * 4);
-      const float asv[4] = {as4.x, as4.y, as4.z, as4.w};
+        for (int r = 0; r < (NT < 4 ? NT : 1); r++) a_op[r] = *reinterpret_cast<const int*>(xa + r * KP + 64 * kb);
+        if constexpr (NT == 1) asv[0] = as_l[(2 * kb + hsel) * 4];
+        else if constexpr (NT == 2) { const float2 v = *reinterpret_cast<const float2*>(as_l + (2 * kb + hsel) * 4); asv[0] = v.x; asv[1] = v.y; }
+        else { const float4 v = *reinterpret_cast<const float4*>(as_l + (2 * kb + hsel) * 4); asv[0] = v.x; asv[1] = v.y; asv[2] = v.z; asv[3] = v.w; }
+#pragma unroll
+        for (int rg = 0; rg < 4; rg++) {
+          const uint32_t P = kb8 < 2 ? sl.w[rg].x : kb8 < 4 ? sl.w[rg].y : kb8 < 6 ? sl.w[rg].z : sl.w[rg].w;
+          const int b_op = (kb8 & 1) ? (int)(P & 0xF0F0F0F0u) : (int)((P << 4) & 0xF0F0F0F0u);
+          const uint32_t S = kb8 < 2 ? sl.s[rg].x : kb8 < 4 ? sl.s[rg].y : kb8 < 6 ? sl.s[rg].z : sl.s[rg].w;
+          const float bs = __uint_as_float((kb8 & 1) ? (S & 0xffff0000u) : (S << 16));
+          if constexpr (NT < 4) {
+#pragma unroll
+            for (int r = 0; r < NT; r++) ac[rg][r] = fmaf(asv[r] * bs, (float)__builtin_amdgcn_sdot4(a_op[r], b_op, 0, false), ac[rg][r]);
+          } else {
+            const v4i d = __builtin_amdgcn_mfma_i32_4x4x4i8(a_op[0], b_op, v4i{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < NT; r++) ac[rg][r] = fmaf(asv[r] * bs, (float)d[r], ac[rg][r]);
+          }
+        }
+        if constexpr (!GATE_UP) __builtin_amdgcn_sched_barrier(0);   // one 64-k block at a time: hoisted over all eight, the operands spill
+      }
+    };
+    for (int s0 = 0; s0 < total; s0 += D)
+      static_for<D>([&](auto dc) {
+        constexpr int d = decltype(dc)::value, m = d % NMAT;
+        compute(ring[d], acc[m], (s0 + d) / NMAT);
+        load_slot(ring[d], std::integral_constant<int, m>{}, s0 + d + D);
+      });
+    // _mm512_reduce_add_ps tree over the 16 AVX lanes (lane bits 5,4,3,2), then /16 (amx_kernels.hpp:3385-3450)
+#pragma unroll
+    for (int m = 0; m < NMAT; m++)
+#pragma unroll
+      for (int rg = 0; rg < 4; rg++)
+#pragma unroll
+        for (int r = 0; r < NT; r++) {
+          float v = acc[m][rg][r];
+          v = v + __shfl_xor(v, 32, 64);
+          v = v + __shfl_xor(v, 16, 64);
+          v = v + __shfl_xor(v, 8, 64);
+          v = v + __shfl_xor(v, 4, 64);
+          acc[m][rg][r] = v / 16.0f;
+        }
+    if (L == 0) {
 #pragma unroll
       for (int rg = 0; rg < 4; rg++) {
-        const uint32_t P = kb8 < 2 ? w[rg].x : kb8 < 4 ? w[rg].y : kb8 < 6 ? w[rg].z : w[rg].w;
-        const int b_op = (kb8 & 1) ? (int)(P & 0xF0F0F0F0u) : (int)((P << 4) & 0xF0F0F0F0u);
-        const uint32_t S = kb8 < 2 ? sc[rg].x : kb8 < 4 ? sc[rg].y : kb8 < 6 ? sc[rg].z : sc[rg].w;
-        const float bs = __uint_as_float((kb8 & 1) ? (S & 0xffff0000u) : (S << 16));
-        const v4i d = __builtin_amdgcn_mfma_i32_4x4x4i8(a_op, b_op, v4i{0, 0, 0, 0}, 0, 0, 0);
+        const int n = strip * 16 + rg * 4 + j;
 #pragma unroll
-        for (int r = 0; r < NT; r++) acc[m][rg][r] = fmaf(asv[r] * bs, (float)d[r], acc[m][rg][r]);
-      }
-    }
-  };
-  using M0 = std::integral_constant<int, 0>;
-  using M1 = std::integral_constant<int, NMAT - 1>;
-  load_step(M0{}, wcur, scur, 0);
-  if constexpr (GATE_UP) {
-    for (int st = 0; st < NS; st++) {
-      load_step(M1{}, wnxt, snxt, st);
-      compute_step(M0{}, wcur, scur, st);
-      if (st + 1 < NS) load_step(M0{}, wcur, scur, st + 1);
-      compute_step(M1{}, wnxt, snxt, st);
-    }
-  } else {
-    for (int st = 0; st < NS; st += 2) {
-      if (st + 1 < NS) load_step(M0{}, wnxt, snxt, st + 1);
-      compute_step(M0{}, wcur, scur, st);
-      if (st + 1 < NS) {
-        if (st + 2 < NS) load_step(M0{}, wcur, scur, st + 2);
-        compute_step(M0{}, wnxt, snxt, st + 1);
-      }
-    }
-  }
-
-  // _mm512_reduce_add_ps tree over the 16 AVX lanes (lane bits 5,4,3,2), then /16 (amx_kernels.hpp:3385-3450)
-#pragma unroll
-  for (int m = 0; m < NMAT; m++)
-#pragma unroll
-    for (int rg = 0; rg < 4; rg++)
-#pragma unroll
-      for (int r = 0; r < NT; r++) {
-        float v = acc[m][rg][r];
-        v = v + __shfl_xor(v, 32, 64);
-        v = v + __shfl_xor(v, 16, 64);
-        v = v + __shfl_xor(v, 8, 64);
-        v = v + __shfl_xor(v, 4, 64);
-        acc[m][rg][r] = v / 16.0f;
-      }
-  if (L == 0) {
-#pragma unroll
-    for (int rg = 0; rg < 4; rg++) {
-      const int n = strip * 16 + rg * 4 + j;
-#pragma unroll
-      for (int r = 0; r < NT; r++) {
-        if (r < tile.nrows) {
-          const bf16_t g = f32_to_bf16(acc[0][rg][r]);
-          bf16_t o = g;
-          if constexpr (GATE_UP) {
-            const bf16_t u = f32_to_bf16(acc[1][rg][r]);
-            o = f32_to_bf16(act_fn(bf16_to_f32(g), bf16_to_f32(u)));
+        for (int r = 0; r < NT; r++) {
+          if (r < tile.nrows) {
+            const bf16_t g = f32_to_bf16(acc[0][rg][r]);
+            bf16_t o = g;
+            if constexpr (GATE_UP) {
+              const bf16_t u = f32_to_bf16(acc[NMAT - 1][rg][r]);
+              o = f32_to_bf16(act_fn(bf16_to_f32(g), bf16_to_f32(u)));
+            }
+            p.out[(size_t)(tile.row0 + r) * p.N + n] = o;
           }
-          p.out[(size_t)(tile.row0 + r) * p.N + n] = o;
         }
       }
     }
-  }
+  };
+  if (tile.nrows == 1) body(std::integral_constant<int, 1>{});
+  else if (tile.nrows == 2) body(std::integral_constant<int, 2>{});
+  else body(std::integral_constant<int, 4>{});
 }
 
 // =====================================================================================================
-// RAWINT4 prompt chunks: the same products on the 16x16x32 int8 MFMA, one MFMA per (32-k group) x (16 rows) x (16 tokens).
+// RAWINT4 prompt chunks: the same products on the 16x16x32 f16 MFMA, one MFMA per (32-k group) x (16 rows) x (16 tokens).
 //
-// The exact kernel above keeps the reference's SIXTEEN fp32 lane accumulators per output, i.e. one convert + multiply + fma per
-// FOUR int8 products (4x4x4 MFMA blocks, four tokens per tile, every weight byte re-read and re-unpacked per four tokens): 38 ms
-// per Kimi-K2 layer at a 2048-token chunk against 1.4 ms for the AMXINT4 format (profiles/r04_final).  A prompt chunk does not
-// need that association: the terms of an output are the per-group sums  (as[t][g] * bs[n][g]) * float(sum_{k in g} a[t][k] * 16 q[n][k])
-// — the reference adds them as 16 interleaved chains + a tree, this kernel as ONE chain over the groups in k order (the
-// integer group sum is exact either way, so only the association of <= K/32 fp32 additions differs: <= a few fp32 ulps before the
-// one bf16 rounding; tests/test_moe_gpu.py::test_rawint4_prompt_chunks holds it to the bound of the FP8 / BF16 formats, whose
-// prompt kernels re-associate in the same way).  Decode and short batches (qlen < 64) keep the exact kernels; dev knob 29 = 1
+// The exact kernel above keeps the reference's SIXTEEN fp32 lane accumulators per output.  A prompt chunk does not need that
+// association: the terms of an output are the per-group sums  as[t][g] * bs[n][g] * sum_{k in g} a[t][k] * q[n][k]  — the reference adds
+// them as 16 interleaved chains + a tree, this kernel as ONE chain over the groups in k order, held to the bound of the FP8 / BF16 formats
+// (tests/test_moe_gpu.py::test_rawint4_prompt_chunks).  Decode and short batches (qlen < 64) keep the exact kernels; dev knob 29 = 1
 // forces them for every size.
+//
+// What bounds it is the VALU work per MFMA, so the operands carry what can be carried exactly: the activation codes are f16 integers, the
+// weights f16 q * bs — 4 and 8 significant bits, exact in f16's 11 for scales of 2^-17 .. 2^11 (ktx_moe_load_rawint4 looks; other scales
+// stay on the exact kernel) — and the products' fp32 sum over a group is exact as well.  What is left per 16 x 16 fragment and group is
+// acc = fma(as, sum, acc): 4 operations instead of the 12 of an int8 MFMA (scale product, conversion, fma).  A group's 8 weights of a lane
+// become f16 in 17 operations for all token fragments: a nibble goes to the top mantissa bits of an f16 (16 + q'), and
+// fma(16 + q', bs, -24 bs) is q * bs with both constants exact.
 //
 // No second copy of the weights: the RAW tiles are read as they lie in HBM.  MFMA lane (i = lane & 15, kc = lane >> 4) needs
 // row i's eight nibbles k = 64 kb + 32 h + 8 kc + [0, 8) of group (kb, h): those are the pieces (L, j) = (8h + 2kc + o, i & 3),
-// o = 0 / 1, of RAW tile rg = i >> 2 — so the lane loads exactly its four pieces q = (h, o) of the strip's four tiles (16 bytes
-// each, every 128-byte line of the 4 KiB used by one wave instruction pair) and nothing moves between lanes.
-//   workgroup = 8 wavefronts = 8 strips of 16 weight rows x (gate, up) x 64 tokens; K walks in the RAW step of 512 (16 groups):
-//   activations + their group scales of the step are double-buffered in LDS, the step's weights + scales in registers.
+// o = 0 / 1, of RAW tile rg = i >> 2 — so the lane loads exactly its four pieces q = (h, o) of the strip's four tiles and nothing moves
+// between lanes; inside 8 k the pairs come out as (0,2) (1,3) (4,6) (5,7), the order in which the activation codes are stored.
+//   workgroup = 4 wavefronts = 4 strips of 16 weight rows x (gate, up), or 8 strips of down, x 64 tokens, two workgroups per CU (one
+//   multiplies while the other waits); K walks in the RAW step of 512, the activations in halves of it.  The next half's activations
+//   (LDS-DMA, XOR-swizzled rows; only the live 16-row groups) and the next step's weights (registers) are requested before the MFMAs
+//   and waited for behind them.
+// At Kimi-K2's sizes, us for the whole forward, int8 operands staged through registers -> here: 64 tokens 2256 -> 929, 256 3068 -> 1625, 2048
+// 5008 -> 4043 (gate|up 3169 -> 2519, down 1693 -> 1389: VALU instructions fill 70 % of the issue slots, two thirds of them the widening).
 // =====================================================================================================
+typedef _Float16 raw_h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 raw_h8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ uint32_t raw_h2_bits(raw_h2 v) { return __builtin_bit_cast(uint32_t, v); }
+// the pairs (byte 0, byte 2) and (byte 1, byte 3) of the low (par 0) or high nibbles of x as q * bs; x: two's complement nibbles ^ 8
+template <int PAR>
+__device__ __forceinline__ void raw_widen(uint32_t x, uint32_t mask, uint32_t top, raw_h2 bs, raw_h2 m24, uint32_t& o0, uint32_t& o1) {
+  const uint32_t e0 = ((PAR ? x << 2 : x << 6) & mask) | top, e1 = ((PAR ? x >> 6 : x >> 2) & mask) | top;
+  o0 = raw_h2_bits(__builtin_elementwise_fma(__builtin_bit_cast(raw_h2, e0), bs, m24));
+  o1 = raw_h2_bits(__builtin_elementwise_fma(__builtin_bit_cast(raw_h2, e1), bs, m24));
+}
+
 template <bool GATE_UP>
-__global__ __launch_bounds__(512) void moe_rawint4_chunk_kernel(RawGemmParams p) {
-  constexpr int NU = 2;                             // B operands per wavefront that share one activation fragment: (gate, up) of a
-                                                    // strip, or two strips of down (one fragment + scale read per two MFMAs: LDS port)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_rawint4_chunk_kernel(RawGemmParams p) {
+  constexpr int NW = 4, NU = 2;                     // NU weight operands per wavefront share one activation fragment: (gate, up) of a
+                                                    // strip, or two strips of down
   constexpr int TOK = 64, MT = 4;
-  constexpr int CS = TOK * 16 + 16;                 // bytes between 16-byte activation columns (+16: staging writes spread over banks)
-  constexpr int XB = 32 * CS;                       // one step of activations: 32 columns x 64 tokens x 16 B
-  constexpr int AB = 16 * TOK * 4;                  // one step of activation scales: [16 groups][64 tokens] fp32
+  constexpr int XB = TOK * 512, AB = 8 * TOK * 4;   // half a step (256 k): activation codes (f16), their group scales [8 groups][64 tokens]
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][XB] | [2][AB]
   __shared__ int s_src[TOK];
   uint8_t* xs = smem;
@@ -1937,63 +1960,73 @@ __global__ __launch_bounds__(512) void moe_rawint4_chunk_kernel(RawGemmParams p)
   const int i = lane & 15, kc = lane >> 4, rg = i >> 2, j = i & 3;
   int ustrip[NU];
 #pragma unroll
-  for (int u = 0; u < NU; u++) ustrip[u] = GATE_UP ? blockIdx.x * 8 + wave : (blockIdx.x * 8 + wave) * 2 + u;
+  for (int u = 0; u < NU; u++) ustrip[u] = GATE_UP ? blockIdx.x * NW + wave : (blockIdx.x * NW + wave) * 2 + u;
   const bool wave_ok = ustrip[0] < nstrips;
 
-  if (tid < TOK) s_src[tid] = tid < tile.nrows ? (p.row_src ? p.row_src[tile.row0 + tid] : tile.row0 + tid) : -1;
+  // rows past the tile read its first row again (their outputs are never stored)
+  if (tid < TOK) {
+    const int r = tile.row0 + (tid < tile.nrows ? tid : 0);
+    s_src[tid] = p.row_src ? p.row_src[r] : r;
+  }
   __syncthreads();
+  const int mt_live = (tile.nrows + 15) >> 4;
 
   // ---- this lane's four pieces of each unit's four RAW tiles, and its row's scales (a strip past N aliases strip 0, not stored)
-  const uint8_t* wb[NU];
-  const bf16_t* sb[NU];
+  const uint8_t* wb[NU];        // uniform bases + 32-bit lane offsets: the registers are full
+  const uint8_t* sb[NU];
+  uint32_t wo[NU], so[NU];
 #pragma unroll
   for (int u = 0; u < NU; u++) {
     const int st = ustrip[u] < nstrips ? ustrip[u] : 0;
-    const uint8_t* w = (GATE_UP && u) ? p.w1 : p.w0;
-    const bf16_t* sc = (GATE_UP && u) ? p.s1 : p.s0;
-    wb[u] = w + (size_t)tile.expert * p.expert_stride + ((size_t)(st * 4 + rg) * NS) * 1024 + (size_t)((2 * kc) * 4 + j) * 16;
-    sb[u] = sc + (size_t)tile.expert * p.scale_stride + ((size_t)(st * 4 + rg) * NS) * 64 + (size_t)(j * 2) * 8;
+    wb[u] = ((GATE_UP && u) ? p.w1 : p.w0) + (size_t)tile.expert * p.expert_stride + (size_t)(st * 4) * NS * 1024;
+    sb[u] = reinterpret_cast<const uint8_t*>(((GATE_UP && u) ? p.s1 : p.s0) + (size_t)tile.expert * p.scale_stride + (size_t)(st * 4) * NS * 64);
+    wo[u] = (uint32_t)(rg * NS * 1024 + ((2 * kc) * 4 + j) * 16);
+    so[u] = (uint32_t)(rg * NS * 128 + j * 32);
   }
   struct WStep { uint4 w[NU][4]; uint4 s[NU][2]; };   // w[u][h * 2 + o]: piece L = 8h + 2kc + o; s[u][h]: 8 bf16 scales (kb = 0..7)
+  constexpr int WLOADS = NU * 6;
   auto load_w = [&](WStep& d, int st) {
 #pragma unroll
     for (int u = 0; u < NU; u++) {
 #pragma unroll
       for (int q = 0; q < 4; q++)
-        d.w[u][q] = *reinterpret_cast<const uint4*>(wb[u] + (size_t)st * 1024 + ((q >> 1) * 8 + (q & 1)) * 64);
+        d.w[u][q] = *reinterpret_cast<const uint4*>(wb[u] + (size_t)st * 1024 + wo[u] + ((q >> 1) * 8 + (q & 1)) * 64);
 #pragma unroll
-      for (int h = 0; h < 2; h++) d.s[u][h] = *reinterpret_cast<const uint4*>(sb[u] + (size_t)st * 64 + h * 8);
+      for (int h = 0; h < 2; h++) d.s[u][h] = *reinterpret_cast<const uint4*>(sb[u] + (size_t)st * 128 + so[u] + h * 16);
+    }
+  };
+  // The compiler does not see the DMAs and would wait for them together with the weights' registers at their first use, behind the NEXT
+  // requests: the registers pass an empty asm behind the step's own wait, where everything has landed.
+  auto settle = [&](WStep& d) {
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        asm volatile("" : "+v"(d.w[u][q].x), "+v"(d.w[u][q].y), "+v"(d.w[u][q].z), "+v"(d.w[u][q].w));
+        d.w[u][q].x ^= 0x88888888u; d.w[u][q].y ^= 0x88888888u; d.w[u][q].z ^= 0x88888888u; d.w[u][q].w ^= 0x88888888u;   // raw_widen's q'
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++) asm volatile("" : "+v"(d.s[u][h].x), "+v"(d.s[u][h].y), "+v"(d.s[u][h].z), "+v"(d.s[u][h].w));
     }
   };
 
-  // ---- staging: thread -> 4 x (token, 16-byte piece) of the step's 64 x 512 activation bytes + (256 threads) one float4 of group
-  // scales.  The requests go out BEFORE the step's MFMAs, the LDS writes after them (20 registers across the step buy the overlap:
-  // with one workgroup per CU nobody else keeps the memory pipe busy while this one computes).
-  struct XStage { uint4 x0, x1, x2, x3; float4 a; };
-  auto load_x = [&](XStage& xg, int st) {
-    uint4 xr[4];
+  // ---- staging: a wavefront brings 16 rows (one DMA instruction: two rows of 512 B; LDS slot s of row r holds the row's 16-byte piece with
+  // its low 4 bits ^ (r & 15)) and the scales of 2 groups (lane = row)
+  const uint32_t lds_x = (uint32_t)(uintptr_t)xs, lds_a = (uint32_t)(uintptr_t)as_l;
+  auto stage = [&](int hs, int buf) {
+    const uint32_t aoff = (uint32_t)s_src[lane] * (uint32_t)G * 4u;   // (rows x groups x 4 B < 4 GiB: checked by the launcher)
+    if (wave < mt_live) {
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-      const int idx = it * 512 + tid, tok = idx >> 5, piece = idx & 31;
-      const int src = s_src[tok];      // unconditional loads from a clamped row (a branch per load serialises the requests)
-      xr[it] = *reinterpret_cast<const uint4*>(p.act_q + (size_t)(src >= 0 ? src : 0) * p.K + (size_t)st * 512 + piece * 16);
+      for (int c = 0; c < 8; c++) {
+        const int row = wave * 16 + c * 2 + (lane >> 5), slot = lane & 31;
+        const int8_t* src = p.act_q + (size_t)s_src[row] * (size_t)(p.K * 2) + (size_t)hs * 512 + ((slot & 16) | ((slot ^ row) & 15)) * 16;
+        moe_dma(src, lds_x + buf * XB + (wave * 16 + c * 2) * 512);
+      }
     }
-    const int tok4 = (tid & 255) >> 2, src4 = s_src[tok4];
-    const float4 av = *reinterpret_cast<const float4*>(p.act_d + (size_t)(src4 >= 0 ? src4 : 0) * G + (size_t)st * 16 + (tid & 3) * 4);
-    const float keep = src4 >= 0 ? 1.0f : 0.0f;              // rows past the tile: scale 0 (their int8 values are then irrelevant)
-    xg.x0 = xr[0]; xg.x1 = xr[1]; xg.x2 = xr[2]; xg.x3 = xr[3];
-    xg.a = make_float4(av.x * keep, av.y * keep, av.z * keep, av.w * keep);
-  };
-  auto store_x = [&](const XStage& xg, int buf) {
-    const uint4 xr[4] = {xg.x0, xg.x1, xg.x2, xg.x3};
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-      const int idx = it * 512 + tid, tok = idx >> 5, piece = idx & 31;
-      *reinterpret_cast<uint4*>(xs + buf * XB + piece * CS + tok * 16) = xr[it];
-    }
-    if (tid < 256) {
-      float* ab = as_l + buf * (AB / 4) + ((tid & 3) * 4) * TOK + (tid >> 2);
-      ab[0] = xg.a.x; ab[TOK] = xg.a.y; ab[2 * TOK] = xg.a.z; ab[3 * TOK] = xg.a.w;
+    for (int c = 0; c < 2; c++) {
+      const int g = wave * 2 + c;
+      gg_dma4(p.act_d + (size_t)hs * 8 + g, aoff, lds_a + buf * AB + g * (TOK * 4));
     }
   };
 
@@ -2005,111 +2038,112 @@ __global__ __launch_bounds__(512) void moe_rawint4_chunk_kernel(RawGemmParams p)
 #pragma unroll
       for (int r = 0; r < 4; r++) acc[u][t][r] = 0.0f;
 
-  // One step = 4 dword positions p4 of the lane's pieces x 2 nibble halves (kb8 = 2 p4 + par) x 2 group halves h = 16 groups.
-  // Two things the compiler does to this loop when left alone, both measured (profiles/r04_j_*): (1) fully unrolled, it unpacks a
-  // whole step's operands up front and spills 460 registers — every group's operand words therefore pass an empty volatile asm
-  // right before their use, which pins the unpack behind the previous group; (2) it SLP-packs the four scale products and fmas of
-  // a fragment into v_pk_mul_f32 / v_pk_fma_f32 plus ~6 register-pair moves per MFMA — slower than the scalar forms beside MFMAs
-  // (MI355X_MICROARCH.md, per-instruction constants) — so the two operations are spelled as single instructions.
-  auto mul1 = [](float a, float b) { float d; asm("v_mul_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b)); return d; };
-  auto fma1 = [](float a, float b, float c) { float d; asm("v_fma_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c)); return d; };
+  const uint32_t xo0 = i * 512 + ((kc ^ i) * 16);   // row i's piece kc; piece 4 c + kc: ^ 64 c
+  // constants the compiler cannot see through: and + or become one v_and_or_b32
+  uint32_t mask, top;
+  asm("s_mov_b32 %0, 0x03C003C0" : "=s"(mask));
+  asm("v_mov_b32 %0, 0x4C004C00" : "=v"(top));
+
   // MTL = 16-token groups of the tile that hold rows (a Kimi-K2 chunk of 2048 tokens leaves ~43 rows per expert: three groups,
-  // not four, for most tiles); one instantiation per count, chosen once per workgroup
-  auto compute_n = [&](auto mtl, const WStep& w, int buf) __attribute__((always_inline)) {
-    constexpr int MTL = decltype(mtl)::value;
+  // not four, for most tiles); one instantiation per count, chosen once per workgroup.  Groups are fenced from each other: left alone, the compiler
+  // widens a whole step's weights up front and spills them.
+  auto compute_n = [&](auto mtl, auto hc, const WStep& w, int buf) __attribute__((always_inline)) {
+    constexpr int MTL = decltype(mtl)::value, HALF = decltype(hc)::value;
     if (!wave_ok) return;
-    const uint8_t* xb = xs + buf * XB + (kc >> 1) * CS + i * 16 + (kc & 1) * 8;
+    const uint8_t* xb = xs + buf * XB;
     const float* ab = as_l + buf * (AB / 4) + kc * 4;
-    // PMC of the first version (profiles/r04_j_rawint4_chunk_pmc.txt): 48 % of the wave cycles parked on s_waitcnt (every group
-    // read its activation fragments and scales from LDS and waited for them), 24 % in issue stalls (a fragment converted right
-    // behind its MFMA).  So: the fragments of group g + 1 are requested before the MFMAs of group g, and a group's eight MFMAs are
-    // issued back to back before the first result is touched.
-    struct Frag { long a[MTL]; float4 s[MTL]; };
-    auto load_frag = [&](Frag& f, int g) __attribute__((always_inline)) {      // g = kb8 * 2 + h: column 2 g, scale row g
+    raw_h8 af[MTL];
+    float4 sf[2][MTL];
+    auto load_a = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
-      for (int t = 0; t < MTL; t++) {
-        f.a[t] = *reinterpret_cast<const long*>(xb + (size_t)(2 * g) * CS + t * 256);
-        f.s[t] = *reinterpret_cast<const float4*>(ab + g * TOK + t * 16);
-      }
+      for (int t = 0; t < MTL; t++) af[t] = *reinterpret_cast<const raw_h8*>(xb + (xo0 ^ ((g & 3) * 64)) + (g >> 2) * 256 + t * 8192);
     };
-    Frag fr[2];
-    load_frag(fr[0], 0);
+    auto load_s = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
-    for (int g = 0; g < 16; g++) {
-      const int kb8 = g >> 1, h = g & 1;
-      const Frag& cur = fr[g & 1];
-      long bop[NU];
-      float bs[NU];
+      for (int t = 0; t < MTL; t++) sf[g & 1][t] = *reinterpret_cast<const float4*>(ab + g * TOK + t * 16);
+    };
+    auto widen = [&](raw_h8 (&bop)[NU], auto gc) __attribute__((always_inline)) {
+      constexpr int g = decltype(gc)::value, kb8 = HALF * 4 + (g >> 1), h = g & 1;   // g = (kb8 of the half) * 2 + h
 #pragma unroll
       for (int u = 0; u < NU; u++) {
         const uint4 &w0 = w.w[u][h * 2], &w1 = w.w[u][h * 2 + 1], &sv = w.s[u][h];
-        uint32_t P0 = kb8 < 2 ? w0.x : kb8 < 4 ? w0.y : kb8 < 6 ? w0.z : w0.w;
-        uint32_t P1 = kb8 < 2 ? w1.x : kb8 < 4 ? w1.y : kb8 < 6 ? w1.z : w1.w;
+        const uint32_t P0 = kb8 < 2 ? w0.x : kb8 < 4 ? w0.y : kb8 < 6 ? w0.z : w0.w;
+        const uint32_t P1 = kb8 < 2 ? w1.x : kb8 < 4 ? w1.y : kb8 < 6 ? w1.z : w1.w;
         const uint32_t S = kb8 < 2 ? sv.x : kb8 < 4 ? sv.y : kb8 < 6 ? sv.z : sv.w;
-        asm volatile("" : "+v"(P0), "+v"(P1));
-        const uint32_t b0 = (kb8 & 1) ? (P0 & 0xF0F0F0F0u) : ((P0 << 4) & 0xF0F0F0F0u);
-        const uint32_t b1 = (kb8 & 1) ? (P1 & 0xF0F0F0F0u) : ((P1 << 4) & 0xF0F0F0F0u);
-        bop[u] = (long)(((unsigned long long)b1 << 32) | b0);
-        bs[u] = __uint_as_float((kb8 & 1) ? (S & 0xffff0000u) : (S << 16));
+        const _Float16 bh = (_Float16)__uint_as_float((kb8 & 1) ? (S & 0xffff0000u) : (S << 16));
+        const raw_h2 bs = {bh, bh}, m24 = bs * raw_h2{(_Float16)-24.0f, (_Float16)-24.0f};
+        uint32_t o[4];
+        raw_widen<(kb8 & 1)>(P0, mask, top, bs, m24, o[0], o[1]);
+        raw_widen<(kb8 & 1)>(P1, mask, top, bs, m24, o[2], o[3]);
+        bop[u] = __builtin_bit_cast(raw_h8, make_uint4(o[0], o[1], o[2], o[3]));
       }
-      if (g + 1 < 16) load_frag(fr[(g + 1) & 1], g + 1);
+    };
+    // a group's MFMAs, the next group's operands behind them, then the group's sums
+    raw_h8 bop[2][NU];
+    load_a(0);
+    load_s(0);
+    widen(bop[0], std::integral_constant<int, 0>{});
+    static_for<8>([&](auto gc) __attribute__((always_inline)) {
+      constexpr int g = decltype(gc)::value;
+      constexpr int TB = MTL < 2 ? MTL : 2;   // (the sums of all fragments at once do not fit the registers)
 #pragma unroll
-      for (int t0 = 0; t0 < MTL; t0 += 2) {          // four MFMAs in flight (two token groups x two operands), then their 16 results
-        v4i d[2][NU];
+      for (int t0 = 0; t0 < MTL; t0 += TB) {
+        v4f d[TB][NU];
 #pragma unroll
-        for (int tt = 0; tt < 2; tt++)
+        for (int t = 0; t < TB && t0 + t < MTL; t++)
 #pragma unroll
-          for (int u = 0; u < NU; u++)
-            if (t0 + tt < MTL) d[tt][u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(cur.a[t0 + tt], bop[u], v4i{0, 0, 0, 0}, 0, 0, 0);
-        // products, conversions, then the fmas: a dependent pair of VALU instructions back to back stalls the issue (the first
-        // version's `mul -> fma` / `cvt -> fma` chains showed as 30 % SQ_WAIT_INST_ANY)
-#pragma unroll
-        for (int tt = 0; tt < 2; tt++) {
-          if (t0 + tt >= MTL) continue;
-          const int t = t0 + tt;
-          const float asv[4] = {cur.s[t].x, cur.s[t].y, cur.s[t].z, cur.s[t].w};
-          float pm[NU][4], cf[NU][4];
-#pragma unroll
-          for (int u = 0; u < NU; u++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) pm[u][r] = mul1(asv[r], bs[u]);
-#pragma unroll
-          for (int u = 0; u < NU; u++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) cf[u][r] = (float)d[tt][u][r];
-#pragma unroll
-          for (int u = 0; u < NU; u++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[u][t][r] = fma1(pm[u][r], cf[u][r], acc[u][t][r]);
+          for (int u = 0; u < NU; u++) d[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t0 + t], bop[g & 1][u], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        if constexpr (g + 1 < 8) {
+          if (t0 + TB >= MTL) { load_a(g + 1); load_s(g + 1); }
+          if (t0 == 0) widen(bop[(g + 1) & 1], std::integral_constant<int, (g + 1) & 7>{});
         }
+#pragma unroll
+        for (int t = 0; t < TB && t0 + t < MTL; t++) {
+          const float4 sv = sf[g & 1][t0 + t];
+          const float asv[4] = {sv.x, sv.y, sv.z, sv.w};
+#pragma unroll
+          for (int u = 0; u < NU; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[u][t0 + t][r] = fmaf(asv[r], d[t][u][r], acc[u][t0 + t][r]);
+        }
+        if constexpr (TB < MTL) __builtin_amdgcn_sched_barrier(0);
       }
-    }
+      __builtin_amdgcn_sched_barrier(0);
+    });
   };
-  const int mt_live = (tile.nrows + 15) >> 4;
-  auto compute = [&](const WStep& w, int buf) __attribute__((always_inline)) {
-    if (mt_live >= 4) compute_n(std::integral_constant<int, 4>{}, w, buf);
-    else if (mt_live == 3) compute_n(std::integral_constant<int, 3>{}, w, buf);
-    else if (mt_live == 2) compute_n(std::integral_constant<int, 2>{}, w, buf);
-    else compute_n(std::integral_constant<int, 1>{}, w, buf);
+  auto compute = [&](auto hc, const WStep& w, int buf) __attribute__((always_inline)) {
+    if (mt_live >= 4) compute_n(std::integral_constant<int, 4>{}, hc, w, buf);
+    else if (mt_live == 3) compute_n(std::integral_constant<int, 3>{}, hc, w, buf);
+    else if (mt_live == 2) compute_n(std::integral_constant<int, 2>{}, hc, w, buf);
+    else compute_n(std::integral_constant<int, 1>{}, hc, w, buf);
+  };
+  using H0 = std::integral_constant<int, 0>;
+  using H1 = std::integral_constant<int, 1>;
+  // one step: the second half's activations are requested before the first half's MFMAs, the next step's weights behind them (they have the
+  // whole step to arrive), the next step's first half before the second half's MFMAs
+  // (unconditional, the last step's requests repeat: the compiler cannot pair a load and a settle under two branches, and waits)
+  auto step = [&](WStep& w, WStep& next, int st) __attribute__((always_inline)) {
+    stage(2 * st + 1, 1);
+    load_w(next, min(st + 1, NS - 1));
+    compute(H0{}, w, 0);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(WLOADS) : "memory");   // the DMAs; the weights' loads are younger
+    __syncthreads();
+    stage(min(2 * st + 2, 2 * NS - 1), 0);
+    compute(H1{}, w, 1);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    settle(next);
+    __syncthreads();
   };
 
   WStep wa, wb2;
-  XStage xg;
   load_w(wa, 0);
-  load_x(xg, 0);
-  store_x(xg, 0);
+  stage(0, 0);
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  settle(wa);
   __syncthreads();
   for (int st = 0; st < NS; st += 2) {
-    if (st + 1 < NS) { load_w(wb2, st + 1); load_x(xg, st + 1); }
-    compute(wa, 0);
-    if (st + 1 < NS) store_x(xg, 1);     // buffer 1 was last read in step st - 1: every wavefront is past that step's barrier
-    __syncthreads();
-    if (st + 1 < NS) {
-      if (st + 2 < NS) { load_w(wa, st + 2); load_x(xg, st + 2); }
-      compute(wb2, 1);
-      if (st + 2 < NS) store_x(xg, 0);
-      __syncthreads();
-    }
+    step(wa, wb2, st);
+    if (st + 1 < NS) step(wb2, wa, st + 1);
   }
 
   if (!wave_ok) return;
@@ -2121,7 +2155,7 @@ __global__ __launch_bounds__(512) void moe_rawint4_chunk_kernel(RawGemmParams p)
       for (int r = 0; r < 4; r++) {
         const int row = t * 16 + kc * 4 + r;
         if (row < tile.nrows) {
-          const bf16_t gv = f32_to_bf16(acc[0][t][r] / 16.0f), uv = f32_to_bf16(acc[1][t][r] / 16.0f);
+          const bf16_t gv = f32_to_bf16(acc[0][t][r]), uv = f32_to_bf16(acc[1][t][r]);
           p.out[(size_t)(tile.row0 + row) * p.N + n] = f32_to_bf16(act_fn(bf16_to_f32(gv), bf16_to_f32(uv)));
         }
       }
@@ -2135,14 +2169,14 @@ __global__ __launch_bounds__(512) void moe_rawint4_chunk_kernel(RawGemmParams p)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
           const int row = t * 16 + kc * 4 + r;
-          if (row < tile.nrows) p.out[(size_t)(tile.row0 + row) * p.N + n] = f32_to_bf16(acc[u][t][r] / 16.0f);
+          if (row < tile.nrows) p.out[(size_t)(tile.row0 + row) * p.N + n] = f32_to_bf16(acc[u][t][r]);
         }
     }
   }
 }
 
-// per-(row, 32-group) int8 quantisation (BufferASmallKGroupImpl::from_mat, amx_buffers.hpp:431-495): one block per row,
-// 8 elements per thread, a group = 4 adjacent lanes
+// HALF: the codes as f16 integers, 8 k in the order (0,2) (1,3) (4,6) (5,7) of moe_rawint4_chunk_kernel's weights
+template <bool HALF>
 __device__ __forceinline__ void quant_row_kgroup_block(const bf16_t* __restrict__ src, int K, int8_t* __restrict__ dst,
                                                        float* __restrict__ d_out) {
   for (int c = threadIdx.x * 8; c < K; c += blockDim.x * 8) {
@@ -2152,11 +2186,21 @@ __device__ __forceinline__ void quant_row_kgroup_block(const bf16_t* __restrict_
     amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
     const float d = amax / 127.0f;
     const float id = d ? 1.0f / d : 0.0f;
-    *reinterpret_cast<uint2*>(dst + c) = quant8(v, id);
+    const uint2 q = quant8(v, id);
+    if constexpr (HALF) {
+      auto pair = [](uint32_t w, int lo, int hi) {
+        const raw_h2 h = {(_Float16)(float)(int8_t)(w >> (8 * lo)), (_Float16)(float)(int8_t)(w >> (8 * hi))};
+        return raw_h2_bits(h);
+      };
+      *reinterpret_cast<uint4*>(dst + 2 * (size_t)c) = make_uint4(pair(q.x, 0, 2), pair(q.x, 1, 3), pair(q.y, 0, 2), pair(q.y, 1, 3));
+    } else {
+      *reinterpret_cast<uint2*>(dst + c) = q;
+    }
     if ((threadIdx.x & 3) == 0) d_out[c >> 5] = d;
   }
 }
 
+template <bool HALF>
 __global__ __launch_bounds__(256) void moe_actquant_kgroup_kernel(const bf16_t* __restrict__ a, int K,
                                                                   int8_t* __restrict__ a_q, float* __restrict__ a_d,
                                                                   const int32_t* counters, const int32_t* d_bsz, int qlen,
@@ -2169,7 +2213,7 @@ __global__ __launch_bounds__(256) void moe_actquant_kgroup_kernel(const bf16_t* 
   } else if (row >= counters[1]) {
     return;
   }
-  quant_row_kgroup_block(a + (size_t)row * K, K, a_q + (size_t)row * K, a_d + (size_t)row * (K / 32));
+  quant_row_kgroup_block<HALF>(a + (size_t)row * K, K, a_q + (size_t)row * K * (HALF ? 2 : 1), a_d + (size_t)row * (K / 32));
 }
 
 // =====================================================================================================
@@ -2443,6 +2487,16 @@ __global__ void pack_rawint4_kernel(const uint8_t* __restrict__ src, int N, int 
   out[idx] = v;
 }
 
+// *out |= 1 when a scale is neither zero nor of magnitude 2^-17 .. 2^11
+__global__ __launch_bounds__(256) void raw_scale_range_kernel(const bf16_t* __restrict__ s, size_t n, int* out) {
+  bool bad = false;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    const float a = fabsf(bf16_to_f32(s[i]));
+    bad |= !(a == 0.0f || (a >= 0x1p-17f && a <= 0x1p11f));
+  }
+  if (bad) atomicOr(out, 1);
+}
+
 // bf16 scales [N][K/32] -> tile order [rg][step][row j][h][8 blocks]; one thread per element
 __global__ void pack_rawint4_scales_kernel(const bf16_t* __restrict__ src, int N, int K, bf16_t* __restrict__ out) {
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2519,6 +2573,7 @@ struct ktx_moe_s {
   int gg_type[3] = {0, 0, 0};     // GGUF: ggml type of gate / up / down
   size_t gg_stride[3] = {0, 0, 0};
   bool loaded_gguf = false;
+  bool raw_f16 = false;           // RAWINT4: every scale times 24 and times a nibble is exact in f16 (moe_rawint4_chunk_kernel)
   bool exact = false;             // ktx_moe_set_exact: no path of this handle may re-associate the reference's fp32 sums
 };
 
@@ -2581,11 +2636,11 @@ extern "C" int ktx_moe_create(const ktx_moe_config* cfg, ktx_moe_t* out) {
     KTX_REQUIRE(cfg->device >= 0 && cfg->device < 64, "ktx_moe_create: device ordinal out of range");
     const bool raw = cfg->format == KTX_FMT_RAWINT4;
     size_t need[12] = {0};
-    need[0] = (size_t)cfg->max_len * H;
+    need[0] = (size_t)cfg->max_len * H * (raw ? 2 : 1);   // (RAWINT4 prompts: the codes as f16)
     need[1] = (size_t)cfg->max_len * sizeof(float) * (raw || gguf ? H / 32 : 1);   // (GGUF: Q8_K has a scale per 256, Q8_0 per 32)
     // int formats: the grouped gate/up GEMM stores g | u (2*I bf16 per row); GGUF: fp32 intermediates
     need[2] = (size_t)h->max_pairs * I * (gguf ? sizeof(float) : 2 * sizeof(bf16_t));
-    need[3] = (size_t)h->max_pairs * I;
+    need[3] = (size_t)h->max_pairs * I * (raw ? 2 : 1);
     need[4] = (size_t)h->max_pairs * sizeof(float) * (raw || gguf ? I / 32 : 1);
     need[5] = (size_t)h->max_pairs * H * (gguf ? sizeof(float) : sizeof(bf16_t));
     need[6] = need[7] = (size_t)h->max_pairs * sizeof(int32_t);
@@ -2834,6 +2889,15 @@ extern "C" int ktx_moe_load_rawint4(ktx_moe_t h, const void* d_gate, const void*
   KTX_ON_DEVICE(h->cfg.device);
   const int E = h->cfg.expert_num, H = h->cfg.hidden_size, I = h->cfg.intermediate_size;
   const size_t dwords = (size_t)I * H / 8, nsc = (size_t)I * (H / 32);
+  int* range = nullptr;
+  int out_of_range = 0;
+  KTX_HIP(hipMalloc(&range, sizeof(int)));
+  KTX_HIP(hipMemcpy(range, &out_of_range, sizeof(int), hipMemcpyHostToDevice));
+  for (const void* sc : {d_gate_scale, d_up_scale, d_down_scale})
+    hipLaunchKernelGGL(raw_scale_range_kernel, dim3(1024), dim3(256), 0, 0, (const bf16_t*)sc, (size_t)E * nsc, range);
+  KTX_HIP(hipMemcpy(&out_of_range, range, sizeof(int), hipMemcpyDeviceToHost));
+  KTX_HIP(hipFree(range));
+  h->raw_f16 = out_of_range == 0;
   for (int e = 0; e < E; e++) {
     const uint8_t* src[3] = {(const uint8_t*)d_gate + (size_t)e * I * H / 2, (const uint8_t*)d_up + (size_t)e * I * H / 2,
                              (const uint8_t*)d_down + (size_t)e * H * I / 2};
@@ -3345,24 +3409,29 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
 }
 
 
-template <int NT, bool GATE_UP>
+template <bool GATE_UP>
 static int launch_rawint4(const RawGemmParams& p, int max_tiles, hipStream_t st) {
   const size_t lds = 4 * (size_t)(p.K + 32) + (size_t)(p.K / 32) * 16;
-  const hipError_t err = ktx_set_max_lds(reinterpret_cast<const void*>(moe_rawint4_gemm_kernel<NT, GATE_UP>), 96 * 1024);
-  KTX_HIP(err);
   KTX_REQUIRE(lds <= 96 * 1024, "ktx_moe_forward: K too large for the RAWINT4 kernel");
-  hipLaunchKernelGGL((moe_rawint4_gemm_kernel<NT, GATE_UP>), dim3((p.N / 16 + 3) / 4, max_tiles), dim3(256), lds, st, p);
-  KTX_HIP(hipGetLastError());
-  return 0;
+  const dim3 grid((p.N / 16 + 3) / 4, max_tiles);
+  const int total = p.K / 512 * (GATE_UP ? 2 : 1);   // (step, matrix) pairs: the ring's depth divides them
+  auto go = [&](auto kern) {
+    KTX_HIP(ktx_set_max_lds(reinterpret_cast<const void*>(kern), 96 * 1024));
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p);
+    KTX_HIP(hipGetLastError());
+    return 0;
+  };
+  if constexpr (GATE_UP) return go(moe_rawint4_rows_kernel<2, GATE_UP>);
+  else return go(moe_rawint4_rows_kernel<1, GATE_UP>);
 }
 
 template <bool GATE_UP>
 static int launch_rawint4_chunk(const RawGemmParams& p, int max_tiles, hipStream_t st) {
-  constexpr size_t lds = 2 * (32 * (64 * 16 + 16) + 16 * 64 * 4);
+  constexpr size_t lds = 2 * (64 * 512 + 8 * 64 * 4);
   const hipError_t err = ktx_set_max_lds(reinterpret_cast<const void*>(moe_rawint4_chunk_kernel<GATE_UP>), (int)lds);
   KTX_HIP(err);
-  const int per_wg = GATE_UP ? 8 : 16;      // strips per workgroup of 8 wavefronts (down: two strips per wavefront)
-  hipLaunchKernelGGL((moe_rawint4_chunk_kernel<GATE_UP>), dim3((p.N / 16 + per_wg - 1) / per_wg, max_tiles), dim3(512), lds, st, p);
+  const int per_wg = GATE_UP ? 4 : 8;       // strips per workgroup of 4 wavefronts (down: two strips per wavefront)
+  hipLaunchKernelGGL((moe_rawint4_chunk_kernel<GATE_UP>), dim3((p.N / 16 + per_wg - 1) / per_wg, max_tiles), dim3(256), lds, st, p);
   KTX_HIP(hipGetLastError());
   return 0;
 }
@@ -3412,7 +3481,7 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
 
   // prompt chunks: 64-row tiles through the group-scaled 16x16x32 kernel (moe_rawint4_chunk_kernel: same terms, one fp32 chain per
   // output instead of the reference's sixteen); short batches and dev knob 29 = 1 keep the exact 4-row kernel
-  const bool chunk = qlen >= 64 && g_dbg[29] != 1 && !h->exact && H % 512 == 0 && I % 512 == 0;
+  const bool chunk = qlen >= 64 && g_dbg[29] != 1 && !h->exact && h->raw_f16 && (size_t)npairs * (std::max(H, I) / 32) * 4 < ((size_t)1 << 32);
   PrepParams pp;
   pp.d_bsz = d_bsz; pp.qlen = qlen; pp.k = k; pp.E = E; pp.expert_begin = h->cfg.expert_begin; pp.H = H;
   pp.rows_per_tile = chunk ? 64 : 4; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
@@ -3421,8 +3490,8 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   {
     ProfScope ps(0, st);
     KTX_HIP(launch_moe_prep(pp, 1, st));
-    hipLaunchKernelGGL(moe_actquant_kgroup_kernel, dim3(qlen), dim3(256), 0, st, (const bf16_t*)d_input, H, ws->x_q, ws->x_d,
-                       ws->counters, d_bsz, qlen, 1);
+    hipLaunchKernelGGL(chunk ? moe_actquant_kgroup_kernel<true> : moe_actquant_kgroup_kernel<false>, dim3(qlen), dim3(256), 0, st,
+                       (const bf16_t*)d_input, H, ws->x_q, ws->x_d, ws->counters, d_bsz, qlen, 1);
   }
   KTX_HIP(hipGetLastError());
   RawGemmParams g1;
@@ -3432,14 +3501,13 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   int rc;
   {
     ProfScope ps(1, st);
-    rc = chunk ? launch_rawint4_chunk<true>(g1, std::min(npairs, E) + npairs / 64, st)
-               : qlen == 1 ? launch_rawint4<1, true>(g1, max_tiles, st) : launch_rawint4<4, true>(g1, max_tiles, st);
+    rc = chunk ? launch_rawint4_chunk<true>(g1, std::min(npairs, E) + npairs / 64, st) : launch_rawint4<true>(g1, max_tiles, st);
   }
   if (rc) return rc;
   {
     ProfScope ps(2, st);
-    hipLaunchKernelGGL(moe_actquant_kgroup_kernel, dim3(npairs), dim3(256), 0, st, ws->a_buf, I, ws->a_q, ws->a_d, ws->counters,
-                       d_bsz, qlen, 0);
+    hipLaunchKernelGGL(chunk ? moe_actquant_kgroup_kernel<true> : moe_actquant_kgroup_kernel<false>, dim3(npairs), dim3(256), 0, st,
+                       ws->a_buf, I, ws->a_q, ws->a_d, ws->counters, d_bsz, qlen, 0);
   }
   KTX_HIP(hipGetLastError());
   RawGemmParams g2;
@@ -3448,8 +3516,7 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   g2.tiles = ws->tiles; g2.counters = ws->counters; g2.out = ws->dn_buf;
   {
     ProfScope ps(3, st);
-    rc = chunk ? launch_rawint4_chunk<false>(g2, std::min(npairs, E) + npairs / 64, st)
-               : qlen == 1 ? launch_rawint4<1, false>(g2, max_tiles, st) : launch_rawint4<4, false>(g2, max_tiles, st);
+    rc = chunk ? launch_rawint4_chunk<false>(g2, std::min(npairs, E) + npairs / 64, st) : launch_rawint4<false>(g2, max_tiles, st);
   }
   if (rc) return rc;
   CombineParams cp{};
@@ -3722,7 +3789,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   GgGemmParams g1{};
   g1.w0 = h->gate_w; g1.w1 = h->up_w; g1.stride0 = h->gg_stride[0]; g1.stride1 = h->gg_stride[1]; g1.N = I; g1.K = H;
   g1.act_q = ws->x_q; g1.act_d = ws->x_d; g1.act_bs = ws->x_bs; g1.act_bsp = x_bsp; g1.act_b256 = x_b256; g1.row_src = ws->src_of_row; g1.tiles = ws->tiles;
-  g1.counters = ws->counters; g1.out = reinterpret_cast<float*>(ws->a_buf); g1.dbg = g_dbg[24];
+  g1.counters = ws->counters; g1.out = reinterpret_cast<float*>(ws->a_buf);
   int rc;
   {
     ProfScope ps(1, st);
@@ -3738,7 +3805,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   GgGemmParams g2{};
   g2.w0 = h->down_w; g2.w1 = nullptr; g2.stride0 = h->gg_stride[2]; g2.stride1 = 0; g2.N = H; g2.K = I;
   g2.act_q = ws->a_q; g2.act_d = ws->a_d; g2.act_bs = ws->a_bs; g2.act_bsp = a_bsp; g2.act_b256 = a_b256; g2.row_src = nullptr; g2.tiles = ws->tiles;
-  g2.counters = ws->counters; g2.out = reinterpret_cast<float*>(ws->dn_buf); g2.dbg = g_dbg[24];
+  g2.counters = ws->counters; g2.out = reinterpret_cast<float*>(ws->dn_buf);
   {
     ProfScope ps(3, st);
     rc = launch_gguf_type<false>(h->gg_type[2], mt, g2, max_tiles, st);
