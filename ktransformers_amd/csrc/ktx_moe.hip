@@ -54,7 +54,8 @@ struct Tile {
   int expert;  // local expert index
   int row0;    // first sorted row
   int nrows;   // <= 16*MT
-  int pad;
+  int idx;     // place among its expert's tiles
+  int cnt;     // the expert's tiles
 };
 
 // =====================================================================================================
@@ -267,7 +268,8 @@ __global__ __launch_bounds__(1024) void moe_prep_kernel(PrepParams p) {
     const int c = s_cnt[e];
     for (int i = 0, r = 0; r < c; i++, r += p.rows_per_tile) {
       Tile t;
-      t.expert = e; t.row0 = s_off[e] + r; t.nrows = min(p.rows_per_tile, c - r); t.pad = 0;
+      t.expert = e; t.row0 = s_off[e] + r; t.nrows = min(p.rows_per_tile, c - r); t.idx = i;
+      t.cnt = (c + p.rows_per_tile - 1) / p.rows_per_tile;
       p.tiles[s_toff[e] + i] = t;
     }
   }
@@ -2647,9 +2649,9 @@ extern "C" int ktx_moe_create(const ktx_moe_config* cfg, ktx_moe_t* out) {
     need[8] = (size_t)h->max_tiles * sizeof(Tile);
     need[9] = (4 + KTX_DEC_MAX_PAIRS * 64) * sizeof(int32_t);   // [4] bucket counters | arrival tickets of the GGUF decode launches
     if (gguf) {
-      // Q8_K 16-sums, and behind them the 32-sums split into two int8 planes (16 B per 256-block: the folded Q4_K kernel's min operand)
-      need[10] = (size_t)cfg->max_len * (H / 16) * sizeof(int16_t) + (size_t)cfg->max_len * (H / 256) * (16 + 4);   // (+ the block sums)
-      need[11] = (size_t)h->max_pairs * (I / 16) * sizeof(int16_t) + (size_t)h->max_pairs * (I / 256) * (16 + 4);
+      // Q8_K 16-sums, and behind them the 32-sums split into two f16 planes (32 B per 256-block: the folded Q4_K kernel's min operand)
+      need[10] = (size_t)cfg->max_len * (H / 16) * sizeof(int16_t) + (size_t)cfg->max_len * (H / 256) * (32 + 4);   // (+ the block sums)
+      need[11] = (size_t)h->max_pairs * (I / 16) * sizeof(int16_t) + (size_t)h->max_pairs * (I / 256) * (32 + 4);
     }
     std::shared_ptr<Workspace> cur = g_ws[cfg->device];
     bool fits = cur != nullptr;
@@ -3592,7 +3594,7 @@ static int launch_gguf(const GgGemmParams& p, int max_tiles, hipStream_t st) {
   const dim3 grid_f((unsigned)((p.N / 16 + 3) / 4) * (unsigned)((max_tiles + 7) / 8 * 8));   // folded kernels: (XCD, tile, strip group) in one dimension
   if constexpr (gg_foldable(WT)) {   // round 6: the folded-operand kernel; dev knob [21] = 1: gg_block's (the bit-identity test, A/B timing)
     if (g_dbg[21] != 1) {
-      const size_t lds_f = 2 * TOK * 256 + 2 * TOK * 4 + TOK * 4 + (WT == GG_Q4K ? 2 * TOK * 16 : WT == GG_IQ1S ? 2 * TOK * 4 + 16384 : 0);
+      const size_t lds_f = 2 * TOK * 256 + 2 * TOK * 4 + TOK * 4 + (WT == GG_Q4K ? 2 * TOK * 32 : WT == GG_IQ1S ? 2 * TOK * 4 + 16384 : 0);
       auto kern = moe_gguf_fold_kernel<WT, MT, GATE_UP>;
       if (lds_f > 64 * 1024) KTX_HIP(ktx_set_max_lds(reinterpret_cast<const void*>(kern), (int)lds_f));
       hipLaunchKernelGGL(kern, grid_f, dim3(256), lds_f, st, p);
@@ -3680,13 +3682,17 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
     return 0;
   }
   int mt = std::min(4, pick_mt(qlen, k, E));
-  // round 6: 128-row tiles for the folded Q4_K / Q6_K kernels once an expert sees ~100 rows — the operand folding of a 256-block is
-  // paid once per tile and strip, so twice the rows halve its share (dev knob [22]: 1 = 64-row tiles always, 2 = 128-row tiles always)
-  if (gg_foldable(h->gg_type[0]) && gg_foldable(h->gg_type[2]) && h->gg_type[0] != GG_IQ1S && h->gg_type[2] != GG_IQ1S &&   // (IQ1_S: its 16 KiB
-      // grid table beside two 32 KiB stages leaves ONE workgroup per CU — measured 1.6x slower than 64-row tiles)
-      g_dbg[21] != 1 && g_dbg[22] != 1 &&
-      (g_dbg[22] == 2 || (double)npairs / std::max(1, E) >= 96.0))
-    mt = 8;
+  // (IQ1_S keeps to pick_mt: its 16 KiB grid table beside two 32 KiB stages leaves ONE workgroup per CU — measured 1.6x slower)
+  if (gg_foldable(h->gg_type[0]) && gg_foldable(h->gg_type[2]) && h->gg_type[0] != GG_IQ1S && h->gg_type[2] != GG_IQ1S && g_dbg[21] != 1) {
+    // Rows per tile: a tile's weights are read and folded once, so low tiles cost passes over the weights and high ones work on absent
+    // rows.  Measured (Q4_K, 16 | 32 | 64-row tiles, us): 64 experts of 2048 x 1536 with 2.3 rows each 83 | 89 | 95, 4.5: 103 | 109 | 118,
+    // 9.4: 123 | 121 | 130, 19: 165 | 145 | 143; 8 experts of 4096 x 14336 with 12 rows 284 | 242 | 264, 25: 353 | 325 | 286, 50: 607 | 469 | 368.
+    // 128-row tiles halve the folding's share; below, few tiles fill the last wave worse (same 8 experts, 64 | 128 rows: 125 rows each
+    // 660 | 680, 175: 848 | 793, 200: 948 | 956, 325: 1400 | 1298, 512: 2114 | 1991).  Dev knob [22]: 1 = 64-row tiles, 2 = 128-row ones.
+    const double rows = (double)npairs / std::max(1, E);
+    mt = rows <= 6.0 ? 1 : rows <= 16.0 ? 2 : rows < 144.0 ? 4 : 8;
+    if (g_dbg[22]) mt = g_dbg[22] == 2 ? 8 : std::min(mt, 4);
+  }
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
 
   // ---- decode fast path: two launches (ktx_moe_gguf.inc, moe_dec_gguf_gateup_kernel) --------------------------------------
@@ -3773,8 +3779,8 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
 
   uint8_t* x_bsp = reinterpret_cast<uint8_t*>(ws->x_bs) + (size_t)h->cfg.max_len * (H / 16) * sizeof(int16_t);
   uint8_t* a_bsp = reinterpret_cast<uint8_t*>(ws->a_bs) + (size_t)h->max_pairs * (I / 16) * sizeof(int16_t);
-  int32_t* x_b256 = reinterpret_cast<int32_t*>(x_bsp + (size_t)h->cfg.max_len * (H / 256) * 16);
-  int32_t* a_b256 = reinterpret_cast<int32_t*>(a_bsp + (size_t)h->max_pairs * (I / 256) * 16);
+  int32_t* x_b256 = reinterpret_cast<int32_t*>(x_bsp + (size_t)h->cfg.max_len * (H / 256) * 32);
+  int32_t* a_b256 = reinterpret_cast<int32_t*>(a_bsp + (size_t)h->max_pairs * (I / 256) * 32);
   PrepParams pp;
   pp.d_bsz = d_bsz; pp.qlen = qlen; pp.k = k; pp.E = E; pp.expert_begin = h->cfg.expert_begin; pp.H = H;
   pp.rows_per_tile = 16 * mt; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;

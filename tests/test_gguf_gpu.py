@@ -192,6 +192,36 @@ def test_folded_prompt_kernels_give_the_unfolded_bits(types, T):
     assert np.abs(y_ref.view(np.uint16).astype(np.int32)).max() > 0
 
 
+@pytest.mark.parametrize("rows", [(1, 0, 0, 0), (0, 129, 0, 16), (65, 1, 0, 300), (128, 256, 33, 0), (17, 143, 81, 513)])
+@pytest.mark.parametrize("height", [0, 2])
+def test_folded_prompt_kernels_on_uneven_experts(rows, height):
+    """The folded kernels deal (tile, strip group) jobs to the 8 XCDs in expert order and leave a 128-row tile's absent 16-row pieces
+    out: experts without rows, of one row past a tile, of many tiles, at the heights the rule picks and at 128 rows (dev knob 22 = 2);
+    the bits are the unfolded kernel's."""
+    from ktransformers_amd import _native as n
+    E, H, I, T = len(rows), 512, 1280, sum(rows)
+    r0 = np.random.default_rng(T)
+    gate, up, down = random_kquant(Q4, E, I, H, r0), random_kquant(Q4, E, I, H, r0), random_kquant(Q6, E, H, I, r0)
+    x = torch.from_numpy(f32_to_bf16(r0.standard_normal((T, H)).astype(np.float32)).view(np.int16)).view(torch.bfloat16).cuda()
+    ids = torch.from_numpy(r0.permutation(np.repeat(np.arange(E), rows)).astype(np.int64)[:, None]).cuda()
+    w = torch.from_numpy(r0.random((T, 1)).astype(np.float32)).cuda()
+    h = n.MoEHandle(E, 1, H, I, max(T, 16), "GGUF", 0)
+    h.load_gguf(torch.from_numpy(gate).cuda(), torch.from_numpy(up).cuda(), torch.from_numpy(down).cuda(), Q4, Q4, Q6)
+    n.force_generic_path(True)
+    try:
+        n.lib.ktx_debug_set(22, height)
+        y_fold = h.forward(x, ids, w).view(torch.int16).cpu().numpy()
+        n.lib.ktx_debug_set(22, 0)
+        n.lib.ktx_debug_set(21, 1)
+        y_ref = h.forward(x, ids, w).view(torch.int16).cpu().numpy()
+    finally:
+        n.lib.ktx_debug_set(22, 0)
+        n.lib.ktx_debug_set(21, 0)
+        n.force_generic_path(False)
+    assert np.array_equal(y_fold, y_ref), f"{int((y_fold != y_ref).sum())} of {y_ref.size} outputs differ"
+    assert np.abs(y_ref.view(np.uint16).astype(np.int32)).max() > 0
+
+
 @pytest.mark.parametrize("T", [1, 4])
 def test_mixtral_8x7b_real_dims(T):
     """BASELINE.json configs[0] (Mixtral-8x7B q4_k_m, kt-kernel/bench/bench_moe.py:166-170): 8 experts, top-2, hidden 4096,
