@@ -3117,6 +3117,31 @@ extern "C" int ktx_moe_forward_side(ktx_moe_t h, const int32_t* d_bsz, int qlen,
   return ktx_linear_forward_fused(side_linear, d_bsz, qlen, d_side_x, d_output, &fu, stream);
 }
 
+// Of a batch that the decode launches could take: do so many of its (token, expert) pairs name an expert again that the grouped kernels, which
+// read an expert once, are faster?  The decode launches read one expert per pair.  pairs and distinct experts are expected values
+// of a uniform routing over the global experts, of which the handle owns expert_num; bytes: an expert's weights.  The grouped
+// path's three more launches and its fill cost 10-25 us, which the repeats' bytes have to outweigh.  Measured (decode | grouped, us, at
+// (pairs - 0.9 distinct) bytes): AMXINT4 82 MB 56 | 47 and 37 | 41, 91: 32 | 34, 120: 54 | 43 and 40 | 39, 235: 48 | 34, 518: 196 | 132;
+// FP8 153: 54 | 61, 239: 74 | 64, 251: 49 | 52, 323: 60 | 54, 646: 125 | 67; RAWINT4 167: 67 | 72, 235: 61 | 63, 247: 176 | 153,
+// 310: 73 | 69, 517: 267 | 186; Q4_K 349: 46 | 50, 487: 80 | 71, 582: 225 | 200, 955: 248 | 217.  With few repeats among many experts the
+// grouped kernels' 16-row tiles hold one row each and stream slower (256 experts of 7168 x 2048, AMXINT4, 8 tokens x 8: decode stays
+// ahead at 285 MB), hence the second condition.  Both ways give the same bits; a batch whose size only the device knows, masked experts, and
+// formats that were not measured stay where they were.
+static bool shares_experts(const ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, size_t bytes) {
+  double mb;
+  switch (h->cfg.format) {
+    case KTX_FMT_AMXINT4: mb = 118; break;
+    case KTX_FMT_FP8: mb = 255; break;
+    case KTX_FMT_RAWINT4: mb = 240; break;
+    case KTX_FMT_GGUF: mb = 700; break;
+    default: return false;
+  }
+  if (d_bsz || h->mask) return false;
+  const double G = h->cfg.global_expert_num, own = h->cfg.expert_num / G;
+  const double pairs = qlen * k * own, distinct = h->cfg.expert_num * (1.0 - std::pow(1.0 - 1.0 / G, (double)qlen * k));
+  return pairs >= 1.25 * distinct && (pairs - 0.9 * distinct) * (double)bytes >= mb * 1e6;
+}
+
 static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, const int64_t* d_expert_ids,
                             const float* d_weights, const void* d_input, void* d_output, int flags, ktx_stream_t stream,
                             const DecSide* side) {
@@ -3131,7 +3156,8 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
   const int E = h->cfg.expert_num, H = h->cfg.hidden_size, I = h->cfg.intermediate_size;
   Workspace* ws = h->ws;
   if (h->cfg.format == KTX_FMT_AMXINT4 || h->cfg.format == KTX_FMT_AMXINT8)
-  if (qlen * k <= KTX_DEC_MAX_PAIRS && k <= 8 && H <= 8192 && I <= 2048 && !g_force_generic) {
+  if (qlen * k <= KTX_DEC_MAX_PAIRS && k <= 8 && H <= 8192 && I <= 2048 && !g_force_generic &&
+      (side || !shares_experts(h, d_bsz, qlen, k, 2 * h->gu_stride + h->dn_stride))) {
     DecParams dp;
     dp.d_bsz = d_bsz; dp.qlen = qlen; dp.k = k; dp.E = E; dp.expert_begin = h->cfg.expert_begin; dp.H = H; dp.I = I;
     dp.ids = d_expert_ids; dp.mask = h->mask; dp.x = (const bf16_t*)d_input; dp.weights = d_weights;
@@ -3313,7 +3339,8 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
   const int d2 = fp8 ? (nks2 % 16 == 0 ? 16 : nks2 % 8 == 0 ? 8 : nks2 % 4 == 0 ? 4 : nks2 % 2 == 0 ? 2 : 1)
                      : (nks2 % 8 == 0 ? 8 : nks2 % 4 == 0 ? 4 : nks2 % 2 == 0 ? 2 : 1);
   const size_t lds_dn = (size_t)k * I * 2 + (size_t)k * 16 * sizeof(float) + (size_t)k * 2 * sizeof(int);
-  if (npairs <= KTX_DEC_MAX_PAIRS && k <= 8 && H <= 16384 && I <= 4096 && lds_dn <= 160 * 1024 && !g_force_generic) {
+  if (npairs <= KTX_DEC_MAX_PAIRS && k <= 8 && H <= 16384 && I <= 4096 && lds_dn <= 160 * 1024 && !g_force_generic &&
+      !shares_experts(h, d_bsz, qlen, k, 2 * h->gu_stride + h->dn_stride)) {
     DecFpParams dp;
     dp.d_bsz = d_bsz; dp.qlen = qlen; dp.k = k; dp.E = E; dp.expert_begin = h->cfg.expert_begin; dp.H = H; dp.I = I;
     dp.ids = d_expert_ids; dp.mask = h->mask; dp.x = (const bf16_t*)d_input; dp.weights = d_weights;
@@ -3449,7 +3476,8 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
 
   // ---- decode fast path: two launches (see moe_dec_raw_gateup_kernel) -----------------------------------------------------
   const size_t lds_rdn = (size_t)k * (I + I / 32 * 4 + 16 * 4 + 8);
-  if (npairs <= KTX_DEC_MAX_PAIRS && k <= 8 && H <= 8192 && I <= 4096 && lds_rdn <= 160 * 1024 && !g_force_generic) {
+  if (npairs <= KTX_DEC_MAX_PAIRS && k <= 8 && H <= 8192 && I <= 4096 && lds_rdn <= 160 * 1024 && !g_force_generic &&
+      !shares_experts(h, d_bsz, qlen, k, 2 * h->gu_stride + h->dn_stride)) {
     RawDecParams dp;
     dp.d_bsz = d_bsz; dp.qlen = qlen; dp.k = k; dp.E = E; dp.expert_begin = h->cfg.expert_begin; dp.H = H; dp.I = I;
     dp.ids = d_expert_ids; dp.mask = h->mask; dp.x = (const bf16_t*)d_input; dp.weights = d_weights;
@@ -3683,7 +3711,8 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   }
   int mt = std::min(4, pick_mt(qlen, k, E));
   // (IQ1_S keeps to pick_mt: its 16 KiB grid table beside two 32 KiB stages leaves ONE workgroup per CU — measured 1.6x slower)
-  if (gg_foldable(h->gg_type[0]) && gg_foldable(h->gg_type[2]) && h->gg_type[0] != GG_IQ1S && h->gg_type[2] != GG_IQ1S && g_dbg[21] != 1) {
+  const bool folds = gg_foldable(h->gg_type[0]) && gg_foldable(h->gg_type[2]) && h->gg_type[0] != GG_IQ1S && h->gg_type[2] != GG_IQ1S && g_dbg[21] != 1;
+  if (folds) {
     // Rows per tile: a tile's weights are read and folded once, so low tiles cost passes over the weights and high ones work on absent
     // rows.  Measured (Q4_K, 16 | 32 | 64-row tiles, us): 64 experts of 2048 x 1536 with 2.3 rows each 83 | 89 | 95, 4.5: 103 | 109 | 118,
     // 9.4: 123 | 121 | 130, 19: 165 | 145 | 143; 8 experts of 4096 x 14336 with 12 rows 284 | 242 | 264, 25: 353 | 325 | 286, 50: 607 | 469 | 368.
@@ -3702,7 +3731,8 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
     const size_t lds_gu = (size_t)H + (size_t)nkb1 * (gg_nbs(tg) + 1) * 4 + 32 + (tg == GG_IQ1S ? 4096 * 8 : 0);   // (+ the arrival flag)
     const size_t lds_dn = (size_t)k * I + (size_t)k * nkb2 * (gg_nbs(td) + 1) * 4 + (size_t)k * (16 + 2) * 4 + 8 +
                           (td == GG_IQ1S ? 4096 * 8 : 0);
-    if (npairs <= KTX_DEC_MAX_PAIRS && k <= 8 && nkb2 <= 64 && lds_gu <= 64 * 1024 && lds_dn <= 64 * 1024 && !g_force_generic) {
+    if (npairs <= KTX_DEC_MAX_PAIRS && k <= 8 && nkb2 <= 64 && lds_gu <= 64 * 1024 && lds_dn <= 64 * 1024 && !g_force_generic &&
+        !(folds && shares_experts(h, d_bsz, qlen, k, h->gg_stride[0] + h->gg_stride[1] + h->gg_stride[2]))) {
       GgDecParams dp;
       dp.d_bsz = d_bsz; dp.qlen = qlen; dp.k = k; dp.E = E; dp.expert_begin = h->cfg.expert_begin; dp.H = H; dp.I = I;
       dp.ids = d_expert_ids; dp.mask = h->mask; dp.x = (const bf16_t*)d_input; dp.weights = d_weights;

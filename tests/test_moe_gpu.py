@@ -623,3 +623,47 @@ def test_rawint4_rows_per_tile_and_scales_outside_f16(oracle, dev, H, I):
                     _check_fp(got, want)
         finally:
             h.close()
+
+
+@pytest.mark.parametrize("method", ["AMXINT4", "FP8", "RAWINT4", "GGUF"])
+def test_batches_that_share_experts_take_the_grouped_kernels(dev, method):
+    """64 (token, expert) pairs over 4 experts: the grouped kernels, which read an expert once, give what the decode launches give (a batch
+    whose size only the device knows stays on them).  The same bits; Q4_K to the order of its fp32 sums of K / 256 block terms, at most
+    16 * 2^-24 of their magnitudes' sum (some 10 rms) in front of one bf16 rounding, which may then fall the other way."""
+    from ktransformers_amd._native import MoEHandle
+    E, k, H, I, T = 4, 2, 4096, 2048, 32
+    g = torch.Generator(device=dev).manual_seed(5)
+    shapes = ((I, H), (I, H), (H, I))
+
+    def byte(*s):
+        return torch.randint(0, 256, s, dtype=torch.uint8, device=dev, generator=g)
+
+    def normal(*s):
+        return torch.randn(s, device=dev, generator=g)
+    h = MoEHandle(E, k, H, I, T, method, 0, group_size={"RAWINT4": 32, "FP8": 128}.get(method, 0))
+    try:
+        if method == "AMXINT4":
+            h.load_bf16(*(normal(E, n, kk).bfloat16() for n, kk in shapes))
+        elif method == "FP8":
+            h.load_fp8(*(normal(E, n, kk).mul_(100).clamp_(-448, 448).to(torch.float8_e4m3fn) for n, kk in shapes),
+                       *(torch.full((E, n // 128, kk // 128), 1e-3, device=dev) for n, kk in shapes))
+        elif method == "RAWINT4":
+            h.load_rawint4(*(byte(E, n, kk // 2) for n, kk in shapes),
+                           *(normal(E, n, kk // 32).mul_(1e-2).bfloat16() for n, kk in shapes))
+        else:
+            blocks = [byte(E, n, kk // 256, 144) for n, kk in shapes]
+            for b in blocks:
+                b[..., 0:4] = torch.tensor([1e-3, 7e-3], dtype=torch.float16, device=dev).view(torch.uint8)
+            h.load_gguf(*(b.flatten(2) for b in blocks), 12, 12, 12)
+        x, w = normal(T, H).bfloat16(), torch.rand((T, k), device=dev, generator=g)
+        ids = torch.stack([torch.randperm(E, device=dev, generator=g)[:k] for _ in range(T)])
+        ids[0, 0], ids[T - 1, 1] = -1, E
+        got = h.forward(x, ids, w).float()
+        want = h.forward(x, ids, w, bsz_tensor=torch.tensor([T], dtype=torch.int32, device=dev)).float()
+    finally:
+        h.close()
+    assert want.abs().max() > 0
+    if method == "GGUF":
+        assert ((got - want).abs() <= want.abs() * 2.0 ** -7 + want.square().mean().sqrt() * 160 * 2.0 ** -24).all()
+    else:
+        assert torch.equal(got, want)
