@@ -37,6 +37,8 @@ struct MlaParams {
   float sm_scale;
   float* part_o;   // [total_q][Hq][nsplit][512]
   float* part_ml;  // [total_q][Hq][nsplit][2]
+  int jobs;        // > 0 (mla_decode_wide_kernel): workgroups per head block that share the tokens' tiles; nsplit is a token's most splits then
+  int* njobs;      // [total_q]: how many it takes
   bf16_t* out1;    // nsplit == 1: the split-KV kernel normalises and stores the result itself (no partials, no merge launch)
   float* lse1;
   // optional fused cache append for decode (one new token per request): latent rows [batch][512], [batch][64]
@@ -108,6 +110,136 @@ __device__ __forceinline__ void mla_dma_row_sa(const bf16_t* gsrc_row, uint32_t 
                : "memory");
 }
 
+// Staging of one 32-token tile, entirely by LDS-DMA (no VGPR destination, nothing the compiler has to wait for inside the
+// loop).  A tile lies inside one page (page_size % 32 == 0 is required by the launcher), whose index is a scalar load.
+// ckv: one 1-KiB row per wave-instruction into Kt[row]; k_pe: eight 128-byte rows per wave-instruction into Kp, 16-byte
+// piece g of row r at position g ^ (r & 7) (the XOR keeps the fragment reads of 16 rows at most 2-way bank-conflicted
+// although the rows are packed).  Rows past the end of the context re-read the last valid row: finite values that the
+// softmax weights them with exactly 0 (their scores are masked), and nothing beyond kv_len is ever touched.
+template <int NWV>
+__device__ __forceinline__ void mla_stage(const MlaParams& p, int req, int kv_end, int app_pos, int tile, int page_v, int wave, int lane,
+                                          uint32_t dK, uint32_t dP) {   // LDS byte addresses of the ckv and the k_pe rows
+  const int tok0 = tile * MLA_TILE;
+  const int page0 = __builtin_amdgcn_readfirstlane(page_v);
+  const size_t row0 = (size_t)page0 * p.page_size + (p.tiles_shift >= 0 ? tok0 & (p.page_size - 1) : tok0 % p.page_size);
+  const int last = kv_end - 1 - tok0;   // last valid row of the tile (>= 0: the tile holds a visible token)
+  // a whole tile without the appended row (all but one or two tiles of a split): one 64-bit product for the tile, then adds — the
+  // general form below spends ~25 scalar instructions per row on clamps, the append override and pointer casts (SQ counters of
+  // the loop: as many SALU as VALU instructions, profiles/r06_Z_pmc_mla_decode_128k.txt)
+  if (last >= MLA_TILE - 1 && (unsigned)(app_pos - tok0) >= (unsigned)MLA_TILE) {
+    const bf16_t* src = p.ckv + (row0 + wave) * p.ckv_ts;
+    const size_t step = (size_t)NWV * p.ckv_ts;
+    uint32_t dst = dK + (uint32_t)wave * (MLA_KROW * 2);
+#pragma unroll
+    for (int r = wave; r < MLA_TILE; r += NWV, src += step, dst += NWV * MLA_KROW * 2) mla_dma_row_sa(src, (uint32_t)lane * 16u, dst);
+    if (wave < 4) {
+      const int r = wave * 8 + (lane >> 3), g = (lane & 7) ^ (lane >> 3);
+      mla_dma_row_a(p.k_pe + (row0 + r) * p.kpe_ts + g * 8, dP + (uint32_t)wave * (8 * MLA_DR * 2));
+    }
+    return;
+  }
+#pragma unroll
+  for (int r = wave; r < MLA_TILE; r += NWV) {   // (every term wave-uniform: scalar arithmetic, mla_dma_row_sa)
+    const int rr = min(r, last);
+    const bf16_t* src = p.ckv + (row0 + rr) * p.ckv_ts;
+    if (tok0 + rr == app_pos) src = p.app_ckv + (size_t)req * MLA_DC;
+    mla_dma_row_sa(src, (uint32_t)lane * 16u, dK + (uint32_t)r * (MLA_KROW * 2));
+  }
+  if (wave < 4) {
+    const int r = wave * 8 + (lane >> 3), rr = min(r, last);
+    const int g = (lane & 7) ^ (lane >> 3);
+    const bf16_t* src = p.k_pe + (row0 + rr) * p.kpe_ts;
+    if (tok0 + rr == app_pos) src = p.app_kpe + (size_t)req * MLA_DR;
+    mla_dma_row_a(src + g * 8, dP + (uint32_t)wave * (8 * MLA_DR * 2));
+  }
+}
+
+// Four of them, 8 KiB apart in the LDS, from one scalar base
+__device__ __forceinline__ void mla_dma_4rows(const bf16_t* base, const uint32_t (&off)[4], uint32_t lds_addr) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %5\n\t"
+               "s_add_u32 m0, m0, 0x2000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %5\n\t"
+               "s_add_u32 m0, m0, 0x2000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %5\n\t"
+               "s_add_u32 m0, m0, 0x2000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, %5\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base), "s"(lds_addr)
+               : "memory", "scc");
+}
+// which request owns query token qt?  Every wavefront resolves it on its own with ONE round of independent loads
+// (lane i looks at request i) — the live-request count *d_bsz is fetched in the same round and applied afterwards, not
+// waited for first: right after a kernel boundary each dependent load is another 1.5-3 us (measured with the phase stamps)
+__device__ __forceinline__ void mla_find_request(const MlaParams& p, int qt, int lane, int& req, int& kv_end, int& page_base, int& app_pos) {
+  req = -1; kv_end = 0; page_base = 0; app_pos = -1;
+  const int bsz_raw = p.d_bsz ? *p.d_bsz : p.batch;
+  for (int b0 = 0; b0 < p.batch && req < 0; b0 += 64) {
+    const int i = b0 + lane;
+    int q0 = 0x7fffffff, q1 = 0, kl = 0, kp = 0;
+    if (i < p.batch) {
+      q0 = p.qo_indptr[i]; q1 = p.qo_indptr[i + 1]; kl = p.kv_len[i]; kp = p.kv_indptr[i];
+      // never index past the pages the request owns: a sequence that outgrew its cache attends to (and appends within)
+      // its last page instead of reading kv_indices / writing HBM out of bounds
+      kl = min(kl, (p.kv_indptr[i + 1] - kp) * p.page_size);
+    }
+    const int B = min(max(bsz_raw, 0), p.batch);
+    const unsigned long long hit = __ballot(i < B && qt >= q0 && qt < q1);
+    if (hit) {
+      const int src = __ffsll((long long)hit) - 1;
+      q0 = __builtin_amdgcn_readlane(q0, src); q1 = __builtin_amdgcn_readlane(q1, src);
+      kl = __builtin_amdgcn_readlane(kl, src); kp = __builtin_amdgcn_readlane(kp, src);
+      req = b0 + src;
+      const int qo_len = q1 - q0;
+      kv_end = max(kl - qo_len + (qt - q0) + 1, 0);   // causal: positions < kv_end are visible
+      page_base = kp;
+      // fused cache append (decode: one new token per request): the newest position is taken from the append buffers
+      if (p.app_ckv && qo_len == 1) app_pos = kl - 1;
+    }
+  }
+}
+
+// The appended token (decode: one new row per request) is taken from the append buffers wherever its position is staged;
+// the workgroup (hb 0) whose split owns its tile also writes it into the cache (StaticCache.update, custom_cache.py:189-195)
+__device__ __forceinline__ void mla_store_appended(const MlaParams& p, int req, int page_base, int app_pos, int tid) {
+  if (tid >= 72) return;
+  const int page = p.kv_indices ? p.kv_indices[page_base + app_pos / p.page_size] : page_base + app_pos / p.page_size;
+  const size_t trow = (size_t)page * p.page_size + app_pos % p.page_size;
+  if (tid < 64) *reinterpret_cast<uint4*>(p.ckv_w + trow * p.ckv_ts + tid * 8) = *reinterpret_cast<const uint4*>(p.app_ckv + (size_t)req * MLA_DC + tid * 8);
+  else *reinterpret_cast<uint4*>(p.kpe_w + trow * p.kpe_ts + (tid - 64) * 8) = *reinterpret_cast<const uint4*>(p.app_kpe + (size_t)req * MLA_DR + (tid - 64) * 8);
+}
+
+template <int NDT>
+__device__ __forceinline__ void mla_store_result(const MlaParams& p, int qt, int head0, int ds, int lane, size_t pidx, bool any, const v4f (&o)[NDT],
+                                                 const float (&m_run)[4], const float (&l_run)[4]) {
+  if (p.out1) {   // one split holds the whole row: the merge kernel's arithmetic for a single partial (weight 1), in place
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int h = head0 + (lane >> 4) * 4 + r;
+      const float l = __shfl(l_run[r], lane & 48), m = __shfl(m_run[r], lane & 48);
+      const float inv = l > 0.f ? 1.0f / l : 0.f;
+      bf16_t* po = p.out1 + ((size_t)qt * p.Hq + h) * MLA_DC + ds * NDT * 16;
+#pragma unroll
+      for (int i = 0; i < NDT; i++) po[i * 16 + (lane & 15)] = f32_to_bf16(o[i][r] * inv);
+      if (p.lse1 && (lane & 15) == 0 && ds == 0)
+        p.lse1[(size_t)qt * p.Hq + h] = l > 0.f ? (m + __logf(l)) * 1.44269504089f : -__builtin_inff();
+    }
+    return;
+  }
+  // ---- partial results: un-normalised O plus (m, l) per head ------------------------------------------------------------
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int hrow = (lane >> 4) * 4 + r;
+    if ((lane & 15) == 0 && ds == 0) {
+      float* ml = p.part_ml + (pidx + (size_t)hrow * p.nsplit) * 2;
+      ml[0] = m_run[r];
+      ml[1] = l_run[r];
+    }
+    if (any) {
+      float* po = p.part_o + (pidx + (size_t)hrow * p.nsplit) * MLA_DC + ds * NDT * 16;
+#pragma unroll
+      for (int i = 0; i < NDT; i++) po[i * 16 + (lane & 15)] = o[i][r];
+    }
+  }
+}
+
 // Workgroup = HBW head blocks (16 heads each) x DSPLIT slices: wave (hbw, ds) computes 512/DSPLIT dims of O += P V (which
 // divides the fp32 accumulator registers — the 128-VGPR O tile of the undivided form left one wave per SIMD running a
 // serial chain of LDS reads and MFMAs, ~7 us per 32-token tile) and every DSPLIT-th 32-wide k-step of S = Q K^T; the DSPLIT
@@ -148,34 +280,8 @@ __global__ __launch_bounds__(HBW * DSPLIT * 64) void mla_decode_kernel(MlaParams
     }
   }
 
-  // which request owns query token qt?  Every wavefront resolves it on its own with ONE round of independent loads
-  // (lane i looks at request i) — the live-request count *d_bsz is fetched in the same round and applied afterwards, not
-  // waited for first: right after a kernel boundary each dependent load is another 1.5-3 us (measured with the phase stamps)
-  int req = -1, kv_end = 0, page_base = 0, app_pos = -1;
-  const int bsz_raw = p.d_bsz ? *p.d_bsz : p.batch;
-  for (int b0 = 0; b0 < p.batch && req < 0; b0 += 64) {
-    const int i = b0 + lane;
-    int q0 = 0x7fffffff, q1 = 0, kl = 0, kp = 0;
-    if (i < p.batch) {
-      q0 = p.qo_indptr[i]; q1 = p.qo_indptr[i + 1]; kl = p.kv_len[i]; kp = p.kv_indptr[i];
-      // never index past the pages the request owns: a sequence that outgrew its cache attends to (and appends within)
-      // its last page instead of reading kv_indices / writing HBM out of bounds
-      kl = min(kl, (p.kv_indptr[i + 1] - kp) * p.page_size);
-    }
-    const int B = min(max(bsz_raw, 0), p.batch);
-    const unsigned long long hit = __ballot(i < B && qt >= q0 && qt < q1);
-    if (hit) {
-      const int src = __ffsll((long long)hit) - 1;
-      q0 = __builtin_amdgcn_readlane(q0, src); q1 = __builtin_amdgcn_readlane(q1, src);
-      kl = __builtin_amdgcn_readlane(kl, src); kp = __builtin_amdgcn_readlane(kp, src);
-      req = b0 + src;
-      const int qo_len = q1 - q0;
-      kv_end = max(kl - qo_len + (qt - q0) + 1, 0);   // causal: positions < kv_end are visible
-      page_base = kp;
-      // fused cache append (decode: one new token per request): the newest position is taken from the append buffers
-      if (p.app_ckv && qo_len == 1) app_pos = kl - 1;
-    }
-  }
+  int req, kv_end, page_base, app_pos;
+  mla_find_request(p, qt, lane, req, kv_end, page_base, app_pos);
   req = __builtin_amdgcn_readfirstlane(req);
   kv_end = __builtin_amdgcn_readfirstlane(kv_end);
   page_base = __builtin_amdgcn_readfirstlane(page_base);
@@ -195,21 +301,8 @@ __global__ __launch_bounds__(HBW * DSPLIT * 64) void mla_decode_kernel(MlaParams
   for (int r = 0; r < 4; r++) { m_run[r] = -__builtin_inff(); l_run[r] = 0.f; }
 
   if (t_begin < t_end) {
-    // The appended token (decode: one new row per request) is taken from the append buffers wherever its position is staged;
-    // the workgroup (hb 0) whose split owns its tile also writes it into the cache (StaticCache.update, custom_cache.py:189-195)
-    if (app_pos >= 0 && hb == 0 && (app_pos / MLA_TILE) % p.nsplit == split && tid < 72) {
-      const int page = p.kv_indices ? p.kv_indices[page_base + app_pos / p.page_size] : page_base + app_pos / p.page_size;
-      const size_t trow = (size_t)page * p.page_size + app_pos % p.page_size;
-      if (tid < 64) *reinterpret_cast<uint4*>(p.ckv_w + trow * p.ckv_ts + tid * 8) = *reinterpret_cast<const uint4*>(p.app_ckv + (size_t)req * MLA_DC + tid * 8);
-      else *reinterpret_cast<uint4*>(p.kpe_w + trow * p.kpe_ts + (tid - 64) * 8) = *reinterpret_cast<const uint4*>(p.app_kpe + (size_t)req * MLA_DR + (tid - 64) * 8);
-    }
+    if (app_pos >= 0 && hb == 0 && (app_pos / MLA_TILE) % p.nsplit == split) mla_store_appended(p, req, page_base, app_pos, tid);
 
-    // Staging of one 32-token tile, entirely by LDS-DMA (no VGPR destination, nothing the compiler has to wait for inside the
-    // loop).  A tile lies inside one page (page_size % 32 == 0 is required by the launcher), whose index is a scalar load.
-    // ckv: one 1-KiB row per wave-instruction into Kt[row]; k_pe: eight 128-byte rows per wave-instruction into Kp, 16-byte
-    // piece g of row r at position g ^ (r & 7) (the XOR keeps the fragment reads of 16 rows at most 2-way bank-conflicted
-    // although the rows are packed).  Rows past the end of the context re-read the last valid row: finite values that the
-    // softmax weights them with exactly 0 (their scores are masked), and nothing beyond kv_len is ever touched.
     // (LDS destinations as byte addresses off the dynamic region's base, Kt = smem: see mla_dma_row_a)
     const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)smem;
     constexpr uint32_t KT_BYTES = MLA_TILE * MLA_KROW * 2, KP_BYTES = MLA_TILE * MLA_DR * 2;
@@ -222,40 +315,7 @@ __global__ __launch_bounds__(HBW * DSPLIT * 64) void mla_decode_kernel(MlaParams
       return p.kv_indices ? p.kv_indices[pidx_] : pidx_;
     };
     auto stage = [&](int tile, int page_v, int buf) {   // buf = which of the two staged tiles
-      const uint32_t dK = lds0 + (uint32_t)buf * KT_BYTES, dP = lds0 + 2 * KT_BYTES + (uint32_t)buf * KP_BYTES;
-      const int tok0 = tile * MLA_TILE;
-      const int page0 = __builtin_amdgcn_readfirstlane(page_v);
-      const size_t row0 = (size_t)page0 * p.page_size + (p.tiles_shift >= 0 ? tok0 & (p.page_size - 1) : tok0 % p.page_size);
-      const int last = kv_end - 1 - tok0;   // last valid row of the tile (>= 0: the tile holds a visible token)
-      // a whole tile without the appended row (all but one or two tiles of a split): one 64-bit product for the tile, then adds — the
-      // general form below spends ~25 scalar instructions per row on clamps, the append override and pointer casts (SQ counters of
-      // the loop: as many SALU as VALU instructions, profiles/r06_Z_pmc_mla_decode_128k.txt)
-      if (last >= MLA_TILE - 1 && (unsigned)(app_pos - tok0) >= (unsigned)MLA_TILE) {
-        const bf16_t* src = p.ckv + (row0 + wave) * p.ckv_ts;
-        const size_t step = (size_t)NWV * p.ckv_ts;
-        uint32_t dst = dK + (uint32_t)wave * (MLA_KROW * 2);
-#pragma unroll
-        for (int r = wave; r < MLA_TILE; r += NWV, src += step, dst += NWV * MLA_KROW * 2) mla_dma_row_sa(src, (uint32_t)lane * 16u, dst);
-        if (wave < 4) {
-          const int r = wave * 8 + (lane >> 3), g = (lane & 7) ^ (lane >> 3);
-          mla_dma_row_a(p.k_pe + (row0 + r) * p.kpe_ts + g * 8, dP + (uint32_t)wave * (8 * MLA_DR * 2));
-        }
-        return;
-      }
-#pragma unroll
-      for (int r = wave; r < MLA_TILE; r += NWV) {   // (every term wave-uniform: scalar arithmetic, mla_dma_row_sa)
-        const int rr = min(r, last);
-        const bf16_t* src = p.ckv + (row0 + rr) * p.ckv_ts;
-        if (tok0 + rr == app_pos) src = p.app_ckv + (size_t)req * MLA_DC;
-        mla_dma_row_sa(src, (uint32_t)lane * 16u, dK + (uint32_t)r * (MLA_KROW * 2));
-      }
-      if (wave < 4) {
-        const int r = wave * 8 + (lane >> 3), rr = min(r, last);
-        const int g = (lane & 7) ^ (lane >> 3);
-        const bf16_t* src = p.k_pe + (row0 + rr) * p.kpe_ts;
-        if (tok0 + rr == app_pos) src = p.app_kpe + (size_t)req * MLA_DR;
-        mla_dma_row_a(src + g * 8, dP + (uint32_t)wave * (8 * MLA_DR * 2));
-      }
+      mla_stage<NWV>(p, req, kv_end, app_pos, tile, page_v, wave, lane, lds0 + (uint32_t)buf * KT_BYTES, lds0 + 2 * KT_BYTES + (uint32_t)buf * KP_BYTES);
     };
 
     stage(t_begin, page_of(t_begin), 0);
@@ -370,34 +430,323 @@ __global__ __launch_bounds__(HBW * DSPLIT * 64) void mla_decode_kernel(MlaParams
   }
   MLA_TS(6);
 
-  if (p.out1) {   // one split holds the whole row: the merge kernel's arithmetic for a single partial (weight 1), in place
+  mla_store_result<NDT>(p, qt, head0, ds, lane, pidx, t_begin < t_end, o, m_run, l_run);
+  MLA_TS(7);
+}
+
+// ---- 64 heads per workgroup: batches, long contexts, prompts ------------------------------------------------------------------------
+// Which query token and which of its KV splits a workgroup of the jobs form works on.  p.jobs workgroups (per head block) are shared out by
+// what the requests hold: D, the tiles per job, is the smallest for which sum_t ceil(tiles_t / D) <= jobs (and no token takes more than
+// nsplit, the workspace's slots); every wavefront finds it alone, lane = query token, from one round of loads.
+struct MlaWork { int qt, split, nsp, req, kv_end, page_base, app_pos; };
+__device__ __forceinline__ MlaWork mla_pick_job(const MlaParams& p, int job, int lane) {
+  int q0 = 0x7fffffff, q1 = 0x7fffffff, kl = 0, kp = 0;
+  const int bsz_raw = p.d_bsz ? *p.d_bsz : p.batch;
+  if (lane < p.batch) {
+    q0 = p.qo_indptr[lane]; q1 = p.qo_indptr[lane + 1]; kl = p.kv_len[lane]; kp = p.kv_indptr[lane];
+    kl = min(kl, (p.kv_indptr[lane + 1] - kp) * p.page_size);   // never past the pages the request owns
+  }
+  const int B = min(max(bsz_raw, 0), p.batch);
+  int r = 0;
+  for (int i = 0; i < B; i++) r += __builtin_amdgcn_readlane(q1, i) <= lane ? 1 : 0;
+  const int src = min(r, 63);
+  const int tq0 = __shfl(q0, src, 64), tq1 = __shfl(q1, src, 64), tkl = __shfl(kl, src, 64), tkp = __shfl(kp, src, 64);
+  const bool live = lane < p.total_q && r < B && lane >= tq0;
+  const int vis = live ? max(tkl - (tq1 - tq0) + (lane - tq0) + 1, 0) : 0;   // causal: positions < vis are visible
+  const int tiles = (vis + 2 * MLA_TILE - 1) / (2 * MLA_TILE);   // steps of 64 tokens
+  const int sum = (int)wave_sum((float)tiles), most = (int)wave_max((float)tiles), nlive = (int)wave_sum(live ? 1.f : 0.f);
+  auto jobs_of = [&](int d) { return live ? max(1, (tiles + d - 1) / d) : 0; };
+  // at D = ceil(sum / (jobs - live tokens)) every token's rounding up is paid for (the launcher gives two jobs a token and more)
+  int lo = max(1, max((sum + p.jobs - 1) / p.jobs, (most + p.nsplit - 1) / p.nsplit));
+  int hi = max(lo, (sum + p.jobs - nlive - 1) / max(1, p.jobs - nlive));
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if ((int)wave_sum((float)jobs_of(mid)) <= p.jobs) hi = mid;
+    else lo = mid + 1;
+  }
+  const int n = jobs_of(lo);
+  int inc = n;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int h = head0 + (lane >> 4) * 4 + r;
-      const float l = __shfl(l_run[r], lane & 48), m = __shfl(m_run[r], lane & 48);
-      const float inv = l > 0.f ? 1.0f / l : 0.f;
-      bf16_t* po = p.out1 + ((size_t)qt * p.Hq + h) * MLA_DC + ds * NDT * 16;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int a = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += a;
+  }
+  const unsigned long long later = __ballot(inc > job);
+  MlaWork w;
+  if (!later) { w.req = -1; return w; }
+  const int t = __ffsll((long long)later) - 1;
+  w.qt = t;
+  w.nsp = __builtin_amdgcn_readlane(n, t);
+  w.split = job - (__builtin_amdgcn_readlane(inc, t) - w.nsp);
+  w.req = __builtin_amdgcn_readlane(r, t);
+  w.kv_end = __builtin_amdgcn_readlane(vis, t);
+  w.page_base = __builtin_amdgcn_readlane(tkp, t);
+  // fused cache append (decode: one new token per request): the newest position is taken from the append buffers
+  w.app_pos = p.app_ckv && __builtin_amdgcn_readlane(tq1 - tq0, t) == 1 ? __builtin_amdgcn_readlane(tkl, t) - 1 : -1;
+  return w;
+}
+
+// Reductions over the four 16-lane rows of a wavefront (lanes l, l ^ 16, l ^ 32, l ^ 48): gfx950's row swaps — v_permlane32_swap
+// exchanges the upper 32 lanes of one register with the lower 32 of another, v_permlane16_swap the odd rows with the even rows — are
+// plain VALU instructions; the ds_bpermute shuffles they replace are LDS-crossbar round trips, four of them in a dependent chain per
+// query tile and key tile.  Sum: (x_l + x_{l^32}) + (that of l ^ 16) — fp32 addition is commutative, so every lane of a query gets the
+// same bits, and they are the bits the shuffle version produced ((x + shfl16) + shfl32 groups the rows as (r0 + r1) + (r2 + r3) for
+// rows 0 / 1 and likewise here after the 32-swap first: see pf_sum_rows).
+typedef unsigned pf_v2u __attribute__((ext_vector_type(2)));
+typedef float pf_v2f __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float pf_max_rows(float x) {
+  pf_v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float pf_sum_rows(float x) {
+  // the shuffle version computed (x + x^16) first, then + the same of l ^ 32: keep that association — rows (r0 + r1) and (r2 + r3)
+  // first (16-swap), then across the halves (32-swap)
+  pf_v2u r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Workgroup = 4 head blocks of 16 x 2 wavefronts, one per CU; a step is 64 tokens, staged once for all 64 heads and double-buffered.  A
+// wavefront computes S of 32 of the tokens x 16 heads, takes the other 32 from its partner through the LDS, and after the softmax (which both
+// do) 256 dims of O.  S and O are computed transposed (tokens x heads, dims x heads), so that a lane owns ONE head: the softmax statistics are
+// one value a lane, and S^T leaves the MFMA with a lane's tokens where P^T enters the next one — the probabilities never leave the
+// registers (V's rows are read in the order 4 g + (0..3), 16 + 4 g + (0..3) that this gives lane group g).
+// What bounds it: the LDS, 576 KB read and 72 KB staged a step of a CU, beside 68 MFMAs a wavefront.  The rows are packed 1 KiB apart with
+// their 16-byte pieces permuted by mla_swz, which keeps both the fragment reads of 16 rows and the transposed reads of 8 rows off each other's
+// banks.  128 heads, 8 requests of 2048 .. 8192 tokens, us for 64 tokens: mla_decode_kernel<4, 2> 5.8 (scores of half the dims exchanged
+// for every 32 tokens, softmax on 4 values a lane and head), this 2.5; no exchange, S computed by both wavefronts 2.9; a wavefront for itself,
+// 512 dims of O for 32 tokens, 3.1 (the registers are full, and every MFMA waits for its LDS read); rows padded to 1168 B + 0.5.
+// distinct for 16 rows, also with rows 4 .. 11 flipped by 1 (ds_read_b128 takes lanes 0-3, 12-15, 20-23, 24-27 together); >> 1 distinct for rows
+// 0-7 and for 8-15 (ds_read_b64_tr_b16 takes 32 lanes together)
+__device__ __forceinline__ uint32_t mla_swz(uint32_t row) { return row & 8 ? ((row & 7) ^ 4) << 1 | 1 : (row & 7) << 1; }
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void mla_decode_wide_kernel(MlaParams p) {
+  constexpr int NWV = 8, NQ = 18, STEP = 2 * MLA_TILE;
+  constexpr uint32_t KT_BYTES = STEP * MLA_DC * 2, KP_BYTES = STEP * MLA_DR * 2;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];         // [2][64][1024 B] ckv | [2][64][128 B] k_pe | [8 waves][2][64] scores
+  float4* Sx = reinterpret_cast<float4*>(smem + 2 * (KT_BYTES + KP_BYTES));
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hb = blockIdx.y;
+  const int ds = wave & 1;
+  const int head = (hb * 4 + (wave >> 1)) * 16 + (lane & 15);
+  MLA_TS(0);
+
+  MlaWork w;
+  if (p.jobs) {
+    w = mla_pick_job(p, blockIdx.x, lane);
+    if (w.req >= 0 && hb == 0 && w.split == 0 && tid == 0) p.njobs[w.qt] = w.nsp;
+  } else {
+    w.qt = blockIdx.z; w.split = blockIdx.x; w.nsp = p.nsplit;
+    mla_find_request(p, w.qt, lane, w.req, w.kv_end, w.page_base, w.app_pos);
+  }
+  if (w.req < 0) return;
+  const int req = __builtin_amdgcn_readfirstlane(w.req), kv_end = __builtin_amdgcn_readfirstlane(w.kv_end);
+  const int page_base = __builtin_amdgcn_readfirstlane(w.page_base), app_pos = __builtin_amdgcn_readfirstlane(w.app_pos);
+  const int qt = __builtin_amdgcn_readfirstlane(w.qt), split = __builtin_amdgcn_readfirstlane(w.split);
+  const int nsp = __builtin_amdgcn_readfirstlane(w.nsp);
+  MLA_TS(1);
+
+  // the split's run of 32-token tiles: whole steps
+  const int ntiles = (kv_end + MLA_TILE - 1) / MLA_TILE;
+  const int each = 2 * (((kv_end + STEP - 1) / STEP + nsp - 1) / nsp);
+  const int t_begin = min(split * each, ntiles), t_end = min(t_begin + each, ntiles);
+
+  v4f o[16];     // O^T: dims 256 ds + 16 i + 4 g + (0..3) of the lane's head
 #pragma unroll
-      for (int i = 0; i < NDT; i++) po[i * 16 + (lane & 15)] = f32_to_bf16(o[i][r] * inv);
-      if (p.lse1 && (lane & 15) == 0 && ds == 0)
-        p.lse1[(size_t)qt * p.Hq + h] = l > 0.f ? (m + __logf(l)) * 1.44269504089f : -__builtin_inff();
+  for (int i = 0; i < 16; i++) o[i] = v4f{0.f, 0.f, 0.f, 0.f};
+  float m_run = -__builtin_inff(), l_run = 0.f;
+
+  if (t_begin < t_end) {
+    if (app_pos >= 0 && hb == 0 && app_pos / MLA_TILE >= t_begin && app_pos / MLA_TILE < t_end) mla_store_appended(p, req, page_base, app_pos, tid);
+
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)smem;
+    auto page_of = [&](int tile) -> int {   // looked up a step ahead of its staging (see mla_decode_kernel); clamped: a tile of this request
+      const int t = min(tile, ntiles - 1);
+      const int pidx_ = __builtin_amdgcn_readfirstlane(page_base + (p.tiles_shift >= 0 ? t >> p.tiles_shift : t * MLA_TILE / p.page_size));
+      return p.kv_indices ? p.kv_indices[pidx_] : pidx_;
+    };
+    // Four ckv rows a wavefront and tile, one 1-KiB row per wave-instruction; k_pe: eight rows per wave-instruction, by wavefronts 0-3 for the
+    // first tile of a step and 4-7 for the second.  Rows past the context re-read its last one: finite, weighted with exactly 0.  A tile that is
+    // all context and does not hold the appended row takes the lanes' offsets from registers: address arithmetic on the scalar unit, 250
+    // instructions a step, held a wavefront up for as long as its MFMAs.
+    uint32_t ro[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) ro[c] = (uint32_t)((wave + c * NWV) * p.ckv_ts * 2) + ((uint32_t)lane ^ mla_swz(wave + c * NWV)) * 16u;
+    const int pr = (wave & 3) * 8 + (lane >> 3);
+    const uint32_t po = (uint32_t)(pr * p.kpe_ts * 2) + ((uint32_t)(lane & 7) ^ ((pr >> 1) & 7)) * 16u;
+    auto stage_tile = [&](int tile, int page_v, uint32_t dK, uint32_t dP, int wsel) {
+      const int tok0 = tile * MLA_TILE, last = kv_end - 1 - tok0;
+      const int page0 = __builtin_amdgcn_readfirstlane(page_v);
+      const size_t row0 = (size_t)page0 * p.page_size + (p.tiles_shift >= 0 ? tok0 & (p.page_size - 1) : tok0 % p.page_size);
+      if (last >= MLA_TILE - 1 && (unsigned)(app_pos - tok0) >= (unsigned)MLA_TILE) {
+        mla_dma_4rows(p.ckv + row0 * p.ckv_ts, ro, dK + (uint32_t)wave * (MLA_DC * 2));
+        if ((wave >> 2) == wsel) mla_dma_row_sa(p.k_pe + row0 * p.kpe_ts, po, dP + (uint32_t)(wave & 3) * (8 * MLA_DR * 2));
+        return;
+      }
+      for (int c = 0; c < MLA_TILE / NWV; c++) {
+        const int r = wave + c * NWV, rr = min(r, last);
+        const bf16_t* src = p.ckv + (row0 + rr) * p.ckv_ts;
+        if (tok0 + rr == app_pos) src = p.app_ckv + (size_t)req * MLA_DC;
+        mla_dma_row_sa(src, ((uint32_t)lane ^ mla_swz(r)) * 16u, dK + (uint32_t)r * (MLA_DC * 2));
+      }
+      if ((wave >> 2) == wsel) {
+        const int rr = min(pr, last);
+        const bf16_t* src = p.k_pe + (row0 + rr) * p.kpe_ts;
+        if (tok0 + rr == app_pos) src = p.app_kpe + (size_t)req * MLA_DR;
+        mla_dma_row_a(src + ((lane & 7) ^ ((pr >> 1) & 7)) * 8, dP + (uint32_t)(wave & 3) * (8 * MLA_DR * 2));
+      }
+    };
+    auto stage = [&](int tile, int pg0, int pg1, int buf) {
+      const uint32_t dK = lds0 + (uint32_t)buf * KT_BYTES, dP = lds0 + 2 * KT_BYTES + (uint32_t)buf * KP_BYTES;
+      stage_tile(tile, pg0, dK, dP, 0);
+      stage_tile(min(tile + 1, ntiles - 1), pg1, dK + KT_BYTES / 2, dP + KP_BYTES / 2, 1);   // (behind the context: its last tile again, masked)
+    };
+
+    // fragment addresses within a stage: K rows 16 t + (lane & 15), piece 4 s + g; V rows 4 g + (lane & 15) / 4 (+ 16), piece 2 i + (lane >> 1 & 1)
+    const uint32_t kx = (ds * MLA_TILE + (lane & 15)) * (MLA_DC * 2) + (((uint32_t)g ^ mla_swz(lane & 15)) * 16);
+    const uint32_t px = (ds * MLA_TILE + (lane & 15)) * (MLA_DR * 2) + (((uint32_t)g ^ ((lane >> 1) & 7)) * 16);
+    const uint32_t vr = 4 * g + ((lane & 15) >> 2);
+    const uint32_t vx = vr * (MLA_DC * 2) + ((((lane >> 1) & 1) ^ mla_swz(vr)) * 16) + (lane & 1) * 8 + ds * 512;
+
+    stage(t_begin, page_of(t_begin), page_of(t_begin + 1), 0);
+    v8bf qf[NQ];   // B[k = (lane >> 4) * 8 .. + 7][n = head] of 16 nope and 2 rope k-steps
+    {
+      const bf16_t* qn = p.q_nope + ((size_t)qt * p.Hq + head) * MLA_DC + g * 8;
+      const bf16_t* qr = p.q_pe + ((size_t)qt * p.Hq + head) * MLA_DR + g * 8;
+#pragma unroll
+      for (int j = 0; j < 16; j++) qf[j] = as_v8bf(*reinterpret_cast<const uint4*>(qn + j * 32));
+#pragma unroll
+      for (int j = 0; j < 2; j++) qf[16 + j] = as_v8bf(*reinterpret_cast<const uint4*>(qr + j * 32));
     }
+    int pn0 = page_of(t_begin + 2), pn1 = page_of(t_begin + 3);
+    MLA_TS(2);
+
+    int cur = 0;
+    for (int tile = t_begin; tile < t_end; tile += 2, cur ^= 1) {
+      // behind this wave's wait and the barrier the step's rows are all there and every wave is done with the other buffer
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (tile + 2 < t_end) {
+        stage(tile + 2, pn0, pn1, cur ^ 1);
+        pn0 = page_of(tile + 4); pn1 = page_of(tile + 5);
+      }
+      const uint8_t* kb = smem + cur * KT_BYTES;
+      const uint8_t* pb = smem + 2 * KT_BYTES + cur * KP_BYTES;
+      const int ntok = kv_end - tile * MLA_TILE;
+
+      // ---- S^T = K Q^T: lane holds tokens 16 t + 4 g + r of its head; this wave's half of the tokens, the other's from the LDS
+      v4f st[4], sm[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      // (a k-step's fragments are read two ahead of the MFMAs: fenced, or the compiler reads one fragment ahead and waits for it)
+      v8bf kf[3][2];
+      auto load_k = [&](int s) __attribute__((always_inline)) {
+        const uint8_t* a = s < 16 ? kb + (kx ^ ((s & 3) * 64)) + (s >> 2) * 256 : pb + (px ^ ((s - 16) * 64));
+#pragma unroll
+        for (int t = 0; t < 2; t++) kf[s % 3][t] = as_v8bf(*reinterpret_cast<const uint4*>(a + t * (s < 16 ? 16 * MLA_DC * 2 : 16 * MLA_DR * 2)));
+      };
+      load_k(0);
+      load_k(1);
+#pragma unroll
+      for (int s = 0; s < NQ; s++) {
+        if (s + 2 < NQ) load_k(s + 2);
+#pragma unroll
+        for (int t = 0; t < 2; t++) sm[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s % 3][t], qf[s], sm[t], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int t = 0; t < 2; t++) Sx[(wave * 2 + t) * 64 + lane] = make_float4(sm[t][0], sm[t][1], sm[t][2], sm[t][3]);
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        const float4 v = Sx[((wave ^ 1) * 2 + t) * 64 + lane];
+        const v4f other = {v.x, v.y, v.z, v.w};
+        st[t] = ds ? other : sm[t];
+        st[2 + t] = ds ? sm[t] : other;
+      }
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) st[t][r] *= p.sm_scale;
+      if (ntok < STEP) {
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            if (16 * t + 4 * g + r >= ntok) st[t][r] = -__builtin_inff();
+      }
+      float mt[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) mt[t] = fmaxf(fmaxf(st[t][0], st[t][1]), fmaxf(st[t][2], st[t][3]));
+      const float m_new = fmaxf(m_run, pf_max_rows(fmaxf(fmaxf(mt[0], mt[1]), fmaxf(mt[2], mt[3]))));   // finite: a step has >= 1 visible token
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) st[t][r] = __expf(st[t][r] - m_new);
+      uint32_t pk[8];
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        mt[t] = (st[t][0] + st[t][1]) + (st[t][2] + st[t][3]);
+        pk[2 * t] = ktx_pk_bf16(st[t][0], st[t][1]);
+        pk[2 * t + 1] = ktx_pk_bf16(st[t][2], st[t][3]);
+      }
+      const float sum = pf_sum_rows((mt[0] + mt[1]) + (mt[2] + mt[3]));
+      const float alpha = __expf(m_run - m_new);
+      l_run = l_run * alpha + sum;
+      m_run = m_new;
+      const v8bf pf[2] = {as_v8bf(make_uint4(pk[0], pk[1], pk[2], pk[3])), as_v8bf(make_uint4(pk[4], pk[5], pk[6], pk[7]))};
+      // the rescale only where some head's running maximum moved (alpha == 1 exactly otherwise)
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0ull) {
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) o[i][r] *= alpha;
+      }
+      // ---- O^T += V^T P^T: transposed reads of the same rows
+      typedef __attribute__((address_space(3))) v4s16 lds_v4;
+      union VFrag { v4s16 h[2]; v8bf v; };
+      VFrag vf[2][4];
+      auto load_v = [&](int j) __attribute__((always_inline)) {
+        const uint8_t* a = kb + (vx ^ (j * 32));
+#pragma unroll
+        for (int q = 0; q < 4; q++) {   // (i, u) = (q >> 1, q & 1)
+          vf[j & 1][q].h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(a + (q >> 1) * 256 + (q & 1) * (32 * MLA_DC * 2)));
+          vf[j & 1][q].h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(a + (q >> 1) * 256 + (q & 1) * (32 * MLA_DC * 2) + 16 * MLA_DC * 2));
+        }
+      };
+      load_v(0);
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        if (j + 1 < 8) load_v(j + 1);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+          for (int i = 0; i < 2; i++) o[i * 8 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j & 1][i * 2 + u].v, pf[u], o[i * 8 + j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  MLA_TS(6);
+
+  const int dim0 = ds * 256 + 4 * g;   // + 16 i
+  if (p.out1) {   // one split holds the whole row: the merge kernel's arithmetic for a single partial (weight 1), in place
+    const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+    bf16_t* po = p.out1 + ((size_t)qt * p.Hq + head) * MLA_DC + dim0;
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+      *reinterpret_cast<uint2*>(po + i * 16) = make_uint2(ktx_pk_bf16(o[i][0] * inv, o[i][1] * inv), ktx_pk_bf16(o[i][2] * inv, o[i][3] * inv));
+    if (p.lse1 && g == 0 && ds == 0)
+      p.lse1[(size_t)qt * p.Hq + head] = l_run > 0.f ? (m_run + __logf(l_run)) * 1.44269504089f : -__builtin_inff();
     return;
   }
-  // ---- partial results: un-normalised O plus (m, l) per head ------------------------------------------------------------
+  // ---- partial results: un-normalised O plus (m, l) per head
+  const size_t pidx = ((size_t)qt * p.Hq + head) * p.nsplit + split;
+  if (g == 0 && ds == 0) *reinterpret_cast<float2*>(p.part_ml + pidx * 2) = make_float2(m_run, l_run);
+  if (t_begin < t_end) {
+    float* po = p.part_o + pidx * MLA_DC + dim0;
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int hrow = (lane >> 4) * 4 + r;
-    if ((lane & 15) == 0 && ds == 0) {
-      float* ml = p.part_ml + (pidx + (size_t)hrow * p.nsplit) * 2;
-      ml[0] = m_run[r];
-      ml[1] = l_run[r];
-    }
-    if (t_begin < t_end) {
-      float* po = p.part_o + (pidx + (size_t)hrow * p.nsplit) * MLA_DC + ds * NDT * 16;
-#pragma unroll
-      for (int i = 0; i < NDT; i++) po[i * 16 + (lane & 15)] = o[i][r];
-    }
+    for (int i = 0; i < 16; i++) *reinterpret_cast<float4*>(po + i * 16) = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
   }
   MLA_TS(7);
 }
@@ -408,7 +757,7 @@ __global__ __launch_bounds__(HBW * DSPLIT * 64) void mla_decode_kernel(MlaParams
 // (m, l) pairs, the partial outputs, the bounds — is issued before the first use: right after the kernel boundary each of
 // them is an L2 miss, and a stats -> weights -> addresses -> loads chain would pay that latency three times over.  A dead
 // split's partial may be stale memory, so it is selected away (not multiplied by 0).
-template <int NS>   // splits per thread: nsplit <= 16 * NS
+template <int NS>   // splits per thread and round
 __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out, float* lse) {
   __shared__ float s_w[1024];
   __shared__ float s_red[8];
@@ -416,6 +765,7 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out
   const int qt = blockIdx.y, h = blockIdx.x, quarter = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int dg = tid & 15, sl = tid >> 4;   // 16 dim groups of 8 dims x 16 split lanes
   const size_t base = ((size_t)qt * p.Hq + h) * p.nsplit;
+  const int nsp = p.jobs ? min(max(p.njobs[qt], 1), p.nsplit) : p.nsplit;   // (no request's token: whatever is there, and nothing is stored)
   // ---- all loads
   int B = p.batch;
   const int bsz_raw = p.d_bsz ? *p.d_bsz : p.batch;
@@ -423,13 +773,13 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int s = tid + i * 256;
-    ml[i] = s < p.nsplit ? *reinterpret_cast<const float2*>(p.part_ml + (base + s) * 2) : make_float2(0.f, 0.f);
+    ml[i] = s < nsp ? *reinterpret_cast<const float2*>(p.part_ml + (base + s) * 2) : make_float2(0.f, 0.f);
   }
   float4 va[NS], vb[NS];
   const float* po = p.part_o + base * MLA_DC + quarter * 128 + dg * 8;
 #pragma unroll
   for (int u = 0; u < NS; u++) {
-    const int s = min(sl + 16 * u, p.nsplit - 1);
+    const int s = min(sl + 16 * u, nsp - 1);
     va[u] = *reinterpret_cast<const float4*>(po + (size_t)s * MLA_DC);
     vb[u] = *reinterpret_cast<const float4*>(po + (size_t)s * MLA_DC + 4);
   }
@@ -450,7 +800,7 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out
   for (int i = 0; i < 4; i++) {
     const int s = tid + i * 256;
     const float w = ml[i].y > 0.f ? __expf(ml[i].x - mstar) : 0.f;
-    if (s < p.nsplit) s_w[s] = w;
+    if (s < nsp) s_w[s] = w;
     lsum += ml[i].y * w;
   }
   lsum = wave_sum(lsum);
@@ -459,14 +809,23 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out
   lsum = (s_red[4] + s_red[5]) + (s_red[6] + s_red[7]);
 
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int c = 0;; c += 16 * NS) {   // (more than one round: a token of the jobs form that holds most of the batch's tiles)
 #pragma unroll
   for (int u = 0; u < NS; u++) {
-    const int s = sl + 16 * u;
-    const float w = s < p.nsplit ? s_w[s] : 0.f;
+    const int s = c + sl + 16 * u;
+    const float w = s < nsp ? s_w[s] : 0.f;
     if (w > 0.f) {
       acc[0] += va[u].x * w; acc[1] += va[u].y * w; acc[2] += va[u].z * w; acc[3] += va[u].w * w;
       acc[4] += vb[u].x * w; acc[5] += vb[u].y * w; acc[6] += vb[u].z * w; acc[7] += vb[u].w * w;
     }
+  }
+  if (c + 16 * NS >= nsp) break;
+#pragma unroll
+  for (int u = 0; u < NS; u++) {
+    const int s = min(c + 16 * NS + sl + 16 * u, nsp - 1);
+    va[u] = *reinterpret_cast<const float4*>(po + (size_t)s * MLA_DC);
+    vb[u] = *reinterpret_cast<const float4*>(po + (size_t)s * MLA_DC + 4);
+  }
   }
 #pragma unroll
   for (int q = 0; q < 8; q++) s_acc[sl][dg * 8 + q] = acc[q];
@@ -554,6 +913,17 @@ extern "C" int ktx_mla_decode_partials(const ktx_mla_config* cfg, const void* d_
                          workspace_bytes, stream, nsplit_out);
 }
 
+// mla_decode_wide_kernel or mla_decode_kernel<4, 2> for a call of the 64-head shape?  The wide one takes 2.5 us for 64 tokens against 5.8 and shares
+// out what the requests hold, but its first step ends 3 us later: it needs some depth.  Measured at (query tokens x 64-token steps of the hint
+// x head blocks), <4, 2> | wide, us with the merge: 80 (8 requests of 300 tokens, 128 heads) 18 | 21, 256 (16 of 1000, 64 heads) 22 | 25, 512: 8 of
+// 2000 26 | 27, 16 of 1000 37 | 31, 1 of 32768 32 | 31, 1024: 4 of 8192 34 | 32, 2048: 8 of 8192 51 | 40.  Past 16 tokens <4, 2> is left with 16
+// splits a token and more workgroups than CUs: 32 of 500, 128 heads 62 | 38, 64 heads 32 | 28, 32 of 4096 110 | 71.
+static bool mla_wide_steps(const ktx_mla_config* cfg, int total_q_tokens, int shape) {
+  if (shape != 4 || total_q_tokens > 64) return false;
+  const long steps = ((long)cfg->kv_len_hint + 2 * MLA_TILE - 1) / (2 * MLA_TILE);
+  return total_q_tokens > 16 || steps * total_q_tokens * (cfg->num_heads / 64) >= 512;
+}
+
 // Workgroup shape and KV split count of a decode call — one place, because the one-launch decode step (ktx_attn.hip) must
 // split the context exactly as the stand-alone kernel does to reproduce its partials bit for bit.
 static void mla_pick_shape(const ktx_mla_config* cfg, int total_q_tokens, size_t workspace_bytes, int* shape_out, int* nsplit_out,
@@ -593,7 +963,8 @@ static void mla_pick_shape(const ktx_mla_config* cfg, int total_q_tokens, size_t
   if (cfg->kv_len_hint > 0) {
     // no more splits than tiles — and no more than the deepest split needs: with T tiles dealt round-robin the launch takes
     // ceil(T / nsplit) tiles' time, so the smallest split count with that depth writes the fewest partials for the merge to read
-    const int tiles = std::max(1, (cfg->kv_len_hint + MLA_TILE - 1) / MLA_TILE);
+    const int unit = mla_wide_steps(cfg, total_q_tokens, shape) ? 2 * MLA_TILE : MLA_TILE;   // (mla_decode_wide_kernel's steps)
+    const int tiles = std::max(1, (cfg->kv_len_hint + unit - 1) / unit);
     nsplit = std::min(nsplit, tiles);
     const int depth = (tiles + nsplit - 1) / nsplit;
     if (ktx_debug_get(7) <= 0) nsplit = (tiles + depth - 1) / depth;
@@ -636,7 +1007,7 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
   const int Hq = cfg->num_heads;
   int shape = 0, nsplit = 0;
   mla_pick_shape(cfg, total_q_tokens, workspace_bytes, &shape, &nsplit);
-  const bool wide = shape == 4;
+  const bool wide = mla_wide_steps(cfg, total_q_tokens, shape);
   const int hbw = shape, nwv = shape == 1 ? 4 : 8;
   const int hblocks = Hq / (16 * hbw);
   KTX_REQUIRE(nsplit >= 1, "ktx_mla_decode: workspace too small");
@@ -657,6 +1028,21 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
   int only = ktx_debug_get(5);   // measurement knob (include/ktx_moe.h): 1 = split-KV kernel only, 2 = merge only
   if (partials_nsplit) { only = 1; *partials_nsplit = nsplit; }   // the caller merges the partials itself (ktx_linear_forward_batched_merge)
   const bool direct = nsplit == 1 && only == 0;
+  // Batches of requests share one workgroup per CU by what they hold: equal splits of unequal contexts wait for the longest, and contexts
+  // shorter than the hint leave workgroups idle (8 requests of 2048 .. 8192 tokens, 128 heads, 5121 on average: 51 us with equal splits of
+  // the form before, 40 so).
+  p.jobs = 0;
+  p.njobs = nullptr;
+  if (wide && !partials_nsplit && nsplit > 1 && total_q_tokens > 1 && total_q_tokens <= 64 && batch <= 64 && ktx_debug_get(7) <= 0) {
+    const size_t rec = (size_t)total_q_tokens * Hq * (MLA_DC + 2) * sizeof(float);   // one split of every token
+    const int jobs = std::max(2 * total_q_tokens, 256 / hblocks);
+    const int cap = (int)std::min<size_t>(std::min(std::min(256, jobs), std::max(1, cfg->max_splits)), (workspace_bytes - (size_t)total_q_tokens * 4) / rec);
+    if (workspace_bytes > (size_t)total_q_tokens * 4 && cap > 1) {
+      p.jobs = jobs; p.nsplit = cap;
+      p.part_ml = p.part_o + (size_t)total_q_tokens * Hq * cap * MLA_DC;
+      p.njobs = reinterpret_cast<int*>(p.part_ml + (size_t)total_q_tokens * Hq * cap * 2);
+    }
+  }
   p.out1 = direct ? (bf16_t*)d_out : nullptr;
   p.lse1 = direct ? d_lse : nullptr;
   p.app_ckv = (const bf16_t*)d_new_ckv; p.app_kpe = (const bf16_t*)d_new_kpe; p.ckv_w = (bf16_t*)d_ckv; p.kpe_w = (bf16_t*)d_k_pe;
@@ -671,12 +1057,18 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
     const hipError_t e2 = ktx_set_max_lds(reinterpret_cast<const void*>(mla_decode_kernel<2, 4>), 128 * 1024);
     KTX_HIP(e2);
     hipLaunchKernelGGL((mla_decode_kernel<2, 4>), grid, dim3(512), lds, st, p);
-  } else if (wide) {
+  } else if (shape == 4 && !wide) {
     KTX_TIMED(st, kv_bytes + (double)total_q_tokens * Hq * (MLA_DC + MLA_DR + MLA_DC) * 2.0,
               "mla_decode_kernel<4,2> T=%d Hq=%d nsplit=%d", total_q_tokens, Hq, nsplit);
     const hipError_t e4 = ktx_set_max_lds(reinterpret_cast<const void*>(mla_decode_kernel<4, 2>), 128 * 1024);
     KTX_HIP(e4);
     hipLaunchKernelGGL((mla_decode_kernel<4, 2>), grid, dim3(512), lds, st, p);
+  } else if (wide) {
+    KTX_TIMED(st, kv_bytes + (double)total_q_tokens * Hq * (MLA_DC + MLA_DR + MLA_DC) * 2.0,
+              "mla_decode_wide_kernel T=%d Hq=%d nsplit=%d", total_q_tokens, Hq, p.nsplit);
+    constexpr size_t lds4 = 2 * 2 * MLA_TILE * (MLA_DC + MLA_DR) * sizeof(bf16_t) + 8 * 2 * 64 * sizeof(float4);   // all of a CU's
+    KTX_HIP(ktx_set_max_lds(reinterpret_cast<const void*>(mla_decode_wide_kernel), 160 * 1024));
+    hipLaunchKernelGGL(mla_decode_wide_kernel, p.jobs ? dim3(p.jobs, hblocks) : grid, dim3(512), lds4, st, p);
   } else {
     KTX_TIMED(st, kv_bytes + (double)total_q_tokens * Hq * (MLA_DC + MLA_DR + MLA_DC) * 2.0,
               "mla_decode_kernel<1,4> T=%d Hq=%d nsplit=%d", total_q_tokens, Hq, nsplit);
@@ -688,9 +1080,10 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
   if (only != 1 && !direct) {
     KTX_TIMED(st, (double)total_q_tokens * Hq * MLA_DC * 2.0, "mla_merge_kernel T=%d Hq=%d nsplit=%d", total_q_tokens, Hq, nsplit);
     const dim3 mg(Hq, total_q_tokens, 4);
-    if (p.nsplit <= 32) hipLaunchKernelGGL(mla_merge_kernel<2>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
-    else if (p.nsplit <= 64) hipLaunchKernelGGL(mla_merge_kernel<4>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
-    else if (p.nsplit <= 144) hipLaunchKernelGGL(mla_merge_kernel<9>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
+    const int ns = p.jobs ? std::min(p.nsplit, 2 * p.jobs / total_q_tokens) : p.nsplit;   // (jobs: twice the mean; the kernel goes on from there)
+    if (ns <= 32) hipLaunchKernelGGL(mla_merge_kernel<2>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
+    else if (ns <= 64) hipLaunchKernelGGL(mla_merge_kernel<4>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
+    else if (ns <= 144) hipLaunchKernelGGL(mla_merge_kernel<9>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
     else hipLaunchKernelGGL(mla_merge_kernel<16>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
   }
   KTX_HIP(hipGetLastError());
@@ -769,29 +1162,6 @@ __device__ __forceinline__ void pf_store_tile(const PfTile& t, bf16_t* Ks, bf16_
   *reinterpret_cast<uint4*>(vd + 32 * PF_VROW) = t.v1;
   *reinterpret_cast<uint4*>(vd + 64 * PF_VROW) = t.v2;
   *reinterpret_cast<uint4*>(vd + 96 * PF_VROW) = t.v3;
-}
-
-// Reductions over the four 16-lane rows of a wavefront (lanes l, l ^ 16, l ^ 32, l ^ 48).  Round 5: gfx950's row swaps — v_permlane32_swap
-// exchanges the upper 32 lanes of one register with the lower 32 of another, v_permlane16_swap the odd rows with the even rows — are
-// plain VALU instructions; the ds_bpermute shuffles they replace are LDS-crossbar round trips, four of them in a dependent chain per
-// query tile and key tile.  Sum: (x_l + x_{l^32}) + (that of l ^ 16) — fp32 addition is commutative, so every lane of a query gets the
-// same bits, and they are the bits the shuffle version produced ((x + shfl16) + shfl32 groups the rows as (r0 + r1) + (r2 + r3) for
-// rows 0 / 1 and likewise here after the 32-swap first: see pf_sum_rows).
-typedef unsigned pf_v2u __attribute__((ext_vector_type(2)));
-typedef float pf_v2f __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float pf_max_rows(float x) {
-  pf_v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float pf_sum_rows(float x) {
-  // the shuffle version computed (x + x^16) first, then + the same of l ^ 32: keep that association — rows (r0 + r1) and (r2 + r3)
-  // first (16-swap), then across the halves (32-swap)
-  pf_v2u r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
 // MINW = wavefronts per SIMD the register allocation must allow.  Unconstrained (MINW = 1) the compiler takes 340 VGPRs: ONE

@@ -61,6 +61,49 @@ def test_ragged_batch_shuffled_pages_page256():
     run_case(128, 256, [700, 5, 2049], [1, 3, 2], seed=3, shuffle_pages=True, rtol=2.0 ** -7)
 
 
+@pytest.mark.parametrize("Hq,page,kv_lens,q_lens,max_splits", [
+    (64, 64, [1, 63, 64, 65, 128, 129, 500, 31, 32, 33] * 2, [1] * 20, 64),   # ends of 64-token steps and of their halves
+    (128, 96, [700, 5, 97, 96, 2049] + [40] * 12, [3, 1, 5, 2, 2] + [1] * 12, 64),   # several query tokens a request, pages of 3 tiles
+    (64, 32, [6000] + [1] * 17, [1] * 18, 64),       # one request holds almost all: its splits are capped, its merge takes several rounds
+    (64, 32, [3000] + [70] * 19, [1] * 20, 256),
+    (128, 64, [300] * 17, [1] * 17, 2),
+    (64, 64, [200] * 17, [1] * 17, 1),               # one split: normalised in place
+])
+def test_batches_that_share_the_workgroups(Hq, page, kv_lens, q_lens, max_splits):
+    run_case(Hq, page, kv_lens, q_lens, seed=len(kv_lens), shuffle_pages=True, max_splits=max_splits, rtol=2.0 ** -7)
+
+
+def test_shared_workgroups_with_append_and_fewer_live_requests():
+    """18 requests of which 17 are live, the newest token of each taken from the append buffers: the live rows equal the oracle's on the
+    appended cache, which ends up updated; the dead request's pages stay as they were."""
+    from ktransformers_amd._native import MLAWrapper
+    g = torch.Generator().manual_seed(19)
+    Hq, page, B, live = 64, 64, 18, 17
+    kv_lens = [130, 64, 1, 65, 128, 700] * 3
+    pages_per = [(n + page - 1) // page for n in kv_lens]
+    kv_buf = torch.randn((sum(pages_per) + 1, page, 576), generator=g).to(torch.bfloat16)
+    q_nope, q_pe = (torch.randn((B, Hq, d), generator=g).to(torch.bfloat16) for d in (512, 64))
+    new_ckv, new_kpe = (torch.randn((B, d), generator=g).to(torch.bfloat16) for d in (512, 64))
+    kv_indices = torch.randperm(sum(pages_per), generator=g).to(torch.int32)
+    kv_indptr = torch.tensor([0] + list(np.cumsum(pages_per)), dtype=torch.int32)
+    qo_indptr, kv_len_arr = torch.arange(B + 1, dtype=torch.int32), torch.tensor(kv_lens, dtype=torch.int32)
+    want = kv_buf.clone()
+    for b in range(live):
+        pos = kv_lens[b] - 1
+        want[int(kv_indices[int(kv_indptr[b]) + pos // page]), pos % page] = torch.cat([new_ckv[b], new_kpe[b]])
+    ref, _ = mla_paged_ref(q_nope, q_pe, want, qo_indptr, kv_indptr, kv_indices, kv_len_arr, 192 ** -0.5)
+    w = MLAWrapper(B, kv_buf.shape[0], device=DEV, max_q_tokens=B)
+    kvd = kv_buf.to(DEV)
+    ckv, k_pe = torch.split(kvd, [512, 64], dim=-1)
+    w.plan(qo_indptr.to(DEV), kv_indptr.to(DEV), kv_indices.to(DEV), kv_len_arr.to(DEV),
+           torch.tensor([live], dtype=torch.int32, device=DEV), Hq, 512, 64, page, 192 ** -0.5)
+    out = w.run(q_nope.to(DEV), q_pe.to(DEV), ckv, k_pe, new_ckv=new_ckv.to(DEV), new_kpe=new_kpe.to(DEV))
+    torch.cuda.synchronize()
+    # kv_len 1: one bf16 ulp (2^-7) of an |out| past 1 exceeds 5e-3
+    torch.testing.assert_close(out[:live].float().cpu(), ref[:live].to(torch.bfloat16).float(), rtol=2.0 ** -7, atol=5e-3)
+    assert torch.equal(kvd.cpu(), want)
+
+
 def test_single_split_equals_many():
     run_case(16, 64, [3000], [1], seed=4, max_splits=1)
 
