@@ -58,6 +58,22 @@ struct Tile {
   int cnt;     // the expert's tiles
 };
 
+// Workgroup -> (tile, strip group) of a grouped GEMM, from a one-dimensional grid: ids are dealt round-robin to the 8 XCDs, so id % 8 is the
+// XCD.  The jobs lie expert after expert, within an expert strip group by strip group, the group's tiles side by side; each XCD takes an
+// eighth of them.  So the XCDs end together whatever the number of tiles, an expert's weights go into one L2 and are read there once for all
+// its tiles, and its rows (the operand every strip group re-reads) stay there too.  False: nothing to do.
+__device__ __forceinline__ bool moe_pick_job(const Tile* tiles, int ntiles, int nsg, Tile& tile, int& sgroup) {
+  const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
+  const int total = ntiles * nsg, per = (total + 7) / 8, job = xcd * per + seq;
+  if (seq >= per || job >= total) return false;
+  tile = tiles[job / nsg];
+  const int first = job / nsg - tile.idx, ofs = job - first * nsg;
+  sgroup = ofs / tile.cnt;
+  if (tile.cnt > 1) tile = tiles[first + ofs % tile.cnt];
+  return true;
+}
+static dim3 moe_job_grid(int max_tiles, int nsg) { return dim3((unsigned)(((size_t)max_tiles * nsg + 7) / 8 * 8)); }
+
 // =====================================================================================================
 // K0: prep — block 0 buckets (t,j) pairs by expert; blocks 1.. quantise one token's activations (a5, a6)
 // =====================================================================================================
@@ -1239,7 +1255,7 @@ __global__ void pack_w8_kernel(const int8_t* __restrict__ q, int N, int K, uint3
 // W tile layout for these formats (k-step = 128, four 16x16x32 MFMAs j = 0..3; fragment element e <-> k = ks*128 +
 // kc*32 + j*8 + e):  FP8: tile 2048 B, lane l owns bytes [l*16, +16) of each of two 1 KiB halves (elements 0..15, 16..31
 // of its 32-k run);  BF16: tile 4096 B, four 1 KiB quarters, quarter j = the lane's fragment for MFMA j.
-// Activations are staged per 256-k chunk as [mt][col = 32][tok = 16][16 B] (same conflict-free scheme as the int path).
+// Activations are staged per 256-k chunk, row by row, by LDS-DMA.
 // =====================================================================================================
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
@@ -1275,30 +1291,30 @@ struct FpGemmParams {
   bf16_t* out;                // [sorted rows][N]
 };
 
-// WIDE (round 4, the prompt configuration MT = 4): 8 wavefronts per workgroup and two B operands per wavefront for BOTH GEMMs (gate and up
-// of a strip; two strips of down).  At 64 rows per expert every weight byte is read once, but every workgroup re-reads the tile's
-// bf16 activations — with 4 strips per workgroup that was as many bytes as the fp8 weights themselves (7.5 GB against 6.4 GB per
-// DeepSeek-V3 gate|up layer; 3.5x the weights for down) and the kernel ran at the CUs' ingest rate, not HBM's (profiles/r04_bench2).
-// Per output the arithmetic is unchanged (same MFMA chain per 128-k group, same scale fma): bit-identical results.
+// the places of a row's pieces: distinct for 16 rows, also with rows 4 .. 11 flipped by 4 (ds_read_b128 takes lanes 0-3, 12-15, 20-23, 24-27 together)
+__device__ __forceinline__ int fp_swz(int row) { return (row & 3) | (int)((0x3102u >> (((row >> 2) & 3) * 4)) & 3u) << 2; }
+// WIDE (MT = 4): 8 wavefronts per workgroup and two B operands per wavefront for BOTH GEMMs (gate and up of a strip; two strips of down): at 64
+// rows every workgroup re-reads the tile's bf16 activations, with 4 strips as many bytes as the fp8 weights themselves.  At 32 rows 4 strips and
+// three wavefronts a SIMD are ahead (DeepSeek-V3 shape, 1000 tokens: 2307 us against 2587 of the wide form).
+// Bound by the weights' way in at few rows (64 tokens 1072 us, the weights alone 1066 at the rate of a large copy), past 16 rows an expert by waves too few to
+// cover widening, LDS reads and MFMAs with the next chunk's loads.  Those used to be waited for in the chunk that requested them: 1000 tokens
+// 2454 -> 2241 us, 64 experts of 2048 x 1408 with 94 rows each 279 -> 250, 8 of 4096 x 1536 with 375 rows 232 -> 212.
 template <bool FP8, int MT, bool GATE_UP, bool WIDE = false>
-__global__ __launch_bounds__(WIDE ? 512 : 256) void moe_gemm_fp_kernel(FpGemmParams p) {
+__global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 2 : MT == 2 ? 3 : 1) void moe_gemm_fp_kernel(FpGemmParams p) {
   constexpr int NMAT = (GATE_UP || WIDE) ? 2 : 1;      // B operands (units) per wavefront
   constexpr int NWV = WIDE ? 8 : 4;
   constexpr int SPC = 2;                      // k-steps per chunk
-  constexpr int COLS = SPC * 16;              // 16-byte columns per chunk (128 bf16 = 256 B per step)
-  constexpr int BUF_BYTES = MT * COLS * 256;
-  constexpr int GROUPS = MT * COLS / 4;       // staging groups of (16 tok x 4 cols)
-  constexpr int UPT = (GROUPS + NWV - 1) / NWV;
+  constexpr int BUF_BYTES = MT * 16 * 512;    // activations of a chunk: 256 k of every row
   constexpr int TILE_BYTES = FP8 ? 2048 : 4096;
   constexpr int NQ = FP8 ? 2 : 4;             // uint4 per lane per k-step per matrix
 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  uint8_t* Bs = smem;                                            // [2][BUF_BYTES]
+  uint8_t* Bs = smem;                                            // [2][row][32 pieces of 16 B, the low 4 bits of the place ^ fp_swz(row)]
   int* s_src = reinterpret_cast<int*>(smem + 2 * BUF_BYTES);     // [MT*16]
 
-  const int tile_idx = blockIdx.y;
-  if (tile_idx >= p.counters[0]) return;
-  const Tile tile = p.tiles[tile_idx];
+  Tile tile;
+  int sgroup;
+  if (!moe_pick_job(p.tiles, p.counters[0], (p.N / 16 + NWV * (GATE_UP ? 1 : NMAT) - 1) / (NWV * (GATE_UP ? 1 : NMAT)), tile, sgroup)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int NKS = p.K / 128;
@@ -1307,12 +1323,15 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void moe_gemm_fp_kernel(FpGemmPar
   bool uok[NMAT];
 #pragma unroll
   for (int m = 0; m < NMAT; m++) {
-    ustrip[m] = GATE_UP ? blockIdx.x * NWV + wave : (WIDE ? (blockIdx.x * NWV + wave) * 2 + m : blockIdx.x * NWV + wave);
+    ustrip[m] = GATE_UP || !WIDE ? sgroup * NWV + wave : (sgroup * NWV + wave) * 2 + m;
     uok[m] = ustrip[m] * 16 < p.N;
   }
   const bool strip_ok = uok[0];      // (a wavefront's second strip of down can only be missing when the first is present)
 
-  if (tid < MT * 16) s_src[tid] = tid < tile.nrows ? (p.row_src ? p.row_src[tile.row0 + tid] : tile.row0 + tid) : -1;
+  if (tid < MT * 16) {   // rows past the tile read its first row again (never stored)
+    const int r = tile.row0 + (tid < tile.nrows ? tid : 0);
+    s_src[tid] = p.row_src ? p.row_src[r] : r;
+  }
   __syncthreads();
 
   const uint8_t* wbase[NMAT];
@@ -1332,114 +1351,111 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void moe_gemm_fp_kernel(FpGemmPar
 #pragma unroll
     for (int t = 0; t < MT; t++) acc[m][t] = v4f{0.f, 0.f, 0.f, 0.f};
 
-  uint4 wA[SPC][NMAT][NQ], wB[SPC][NMAT][NQ];
-  uint4 breg[UPT];
-
-  auto load_w = [&](uint4(&dst)[SPC][NMAT][NQ], int c) {
+  // The weights of a chunk: a k-step's registers are requested again for the next chunk as soon as they are widened.  Loads and settle are
+  // unconditional (the last chunk's requests repeat, an odd last k-step repeats its neighbour): under branches the compiler cannot count the loads
+  // and waited for the chunk just requested, a memory round trip per chunk.
+  uint4 w[SPC][NMAT][NQ];
+  float sc[SPC][NMAT];
+  auto load_w = [&](int s, int c) {
+    const int ks = min(c * SPC + s, NKS - 1);
+#pragma unroll
+    for (int m = 0; m < NMAT; m++) {
+#pragma unroll
+      for (int q = 0; q < NQ; q++) w[s][m][q] = *reinterpret_cast<const uint4*>(wbase[m] + (size_t)ks * TILE_BYTES + q * 1024 + lane * 16);
+      if constexpr (FP8) sc[s][m] = sbase[m][ks];
+    }
+  };
+  auto settle = [&]() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int s = 0; s < SPC; s++)
+#pragma unroll
+      for (int m = 0; m < NMAT; m++) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) asm volatile("" : "+v"(w[s][m][q].x), "+v"(w[s][m][q].y), "+v"(w[s][m][q].z), "+v"(w[s][m][q].w));
+        if constexpr (FP8) asm volatile("" : "+v"(sc[s][m]));
+      }
+  };
+  // activations by LDS-DMA, two rows of 512 B a wave-instruction
+  constexpr int DPW = MT * 8 / NWV;
+  const uint32_t lds_b = (uint32_t)(uintptr_t)Bs;
+  const bf16_t* arow[DPW];
+  int apc[DPW];
+#pragma unroll
+  for (int i = 0; i < DPW; i++) {
+    const int row = (wave * DPW + i) * 2 + (lane >> 5), slot = lane & 31;
+    apc[i] = ((slot & 16) | ((slot ^ fp_swz(row)) & 15)) * 8;
+    arow[i] = p.act + (size_t)s_src[row] * p.K;
+  }
+  auto stage = [&](int c, int buf) {
+#pragma unroll
+    for (int i = 0; i < DPW; i++) {
+      const int k = c * SPC * 128 + apc[i];
+      moe_dma(arow[i] + (k < p.K ? k : 0), lds_b + buf * BUF_BYTES + (wave * DPW + i) * 1024);   // (behind an odd last k-step: not used)
+    }
+  };
+  // B fragment of MFMA j in step s: token lane & 15, piece s * 16 + kc * 4 + j
+  const int frow = lane & 15;
+  const uint32_t xo = frow * 512 + (((lane >> 4) * 4) ^ fp_swz(frow)) * 16;
+  auto chunk = [&](int c, int buf) __attribute__((always_inline)) {
+    const int nc = min(c + 1, NC - 1);
+    stage(nc, buf ^ 1);
+    const uint8_t* bb = Bs + buf * BUF_BYTES;
 #pragma unroll
     for (int s = 0; s < SPC; s++) {
-      const int ks = c * SPC + s;
-      if (strip_ok && ks < NKS) {
+      v8bf a[NMAT][4];
+      float csc[NMAT];
 #pragma unroll
-        for (int m = 0; m < NMAT; m++)
+      for (int m = 0; m < NMAT; m++) {
+        csc[m] = FP8 ? sc[s][m] : 1.0f;
+        if constexpr (FP8) {
 #pragma unroll
-          for (int q = 0; q < NQ; q++)
-            dst[s][m][q] = *reinterpret_cast<const uint4*>(wbase[m] + (size_t)ks * TILE_BYTES + q * 1024 + lane * 16);
+          for (int q = 0; q < 2; q++) {
+            const uint2 e0 = fp8x4_to_bf16x4(w[s][m][q].x), e1 = fp8x4_to_bf16x4(w[s][m][q].y);
+            const uint2 e2 = fp8x4_to_bf16x4(w[s][m][q].z), e3 = fp8x4_to_bf16x4(w[s][m][q].w);
+            a[m][q * 2] = u4_as_v8bf(make_uint4(e0.x, e0.y, e1.x, e1.y));
+            a[m][q * 2 + 1] = u4_as_v8bf(make_uint4(e2.x, e2.y, e3.x, e3.y));
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; j++) a[m][j] = u4_as_v8bf(w[s][m][j]);
+        }
       }
-    }
-  };
-  auto load_b = [&](int c) {
+      load_w(s, nc);
+      if (s > 0 && c * SPC + s >= NKS) break;   // an odd last k-step
 #pragma unroll
-    for (int it = 0; it < UPT; it++) {
-      const int g = it * NWV + wave;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (g < GROUPS) {
-        const int mt = g / (COLS / 4), col = (g % (COLS / 4)) * 4 + (lane >> 4);
-        const int src = s_src[mt * 16 + (lane & 15)];
-        const int kb = c * SPC * 128 + col * 8;   // bf16 element index of this 16-byte column
-        if (src >= 0 && kb < p.K) v = *reinterpret_cast<const uint4*>(p.act + (size_t)src * p.K + kb);
-      }
-      breg[it] = v;
-    }
-  };
-  auto store_b = [&](int buf) {
+      for (int t = 0; t < MT; t++) {
+        v8bf b[4];
 #pragma unroll
-    for (int it = 0; it < UPT; it++) {
-      const int g = it * NWV + wave;
-      if (g < GROUPS) {
-        const int mt = g / (COLS / 4), col = (g % (COLS / 4)) * 4 + (lane >> 4);
-        *reinterpret_cast<uint4*>(Bs + buf * BUF_BYTES + ((mt * COLS + col) * 16 + (lane & 15)) * 16) = breg[it];
-      }
-    }
-  };
-  auto compute = [&](uint4(&w)[SPC][NMAT][NQ], int c, int buf) {
-    if (!strip_ok) return;
-    // B fragment of MFMA j in step s: column s*16 + kc*4 + j, token lane&15
-    const uint8_t* bb = Bs + buf * BUF_BYTES + ((lane >> 4) * 4 * 16 + (lane & 15)) * 16;
+        for (int j = 0; j < 4; j++) b[j] = u4_as_v8bf(*reinterpret_cast<const uint4*>(bb + t * 8192 + s * 256 + (xo ^ (j * 16))));
+        v4f tmp[NMAT];
 #pragma unroll
-    for (int s = 0; s < SPC; s++) {
-      const int ks = c * SPC + s;
-      if (ks < NKS) {
-        v8bf a[NMAT][4];
+        for (int m = 0; m < NMAT; m++) tmp[m] = FP8 ? v4f{0.f, 0.f, 0.f, 0.f} : acc[m][t];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int m = 0; m < NMAT; m++) tmp[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m][j], b[j], tmp[m], 0, 0, 0);
 #pragma unroll
         for (int m = 0; m < NMAT; m++) {
           if constexpr (FP8) {
 #pragma unroll
-            for (int q = 0; q < 2; q++) {
-              const uint2 e0 = fp8x4_to_bf16x4(w[s][m][q].x), e1 = fp8x4_to_bf16x4(w[s][m][q].y);
-              const uint2 e2 = fp8x4_to_bf16x4(w[s][m][q].z), e3 = fp8x4_to_bf16x4(w[s][m][q].w);
-              a[m][q * 2] = u4_as_v8bf(make_uint4(e0.x, e0.y, e1.x, e1.y));
-              a[m][q * 2 + 1] = u4_as_v8bf(make_uint4(e2.x, e2.y, e3.x, e3.y));
-            }
+            for (int r = 0; r < 4; r++) acc[m][t][r] = fmaf(tmp[m][r], csc[m], acc[m][t][r]);  // apply_scale_kgroup
           } else {
-#pragma unroll
-            for (int j = 0; j < 4; j++) a[m][j] = u4_as_v8bf(w[s][m][j]);
-          }
-        }
-        float sc[NMAT];
-#pragma unroll
-        for (int m = 0; m < NMAT; m++) sc[m] = FP8 ? sbase[m][ks] : 1.0f;
-#pragma unroll
-        for (int t = 0; t < MT; t++) {
-          v4f tmp[NMAT];
-#pragma unroll
-          for (int m = 0; m < NMAT; m++) tmp[m] = FP8 ? v4f{0.f, 0.f, 0.f, 0.f} : acc[m][t];
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const v8bf b = u4_as_v8bf(*reinterpret_cast<const uint4*>(bb + ((t * COLS + s * 16 + j) * 16) * 16));
-#pragma unroll
-            for (int m = 0; m < NMAT; m++) tmp[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m][j], b, tmp[m], 0, 0, 0);
-          }
-#pragma unroll
-          for (int m = 0; m < NMAT; m++) {
-            if constexpr (FP8) {
-#pragma unroll
-              for (int r = 0; r < 4; r++) acc[m][t][r] = fmaf(tmp[m][r], sc[m], acc[m][t][r]);  // apply_scale_kgroup
-            } else {
-              acc[m][t] = tmp[m];
-            }
+            acc[m][t] = tmp[m];
           }
         }
       }
     }
+    settle();
+    __syncthreads();
   };
 
-  load_w(wA, 0);
-  load_b(0);
-  store_b(0);
+  stage(0, 0);
+#pragma unroll
+  for (int s = 0; s < SPC; s++) load_w(s, 0);
+  settle();
   __syncthreads();
-  for (int c = 0; c < NC; c += 2) {
-    if (c + 1 < NC) { load_b(c + 1); load_w(wB, c + 1); }
-    compute(wA, c, 0);
-    if (c + 1 < NC) store_b(1);
-    __syncthreads();
-    if (c + 1 < NC) {
-      if (c + 2 < NC) { load_b(c + 2); load_w(wA, c + 2); }
-      compute(wB, c + 1, 1);
-      if (c + 2 < NC) store_b(0);
-      __syncthreads();
-    }
-  }
+  for (int c = 0; c < NC; c++) chunk(c, c & 1);
 
   if (!strip_ok) return;
   const int tok = lane & 15;
@@ -2998,7 +3014,7 @@ static int launch_gemm_fp(int mt, const FpGemmParams& p, int max_tiles, hipStrea
     constexpr size_t lds = 2 * (MT * 32 * 256) + MT * 16 * sizeof(int);                                                       \
     const hipError_t err = ktx_set_max_lds(reinterpret_cast<const void*>(moe_gemm_fp_kernel<FP8, MT, GATE_UP, WIDE>), (int)lds);                        \
     KTX_HIP(err);                                                                                                             \
-    hipLaunchKernelGGL((moe_gemm_fp_kernel<FP8, MT, GATE_UP, WIDE>), dim3((nstrips + PER_WG - 1) / PER_WG, max_tiles), dim3(NTH), lds, st, p); \
+    hipLaunchKernelGGL((moe_gemm_fp_kernel<FP8, MT, GATE_UP, WIDE>), moe_job_grid(max_tiles, (nstrips + PER_WG - 1) / PER_WG), dim3(NTH), lds, st, p); \
   } while (0)
   if (mt == 1) KTX_FP_LAUNCH(1, false, 4, 256);
   else if (mt == 2) KTX_FP_LAUNCH(2, false, 4, 256);
@@ -3328,8 +3344,12 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
   Workspace* ws = h->ws;
   const int E = h->cfg.expert_num, H = h->cfg.hidden_size, I = h->cfg.intermediate_size;
   const bool fp8 = h->cfg.format == KTX_FMT_FP8 || h->cfg.format == KTX_FMT_FP8_PERCHANNEL;   // per-channel: block scales = 1 + row scales
-  const int mt = std::min(4, pick_mt(qlen, k, E));
   const int npairs = qlen * k;
+  // Rows per tile.  Measured (us, 16 | 32 | 64 rows): 256 experts of 7168 x 2048 with 3.1 rows each 1214 | 1202 | 1382, 15.6: 1981 | 1823 | 2029,
+  // 47: 3423 | 2873 | 2944, 62: 4142 | 3353 | 3290; 64 of 2048 x 1408, 9.4: 115 | 116 | 135, 66: 245 | 206 | 223, 94: 312 | 251 | 259, 141: 431 | 349 | 340;
+  // 8 of 4096 x 1536, 25: 56 | 55 | 74, 75: 88 | 80 | 76, 250: 196 | 160 | 155
+  const double rows = (double)npairs / std::max(1, E);
+  const int mt = rows <= 2.5 ? 1 : rows <= 60.0 ? 2 : 4;
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
 
   // ---- decode fast path: two launches (see moe_dec_fp_gateup_kernel) ------------------------------------------------------
@@ -3619,7 +3639,7 @@ static int launch_gguf(const GgGemmParams& p, int max_tiles, hipStream_t st) {
   constexpr int TOK = MT * 16, US = TOK * 16 + 16, NBS = gg_nbs(WT);
   const size_t lds = 2 * 16 * US + 2 * NBS * TOK * 4 + 2 * TOK * 4 + TOK * 4 + (WT == GG_IQ1S ? 4096 * 8 : 0);
   const dim3 grid((p.N / 16 + 3) / 4, max_tiles);
-  const dim3 grid_f((unsigned)((p.N / 16 + 3) / 4) * (unsigned)((max_tiles + 7) / 8 * 8));   // folded kernels: (XCD, tile, strip group) in one dimension
+  const dim3 grid_f = moe_job_grid(max_tiles, (p.N / 16 + 3) / 4);
   if constexpr (gg_foldable(WT)) {   // round 6: the folded-operand kernel; dev knob [21] = 1: gg_block's (the bit-identity test, A/B timing)
     if (g_dbg[21] != 1) {
       const size_t lds_f = 2 * TOK * 256 + 2 * TOK * 4 + TOK * 4 + (WT == GG_Q4K ? 2 * TOK * 32 : WT == GG_IQ1S ? 2 * TOK * 4 + 16384 : 0);

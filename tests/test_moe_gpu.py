@@ -667,3 +667,30 @@ def test_batches_that_share_experts_take_the_grouped_kernels(dev, method):
         assert ((got - want).abs() <= want.abs() * 2.0 ** -7 + want.square().mean().sqrt() * 160 * 2.0 ** -24).all()
     else:
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("fmt", ["FP8", "BF16"])
+@pytest.mark.parametrize("H,I", [(128, 128), (384, 640), (256, 1152)])
+@pytest.mark.parametrize("rows", [(1, 0, 2, 3), (33, 0, 1, 32), (65, 0, 257, 16)])
+def test_fp_grouped_edges(oracle, dev, fmt, H, I, rows):
+    """The grouped kernels at each tile height (2.5 and 60 rows an expert on average divide them): odd numbers of 128-k steps, one step, experts
+    without rows, of one row past a tile, of several tiles (the XCDs' shares cut through them), strip groups that are not full."""
+    from helpers import fp8_block_quant
+    from ktransformers_amd import _native
+    E, k, T = len(rows), 1, sum(rows)
+    c = make_case(41, E, k, H, I, T)
+    c["ids"] = np.random.default_rng(T).permutation(np.repeat(np.arange(E), rows)).astype(np.int64)[:, None]
+    h = _native.MoEHandle(E, k, H, I, max_len=max(T, 8), method=fmt, device=0, group_size=128 if fmt == "FP8" else 0)
+    try:
+        if fmt == "FP8":
+            q = [fp8_block_quant(bf16_to_f32(c[n])) for n in ("gate", "up", "down")]
+            mo = oracle.make_moe_fp8(q[0][0], q[1][0], q[2][0], q[0][1], q[1][1], q[2][1])
+            h.load_fp8(*[torch.from_numpy(x[0]).to(dev) for x in q], *[torch.from_numpy(x[1]).to(dev) for x in q])
+        else:
+            mo = oracle.make_moe_bf16(c["gate"], c["up"], c["down"])
+            h.load_bf16(torch_bf16(c["gate"], dev), torch_bf16(c["up"], dev), torch_bf16(c["down"], dev))
+        _native.force_generic_path(True)
+        _check_fp(run(h, c, dev), oracle.moe_forward(mo, c["ids"], c["w"], c["x"]))
+    finally:
+        _native.force_generic_path(False)
+        h.close()
