@@ -370,49 +370,46 @@ struct GemmParams {
   bf16_t* out;  // [sorted rows][N]
 };
 
+// Four strips of 16 weight rows (x gate, up) against a tile of MT x 16 rows, chunk by chunk of SPC k-steps.  At few rows the weights' way in bounds it
+// (256 experts of 7168 x 2048, 32 tokens: 396 us, 6 TB/s); past 16 rows the LDS reads and barriers beside MFMAs that 3-4 wavefronts a SIMD do not
+// hide.  Requests that outlive their chunk, activations by LDS-DMA and an expert's tiles side by side on one XCD: 8 experts of 4096 x 1536, 100 rows
+// each 63 -> 53 us, 64 of 2048 x 1408, 75: 166 -> 138, 37: 120 -> 109.
 template <int WBITS, int MT, int SPC, bool GATE_UP>
 __global__ __launch_bounds__(256) void moe_gemm_kernel(GemmParams p) {
   constexpr int NMAT = GATE_UP ? 2 : 1;
   constexpr int KC = SPC * 128;
-  constexpr int COLS = KC / 16;                       // 16-byte columns per chunk
-  constexpr int BUF_BYTES = MT * COLS * 256;          // one LDS activation buffer
-  constexpr int GROUPS = MT * SPC * 2;                // staging groups of (16 tok x 4 cols)
-  constexpr int UPT = (GROUPS + 3) / 4;               // staging units per thread
+  constexpr int BUF_BYTES = MT * 16 * KC;             // one LDS activation buffer
+  constexpr int PPR = KC / 16;                        // 16-byte pieces per row and chunk
+  constexpr int DPW = MT * SPC / 2;                   // DMA instructions per wavefront and chunk (64 / PPR rows each)
   constexpr int TILE_BYTES = (WBITS == 4) ? 1024 : 2048;
 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  uint8_t* Bs = smem;                                               // [2][BUF_BYTES]
+  uint8_t* Bs = smem;                                               // [2][row][PPR pieces of 16 B, the low 4 bits of the place ^ row]
   float* s_ad = reinterpret_cast<float*>(smem + 2 * BUF_BYTES);     // [MT*16]
   int* s_src = reinterpret_cast<int*>(s_ad + MT * 16);              // [MT*16]
 
-  // (an XCD-aware remap that runs the 3-4 token tiles sharing an expert's weight strips back to back on one XCD was
-  // measured: no change at T = 2048 — the re-reads are absorbed by the 256 MB Infinity Cache; the kernel is bound by the
-  // one-chunk prefetch distance)
-  const int tile_idx = blockIdx.y;
-  if (tile_idx >= p.counters[0]) return;
-  const Tile tile = p.tiles[tile_idx];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int strip = blockIdx.x * 4 + wave;
+  Tile tile;
+  int sgroup;
+  if (!moe_pick_job(p.tiles, p.counters[0], (p.N / 16 + 3) / 4, tile, sgroup)) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int strip = sgroup * 4 + wave;
   const int NKS = p.K / 128;
   const int NC = (NKS + SPC - 1) / SPC;
   const bool strip_ok = strip * 16 < p.N;  // wave-uniform
 
-  // rows of this tile: source row + activation scale
+  // rows of this tile: source row + activation scale; rows past it read its first row again (never stored)
   if (tid < MT * 16) {
-    int src = -1;
-    float ad = 0.0f;
-    if (tid < tile.nrows) {
-      src = p.row_src ? p.row_src[tile.row0 + tid] : (tile.row0 + tid);
-      ad = p.act_d[src];
-    }
+    const int r = tile.row0 + (tid < tile.nrows ? tid : 0), src = p.row_src ? p.row_src[r] : r;
     s_src[tid] = src;
-    s_ad[tid] = ad;
+    s_ad[tid] = p.act_d[src];
   }
   __syncthreads();
 
   const uint8_t* wbase[NMAT];
-  wbase[0] = p.w0 + (size_t)tile.expert * p.expert_stride + (size_t)strip * NKS * TILE_BYTES;
-  if constexpr (GATE_UP) wbase[1] = p.w1 + (size_t)tile.expert * p.expert_stride + (size_t)strip * NKS * TILE_BYTES;
+  const size_t wofs = (size_t)tile.expert * p.expert_stride + (size_t)(strip_ok ? strip : 0) * NKS * TILE_BYTES;   // (a strip past N aliases strip 0, not stored)
+  wbase[0] = p.w0 + wofs;
+  if constexpr (GATE_UP) wbase[1] = p.w1 + wofs;
 
   v4i acc[NMAT][MT];
 #pragma unroll
@@ -420,95 +417,78 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(GemmParams p) {
 #pragma unroll
     for (int t = 0; t < MT; t++) acc[m][t] = v4i{0, 0, 0, 0};
 
-  WFrag<WBITS> wA[SPC][NMAT], wB[SPC][NMAT];
-  uint4 breg[UPT];
-
-  auto load_w = [&](WFrag<WBITS>(&dst)[SPC][NMAT], int c) {
+  // The weights of a chunk: a k-step's registers are requested again for the next chunk as soon as they are unpacked.  Loads and settle are
+  // unconditional (the last chunk's requests repeat): under branches the compiler cannot count the loads and waits for the chunk just requested.
+  WFrag<WBITS> w[SPC][NMAT];
+  auto load_w = [&](int s, int c) {
+    const int ks = min(c * SPC + s, NKS - 1);
 #pragma unroll
-    for (int s = 0; s < SPC; s++) {
-      const int ks = c * SPC + s;
-      if (strip_ok && ks < NKS) {
-#pragma unroll
-        for (int m = 0; m < NMAT; m++) dst[s][m] = load_wfrag<WBITS>(wbase[m] + (size_t)ks * TILE_BYTES, lane);
-      }
-    }
+    for (int m = 0; m < NMAT; m++) w[s][m] = load_wfrag<WBITS>(wbase[m] + (size_t)ks * TILE_BYTES, lane);
   };
-  // staging unit `it` of this thread: a fixed (token row, 16-byte column) — its global row pointer and LDS slot are
-  // computed once, the chunk loop only adds c*KC (the per-chunk address arithmetic was ~1/4 of the kernel's instructions)
-  const int8_t* gsrc[UPT];
-  int gcol[UPT], lds_off[UPT];
+  auto settle = [&]() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 #pragma unroll
-  for (int it = 0; it < UPT; it++) {
-    const int g = it * 4 + wave;
-    gsrc[it] = nullptr;
-    gcol[it] = 0;
-    lds_off[it] = 0;
-    if (g < GROUPS) {
-      const int mt = g / (SPC * 2), col = (g % (SPC * 2)) * 4 + (lane >> 4);
-      const int src = s_src[mt * 16 + (lane & 15)];
-      gcol[it] = col * 16;
-      lds_off[it] = ((mt * COLS + col) * 16 + (lane & 15)) * 16;
-      if (src >= 0) gsrc[it] = p.act_q + (size_t)src * p.K + col * 16;
-    }
+    for (int s = 0; s < SPC; s++)
+#pragma unroll
+      for (int m = 0; m < NMAT; m++) settle_wfrag<WBITS>(w[s][m]);
+  };
+  // activations by LDS-DMA
+  const uint32_t lds_b = (uint32_t)(uintptr_t)Bs;
+  const int8_t* arow[DPW];
+  int apc[DPW];
+#pragma unroll
+  for (int i = 0; i < DPW; i++) {
+    const int row = (wave * DPW + i) * (64 / PPR) + lane / PPR, slot = lane % PPR;
+    apc[i] = ((slot & ~15) | ((slot ^ row) & 15)) * 16;
+    arow[i] = p.act_q + (size_t)s_src[row] * p.K;
   }
-  auto load_b = [&](int c) {
+  auto stage = [&](int c, int buf) {
 #pragma unroll
-    for (int it = 0; it < UPT; it++) {
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (gsrc[it] && c * KC + gcol[it] < p.K) v = *reinterpret_cast<const uint4*>(gsrc[it] + c * KC);
-      breg[it] = v;
+    for (int i = 0; i < DPW; i++) {
+      const int k = c * KC + apc[i];
+      moe_dma(arow[i] + (k < p.K ? k : 0), lds_b + buf * BUF_BYTES + (wave * DPW + i) * 1024);   // (behind the last k-step: not used)
     }
   };
-  auto store_b = [&](int buf) {
-#pragma unroll
-    for (int it = 0; it < UPT; it++)
-      if (it * 4 + wave < GROUPS) *reinterpret_cast<uint4*>(Bs + buf * BUF_BYTES + lds_off[it]) = breg[it];
-  };
-  auto compute = [&](WFrag<WBITS>(&w)[SPC][NMAT], int c, int buf) {
-    if (!strip_ok) return;
-    const uint8_t* bb = Bs + buf * BUF_BYTES + ((lane >> 4) * 2 * 16 + (lane & 15)) * 16;
+  // fragment h of k-step s: token lane & 15, piece s * 8 + kc * 2 + h
+  const int frow = lane & 15;
+  const uint32_t xo = frow * KC + (((lane >> 4) * 2) ^ frow) * 16;
+  auto chunk = [&](int c, int buf) __attribute__((always_inline)) {
+    const int nc = min(c + 1, NC - 1);
+    stage(nc, buf ^ 1);
+    const uint8_t* bb = Bs + buf * BUF_BYTES;
 #pragma unroll
     for (int s = 0; s < SPC; s++) {
-      if (c * SPC + s < NKS) {
-        v4i a[NMAT][2];
+      v4i a[NMAT][2];
 #pragma unroll
-        for (int m = 0; m < NMAT; m++) unpack_wfrag<WBITS>(w[s][m], a[m][0], a[m][1]);
-        // both halves of every (matrix, token-tile) accumulator are issued a full round apart: back-to-back MFMAs on the
-        // same accumulator would each wait out the previous one's latency
-        v4i b[MT][2];
+      for (int m = 0; m < NMAT; m++) unpack_wfrag<WBITS>(w[s][m], a[m][0], a[m][1]);
+      load_w(s, nc);
+      if (s > 0 && c * SPC + s >= NKS) break;
+      // both halves of every (matrix, token-tile) accumulator are issued a full round apart: back-to-back MFMAs on the
+      // same accumulator would each wait out the previous one's latency
+      v4i b[MT][2];
 #pragma unroll
-        for (int t = 0; t < MT; t++) {
-          b[t][0] = *reinterpret_cast<const v4i*>(bb + ((t * COLS + s * 8) * 16) * 16);
-          b[t][1] = *reinterpret_cast<const v4i*>(bb + ((t * COLS + s * 8 + 1) * 16) * 16);
-        }
+      for (int t = 0; t < MT; t++)
 #pragma unroll
         for (int hh = 0; hh < 2; hh++)
+          b[t][hh] = *reinterpret_cast<const v4i*>(bb + t * 16 * KC + (s >> 1) * 256 + (xo ^ ((s & 1) * 128 + hh * 16)));
 #pragma unroll
-          for (int t = 0; t < MT; t++)
+      for (int hh = 0; hh < 2; hh++)
 #pragma unroll
-            for (int m = 0; m < NMAT; m++)
-              acc[m][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[m][hh], b[t][hh], acc[m][t], 0, 0, 0);
-      }
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+          for (int m = 0; m < NMAT; m++)
+            acc[m][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[m][hh], b[t][hh], acc[m][t], 0, 0, 0);
     }
+    settle();
+    __syncthreads();
   };
 
-  // ---- software pipeline: weights for chunk c+1 and activations for chunk c+1 are in flight while chunk c computes
-  load_w(wA, 0);
-  load_b(0);
-  store_b(0);
+  stage(0, 0);
+#pragma unroll
+  for (int s = 0; s < SPC; s++) load_w(s, 0);
+  settle();
   __syncthreads();
-  for (int c = 0; c < NC; c += 2) {
-    if (c + 1 < NC) { load_b(c + 1); load_w(wB, c + 1); }
-    compute(wA, c, 0);
-    if (c + 1 < NC) store_b(1);
-    __syncthreads();
-    if (c + 1 < NC) {
-      if (c + 2 < NC) { load_b(c + 2); load_w(wA, c + 2); }
-      compute(wB, c + 1, 1);
-      if (c + 2 < NC) store_b(0);
-      __syncthreads();
-    }
-  }
+  for (int c = 0; c < NC; c++) chunk(c, c & 1);
 
   // ---- epilogue: scale, round to bf16 (a9), activation (a10), store 4 consecutive n per lane --------------------
   if (!strip_ok) return;
@@ -553,6 +533,7 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(GemmParams p) {
 //   * each of the 8 waves owns FOUR 16-row weight strips (gate/up: 2 strips x {gate, up}; down: 4 strips), so one
 //     activation fragment read feeds 4 MFMAs (LDS port at <= 50 %) and 16 independent accumulators hide MFMA latency;
 //   * weights stream through a D-deep register ring per wave, D k-steps (>= 0.8 us of MFMA work) ahead of use.
+// moe_pick_job's eighths against tiles in launch order: 256 experts of 7168 x 2048, 64 rows each 1631 -> 1580 us, 64 of 6144 x 3072, 256: 1326 -> 1284.
 // Integer arithmetic and epilogue are those of moe_gemm_kernel, so results are bit-identical.
 // =====================================================================================================
 template <int N, class F, int I = 0>
@@ -576,12 +557,9 @@ __global__ __launch_bounds__(512) void moe_gemm_stream_kernel(GemmParams p, int 
   float* s_ad = reinterpret_cast<float*>(smem + (size_t)CCOL * CS);  // [TOK]
   int* s_src = reinterpret_cast<int*>(s_ad + TOK);                   // [TOK]
 
-  // (grid mappings that give all tiles x strip groups of one expert consecutive slots of ONE XCD, so that its L2 serves
-  // the re-reads, were measured: -5 % at best with uniform routing, +25 % with skewed routing because of the padding
-  // workgroups a fixed slots-per-expert layout needs — plain tile-major it is)
-  const int bx = blockIdx.x, tile_idx = blockIdx.y;
-  if (tile_idx >= p.counters[0]) return;
-  const Tile tile = p.tiles[tile_idx];
+  Tile tile;
+  int bx;
+  if (!moe_pick_job(p.tiles, p.counters[0], (p.N / 16 + 8 * SPW - 1) / (8 * SPW), tile, bx)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int strip0 = (bx * 8 + wave) * SPW;
@@ -2964,8 +2942,7 @@ static int launch_gemm(const GemmParams& p, int max_tiles, hipStream_t st) {
   auto kern = moe_gemm_kernel<WBITS, MT, SPC, GATE_UP>;
   const hipError_t attr_err = ktx_set_max_lds(reinterpret_cast<const void*>(kern), (int)lds);
   KTX_HIP(attr_err);
-  const dim3 grid((p.N / 16 + 3) / 4, max_tiles);
-  hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p);
+  hipLaunchKernelGGL(kern, moe_job_grid(max_tiles, (p.N / 16 + 3) / 4), dim3(256), lds, st, p);
   KTX_HIP(hipGetLastError());
   return 0;
 }
@@ -2980,7 +2957,7 @@ static int launch_gemm_stream(const GemmParams& p, int max_tiles, hipStream_t st
   const hipError_t attr_err = ktx_set_max_lds(reinterpret_cast<const void*>(kern), 160 * 1024);
   KTX_HIP(attr_err);
   const int strips_per_wg = 8 * (GATE_UP ? 2 : 4);
-  hipLaunchKernelGGL(kern, dim3((p.N / 16 + strips_per_wg - 1) / strips_per_wg, max_tiles), dim3(512), lds, st, p, kch);
+  hipLaunchKernelGGL(kern, moe_job_grid(max_tiles, (p.N / 16 + strips_per_wg - 1) / strips_per_wg), dim3(512), lds, st, p, kch);
   KTX_HIP(hipGetLastError());
   return 0;
 }
@@ -3275,12 +3252,23 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
   if (h->cfg.format == KTX_FMT_GGUF)
     return forward_gguf(h, d_bsz, qlen, k, d_expert_ids, d_weights, d_input, d_output, flags, st);
   int mt = pick_mt(qlen, k, E);
-  const bool use_rt = mt == 4 && g_dbg[4] == 3;   // register-tile kernels (256-row tiles): parity-tested, not yet timed
-  if (use_rt) mt = 16;
   const int npairs = qlen * k;
-  // 64-row tiles (prompts) of large expert matrices take the streaming kernels: measured 1.35x (gate/up) - 1.55x (down) on
-  // DeepSeek-V3-shaped experts (7168 x 2048), a wash on V2-Lite's 2048 x 1408.  Dev knob [4]: 1 = never, 2 = always (tests).
-  const bool use_stream = mt == 4 && g_dbg[4] != 1 && (g_dbg[4] == 2 || (size_t)H * I >= ((size_t)4 << 20));
+  // 64-row tiles (prompts) of large expert matrices take the streaming kernels, one workgroup a CU, where they have enough workgroups to go round;
+  // the others stay on moe_gemm_kernel.  Measured for AMXINT4 (us, 32 rows | streaming | 64 rows): 256 experts of 7168 x 2048 with 9.4 rows each
+  // 880 | 869 | 920, 16: 1036 | 993 | 1062, 64: 1900 | 1580 | 1766; 64 of 6144 x 3072, 37: 467 | 418 | 451; 32 of them, 62 (756 workgroups): 311 | 299 |
+  // 296; 16 of 6144 x 2048, 62 (376): 123 | 125 | 120, 256 (640): 321 | 292 | 278; 8 of 4096 x 1536, 100 (120): 53 | 72 | 58, 512: 176 | 170 | 156.
+  // 16 against 32 rows: 3.1 rows 660 | 669, 64 experts of 2048 x 1408, 3: 59 | 63, 9.4: 77 | 77.  32 against 64 rows where nothing streams: 25 rows
+  // 134 | 135, 37: 109 | 109, 50: 177 | 169, 75: 152 | 138; with 8 experts 25: 35 | 41, 100: 53 | 58, 125: 60 | 59, 200: 82 | 75 — few tiles leave
+  // CUs idle longer.  Dev knob [4]: 1 = never stream, 2 = always at 64 rows (tests).
+  const auto tiles64 = [&](int strips) { return (std::min(npairs, E) + npairs / 64) * ((I / 16 + strips - 1) / strips); };   // workgroups of gate|up
+  bool use_stream = mt == 4 && g_dbg[4] != 1 && (g_dbg[4] == 2 || (size_t)H * I >= ((size_t)4 << 20));
+  if (h->cfg.format == KTX_FMT_AMXINT4 && g_dbg[4] < 2) {
+    const double rows = (double)npairs / std::max(1, E);
+    use_stream = g_dbg[4] != 1 && rows > 9.0 && (size_t)H * I >= ((size_t)4 << 20) && tiles64(16) >= 700;
+    mt = rows <= 4.0 ? 1 : use_stream || (rows > 40.0 && tiles64(4) >= 512) ? 4 : 2;
+  }
+  const bool use_rt = mt == 4 && g_dbg[4] == 3;   // register-tile kernels (256-row tiles): parity-tested, not yet timed
+  if (use_rt) { mt = 16; use_stream = false; }
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
 
   PrepParams pp;

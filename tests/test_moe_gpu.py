@@ -694,3 +694,27 @@ def test_fp_grouped_edges(oracle, dev, fmt, H, I, rows):
     finally:
         _native.force_generic_path(False)
         h.close()
+
+
+@pytest.mark.parametrize("method", ["AMXINT4", "AMXINT8"])
+@pytest.mark.parametrize("H,I", [(128, 128), (384, 640), (1152, 256)])
+@pytest.mark.parametrize("rows", [(1, 0, 2, 3), (33, 0, 1, 32), (65, 0, 257, 16)])
+def test_int_grouped_edges(oracle, dev, method, H, I, rows):
+    """As test_fp_grouped_edges, bit for bit: k-steps that do not fill a chunk, uneven experts, at each tile height, with and without the
+    streaming kernels (dev knob 4: 1 = never, 2 = at 64-row tiles whatever the sizes)."""
+    from ktransformers_amd import _native
+    E, k, T = len(rows), 1, sum(rows)
+    c = make_case(43, E, k, H, I, T)
+    c["ids"] = np.random.default_rng(T).permutation(np.repeat(np.arange(E), rows)).astype(np.int64)[:, None]
+    want = oracle.moe_forward(oracle.make_moe(FMT[method], c["gate"], c["up"], c["down"]), c["ids"], c["w"], c["x"])
+    h = make_handle(method, c, E, k, H, I, max(T, 8), dev)
+    try:
+        _native.force_generic_path(True)
+        for knob in (0, 1, 2):
+            _native.lib.ktx_debug_set(4, knob)
+            got = run(h, c, dev)
+            assert np.array_equal(got, want), f"{int((got != want).sum())} outputs differ (knob {knob})"
+    finally:
+        _native.lib.ktx_debug_set(4, 0)
+        _native.force_generic_path(False)
+        h.close()
