@@ -1922,7 +1922,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATE_UP ? 2
 //   (LDS-DMA, XOR-swizzled rows; only the live 16-row groups) and the next step's weights (registers) are requested before the MFMAs
 //   and waited for behind them.
 // At Kimi-K2's sizes, us for the whole forward, int8 operands staged through registers -> here: 64 tokens 2256 -> 929, 256 3068 -> 1625, 2048
-// 5008 -> 4043 (gate|up 3169 -> 2519, down 1693 -> 1389: VALU instructions fill 70 % of the issue slots, two thirds of them the widening).
+// 5052 -> 4172 (VALU instructions fill 70 % of the issue slots, two thirds of them the widening; 13 of them a group instead of 17 changed nothing).
 // =====================================================================================================
 typedef _Float16 raw_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 raw_h8 __attribute__((ext_vector_type(8)));
