@@ -680,8 +680,8 @@ class LinearHandle:
     PROMPT_MIN_T = 512          # below this exact integer weights (ktx_linear_forward_ws); from here Marlin's rounded multiplicand
     # up to this many rows a product of few 256 x 256 tiles cuts K on ktx_linear_forward_ws instead of expanding the weights for a GEMM that
     # leaves most of the chip idle (512 rows, us, expansion / tiles: 16384 -> 7168 321 / 177, 7168 -> 2112 87 / 51; 1536 -> 24576, 192 tiles:
-    # 55 / 76; 700 rows of 7168 -> 4096: 91 / 100)
-    W4_CHUNKED_MAX_T = 640
+    # 55 / 76; a fifth tile of 128 rows and the expansion is ahead again: 529 rows of 7168 -> 4096 91 / 100)
+    W4_CHUNKED_MAX_T = 512
     PROMPT_MIN_TILES = 192
     _DEQ_SCRATCH: dict = {}
 

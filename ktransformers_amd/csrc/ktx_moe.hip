@@ -62,7 +62,16 @@ struct Tile {
 // XCD.  The jobs lie expert after expert, within an expert strip group by strip group, the group's tiles side by side; each XCD takes an
 // eighth of them.  So the XCDs end together whatever the number of tiles, an expert's weights go into one L2 and are read there once for all
 // its tiles, and its rows (the operand every strip group re-reads) stay there too.  False: nothing to do.
+// SHARE false: launch order, for tiles so low that an expert mostly has one (256 experts of 7168 x 2048, AMXINT4, 114 tokens: shares cost 1 %).
+template <bool SHARE = true>
 __device__ __forceinline__ bool moe_pick_job(const Tile* tiles, int ntiles, int nsg, Tile& tile, int& sgroup) {
+  if constexpr (!SHARE) {
+    const int t = blockIdx.x / nsg;
+    if (t >= ntiles) return false;
+    tile = tiles[t];
+    sgroup = blockIdx.x - t * nsg;
+    return true;
+  }
   const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
   const int total = ntiles * nsg, per = (total + 7) / 8, job = xcd * per + seq;
   if (seq >= per || job >= total) return false;
@@ -390,7 +399,7 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(GemmParams p) {
 
   Tile tile;
   int sgroup;
-  if (!moe_pick_job(p.tiles, p.counters[0], (p.N / 16 + 3) / 4, tile, sgroup)) return;
+  if (!moe_pick_job<(MT > 1)>(p.tiles, p.counters[0], (p.N / 16 + 3) / 4, tile, sgroup)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int strip = sgroup * 4 + wave;
@@ -1292,7 +1301,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 2 : MT == 2 ? 3 : 1) void 
 
   Tile tile;
   int sgroup;
-  if (!moe_pick_job(p.tiles, p.counters[0], (p.N / 16 + NWV * (GATE_UP ? 1 : NMAT) - 1) / (NWV * (GATE_UP ? 1 : NMAT)), tile, sgroup)) return;
+  if (!moe_pick_job<(MT > 1)>(p.tiles, p.counters[0], (p.N / 16 + NWV * (GATE_UP ? 1 : NMAT) - 1) / (NWV * (GATE_UP ? 1 : NMAT)), tile, sgroup)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int NKS = p.K / 128;
@@ -3257,15 +3266,16 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
   // the others stay on moe_gemm_kernel.  Measured for AMXINT4 (us, 32 rows | streaming | 64 rows): 256 experts of 7168 x 2048 with 9.4 rows each
   // 880 | 869 | 920, 16: 1036 | 993 | 1062, 64: 1900 | 1580 | 1766; 64 of 6144 x 3072, 37: 467 | 418 | 451; 32 of them, 62 (756 workgroups): 311 | 299 |
   // 296; 16 of 6144 x 2048, 62 (376): 123 | 125 | 120, 256 (640): 321 | 292 | 278; 8 of 4096 x 1536, 100 (120): 53 | 72 | 58, 512: 176 | 170 | 156.
-  // 16 against 32 rows: 3.1 rows 660 | 669, 64 experts of 2048 x 1408, 3: 59 | 63, 9.4: 77 | 77.  32 against 64 rows where nothing streams: 25 rows
+  // A short K or few workgroups stream no better: 64 of 1536 x 3072, 20 rows 130 | 137, 64 of 2560 x 2048, 32 (768): 160 | 174.  16 against 32 rows: 3.1 rows 660 | 669, 6.6: 750 | 778, 64 experts of
+  // 2048 x 1408, 3: 59 | 63, 9.4: 77 | 77.  32 against 64 rows where nothing streams: 25 rows
   // 134 | 135, 37: 109 | 109, 50: 177 | 169, 75: 152 | 138; with 8 experts 25: 35 | 41, 100: 53 | 58, 125: 60 | 59, 200: 82 | 75 — few tiles leave
   // CUs idle longer.  Dev knob [4]: 1 = never stream, 2 = always at 64 rows (tests).
   const auto tiles64 = [&](int strips) { return (std::min(npairs, E) + npairs / 64) * ((I / 16 + strips - 1) / strips); };   // workgroups of gate|up
   bool use_stream = mt == 4 && g_dbg[4] != 1 && (g_dbg[4] == 2 || (size_t)H * I >= ((size_t)4 << 20));
   if (h->cfg.format == KTX_FMT_AMXINT4 && g_dbg[4] < 2) {
     const double rows = (double)npairs / std::max(1, E);
-    use_stream = g_dbg[4] != 1 && rows > 9.0 && (size_t)H * I >= ((size_t)4 << 20) && tiles64(16) >= 700;
-    mt = rows <= 4.0 ? 1 : use_stream || (rows > 40.0 && tiles64(4) >= 512) ? 4 : 2;
+    use_stream = g_dbg[4] != 1 && rows > 12.0 && std::min(H, I) >= 2048 && (size_t)H * I >= ((size_t)4 << 20) && tiles64(16) >= 1200;
+    mt = rows <= 8.0 ? 1 : use_stream || (rows > 40.0 && tiles64(4) >= 512) ? 4 : 2;
   }
   const bool use_rt = mt == 4 && g_dbg[4] == 3;   // register-tile kernels (256-row tiles): parity-tested, not yet timed
   if (use_rt) { mt = 16; use_stream = false; }
@@ -3335,9 +3345,9 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
   const int npairs = qlen * k;
   // Rows per tile.  Measured (us, 16 | 32 | 64 rows): 256 experts of 7168 x 2048 with 3.1 rows each 1214 | 1202 | 1382, 15.6: 1981 | 1823 | 2029,
   // 47: 3423 | 2873 | 2944, 62: 4142 | 3353 | 3290; 64 of 2048 x 1408, 9.4: 115 | 116 | 135, 66: 245 | 206 | 223, 94: 312 | 251 | 259, 141: 431 | 349 | 340;
-  // 8 of 4096 x 1536, 25: 56 | 55 | 74, 75: 88 | 80 | 76, 250: 196 | 160 | 155
+  // 8 of 4096 x 1536, 25: 56 | 55 | 74, 75: 88 | 80 | 76, 250: 196 | 160 | 155; 128 of 4608 x 512, 7.4: 158 | 165
   const double rows = (double)npairs / std::max(1, E);
-  const int mt = rows <= 2.5 ? 1 : rows <= 60.0 ? 2 : 4;
+  const int mt = rows <= 8.0 ? 1 : rows <= 60.0 ? 2 : 4;
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
 
   // ---- decode fast path: two launches (see moe_dec_fp_gateup_kernel) ------------------------------------------------------

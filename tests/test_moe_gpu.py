@@ -673,7 +673,7 @@ def test_batches_that_share_experts_take_the_grouped_kernels(dev, method):
 @pytest.mark.parametrize("H,I", [(128, 128), (384, 640), (256, 1152)])
 @pytest.mark.parametrize("rows", [(1, 0, 2, 3), (33, 0, 1, 32), (65, 0, 257, 16)])
 def test_fp_grouped_edges(oracle, dev, fmt, H, I, rows):
-    """The grouped kernels at each tile height (2.5 and 60 rows an expert on average divide them): odd numbers of 128-k steps, one step, experts
+    """The grouped kernels at each tile height (8 and 60 rows an expert on average divide them): odd numbers of 128-k steps, one step, experts
     without rows, of one row past a tile, of several tiles (the XCDs' shares cut through them), strip groups that are not full."""
     from helpers import fp8_block_quant
     from ktransformers_amd import _native
