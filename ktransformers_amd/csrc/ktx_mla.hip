@@ -757,7 +757,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // (m, l) pairs, the partial outputs, the bounds — is issued before the first use: right after the kernel boundary each of
 // them is an L2 miss, and a stats -> weights -> addresses -> loads chain would pay that latency three times over.  A dead
 // split's partial may be stale memory, so it is selected away (not multiplied by 0).
-template <int NS>   // splits per thread and round
+template <int NS, bool JOBS>   // splits per thread and round; JOBS: a token's number of splits is the decode kernel's (njobs)
 __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out, float* lse) {
   __shared__ float s_w[1024];
   __shared__ float s_red[8];
@@ -765,7 +765,7 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out
   const int qt = blockIdx.y, h = blockIdx.x, quarter = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int dg = tid & 15, sl = tid >> 4;   // 16 dim groups of 8 dims x 16 split lanes
   const size_t base = ((size_t)qt * p.Hq + h) * p.nsplit;
-  const int nsp = p.jobs ? min(max(p.njobs[qt], 1), p.nsplit) : p.nsplit;   // (no request's token: whatever is there, and nothing is stored)
+  const int nsp = JOBS ? min(max(p.njobs[qt], 1), p.nsplit) : p.nsplit;   // (no request's token: whatever is there, and nothing is stored)
   // ---- all loads
   int B = p.batch;
   const int bsz_raw = p.d_bsz ? *p.d_bsz : p.batch;
@@ -819,7 +819,7 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out
       acc[4] += vb[u].x * w; acc[5] += vb[u].y * w; acc[6] += vb[u].z * w; acc[7] += vb[u].w * w;
     }
   }
-  if (c + 16 * NS >= nsp) break;
+  if (!JOBS || c + 16 * NS >= nsp) break;
 #pragma unroll
   for (int u = 0; u < NS; u++) {
     const int s = min(c + 16 * NS + sl + 16 * u, nsp - 1);
@@ -1081,10 +1081,11 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
     KTX_TIMED(st, (double)total_q_tokens * Hq * MLA_DC * 2.0, "mla_merge_kernel T=%d Hq=%d nsplit=%d", total_q_tokens, Hq, nsplit);
     const dim3 mg(Hq, total_q_tokens, 4);
     const int ns = p.jobs ? std::min(p.nsplit, 2 * p.jobs / total_q_tokens) : p.nsplit;   // (jobs: twice the mean; the kernel goes on from there)
-    if (ns <= 32) hipLaunchKernelGGL(mla_merge_kernel<2>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
-    else if (ns <= 64) hipLaunchKernelGGL(mla_merge_kernel<4>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
-    else if (ns <= 144) hipLaunchKernelGGL(mla_merge_kernel<9>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
-    else hipLaunchKernelGGL(mla_merge_kernel<16>, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse);
+    auto merge = [&](auto kern) { hipLaunchKernelGGL(kern, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse); };
+    if (ns <= 32) p.jobs ? merge(mla_merge_kernel<2, true>) : merge(mla_merge_kernel<2, false>);
+    else if (ns <= 64) p.jobs ? merge(mla_merge_kernel<4, true>) : merge(mla_merge_kernel<4, false>);
+    else if (ns <= 144) p.jobs ? merge(mla_merge_kernel<9, true>) : merge(mla_merge_kernel<9, false>);
+    else p.jobs ? merge(mla_merge_kernel<16, true>) : merge(mla_merge_kernel<16, false>);
   }
   KTX_HIP(hipGetLastError());
   return 0;
