@@ -1915,12 +1915,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATE_UP ? 2
 // (tests/test_moe_gpu.py::test_rawint4_prompt_chunks).  Decode and short batches (qlen < 64) keep the exact kernels; dev knob 29 = 1
 // forces them for every size.
 //
-// What bounds it is the VALU work per MFMA, so the operands carry what can be carried exactly: the activation codes are f16 integers, the
-// weights f16 q * bs — 4 and 8 significant bits, exact in f16's 11 for scales of 2^-17 .. 2^11 (ktx_moe_load_rawint4 looks; other scales
-// stay on the exact kernel) — and the products' fp32 sum over a group is exact as well.  What is left per 16 x 16 fragment and group is
-// acc = fma(as, sum, acc): 4 operations instead of the 12 of an int8 MFMA (scale product, conversion, fma).  A group's 8 weights of a lane
-// become f16 in 17 operations for all token fragments: a nibble goes to the top mantissa bits of an f16 (16 + q'), and
-// fma(16 + q', bs, -24 bs) is q * bs with both constants exact.
+// The VALU has more to do per MFMA than anything else here, so the operands are what costs it least: codes and nibbles as f16 integers, whose sum
+// over a group the f16 MFMA gives exactly and in fp32 already (below 2^15), so that a 16 x 16 fragment and group takes a scale product and an fma
+// per output where an int8 MFMA takes a conversion as well: the terms are the reference's, with any scale.  A group's 8 weights of a lane
+// become f16 in 12 operations for all token fragments: a nibble goes to the top mantissa bits of an f16 (16 + q'), minus 24 is q.
+// (The weight's scale inside the f16 operand saves the scale products, at 2048 tokens 4 %, but holds for scales of 2^-17 .. 2^11 only and rounds
+// otherwise than the reference's terms.)
 //
 // No second copy of the weights: the RAW tiles are read as they lie in HBM.  MFMA lane (i = lane & 15, kc = lane >> 4) needs
 // row i's eight nibbles k = 64 kb + 32 h + 8 kc + [0, 8) of group (kb, h): those are the pieces (L, j) = (8h + 2kc + o, i & 3),
@@ -1930,18 +1930,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATE_UP ? 2
 //   multiplies while the other waits); K walks in the RAW step of 512, the activations in halves of it.  The next half's activations
 //   (LDS-DMA, XOR-swizzled rows; only the live 16-row groups) and the next step's weights (registers) are requested before the MFMAs
 //   and waited for behind them.
-// At Kimi-K2's sizes, us for the whole forward, int8 operands staged through registers -> here: 64 tokens 2256 -> 929, 256 3068 -> 1625, 2048
-// 5052 -> 4172 (VALU instructions fill 70 % of the issue slots, two thirds of them the widening; 13 of them a group instead of 17 changed nothing).
+// At Kimi-K2's sizes, us for the whole forward, int8 operands staged through registers -> here (the same bits): 64 tokens 1409 -> 996, 256
+// 2313 -> 1705, 1000 3537 -> 2884, 2048 5084 -> 4392.
 // =====================================================================================================
 typedef _Float16 raw_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 raw_h8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ uint32_t raw_h2_bits(raw_h2 v) { return __builtin_bit_cast(uint32_t, v); }
-// the pairs (byte 0, byte 2) and (byte 1, byte 3) of the low (par 0) or high nibbles of x as q * bs; x: two's complement nibbles ^ 8
+// the pairs (byte 0, byte 2) and (byte 1, byte 3) of the low (par 0) or high nibbles of x; x: two's complement nibbles ^ 8
 template <int PAR>
-__device__ __forceinline__ void raw_widen(uint32_t x, uint32_t mask, uint32_t top, raw_h2 bs, raw_h2 m24, uint32_t& o0, uint32_t& o1) {
+__device__ __forceinline__ void raw_widen(uint32_t x, uint32_t mask, uint32_t top, uint32_t& o0, uint32_t& o1) {
   const uint32_t e0 = ((PAR ? x << 2 : x << 6) & mask) | top, e1 = ((PAR ? x >> 6 : x >> 2) & mask) | top;
-  o0 = raw_h2_bits(__builtin_elementwise_fma(__builtin_bit_cast(raw_h2, e0), bs, m24));
-  o1 = raw_h2_bits(__builtin_elementwise_fma(__builtin_bit_cast(raw_h2, e1), bs, m24));
+  const raw_h2 m24 = {(_Float16)-24.0f, (_Float16)-24.0f};
+  o0 = raw_h2_bits(__builtin_bit_cast(raw_h2, e0) + m24);
+  o1 = raw_h2_bits(__builtin_bit_cast(raw_h2, e1) + m24);
 }
 
 template <bool GATE_UP>
@@ -2067,6 +2068,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int t = 0; t < MTL; t++) sf[g & 1][t] = *reinterpret_cast<const float4*>(ab + g * TOK + t * 16);
     };
+    float bs[2][NU];   // the groups' weight scales, of the lane's row
     auto widen = [&](raw_h8 (&bop)[NU], auto gc) __attribute__((always_inline)) {
       constexpr int g = decltype(gc)::value, kb8 = HALF * 4 + (g >> 1), h = g & 1;   // g = (kb8 of the half) * 2 + h
 #pragma unroll
@@ -2075,11 +2077,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const uint32_t P0 = kb8 < 2 ? w0.x : kb8 < 4 ? w0.y : kb8 < 6 ? w0.z : w0.w;
         const uint32_t P1 = kb8 < 2 ? w1.x : kb8 < 4 ? w1.y : kb8 < 6 ? w1.z : w1.w;
         const uint32_t S = kb8 < 2 ? sv.x : kb8 < 4 ? sv.y : kb8 < 6 ? sv.z : sv.w;
-        const _Float16 bh = (_Float16)__uint_as_float((kb8 & 1) ? (S & 0xffff0000u) : (S << 16));
-        const raw_h2 bs = {bh, bh}, m24 = bs * raw_h2{(_Float16)-24.0f, (_Float16)-24.0f};
+        bs[g & 1][u] = __uint_as_float((kb8 & 1) ? (S & 0xffff0000u) : (S << 16));
         uint32_t o[4];
-        raw_widen<(kb8 & 1)>(P0, mask, top, bs, m24, o[0], o[1]);
-        raw_widen<(kb8 & 1)>(P1, mask, top, bs, m24, o[2], o[3]);
+        raw_widen<(kb8 & 1)>(P0, mask, top, o[0], o[1]);
+        raw_widen<(kb8 & 1)>(P1, mask, top, o[2], o[3]);
         bop[u] = __builtin_bit_cast(raw_h8, make_uint4(o[0], o[1], o[2], o[3]));
       }
     };
@@ -2109,7 +2110,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
           for (int u = 0; u < NU; u++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) acc[u][t0 + t][r] = fmaf(asv[r], d[t][u][r], acc[u][t0 + t][r]);
+            for (int r = 0; r < 4; r++) acc[u][t0 + t][r] = fmaf(asv[r] * bs[g & 1][u], d[t][u][r], acc[u][t0 + t][r]);
         }
         if constexpr (TB < MTL) __builtin_amdgcn_sched_barrier(0);
       }
@@ -2492,16 +2493,6 @@ __global__ void pack_rawint4_kernel(const uint8_t* __restrict__ src, int N, int 
   out[idx] = v;
 }
 
-// *out |= 1 when a scale is neither zero nor of magnitude 2^-17 .. 2^11
-__global__ __launch_bounds__(256) void raw_scale_range_kernel(const bf16_t* __restrict__ s, size_t n, int* out) {
-  bool bad = false;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-    const float a = fabsf(bf16_to_f32(s[i]));
-    bad |= !(a == 0.0f || (a >= 0x1p-17f && a <= 0x1p11f));
-  }
-  if (bad) atomicOr(out, 1);
-}
-
 // bf16 scales [N][K/32] -> tile order [rg][step][row j][h][8 blocks]; one thread per element
 __global__ void pack_rawint4_scales_kernel(const bf16_t* __restrict__ src, int N, int K, bf16_t* __restrict__ out) {
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2578,7 +2569,6 @@ struct ktx_moe_s {
   int gg_type[3] = {0, 0, 0};     // GGUF: ggml type of gate / up / down
   size_t gg_stride[3] = {0, 0, 0};
   bool loaded_gguf = false;
-  bool raw_f16 = false;           // RAWINT4: every scale times 24 and times a nibble is exact in f16 (moe_rawint4_chunk_kernel)
   bool exact = false;             // ktx_moe_set_exact: no path of this handle may re-associate the reference's fp32 sums
 };
 
@@ -2894,15 +2884,6 @@ extern "C" int ktx_moe_load_rawint4(ktx_moe_t h, const void* d_gate, const void*
   KTX_ON_DEVICE(h->cfg.device);
   const int E = h->cfg.expert_num, H = h->cfg.hidden_size, I = h->cfg.intermediate_size;
   const size_t dwords = (size_t)I * H / 8, nsc = (size_t)I * (H / 32);
-  int* range = nullptr;
-  int out_of_range = 0;
-  KTX_HIP(hipMalloc(&range, sizeof(int)));
-  KTX_HIP(hipMemcpy(range, &out_of_range, sizeof(int), hipMemcpyHostToDevice));
-  for (const void* sc : {d_gate_scale, d_up_scale, d_down_scale})
-    hipLaunchKernelGGL(raw_scale_range_kernel, dim3(1024), dim3(256), 0, 0, (const bf16_t*)sc, (size_t)E * nsc, range);
-  KTX_HIP(hipMemcpy(&out_of_range, range, sizeof(int), hipMemcpyDeviceToHost));
-  KTX_HIP(hipFree(range));
-  h->raw_f16 = out_of_range == 0;
   for (int e = 0; e < E; e++) {
     const uint8_t* src[3] = {(const uint8_t*)d_gate + (size_t)e * I * H / 2, (const uint8_t*)d_up + (size_t)e * I * H / 2,
                              (const uint8_t*)d_down + (size_t)e * H * I / 2};
@@ -3529,7 +3510,7 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
 
   // prompt chunks: 64-row tiles through the group-scaled 16x16x32 kernel (moe_rawint4_chunk_kernel: same terms, one fp32 chain per
   // output instead of the reference's sixteen); short batches and dev knob 29 = 1 keep the exact 4-row kernel
-  const bool chunk = qlen >= 64 && g_dbg[29] != 1 && !h->exact && h->raw_f16 && (size_t)npairs * (std::max(H, I) / 32) * 4 < ((size_t)1 << 32);
+  const bool chunk = qlen >= 64 && g_dbg[29] != 1 && !h->exact && (size_t)npairs * (std::max(H, I) / 32) * 4 < ((size_t)1 << 32);
   PrepParams pp;
   pp.d_bsz = d_bsz; pp.qlen = qlen; pp.k = k; pp.E = E; pp.expert_begin = h->cfg.expert_begin; pp.H = H;
   pp.rows_per_tile = chunk ? 64 : 4; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
