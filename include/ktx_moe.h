@@ -124,9 +124,11 @@ int ktx_moe_combine(int qlen, int k, int hidden, const void* d_rows, const int32
 /* should_skip_expert mask (operators/common.hpp:241-258): mask[e] != 0 => expert e contributes nothing. HOST ptr, may be NULL. */
 int ktx_moe_set_expert_mask(ktx_moe_t h, const uint8_t* mask);
 
-/* Exact / fast switch of a handle (default 0 = fast).  Every decode-sized call, and every format but RAWINT4 at any size, reproduces
- * the reference's fp32 summation order bit for bit either way.  RAWINT4 (Kimi-K2) prompt chunks of >= 64 tokens are the one place a
- * faster kernel re-associates: moe_rawint4_chunk_kernel adds a row's K/32 group terms (d_a * d_w * int32 dot, the same terms) as ONE
+/* Exact / fast switch of a handle (default 0 = fast).  It concerns RAWINT4 alone.  The integer formats reproduce the reference's sums bit
+ * for bit either way, and so do RAWINT4's decode-sized calls (qlen * k <= 64, or fewer than 64 tokens); FP8, BF16 and GGUF hold bounds
+ * instead, either way: an output's fp32 sums over K are ordered by the kernel that takes the call, and a batch of up to 64 pairs whose
+ * experts repeat takes a prompt's kernels unless d_bsz is given.  RAWINT4 (Kimi-K2) prompt chunks of >= 64 tokens are where a
+ * faster kernel re-associates the integers' sums: moe_rawint4_chunk_kernel adds a row's K/32 group terms (d_a * d_w * int32 dot, the same terms) as ONE
  * fp32 chain, the reference keeps sixteen interleaved chains and a final tree (la/amx_kernels.hpp:3385-3455).  Measured bound of the
  * fast path against the reference on its own test's data (tests/test_moe_gpu.py): |y - ref| <= 2^-7 |ref| + 2^-9 max|ref| (two bf16
  * ulp element-wise), < 5 % of the outputs different, mean error < 1e-3; ~6.7x the exact kernel's prompt rate (16 k vs 2.4 k tok/s at

@@ -3108,8 +3108,9 @@ extern "C" int ktx_moe_forward_side(ktx_moe_t h, const int32_t* d_bsz, int qlen,
 // FP8 153: 54 | 61, 239: 74 | 64, 251: 49 | 52, 323: 60 | 54, 646: 125 | 67; RAWINT4 167: 67 | 72, 235: 61 | 63, 247: 176 | 153,
 // 310: 73 | 69, 517: 267 | 186; Q4_K 349: 46 | 50, 487: 80 | 71, 582: 225 | 200, 955: 248 | 217.  With few repeats among many experts the
 // grouped kernels' 16-row tiles hold one row each and stream slower (256 experts of 7168 x 2048, AMXINT4, 8 tokens x 8: decode stays
-// ahead at 285 MB), hence the second condition.  Both ways give the same bits; a batch whose size only the device knows, masked experts, and
-// formats that were not measured stay where they were.
+// ahead at 285 MB), hence the second condition.  AMXINT4, FP8 and RAWINT4 give the same bits either way; the K-quants add a row's blocks in another
+// order (the grouped kernels in k order, the decode launches K piece by K piece), to 16 * 2^-24 of the terms' magnitudes before the bf16
+// rounding.  A batch whose size only the device knows, masked experts, and formats that were not measured stay on the decode launches.
 static bool shares_experts(const ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, size_t bytes) {
   double mb;
   switch (h->cfg.format) {
@@ -3475,8 +3476,9 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
 
   // ---- decode fast path: two launches (see moe_dec_raw_gateup_kernel) -----------------------------------------------------
   const size_t lds_rdn = (size_t)k * (I + I / 32 * 4 + 16 * 4 + 8);
+  // (64 tokens of one expert each stay here although they share: grouped they would be a prompt, and a decode-sized call keeps the reference's sums)
   if (npairs <= KTX_DEC_MAX_PAIRS && k <= 8 && H <= 8192 && I <= 4096 && lds_rdn <= 160 * 1024 && !g_force_generic &&
-      !shares_experts(h, d_bsz, qlen, k, 2 * h->gu_stride + h->dn_stride)) {
+      (qlen >= 64 || !shares_experts(h, d_bsz, qlen, k, 2 * h->gu_stride + h->dn_stride))) {
     RawDecParams dp;
     dp.d_bsz = d_bsz; dp.qlen = qlen; dp.k = k; dp.E = E; dp.expert_begin = h->cfg.expert_begin; dp.H = H; dp.I = I;
     dp.ids = d_expert_ids; dp.mask = h->mask; dp.x = (const bf16_t*)d_input; dp.weights = d_weights;

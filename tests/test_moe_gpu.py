@@ -679,6 +679,28 @@ def test_batches_that_share_experts_take_the_grouped_kernels(dev, method):
         assert torch.equal(got, want)
 
 
+def test_rawint4_64_tokens_of_one_expert_each_keep_the_reference_sums(dev):
+    """A decode-sized call (64 pairs) of 64 tokens that name 4 experts again and again: the same bits as with set_exact and as on the decode
+    launches, not the prompt kernel's."""
+    from ktransformers_amd._native import MoEHandle
+    E, k, H, I, T = 4, 1, 4096, 2048, 64
+    g = torch.Generator(device=dev).manual_seed(9)
+    shapes = ((I, H), (I, H), (H, I))
+    h = MoEHandle(E, k, H, I, T, "RAWINT4", 0, group_size=32)
+    try:
+        h.load_rawint4(*(torch.randint(0, 256, (E, n, kk // 2), dtype=torch.uint8, device=dev, generator=g) for n, kk in shapes),
+                       *(torch.rand((E, n, kk // 32), device=dev, generator=g).add_(0.5).mul_(1e-2).bfloat16() for n, kk in shapes))
+        x, w = torch.randn((T, H), device=dev, generator=g).bfloat16(), torch.rand((T, k), device=dev, generator=g)
+        ids = torch.randint(0, E, (T, k), device=dev, generator=g)
+        got = h.forward(x, ids, w)
+        assert got.abs().max() > 0
+        assert torch.equal(got, h.forward(x, ids, w, bsz_tensor=torch.tensor([T], dtype=torch.int32, device=dev)))
+        h.set_exact(True)
+        assert torch.equal(got, h.forward(x, ids, w))
+    finally:
+        h.close()
+
+
 @pytest.mark.parametrize("fmt", ["FP8", "BF16"])
 @pytest.mark.parametrize("H,I", [(128, 128), (384, 640), (256, 1152)])
 @pytest.mark.parametrize("rows", [(1, 0, 2, 3), (33, 0, 1, 32), (65, 0, 257, 16)])
