@@ -677,12 +677,7 @@ class LinearHandle:
 
     # ---- prompt-sized W4 calls: de-quantise once (Marlin's rounding), then the library's own BF16 GEMM (csrc/ktx_gemm.hip;
     # KTX_VENDOR_GEMM=1 sends the product to torch's F.linear instead — the A/B switch of scripts/gemm_bench.py) ------------
-    PROMPT_MIN_T = 512          # below this exact integer weights (ktx_linear_forward_ws); from here Marlin's rounded multiplicand
-    # up to this many rows a product of few 256 x 256 tiles cuts K on ktx_linear_forward_ws instead of expanding the weights for a GEMM that
-    # leaves most of the chip idle (512 rows, us, expansion / tiles: 16384 -> 7168 321 / 177, 7168 -> 2112 87 / 51; 1536 -> 24576, 192 tiles:
-    # 55 / 76; a fifth tile of 128 rows and the expansion is ahead again: 529 rows of 7168 -> 4096 91 / 100)
-    W4_CHUNKED_MAX_T = 512
-    PROMPT_MIN_TILES = 192
+    PROMPT_MIN_T = 512          # below this, and for calls that the GEMM doesn't take: exact integer weights (ktx_linear_forward_ws)
     _DEQ_SCRATCH: dict = {}
 
     def dequant_bf16(self, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -811,8 +806,7 @@ class LinearHandle:
         # kernels, which take any out_features)
         gemm_ok = (self.batch == 1 and bsz_tensor is None and self.N % 8 == 0 and self.K % 64 == 0 and x2.data_ptr() % 16 == 0
                    and (x2.stride(0) * 2) % 16 == 0 and not torch.cuda.is_current_stream_capturing())
-        if (self.fmt == "W4" and gemm_ok and T >= self.PROMPT_MIN_T
-                and (T > self.W4_CHUNKED_MAX_T or -(-T // 256) * -(-self.N // 256) >= self.PROMPT_MIN_TILES) and not os.environ.get("KTX_W4_PROMPT_KERNEL")):
+        if self.fmt == "W4" and gemm_ok and T >= self.PROMPT_MIN_T and not os.environ.get("KTX_W4_PROMPT_KERNEL"):
             if norm is not None:
                 x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)
             return self._prompt_forward(x2, out, add1, add2, glu).reshape(*x.shape[:-1], n_out)
@@ -859,11 +853,11 @@ class LinearHandle:
         return out.reshape(*x.shape[:-1], n_out)
 
     def _forward_ws(self, bsz, T: int, x2: torch.Tensor, out: torch.Tensor, fu) -> None:
-        """ktx_linear_forward_ws with its scratch from torch's allocator (freed to the stream's pool behind the launches)."""
+        """ktx_linear_forward_ws with its scratch from torch's allocator (freed to the stream's pool behind the launches).  FP8 prompts take the
+        K = 128 MFMA whether the call is eager, captured or has its row count on the device."""
         need = int(lib.ktx_linear_workspace_bytes(self._h, T, 1 if bsz is None and fu is None else 0))
         ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
-        prompt = (T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")) if self.fmt == "FP8" else \
-            (T >= self.PROMPT_MIN_T and not os.environ.get("KTX_W4_PROMPT_KERNEL"))
+        prompt = self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")
         check(lib.ktx_linear_forward_ws(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), fu, 1 if prompt else 0, ws.data_ptr() if need else None, need,
                                         _stream_ptr(self.device)))
 

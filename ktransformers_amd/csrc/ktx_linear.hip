@@ -2204,8 +2204,7 @@ extern "C" int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T
     return prompt && o.mt >= 4 ? forward_tile<F_FP8, 128, true>(o, q, st) : forward_tile<F_FP8, 128>(o, q, st);
   }
   const int g = h->cfg.group_size;
-  const bool alt = prompt && h->cfg.format == KTX_LIN_W4 && o.mt >= 4;
-  if (o.sT_bytes && !alt) {
+  if (o.sT_bytes) {
     const dim3 grid((unsigned)((q.s_ld * (p.Kx / 8) + 255) / 256));
     KTX_TIMED(st, (double)T * p.Kx * 2.0, "lin_tile_sums_kernel T=%d K=%d", T, p.Kx);
     if (g == 32) hipLaunchKernelGGL(lin_tile_sums_kernel<32>, grid, dim3(256), 0, st, p.x, ldx, T, p.Kx, (float*)q.sT, q.s_ld);
@@ -2216,9 +2215,7 @@ extern "C" int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T
   switch (h->cfg.format) {
     case KTX_LIN_BF16: return forward_tile<F_BF16, 128>(o, q, st);
     case KTX_LIN_W8: return g == 32 ? forward_tile<F_W8, 32>(o, q, st) : g == 64 ? forward_tile<F_W8, 64>(o, q, st) : forward_tile<F_W8, 128>(o, q, st);
-    default:
-      if (alt) return g == 32 ? forward_tile<F_W4, 32, true>(o, q, st) : g == 64 ? forward_tile<F_W4, 64, true>(o, q, st) : forward_tile<F_W4, 128, true>(o, q, st);
-      return g == 32 ? forward_tile<F_W4, 32>(o, q, st) : g == 64 ? forward_tile<F_W4, 64>(o, q, st) : forward_tile<F_W4, 128>(o, q, st);
+    default: return g == 32 ? forward_tile<F_W4, 32>(o, q, st) : g == 64 ? forward_tile<F_W4, 64>(o, q, st) : forward_tile<F_W4, 128>(o, q, st);
   }
 }
 
