@@ -745,3 +745,40 @@ def test_batches_and_short_prompts_on_tiles(fmt, K, N, T):
         close(h.forward(xc, glu=True), (s * g[:, :, 1]).reshape(T, N // 2).cpu(), rel=5e-3)
     if N > 256 and T < 512:
         assert torch.equal(handle(256, False).forward(xc), y[:, :256]), "a merged operator's rows"
+
+
+@pytest.mark.parametrize("G", [32, 64, 128])
+@pytest.mark.parametrize("K,N,T,how", [(2048, 577, 513, "odd"), (1024, 1000, 512, "rows"), (7168, 264, 640, "capture"), (2048, 12296, 600, "rows"), (384, 33, 1030, "odd")])
+def test_w4_prompts_off_the_gemm_multiply_exact_integers(G, K, N, T, how):
+    """512 rows and more that the expansion GEMM doesn't take (out_features % 8 != 0, a device-side row count, stream capture) multiply
+    (q - 8) exactly and scale in fp32; only the GEMM's multiplicand is rounded to bf16.  Against 64-bit sums an exact product is off by the
+    outputs' rounding alone: uniform in half an ulp, 2^-8 / sqrt(12) = 1.1e-3 of a power of two and 1.66e-3 in the norm over mantissas; the
+    rounded multiplicand adds an independent error to every term whose (q - 8) * s doesn't fit bf16: 2.1e-3 and more.  2.0e-3 parts the two."""
+    n = native()
+    torch.manual_seed(K + N + T + G)
+    w = (torch.randn(N, K) / 10).to(torch.bfloat16)
+    x = (torch.randn(T, K) / 10).to(torch.bfloat16)
+    q, s = quantize_weights_ref(w.T.contiguous(), G)
+    want = x.cuda().double() @ ((q.double().cuda() - 8.0) * s.cuda().double().repeat_interleave(G, dim=0))
+    h = n.LinearHandle(K, N, "W4", G, T)
+    h.load_bf16(w.cuda())
+    xc = x.cuda()
+    if how == "odd":
+        y = h.forward(xc)
+    elif how == "rows":
+        y = h.forward(xc, bsz_tensor=torch.tensor([T], dtype=torch.int32, device="cuda"))
+    else:
+        y = torch.empty(T, N, dtype=torch.bfloat16, device="cuda")
+        h.forward(xc, out=y)
+        eager = y.clone()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            h.forward(xc, out=y)
+        for _ in range(3):
+            y.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert float((y.double() - want).norm() / want.norm()) < 2.0e-3
+        assert float((eager.double() - want).norm() / want.norm()) > 2.0e-3     # (the eager call is the GEMM's)
+    close(y, want.float().cpu())
+    assert float((y.double() - want).norm() / want.norm()) < 2.0e-3
