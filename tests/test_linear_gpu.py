@@ -129,7 +129,17 @@ def test_fp8_prompt_gemm_against_the_strip_kernel(K, N, T, monkeypatch):
     calls = [dict(), dict(add1=add1), dict(norm=(nw, 1e-6)), dict(add1=add1, add2=add1)]
     if N % 16 == 0 and bias is None:
         calls.append(dict(glu=True))
-    # round 6: the default GEMM sums a 128-block in ONE K = 128 MFMA (twice the rate; the hardware's own order inside the block) —
+    # the GEMM at every size (ktx_linear_forward_ws would take most of these), and the strip kernel itself to compare with (dev knob 12 keeps it)
+    monkeypatch.setattr(n.LinearHandle, "FP8_CHUNKED_MAX_T", 0)
+    monkeypatch.setattr(n.LinearHandle, "FP8_GEMM_MIN_OUT", 0)
+    n.timing_enable(2)
+    try:
+        h.forward(x)
+        labels = [t[0] for t in n.timing_collect()]
+    finally:
+        n.timing_enable(0)
+    assert any("lin_fp8_gemm_kernel" in t for t in labels), labels
+    # the default GEMM sums a 128-block in ONE K = 128 MFMA (twice the rate; the hardware's own order inside the block) —
     # within one bf16 ulp of the strip kernel; dev knob 27 = 1 keeps the four K = 32 MFMAs, which ARE the strip kernel's bits
     fast = [h.forward(x, **kw) for kw in calls] + [h.forward(xs)]
     n.check(n.lib.ktx_debug_set(27, 1))
@@ -138,7 +148,11 @@ def test_fp8_prompt_gemm_against_the_strip_kernel(K, N, T, monkeypatch):
     finally:
         n.check(n.lib.ktx_debug_set(27, 0))
     monkeypatch.setenv("KTX_FP8_PROMPT_KERNEL", "1")
-    want = [h.forward(x, **kw) for kw in calls] + [h.forward(xs)]
+    n.check(n.lib.ktx_debug_set(12, 1))
+    try:
+        want = [h.forward(x, **kw) for kw in calls] + [h.forward(xs)]
+    finally:
+        n.check(n.lib.ktx_debug_set(12, 0))
     for a, b, f, kw in zip(got, want, fast, calls + [dict(strided=True)]):
         assert a.shape == b.shape and torch.equal(a, b), f"{kw.keys()}: {(a != b).sum().item()} of {a.numel()} outputs differ"
         d = (f.float() - b.float()).abs()
@@ -147,6 +161,34 @@ def test_fp8_prompt_gemm_against_the_strip_kernel(K, N, T, monkeypatch):
         assert float((f != b).float().mean()) < 0.02, f"{kw.keys()}: {float((f != b).float().mean()):.4f} of the outputs differ"
     close(got[0], linear_fp8_ref(x.cpu(), w, sc, bias), rel=2e-3)
     close(fast[0], linear_fp8_ref(x.cpu(), w, sc, bias), rel=2e-3)
+
+
+@pytest.mark.parametrize("K,N,T", [(256, 64, 128), (2048, 577, 300), (7168, 2112, 300), (7168, 2112, 1000), (16384, 7168, 130)])
+def test_fp8_tiles_of_prompts_in_one_mfma_a_block(K, N, T, monkeypatch):
+    """The tiles of ktx_linear_forward_ws take a 128-block of an FP8 prompt in one MFMA of K = 128, with KTX_FP8_PROMPT_KERNEL=1 in four of K = 32:
+    within one bf16 ulp of each other, few outputs different, and of the oracle at the bound of this file; with a row count the eager bits."""
+    n = native()
+    torch.manual_seed(K + N + T)
+    w = (torch.randn(N, K) / 4).to(torch.float8_e4m3fn)
+    sc = (torch.rand((N + 127) // 128, K // 128) + 0.5) / 32
+    x = (torch.randn(T, K) / 10).to(torch.bfloat16).cuda()
+    h = n.LinearHandle(K, N, "FP8", 128, T)
+    h.load_fp8(w.cuda(), sc.cuda())
+    n.timing_enable(2)
+    try:
+        one = h.forward(x)
+        labels = [t[0] for t in n.timing_collect()]
+    finally:
+        n.timing_enable(0)
+    assert any("lin_tile_kernel" in t for t in labels), labels
+    rows = h.forward(x, bsz_tensor=torch.tensor([T], dtype=torch.int32, device="cuda"))
+    assert torch.equal(one, rows)
+    monkeypatch.setenv("KTX_FP8_PROMPT_KERNEL", "1")
+    four = h.forward(x)
+    close(one, linear_fp8_ref(x.cpu(), w, sc, None), rel=2e-3)
+    d = (one.float() - four.float()).abs()
+    assert bool((d <= 2.0 ** -7 * four.float().abs() + 2.0 ** -10 * float(four.float().abs().max())).all())
+    assert float((one != four).float().mean()) < 0.02
 
 
 @pytest.mark.parametrize("K,N,G", [(2048, 576, 64), (1536, 200, 32), (7168, 2112, 128), (1024, 64, -1), (384, 48, 128)])
@@ -782,3 +824,32 @@ def test_w4_prompts_off_the_gemm_multiply_exact_integers(G, K, N, T, how):
         assert float((eager.double() - want).norm() / want.norm()) > 2.0e-3     # (the eager call is the GEMM's)
     close(y, want.float().cpu())
     assert float((y.double() - want).norm() / want.norm()) < 2.0e-3
+
+
+@pytest.mark.parametrize("N", [24576, 24584])
+def test_bf16_prompts_on_the_gemm_of_decode_tiles(N):
+    """520 rows of 2048 -> 24576 (whole strips) and 24584 (half a strip at the end) fill the chip with 256 x 256 tiles over the whole K: the GEMM
+    reads the decode tiles and writes y itself.  Against 64-bit sums at the file's bound; into strided rows of a larger buffer; with a bias or a
+    row count the same sums go through fp32 to the tiles' epilogue: the same bits as the rounded sums with the bias added."""
+    n = native()
+    K, T = 2048, 520
+    torch.manual_seed(N)
+    w, x = (torch.randn(N, K, device="cuda") / 10).to(torch.bfloat16), (torch.randn(T, K, device="cuda") / 10).to(torch.bfloat16)
+    bias = (torch.randn(N, device="cuda") / 10).to(torch.bfloat16)
+    h, hb = n.LinearHandle(K, N, "BF16", 0, T), n.LinearHandle(K, N, "BF16", 0, T)
+    h.load_bf16(w)
+    hb.load_bf16(w, bias)
+    n.timing_enable(2)
+    try:
+        y = h.forward(x)
+        labels = [t[0] for t in n.timing_collect()]
+    finally:
+        n.timing_enable(0)
+    assert len(labels) == 1 and "gemm256_bf16_nt_kernel<bf16,tiles>" in labels[0], labels
+    close(y, (x.double() @ w.double().T).float().cpu())
+    wide = torch.zeros(T, K + 64, dtype=torch.bfloat16, device="cuda")
+    wide[:, 8:K + 8] = x
+    assert torch.equal(h.forward(wide[:, 8:K + 8]), y), "strided rows"
+    assert torch.equal(hb.forward(x), (y.float() + bias.float()).to(torch.bfloat16)), "bias"
+    got = h.forward(x, bsz_tensor=torch.tensor([T - 3], dtype=torch.int32, device="cuda"))
+    assert torch.equal(got[: T - 3], y[: T - 3]) and not bool(got[T - 3:].any())
