@@ -514,11 +514,16 @@ __device__ __forceinline__ float pf_sum_rows(float x) {
 // do) 256 dims of O.  S and O are computed transposed (tokens x heads, dims x heads), so that a lane owns ONE head: the softmax statistics are
 // one value a lane, and S^T leaves the MFMA with a lane's tokens where P^T enters the next one — the probabilities never leave the
 // registers (V's rows are read in the order 4 g + (0..3), 16 + 4 g + (0..3) that this gives lane group g).
-// What bounds it: the LDS, 576 KB read and 72 KB staged a step of a CU, beside 68 MFMAs a wavefront.  The rows are packed 1 KiB apart with
+// What bounds it: the LDS, 576 KB read and 72 KB staged a step of a CU, beside 100 MFMAs a wavefront.  The rows are packed 1 KiB apart with
 // their 16-byte pieces permuted by mla_swz, which keeps both the fragment reads of 16 rows and the transposed reads of 8 rows off each other's
-// banks.  128 heads, 8 requests of 2048 .. 8192 tokens, us for 64 tokens: mla_decode_kernel<4, 2> 5.8 (scores of half the dims exchanged
-// for every 32 tokens, softmax on 4 values a lane and head), this 2.5; no exchange, S computed by both wavefronts 2.9; a wavefront for itself,
-// 512 dims of O for 32 tokens, 3.1 (the registers are full, and every MFMA waits for its LDS read); rows padded to 1168 B + 0.5.
+// banks.
+// P enters the product as two bf16, the second what rounding the first left over.  One bf16 is off by its rounding except where P is exactly 1, a
+// split's largest entry, and here a split is longer than in mla_decode_kernel: the error against 64-bit sums grew by 1 to 4 % (32 requests
+// of 500 tokens, 128 heads 1.77e-3 -> 1.84e-3).  With two it is the outputs' rounding alone, 1.66e-3 at every size.
+// 128 heads, 8 requests, us for 64 tokens (8192 -> 16384 tokens each): mla_decode_kernel<4, 2> 4.2 (scores of half the dims exchanged for every 32
+// tokens, softmax on 4 values a lane and head), this 3.1; with P in one bf16 2.7.  With one bf16 also: no exchange, S computed by both wavefronts
+// + 0.4; a wavefront for itself, 512 dims of O for 32 tokens, + 0.6 (the registers are full, and every MFMA waits for its LDS read); rows
+// padded to 1168 B + 0.5.
 // distinct for 16 rows, also with rows 4 .. 11 flipped by 1 (ds_read_b128 takes lanes 0-3, 12-15, 20-23, 24-27 together); >> 1 distinct for rows
 // 0-7 and for 8-15 (ds_read_b64_tr_b16 takes 32 lanes together)
 __device__ __forceinline__ uint32_t mla_swz(uint32_t row) { return row & 8 ? ((row & 7) ^ 4) << 1 | 1 : (row & 7) << 1; }
@@ -696,6 +701,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       l_run = l_run * alpha + sum;
       m_run = m_new;
       const v8bf pf[2] = {as_v8bf(make_uint4(pk[0], pk[1], pk[2], pk[3])), as_v8bf(make_uint4(pk[4], pk[5], pk[6], pk[7]))};
+      // what the rounding left over
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+          pk[2 * t + h] = ktx_pk_bf16(st[t][2 * h] - __uint_as_float(pk[2 * t + h] << 16), st[t][2 * h + 1] - __uint_as_float(pk[2 * t + h] & 0xffff0000u));
+      const v8bf pl[2] = {as_v8bf(make_uint4(pk[0], pk[1], pk[2], pk[3])), as_v8bf(make_uint4(pk[4], pk[5], pk[6], pk[7]))};
       // the rescale only where some head's running maximum moved (alpha == 1 exactly otherwise)
       if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0ull) {
 #pragma unroll

@@ -104,6 +104,37 @@ def test_shared_workgroups_with_append_and_fewer_live_requests():
     assert torch.equal(kvd.cpu(), want)
 
 
+def decode_batch(Hq, lens, page=64, seed=7):
+    """A wrapper planned (with the longest context as its hint) for one token of each request, its run(), and the 64-bit result."""
+    from ktransformers_amd._native import MLAWrapper
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    B, pages = len(lens), [(n + page - 1) // page for n in lens]
+    first = [0] + list(np.cumsum(pages))
+    table = torch.randperm(first[-1], device=DEV, generator=g).to(torch.int32)
+    cache, q_nope, q_pe = (torch.randn(s, device=DEV, generator=g).to(torch.bfloat16) for s in ((first[-1], page, 576), (B, Hq, 512), (B, Hq, 64)))
+    w = MLAWrapper(B, first[-1], use_cuda_graph=False, device=DEV, max_q_tokens=B)
+    dev = [torch.tensor(a, dtype=torch.int32, device=DEV) for a in (range(B + 1), first, lens, [B])]
+    w.plan(dev[0], dev[1], table, dev[2], dev[3], Hq, 512, 64, page, 192 ** -0.5, max_kv_len=max(lens))
+
+    def exact():
+        out = []
+        for b, n in enumerate(lens):
+            rows = cache[table[first[b]:first[b + 1]].long()].view(-1, 576)[:n].double()
+            out.append(torch.softmax(torch.cat((q_nope[b], q_pe[b]), dim=1).double() @ rows.T * 192 ** -0.5, dim=1) @ rows[:, :512])
+        return torch.stack(out)
+    return (lambda: w.run(q_nope, q_pe, cache[:, :, :512], cache[:, :, 512:])), exact
+
+
+@pytest.mark.parametrize("Hq,lens", [(64, [1000] * 20), (128, [500] * 17 + [130, 64, 1]), (128, [8192, 2100, 5000, 8192, 8000, 7000, 6000, 64]), (64, [64, 33] * 10)])
+def test_wide_decode_is_off_by_the_rounding_of_its_outputs(Hq, lens):
+    """mla_decode_wide_kernel multiplies P as two bf16 (2^-17 of it is lost) and adds in fp32: against 64-bit sums the result is off by what rounding
+    the exact result to bf16 is off by, to 1 %."""
+    run, exact = decode_batch(Hq, lens)
+    want = exact()
+    floor = float((want.to(torch.bfloat16).double() - want).norm())
+    assert float((run().double() - want).norm()) <= 1.01 * floor
+
+
 def test_single_split_equals_many():
     run_case(16, 64, [3000], [1], seed=4, max_splits=1)
 
