@@ -735,6 +735,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int u = 0; u < 2; u++)
 #pragma unroll
           for (int i = 0; i < 2; i++) o[i * 8 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j & 1][i * 2 + u].v, pf[u], o[i * 8 + j], 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+          for (int i = 0; i < 2; i++) o[i * 8 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j & 1][i * 2 + u].v, pl[u], o[i * 8 + j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -925,21 +929,29 @@ extern "C" int ktx_mla_decode_partials(const ktx_mla_config* cfg, const void* d_
                          workspace_bytes, stream, nsplit_out);
 }
 
-// mla_decode_wide_kernel or mla_decode_kernel<4, 2> for a call of the 64-head shape?  The wide one takes 2.5 us for 64 tokens against 5.8 and shares
-// out what the requests hold, but its first step ends 3 us later: it needs some depth.  Measured at (query tokens x 64-token steps of the hint
-// x head blocks), <4, 2> | wide, us with the merge: 80 (8 requests of 300 tokens, 128 heads) 18 | 21, 256 (16 of 1000, 64 heads) 22 | 25, 512: 8 of
-// 2000 26 | 27, 16 of 1000 37 | 31, 1 of 32768 32 | 31, 1024: 4 of 8192 34 | 32, 2048: 8 of 8192 51 | 40.  Past 16 tokens <4, 2> is left with 16
-// splits a token and more workgroups than CUs: 32 of 500, 128 heads 62 | 38, 64 heads 32 | 28, 32 of 4096 110 | 71.
-static bool mla_wide_steps(const ktx_mla_config* cfg, int total_q_tokens, int shape) {
-  if (shape != 4 || total_q_tokens > 64) return false;
-  const long steps = ((long)cfg->kv_len_hint + 2 * MLA_TILE - 1) / (2 * MLA_TILE);
-  return total_q_tokens > 16 || steps * total_q_tokens * (cfg->num_heads / 64) >= 512;
+// mla_decode_wide_kernel or mla_decode_kernel<4, 2> for a call of the 64-head shape?  narrow: the splits that the latter would take.  The wide one
+// walks 64 tokens in 3.1 us against 4.2 and shares out what the requests hold, but its first step ends 3 us later, and its shares
+// write 256 workgroups' partials.  Measured with the merge (us, <4, 2> | wide, requests of equal length; of unequal ones the wide one gains 5-20 % more):
+//   one step of 64 tokens: 24 of 40, 64 heads 19 | 14 (nothing to merge);
+//   more workgroups of <4, 2> than CUs, a second round: 16 of 1000, 128 heads 38 | 32; 3 of 8192, 64 heads 34 | 29; 32 of 400, 64 heads (W = 224) 31 | 28;
+//     of 200 tokens at most lost: 20 of 200, 128 heads (W = 160) 32 | 32, unequal 27 | 31;
+//   one round: as <4, 2>'s splits deepen (in tiles of 32): 128 heads, 8 of 3000 (6) 31 | 33, of 4096 (8) 35 | 36, unequal 34 | 32, of 8192 (16) 52 | 49; 64 heads,
+//     where a split's partials weigh twice as much against its tokens, 8 of 4096 (8) 32 | 33, of 6000 (12) 40 | 37, 20 of 600 (2) 22 | 27.
+// Without a hint of the contexts' length: past 16 tokens.
+static bool mla_wide_steps(const ktx_mla_config* cfg, int total_q_tokens, int narrow) {
+  if (total_q_tokens > 64) return false;
+  if (cfg->kv_len_hint <= 0) return total_q_tokens > 16;
+  const long hblocks = cfg->num_heads / 64, steps = (cfg->kv_len_hint + 2 * MLA_TILE - 1) / (2 * MLA_TILE);
+  if (steps == 1) return true;
+  if (narrow * total_q_tokens * hblocks > 256) return steps * total_q_tokens * hblocks >= 192;
+  const int tiles = (cfg->kv_len_hint + MLA_TILE - 1) / MLA_TILE;
+  return (tiles + narrow - 1) / narrow >= (hblocks == 1 ? 10 : 8);
 }
 
 // Workgroup shape and KV split count of a decode call — one place, because the one-launch decode step (ktx_attn.hip) must
 // split the context exactly as the stand-alone kernel does to reproduce its partials bit for bit.
 static void mla_pick_shape(const ktx_mla_config* cfg, int total_q_tokens, size_t workspace_bytes, int* shape_out, int* nsplit_out,
-                           bool one_launch = false) {
+                           bool* wide_out, bool one_launch = false) {
   const int Hq = cfg->num_heads;
   // workgroup shape (head blocks x dim slices): decode-sized calls of many-headed models take 2x4 (32 heads share one staged
   // KV tile, 128 output dims per wave), prompts of those models 4x2, everything else 1x4
@@ -972,24 +984,27 @@ static void mla_pick_shape(const ktx_mla_config* cfg, int total_q_tokens, size_t
   if (long_hint) nsplit = std::min(nsplit, 128);
   if (shape == 2) nsplit = std::min(nsplit, std::max(16, 256 / std::max(1, hblocks * total_q_tokens)));
   if (ktx_debug_get(7) > 0) nsplit = ktx_debug_get(7);
-  if (cfg->kv_len_hint > 0) {
-    // no more splits than tiles — and no more than the deepest split needs: with T tiles dealt round-robin the launch takes
-    // ceil(T / nsplit) tiles' time, so the smallest split count with that depth writes the fewest partials for the merge to read
-    const int unit = mla_wide_steps(cfg, total_q_tokens, shape) ? 2 * MLA_TILE : MLA_TILE;   // (mla_decode_wide_kernel's steps)
-    const int tiles = std::max(1, (cfg->kv_len_hint + unit - 1) / unit);
-    nsplit = std::min(nsplit, tiles);
-    const int depth = (tiles + nsplit - 1) / nsplit;
-    if (ktx_debug_get(7) <= 0) nsplit = (tiles + depth - 1) / depth;
-  }
+  // no more splits than tiles — and no more than the deepest split needs: with T tiles dealt round-robin the launch takes
+  // ceil(T / nsplit) tiles' time, so the smallest split count with that depth writes the fewest partials for the merge to read
+  auto splits_of = [&](int unit) {
+    if (cfg->kv_len_hint <= 0) return nsplit;
+    const int tiles = std::max(1, (cfg->kv_len_hint + unit - 1) / unit), n = std::min(nsplit, tiles), depth = (tiles + n - 1) / n;
+    return ktx_debug_get(7) <= 0 ? (tiles + depth - 1) / depth : n;
+  };
+  const int narrow = splits_of(MLA_TILE);
+  const bool wide = shape == 4 && mla_wide_steps(cfg, total_q_tokens, narrow);
+  nsplit = wide ? splits_of(2 * MLA_TILE) : narrow;   // (mla_decode_wide_kernel's steps)
   // <= 256 splits: the merge kernel keeps splits/16 partial rows per thread in registers (NS = 16 is its largest, spill-free
   // instantiation); longer contexts simply put more 32-token tiles into each split
   nsplit = std::min(nsplit, std::min(256, std::max(1, cfg->max_splits)));
   nsplit = (int)std::min<size_t>((size_t)nsplit, workspace_bytes / ((size_t)total_q_tokens * Hq * (MLA_DC + 2) * sizeof(float)));
   *shape_out = shape;
   *nsplit_out = nsplit;
+  *wide_out = wide;
 }
 extern "C" int ktx_mla_decode_nsplit(const ktx_mla_config* cfg, int total_q_tokens, size_t workspace_bytes) {   // ktx_internal.h
   int shape = 0, nsplit = 0;
+  bool wide = false;
   if (!cfg || total_q_tokens <= 0) return 0;
   // Up to 40 K tokens the one launch wins with deeper 2x4 splits: 61.7 vs 68.4 us per layer at 12 K, 64.1 vs 72.0 at 16 K, 77.9 vs 80.5 at
   // 32 K, 81.7 vs 83.4 at 36 K, even from 40 K on (84.8 / 84.8; 48 K 95.1 vs 89.0 before phase C's staging fast path) — the five launches
@@ -997,7 +1012,7 @@ extern "C" int ktx_mla_decode_nsplit(const ktx_mla_config* cfg, int total_q_toke
   // before the launch lost 7 us to section 4.1.6).
   const int bound_k = ktx_debug_get(1);   // dev knob 1: the bound in K tokens (scripts/attn_fused_bench.py, ATTN_BOUND_K)
   if (cfg->kv_len_hint >= (bound_k > 0 ? bound_k * 1024 : 40960)) return 0;
-  mla_pick_shape(cfg, total_q_tokens, workspace_bytes, &shape, &nsplit, true);
+  mla_pick_shape(cfg, total_q_tokens, workspace_bytes, &shape, &nsplit, &wide, true);
   return shape == 2 ? nsplit : 0;   // the one-launch step is built on the 2x4 workgroup shape only
 }
 
@@ -1018,8 +1033,8 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
   hipStream_t st = (hipStream_t)stream;
   const int Hq = cfg->num_heads;
   int shape = 0, nsplit = 0;
-  mla_pick_shape(cfg, total_q_tokens, workspace_bytes, &shape, &nsplit);
-  const bool wide = mla_wide_steps(cfg, total_q_tokens, shape);
+  bool wide = false;
+  mla_pick_shape(cfg, total_q_tokens, workspace_bytes, &shape, &nsplit, &wide);
   const int hbw = shape, nwv = shape == 1 ? 4 : 8;
   const int hblocks = Hq / (16 * hbw);
   KTX_REQUIRE(nsplit >= 1, "ktx_mla_decode: workspace too small");

@@ -135,6 +135,24 @@ def test_wide_decode_is_off_by_the_rounding_of_its_outputs(Hq, lens):
     assert float((run().double() - want).norm()) <= 1.01 * floor
 
 
+@pytest.mark.parametrize("Hq,lens,wide", [(64, [600] * 20, False), (64, [300] * 24, False), (128, [200] * 16, False), (64, [16384] * 2, False), (128, [2000] * 8, False),
+                                          (64, [50] * 20, True), (64, [1000] * 20, True), (128, [1000] * 12, True), (128, [8192] * 8, True), (64, [8192] * 3, True)])
+def test_which_decode_kernel_a_batch_takes(Hq, lens, wide):
+    """The 64-token kernel where it was measured faster (mla_wide_steps): whole second rounds of the other one's workgroups, deep splits, one step; not
+    for short contexts in one round.  Both within the bound of the outputs' rounding and P's."""
+    from ktransformers_amd import _native as n
+    run, exact = decode_batch(Hq, lens)
+    n.timing_enable(2)
+    try:
+        out = run()
+        labels = [t[0] for t in n.timing_collect()]
+    finally:
+        n.timing_enable(0)
+    assert any("mla_decode_wide_kernel" in t for t in labels) == wide, labels
+    want = exact()
+    assert float((out.double() - want).norm() / want.norm()) < 2.4e-3      # (sqrt(2) of 1.66e-3: outputs and probabilities in bf16)
+
+
 def test_single_split_equals_many():
     run_case(16, 64, [3000], [1], seed=4, max_splits=1)
 
