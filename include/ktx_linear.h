@@ -117,10 +117,12 @@ int ktx_linear_decode_eligible(ktx_linear_t h, int T);
  * ktx_linear_workspace_bytes says how much d_ws such a call of T rows needs; 0: none (d_ws may be NULL).  plain: 1 for a call without
  * d_bsz, addends and GLU (long bf16 prompts then need none).  d_ws: device memory, 16-byte
  * aligned, used by this call alone until its work on `stream` is done.  Calls that the tiles don't cover (no or too little d_ws,
- * in_features % 128 != 0, rows that are not 16-byte aligned, decode-sized T) run as ktx_linear_forward_fused.  `fusion` may be NULL.
+ * in_features % 128 != 0, rows that are not 16-byte aligned, decode-sized T) or are slower for (short K, a chip that the strips fill) run as
+ * ktx_linear_forward_fused.  `fusion` may be NULL.
  * prompt (FP8, T > 32): 1 takes a 128-block in one K = 128 MFMA instead of four of K = 32 (the order of ktx_linear_forward): the same
  * error against 64-bit sums, other last bits.  W4 multiplies exact integers, as ktx_linear_forward does. */
 size_t ktx_linear_workspace_bytes(ktx_linear_t h, int T, int plain);
+int ktx_linear_tiled(ktx_linear_t h, int T);   /* 1: ktx_linear_forward_ws takes T rows on the tiles (or the GEMM), given its scratch */
 int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T, const void* d_x, void* d_y, const ktx_linear_fusion* fusion,
                           int prompt, void* d_ws, size_t ws_bytes, ktx_stream_t stream);
 

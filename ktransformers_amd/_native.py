@@ -136,6 +136,7 @@ def _load() -> C.CDLL:
                                              C.c_void_p]
     lib.ktx_linear_workspace_bytes.argtypes = [C.c_void_p, C.c_int, C.c_int]
     lib.ktx_linear_workspace_bytes.restype = C.c_size_t
+    lib.ktx_linear_tiled.argtypes = [C.c_void_p, C.c_int]
     lib.ktx_linear_forward_ws.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.POINTER(_LinearFusion), C.c_int, C.c_void_p,
                                           C.c_size_t, C.c_void_p]
     lib.ktx_linear_decode_eligible.argtypes = [C.c_void_p, C.c_int]
@@ -649,6 +650,7 @@ class LinearHandle:
         self.device, self.fmt, self.K, self.N, self.max_len = dev, fmt, in_features, out_features, max_len
         self.group_size = {"BF16": 0, "FP8": 128}.get(fmt, group_size)
         self.batch = max(int(batch), 1)
+        self._ws_need: dict = {}
         cfg = _LinearConfig(in_features, out_features, LIN_FMT[fmt], self.group_size, max_len, dev.index or 0, self.batch)
         h = C.c_void_p()
         check(lib.ktx_linear_create(C.byref(cfg), C.byref(h)))
@@ -673,6 +675,7 @@ class LinearHandle:
 
     def _bias(self, bias):
         self._bias_t = None if bias is None else self._chk(bias, torch.bfloat16, (self.N,), "bias")
+        self._ws_need.clear()
         return self._bias_t
 
     # ---- prompt-sized W4 calls: de-quantise once (Marlin's rounding), then the library's own BF16 GEMM (csrc/ktx_gemm.hip;
@@ -711,11 +714,13 @@ class LinearHandle:
         return y
 
     # ---- prompt-sized FP8 calls: act_quant once per call + the block-scaled fp8 GEMM on the handle's own tiles
-    # (csrc/ktx_linear_fp8gemm.inc; bit-identical to ktx_linear_forward; KTX_FP8_PROMPT_KERNEL=1 keeps the strip kernel for A/B) ----
+    # (csrc/ktx_linear_fp8gemm.inc; a 128-block in one MFMA of K = 128, within a bf16 ulp of ktx_linear_forward; KTX_FP8_PROMPT_KERNEL=1: four of
+    # K = 32, on the kernels of ktx_linear_forward_ws) ----
     FP8_PROMPT_MIN_T = 128
-    FP8_CHUNKED_MAX_T = 1024    # up to here a call with K > 2048 cuts K (ktx_linear_forward_ws): 300 rows of 7168 -> 2112 93 us here, 28 there;
-                                # where K stays whole the 128 x 128 tiles of this path give the same bits, and win on large products
-    FP8_GEMM_MIN_OUT = 4 << 20  # (256 rows of 1536 -> 24576: 31 us against 37; 1000 rows of 2048 -> 576: 36 against 20)
+    # T * N past which the GEMM's 128 x 128 tiles fill the chip and win over the tiles of ktx_linear_forward_ws (us, GEMM | there: 384 rows of 2560 -> 12008
+    # 46 | 54, 700 of 5120 -> 9000 77 | 85, 700 of 2048 -> 7168 41 | 39; below, 300 of 7168 -> 2112 93 | 28, 1000 of 7168 -> 4096 98 | 66).  Those cut a K past
+    # 2048 up to 1024 rows; whole it loses earlier (1500 of 7168 -> 2112 102 | 115, 2048 of 4096 -> 1000 67 | 44; 1025 of 2048 -> 3072 38 | 31)
+    FP8_GEMM_OUT = (4 << 20, 3 << 20)
 
     def _prompt_forward_fp8(self, x2: torch.Tensor, out, add1, add2, glu: bool) -> torch.Tensor:
         T = x2.shape[0]
@@ -810,7 +815,8 @@ class LinearHandle:
             if norm is not None:
                 x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)
             return self._prompt_forward(x2, out, add1, add2, glu).reshape(*x.shape[:-1], n_out)
-        if (self.fmt == "FP8" and gemm_ok and T >= self.FP8_PROMPT_MIN_T and (T > self.FP8_CHUNKED_MAX_T or self.K <= 2048) and T * self.N >= self.FP8_GEMM_MIN_OUT and not os.environ.get("KTX_FP8_PROMPT_KERNEL")):
+        if (self.fmt == "FP8" and gemm_ok and T >= self.FP8_PROMPT_MIN_T and T * self.N > self.FP8_GEMM_OUT[T > 1024 and self.K > 2048]
+                and not os.environ.get("KTX_FP8_PROMPT_KERNEL")):
             if norm is not None:
                 x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)
             return self._prompt_forward_fp8(x2, out, add1, add2, glu).reshape(*x.shape[:-1], n_out)
@@ -823,8 +829,9 @@ class LinearHandle:
                 raise KtxError("forward: bsz_tensor must be int32 on the handle's device")
             bsz = bsz_tensor.data_ptr()
         if norm is None and add1 is None and add2 is None and not strided and not glu:
-            if T > 8:
-                self._forward_ws(bsz, T, x2, out, None)
+            need = self._scratch(T, bsz is None) if T > 8 else None
+            if need is not None:
+                self._forward_ws(bsz, T, x2, out, None, need)
             else:
                 check(lib.ktx_linear_forward(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), _stream_ptr(self.device)))
             return out.reshape(*x.shape[:-1], self.N)
@@ -846,16 +853,24 @@ class LinearHandle:
                 setattr(fu, name, a2.data_ptr())
                 setattr(fu, name + "_ld", a2.stride(0))
                 keep.append(a2)
-        if T > 8:
-            self._forward_ws(bsz, T, x2, out, C.byref(fu))
+        need = self._scratch(T, False) if T > 8 else None
+        if need is not None:
+            self._forward_ws(bsz, T, x2, out, C.byref(fu), need)
         else:
             check(lib.ktx_linear_forward_fused(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), C.byref(fu), _stream_ptr(self.device)))
         return out.reshape(*x.shape[:-1], n_out)
 
-    def _forward_ws(self, bsz, T: int, x2: torch.Tensor, out: torch.Tensor, fu) -> None:
+    def _scratch(self, T: int, plain: bool):
+        """Bytes of scratch that ktx_linear_forward_ws takes for T rows, or None where it runs as ktx_linear_forward does.  Kept: a function of the
+        handle's sizes and of whether it has a bias, and two calls into the library beside a launch of 12 us."""
+        key = T if plain else -T
+        if key not in self._ws_need:
+            self._ws_need[key] = int(lib.ktx_linear_workspace_bytes(self._h, T, int(plain))) if lib.ktx_linear_tiled(self._h, T) else None
+        return self._ws_need[key]
+
+    def _forward_ws(self, bsz, T: int, x2: torch.Tensor, out: torch.Tensor, fu, need: int) -> None:
         """ktx_linear_forward_ws with its scratch from torch's allocator (freed to the stream's pool behind the launches).  FP8 prompts take the
         K = 128 MFMA whether the call is eager, captured or has its row count on the device."""
-        need = int(lib.ktx_linear_workspace_bytes(self._h, T, 1 if bsz is None and fu is None else 0))
         ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
         prompt = self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")
         check(lib.ktx_linear_forward_ws(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), fu, 1 if prompt else 0, ws.data_ptr() if need else None, need,

@@ -2154,6 +2154,11 @@ extern "C" size_t ktx_linear_workspace_bytes(ktx_linear_t h, int T, int plain) {
   return tile_plan(h, T, &o) ? o.part_bytes + o.sT_bytes + o.xq_bytes : 0;
 }
 
+extern "C" int ktx_linear_tiled(ktx_linear_t h, int T) {
+  LinTilePlan o;
+  return h && tile_eligible(h, T) && (gemm_parts(h, T) || tile_plan(h, T, &o)) ? 1 : 0;
+}
+
 extern "C" int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T, const void* d_x, void* d_y, const ktx_linear_fusion* fu,
                                      int prompt, void* d_ws, size_t ws_bytes, ktx_stream_t stream) {
   KTX_REQUIRE(h && d_x && d_y, "ktx_linear_forward_ws: null argument");

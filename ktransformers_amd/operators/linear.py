@@ -146,8 +146,8 @@ class KLinearMarlin(KLinearBase):
         decode GEMVs and prompt GEMM of csrc/ktx_linear.hip.
       * num_bits = 8: the native W8 format (round 4) — one byte per weight + bf16 group scales in HBM, Marlin's own multiplicand
         bf16((q - 128) * s) formed in registers in front of the bf16 MFMA: the same products and fp32 accumulation as
-        gptq_marlin_gemm's 8-bit path, bit-identical to holding that matrix as a BF16 handle (which is what rounds 2-3 did, and what
-        still happens for group sizes the W8 tiles do not carry: anything but 32, 64 or a multiple of 128).
+        gptq_marlin_gemm's 8-bit path, bit-identical to holding that matrix as a BF16 handle below the 256 rows where that one may take
+        the GEMM (and what still happens for group sizes the W8 tiles do not carry: anything but 32, 64 or a multiple of 128).
       * act_order: the reference "simulates" it by a random permutation of the K rows of the STORED q_w with g_idx / sort_indices
         undoing it inside the kernel (quant_utils.py:15-33,82-92) — scales and quantised values are computed before the permutation,
         so the product x @ dequant(w) is the same matrix product; this layout needs no such permutation and the flag is accepted."""

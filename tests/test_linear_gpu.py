@@ -130,8 +130,7 @@ def test_fp8_prompt_gemm_against_the_strip_kernel(K, N, T, monkeypatch):
     if N % 16 == 0 and bias is None:
         calls.append(dict(glu=True))
     # the GEMM at every size (ktx_linear_forward_ws would take most of these), and the strip kernel itself to compare with (dev knob 12 keeps it)
-    monkeypatch.setattr(n.LinearHandle, "FP8_CHUNKED_MAX_T", 0)
-    monkeypatch.setattr(n.LinearHandle, "FP8_GEMM_MIN_OUT", 0)
+    monkeypatch.setattr(n.LinearHandle, "FP8_GEMM_OUT", (0, 0))
     n.timing_enable(2)
     try:
         h.forward(x)
@@ -163,7 +162,7 @@ def test_fp8_prompt_gemm_against_the_strip_kernel(K, N, T, monkeypatch):
     close(fast[0], linear_fp8_ref(x.cpu(), w, sc, bias), rel=2e-3)
 
 
-@pytest.mark.parametrize("K,N,T", [(256, 64, 128), (2048, 577, 300), (7168, 2112, 300), (7168, 2112, 1000), (16384, 7168, 130)])
+@pytest.mark.parametrize("K,N,T", [(1024, 64, 128), (2048, 577, 300), (7168, 2112, 300), (7168, 2112, 1000), (16384, 7168, 130)])
 def test_fp8_tiles_of_prompts_in_one_mfma_a_block(K, N, T, monkeypatch):
     """The tiles of ktx_linear_forward_ws take a 128-block of an FP8 prompt in one MFMA of K = 128, with KTX_FP8_PROMPT_KERNEL=1 in four of K = 32:
     within one bf16 ulp of each other, few outputs different, and of the oracle at the bound of this file; with a row count the eager bits."""
@@ -739,7 +738,7 @@ def test_five_to_eight_rows_run_as_four_row_passes_of_the_decode_kernel(fmt, K, 
 
 @pytest.mark.parametrize("fmt", ["W4", "FP8", "BF16"])
 @pytest.mark.parametrize("K,N,T", [(128, 17, 9), (384, 200, 33), (2176, 577, 16), (7168, 2112, 65), (2176, 1040, 130), (2048, 4104, 300),
-                                   (7168, 1536, 513), (2048, 12288, 520)])
+                                   (5248, 577, 16), (2816, 1040, 40), (7168, 1536, 513), (2048, 12288, 520)])
 def test_batches_and_short_prompts_on_tiles(fmt, K, N, T):
     """ktx_linear_forward_ws (ktx_linear_tile.inc; BF16 of 256 rows and more, where they fill the chip, the GEMM's 256 x 256 tiles in parts of K):
     ragged rows, features and last k-chunk, split and whole K, bias, addends, GLU, strided and misaligned rows, a device-side row count —
@@ -853,3 +852,29 @@ def test_bf16_prompts_on_the_gemm_of_decode_tiles(N):
     assert torch.equal(hb.forward(x), (y.float() + bias.float()).to(torch.bfloat16)), "bias"
     got = h.forward(x, bsz_tensor=torch.tensor([T - 3], dtype=torch.int32, device="cuda"))
     assert torch.equal(got[: T - 3], y[: T - 3]) and not bool(got[T - 3:].any())
+
+
+@pytest.mark.parametrize("fmt,K,N,T,kernel", [
+    ("BF16", 2048, 7168, 192, "lin_gemm_kernel"), ("BF16", 1536, 4096, 48, "lin_gemm_kernel"), ("BF16", 7168, 2112, 64, "lin_tile_kernel"),
+    ("BF16", 4096, 1000, 1025, "lin_gemm_kernel"), ("BF16", 2048, 12288, 1000, "gemm256_bf16_nt_kernel"),
+    ("W8", 2048, 3072, 64, "lin_gemm_kernel"), ("W8", 7168, 2112, 64, "lin_tile_kernel"), ("W8", 7168, 2112, 700, "lin_gemm_kernel"),
+    ("W4", 2048, 3072, 16, "lin_gemm"), ("W4", 7168, 2112, 16, "lin_tile_kernel"), ("W4", 1536, 2048, 48, "lin_tile_kernel"),
+    ("FP8", 2048, 3072, 16, "lin_gemm_kernel"), ("FP8", 2048, 3072, 48, "lin_tile_kernel"), ("FP8", 5120, 9000, 700, "lin_fp8_gemm_kernel"),
+    ("FP8", 7168, 2112, 1500, "lin_fp8_gemm_kernel"), ("FP8", 2048, 3072, 1025, "lin_tile_kernel")])
+def test_which_kernel_a_batch_takes(fmt, K, N, T, kernel):
+    """Strip kernels, tiles or GEMM, where each was measured faster (lin_tile_wins, lin_gemm_parts, LinearHandle.FP8_GEMM_OUT)."""
+    n = native()
+    h = n.LinearHandle(K, N, fmt, {"W4": 64, "W8": 64, "FP8": 128, "BF16": 0}[fmt], T)
+    if fmt == "FP8":
+        h.load_fp8(torch.randn(N, K, device="cuda").to(torch.float8_e4m3fn), torch.ones((N + 127) // 128, K // 128, device="cuda"))
+    elif fmt == "W8":
+        h.load_w8(torch.randint(0, 256, (K, N), dtype=torch.uint8, device="cuda"), torch.ones(K // 64, N, dtype=torch.bfloat16, device="cuda"))
+    else:
+        h.load_bf16(torch.randn(N, K, device="cuda").to(torch.bfloat16))
+    n.timing_enable(2)
+    try:
+        h.forward(torch.randn(T, K, device="cuda").to(torch.bfloat16))
+        labels = [t[0] for t in n.timing_collect()]
+    finally:
+        n.timing_enable(0)
+    assert any(t.startswith(kernel) for t in labels), labels
