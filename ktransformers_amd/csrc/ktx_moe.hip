@@ -1761,13 +1761,13 @@ struct RawGemmParams {
 
 // Bound by the weights' bytes while an expert sees a token or two (a decode batch: 16 tokens over 384 experts) and by the VALU from about four
 // on: a scale product, a conversion and an fma per (token, weight row, 4 k).  So the work per (weight row, 4 k) follows the tile's rows
-// (1, 2 or up to 4: a v_dot4 per token, from 3 on one 4x4x4 MFMA for all of them: the same integers), and D = 2 512-k steps of weights stay
-// requested per wavefront, two workgroups per CU (4 steps spill).  The kernel before it did four tokens' work for every tile and kept 408 registers (one
+// (1, 2 or up to 4: a v_dot4 per token, from 3 on one 4x4x4 MFMA for all of them: the same integers), and a 512-k step of weights (of gate and up
+// both) stays requested per wavefront, with two workgroups per CU, four for down (two steps of gate|up spill).  The kernel before it did four tokens' work for every tile and kept 408 registers (one
 // wavefront per SIMD, one step in flight): 16 tokens at Kimi-K2's sizes, gate|up + down: 489 + 150 us -> 262 + 133 (2.1 GB of weights and scales: 390 us at the
 // rate a large read reaches).
-template <int D, bool GATE_UP>
+template <bool GATE_UP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATE_UP ? 2 : 4, 4))) void moe_rawint4_rows_kernel(RawGemmParams p) {
-  constexpr int NMAT = GATE_UP ? 2 : 1;
+  constexpr int NMAT = GATE_UP ? 2 : 1, D = NMAT;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int KP = p.K + 32;                                        // padded activation row (bank spread of the 4 tokens)
   int8_t* xq = reinterpret_cast<int8_t*>(smem);                   // [4][K+32]
@@ -1784,7 +1784,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATE_UP ? 2
   const int NS = p.K / 512, G = p.K / 32;
   const int L = lane >> 2, j = lane & 3, hsel = L >> 3;
 
-  // (step, matrix) pairs in turns through a ring of D slots; the launcher picks D so that it divides their number
+  // (step, matrix) pairs in turns through a ring of D slots
   struct Slot { uint4 w[4], s[4]; };
   const uint8_t* wb[NMAT];
   const bf16_t* sb[NMAT];
@@ -2224,7 +2224,7 @@ __global__ __launch_bounds__(256) void moe_actquant_kgroup_kernel(const bf16_t* 
 
 // =====================================================================================================
 // Decode fast path of the RAWINT4 experts (qlen*k <= KTX_DEC_MAX_PAIRS): the two-launch structure of the other formats with
-// the arithmetic of moe_rawint4_gemm_kernel above for ONE token: lane (L, j) needs only token 0's entry of each 4x4x4 block
+// the arithmetic of moe_rawint4_rows_kernel above for ONE token: lane (L, j) needs only token 0's entry of each 4x4x4 block
 // product, which is a plain 4-element int8 dot (v_dot4c_i32_i8) — same integers, a quarter of the registers.  Before this path a decode token went bucket -> x-quant -> gate/up -> requant -> down -> combine: six
 // launches with a one-step prefetch; here the per-32-group activation quantisation (BufferASmallKGroupImpl::from_mat,
 // amx_buffers.hpp:431-495) happens in the consuming workgroup and the RAW tiles stream through a D-step register ring.
@@ -2260,7 +2260,7 @@ __device__ __forceinline__ RawSlot raw_load_slot(const uint8_t* wb, const bf16_t
   return r;
 }
 // acc[rg] += the step's 8 blocks of 64 k for the lane's (AVX lane L, weight row j); xa = LDS int8 row + 4L, as1 = LDS group
-// scales + hsel.  Same expression order as compute_step of moe_rawint4_gemm_kernel (token 0 of its 4).
+// scales + hsel.  Same expression order as compute of moe_rawint4_rows_kernel.
 __device__ __forceinline__ void raw_dec_step(const RawSlot& sl, const int8_t* xa, const float* as1, int st, float (&acc)[4]) {
 #pragma unroll
   for (int kb8 = 0; kb8 < 8; kb8++) {
@@ -3443,15 +3443,10 @@ static int launch_rawint4(const RawGemmParams& p, int max_tiles, hipStream_t st)
   const size_t lds = 4 * (size_t)(p.K + 32) + (size_t)(p.K / 32) * 16;
   KTX_REQUIRE(lds <= 96 * 1024, "ktx_moe_forward: K too large for the RAWINT4 kernel");
   const dim3 grid((p.N / 16 + 3) / 4, max_tiles);
-  const int total = p.K / 512 * (GATE_UP ? 2 : 1);   // (step, matrix) pairs: the ring's depth divides them
-  auto go = [&](auto kern) {
-    KTX_HIP(ktx_set_max_lds(reinterpret_cast<const void*>(kern), 96 * 1024));
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p);
-    KTX_HIP(hipGetLastError());
-    return 0;
-  };
-  if constexpr (GATE_UP) return go(moe_rawint4_rows_kernel<2, GATE_UP>);
-  else return go(moe_rawint4_rows_kernel<1, GATE_UP>);
+  KTX_HIP(ktx_set_max_lds(reinterpret_cast<const void*>(moe_rawint4_rows_kernel<GATE_UP>), 96 * 1024));
+  hipLaunchKernelGGL((moe_rawint4_rows_kernel<GATE_UP>), grid, dim3(256), lds, st, p);
+  KTX_HIP(hipGetLastError());
+  return 0;
 }
 
 template <bool GATE_UP>
