@@ -192,9 +192,10 @@ int ktx_linear_dequant_bf16(ktx_linear_t h, void* d_out, int64_t ld_out, ktx_str
  *                        amax(x[t][128 kb .. 128 kb + 127]) / 448 (block-major, so a tile's scales of one k-step are contiguous);
  *   ktx_linear_gemm_fp8 — y bf16 [T][ldy] = fp8_gemm(d_q, scales, W, scale_inv) (+ bias): 128 x 128 output tiles, k-step = one
  *                        128-block, accumulator += dot * a_s * b_s (fp8gemm.py:156).  s_ld >= ceil(T / 128) * 128, a multiple of 4.
- * Same products and scalings as ktx_linear_forward on the same handle; the decode layout of the weights is read in place.  Columns
- * [T, min(s_ld, ceil(T / 128) * 128)) of d_scales_t are set to zero. */
+ * Same products and scalings as ktx_linear_forward on the same handle; the decode layout of the weights is read in place.  The GEMM reads
+ * the scales of whole tiles of 128 rows: ktx_fp8_act_quant writes those of T rows, ktx_fp8_act_quant_padded zeros for the others too. */
 int ktx_fp8_act_quant(const void* d_x, int64_t ldx, int T, int K, void* d_q, float* d_scales_t, int64_t s_ld, ktx_stream_t stream);
+int ktx_fp8_act_quant_padded(const void* d_x, int64_t ldx, int T, int K, void* d_q, float* d_scales_t, int64_t s_ld, ktx_stream_t stream);
 int ktx_linear_gemm_fp8(ktx_linear_t h, const void* d_q, const float* d_scales_t, int64_t s_ld, int T, void* d_y, int64_t ldy,
                         ktx_stream_t stream);
 

@@ -2204,7 +2204,7 @@ extern "C" int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T
   q.sT = (const float*)(ws + o.part_bytes);
   q.xq = ws + o.part_bytes + o.sT_bytes;
   if (h->cfg.format == KTX_LIN_FP8) {
-    const int rc = ktx_fp8_act_quant(d_x, ldx, T, p.Kx, (void*)q.xq, (float*)q.sT, q.s_ld, stream);
+    const int rc = ktx_fp8_act_quant_padded(d_x, ldx, T, p.Kx, (void*)q.xq, (float*)q.sT, q.s_ld, stream);
     if (rc) return rc;
     return prompt && o.mt >= 4 ? forward_tile<F_FP8, 128, true>(o, q, st) : forward_tile<F_FP8, 128>(o, q, st);
   }

@@ -190,6 +190,21 @@ def test_fp8_tiles_of_prompts_in_one_mfma_a_block(K, N, T, monkeypatch):
     assert float((one != four).float().mean()) < 0.02
 
 
+@pytest.mark.parametrize("T", [1, 127, 128, 130])
+def test_fp8_act_quant_writes_its_rows_only(T):
+    """ktx_fp8_act_quant leaves the scales behind its T rows as they are (they may be another call's); the padded form zeroes them up to whole tiles."""
+    n = native()
+    K, ld = 384, 512
+    x = torch.randn(T, K, device="cuda").to(torch.bfloat16)
+    q = torch.empty(T, K, dtype=torch.uint8, device="cuda")
+    want = (x.float().view(T, K // 128, 128).abs().amax(-1) / 448.0).T
+    for fn, zeros in ((n.lib.ktx_fp8_act_quant, T), (n.lib.ktx_fp8_act_quant_padded, (T + 127) // 128 * 128)):
+        sT = torch.full((K // 128, ld), 7.0, device="cuda")
+        n.check(fn(x.data_ptr(), K, T, K, q.data_ptr(), sT.data_ptr(), ld, torch.cuda.current_stream().cuda_stream))
+        torch.testing.assert_close(sT[:, :T], want, rtol=2.0 ** -22, atol=0.0)      # (an ulp: torch may multiply by the reciprocal)
+        assert not bool(sT[:, T:zeros].any()) and bool((sT[:, zeros:] == 7.0).all())
+
+
 @pytest.mark.parametrize("K,N,G", [(2048, 576, 64), (1536, 200, 32), (7168, 2112, 128), (1024, 64, -1), (384, 48, 128)])
 def test_w8_format_is_the_bf16_kernel_on_marlins_multiplicand_bit_for_bit(K, N, G):
     """The W8 format (include/ktx_linear.h: KTX_LIN_W8, round 4): one byte per weight in HBM, bf16((q - 128) * s) formed in registers
