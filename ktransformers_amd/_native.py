@@ -730,7 +730,7 @@ class LinearHandle:
         st = torch.empty((self.K // 128, tp), dtype=torch.float32, device=self.device)
         y = torch.empty((T, self.N), dtype=torch.bfloat16, device=self.device)
         sp = _stream_ptr(self.device)
-        check(lib.ktx_fp8_act_quant(x2.data_ptr(), x2.stride(0), T, self.K, q.data_ptr(), st.data_ptr(), tp, sp))
+        check(lib.ktx_fp8_act_quant_padded(x2.data_ptr(), x2.stride(0), T, self.K, q.data_ptr(), st.data_ptr(), tp, sp))
         check(lib.ktx_linear_gemm_fp8(self._h, q.data_ptr(), st.data_ptr(), tp, T, y.data_ptr(), self.N, sp))
         if glu:   # rows are interleaved per 16-row strip as [8 gate | 8 up]
             y = silu_mul(y.view(T, self.N // 16, 2, 8).permute(0, 2, 1, 3).reshape(T, self.N))
@@ -872,9 +872,12 @@ class LinearHandle:
     def _forward_ws(self, bsz, T: int, x2: torch.Tensor, out: torch.Tensor, fu, need: int) -> None:
         """ktx_linear_forward_ws with its scratch from torch's allocator (freed to the stream's pool behind the launches).  FP8 prompts take the
         K = 128 MFMA whether the call is eager, captured or has its row count on the device."""
-        ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
+        try:
+            ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
+        except torch.cuda.OutOfMemoryError:   # (the strip kernels need none)
+            ws, need = None, 0
         prompt = self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")
-        check(lib.ktx_linear_forward_ws(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), fu, 1 if prompt else 0, ws.data_ptr() if need else None, need,
+        check(lib.ktx_linear_forward_ws(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), fu, 1 if prompt else 0, ws.data_ptr() if ws is not None else None, need,
                                         _stream_ptr(self.device)))
 
     def _forward_glu_in(self, x, bsz_tensor, out, norm, add1, add2, glu):

@@ -893,3 +893,29 @@ def test_which_kernel_a_batch_takes(fmt, K, N, T, kernel):
     finally:
         n.timing_enable(0)
     assert any(t.startswith(kernel) for t in labels), labels
+
+
+def test_a_batch_without_memory_for_scratch_runs_on_the_strip_kernels(monkeypatch):
+    """The scratch is a want, not a need: where the allocator has none left the call runs as it does without, on the strip kernels."""
+    n = native()
+    K, N, T = 7168, 264, 48
+    torch.manual_seed(1)
+    w, x = (torch.randn(N, K) / 10).to(torch.bfloat16), (torch.randn(T, K) / 10).to(torch.bfloat16)
+    h = n.LinearHandle(K, N, "W4", 64, T)
+    h.load_bf16(w.cuda())
+    real, xc = torch.empty, x.cuda()
+
+    def empty(*a, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.cuda.OutOfMemoryError("none left")
+        return real(*a, **kw)
+    monkeypatch.setattr(torch, "empty", empty)
+    n.timing_enable(2)
+    try:
+        y = h.forward(xc)
+        labels = [t[0] for t in n.timing_collect()]
+    finally:
+        n.timing_enable(0)
+        monkeypatch.undo()
+    assert len(labels) == 1 and labels[0].startswith("lin_gemm"), labels
+    close(y, linear_w4_ref(x, *quantize_weights_ref(w.T.contiguous(), 64), 64))
