@@ -1918,7 +1918,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATE_UP ? 2
 // The VALU has more to do per MFMA than anything else here, so the operands are what costs it least: codes and nibbles as f16 integers, whose sum
 // over a group the f16 MFMA gives exactly and in fp32 already (below 2^15), so that a 16 x 16 fragment and group takes a scale product and an fma
 // per output where an int8 MFMA takes a conversion as well: the terms are the reference's, with any scale.  A group's 8 weights of a lane
-// become f16 in 12 operations for all token fragments: a nibble goes to the top mantissa bits of an f16 (16 + q'), minus 24 is q.
+// become f16 in 10 operations for all token fragments: a nibble becomes the low mantissa bits of 1024 where it lies, or after a shift by a byte.
 // (The weight's scale inside the f16 operand saves the scale products, at 2048 tokens 4 %, but holds for scales of 2^-17 .. 2^11 only and rounds
 // otherwise than the reference's terms.)
 //
@@ -1930,8 +1930,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATE_UP ? 2
 //   multiplies while the other waits); K walks in the RAW step of 512, the activations in halves of it.  The next half's activations
 //   (LDS-DMA, XOR-swizzled rows; only the live 16-row groups) and the next step's weights (registers) are requested before the MFMAs
 //   and waited for behind them.
-// At Kimi-K2's sizes, us for the whole forward, int8 operands staged through registers -> here (the same bits): 64 tokens 1409 -> 996, 256
-// 2313 -> 1705, 1000 3537 -> 2884, 2048 5084 -> 4392.
+// At Kimi-K2's sizes, us for the whole forward, int8 operands staged through registers -> here (the same bits): 64 tokens 1409 -> 951, 256
+// 2313 -> 1631, 1000 3537 -> 2804, 2048 5084 -> 4255.
 // =====================================================================================================
 typedef _Float16 raw_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 raw_h8 __attribute__((ext_vector_type(8)));
@@ -1939,10 +1939,13 @@ __device__ __forceinline__ uint32_t raw_h2_bits(raw_h2 v) { return __builtin_bit
 // the pairs (byte 0, byte 2) and (byte 1, byte 3) of the low (par 0) or high nibbles of x; x: two's complement nibbles ^ 8
 template <int PAR>
 __device__ __forceinline__ void raw_widen(uint32_t x, uint32_t mask, uint32_t top, uint32_t& o0, uint32_t& o1) {
-  const uint32_t e0 = ((PAR ? x << 2 : x << 6) & mask) | top, e1 = ((PAR ? x >> 6 : x >> 2) & mask) | top;
-  const raw_h2 m24 = {(_Float16)-24.0f, (_Float16)-24.0f};
-  o0 = raw_h2_bits(__builtin_bit_cast(raw_h2, e0) + m24);
-  o1 = raw_h2_bits(__builtin_bit_cast(raw_h2, e1) + m24);
+  auto value = [](uint32_t e) {   // low nibbles 1024 + q' -> q' - 8; high ones 1024 + 16 q' -> q' - 8
+    const raw_h2 v = __builtin_bit_cast(raw_h2, e);
+    if constexpr (PAR == 0) return raw_h2_bits(v + raw_h2{(_Float16)-1032.0f, (_Float16)-1032.0f});
+    else return raw_h2_bits(__builtin_elementwise_fma(v, raw_h2{(_Float16)0.0625f, (_Float16)0.0625f}, raw_h2{(_Float16)-72.0f, (_Float16)-72.0f}));
+  };
+  o0 = value((x & mask) | top);
+  o1 = value(((x >> 8) & mask) | top);
 }
 
 template <bool GATE_UP>
@@ -2046,9 +2049,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   const uint32_t xo0 = i * 512 + ((kc ^ i) * 16);   // row i's piece kc; piece 4 c + kc: ^ 64 c
   // constants the compiler cannot see through: and + or become one v_and_or_b32
-  uint32_t mask, top;
-  asm("s_mov_b32 %0, 0x03C003C0" : "=s"(mask));
-  asm("v_mov_b32 %0, 0x4C004C00" : "=v"(top));
+  uint32_t mask[2], top;
+  asm("s_mov_b32 %0, 0x000F000F" : "=s"(mask[0]));
+  asm("s_mov_b32 %0, 0x00F000F0" : "=s"(mask[1]));
+  asm("v_mov_b32 %0, 0x64006400" : "=v"(top));
 
   // MTL = 16-token groups of the tile that hold rows (a Kimi-K2 chunk of 2048 tokens leaves ~43 rows per expert: three groups,
   // not four, for most tiles); one instantiation per count, chosen once per workgroup.  Groups are fenced from each other: left alone, the compiler
@@ -2079,8 +2083,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const uint32_t S = kb8 < 2 ? sv.x : kb8 < 4 ? sv.y : kb8 < 6 ? sv.z : sv.w;
         bs[g & 1][u] = __uint_as_float((kb8 & 1) ? (S & 0xffff0000u) : (S << 16));
         uint32_t o[4];
-        raw_widen<(kb8 & 1)>(P0, mask, top, o[0], o[1]);
-        raw_widen<(kb8 & 1)>(P1, mask, top, o[2], o[3]);
+        raw_widen<(kb8 & 1)>(P0, mask[kb8 & 1], top, o[0], o[1]);
+        raw_widen<(kb8 & 1)>(P1, mask[kb8 & 1], top, o[2], o[3]);
         bop[u] = __builtin_bit_cast(raw_h8, make_uint4(o[0], o[1], o[2], o[3]));
       }
     };
