@@ -514,9 +514,11 @@ __device__ __forceinline__ float pf_sum_rows(float x) {
 // do) 256 dims of O.  S and O are computed transposed (tokens x heads, dims x heads), so that a lane owns ONE head: the softmax statistics are
 // one value a lane, and S^T leaves the MFMA with a lane's tokens where P^T enters the next one — the probabilities never leave the
 // registers (V's rows are read in the order 4 g + (0..3), 16 + 4 g + (0..3) that this gives lane group g).
-// What bounds it: the LDS, 576 KB read and 72 KB staged a step of a CU, beside 100 MFMAs a wavefront.  The rows are packed 1 KiB apart with
-// their 16-byte pieces permuted by mla_swz, which keeps both the fragment reads of 16 rows and the transposed reads of 8 rows off each other's
-// banks.
+// What bounds it: a step's three phases, S, softmax and O, which its two barriers keep one after the other in both wavefronts of a SIMD.  Of a step's
+// 7400 cycles the LDS works 2900 (576 KB read), the matrix pipe 3200 (100 MFMAs a wavefront), the vector ALU 2500 (rocprofv3 counters of
+// the whole launch, 8 requests of 2048 .. 8192 tokens: 13, 18 and 21 % busy, no bank conflicts, two thirds of the waves' time waits).  The rows are
+// packed 1 KiB apart with their 16-byte pieces permuted by mla_swz, which keeps both the fragment reads of 16 rows and the transposed reads of
+// 8 rows off each other's banks.
 // P enters the product as two bf16, the second what rounding the first left over.  One bf16 is off by its rounding except where P is exactly 1, a
 // split's largest entry, and here a split is longer than in mla_decode_kernel: the error against 64-bit sums grew by 1 to 4 % (32 requests
 // of 500 tokens, 128 heads 1.77e-3 -> 1.84e-3).  With two it is the outputs' rounding alone, 1.66e-3 at every size.

@@ -1915,7 +1915,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATE_UP ? 2
 // (tests/test_moe_gpu.py::test_rawint4_prompt_chunks).  Decode and short batches (qlen < 64) keep the exact kernels; dev knob 29 = 1
 // forces them for every size.
 //
-// The VALU has more to do per MFMA than anything else here, so the operands are what costs it least: codes and nibbles as f16 integers, whose sum
+// The vector ALU bounds it, 16 instructions an MFMA and busy 78 % of the time at 2048 tokens of Kimi-K2's sizes (the matrix pipe 19, rocprofv3 counters),
+// so the operands are what costs it least: codes and nibbles as f16 integers, whose sum
 // over a group the f16 MFMA gives exactly and in fp32 already (below 2^15), so that a 16 x 16 fragment and group takes a scale product and an fma
 // per output where an int8 MFMA takes a conversion as well: the terms are the reference's, with any scale.  A group's 8 weights of a lane
 // become f16 in 10 operations for all token fragments: a nibble becomes the low mantissa bits of 1024 where it lies, or after a shift by a byte.
