@@ -38,6 +38,7 @@
 #include "../../include/ktx_moe.h"
 #include "ktx_common.h"
 #include "ktx_internal.h"
+#include "ktx_moe_raw.h"
 
 // (the error slot — ktx_fail / ktx_last_error — lives in ktx_err.hip, which the small sequence-mixer library links as well)
 
@@ -49,14 +50,6 @@
 namespace ktxw4 {
 #include "ktx_w4_step.inc"
 }
-
-struct Tile {
-  int expert;  // local expert index
-  int row0;    // first sorted row
-  int nrows;   // <= 16*MT
-  int idx;     // place among its expert's tiles
-  int cnt;     // the expert's tiles
-};
 
 // Workgroup -> (tile, strip group) of a grouped GEMM, from a one-dimensional grid: ids are dealt round-robin to the 8 XCDs, so id % 8 is the
 // XCD.  The jobs lie expert after expert, within an expert strip group by strip group, the group's tiles side by side; each XCD takes an
@@ -545,14 +538,6 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(GemmParams p) {
 // moe_pick_job's eighths against tiles in launch order: 256 experts of 7168 x 2048, 64 rows each 1631 -> 1580 us, 64 of 6144 x 3072, 256: 1326 -> 1284.
 // Integer arithmetic and epilogue are those of moe_gemm_kernel, so results are bit-identical.
 // =====================================================================================================
-template <int N, class F, int I = 0>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, F, I + 1>(static_cast<F&&>(f));
-  }
-}
-
 template <int WBITS, int MT, int D, bool GATE_UP>
 __global__ __launch_bounds__(512) void moe_gemm_stream_kernel(GemmParams p, int kch) {
   constexpr int NJ = 4;                              // (strip, matrix) units per wave
@@ -1745,19 +1730,6 @@ __global__ void pack_wfp_kernel(const uint8_t* __restrict__ src, int N, int K, i
 // high nibble = q[row j][64*(8*step+2p+1) + 4L + b] (two's complement nibbles), so ((P<<4)&0xF0F0F0F0, P&0xF0F0F0F0)
 // are the two B operands (multiplicand 16q, as in the reference).  Scales stay bf16: [rg][step][row j][h][8 blocks].
 // =====================================================================================================
-struct RawGemmParams {
-  const uint8_t *w0, *w1;      // RAW tiles (gate | down, up)
-  const bf16_t *s0, *s1;       // bf16 scales in the tile order above
-  size_t expert_stride;        // bytes of weights per expert matrix
-  size_t scale_stride;         // bf16 elements of scales per expert matrix
-  int N, K;
-  const int8_t* act_q;         // [src rows][K]
-  const float* act_d;          // [src rows][K/32]
-  const int32_t* row_src;
-  const Tile* tiles;           // <= 4 rows per tile
-  const int32_t* counters;
-  bf16_t* out;                 // [sorted rows][N]
-};
 
 // Bound by the weights' bytes while an expert sees a token or two (a decode batch: 16 tokens over 384 experts) and by the VALU from about four
 // on: a scale product, a conversion and an fma per (token, weight row, 4 k).  So the work per (weight row, 4 k) follows the tile's rows
@@ -1904,286 +1876,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GATE_UP ? 2
   if (tile.nrows == 1) body(std::integral_constant<int, 1>{});
   else if (tile.nrows == 2) body(std::integral_constant<int, 2>{});
   else body(std::integral_constant<int, 4>{});
-}
-
-// =====================================================================================================
-// RAWINT4 prompt chunks: the same products on the 16x16x32 f16 MFMA, one MFMA per (32-k group) x (16 rows) x (16 tokens).
-//
-// The exact kernel above keeps the reference's SIXTEEN fp32 lane accumulators per output.  A prompt chunk does not need that
-// association: the terms of an output are the per-group sums  as[t][g] * bs[n][g] * sum_{k in g} a[t][k] * q[n][k]  — the reference adds
-// them as 16 interleaved chains + a tree, this kernel as ONE chain over the groups in k order, held to the bound of the FP8 / BF16 formats
-// (tests/test_moe_gpu.py::test_rawint4_prompt_chunks).  Decode and short batches (qlen < 64) keep the exact kernels; dev knob 29 = 1
-// forces them for every size.
-//
-// The vector ALU bounds it, 16 instructions an MFMA and busy 78 % of the time at 2048 tokens of Kimi-K2's sizes (the matrix pipe 19, rocprofv3 counters),
-// so the operands are what costs it least: codes and nibbles as f16 integers, whose sum
-// over a group the f16 MFMA gives exactly and in fp32 already (below 2^15), so that a 16 x 16 fragment and group takes a scale product and an fma
-// per output where an int8 MFMA takes a conversion as well: the terms are the reference's, with any scale.  A group's 8 weights of a lane
-// become f16 in 10 operations for all token fragments: a nibble becomes the low mantissa bits of 1024 where it lies, or after a shift by a byte.
-// (The weight's scale inside the f16 operand saves the scale products, at 2048 tokens 4 %, but holds for scales of 2^-17 .. 2^11 only and rounds
-// otherwise than the reference's terms.)
-//
-// No second copy of the weights: the RAW tiles are read as they lie in HBM.  MFMA lane (i = lane & 15, kc = lane >> 4) needs
-// row i's eight nibbles k = 64 kb + 32 h + 8 kc + [0, 8) of group (kb, h): those are the pieces (L, j) = (8h + 2kc + o, i & 3),
-// o = 0 / 1, of RAW tile rg = i >> 2 — so the lane loads exactly its four pieces q = (h, o) of the strip's four tiles and nothing moves
-// between lanes; inside 8 k the pairs come out as (0,2) (1,3) (4,6) (5,7), the order in which the activation codes are stored.
-//   workgroup = 4 wavefronts = 4 strips of 16 weight rows x (gate, up), or 8 strips of down, x 64 tokens, two workgroups per CU (one
-//   multiplies while the other waits); K walks in the RAW step of 512, the activations in halves of it.  The next half's activations
-//   (LDS-DMA, XOR-swizzled rows; only the live 16-row groups) and the next step's weights (registers) are requested before the MFMAs
-//   and waited for behind them.
-// At Kimi-K2's sizes, us for the whole forward, int8 operands staged through registers -> here (the same bits): 64 tokens 1409 -> 951, 256
-// 2313 -> 1631, 1000 3537 -> 2804, 2048 5084 -> 4255.
-// =====================================================================================================
-typedef _Float16 raw_h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 raw_h8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ uint32_t raw_h2_bits(raw_h2 v) { return __builtin_bit_cast(uint32_t, v); }
-// the pairs (byte 0, byte 2) and (byte 1, byte 3) of the low (par 0) or high nibbles of x; x: two's complement nibbles ^ 8
-template <int PAR>
-__device__ __forceinline__ void raw_widen(uint32_t x, uint32_t mask, uint32_t top, uint32_t& o0, uint32_t& o1) {
-  auto value = [](uint32_t e) {   // low nibbles 1024 + q' -> q' - 8; high ones 1024 + 16 q' -> q' - 8
-    const raw_h2 v = __builtin_bit_cast(raw_h2, e);
-    if constexpr (PAR == 0) return raw_h2_bits(v + raw_h2{(_Float16)-1032.0f, (_Float16)-1032.0f});
-    else return raw_h2_bits(__builtin_elementwise_fma(v, raw_h2{(_Float16)0.0625f, (_Float16)0.0625f}, raw_h2{(_Float16)-72.0f, (_Float16)-72.0f}));
-  };
-  o0 = value((x & mask) | top);
-  o1 = value(((x >> 8) & mask) | top);
-}
-
-template <bool GATE_UP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_rawint4_chunk_kernel(RawGemmParams p) {
-  constexpr int NW = 4, NU = 2;                     // NU weight operands per wavefront share one activation fragment: (gate, up) of a
-                                                    // strip, or two strips of down
-  constexpr int TOK = 64, MT = 4;
-  constexpr int XB = TOK * 512, AB = 8 * TOK * 4;   // half a step (256 k): activation codes (f16), their group scales [8 groups][64 tokens]
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][XB] | [2][AB]
-  __shared__ int s_src[TOK];
-  uint8_t* xs = smem;
-  float* as_l = reinterpret_cast<float*>(smem + 2 * XB);
-
-  const int tile_idx = blockIdx.y;
-  if (tile_idx >= p.counters[0]) return;
-  const Tile tile = p.tiles[tile_idx];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nstrips = p.N / 16;
-  const int NS = p.K / 512, G = p.K / 32;
-  const int i = lane & 15, kc = lane >> 4, rg = i >> 2, j = i & 3;
-  int ustrip[NU];
-#pragma unroll
-  for (int u = 0; u < NU; u++) ustrip[u] = GATE_UP ? blockIdx.x * NW + wave : (blockIdx.x * NW + wave) * 2 + u;
-  const bool wave_ok = ustrip[0] < nstrips;
-
-  // rows past the tile read its first row again (their outputs are never stored)
-  if (tid < TOK) {
-    const int r = tile.row0 + (tid < tile.nrows ? tid : 0);
-    s_src[tid] = p.row_src ? p.row_src[r] : r;
-  }
-  __syncthreads();
-  const int mt_live = (tile.nrows + 15) >> 4;
-
-  // ---- this lane's four pieces of each unit's four RAW tiles, and its row's scales (a strip past N aliases strip 0, not stored)
-  const uint8_t* wb[NU];        // uniform bases + 32-bit lane offsets: the registers are full
-  const uint8_t* sb[NU];
-  uint32_t wo[NU], so[NU];
-#pragma unroll
-  for (int u = 0; u < NU; u++) {
-    const int st = ustrip[u] < nstrips ? ustrip[u] : 0;
-    wb[u] = ((GATE_UP && u) ? p.w1 : p.w0) + (size_t)tile.expert * p.expert_stride + (size_t)(st * 4) * NS * 1024;
-    sb[u] = reinterpret_cast<const uint8_t*>(((GATE_UP && u) ? p.s1 : p.s0) + (size_t)tile.expert * p.scale_stride + (size_t)(st * 4) * NS * 64);
-    wo[u] = (uint32_t)(rg * NS * 1024 + ((2 * kc) * 4 + j) * 16);
-    so[u] = (uint32_t)(rg * NS * 128 + j * 32);
-  }
-  struct WStep { uint4 w[NU][4]; uint4 s[NU][2]; };   // w[u][h * 2 + o]: piece L = 8h + 2kc + o; s[u][h]: 8 bf16 scales (kb = 0..7)
-  constexpr int WLOADS = NU * 6;
-  auto load_w = [&](WStep& d, int st) {
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        d.w[u][q] = *reinterpret_cast<const uint4*>(wb[u] + (size_t)st * 1024 + wo[u] + ((q >> 1) * 8 + (q & 1)) * 64);
-#pragma unroll
-      for (int h = 0; h < 2; h++) d.s[u][h] = *reinterpret_cast<const uint4*>(sb[u] + (size_t)st * 128 + so[u] + h * 16);
-    }
-  };
-  // The compiler does not see the DMAs and would wait for them together with the weights' registers at their first use, behind the NEXT
-  // requests: the registers pass an empty asm behind the step's own wait, where everything has landed.
-  auto settle = [&](WStep& d) {
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        asm volatile("" : "+v"(d.w[u][q].x), "+v"(d.w[u][q].y), "+v"(d.w[u][q].z), "+v"(d.w[u][q].w));
-        d.w[u][q].x ^= 0x88888888u; d.w[u][q].y ^= 0x88888888u; d.w[u][q].z ^= 0x88888888u; d.w[u][q].w ^= 0x88888888u;   // raw_widen's q'
-      }
-#pragma unroll
-      for (int h = 0; h < 2; h++) asm volatile("" : "+v"(d.s[u][h].x), "+v"(d.s[u][h].y), "+v"(d.s[u][h].z), "+v"(d.s[u][h].w));
-    }
-  };
-
-  // ---- staging: a wavefront brings 16 rows (one DMA instruction: two rows of 512 B; LDS slot s of row r holds the row's 16-byte piece with
-  // its low 4 bits ^ (r & 15)) and the scales of 2 groups (lane = row)
-  const uint32_t lds_x = (uint32_t)(uintptr_t)xs, lds_a = (uint32_t)(uintptr_t)as_l;
-  auto stage = [&](int hs, int buf) {
-    const uint32_t aoff = (uint32_t)s_src[lane] * (uint32_t)G * 4u;   // (rows x groups x 4 B < 4 GiB: checked by the launcher)
-    if (wave < mt_live) {
-#pragma unroll
-      for (int c = 0; c < 8; c++) {
-        const int row = wave * 16 + c * 2 + (lane >> 5), slot = lane & 31;
-        const int8_t* src = p.act_q + (size_t)s_src[row] * (size_t)(p.K * 2) + (size_t)hs * 512 + ((slot & 16) | ((slot ^ row) & 15)) * 16;
-        moe_dma(src, lds_x + buf * XB + (wave * 16 + c * 2) * 512);
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      const int g = wave * 2 + c;
-      gg_dma4(p.act_d + (size_t)hs * 8 + g, aoff, lds_a + buf * AB + g * (TOK * 4));
-    }
-  };
-
-  float acc[NU][MT][4];
-#pragma unroll
-  for (int u = 0; u < NU; u++)
-#pragma unroll
-    for (int t = 0; t < MT; t++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) acc[u][t][r] = 0.0f;
-
-  const uint32_t xo0 = i * 512 + ((kc ^ i) * 16);   // row i's piece kc; piece 4 c + kc: ^ 64 c
-  // constants the compiler cannot see through: and + or become one v_and_or_b32
-  uint32_t mask[2], top;
-  asm("s_mov_b32 %0, 0x000F000F" : "=s"(mask[0]));
-  asm("s_mov_b32 %0, 0x00F000F0" : "=s"(mask[1]));
-  asm("v_mov_b32 %0, 0x64006400" : "=v"(top));
-
-  // MTL = 16-token groups of the tile that hold rows (a Kimi-K2 chunk of 2048 tokens leaves ~43 rows per expert: three groups,
-  // not four, for most tiles); one instantiation per count, chosen once per workgroup.  Groups are fenced from each other: left alone, the compiler
-  // widens a whole step's weights up front and spills them.
-  auto compute_n = [&](auto mtl, auto hc, const WStep& w, int buf) __attribute__((always_inline)) {
-    constexpr int MTL = decltype(mtl)::value, HALF = decltype(hc)::value;
-    if (!wave_ok) return;
-    const uint8_t* xb = xs + buf * XB;
-    const float* ab = as_l + buf * (AB / 4) + kc * 4;
-    raw_h8 af[MTL];
-    float4 sf[2][MTL];
-    auto load_a = [&](int g) __attribute__((always_inline)) {
-#pragma unroll
-      for (int t = 0; t < MTL; t++) af[t] = *reinterpret_cast<const raw_h8*>(xb + (xo0 ^ ((g & 3) * 64)) + (g >> 2) * 256 + t * 8192);
-    };
-    auto load_s = [&](int g) __attribute__((always_inline)) {
-#pragma unroll
-      for (int t = 0; t < MTL; t++) sf[g & 1][t] = *reinterpret_cast<const float4*>(ab + g * TOK + t * 16);
-    };
-    float bs[2][NU];   // the groups' weight scales, of the lane's row
-    auto widen = [&](raw_h8 (&bop)[NU], auto gc) __attribute__((always_inline)) {
-      constexpr int g = decltype(gc)::value, kb8 = HALF * 4 + (g >> 1), h = g & 1;   // g = (kb8 of the half) * 2 + h
-#pragma unroll
-      for (int u = 0; u < NU; u++) {
-        const uint4 &w0 = w.w[u][h * 2], &w1 = w.w[u][h * 2 + 1], &sv = w.s[u][h];
-        const uint32_t P0 = kb8 < 2 ? w0.x : kb8 < 4 ? w0.y : kb8 < 6 ? w0.z : w0.w;
-        const uint32_t P1 = kb8 < 2 ? w1.x : kb8 < 4 ? w1.y : kb8 < 6 ? w1.z : w1.w;
-        const uint32_t S = kb8 < 2 ? sv.x : kb8 < 4 ? sv.y : kb8 < 6 ? sv.z : sv.w;
-        bs[g & 1][u] = __uint_as_float((kb8 & 1) ? (S & 0xffff0000u) : (S << 16));
-        uint32_t o[4];
-        raw_widen<(kb8 & 1)>(P0, mask[kb8 & 1], top, o[0], o[1]);
-        raw_widen<(kb8 & 1)>(P1, mask[kb8 & 1], top, o[2], o[3]);
-        bop[u] = __builtin_bit_cast(raw_h8, make_uint4(o[0], o[1], o[2], o[3]));
-      }
-    };
-    // a group's MFMAs, the next group's operands behind them, then the group's sums
-    raw_h8 bop[2][NU];
-    load_a(0);
-    load_s(0);
-    widen(bop[0], std::integral_constant<int, 0>{});
-    static_for<8>([&](auto gc) __attribute__((always_inline)) {
-      constexpr int g = decltype(gc)::value;
-      constexpr int TB = MTL < 2 ? MTL : 2;   // (the sums of all fragments at once do not fit the registers)
-#pragma unroll
-      for (int t0 = 0; t0 < MTL; t0 += TB) {
-        v4f d[TB][NU];
-#pragma unroll
-        for (int t = 0; t < TB && t0 + t < MTL; t++)
-#pragma unroll
-          for (int u = 0; u < NU; u++) d[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t0 + t], bop[g & 1][u], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-        if constexpr (g + 1 < 8) {
-          if (t0 + TB >= MTL) { load_a(g + 1); load_s(g + 1); }
-          if (t0 == 0) widen(bop[(g + 1) & 1], std::integral_constant<int, (g + 1) & 7>{});
-        }
-#pragma unroll
-        for (int t = 0; t < TB && t0 + t < MTL; t++) {
-          const float4 sv = sf[g & 1][t0 + t];
-          const float asv[4] = {sv.x, sv.y, sv.z, sv.w};
-#pragma unroll
-          for (int u = 0; u < NU; u++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[u][t0 + t][r] = fmaf(asv[r] * bs[g & 1][u], d[t][u][r], acc[u][t0 + t][r]);
-        }
-        if constexpr (TB < MTL) __builtin_amdgcn_sched_barrier(0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    });
-  };
-  auto compute = [&](auto hc, const WStep& w, int buf) __attribute__((always_inline)) {
-    if (mt_live >= 4) compute_n(std::integral_constant<int, 4>{}, hc, w, buf);
-    else if (mt_live == 3) compute_n(std::integral_constant<int, 3>{}, hc, w, buf);
-    else if (mt_live == 2) compute_n(std::integral_constant<int, 2>{}, hc, w, buf);
-    else compute_n(std::integral_constant<int, 1>{}, hc, w, buf);
-  };
-  using H0 = std::integral_constant<int, 0>;
-  using H1 = std::integral_constant<int, 1>;
-  // one step: the second half's activations are requested before the first half's MFMAs, the next step's weights behind them (they have the
-  // whole step to arrive), the next step's first half before the second half's MFMAs
-  // (unconditional, the last step's requests repeat: the compiler cannot pair a load and a settle under two branches, and waits)
-  auto step = [&](WStep& w, WStep& next, int st) __attribute__((always_inline)) {
-    stage(2 * st + 1, 1);
-    load_w(next, min(st + 1, NS - 1));
-    compute(H0{}, w, 0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(WLOADS) : "memory");   // the DMAs; the weights' loads are younger
-    __syncthreads();
-    stage(min(2 * st + 2, 2 * NS - 1), 0);
-    compute(H1{}, w, 1);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    settle(next);
-    __syncthreads();
-  };
-
-  WStep wa, wb2;
-  load_w(wa, 0);
-  stage(0, 0);
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-  settle(wa);
-  __syncthreads();
-  for (int st = 0; st < NS; st += 2) {
-    step(wa, wb2, st);
-    if (st + 1 < NS) step(wb2, wa, st + 1);
-  }
-
-  if (!wave_ok) return;
-  if constexpr (GATE_UP) {
-    const int n = ustrip[0] * 16 + i;
-#pragma unroll
-    for (int t = 0; t < MT; t++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = t * 16 + kc * 4 + r;
-        if (row < tile.nrows) {
-          const bf16_t gv = f32_to_bf16(acc[0][t][r]), uv = f32_to_bf16(acc[1][t][r]);
-          p.out[(size_t)(tile.row0 + row) * p.N + n] = f32_to_bf16(act_fn(bf16_to_f32(gv), bf16_to_f32(uv)));
-        }
-      }
-  } else {
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      if (ustrip[u] >= nstrips) continue;
-      const int n = ustrip[u] * 16 + i;
-#pragma unroll
-      for (int t = 0; t < MT; t++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int row = t * 16 + kc * 4 + r;
-          if (row < tile.nrows) p.out[(size_t)(tile.row0 + row) * p.N + n] = f32_to_bf16(acc[u][t][r]);
-        }
-    }
-  }
 }
 
 // HALF: the codes as f16 integers, 8 k in the order (0,2) (1,3) (4,6) (5,7) of moe_rawint4_chunk_kernel's weights
@@ -2498,15 +2190,17 @@ __global__ void pack_rawint4_kernel(const uint8_t* __restrict__ src, int N, int 
   out[idx] = v;
 }
 
-// bf16 scales [N][K/32] -> tile order [rg][step][row j][h][8 blocks]; one thread per element
-__global__ void pack_rawint4_scales_kernel(const bf16_t* __restrict__ src, int N, int K, bf16_t* __restrict__ out) {
+// bf16 scales [N][K/32] -> tile order [rg][step][row j][h][8 blocks]; one thread per element.  *outside: set if one is outside raw_scale_fits
+__global__ void pack_rawint4_scales_kernel(const bf16_t* __restrict__ src, int N, int K, bf16_t* __restrict__ out, int* outside) {
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int G = K / 32, NS = K / 512;
   if (idx >= (size_t)N * G) return;
   const int kb8 = (int)(idx % 8), h = (int)((idx / 8) % 2), jrow = (int)((idx / 16) % 4);
   const size_t t = idx / 64;
   const int st = (int)(t % NS), rg = (int)(t / NS);
-  out[idx] = src[(size_t)(rg * 4 + jrow) * G + 2 * (8 * st + kb8) + h];
+  const bf16_t s = src[(size_t)(rg * 4 + jrow) * G + 2 * (8 * st + kb8) + h];
+  out[idx] = s;
+  if (!raw_scale_fits(s)) atomicOr(outside, 1);
 }
 
 #include "ktx_moe_gguf.inc"
@@ -2574,6 +2268,7 @@ struct ktx_moe_s {
   int gg_type[3] = {0, 0, 0};     // GGUF: ggml type of gate / up / down
   size_t gg_stride[3] = {0, 0, 0};
   bool loaded_gguf = false;
+  int* raw_outside = nullptr;     // RAWINT4, [expert]: not 0 where a weight scale does not fit the prompt kernel's operands (raw_scale_fits)
   bool exact = false;             // ktx_moe_set_exact: no path of this handle may re-associate the reference's fp32 sums
 };
 
@@ -2682,7 +2377,7 @@ extern "C" int ktx_moe_create(const ktx_moe_config* cfg, ktx_moe_t* out) {
 extern "C" int ktx_moe_destroy(ktx_moe_t h) {
   if (!h) return 0;
   DeviceGuard _dg(h->cfg.device);
-  void* ptrs[] = {h->gate_w, h->up_w, h->down_w, h->gate_s, h->up_s, h->down_s, h->gate_r, h->up_r, h->down_r, h->mask};
+  void* ptrs[] = {h->gate_w, h->up_w, h->down_w, h->gate_s, h->up_s, h->down_s, h->gate_r, h->up_r, h->down_r, h->mask, h->raw_outside};
   for (void* p : ptrs)
     if (p) hipFree(p);
   delete h;
@@ -2889,6 +2584,8 @@ extern "C" int ktx_moe_load_rawint4(ktx_moe_t h, const void* d_gate, const void*
   KTX_ON_DEVICE(h->cfg.device);
   const int E = h->cfg.expert_num, H = h->cfg.hidden_size, I = h->cfg.intermediate_size;
   const size_t dwords = (size_t)I * H / 8, nsc = (size_t)I * (H / 32);
+  if (!h->raw_outside) KTX_HIP(hipMalloc(&h->raw_outside, E * sizeof(int)));
+  KTX_HIP(hipMemset(h->raw_outside, 0, E * sizeof(int)));
   for (int e = 0; e < E; e++) {
     const uint8_t* src[3] = {(const uint8_t*)d_gate + (size_t)e * I * H / 2, (const uint8_t*)d_up + (size_t)e * I * H / 2,
                              (const uint8_t*)d_down + (size_t)e * H * I / 2};
@@ -2901,7 +2598,7 @@ extern "C" int ktx_moe_load_rawint4(ktx_moe_t h, const void* d_gate, const void*
       hipLaunchKernelGGL(pack_rawint4_kernel, dim3((unsigned)((dwords + 255) / 256)), dim3(256), 0, 0, src[m], Ns[m], Ks[m],
                          reinterpret_cast<uint32_t*>(dst[m]));
       hipLaunchKernelGGL(pack_rawint4_scales_kernel, dim3((unsigned)((nsc + 255) / 256)), dim3(256), 0, 0, ssrc[m], Ns[m],
-                         Ks[m], sdst[m]);
+                         Ks[m], sdst[m], h->raw_outside + e);
     }
   }
   KTX_HIP(hipGetLastError());
@@ -3454,17 +3151,6 @@ static int launch_rawint4(const RawGemmParams& p, int max_tiles, hipStream_t st)
   return 0;
 }
 
-template <bool GATE_UP>
-static int launch_rawint4_chunk(const RawGemmParams& p, int max_tiles, hipStream_t st) {
-  constexpr size_t lds = 2 * (64 * 512 + 8 * 64 * 4);
-  const hipError_t err = ktx_set_max_lds(reinterpret_cast<const void*>(moe_rawint4_chunk_kernel<GATE_UP>), (int)lds);
-  KTX_HIP(err);
-  const int per_wg = GATE_UP ? 4 : 8;       // strips per workgroup of 4 wavefronts (down: two strips per wavefront)
-  hipLaunchKernelGGL((moe_rawint4_chunk_kernel<GATE_UP>), dim3((p.N / 16 + per_wg - 1) / per_wg, max_tiles), dim3(256), lds, st, p);
-  KTX_HIP(hipGetLastError());
-  return 0;
-}
-
 // RAWINT4: bucket (4-row tiles) -> per-group activation quant -> gate/up -> per-group requant -> down -> combine
 static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const int64_t* d_expert_ids,
                            const float* d_weights, const void* d_input, void* d_output, int flags, hipStream_t st) {
@@ -3515,7 +3201,7 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   const bool chunk = qlen >= 64 && g_dbg[29] != 1 && !h->exact && (size_t)npairs * (std::max(H, I) / 32) * 4 < ((size_t)1 << 32);
   PrepParams pp;
   pp.d_bsz = d_bsz; pp.qlen = qlen; pp.k = k; pp.E = E; pp.expert_begin = h->cfg.expert_begin; pp.H = H;
-  pp.rows_per_tile = chunk ? 64 : 4; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
+  pp.rows_per_tile = chunk ? RAW_ROWS : 4; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
   pp.x_q = ws->x_q; pp.x_d = ws->x_d; pp.row_of_pair = ws->row_of_pair; pp.src_of_row = ws->src_of_row;
   pp.tiles = ws->tiles; pp.counters = ws->counters;
   {
@@ -3528,11 +3214,11 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   RawGemmParams g1;
   g1.w0 = h->gate_w; g1.w1 = h->up_w; g1.s0 = (const bf16_t*)h->gate_s; g1.s1 = (const bf16_t*)h->up_s;
   g1.expert_stride = h->gu_stride; g1.scale_stride = nsc_gu; g1.N = I; g1.K = H; g1.act_q = ws->x_q; g1.act_d = ws->x_d;
-  g1.row_src = ws->src_of_row; g1.tiles = ws->tiles; g1.counters = ws->counters; g1.out = ws->a_buf;
+  g1.row_src = ws->src_of_row; g1.tiles = ws->tiles; g1.counters = ws->counters; g1.out = ws->a_buf; g1.outside = h->raw_outside;
   int rc;
   {
     ProfScope ps(1, st);
-    rc = chunk ? launch_rawint4_chunk<true>(g1, std::min(npairs, E) + npairs / 64, st) : launch_rawint4<true>(g1, max_tiles, st);
+    rc = chunk ? moe_launch_rawint4_chunk(true, g1, std::min(npairs, E) + npairs / RAW_ROWS, st) : launch_rawint4<true>(g1, max_tiles, st);
   }
   if (rc) return rc;
   {
@@ -3544,10 +3230,10 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   RawGemmParams g2;
   g2.w0 = h->down_w; g2.w1 = nullptr; g2.s0 = (const bf16_t*)h->down_s; g2.s1 = nullptr; g2.expert_stride = h->dn_stride;
   g2.scale_stride = nsc_dn; g2.N = H; g2.K = I; g2.act_q = ws->a_q; g2.act_d = ws->a_d; g2.row_src = nullptr;
-  g2.tiles = ws->tiles; g2.counters = ws->counters; g2.out = ws->dn_buf;
+  g2.tiles = ws->tiles; g2.counters = ws->counters; g2.out = ws->dn_buf; g2.outside = h->raw_outside;
   {
     ProfScope ps(3, st);
-    rc = chunk ? launch_rawint4_chunk<false>(g2, std::min(npairs, E) + npairs / 64, st) : launch_rawint4<false>(g2, max_tiles, st);
+    rc = chunk ? moe_launch_rawint4_chunk(false, g2, std::min(npairs, E) + npairs / RAW_ROWS, st) : launch_rawint4<false>(g2, max_tiles, st);
   }
   if (rc) return rc;
   CombineParams cp{};

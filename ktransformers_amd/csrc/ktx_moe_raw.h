@@ -1,0 +1,54 @@
+// ktx_moe_raw.h — what ktx_moe.hip (which buckets, quantises and combines) and ktx_moe_raw.hip (the prompt GEMM of RAWINT4 experts) share.
+#ifndef KTX_MOE_RAW_H
+#define KTX_MOE_RAW_H
+#include <type_traits>
+
+#include "ktx_common.h"
+
+template <int N, class F, int I = 0>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, F, I + 1>(static_cast<F&&>(f));
+  }
+}
+
+struct Tile {
+  int expert;  // local expert index
+  int row0;    // first sorted row
+  int nrows;   // <= 16*MT
+  int idx;     // place among its expert's tiles
+  int cnt;     // the expert's tiles
+};
+
+struct RawGemmParams {
+  const uint8_t *w0, *w1;      // RAW tiles (gate | down, up)
+  const bf16_t *s0, *s1;       // bf16 scales in the tile order above
+  size_t expert_stride;        // bytes of weights per expert matrix
+  size_t scale_stride;         // bf16 elements of scales per expert matrix
+  int N, K;
+  const int8_t* act_q;         // [src rows][K]
+  const float* act_d;          // [src rows][K/32]
+  const int32_t* row_src;
+  const Tile* tiles;           // <= 4 rows per tile
+  const int32_t* counters;
+  bf16_t* out;                 // [sorted rows][N]
+  const int* outside;          // [expert]: not 0 if a scale of its matrices is outside raw_scale_fits
+};
+
+typedef _Float16 raw_h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 raw_h8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ uint32_t raw_h2_bits(raw_h2 v) { return __builtin_bit_cast(uint32_t, v); }
+
+// What a widened nibble's operand carries: RAW_LIFT (8) times (q - 8) times the group's scale times 2^RAW_LIFT_S; the epilogue takes both back.
+constexpr int RAW_LIFT = 8, RAW_LIFT_S = 6;
+// A scale (bf16) whose operands are exact f16: 0 or magnitudes of 2^-23 .. 4.  2^6 s keeps its 8 significant bits down to f16's last one, 2^-24; 192 * 2^6 s stays
+// below 65504; 8 q 2^6 s is a normal f16.
+__host__ __device__ inline bool raw_scale_fits(bf16_t s) {
+  const unsigned m = s & 0x7fffu;
+  return m == 0 || (m >= (127u - 23u) << 7 && m < (127u + 2u) << 7);
+}
+constexpr int RAW_ROWS = 64;   // rows of a prompt tile
+// One grouped GEMM of a RAWINT4 prompt on tiles of RAW_ROWS rows.
+int moe_launch_rawint4_chunk(bool gate_up, const RawGemmParams& p, int max_tiles, hipStream_t st);
+#endif

@@ -1,0 +1,334 @@
+// ktx_moe_raw.hip — prompt GEMM of RAWINT4 experts (its own translation unit: it takes as long to compile as ktx_moe.hip).
+#include <hip/hip_runtime.h>
+#include <type_traits>
+
+#include "ktx_common.h"
+#include "ktx_moe_dec.inc"
+#include "ktx_moe_raw.h"
+
+// =====================================================================================================
+// RAWINT4 prompt chunks: the same products on the 16x16x32 f16 MFMA, one MFMA per (32-k group) x (16 rows) x (16 tokens).
+//
+// The exact kernel (ktx_moe.hip) keeps the reference's SIXTEEN fp32 lane accumulators per output.  A prompt chunk does not need that
+// association: the terms of an output are the per-group sums  as[t][g] * bs[n][g] * sum_{k in g} a[t][k] * q[n][k]  — the reference adds
+// them as 16 interleaved chains + a tree, this kernel as ONE chain over the groups in k order, held to the bound of the FP8 / BF16 formats
+// (tests/test_moe_gpu.py::test_rawint4_prompt_chunks).  Decode and short batches (qlen < 64) keep the exact kernels; dev knob 29 = 1
+// forces them for every size.
+//
+// The vector ALU bounds it (busy 70 % of the time at 2048 tokens of Kimi-K2's sizes, 12 instructions an MFMA, the matrix pipe 22 %, rocprofv3 counters), so the
+// operands are what costs it least.  Codes are f16 integers.  A weight's operand is its nibble times its group's scale, which f16 holds exactly
+// (4 and 8 significant bits): the MFMA's sum over a group has at most 23 significant bits, is exact in fp32, and a fragment takes one fma an output (with
+// the activation's scale) where the product of both scales took a multiplication as well.  The term is rounded once, in that fma; before, the product of
+// the scales was, too.  Widening costs 16 instructions per 8 weights of a lane, for all of its row groups.  Scales that f16 does not hold (raw_scale_fits;
+// an expert has one, or it has none) stay outside the operands, in fp32, with the multiplication.
+//
+// No second copy of the weights: the RAW tiles are read as they lie in HBM.  MFMA lane (i = lane & 15, kc = lane >> 4) needs
+// row i's eight nibbles k = 64 kb + 32 h + 8 kc + [0, 8) of group (kb, h): those are the pieces (L, j) = (8h + 2kc + o, i & 3),
+// o = 0 / 1, of RAW tile rg = i >> 2 — so the lane loads exactly its four pieces q = (h, o) of the strip's four tiles and nothing moves
+// between lanes; inside 8 k the pairs come out as (0,2) (1,3) (4,6) (5,7), the order in which the activation codes are stored.
+//   workgroup = 4 wavefronts = 4 strips of 16 weight rows x (gate, up), or 8 strips of down, x 64 rows of the expert, two workgroups per CU (one
+//   multiplies while the other waits: 8 wavefronts on 128 rows are 2 to 20 % slower, though no expert of 65 .. 128 rows is widened twice).  K walks in the RAW
+//   step of 512: its weights go through the LDS into registers (the LDS holds the next step's meanwhile: two steps in registers leave none for
+//   the sums of two rounds), the activations in quarters of it, all by LDS-DMA.
+// At Kimi-K2's sizes, us for the whole forward, scales multiplied behind the MFMAs and weights of two steps in registers -> here: 500 tokens
+// 2015 -> 1905, 2048 4280 -> 3850; 64 experts of 2048 x 1024, top-8: 360 tokens 168 -> 149, 2048 537 -> 474.
+// =====================================================================================================
+__host__ __device__ constexpr float raw_unlift(bool scaled) { return 1.0f / (float)(scaled ? RAW_LIFT << RAW_LIFT_S : RAW_LIFT); }
+// the pairs (byte 0, byte 2) and (byte 1, byte 3) of the low (par 0) or high nibbles of x, as RAW_LIFT * q * s; x: two's complement nibbles.
+// A nibble (its top bit turned: q + 8) becomes bits 6..9 of an f16 of exponent 2^7: 128 + 8 (q + 8).  s (an f16 with 8 significant bits) times that, less
+// 192 s (= 3 * 64 s: exact), is 8 q s with 11 significant bits at most: exact as well.
+template <int PAR>
+__device__ __forceinline__ void raw_widen(uint32_t x, uint32_t mask, uint32_t top, raw_h2 s, raw_h2 c, uint32_t& o0, uint32_t& o1) {
+  auto value = [&](uint32_t e) { return raw_h2_bits(__builtin_elementwise_fma(__builtin_bit_cast(raw_h2, (e & mask) ^ top), s, c)); };
+  if constexpr (PAR == 0) { o0 = value(x << 6); o1 = value(x >> 2); }
+  else { o0 = value(x << 2); o1 = value(x >> 6); }
+}
+
+// 4 wavefronts of one strip (x gate, up; or two strips of down) each, up to RAW_ROWS rows of one expert.
+template <bool GATE_UP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_rawint4_chunk_kernel(RawGemmParams p) {
+  constexpr int NW = 4, NU = 2;                     // weight operands per wavefront that share one activation fragment: (gate, up) of a
+                                                    // strip, or two strips of down
+  constexpr int TOK = NW * 16, MT = NW;
+  // activations in quarter steps (128 k), two buffers of up to TOK rows or four of up to TOK / 2: codes (f16), group scales [4 groups][rows]
+  constexpr int XBYTES = 2 * TOK * 256, AB = 4 * TOK * 4, ABYTES = 4 * AB;
+  constexpr int WB = NU * 4096 + NU * 512;          // a wavefront's weights of a step: [u][q] pieces of 1 KB, [u][row][h] scales of 16 B
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // XBYTES | ABYTES | [NW][WB]
+  __shared__ int s_src[TOK];
+
+  const int tile_idx = blockIdx.y, sgroup = blockIdx.x;
+  if (tile_idx >= p.counters[0]) return;
+  const Tile tile = p.tiles[tile_idx];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nstrips = p.N / 16;
+  const int NS = p.K / 512, G = p.K / 32;
+  const int i = lane & 15, kc = lane >> 4, rg = i >> 2, j = i & 3;
+  int ustrip[NU];
+#pragma unroll
+  for (int u = 0; u < NU; u++) ustrip[u] = GATE_UP ? sgroup * NW + wave : (sgroup * NW + wave) * 2 + u;
+  const bool wave_ok = ustrip[0] < nstrips;
+
+  // rows past the tile read its first row again (their outputs are never stored)
+  if (tid < TOK) {
+    const int r = tile.row0 + (tid < tile.nrows ? tid : 0);
+    s_src[tid] = p.row_src ? p.row_src[r] : r;
+  }
+  __syncthreads();
+  const int mt_live = (tile.nrows + 15) >> 4;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+
+  // ---- weights: this lane's four pieces of each unit's four RAW tiles, and a row's scales (a strip past N aliases strip 0, not stored)
+  const uint8_t* wb[NU];
+  const uint8_t* sb;            // lanes 0..31 bring unit 0's scales, 32..63 unit 1's: row (lane >> 1) & 15, h = lane & 1
+  const uint32_t wo = (uint32_t)(rg * NS * 1024 + ((2 * kc) * 4 + j) * 16);
+  {
+    const uint8_t* sbu[NU];
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      const int st = ustrip[u] < nstrips ? ustrip[u] : 0;
+      wb[u] = ((GATE_UP && u) ? p.w1 : p.w0) + (size_t)tile.expert * p.expert_stride + (size_t)(st * 4) * NS * 1024;
+      sbu[u] = reinterpret_cast<const uint8_t*>(((GATE_UP && u) ? p.s1 : p.s0) + (size_t)tile.expert * p.scale_stride + (size_t)(st * 4) * NS * 64);
+    }
+    const int row = (lane >> 1) & 15;
+    sb = (lane < 32 ? sbu[0] : sbu[1]) + (size_t)((row >> 2) * NS * 128 + (row & 3) * 32 + (lane & 1) * 16);
+  }
+  const uint32_t lds_w = lds0 + XBYTES + ABYTES + wave * WB;
+  const uint8_t* my_w = smem + XBYTES + ABYTES + wave * WB;
+  constexpr int WDMA = NU * 4 + 1;
+  auto stage_w = [&](int st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NU; u++)
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        moe_dma(wb[u] + (size_t)st * 1024 + wo + ((q >> 1) * 8 + (q & 1)) * 64, lds_w + (u * 4 + q) * 1024);
+    moe_dma(sb + (size_t)st * 128, lds_w + NU * 4096);
+  };
+  struct WStep { uint4 w[NU][4]; uint4 s[NU][2]; };   // w[u][h * 2 + o]: piece L = 8h + 2kc + o; s[u][h]: 8 bf16 scales (kb = 0..7)
+  auto fetch_w = [&](auto scaled, WStep& d) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) d.w[u][q] = *reinterpret_cast<const uint4*>(my_w + (u * 4 + q) * 1024 + lane * 16);
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        d.s[u][h] = *reinterpret_cast<const uint4*>(my_w + NU * 4096 + u * 512 + i * 32 + h * 16);
+        // 2^RAW_LIFT_S in both exponents of a pair; a zero becomes 2^-121, which is zero as an f16 (the pack kernel lets no other scale through
+        // whose exponent could overflow or whose f16 would round)
+        if constexpr (decltype(scaled)::value) {
+          constexpr uint32_t up = (uint32_t)RAW_LIFT_S * 0x00800080u;
+          d.s[u][h].x += up; d.s[u][h].y += up; d.s[u][h].z += up; d.s[u][h].w += up;
+        }
+      }
+    }
+    // read before the next step's DMAs may overwrite them
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) asm volatile("" : "+v"(d.w[u][q].x), "+v"(d.w[u][q].y), "+v"(d.w[u][q].z), "+v"(d.w[u][q].w)::"memory");
+#pragma unroll
+      for (int h = 0; h < 2; h++) asm volatile("" : "+v"(d.s[u][h].x), "+v"(d.s[u][h].y), "+v"(d.s[u][h].z), "+v"(d.s[u][h].w)::"memory");
+    }
+  };
+
+  // ---- activations of a quarter step: one DMA instruction per four rows of 256 B (LDS slot s of row r holds the row's 16-byte piece s ^ (r & 15)), dealt
+  // over the wavefronts; and the scales of the rows for one group (lane = row)
+  auto stage = [&](auto mtl, int qs, int buf) __attribute__((always_inline)) {
+    constexpr int MTL = decltype(mtl)::value, NBUF = MTL * 2 > MT ? 2 : 4;
+#pragma unroll
+    for (int c = 0; c < MTL; c++) {
+      const int piece = c * NW + wave, row = piece * 4 + (lane >> 4);
+      const int8_t* src = p.act_q + (size_t)s_src[row] * (size_t)(p.K * 2) + (size_t)qs * 256 + ((lane ^ row) & 15) * 16;
+      moe_dma(src, lds0 + buf * (XBYTES / NBUF) + piece * 1024);
+    }
+    const uint32_t aoff = (uint32_t)s_src[lane] * (uint32_t)G * 4u;   // (rows x groups x 4 B < 4 GiB: checked by the launcher)
+    gg_dma4(p.act_d + (size_t)qs * 4 + wave, aoff, lds0 + XBYTES + buf * AB + wave * (TOK * 4));
+  };
+
+  const uint32_t xo0 = i * 256 + ((kc ^ i) * 16);   // row i's piece kc; piece 4 g + kc: ^ 64 g
+  // constants the compiler cannot see through: and + xor become one v_bitop3_b32
+  uint32_t mask, top;
+  asm("s_mov_b32 %0, 0x03C003C0" : "=s"(mask));
+  asm("v_mov_b32 %0, 0x5A005A00" : "=v"(top));      // 128 = 0x5800, and the nibble's top bit (0x0200) turned
+
+  // MTL = 16-row groups of the tile that hold rows; one instantiation per count, chosen once per workgroup.
+  auto run = [&](auto mtl, auto scaled) __attribute__((always_inline)) {
+    constexpr int MTL = decltype(mtl)::value;
+    constexpr bool SCALED = decltype(scaled)::value;
+    constexpr int TB = MTL < 2 ? MTL : 2, NP = (MTL + TB - 1) / TB;   // fragments whose sums are in registers at once; rounds of them
+    float acc[NU][MTL][4];
+#pragma unroll
+    for (int u = 0; u < NU; u++)
+#pragma unroll
+      for (int t = 0; t < MTL; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[u][t][r] = 0.0f;
+
+    // A quarter step: four groups (kb = 2 Q, 2 Q + 1; h) in rounds of TB fragments.  A round's MFMAs are issued before the sums of the round before it, with
+    // the operands' loads and the next group's widening between, so that a wavefront by itself keeps both units busy.  Rounds are fenced from each
+    // other: left alone, the compiler widens a whole step's weights up front and spills them.
+    constexpr int R = 4 * NP, NBUF = MTL * 2 > MT ? 2 : 4, XB = XBYTES / NBUF;
+    raw_h8 bop[2][NU];
+    auto scale = [&](const WStep& w, auto qc, auto gc, int u) __attribute__((always_inline)) {   // of the lane's row
+      constexpr int Q = decltype(qc)::value, g = decltype(gc)::value;
+      const uint4& sv = w.s[u][g & 1];
+      const uint32_t S = Q == 0 ? sv.x : Q == 1 ? sv.y : Q == 2 ? sv.z : sv.w;
+      return __uint_as_float((g >> 1) ? (S & 0xffff0000u) : (S << 16));
+    };
+    auto widen = [&](const WStep& w, auto qc, auto gc) __attribute__((always_inline)) {
+      constexpr int Q = decltype(qc)::value, g = decltype(gc)::value, par = g >> 1, h = g & 1;
+#pragma unroll
+      for (int u = 0; u < NU; u++) {
+        const uint4 &w0 = w.w[u][h * 2], &w1 = w.w[u][h * 2 + 1];
+        const uint32_t P0 = Q == 0 ? w0.x : Q == 1 ? w0.y : Q == 2 ? w0.z : w0.w;
+        const uint32_t P1 = Q == 0 ? w1.x : Q == 1 ? w1.y : Q == 2 ? w1.z : w1.w;
+        const _Float16 s = SCALED ? (_Float16)scale(w, qc, gc, u) : (_Float16)1.0f, c = s * (_Float16)-192.0f;
+        uint32_t o[4];
+        raw_widen<par>(P0, mask, top, raw_h2{s, s}, raw_h2{c, c}, o[0], o[1]);
+        raw_widen<par>(P1, mask, top, raw_h2{s, s}, raw_h2{c, c}, o[2], o[3]);
+        bop[g & 1][u] = __builtin_bit_cast(raw_h8, make_uint4(o[0], o[1], o[2], o[3]));
+      }
+    };
+    auto compute = [&](auto qc, const WStep& w) __attribute__((always_inline)) {
+      constexpr int Q = decltype(qc)::value, buf = Q % NBUF;
+      const uint8_t* xb = smem + buf * XB;
+      const float* ab = reinterpret_cast<const float*>(smem + XBYTES + buf * AB) + kc * 4;
+      raw_h8 af[2][TB];
+      float4 sf[2][TB];
+      v4f d[2][TB][NU];
+      auto load_a = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TB; t++)
+          if ((r % NP) * TB + t < MTL) af[r & 1][t] = *reinterpret_cast<const raw_h8*>(xb + (xo0 ^ ((r / NP) * 64)) + ((r % NP) * TB + t) * 4096);
+      };
+      auto load_s = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TB; t++)
+          if ((r % NP) * TB + t < MTL) sf[r & 1][t] = *reinterpret_cast<const float4*>(ab + (r / NP) * TOK + ((r % NP) * TB + t) * 16);
+      };
+      auto mul = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TB; t++)
+          if ((r % NP) * TB + t < MTL)
+#pragma unroll
+            for (int u = 0; u < NU; u++) d[r & 1][t][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[r & 1][t], bop[(r / NP) & 1][u], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      };
+      load_a(0);
+      load_s(0);
+      if constexpr (Q == 0) widen(w, qc, std::integral_constant<int, 0>{});
+      if constexpr (NP == 1) widen(w, qc, std::integral_constant<int, 1>{});
+      mul(0);
+      load_a(1);
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<R>([&](auto rc) __attribute__((always_inline)) {
+        constexpr int r = decltype(rc)::value;
+        if constexpr (r + 1 < R) { mul(r + 1); load_s(r + 1); }
+        if constexpr (r + 2 < R) load_a(r + 2);
+        // the group of round r + 2 if that is its first (its operands' buffer was last read by the MFMAs two groups before it)
+        if constexpr (r + 2 < R && (r + 2) % NP == 0) widen(w, qc, std::integral_constant<int, ((r + 2) / NP) & 3>{});
+        if constexpr (r + 1 == R && Q < 3) widen(w, std::integral_constant<int, (Q + 1) & 3>{}, std::integral_constant<int, 0>{});
+        float bsr[NU];
+#pragma unroll
+        for (int u = 0; u < NU; u++) bsr[u] = SCALED ? 1.0f : scale(w, qc, std::integral_constant<int, r / NP>{}, u);
+#pragma unroll
+        for (int t = 0; t < TB; t++) {
+          if ((r % NP) * TB + t >= MTL) continue;
+          const float4 sv = sf[r & 1][t];
+          const float asv[4] = {sv.x, sv.y, sv.z, sv.w};
+#pragma unroll
+          for (int u = 0; u < NU; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              float& o = acc[u][(r % NP) * TB + t][e];
+              o = fmaf(SCALED ? asv[e] : asv[e] * bsr[u], d[r & 1][t][u][e], o);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+
+    // A step of 512 k: its weights come from the LDS into registers, then the next step's are requested; a quarter's activations are requested NBUF - 1 quarters
+    // ahead.  The waits leave what was requested after the quarter needed next: SD requests a quarter, WDMA of weights in the first one.  Requests
+    // past the end repeat the last ones.  (Wavefronts of their own for the weights' and the activations' requests, so that neither waits for the
+    // other's: 4 % slower, the four are no longer even.)
+    constexpr int SD = MTL + 1;
+    auto quarter = [&](auto qc, int st, const WStep& w) __attribute__((always_inline)) {
+      constexpr int Q = decltype(qc)::value;
+      stage(mtl, min(4 * st + Q + NBUF - 1, 4 * NS - 1), (Q + NBUF - 1) % NBUF);
+      if constexpr (Q == 0) stage_w(min(st + 1, NS - 1));
+      if (wave_ok) compute(qc, w);
+      // needed next: quarter Q + 1's activations, requested NBUF - 2 quarters ago (before that quarter's weights, if it was the first); at the end of the
+      // step the weights as well
+      constexpr int younger = (NBUF - 2) * SD, left = Q == 3 ? (younger < 2 * SD ? younger : 2 * SD) : Q <= NBUF - 2 ? younger + WDMA : younger;
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(left) : "memory");
+      __syncthreads();
+    };
+    stage_w(0);
+#pragma unroll
+    for (int q = 0; q < NBUF - 1; q++) stage(mtl, q, q);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 2) * SD) : "memory");
+    __syncthreads();
+    for (int st = 0; st < NS; st++) {
+      WStep w;
+      fetch_w(scaled, w);
+      quarter(std::integral_constant<int, 0>{}, st, w);
+      quarter(std::integral_constant<int, 1>{}, st, w);
+      quarter(std::integral_constant<int, 2>{}, st, w);
+      quarter(std::integral_constant<int, 3>{}, st, w);
+    }
+
+    if (!wave_ok) return;
+    constexpr float unlift = raw_unlift(SCALED);
+    if constexpr (GATE_UP) {
+      const int n = ustrip[0] * 16 + i;
+#pragma unroll
+      for (int t = 0; t < MTL; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int row = t * 16 + kc * 4 + r;
+          if (row < tile.nrows) {
+            const bf16_t gv = f32_to_bf16(acc[0][t][r] * unlift), uv = f32_to_bf16(acc[1][t][r] * unlift);
+            p.out[(size_t)(tile.row0 + row) * p.N + n] = f32_to_bf16(act_fn(bf16_to_f32(gv), bf16_to_f32(uv)));
+          }
+        }
+    } else {
+#pragma unroll
+      for (int u = 0; u < NU; u++) {
+        if (ustrip[u] >= nstrips) continue;
+        const int n = ustrip[u] * 16 + i;
+#pragma unroll
+        for (int t = 0; t < MTL; t++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const int row = t * 16 + kc * 4 + r;
+            if (row < tile.nrows) p.out[(size_t)(tile.row0 + row) * p.N + n] = f32_to_bf16(acc[u][t][r] * unlift);
+          }
+      }
+    }
+  };
+  if (p.outside[tile.expert]) {   // (rare: two instantiations will do; rows that are not there compute on what the LDS holds, and are not stored)
+    if (mt_live <= MT / 2) run(std::integral_constant<int, MT / 2>{}, std::false_type{});
+    else run(std::integral_constant<int, MT>{}, std::false_type{});
+    return;
+  }
+#define KTX_RAW_CASE(m) case m: run(std::integral_constant<int, m>{}, std::true_type{}); break;
+  switch (mt_live) {
+    KTX_RAW_CASE(1) KTX_RAW_CASE(2) KTX_RAW_CASE(3) KTX_RAW_CASE(4)
+  }
+#undef KTX_RAW_CASE
+}
+
+template <bool GATE_UP>
+static int launch_rawint4_chunk(const RawGemmParams& p, int max_tiles, hipStream_t st) {
+  constexpr size_t lds = 4 * (2 * 16 * 256 + 4 * 4 * 16 * 4 + 2 * 4608);
+  const hipError_t err = ktx_set_max_lds(reinterpret_cast<const void*>(moe_rawint4_chunk_kernel<GATE_UP>), (int)lds);
+  KTX_HIP(err);
+  const int per_wg = GATE_UP ? 4 : 8;       // strips per workgroup (down: two strips per wavefront)
+  hipLaunchKernelGGL((moe_rawint4_chunk_kernel<GATE_UP>), dim3((p.N / 16 + per_wg - 1) / per_wg, max_tiles), dim3(256), lds, st, p);
+  KTX_HIP(hipGetLastError());
+  return 0;
+}
+
+int moe_launch_rawint4_chunk(bool gate_up, const RawGemmParams& p, int max_tiles, hipStream_t st) {
+  return gate_up ? launch_rawint4_chunk<true>(p, max_tiles, st) : launch_rawint4_chunk<false>(p, max_tiles, st);
+}

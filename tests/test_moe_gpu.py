@@ -459,7 +459,7 @@ def test_rawint4_bit_exact(oracle, dev, shape):
 def test_rawint4_prompt_chunks(oracle, dev, shape):
     """Prompt chunks (qlen >= 64) of the RAWINT4 format go through moe_rawint4_chunk_kernel: the same int8 x int4 products and the
     same per-group scale products as the reference's GemmKernel224Int4SmallKGroup, summed as ONE fp32 chain over the 32-k groups
-    instead of sixteen interleaved chains + a tree (csrc/ktx_moe.hip).  Bound: that of the FP8 / BF16 formats, whose prompt kernels
+    instead of sixteen interleaved chains + a tree (csrc/ktx_moe_raw.hip).  Bound: that of the FP8 / BF16 formats, whose prompt kernels
     re-associate the same way (element-wise 2^-7 |ref| + 2^-9 max|ref|, < 5 % of the bf16 outputs different at all, mean error
     < 1e-3 of the mean magnitude); and against the exact kernels of this library on the same input (MoEHandle.set_exact), Kimi-K2's
     expert shape included, ragged tiles and invalid ids included."""
@@ -633,6 +633,37 @@ def test_rawint4_rows_per_tile_and_any_scale(oracle, dev, H, I):
                 plain = got
         finally:
             h.close()
+
+
+@pytest.mark.parametrize("H,I", [(512, 1024), (1024, 512)])
+def test_rawint4_prompt_scales_at_the_edges_of_the_operands(dev, H, I):
+    """The prompt kernel's f16 operands carry weight scales of 2^-23 .. 4 and 0; an expert with any other one is multiplied with its scales outside them.
+    Each expert has one scale at or beside an edge (smallest and largest that fit with all their bits, the next outside, zero), in each matrix, and 1, 16,
+    17, 33, 64 or 65 rows (every count of 16-row groups, and a second tile).  Bound: the one of the prompt kernel against this library's exact kernels."""
+    from helpers import rawint4_quantize
+    from ktransformers_amd._native import MoEHandle
+    rows, edge = (1, 16, 17, 33, 64, 65), (0.0, 2.0 ** -23 * (1 + 127 / 128), 4 * (1 - 1 / 256), 2.0 ** -24, 4.0, 2.0 ** -23)
+    E, T = len(rows), sum(rows)
+    c = make_case(33, E, 1, H, I, T)
+    of = np.repeat(np.arange(E), rows)
+    q = [rawint4_quantize(bf16_to_f32(c[n])) for n in ("gate", "up", "down")]
+    s = [x[1].copy() for x in q]
+    for e in range(E):
+        for m in range(3):
+            s[m][e, 3 + e, (2 * e + m) % s[m].shape[2]] = f32_to_bf16(np.array([edge[(e + m) % E]], np.float32))[0]
+    d = dict(c, ids=of[:, None].astype(np.int64))
+    h = MoEHandle(E, 1, H, I, max_len=T, method="RAWINT4", device=0, group_size=32)
+    try:
+        h.load_rawint4(*[torch.from_numpy(x[0]).to(dev) for x in q], *[torch_bf16(x, dev) for x in s])
+        got = run(h, d, dev)
+        h.set_exact(True)
+        want = run(h, d, dev)
+    finally:
+        h.close()
+    for e in range(E):
+        large = np.arange(H) == 3 + e      # (the edge scale of down: a column of its own magnitude)
+        _check_fp(got[of == e][:, ~large], want[of == e][:, ~large])
+        _check_fp(got[of == e][:, large], want[of == e][:, large])
 
 
 @pytest.mark.parametrize("method", ["AMXINT4", "FP8", "RAWINT4", "GGUF"])
