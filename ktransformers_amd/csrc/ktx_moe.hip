@@ -3349,6 +3349,9 @@ static int launch_gguf_type(int type, int mt, const GgGemmParams& p, int max_til
   }
 }
 
+// Whether the grouped kernel of this type reads Q8_K codes in unit order (launch_gguf)
+static int gg_unit_codes(int type) { return type == GG_Q4K && g_dbg[21] != 1; }
+
 // GGUF: bucket -> Q8_K(x) -> gate/up (+ act, fp32) -> Q8_K(a) -> down (fp32) -> combine (llamafile/moe.hpp:461-747)
 static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const int64_t* d_expert_ids,
                         const float* d_weights, const void* d_input, void* d_output, int flags, hipStream_t st) {
@@ -3506,7 +3509,8 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   {
     ProfScope ps(0, st);
     KTX_HIP(launch_moe_prep(pp, 1, st));
-    hipLaunchKernelGGL(q8k_quant_kernel<false>, dim3(qlen), dim3(256), 0, st, d_input, H, ws->x_q, ws->x_d, ws->x_bs, x_bsp, x_b256, d_bsz, 1, qlen);
+    hipLaunchKernelGGL(q8k_quant_kernel<false>, dim3(qlen), dim3(256), 0, st, d_input, H, ws->x_q, ws->x_d, ws->x_bs, x_bsp, x_b256, d_bsz, 1, qlen,
+                       gg_unit_codes(h->gg_type[0]));
   }
   KTX_HIP(hipGetLastError());
   GgGemmParams g1{};
@@ -3522,7 +3526,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   {
     ProfScope ps(2, st);
     hipLaunchKernelGGL(q8k_quant_kernel<true>, dim3(npairs), dim3(256), 0, st, (const void*)ws->a_buf, I, ws->a_q, ws->a_d, ws->a_bs,
-                       a_bsp, a_b256, ws->counters, 0, npairs);
+                       a_bsp, a_b256, ws->counters, 0, npairs, gg_unit_codes(h->gg_type[2]));
   }
   KTX_HIP(hipGetLastError());
   GgGemmParams g2{};

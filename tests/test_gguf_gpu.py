@@ -222,6 +222,31 @@ def test_folded_prompt_kernels_on_uneven_experts(rows, height):
     assert np.abs(y_ref.view(np.uint16).astype(np.int32)).max() > 0
 
 
+@pytest.mark.parametrize("rows", [(1, 15, 16, 17, 8, 16), (17, 32, 33, 48, 49, 64), (16, 63, 65, 80, 1, 31), (3, 3, 4, 4, 5, 6)])
+def test_folded_q4k_tiles_of_every_row_count(rows):
+    """The folded Q4_K kernel multiplies the 16-row groups of a tile that hold rows, a constant of its own for each count, on codes in unit order: 16-, 32- and
+    64-row tiles of 1 .. 4 groups, first and last tiles of an expert, in gate | up and down; the bits are the unfolded kernel's."""
+    from ktransformers_amd import _native as n
+    E, H, I, T = len(rows), 768, 512, sum(rows)
+    r0 = np.random.default_rng(T)
+    mats = [torch.from_numpy(random_kquant(Q4, E, a, b, r0)).cuda() for a, b in ((I, H), (I, H), (H, I))]
+    x = torch.from_numpy(f32_to_bf16(r0.standard_normal((T, H)).astype(np.float32)).view(np.int16)).view(torch.bfloat16).cuda()
+    ids = torch.from_numpy(r0.permutation(np.repeat(np.arange(E), rows)).astype(np.int64)[:, None]).cuda()
+    w = torch.from_numpy(r0.random((T, 1)).astype(np.float32)).cuda()
+    h = n.MoEHandle(E, 1, H, I, T, "GGUF", 0)
+    h.load_gguf(*mats, Q4, Q4, Q4)
+    n.force_generic_path(True)
+    try:
+        y_fold = h.forward(x, ids, w).view(torch.int16).cpu().numpy()
+        n.lib.ktx_debug_set(21, 1)
+        y_ref = h.forward(x, ids, w).view(torch.int16).cpu().numpy()
+    finally:
+        n.lib.ktx_debug_set(21, 0)
+        n.force_generic_path(False)
+    assert np.array_equal(y_fold, y_ref), f"{int((y_fold != y_ref).sum())} of {y_ref.size} outputs differ"
+    assert np.abs(y_ref.view(np.uint16).astype(np.int32)).max() > 0
+
+
 @pytest.mark.parametrize("T", [1, 4])
 def test_mixtral_8x7b_real_dims(T):
     """BASELINE.json configs[0] (Mixtral-8x7B q4_k_m, kt-kernel/bench/bench_moe.py:166-170): 8 experts, top-2, hidden 4096,
