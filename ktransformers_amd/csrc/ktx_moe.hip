@@ -39,6 +39,7 @@
 #include "ktx_common.h"
 #include "ktx_internal.h"
 #include "ktx_moe_raw.h"
+#include "ktx_moe_stream.h"
 
 // (the error slot — ktx_fail / ktx_last_error — lives in ktx_err.hip, which the small sequence-mixer library links as well)
 
@@ -50,31 +51,6 @@
 namespace ktxw4 {
 #include "ktx_w4_step.inc"
 }
-
-// Workgroup -> (tile, strip group) of a grouped GEMM, from a one-dimensional grid: ids are dealt round-robin to the 8 XCDs, so id % 8 is the
-// XCD.  The jobs lie expert after expert, within an expert strip group by strip group, the group's tiles side by side; each XCD takes an
-// eighth of them.  So the XCDs end together whatever the number of tiles, an expert's weights go into one L2 and are read there once for all
-// its tiles, and its rows (the operand every strip group re-reads) stay there too.  False: nothing to do.
-// SHARE false: launch order, for tiles so low that an expert mostly has one (256 experts of 7168 x 2048, AMXINT4, 114 tokens: shares cost 1 %).
-template <bool SHARE = true>
-__device__ __forceinline__ bool moe_pick_job(const Tile* tiles, int ntiles, int nsg, Tile& tile, int& sgroup) {
-  if constexpr (!SHARE) {
-    const int t = blockIdx.x / nsg;
-    if (t >= ntiles) return false;
-    tile = tiles[t];
-    sgroup = blockIdx.x - t * nsg;
-    return true;
-  }
-  const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-  const int total = ntiles * nsg, per = (total + 7) / 8, job = xcd * per + seq;
-  if (seq >= per || job >= total) return false;
-  tile = tiles[job / nsg];
-  const int first = job / nsg - tile.idx, ofs = job - first * nsg;
-  sgroup = ofs / tile.cnt;
-  if (tile.cnt > 1) tile = tiles[first + ofs % tile.cnt];
-  return true;
-}
-static dim3 moe_job_grid(int max_tiles, int nsg) { return dim3((unsigned)(((size_t)max_tiles * nsg + 7) / 8 * 8)); }
 
 // =====================================================================================================
 // K0: prep — block 0 buckets (t,j) pairs by expert; blocks 1.. quantise one token's activations (a5, a6)
@@ -357,21 +333,6 @@ __global__ __launch_bounds__(256) void moe_actquant_kernel(const bf16_t* __restr
 // =====================================================================================================
 // K1 / K2: grouped W4A8 / W8A8 GEMM on MFMA i8 (a8, a9, a10)
 // =====================================================================================================
-struct GemmParams {
-  const uint8_t* w0;   // gate (GATE_UP) or down
-  const uint8_t* w1;   // up   (GATE_UP) or nullptr
-  const float* s0;     // scales [E][N]
-  const float* s1;
-  size_t expert_stride;  // bytes of one expert's matrix
-  int N, K;
-  const int8_t* act_q;      // [src rows][K]
-  const float* act_d;       // [src rows]
-  const int32_t* row_src;   // sorted row -> source row (nullptr: identity)
-  const Tile* tiles;
-  const int32_t* counters;
-  bf16_t* out;  // [sorted rows][N]
-};
-
 // Four strips of 16 weight rows (x gate, up) against a tile of MT x 16 rows, chunk by chunk of SPC k-steps.  At few rows the weights' way in bounds it
 // (256 experts of 7168 x 2048, 32 tokens: 396 us, 6 TB/s); past 16 rows the LDS reads and barriers beside MFMAs that 3-4 wavefronts a SIMD do not
 // hide.  Requests that outlive their chunk, activations by LDS-DMA and an expert's tiles side by side on one XCD: 8 experts of 4096 x 1536, 100 rows
@@ -521,192 +482,6 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(GemmParams p) {
       if constexpr (GATE_UP)
         *reinterpret_cast<uint2*>(p.out + (size_t)(tile.row0 + row) * ld + p.N + n0) =
             make_uint2((uint32_t)o2[0] | ((uint32_t)o2[1] << 16), (uint32_t)o2[2] | ((uint32_t)o2[3] << 16));
-    }
-  }
-}
-
-// =====================================================================================================
-// K1s / K2s: "streaming" grouped GEMM for prompts (token tiles of 64 rows).
-// The chunk-pipelined kernel above re-reads one 1 KB activation fragment from LDS for every two MFMAs of a wave — exactly
-// the LDS port's 128 B/clk at full MFMA rate — and synchronises all waves every chunk (PMC at T=2048: MFMA busy 21 %, 55 %
-// of wave cycles waiting).  Here:
-//   * the tile's int8 activation rows are staged in LDS once per <= 2048-column chunk of K (one chunk for DeepSeek-V2-Lite
-//     and for every down projection) — no barrier inside a chunk;
-//   * each of the 8 waves owns FOUR 16-row weight strips (gate/up: 2 strips x {gate, up}; down: 4 strips), so one
-//     activation fragment read feeds 4 MFMAs (LDS port at <= 50 %) and 16 independent accumulators hide MFMA latency;
-//   * weights stream through a D-deep register ring per wave, D k-steps (>= 0.8 us of MFMA work) ahead of use.
-// moe_pick_job's eighths against tiles in launch order: 256 experts of 7168 x 2048, 64 rows each 1631 -> 1580 us, 64 of 6144 x 3072, 256: 1326 -> 1284.
-// Integer arithmetic and epilogue are those of moe_gemm_kernel, so results are bit-identical.
-// =====================================================================================================
-template <int WBITS, int MT, int D, bool GATE_UP>
-__global__ __launch_bounds__(512) void moe_gemm_stream_kernel(GemmParams p, int kch) {
-  constexpr int NJ = 4;                              // (strip, matrix) units per wave
-  constexpr int TOK = MT * 16;
-  constexpr int CS = TOK * 16;                       // LDS stride between 16-byte columns; token slot XOR-swizzled per column
-  constexpr int TILE_BYTES = (WBITS == 4) ? 1024 : 2048;
-  constexpr int SPW = GATE_UP ? 2 : 4;               // strips per wave
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  const int NKS = p.K / 128, KSC = kch / 128, CCOL = kch / 16;
-  uint8_t* xs = smem;                                                // [CCOL][TOK][16 B] (+pad)
-  float* s_ad = reinterpret_cast<float*>(smem + (size_t)CCOL * CS);  // [TOK]
-  int* s_src = reinterpret_cast<int*>(s_ad + TOK);                   // [TOK]
-
-  Tile tile;
-  int bx;
-  if (!moe_pick_job(p.tiles, p.counters[0], (p.N / 16 + 8 * SPW - 1) / (8 * SPW), tile, bx)) return;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int strip0 = (bx * 8 + wave) * SPW;
-  const int nstrips = p.N / 16;
-
-  // ---- weight ring first (addresses depend on the tile record only); strips past N alias strip 0 and are not stored
-  const uint8_t* wb[NJ];
-#pragma unroll
-  for (int j = 0; j < NJ; j++) {
-    const int st = strip0 + (GATE_UP ? (j >> 1) : j);
-    const uint8_t* base = (GATE_UP && (j & 1)) ? p.w1 : p.w0;
-    wb[j] = base + (size_t)tile.expert * p.expert_stride + (size_t)(st < nstrips ? st : 0) * NKS * TILE_BYTES;
-  }
-  WFrag<WBITS> ring[D][NJ];
-#pragma unroll
-  for (int d = 0; d < D; d++) {
-    const int ks = d < NKS ? d : NKS - 1;
-#pragma unroll
-    for (int j = 0; j < NJ; j++) ring[d][j] = load_wfrag<WBITS>(wb[j] + (size_t)ks * TILE_BYTES, lane);
-  }
-
-  if (tid < TOK) {
-    int src = -1;
-    float ad = 0.0f;
-    if (tid < tile.nrows) {
-      src = p.row_src ? p.row_src[tile.row0 + tid] : (tile.row0 + tid);
-      ad = p.act_d[src];
-    }
-    s_src[tid] = src;
-    s_ad[tid] = ad;
-  }
-
-  // B fragment of k-step s (within the chunk), half hh, token tile t: column s*8 + kc*2 + hh, token t*16 + (lane&15).
-  // LDS address of (col, tok) = col*CS + ((tok ^ f(col)) << 4), f(col) = (col & 3) | (col & 4 ? 12 : 0): ds_read_b128 is
-  // served in the lane groups {0-3,12-15,20-27}, {4-11,16-19,28-31}, ... over a 256-byte bank row — f keeps the token sets
-  // {0-3,12-15} / {4-11} of the two kc in a group disjoint (conflict-free reads; the unswizzled layout was 2-way), and gives
-  // the 8 consecutive columns one staging ds_write_b128 group covers 8 different 16-byte slots (conflict-free writes).
-  const int kc = lane >> 4;
-  const int fsw = ((kc & 1) << 1) | ((kc & 2) ? 12 : 0);
-  const uint8_t* bb0 = xs + (size_t)(kc * 2) * CS + (((lane & 15) ^ fsw) << 4);
-  const uint8_t* bb1 = xs + (size_t)(kc * 2 + 1) * CS + (((lane & 15) ^ (fsw | 1)) << 4);
-  const bool wave_ok = strip0 < nstrips;  // wave-uniform
-
-  v4i acc[NJ][MT];
-#pragma unroll
-  for (int j = 0; j < NJ; j++)
-#pragma unroll
-    for (int t = 0; t < MT; t++) acc[j][t] = v4i{0, 0, 0, 0};
-  for (int c0 = 0; c0 < NKS; c0 += KSC) {
-    const int c1 = c0 + KSC < NKS ? c0 + KSC : NKS;
-    const int ncol = (c1 - c0) * 8;
-    __syncthreads();  // previous chunk fully consumed (and s_src visible on the first pass)
-    // ---- stage the chunk: wavefront -> rows wave, wave + 8, ...; lane -> the row's 16-byte columns lane, lane + 64 (2 KB of one
-    // row per pass: coalesced, and NO integer division — the round-1..5 mapping idx -> (idx / ncol, idx % ncol) spent as many
-    // VALU instructions as the whole k loop: 4.5 VALU per MFMA in profiles/r06_w_pmc_stream8192.txt; the launch time did not
-    // move).  4 rows = 8 loads in flight per thread before the LDS writes.
-    // (unconditional loads from clamped rows / columns + an explicit vmcnt(0): every path into the k loop then has no load
-    // pending, which lets the compiler's waitcnt pass keep the ring's vmcnt(12..15) waits exact)
-    auto stage = [&](auto uc, int r0) {
-      constexpr int U = decltype(uc)::value;
-      uint4 v[U][2];
-      int off[U][2];
-      bool live[U];
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int row = r0 + u * 8;
-        const int src = s_src[row];
-        live[u] = src >= 0;
-        const int8_t* rp = p.act_q + (size_t)(src >= 0 ? src : 0) * p.K + (size_t)c0 * 128;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-          const int col = lane + h * 64 < ncol ? lane + h * 64 : ncol - 1;
-          off[u][h] = col * CS + (((row & ~15) | ((row & 15) ^ ((col & 3) | ((col & 4) ? 12 : 0)))) << 4);
-          v[u][h] = *reinterpret_cast<const uint4*>(rp + col * 16);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++)
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-          if (lane + h * 64 < ncol) *reinterpret_cast<uint4*>(xs + off[u][h]) = live[u] ? v[u][h] : make_uint4(0, 0, 0, 0);
-    };
-    static_assert(TOK % 16 == 0, "rows per wavefront");
-    {                                  // (kch <= 2048: at most two 64-column passes per row)
-      int r0 = wave;
-      for (; r0 + 24 < TOK; r0 += 32) stage(std::integral_constant<int, 4>{}, r0);
-      for (; r0 < TOK; r0 += 16) stage(std::integral_constant<int, 2>{}, r0);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __syncthreads();
-    if (wave_ok) {
-      // one k-step: consume ring slot d, refill it D steps ahead (clamped: branch-free, so the compiler keeps exact
-      // vmcnt(N) waits instead of draining the ring at every control-flow join), 2 x MT x NJ MFMAs
-      auto step = [&](auto dc, auto refill, int ks) {
-        constexpr int d = decltype(dc)::value;
-        v4i a[NJ][2];
-#pragma unroll
-        for (int j = 0; j < NJ; j++) unpack_wfrag<WBITS>(ring[d][j], a[j][0], a[j][1]);
-        if constexpr (decltype(refill)::value) {
-          const int kn = ks + D < NKS ? ks + D : NKS - 1;
-#pragma unroll
-          for (int j = 0; j < NJ; j++) ring[d][j] = load_wfrag<WBITS>(wb[j] + (size_t)kn * TILE_BYTES, lane);
-        }
-        __builtin_amdgcn_sched_barrier(0);  // keep the refill HERE (the scheduler otherwise sinks all loads to the loop end)
-        const size_t koff = (size_t)((ks - c0) * 8) * CS;
-#pragma unroll
-        for (int hh = 0; hh < 2; hh++) {
-          const uint8_t* bk = (hh ? bb1 : bb0) + koff;
-          v4i b[MT];
-#pragma unroll
-          for (int t = 0; t < MT; t++) b[t] = *reinterpret_cast<const v4i*>(bk + t * 256);
-#pragma unroll
-          for (int t = 0; t < MT; t++)
-#pragma unroll
-            for (int j = 0; j < NJ; j++)
-              acc[j][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j][hh], b[t], acc[j][t], 0, 0, 0);
-        }
-      };
-      int s0 = c0;
-      for (; s0 + D <= c1; s0 += D)
-        static_for<D>([&](auto dc) { step(dc, std::true_type{}, s0 + decltype(dc)::value); });
-      // tail (< D steps, only ever at the end of K): nothing left to prefetch
-      static_for<D>([&](auto dc) {
-        if (s0 + decltype(dc)::value < c1) step(dc, std::false_type{}, s0 + decltype(dc)::value);
-      });
-    }
-  }
-  if (!wave_ok) return;
-
-  // ---- epilogue: the arithmetic of moe_gemm_kernel's (GemmKernel224Int4::apply_scale, la/amx_kernels.hpp:1808-1846)
-  const int tok = lane & 15;
-  const int ld = GATE_UP ? 2 * p.N : p.N;
-#pragma unroll
-  for (int j = 0; j < NJ; j++) {
-    const int st = strip0 + (GATE_UP ? (j >> 1) : j);
-    if (st < nstrips) {
-      const int n0 = st * 16 + (lane >> 4) * 4;
-      const float* sp = (GATE_UP && (j & 1)) ? p.s1 : p.s0;
-      const float4 sc = *reinterpret_cast<const float4*>(sp + (size_t)tile.expert * p.N + n0);
-      const float sv[4] = {sc.x, sc.y, sc.z, sc.w};
-      const int coff = (GATE_UP && (j & 1)) ? p.N : 0;
-#pragma unroll
-      for (int t = 0; t < MT; t++) {
-        const int row = t * 16 + tok;
-        if (row < tile.nrows) {
-          const float ad = s_ad[row];
-          bf16_t o[4];
-#pragma unroll
-          for (int r = 0; r < 4; r++) o[r] = f32_to_bf16((ad * sv[r]) * (float)acc[j][t][r]);
-          *reinterpret_cast<uint2*>(p.out + (size_t)(tile.row0 + row) * ld + coff + n0) =
-              make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
-        }
-      }
     }
   }
 }
@@ -2641,20 +2416,6 @@ static int launch_gemm(const GemmParams& p, int max_tiles, hipStream_t st) {
 
 static int g_dbg[32] = {0};  // dev knobs: [0] waves/workgroup override of the decode gate/up kernel, [1] ablation bits
 template <int WBITS, bool GATE_UP>
-static int launch_gemm_stream(const GemmParams& p, int max_tiles, hipStream_t st) {
-  constexpr int MT = 4, D = (WBITS == 4) ? 4 : 2, TOK = MT * 16, CS = TOK * 16;
-  const int kch = std::min(p.K, 2048);
-  const size_t lds = (size_t)(kch / 16) * CS + TOK * 8;
-  auto kern = moe_gemm_stream_kernel<WBITS, MT, D, GATE_UP>;
-  const hipError_t attr_err = ktx_set_max_lds(reinterpret_cast<const void*>(kern), 160 * 1024);
-  KTX_HIP(attr_err);
-  const int strips_per_wg = 8 * (GATE_UP ? 2 : 4);
-  hipLaunchKernelGGL(kern, moe_job_grid(max_tiles, (p.N / 16 + strips_per_wg - 1) / strips_per_wg), dim3(512), lds, st, p, kch);
-  KTX_HIP(hipGetLastError());
-  return 0;
-}
-
-template <int WBITS, bool GATE_UP>
 static int launch_gemm_rt(const GemmParams& p, int max_tiles, hipStream_t st) {
   const size_t lds = 2 * (8 * 256 * 16 + 16 * 2048) + 256 * 8;
   auto kern = moe_gemm_rt_kernel<WBITS, GATE_UP>;
@@ -2946,21 +2707,27 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
     return forward_gguf(h, d_bsz, qlen, k, d_expert_ids, d_weights, d_input, d_output, flags, st);
   int mt = pick_mt(qlen, k, E);
   const int npairs = qlen * k;
-  // 64-row tiles (prompts) of large expert matrices take the streaming kernels, one workgroup a CU, where they have enough workgroups to go round;
-  // the others stay on moe_gemm_kernel.  Measured for AMXINT4 (us, 32 rows | streaming | 64 rows): 256 experts of 7168 x 2048 with 9.4 rows each
-  // 880 | 869 | 920, 16: 1036 | 993 | 1062, 64: 1900 | 1580 | 1766; 64 of 6144 x 3072, 37: 467 | 418 | 451; 32 of them, 62 (756 workgroups): 311 | 299 |
-  // 296; 16 of 6144 x 2048, 62 (376): 123 | 125 | 120, 256 (640): 321 | 292 | 278; 8 of 4096 x 1536, 100 (120): 53 | 72 | 58, 512: 176 | 170 | 156.
-  // A short K or few workgroups stream no better: 64 of 1536 x 3072, 20 rows 130 | 137, 64 of 2560 x 2048, 32 (768): 160 | 174.  16 against 32 rows: 3.1 rows 660 | 669, 6.6: 750 | 778, 64 experts of
+  // 64-row tiles (prompts) of large expert matrices take the streaming kernel, where it has enough work to go round; the others stay on moe_gemm_kernel.
+  // With 8 wavefronts a workgroup (one a CU) it reads the activations half as often as with 4 (two a CU), which counts while weights fill the memory's
+  // way in; 4 start and end beside each other.  Measured for AMXINT4 (us, moe_gemm_kernel | 8 | 4): 256 experts of 7168 x 2048 with 16 rows each 1014 | 972
+  // | 1019, 31: 1322 | 1150 | 1218, 64: 1757 | 1553 | 1567, 128: 2676 | 2316 | 2331; 64 of 6144 x 3072, 37: 476 | 418 | 446, 94: 652 | 568 | 585; 32 of them, 50:
+  // 278 | 279 | 264, 62: 307 | 299 | 285; 16 of 6144 x 2048, 62: 111 | 122 | 119, 87: 140 | 132 | 129, 125: 166 | 163 | 153, 250: 260 | 262 | 240; 64 of 3072 x 3072,
+  // 125: 465 | 442 | 433; 128 of 4096 x 1536, 50: 382 | 374 | 360; 8 of 4096 x 1536, 100: 51 | 65 | 61, 512: 139 | 153 | 148; 16 of 5120 x 1536, 100: 99 | 103 | 98,
+  // 256: 211 | 194 | 199; 64 of 1536 x 3072, 75: 206 | 227 | 216.  AMXINT8: 64 of 2560 x 2048, 50: 260 | 266 | 275, 250: 603 | 620 | 605; 256 of 7168 x 2048, 64: 2650 | 2631 |
+  // 2670.  A short K or few workgroups stream no better: 64 of 1536 x 3072, 20 rows 130 | 137.  16 against 32 rows: 3.1 rows 660 | 669, 6.6: 750 | 778, 64 experts of
   // 2048 x 1408, 3: 59 | 63, 9.4: 77 | 77.  32 against 64 rows where nothing streams: 25 rows
   // 134 | 135, 37: 109 | 109, 50: 177 | 169, 75: 152 | 138; with 8 experts 25: 35 | 41, 100: 53 | 58, 125: 60 | 59, 200: 82 | 75 — few tiles leave
-  // CUs idle longer.  Dev knob [4]: 1 = never stream, 2 = always at 64 rows (tests).
+  // CUs idle longer.  Dev knobs (tests) [4]: 1 = never stream, 2 = always at 64 rows; [5]: 1 = 4 wavefronts, 2 = 8.
   const auto tiles64 = [&](int strips) { return (std::min(npairs, E) + npairs / 64) * ((I / 16 + strips - 1) / strips); };   // workgroups of gate|up
-  bool use_stream = mt == 4 && g_dbg[4] != 1 && (g_dbg[4] == 2 || (size_t)H * I >= ((size_t)4 << 20));
+  const double rows = (double)npairs / std::max(1, E);
+  const bool large = (size_t)H * I >= ((size_t)4 << 20), fills8 = std::min(H, I) >= 2048 && tiles64(16) >= 1200;
+  bool use_stream = mt == 4 && g_dbg[4] != 1 && (g_dbg[4] == 2 || large);
   if (h->cfg.format == KTX_FMT_AMXINT4 && g_dbg[4] < 2) {
-    const double rows = (double)npairs / std::max(1, E);
-    use_stream = g_dbg[4] != 1 && rows > 12.0 && std::min(H, I) >= 2048 && (size_t)H * I >= ((size_t)4 << 20) && tiles64(16) >= 1200;
+    const bool fills4 = H >= 2048 && I >= 1024 && (double)tiles64(8) * H >= 3.6e6;
+    use_stream = g_dbg[4] != 1 && large && ((rows > 12.0 && fills8) || (rows >= 48.0 && fills4));
     mt = rows <= 8.0 ? 1 : use_stream || (rows > 40.0 && tiles64(4) >= 512) ? 4 : 2;
   }
+  const int stream_nw = g_dbg[5] ? 4 * g_dbg[5] : (fills8 && (H >= 4096 || rows < 48.0)) || (h->wbits == 8 && rows < 56.0) ? 8 : 4;
   const bool use_rt = mt == 4 && g_dbg[4] == 3;   // register-tile kernels (256-row tiles): parity-tested, not yet timed
   if (use_rt) { mt = 16; use_stream = false; }
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
@@ -2984,7 +2751,7 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
   {
     ProfScope ps(1, st);
     if (use_rt) rc = h->wbits == 4 ? launch_gemm_rt<4, true>(g1, max_tiles, st) : launch_gemm_rt<8, true>(g1, max_tiles, st);
-    else if (use_stream) rc = h->wbits == 4 ? launch_gemm_stream<4, true>(g1, max_tiles, st) : launch_gemm_stream<8, true>(g1, max_tiles, st);
+    else if (use_stream) rc = moe_launch_gemm_stream(h->wbits, stream_nw, true, g1, max_tiles, st);
     else rc = h->wbits == 4 ? launch_gemm_mt<4, true>(mt, g1, max_tiles, st) : launch_gemm_mt<8, true>(mt, g1, max_tiles, st);
   }
   if (rc) return rc;
@@ -3002,7 +2769,7 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
   {
     ProfScope ps(3, st);
     if (use_rt) rc = h->wbits == 4 ? launch_gemm_rt<4, false>(g2, max_tiles, st) : launch_gemm_rt<8, false>(g2, max_tiles, st);
-    else if (use_stream) rc = h->wbits == 4 ? launch_gemm_stream<4, false>(g2, max_tiles, st) : launch_gemm_stream<8, false>(g2, max_tiles, st);
+    else if (use_stream) rc = moe_launch_gemm_stream(h->wbits, stream_nw, false, g2, max_tiles, st);
     else rc = h->wbits == 4 ? launch_gemm_mt<4, false>(mt, g2, max_tiles, st) : launch_gemm_mt<8, false>(mt, g2, max_tiles, st);
   }
   if (rc) return rc;

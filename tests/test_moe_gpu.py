@@ -760,6 +760,31 @@ def test_fp_grouped_edges(oracle, dev, fmt, H, I, rows):
 
 
 @pytest.mark.parametrize("method", ["AMXINT4", "AMXINT8"])
+@pytest.mark.parametrize("H,I", [(1152, 1664), (2048, 512)])   # 9 and 13 k-steps (chunks of 4 and 8, with a rest), 16 and 4; strip groups that are not full
+@pytest.mark.parametrize("rows", [(16, 17, 33, 49, 130), (1, 64, 65, 128)])   # each count of 16-row groups, alone and behind a full tile
+def test_int_streaming_groups(oracle, dev, method, H, I, rows):
+    """moe_gemm_stream_kernel with 4 and with 8 wavefronts a workgroup (dev knob 5), bit for bit."""
+    from ktransformers_amd import _native
+    E, k, T = len(rows), 1, sum(rows)
+    c = make_case(47, E, k, H, I, T)
+    c["ids"] = np.random.default_rng(T).permutation(np.repeat(np.arange(E), rows)).astype(np.int64)[:, None]
+    want = oracle.moe_forward(oracle.make_moe(FMT[method], c["gate"], c["up"], c["down"]), c["ids"], c["w"], c["x"])
+    h = make_handle(method, c, E, k, H, I, T, dev)
+    try:
+        _native.force_generic_path(True)
+        _native.lib.ktx_debug_set(4, 2)
+        for knob in (1, 2):
+            _native.lib.ktx_debug_set(5, knob)
+            got = run(h, c, dev)
+            assert np.array_equal(got, want), f"{int((got != want).sum())} outputs differ ({4 * knob} wavefronts)"
+    finally:
+        _native.lib.ktx_debug_set(4, 0)
+        _native.lib.ktx_debug_set(5, 0)
+        _native.force_generic_path(False)
+        h.close()
+
+
+@pytest.mark.parametrize("method", ["AMXINT4", "AMXINT8"])
 @pytest.mark.parametrize("H,I", [(128, 128), (384, 640), (1152, 256)])
 @pytest.mark.parametrize("rows", [(1, 0, 2, 3), (33, 0, 1, 32), (65, 0, 257, 16)])
 def test_int_grouped_edges(oracle, dev, method, H, I, rows):
