@@ -39,6 +39,7 @@
 #include "ktx_common.h"
 #include "ktx_internal.h"
 #include "ktx_moe_raw.h"
+#include "ktx_moe_route.h"
 #include "ktx_moe_stream.h"
 
 // (the error slot — ktx_fail / ktx_last_error — lives in ktx_err.hip, which the small sequence-mixer library links as well)
@@ -53,242 +54,11 @@ namespace ktxw4 {
 }
 
 // =====================================================================================================
-// K0: prep — block 0 buckets (t,j) pairs by expert; blocks 1.. quantise one token's activations (a5, a6)
-// =====================================================================================================
-#define KTX_EMAX 1024
-
-struct PrepParams {
-  const int32_t* d_bsz;
-  int qlen, k, E, expert_begin, H;
-  int rows_per_tile;  // 16*MT
-  const int64_t* ids;
-  const uint8_t* mask;
-  const bf16_t* x;
-  int8_t* x_q;
-  float* x_d;
-  int32_t* row_of_pair;  // [qlen*k]  -> sorted row or -1
-  int32_t* src_of_row;   // [qlen*k]  sorted row -> token index
-  Tile* tiles;
-  int32_t* counters;  // [0] = num_tiles, [1] = num_rows
-  int bm_words;       // set by launch_moe_prep: 32-token words per expert in one window of the scatter's bitmaps
-};
-
-__device__ __forceinline__ void quant_row_block(const bf16_t* __restrict__ src, int K, int8_t* __restrict__ dst,
-                                                float* __restrict__ d_out, float* red /* LDS [nwaves] */) {
-  // per row: d = amax/127, id = d ? 1/d : 0, q = sat8(rne(x*id))   (amx_buffers.hpp:47-98)
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  float amax = 0.0f;
-  for (int j = tid * 8; j < K; j += nthr * 8) {
-    uint4 v = *reinterpret_cast<const uint4*>(src + j);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      amax = fmaxf(amax, fabsf(bf16_to_f32((bf16_t)(w[q] & 0xffffu))));
-      amax = fmaxf(amax, fabsf(bf16_to_f32((bf16_t)(w[q] >> 16))));
-    }
-  }
-  amax = wave_max(amax);
-  if ((tid & 63) == 0) red[tid >> 6] = amax;
-  __syncthreads();
-  float m = 0.0f;
-  for (int w = 0; w < (nthr >> 6); w++) m = fmaxf(m, red[w]);
-  const float d = m / 127.0f;
-  const float id = d ? 1.0f / d : 0.0f;
-  for (int j = tid * 8; j < K; j += nthr * 8) {
-    uint4 v = *reinterpret_cast<const uint4*>(src + j);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-    uint32_t o[2] = {0, 0};
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      int a = quant_rne_sat8(bf16_to_f32((bf16_t)(w[q] & 0xffffu)) * id);
-      int b = quant_rne_sat8(bf16_to_f32((bf16_t)(w[q] >> 16)) * id);
-      o[q >> 1] |= ((uint32_t)(a & 0xff) | ((uint32_t)(b & 0xff) << 8)) << ((q & 1) * 16);
-    }
-    *reinterpret_cast<uint2*>(dst + j) = make_uint2(o[0], o[1]);
-  }
-  if (tid == 0) *d_out = d;
-}
-
-__global__ __launch_bounds__(1024) void moe_prep_kernel(PrepParams p) {
-  __shared__ int s_cnt[KTX_EMAX];
-  __shared__ int s_off[KTX_EMAX];
-  __shared__ int s_toff[KTX_EMAX];
-  __shared__ int s_cur[KTX_EMAX];
-  __shared__ float s_red[16];
-  const int tid = threadIdx.x;
-  int T = p.qlen;
-  if (p.d_bsz) T = min(max(*p.d_bsz, 0), p.qlen);
-
-  if (blockIdx.x > 0) {
-    const int t = blockIdx.x - 1;
-    if (t >= T) return;
-    quant_row_block(p.x + (size_t)t * p.H, p.H, p.x_q + (size_t)t * p.H, p.x_d + t, s_red);
-    return;
-  }
-
-  // ---- block 0: histogram -> offsets -> STABLE scatter -> tile list -------------------------------------
-  // Rows of an expert are laid out in (token, slot) order — the reference's m_local_pos_ (moe_base.hpp:208-227): the row of a
-  // pair depends on the routing table only, never on arrival order.  Two implementations of the rank "how many earlier pairs
-  // chose the same expert":
-  //  * per-expert token bitmaps (the common case: a token names an expert at most once).  A window of 32 * bm_words tokens at a
-  //    time: every pair sets its token's bit in its expert's bitmap (an OR: order-free), one thread per expert turns the words
-  //    into exclusive popcount prefixes, and a pair's rank is prefix[word] + popcount(bits below its token) — O(1) per pair;
-  //  * a wavefront-ballot counting sort for routing tables in which a token names one expert twice (detected by the OR): a wave
-  //    finds the lanes holding the same expert with one ballot per distinct expert (match-any loop), the rank inside the wave
-  //    is a popcount of the lower lanes, the 16 waves of a 1024-pair chunk are chained through a per-(wave, expert) count
-  //    window in LDS, chunks through a running count.
-  extern __shared__ int s_dyn[];
-  __shared__ int s_dup;
-  const int E = p.E, npairs = T * p.k;
-  const int lane = tid & 63, wave = tid >> 6;
-  for (int e = tid; e < E; e += blockDim.x) { s_cnt[e] = 0; s_cur[e] = 0; }
-  if (tid == 0) s_dup = 0;
-  __syncthreads();
-  auto expert_of = [&](int i) -> int {
-    if (i >= npairs) return -1;
-    const long long id = p.ids[i] - p.expert_begin;
-    return (id >= 0 && id < E && !(p.mask && p.mask[id])) ? (int)id : -1;
-  };
-  for (int i = tid; i < npairs; i += blockDim.x) {   // per-expert totals (an integer sum: the order of the adds does not matter)
-    const int e = expert_of(i);
-    if (e >= 0) atomicAdd(&s_cnt[e], 1);
-  }
-  __syncthreads();
-  if (tid < 64) {  // wave 0: exclusive scans of counts and of tile counts
-    const int per = (E + 63) / 64;
-    const int e0 = tid * per;
-    int sum = 0, tsum = 0;
-    for (int e = e0; e < min(e0 + per, E); e++) {
-      sum += s_cnt[e];
-      tsum += (s_cnt[e] + p.rows_per_tile - 1) / p.rows_per_tile;
-    }
-    int inc = sum, tinc = tsum;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      int a = __shfl_up(inc, o, 64), b = __shfl_up(tinc, o, 64);
-      if (tid >= o) { inc += a; tinc += b; }
-    }
-    int run = inc - sum, trun = tinc - tsum;
-    for (int e = e0; e < min(e0 + per, E); e++) {
-      s_off[e] = run;
-      s_toff[e] = trun;
-      run += s_cnt[e];
-      trun += (s_cnt[e] + p.rows_per_tile - 1) / p.rows_per_tile;
-    }
-    if (tid == 63) { p.counters[0] = tinc; p.counters[1] = inc; }
-  }
-  __syncthreads();
-  {   // ---- bitmap scatter, window by window
-    const int nw = p.bm_words, WT = nw * 32;
-    unsigned* bm = reinterpret_cast<unsigned*>(s_dyn);   // [E][nw]
-    int* pc = s_dyn + E * nw;                             // [E][nw + 1]: exclusive popcount prefixes, window total last
-    for (int t0 = 0; t0 < T && !s_dup; t0 += WT) {
-      const int i0 = t0 * p.k, i1 = min(T, t0 + WT) * p.k;
-      for (int i = tid; i < E * nw; i += blockDim.x) bm[i] = 0u;
-      __syncthreads();
-      for (int i = i0 + tid; i < i1; i += blockDim.x) {
-        const int e = expert_of(i);
-        if (e >= 0) {
-          const int t = i / p.k - t0;
-          const unsigned bit = 1u << (t & 31);
-          if (atomicOr(&bm[e * nw + (t >> 5)], bit) & bit) s_dup = 1;   // the token names this expert twice
-        }
-      }
-      __syncthreads();
-      if (s_dup) break;
-      for (int e = wave; e < E; e += 16) {   // one wave per expert: lane = bitmap word (nw <= 64), shuffle prefix sum
-        const int c = lane < nw ? __popc(bm[e * nw + lane]) : 0;
-        int inc = c;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const int a = __shfl_up(inc, o, 64);
-          if (lane >= o) inc += a;
-        }
-        if (lane < nw) pc[e * (nw + 1) + lane] = inc - c;
-        if (lane == 63) pc[e * (nw + 1) + nw] = inc;
-      }
-      __syncthreads();
-      for (int i = i0 + tid; i < i1; i += blockDim.x) {
-        const int e = expert_of(i);
-        int r = -1;
-        if (e >= 0) {
-          const int t = i / p.k - t0, w = t >> 5;
-          r = s_off[e] + s_cur[e] + pc[e * (nw + 1) + w] + __popc(bm[e * nw + w] & ((1u << (t & 31)) - 1u));
-          p.src_of_row[r] = i / p.k;
-        }
-        p.row_of_pair[i] = r;
-      }
-      __syncthreads();
-      for (int e = tid; e < E; e += blockDim.x) s_cur[e] += pc[e * (nw + 1) + nw];
-      __syncthreads();
-    }
-  }
-  if (s_dup) {   // ---- ballot counting sort over ALL pairs (rows already written by the bitmap windows are rewritten identically)
-    int* s_wcnt = s_dyn;   // [16 waves][E]: zero outside the current chunk's window
-    for (int e = tid; e < E; e += blockDim.x) s_cur[e] = 0;
-    for (int i = tid; i < 16 * E; i += blockDim.x) s_wcnt[i] = 0;
-    __syncthreads();
-    for (int base = 0; base < npairs; base += 1024) {
-      const int i = base + tid;
-      const int e = expert_of(i);
-      int rank = 0;
-      unsigned long long rem = __ballot(e >= 0);
-      while (rem) {   // wave-uniform loop: one round per distinct expert among the wave's 64 pairs
-        const int lead = __builtin_amdgcn_readfirstlane(__ffsll((long long)rem) - 1);
-        const int e0 = __builtin_amdgcn_readlane(e, lead);
-        const unsigned long long m = __ballot(e == e0);
-        if (e == e0) rank = __popcll(m & ((1ull << lane) - 1ull));
-        if (lane == lead) s_wcnt[wave * E + e0] = __popcll(m);
-        rem &= ~m;
-      }
-      __syncthreads();
-      int r = -1;
-      if (e >= 0) {
-        int pre = 0;
-        for (int w = 0; w < wave; w++) pre += s_wcnt[w * E + e];
-        r = s_off[e] + s_cur[e] + pre + rank;
-        p.src_of_row[r] = i / p.k;
-      }
-      if (i < npairs) p.row_of_pair[i] = r;
-      __syncthreads();
-      if (e >= 0 && rank == 0) {   // one lane per (wave, expert): advance the running count, close the window
-        atomicAdd(&s_cur[e], s_wcnt[wave * E + e]);
-        s_wcnt[wave * E + e] = 0;
-      }
-      __syncthreads();
-    }
-  }
-  for (int e = tid; e < E; e += blockDim.x) {
-    const int c = s_cnt[e];
-    for (int i = 0, r = 0; r < c; i++, r += p.rows_per_tile) {
-      Tile t;
-      t.expert = e; t.row0 = s_off[e] + r; t.nrows = min(p.rows_per_tile, c - r); t.idx = i;
-      t.cnt = (c + p.rows_per_tile - 1) / p.rows_per_tile;
-      p.tiles[s_toff[e] + i] = t;
-    }
-  }
-}
-
-// launch: the scatter's bitmaps / count window live in dynamic LDS (beyond 48 KB the attribute is needed)
-static hipError_t launch_moe_prep(const PrepParams& pp, int nblocks, hipStream_t st) {
-  const hipError_t attr_err = ktx_set_max_lds(reinterpret_cast<const void*>(moe_prep_kernel), 96 * 1024);
-  if (attr_err != hipSuccess) return attr_err;
-  PrepParams p2 = pp;
-  const int E = std::max(pp.E, 1);
-  p2.bm_words = std::max(1, std::min(64, (64 * 1024) / (8 * E)));   // ~64 KB of bitmaps + prefixes per window
-  const size_t smem = std::max((size_t)16 * E * sizeof(int), (size_t)E * (2 * p2.bm_words + 1) * sizeof(int));
-  hipLaunchKernelGGL(moe_prep_kernel, dim3(nblocks), dim3(1024), smem, st, p2);
-  return hipGetLastError();
-}
-
-// =====================================================================================================
 // Kq: per-row int8 quantisation of the activated intermediate (a11: down_ba_->from_mat, moe_base.hpp:378-384)
 // =====================================================================================================
-__device__ __forceinline__ uint2 quant8(const uint4& v, float id);
-__device__ __forceinline__ float amax8(const uint4& v, float m);
 // One workgroup per sorted row.  gu = [row][g | u] bf16 from the gate/up GEMM: a = bf16(act_fn(g, u)) (a10,
 // moe_base.hpp:693-726) is formed in registers (K <= 8192: four 8-element pieces per thread), then quantised per row exactly
-// like quant_row_block (d = amax/127, q = sat8(rne(a * (1/d)))).
+// like moe_prep_kernel (d = amax/127, q = sat8(rne(a * (1/d)))).
 __global__ __launch_bounds__(256) void moe_actquant_kernel(const bf16_t* __restrict__ gu, int K, int8_t* __restrict__ a_q,
                                                            float* __restrict__ a_d, const int32_t* counters) {
   __shared__ float s_red[4];
@@ -860,62 +630,6 @@ void moe_dec_down_kernel(DecParams p) {
       *yp = ob;
     }
   }
-}
-
-// =====================================================================================================
-// K3: weighted combine in slot order (a12) + merge/incremental + bf16 (a4)
-// =====================================================================================================
-struct CombineParams {
-  const int32_t* d_bsz;
-  int qlen, k, H;
-  const bf16_t* dn;            // [sorted rows][H]
-  const int32_t* row_of_pair;  // [qlen*k]
-  const float* weights;        // [qlen][k]
-  bf16_t* y;                   // [qlen][H]  (float* when partial_f32)
-  int incremental;
-  int partial_f32;
-  int dn_f32;                  // GGUF path: dn is fp32 and the sum is `out += dn * w` (llamafile/moe.hpp:447-449)
-};
-
-__global__ __launch_bounds__(256) void moe_combine_kernel(CombineParams p) {
-  int T = p.qlen;
-  if (p.d_bsz) T = min(max(*p.d_bsz, 0), p.qlen);
-  const int t = blockIdx.y;
-  if (t >= T) return;
-  const int h = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (h >= p.H) return;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int j = 0; j < p.k; j++) {
-    const int r = p.row_of_pair[t * p.k + j];
-    if (r < 0) continue;
-    const float w = p.weights[t * p.k + j];
-    if (p.dn_f32) {
-      const float4 f = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(p.dn) + (size_t)r * p.H + h);
-      acc[0] = acc[0] + f.x * w; acc[1] = acc[1] + f.y * w; acc[2] = acc[2] + f.z * w; acc[3] = acc[3] + f.w * w;
-      continue;
-    }
-    const uint2 v = *reinterpret_cast<const uint2*>(p.dn + (size_t)r * p.H + h);
-    acc[0] = fmaf(bf16_to_f32((bf16_t)(v.x & 0xffffu)), w, acc[0]);
-    acc[1] = fmaf(bf16_to_f32((bf16_t)(v.x >> 16)), w, acc[1]);
-    acc[2] = fmaf(bf16_to_f32((bf16_t)(v.y & 0xffffu)), w, acc[2]);
-    acc[3] = fmaf(bf16_to_f32((bf16_t)(v.y >> 16)), w, acc[3]);
-  }
-  if (p.partial_f32) {  // expert-parallel partial: un-rounded fp32 sums, reduced across ranks by the caller
-    float* fp = reinterpret_cast<float*>(p.y) + (size_t)t * p.H + h;
-    *reinterpret_cast<float4*>(fp) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-    return;
-  }
-  bf16_t* yp = p.y + (size_t)t * p.H + h;
-  if (p.incremental) {
-    const uint2 o = *reinterpret_cast<const uint2*>(yp);
-    acc[0] = acc[0] + bf16_to_f32((bf16_t)(o.x & 0xffffu));
-    acc[1] = acc[1] + bf16_to_f32((bf16_t)(o.x >> 16));
-    acc[2] = acc[2] + bf16_to_f32((bf16_t)(o.y & 0xffffu));
-    acc[3] = acc[3] + bf16_to_f32((bf16_t)(o.y >> 16));
-  }
-  const uint32_t lo = (uint32_t)f32_to_bf16(acc[0]) | ((uint32_t)f32_to_bf16(acc[1]) << 16);
-  const uint32_t hi = (uint32_t)f32_to_bf16(acc[2]) | ((uint32_t)f32_to_bf16(acc[3]) << 16);
-  *reinterpret_cast<uint2*>(yp) = make_uint2(lo, hi);
 }
 
 // =====================================================================================================
@@ -2739,7 +2453,7 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
   pp.tiles = ws->tiles; pp.counters = ws->counters;
   {
     ProfScope ps(0, st);
-    KTX_HIP(launch_moe_prep(pp, qlen + 1, st));
+    KTX_HIP(moe_launch_prep(pp, true, st));
   }
   KTX_HIP(hipGetLastError());
 
@@ -2780,7 +2494,7 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
   cp.partial_f32 = (flags & KTX_FWD_PARTIAL_F32) ? 1 : 0;
   {
     ProfScope ps(4, st);
-    hipLaunchKernelGGL(moe_combine_kernel, dim3((H / 4 + 255) / 256, qlen), dim3(256), 0, st, cp);
+    KTX_HIP(moe_launch_combine(cp, st));
   }
   KTX_HIP(hipGetLastError());
   return 0;
@@ -2869,7 +2583,7 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
   pp.tiles = ws->tiles; pp.counters = ws->counters;
   {
     ProfScope ps(0, st);
-    KTX_HIP(launch_moe_prep(pp, 1, st));  // block 0 only: bucketing, no quantisation
+    KTX_HIP(moe_launch_prep(pp, false, st));   // bucketing only
   }
   KTX_HIP(hipGetLastError());
 
@@ -2900,7 +2614,7 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
   cp.partial_f32 = (flags & KTX_FWD_PARTIAL_F32) ? 1 : 0;
   {
     ProfScope ps(4, st);
-    hipLaunchKernelGGL(moe_combine_kernel, dim3((H / 4 + 255) / 256, qlen), dim3(256), 0, st, cp);
+    KTX_HIP(moe_launch_combine(cp, st));
   }
   KTX_HIP(hipGetLastError());
   return 0;
@@ -2973,7 +2687,7 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   pp.tiles = ws->tiles; pp.counters = ws->counters;
   {
     ProfScope ps(0, st);
-    KTX_HIP(launch_moe_prep(pp, 1, st));
+    KTX_HIP(moe_launch_prep(pp, false, st));
     hipLaunchKernelGGL(chunk ? moe_actquant_kgroup_kernel<true> : moe_actquant_kgroup_kernel<false>, dim3(qlen), dim3(256), 0, st,
                        (const bf16_t*)d_input, H, ws->x_q, ws->x_d, ws->counters, d_bsz, qlen, 1);
   }
@@ -3009,7 +2723,7 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   cp.partial_f32 = (flags & KTX_FWD_PARTIAL_F32) ? 1 : 0;
   {
     ProfScope ps(4, st);
-    hipLaunchKernelGGL(moe_combine_kernel, dim3((H / 4 + 255) / 256, qlen), dim3(256), 0, st, cp);
+    KTX_HIP(moe_launch_combine(cp, st));
   }
   KTX_HIP(hipGetLastError());
   return 0;
@@ -3025,7 +2739,7 @@ extern "C" int ktx_moe_combine(int qlen, int k, int hidden, const void* d_rows, 
   CombineParams cp{};
   cp.d_bsz = nullptr; cp.qlen = qlen; cp.k = k; cp.H = hidden; cp.dn = (const bf16_t*)d_rows; cp.row_of_pair = d_row_of_pair;
   cp.weights = d_weights; cp.y = (bf16_t*)d_output; cp.incremental = incremental ? 1 : 0;
-  hipLaunchKernelGGL(moe_combine_kernel, dim3((hidden / 4 + 255) / 256, qlen), dim3(256), 0, (hipStream_t)stream, cp);
+  KTX_HIP(moe_launch_combine(cp, (hipStream_t)stream));
   KTX_HIP(hipGetLastError());
   return 0;
 }
@@ -3135,7 +2849,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
     pp.rows_per_tile = 16; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
     pp.x_q = ws->x_q; pp.x_d = ws->x_d; pp.row_of_pair = ws->row_of_pair; pp.src_of_row = ws->src_of_row;
     pp.tiles = ws->tiles; pp.counters = ws->counters;
-    KTX_HIP(launch_moe_prep(pp, 1, st));
+    KTX_HIP(moe_launch_prep(pp, false, st));
     hipLaunchKernelGGL(q80_quant_kernel<false>, dim3(qlen), dim3(256), 0, st, d_input, H, ws->x_q, ws->x_d, d_bsz, 1, qlen);
     KTX_HIP(hipGetLastError());
     GlGemmParams g1{};
@@ -3162,7 +2876,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
     cp.d_bsz = d_bsz; cp.qlen = qlen; cp.k = k; cp.H = H; cp.dn = ws->dn_buf; cp.row_of_pair = ws->row_of_pair;
     cp.weights = d_weights; cp.y = (bf16_t*)d_output; cp.incremental = (flags & KTX_FWD_INCREMENTAL) ? 1 : 0;
     cp.partial_f32 = (flags & KTX_FWD_PARTIAL_F32) ? 1 : 0; cp.dn_f32 = 1;
-    hipLaunchKernelGGL(moe_combine_kernel, dim3((H / 4 + 255) / 256, qlen), dim3(256), 0, st, cp);
+    KTX_HIP(moe_launch_combine(cp, st));
     KTX_HIP(hipGetLastError());
     return 0;
   }
@@ -3275,7 +2989,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   pp.tiles = ws->tiles; pp.counters = ws->counters;
   {
     ProfScope ps(0, st);
-    KTX_HIP(launch_moe_prep(pp, 1, st));
+    KTX_HIP(moe_launch_prep(pp, false, st));
     hipLaunchKernelGGL(q8k_quant_kernel<false>, dim3(qlen), dim3(256), 0, st, d_input, H, ws->x_q, ws->x_d, ws->x_bs, x_bsp, x_b256, d_bsz, 1, qlen,
                        gg_unit_codes(h->gg_type[0]));
   }
@@ -3311,7 +3025,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   cp.partial_f32 = (flags & KTX_FWD_PARTIAL_F32) ? 1 : 0; cp.dn_f32 = 1;
   {
     ProfScope ps(4, st);
-    hipLaunchKernelGGL(moe_combine_kernel, dim3((H / 4 + 255) / 256, qlen), dim3(256), 0, st, cp);
+    KTX_HIP(moe_launch_combine(cp, st));
   }
   KTX_HIP(hipGetLastError());
   return 0;
