@@ -1134,8 +1134,7 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
 // One workgroup: 4 wavefronts x 2 query tiles of 16 = 128 queries, one head; keys in tiles of 64.
 // =====================================================================================================
 #define PF_BN 64
-#define PF_KROW 200     // 192 + 8 bf16: 400 B rows (25 x 16 B)
-#define PF_VROW 72      // 64 + 8 bf16: 144 B rows (9 x 16 B)
+constexpr int PF_KN = PF_BN * 256, PF_KB = PF_KN + PF_BN * 128, PF_VB = 128 * 128;   // LDS bytes of a key tile: [key][128] | [key][64] | V^T [dim][64 keys]
 struct MlaPrefillParams {
   const bf16_t *q_nope, *q_pe;   // [T][H][128] / [T][H][64] with element strides below
   long long qn_ts, qn_hs, qp_ts, qp_hs;
@@ -1146,68 +1145,26 @@ struct MlaPrefillParams {
   bf16_t* out;                   // [T][H][128]
   int T, H, kv_len, kv_pad;
   float sm_scale;
-  int no_skip;                   // dev knob 23 = 1: round 3's unconditional mask and rescale (A/B)
   int nqb;                       // > 0: 1-D XCD-aware grid of nqb query blocks x H heads (H % 8 == 0); 0: grid (query blocks, heads)
 };
 
-// one 64-key tile of one head in flight in registers: K_nope (64 keys x 16 pieces, contiguous), k_pe (64 keys x 8 pieces of the
-// cache rows; nothing is valid past kv_len), V^T (128 dims x 8 pieces of 8 keys).  Branch-free and by value, so it lives in
-// VGPRs (a lambda filling captured arrays under a condition was demoted to scratch memory).
-struct PfTile { uint4 k0, k1, k2, k3, r0, r1, v0, v1, v2, v3; };
-__device__ __forceinline__ uint4 pf_kpe_piece(const MlaPrefillParams& p, int j0, int idx) {
-  const int key = j0 + (idx >> 3);
-  const uint4 v = *reinterpret_cast<const uint4*>(p.k_pe + (size_t)min(key, p.kv_len - 1) * p.kpe_ts + (idx & 7) * 8);
-  const uint32_t keep = key < p.kv_len ? 0xffffffffu : 0u;
-  return make_uint4(v.x & keep, v.y & keep, v.z & keep, v.w & keep);
-}
-__device__ __forceinline__ PfTile pf_load_tile(const MlaPrefillParams& p, const bf16_t* kn, const bf16_t* vt, int tile, int tid) {
-  const int j0 = tile * PF_BN;
-  const bf16_t* kb = kn + (size_t)j0 * 128 + (size_t)tid * 8;
-  const bf16_t* vb = vt + (size_t)(tid >> 3) * p.kv_pad + j0 + (tid & 7) * 8;
-  const size_t vs = (size_t)32 * p.kv_pad;           // 256 threads = 32 dim rows per step
-  PfTile t;
-  t.k0 = *reinterpret_cast<const uint4*>(kb);
-  t.k1 = *reinterpret_cast<const uint4*>(kb + 2048);
-  t.k2 = *reinterpret_cast<const uint4*>(kb + 4096);
-  t.k3 = *reinterpret_cast<const uint4*>(kb + 6144);
-  t.r0 = pf_kpe_piece(p, j0, tid);
-  t.r1 = pf_kpe_piece(p, j0, tid + 256);
-  t.v0 = *reinterpret_cast<const uint4*>(vb);
-  t.v1 = *reinterpret_cast<const uint4*>(vb + vs);
-  t.v2 = *reinterpret_cast<const uint4*>(vb + 2 * vs);
-  t.v3 = *reinterpret_cast<const uint4*>(vb + 3 * vs);
-  return t;
-}
-__device__ __forceinline__ void pf_store_tile(const PfTile& t, bf16_t* Ks, bf16_t* Vs, int tid) {
-  bf16_t* kd = Ks + (tid >> 4) * PF_KROW + (tid & 15) * 8;       // 256 threads = 16 key rows per step
-  *reinterpret_cast<uint4*>(kd) = t.k0;
-  *reinterpret_cast<uint4*>(kd + 16 * PF_KROW) = t.k1;
-  *reinterpret_cast<uint4*>(kd + 32 * PF_KROW) = t.k2;
-  *reinterpret_cast<uint4*>(kd + 48 * PF_KROW) = t.k3;
-  bf16_t* rd = Ks + (tid >> 3) * PF_KROW + 128 + (tid & 7) * 8;  // 32 key rows per step
-  *reinterpret_cast<uint4*>(rd) = t.r0;
-  *reinterpret_cast<uint4*>(rd + 32 * PF_KROW) = t.r1;
-  bf16_t* vd = Vs + (tid >> 3) * PF_VROW + (tid & 7) * 8;
-  *reinterpret_cast<uint4*>(vd) = t.v0;
-  *reinterpret_cast<uint4*>(vd + 32 * PF_VROW) = t.v1;
-  *reinterpret_cast<uint4*>(vd + 64 * PF_VROW) = t.v2;
-  *reinterpret_cast<uint4*>(vd + 96 * PF_VROW) = t.v3;
-}
-
-// MINW = wavefronts per SIMD the register allocation must allow.  Unconstrained (MINW = 1) the compiler takes 340 VGPRs: ONE
-// wavefront per SIMD, one workgroup per CU, so the QK MFMAs, the softmax VALU chain, the PV MFMAs and the staging of the next
-// tile run strictly one after the other (0.10 of the MFMA peak).  MINW = 2 caps the allocation at 256 (7 values
-// spill to scratch) and two workgroups share a CU: one's softmax runs under the other's MFMAs.  Dev knob 22 = 1 selects MINW = 1.
-// NU = query tiles of 16 per wavefront: 2 (default: 128 queries per workgroup, every K fragment read feeds two MFMAs) or 1 (dev knob 31:
-// 64 queries per workgroup, half the registers -> three wavefronts per SIMD; measured in DESIGN.md 4.2.4)
-template <int MINW, int NU>
-__global__ __launch_bounds__(256, MINW) void mla_prefill_kernel(MlaPrefillParams p) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  bf16_t* Ks = reinterpret_cast<bf16_t*>(smem);      // [64][PF_KROW]
-  bf16_t* Vs = Ks + PF_BN * PF_KROW;                 // [128][PF_VROW]
+// S of the NEXT tile is computed beside the softmax of this one: 48 MFMAs and ~200 vector instructions that do not wait for each other, in one stream (before,
+// 1280 cycles of MFMAs and ~1450 of vector ALU a tile ran one after the other, and two workgroups a CU hid a third of that).  That takes a second set of scores, 32
+// registers, which the tiles' way through registers left no room for: K, k_pe and V^T come by LDS-DMA, double-buffered, 80 KB a workgroup, two workgroups a CU.
+// A lane's 8 probabilities of a half tile are those of 8 keys that follow each other (which K rows a fragment takes is free), so a V^T fragment is one read.
+// Rows lie unpadded, their 16-byte pieces permuted so that no read has bank conflicts (ds_read_b128 takes lanes 0-3, 12-15, 20-23 and 24-27 together): with i the lane
+// that reads the row, K: piece c in slot c ^ i; k_pe and V^T, 8 pieces a row: c ^ (i >> 1).
+// 128 heads, us, one after the other -> here: 1000 tokens behind 3096 367 -> 317 (788 -> 930 TFLOP/s), 2048 of 8192 1332 -> 1126, 2048 of 2048 260 -> 226, 512 of 512 32 -> 29; 16
+// heads, 300 of 1500: 50 -> 41.  Matrix pipe 44 % busy, vector ALU 42 %, LDS 17 % (58 % with two b64 reads a V^T fragment and padded rows); the clock is 2.0 GHz.  Left to
+// its own order the compiler puts the products first, each fragment's read directly before its use, and the softmax behind them: 325 us.
+// DMA false: operands that do not lie on 16 bytes come through registers, into the same places.
+template <bool DMA>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void mla_prefill_kernel(MlaPrefillParams p) {
+  constexpr int NU = 2;                              // query tiles of 16 per wavefront: every K fragment read feeds two MFMAs
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][PF_KB] | [2][PF_VB]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // blockIdx -> (head, query block).  Round 5, XCD-aware (p.nqb > 0: a 1-D grid): workgroup ids are dealt round-robin to the 8 XCDs, so
+  // blockIdx -> (head, query block).  XCD-aware (p.nqb > 0: a 1-D grid): workgroup ids are dealt round-robin to the 8 XCDs, so
   // id % 8 picks the XCD; all query blocks of ONE head go to one XCD (head % 8 == XCD) and run there back to back — the head's K / V^T
   // (1 MB at 2048 keys) is fetched into that XCD's L2 once instead of into all eight.  Within a head: heaviest query blocks first
   // (causal: the last block sees the whole context).
@@ -1223,6 +1180,37 @@ __global__ __launch_bounds__(256, MINW) void mla_prefill_kernel(MlaPrefillParams
   const int q0 = qb * (64 * NU) + wave * (16 * NU);
   const int qi = lane & 15, g = lane >> 4;
   const int pos_off = p.kv_len - p.T;                // query t sits at position pos_off + t
+  const int pos_max = pos_off + min(qb * (64 * NU) + 64 * NU - 1, p.T - 1);
+  const int ntiles = min(pos_max, p.kv_len - 1) / PF_BN + 1;
+  const bf16_t* kn = p.k_nope + (size_t)h * p.kv_pad * 128;
+  const bf16_t* vt = p.v_t + (size_t)h * 128 * p.kv_pad;
+
+  // ---- a tile's requests, 10 a wavefront: 4 rows of K, 8 of k_pe or of V^T each.  Rows of k_pe past kv_len read the last one (their scores are masked).
+  const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+  const int er = wave * 8 + (lane >> 3), ep = (lane & 7) ^ (wave * 2 + ((lane >> 4) & 1)), vp = (lane & 7) ^ ((wave * 4 + (lane >> 4)) & 7);
+  const uint32_t ko_dma = (wave * 4 + (lane >> 4)) * 256 + ((lane & 15) ^ ((wave >> 1) * 4 + (lane >> 4))) * 16, vo_dma = (uint32_t)er * (uint32_t)p.kv_pad * 2u + vp * 16;
+  auto bring = [&](const bf16_t* base, uint32_t lane_bytes, uint32_t at) __attribute__((always_inline)) {   // 16 bytes a lane
+    if constexpr (DMA) mla_dma_row_sa(base, lane_bytes, lds0 + at);
+    else *reinterpret_cast<uint4*>(smem + at + lane * 16) = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(base) + lane_bytes);
+  };
+  auto stage_k = [&](int tile, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 4; c++) bring(kn + (size_t)(tile * PF_BN + c * 16) * 128, ko_dma ^ ((c & 1) * 128), buf * PF_KB + (c * 4 + wave) * 1024);
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const bf16_t* src = p.k_pe + (size_t)min(tile * PF_BN + c * 32 + er, p.kv_len - 1) * p.kpe_ts + ep * 8;
+      const uint32_t at = buf * PF_KB + PF_KN + (c * 4 + wave) * 1024;
+      if constexpr (DMA) mla_dma_row_a(src, lds0 + at);
+      else *reinterpret_cast<uint4*>(smem + at + lane * 16) = *reinterpret_cast<const uint4*>(src);
+    }
+  };
+  auto stage_v = [&](int tile, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 4; c++) bring(vt + (size_t)c * 32 * p.kv_pad + tile * PF_BN, vo_dma, 2 * PF_KB + buf * PF_VB + (c * 4 + wave) * 1024);
+  };
+  stage_k(0, 0);
+  stage_v(0, 0);
+  if (ntiles > 1) stage_k(1, 1);
 
   // Q^T fragments: lane (query qi, k-chunk g)
   v8bf qf[NU][6];
@@ -1246,117 +1234,138 @@ __global__ __launch_bounds__(256, MINW) void mla_prefill_kernel(MlaPrefillParams
     m_run[u] = -__builtin_inff();
     l_run[u] = 0.f;
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
 
-  const int pos_max = pos_off + min(qb * (64 * NU) + 64 * NU - 1, p.T - 1);
-  const int ntiles = min(pos_max, p.kv_len - 1) / PF_BN + 1;
-  const bf16_t* kn = p.k_nope + (size_t)h * p.kv_pad * 128;
-  const bf16_t* vt = p.v_t + (size_t)h * 128 * p.kv_pad;
-
-  // next tile in registers while the current one is consumed from LDS
-  PfTile nxt = pf_load_tile(p, kn, vt, 0, tid);
-  for (int tile = 0; tile < ntiles; tile++) {
-    __syncthreads();                                 // the previous tile's readers are done
-    pf_store_tile(nxt, Ks, Vs, tid);
-    __syncthreads();
-    nxt = pf_load_tile(p, kn, vt, min(tile + 1, ntiles - 1), tid);   // (unconditional: the last iteration re-reads its tile)
-    const int j0 = tile * PF_BN;
-    // ---- S^T = K Q^T: st[u][kt][r] = S[query qi of tile u][key j0 + 16*kt + 4*g + r] -------------------------------------
-    v4f st[NU][4];
-#pragma unroll
-    for (int u = 0; u < NU; u++)
-#pragma unroll
-      for (int kt = 0; kt < 4; kt++) st[u][kt] = v4f{0.f, 0.f, 0.f, 0.f};
-    // (k-chunk outermost, round 6: 4 x NU independent accumulators between two MFMAs of one chain — with the key tile outermost
-    // every MFMA waited for its predecessor's 8 passes with only the other query tile's MFMA in between; each accumulator still
-    // sums its six chunks in the same order)
+  const int fq = (qi >> 1) & 7;
+  const int kq = (qi >> 2) * 8 + (qi & 3);            // row i of a K fragment is key (i >> 2) * 8 + (i & 3), + 4 for odd kt, + 32 for kt >= 2
+  const int ko = kq * 256 + ((g ^ qi) << 4), ro = PF_KN + kq * 128 + ((g ^ fq) << 4), vo = 2 * PF_KB + qi * 128 + ((g ^ fq) << 4);
+  // ---- S^T = K Q^T: st[u][kt][r] = S[query qi of tile u][key 32*(kt/2) + 8*g + 4*(kt%2) + r].  k-chunk outermost: 4 x NU independent accumulators between two MFMAs of one chain
+  auto qk = [&](int buf, v4f (&st)[NU][4]) __attribute__((always_inline)) {
+    const uint8_t* kb = smem + buf * PF_KB;
 #pragma unroll
     for (int s = 0; s < 6; s++) {
 #pragma unroll
       for (int kt = 0; kt < 4; kt++) {
-        const v8bf a = as_v8bf(*reinterpret_cast<const uint4*>(Ks + (kt * 16 + qi) * PF_KROW + g * 8 + s * 32));
+        const v8bf a = as_v8bf(*reinterpret_cast<const uint4*>(s < 4 ? kb + (kt >> 1) * 8192 + (kt & 1) * 1024 + (ko ^ (s * 64)) : kb + (kt >> 1) * 4096 + (kt & 1) * 512 + (ro ^ ((s - 4) * 64))));
 #pragma unroll
-        for (int u = 0; u < NU; u++) st[u][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[u][s], st[u][kt], 0, 0, 0);
+        for (int u = 0; u < NU; u++) st[u][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[u][s], s ? st[u][kt] : v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
       }
     }
-    // ---- online softmax, per query (lane & 15; the 4 key-chunk lanes g of a query agree after the two exchanges) ---------
-    // Round 5: the causal mask only exists on a query block's last two key tiles — a tile every query of the wavefront sees whole
-    // (wave-uniform test) skips the 32 compares + selects, and the 64 multiplies of `o *= alpha` are skipped whenever no lane's running
-    // maximum moved (alpha == 1 exactly: the common case once the first tiles are past).  Same bits either way.
-    const bool tile_full = !p.no_skip && j0 + PF_BN - 1 <= min(pos_off + min(q0, p.T - 1), p.kv_len - 1);
-    // Round 6 (the kernel was VALU-issue-bound: 5.4 VALU per MFMA): the running maximum is kept on the RAW scores and the softmax
-    // scale rides in the exponent's multiply — p = exp2(s * c - m * c), c = sm_scale * log2(e): one packed fma (two scores per
-    // instruction) + v_exp instead of multiply, subtract, multiply, v_exp per score; the row sum is accumulated two scores per
-    // packed add.  sm_scale > 0, so max(s * scale) = scale * max(s): the same softmax to within fp32 rounding of the exponent
-    // (tests: rtol 2^-7 on the bf16 outputs against an fp32 softmax).
-    const float cexp = p.sm_scale * 1.44269504088896340736f;
-    uint4 pb[NU][2];
+  };
+
+  // One key tile of parity par: its scores are in st; MORE: the next tile's go to nx.
+  const float cexp = p.sm_scale * 1.44269504088896340736f;
+  auto step = [&](auto more, int par, int tile, v4f (&st)[NU][4], v4f (&nx)[NU][4]) __attribute__((always_inline)) {
+    constexpr bool MORE = decltype(more)::value;
+    if constexpr (MORE) {   // (the buffers' last readers were a step ago)
+      if (tile + 2 < ntiles) stage_k(tile + 2, par);
+      stage_v(tile + 1, par ^ 1);
+    }
+    const int j0 = tile * PF_BN;
+    // The causal mask only exists on a query block's last two key tiles: a tile every query of the wavefront sees whole (wave-uniform test) skips it.
+    // (the empty asm keeps this a wave-uniform BRANCH: speculated into selects, its compares + selects ran on every tile)
+    if (!(j0 + PF_BN - 1 <= min(pos_off + min(q0, p.T - 1), p.kv_len - 1))) {
 #pragma unroll
-    for (int u = 0; u < NU; u++) {
-      const int lim = min(pos_off + tq[u], p.kv_len - 1);       // last visible key of this lane's query
-      float mx = -__builtin_inff();
-      if (!tile_full) {
-        // (the empty asm keeps this a wave-uniform BRANCH: speculated into selects, its 31 compares + selects ran on every tile)
+      for (int u = 0; u < NU; u++) {
+        const int lim = min(pos_off + tq[u], p.kv_len - 1);       // last visible key of this lane's query
 #pragma unroll
         for (int kt = 0; kt < 4; kt++) {
 #pragma unroll
           for (int r = 0; r < 4; r++) {
-            const int key = j0 + kt * 16 + g * 4 + r;
+            const int key = j0 + (kt >> 1) * 32 + g * 8 + (kt & 1) * 4 + r;
             st[u][kt][r] = key <= lim ? st[u][kt][r] : -__builtin_inff();
           }
           asm volatile("" : "+v"(st[u][kt]));
         }
       }
+    }
+    // ---- online softmax, per query (lane & 15; the 4 key-chunk lanes g of a query agree after the two exchanges), beside the next tile's products.
+    // The running maximum is kept on the RAW scores and the softmax scale rides in the exponent's multiply: p = exp2(s * c - m * c), c = sm_scale * log2(e).
+    if constexpr (MORE) qk(par ^ 1, nx);
+    uint4 pb[NU][2];
+    float alpha[NU];
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      float mx = -__builtin_inff();
 #pragma unroll
       for (int kt = 0; kt < 4; kt++)
 #pragma unroll
         for (int r = 0; r < 4; r++) mx = fmaxf(mx, st[u][kt][r]);
       mx = pf_max_rows(mx);                                     // over the query's four key-chunk lanes (qi, qi + 16, + 32, + 48)
       const float m_new = fmaxf(m_run[u], mx);                  // finite from tile 0 on: key 0 is visible to every query
-      const float alpha = __builtin_amdgcn_exp2f((m_run[u] - m_new) * cexp);
-      const pf_v2f mc = {-m_new * cexp, -m_new * cexp}, cc = {cexp, cexp};
-      pf_v2f sum2 = {0.f, 0.f};
+      alpha[u] = __builtin_amdgcn_exp2f((m_run[u] - m_new) * cexp);
+      const float mc = -m_new * cexp;
+      float sum2[2] = {0.f, 0.f};
       float pv[4][4];
 #pragma unroll
       for (int kt = 0; kt < 4; kt++)
 #pragma unroll
-        for (int r = 0; r < 4; r += 2) {
-          const pf_v2f e = __builtin_elementwise_fma(pf_v2f{st[u][kt][r], st[u][kt][r + 1]}, cc, mc);
-          pv[kt][r] = __builtin_amdgcn_exp2f(e[0]);
-          pv[kt][r + 1] = __builtin_amdgcn_exp2f(e[1]);
-          sum2 += pf_v2f{pv[kt][r], pv[kt][r + 1]};
+        for (int r = 0; r < 4; r++) {
+          pv[kt][r] = __builtin_amdgcn_exp2f(fmaf(st[u][kt][r], cexp, mc));
+          sum2[r & 1] += pv[kt][r];
         }
-      const float sum = pf_sum_rows(sum2[0] + sum2[1]);
-      l_run[u] = l_run[u] * alpha + sum;
+      l_run[u] = l_run[u] * alpha[u] + pf_sum_rows(sum2[0] + sum2[1]);
       m_run[u] = m_new;
-      if (p.no_skip || !__all(alpha == 1.0f)) {
-        const pf_v2f a2 = {alpha, alpha};
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-#pragma unroll
-          for (int r = 0; r < 4; r += 2) {
-            const pf_v2f t = pf_v2f{o[u][i][r], o[u][i][r + 1]} * a2;
-            o[u][i][r] = t[0];
-            o[u][i][r + 1] = t[1];
-          }
-      }
 #pragma unroll
       for (int ks = 0; ks < 2; ks++)
         pb[u][ks] = make_uint4(ktx_pk_bf16(pv[2 * ks][0], pv[2 * ks][1]), ktx_pk_bf16(pv[2 * ks][2], pv[2 * ks][3]),
                                ktx_pk_bf16(pv[2 * ks + 1][0], pv[2 * ks + 1][1]), ktx_pk_bf16(pv[2 * ks + 1][2], pv[2 * ks + 1][3]));
     }
-    // ---- O^T += V^T P^T: o[u][i][r] = O[query qi][dim 16*i + 4*g + r] ----------------------------------------------------
+    if constexpr (MORE) {   // the order of that stream: a fragment's two MFMAs, the read of the fragment four further, the softmax's next instructions
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) {                  // (key half outermost: 8 x NU independent accumulators, same order per accumulator)
+      for (int f = 0; f < 24; f++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        if (f < 20) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x402, 6, 0);
+      }
+    }
+    // the multiplies of `o *= alpha` are skipped whenever no lane's running maximum moved (alpha == 1 exactly: the common case once the first tiles are past)
+#pragma unroll
+    for (int u = 0; u < NU; u++)
+      if (!__all(alpha[u] == 1.0f)) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) o[u][i] *= alpha[u];
+      }
+    // ---- O^T += V^T P^T: o[u][i][r] = O[query qi][dim 16*i + 4*g + r] ----------------------------------------------------
+    const uint8_t* vb = smem + par * PF_VB;
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {                  // (key half outermost: 8 x NU independent accumulators)
 #pragma unroll
       for (int i = 0; i < 8; i++) {
-        const bf16_t* vb = Vs + (i * 16 + qi) * PF_VROW + g * 4 + ks * 32;
-        const uint2 lo = *reinterpret_cast<const uint2*>(vb), hi = *reinterpret_cast<const uint2*>(vb + 16);
-        const v8bf a = as_v8bf(make_uint4(lo.x, lo.y, hi.x, hi.y));
+        const v8bf a = as_v8bf(*reinterpret_cast<const uint4*>(vb + i * 2048 + (vo ^ (ks * 64))));
 #pragma unroll
         for (int u = 0; u < NU; u++) o[u][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, as_v8bf(pb[u][ks]), o[u][i], 0, 0, 0);
       }
     }
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 1);
+#pragma unroll
+    for (int f = 0; f < 16; f++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 1);
+      if (f < 12) __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+    }
+    if constexpr (MORE) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (a step old)
+      __syncthreads();
+    }
+  };
+  v4f sa[NU][4], sb[NU][4];
+  qk(0, sa);
+  __syncthreads();   // (the first step's requests overwrite what this read)
+  int tile = 0;
+  for (; tile + 2 < ntiles; tile += 2) {
+    step(std::true_type{}, 0, tile, sa, sb);
+    step(std::true_type{}, 1, tile + 1, sb, sa);
   }
+  if (tile + 1 < ntiles) {
+    step(std::true_type{}, 0, tile++, sa, sb);
+#pragma unroll
+    for (int u = 0; u < NU; u++)
+#pragma unroll
+      for (int kt = 0; kt < 4; kt++) sa[u][kt] = sb[u][kt];
+  }
+  step(std::false_type{}, tile & 1, tile, sa, sb);
 #pragma unroll
   for (int u = 0; u < NU; u++) {
     const int t = q0 + u * 16 + qi;
@@ -1386,19 +1395,18 @@ extern "C" int ktx_mla_prefill(int T, int num_heads, int kv_len, int kv_pad, flo
   p.k_nope = (const bf16_t*)d_k_nope; p.k_pe = (const bf16_t*)d_k_pe; p.kpe_ts = kpe_token_stride;
   p.v_t = (const bf16_t*)d_v_t; p.out = (bf16_t*)d_out;
   p.T = T; p.H = num_heads; p.kv_len = kv_len; p.kv_pad = kv_pad; p.sm_scale = sm_scale;
-  p.no_skip = ktx_debug_get(23) == 1 ? 1 : 0;
-  const size_t lds = (size_t)(PF_BN * PF_KROW + 128 * PF_VROW) * sizeof(bf16_t);
+  constexpr int lds = 2 * (PF_KB + PF_VB);
+  const bool aligned = ((reinterpret_cast<uintptr_t>(d_k_nope) | reinterpret_cast<uintptr_t>(d_k_pe) | reinterpret_cast<uintptr_t>(d_v_t)) & 15) == 0;
+  KTX_HIP(ktx_set_max_lds(aligned ? reinterpret_cast<const void*>(mla_prefill_kernel<true>) : reinterpret_cast<const void*>(mla_prefill_kernel<false>), lds));
   hipStream_t st = (hipStream_t)stream;
   // per (query, key, head): 2*(192 + 128) flop over the causal half
   KTX_TIMED(st, 0.0, "mla_prefill_kernel T=%d Hq=%d kv=%d", T, num_heads, kv_len);
-  const bool one_tile = ktx_debug_get(31) == 1;                      // dev knob 31 = 1: one query tile per wavefront, three wavefronts per SIMD
-  const int nqb = one_tile ? (T + 63) / 64 : (T + 127) / 128;
-  const bool xcd = num_heads % 8 == 0 && ktx_debug_get(24) != 1;     // dev knob 24 = 1: the 2-D grid of rounds 2-4 (A/B)
+  const int nqb = (T + 127) / 128;
+  const bool xcd = num_heads % 8 == 0;
   p.nqb = xcd ? nqb : 0;
   const dim3 grid = xcd ? dim3((unsigned)(nqb * num_heads)) : dim3(nqb, num_heads);
-  if (one_tile) hipLaunchKernelGGL((mla_prefill_kernel<3, 1>), grid, dim3(256), lds, st, p);
-  else if (ktx_debug_get(22) == 1) hipLaunchKernelGGL((mla_prefill_kernel<1, 2>), grid, dim3(256), lds, st, p);
-  else hipLaunchKernelGGL((mla_prefill_kernel<2, 2>), grid, dim3(256), lds, st, p);
+  if (aligned) hipLaunchKernelGGL(mla_prefill_kernel<true>, grid, dim3(256), lds, st, p);
+  else hipLaunchKernelGGL(mla_prefill_kernel<false>, grid, dim3(256), lds, st, p);
   KTX_HIP(hipGetLastError());
   return 0;
 }

@@ -263,6 +263,34 @@ def test_prefill_expanded_against_fp32_attention(H, T, kv_len, knob22):
     torch.testing.assert_close(out.float(), ref.to(torch.bfloat16).float(), rtol=2.0 ** -7, atol=5e-3)
 
 
+@pytest.mark.parametrize("offset", [0, 4])   # elements: operands on 16 bytes come by LDS-DMA, others through registers
+@pytest.mark.parametrize("H,T,kv_len", [(1, 1, 1), (2, 1, 64), (2, 1, 65), (3, 129, 128 + 129), (8, 33, 320), (2, 256, 4160)])
+def test_prefill_tiles_of_keys(H, T, kv_len, offset):
+    """One key tile, two, odd and even counts of them, against attention in 64 bits.  Probabilities enter the product as bf16 (2^-8 of their size, and they sum to one)
+    and the output is rounded to bf16: 2^-8 of the largest value each, at most."""
+    from ktransformers_amd._native import mla_prefill
+    g = torch.Generator().manual_seed(H * 1000 + T + kv_len)
+    kv_pad = (kv_len + 63) // 64 * 64
+
+    def at_offset(x):
+        flat = torch.empty(x.numel() + offset, dtype=torch.bfloat16, device=DEV)
+        flat[offset:] = x.reshape(-1).to(DEV)
+        return flat[offset:].view(x.shape)
+
+    q = torch.randn((T, H, 192), generator=g).to(torch.bfloat16)
+    k_nope, v = torch.zeros((2, H, kv_pad, 128), dtype=torch.bfloat16)
+    k_nope[:, :kv_len] = torch.randn((H, kv_len, 128), generator=g).to(torch.bfloat16)
+    v[:, :kv_len] = torch.randn((H, kv_len, 128), generator=g).to(torch.bfloat16)
+    cache = torch.randn((kv_len, 576), generator=g).to(torch.bfloat16)
+    qd = q.to(DEV)
+    out = mla_prefill(qd[:, :, :128], qd[:, :, 128:], at_offset(k_nope), at_offset(cache)[:, 512:], at_offset(v.transpose(1, 2).contiguous()), kv_len, 192 ** -0.5)
+    k = torch.cat([k_nope[:, :kv_len].double(), cache[:, 512:].double()[None].expand(H, -1, -1)], dim=-1)
+    s = torch.matmul(q.double().transpose(0, 1), k.transpose(1, 2)) * 192 ** -0.5
+    s = s.masked_fill(torch.arange(kv_len)[None, :] > torch.arange(T)[:, None] + (kv_len - T), float("-inf"))
+    ref = torch.matmul(torch.softmax(s, dim=-1), v[:, :kv_len].double()).transpose(0, 1)
+    assert float((out.cpu().double() - ref).abs().max()) <= 2.0 ** -7 * float(v.double().abs().max())
+
+
 @pytest.mark.parametrize("Hq,kv_len,T", [(128, 4023, 1), (64, 700, 1), (128, 33, 1), (64, 5000, 3)])
 def test_merge_riding_the_unabsorb_launch(Hq, kv_len, T):
     """ktx_mla_decode_partials + ktx_linear_forward_batched_merge (the KV-split merge inside the launch of the per-head un-absorb
