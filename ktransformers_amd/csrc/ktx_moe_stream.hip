@@ -13,7 +13,7 @@
 // no work that no row needs and keeps both units fed:
 //   * a tile multiplies the 16-row groups that hold rows, by an instantiation for each count (a quarter of a 64-row tile is absent at 64 rows an expert);
 //   * each wavefront owns four 16-row weight strips (gate|up: two strips of both; down: four), so a fragment of activations feeds 4 MFMAs; weights stream
-//     through a ring of registers, 4 k-steps deep, or 8 where at most two groups' sums leave room;
+//     through a ring of registers, 4 k-steps deep.  That is 128 KB a CU, as much as its share of the L2 holds; 8 deep is slower (31 rows an expert: 1151 us against 1131);
 //   * activations come by LDS-DMA into one of two buffers of 4 or 8 k-steps while the other is multiplied.  Before, 2048 columns were staged at once, and nothing
 //     multiplied meanwhile: a fifth of the time of a 64-row tile.
 // NW = 8: one workgroup a CU.  NW = 4: two, of half the strips and half the LDS each, so that one starts or ends beside the other's MFMAs, and a job is half as
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   auto run = [&](auto mtl) __attribute__((always_inline)) {
     constexpr int MTL = decltype(mtl)::value;
     constexpr int SC = NW == 8 || MTL <= MT / 2 ? 8 : 4, ROWB = SC * 128;             // k-steps of a chunk; its bytes per row
-    constexpr int D = (MTL <= MT / 2 ? 8 : 4) / (WBITS / 4);               // k-steps of weights in flight
+    constexpr int D = 16 / WBITS;                                          // k-steps of weights in flight
     int xo[2][2];
 #pragma unroll
     for (int par = 0; par < 2; par++)
