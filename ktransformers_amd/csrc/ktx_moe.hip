@@ -718,42 +718,6 @@ __global__ void pack_w8_kernel(const int8_t* __restrict__ q, int N, int K, uint3
 // of its 32-k run);  BF16: tile 4096 B, four 1 KiB quarters, quarter j = the lane's fragment for MFMA j.
 // Activations are staged per 256-k chunk, row by row, by LDS-DMA.
 // =====================================================================================================
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ v8bf u4_as_v8bf(const uint4& u) {
-  union { uint4 u; v8bf v; } c;
-  c.u = u;
-  return c.v;
-}
-
-// 4 e4m3 bytes -> 4 bf16 (two dwords): v_cvt_pk_f32_fp8 is exact, and every e4m3 value is exact in bf16, so taking the
-// upper halves of the fp32 results is exact (OCP e4m3fn on gfx950; 0x7F/0xFF are NaN here, +-480 in the reference's LUT).
-__device__ __forceinline__ uint2 fp8x4_to_bf16x4(uint32_t v) {
-  // gfx950: v_cvt_scalef32_pk_bf16_fp8 converts two e4m3 bytes straight to two bf16 (scale 1.0): 2 VALU instructions per four weights
-  // instead of two converts + two packs (scripts/fp8_cvt_probe.hip: the same bits as the two-step path for all 256 codes)
-  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-  union { bf2 v; uint32_t u; } lo, hi;
-  lo.v = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, false);
-  hi.v = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, true);
-  return make_uint2(lo.u, hi.u);
-}
-
-struct FpGemmParams {
-  const uint8_t *w0, *w1;     // tiled weights (gate | down, up)
-  const float *s0, *s1;       // FP8: scale_inv [E][N/128][K/128]; BF16: nullptr
-  const float *r0, *r1;       // FP8_PERCHANNEL: scale per output row [E][N] (the block scales are then all 1), else nullptr
-  size_t expert_stride;       // bytes per expert matrix
-  size_t scale_stride;        // floats per expert
-  int N, K;
-  const bf16_t* act;          // [src rows][K] bf16
-  const int32_t* row_src;     // sorted row -> source row (nullptr: identity)
-  const Tile* tiles;
-  const int32_t* counters;
-  bf16_t* out;                // [sorted rows][N]
-};
-
-// the places of a row's pieces: distinct for 16 rows, also with rows 4 .. 11 flipped by 4 (ds_read_b128 takes lanes 0-3, 12-15, 20-23, 24-27 together)
-__device__ __forceinline__ int fp_swz(int row) { return (row & 3) | (int)((0x3102u >> (((row >> 2) & 3) * 4)) & 3u) << 2; }
 // WIDE (MT = 4): 8 wavefronts per workgroup and two B operands per wavefront for BOTH GEMMs (gate and up of a strip; two strips of down): at 64
 // rows every workgroup re-reads the tile's bf16 activations, with 4 strips as many bytes as the fp8 weights themselves.  At 32 rows 4 strips and
 // three wavefronts a SIMD are ahead (DeepSeek-V3 shape, 1000 tokens: 2307 us against 2587 of the wide form).
@@ -2512,7 +2476,14 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
   // 47: 3423 | 2873 | 2944, 62: 4142 | 3353 | 3290; 64 of 2048 x 1408, 9.4: 115 | 116 | 135, 66: 245 | 206 | 223, 94: 312 | 251 | 259, 141: 431 | 349 | 340;
   // 8 of 4096 x 1536, 25: 56 | 55 | 74, 75: 88 | 80 | 76, 250: 196 | 160 | 155; 128 of 4608 x 512, 7.4: 158 | 165
   const double rows = (double)npairs / std::max(1, E);
-  const int mt = rows <= 8.0 ? 1 : rows <= 60.0 ? 2 : 4;
+  // The streaming kernel (32 rows) where it has enough workgroups and rows.  Measured (us, the others | streaming): 256 of 7168 x 2048, 9.4 rows 1567 | 1617, 16: 1756 | 1782,
+  // 19: 1946 | 1903, 31: 2298 | 2185, 47: 2795 | 2641, 64: 3338 | 3012; 64 of 6144 x 3072, 15: 597 | 618, 37: 821 | 798, 94: 1243 | 1175; 128 of 5120 x 2048, 31: 875 | 828; 64 of
+  // 2048 x 1408, 28: 148 | 152, 48: 170 | 163, 75: 225 | 197, 192: 408 | 378; 64 of 2560 x 2048, 50: 294 | 276; 128 of 2048 x 512, 128: 289 | 257; with few workgroups either may be
+  // ahead: 8 of 4096 x 1536, 70 (300): 69 | 76, 100 (396): 88 | 75; 8 of 6144 x 3072, 100 (792): 200 | 209; 32 of 2560 x 1024, 50 (656): 83 | 89, 125 (1256): 164 | 146.
+  // Dev knob [6] (tests): 1 = never, 2 = always.
+  const bool fills = (std::min(npairs, E) + npairs / 32) * (I / 128) >= 1200 && rows >= ((size_t)H * I >= ((size_t)8 << 20) ? 24.0 : 48.0);
+  const bool stream = fp8 && g_dbg[6] != 1 && (g_dbg[6] == 2 || fills) && fp8_stream_lds(std::max(H, I)) <= 160 * 1024;
+  const int mt = stream ? 2 : rows <= 8.0 ? 1 : rows <= 60.0 ? 2 : 4;
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
 
   // ---- decode fast path: two launches (see moe_dec_fp_gateup_kernel) ------------------------------------------------------
@@ -2595,7 +2566,7 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
   int rc;
   {
     ProfScope ps(1, st);
-    rc = fp8 ? launch_gemm_fp<true, true>(mt, g1, max_tiles, st) : launch_gemm_fp<false, true>(mt, g1, max_tiles, st);
+    rc = stream ? moe_launch_fp8_stream(true, g1, max_tiles, st) : fp8 ? launch_gemm_fp<true, true>(mt, g1, max_tiles, st) : launch_gemm_fp<false, true>(mt, g1, max_tiles, st);
   }
   if (rc) return rc;
   FpGemmParams g2;
@@ -2605,7 +2576,7 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
   g2.tiles = ws->tiles; g2.counters = ws->counters; g2.out = ws->dn_buf;
   {
     ProfScope ps(3, st);
-    rc = fp8 ? launch_gemm_fp<true, false>(mt, g2, max_tiles, st) : launch_gemm_fp<false, false>(mt, g2, max_tiles, st);
+    rc = stream ? moe_launch_fp8_stream(false, g2, max_tiles, st) : fp8 ? launch_gemm_fp<true, false>(mt, g2, max_tiles, st) : launch_gemm_fp<false, false>(mt, g2, max_tiles, st);
   }
   if (rc) return rc;
   CombineParams cp{};

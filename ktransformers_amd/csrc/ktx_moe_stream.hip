@@ -1,4 +1,4 @@
-// ktx_moe_stream.hip — prompt GEMM of AMXINT4 / AMXINT8 experts (its own translation unit, compiled beside ktx_moe.hip).
+// ktx_moe_stream.hip — streaming prompt GEMMs of AMXINT4 / AMXINT8 and of FP8 experts (a translation unit of its own, compiled beside ktx_moe.hip).
 #include <hip/hip_runtime.h>
 #include <type_traits>
 
@@ -211,4 +211,199 @@ static int launch_gemm_stream(bool gate_up, const GemmParams& p, int max_tiles, 
 int moe_launch_gemm_stream(int wbits, int nw, bool gate_up, const GemmParams& p, int max_tiles, hipStream_t st) {
   if (wbits == 4) return nw == 4 ? launch_gemm_stream<4, 4>(gate_up, p, max_tiles, st) : launch_gemm_stream<4, 8>(gate_up, p, max_tiles, st);
   return nw == 4 ? launch_gemm_stream<8, 4>(gate_up, p, max_tiles, st) : launch_gemm_stream<8, 8>(gate_up, p, max_tiles, st);
+}
+
+// =====================================================================================================
+// The same for FP8 experts, on tiles of 32 rows, 4 wavefronts, two workgroups a CU; bf16 activations, 4 k-steps a buffer; weights 2 k-steps ahead, widened to bf16 a
+// quarter k-step before their MFMAs: 3.3 vector instructions an MFMA (6.2 in moe_gemm_fp_kernel, which waits for a chunk's weights at the end of the chunk before
+// it).  4 k-steps ahead, 256 KB a CU, are more than the L2 holds: 1000 tokens 2216 us against 2185.  8 wavefronts, one workgroup a CU: 2223.  Arithmetic, summation order and epilogue are moe_gemm_fp_kernel's: results are bit-identical.
+// Whole forward, us, moe_gemm_fp_kernel -> here: 256 experts of 7168 x 2048, top-8: 1000 tokens 2298 -> 2185, 2048 3338 -> 3012, 8192 8697 -> 8131; 64 of 2048 x 1408, top-6, 800: 225
+// -> 197; 64 of 6144 x 3072, top-6, 1000: 1243 -> 1175.  At fewer rows than the caller's rule asks for, more wavefronts of few registers stream better.
+// =====================================================================================================
+template <bool GATE_UP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_fp8_stream_kernel(FpGemmParams p) {
+  constexpr int NW = 4, NJ = 4, SPW = GATE_UP ? 2 : 4, SC = 4, D = 2;
+  constexpr int ROWB = SC * 256, XB = FP_STREAM_ROWS * ROWB, TILE_BYTES = 2048;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][XB] | scales [NW][2][NKS]
+
+  Tile tile;
+  int bx;
+  if (!moe_pick_job(p.tiles, p.counters[0], (p.N / 16 + NW * SPW - 1) / (NW * SPW), tile, bx)) return;
+  const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, kc = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int strip0 = (bx * NW + wave) * SPW, nstrips = p.N / 16, NKS = p.K / 128;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+
+  const uint8_t* wb[NJ];   // strips past N alias strip 0 and are not stored
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    const int st = strip0 + (GATE_UP ? (j >> 1) : j);
+    wb[j] = ((GATE_UP && (j & 1)) ? p.w1 : p.w0) + (size_t)tile.expert * p.expert_stride + (size_t)(st < nstrips ? st : 0) * NKS * TILE_BYTES;
+  }
+  float* s_sc = reinterpret_cast<float*>(smem + 2 * XB) + wave * 2 * NKS;   // a wavefront's strips lie in one block of 128 rows
+
+  auto run = [&](auto mtl) __attribute__((always_inline)) {
+    constexpr int MTL = decltype(mtl)::value;
+    uint4 ring[D][NJ][2];
+    int wlane = lane;
+    asm volatile("" : "+v"(wlane));   // (the instantiations' first loads are the same: merged, they would be held across each other's loops)
+    auto load_w = [&](int d, int ks) __attribute__((always_inline)) {
+      const int kn = ks < NKS ? ks : NKS - 1;
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int q = 0; q < 2; q++) ring[d][j][q] = *reinterpret_cast<const uint4*>(wb[j] + (size_t)kn * TILE_BYTES + q * 1024 + wlane * 16);
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++) load_w(d, d);
+    // A chunk's rows, one a request, dealt over the wavefronts.  A row past the tile reads its first one (not stored).
+    constexpr int NQ = MTL * 16 / NW;
+    int src[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      const int row = q * NW + wave, r = tile.row0 + (row < tile.nrows ? row : 0);
+      src[q] = __builtin_amdgcn_readfirstlane(p.row_src ? p.row_src[r] : r);
+    }
+    auto stage = [&](int q, int chunk) __attribute__((always_inline)) {
+      const int row = q * NW + wave;
+      int l = wlane;
+      asm volatile("" : "+v"(l));   // (the compiler otherwise keeps every request's offset in registers that the loop has not got)
+      const int piece = chunk * (ROWB / 16) + (l ^ fp_swz(row & 15));
+      moe_dma(p.act + (size_t)src[q] * p.K + min(piece, p.K / 8 - 1) * 8, lds0 + (chunk & 1) * XB + row * ROWB);
+    };
+#pragma unroll
+    for (int q = 0; q < NQ; q++) stage(q, 0);
+    for (int ks = lane; ks < NKS; ks += 64)
+#pragma unroll
+      for (int m = 0; m < (GATE_UP ? 2 : 1); m++) {
+        const int st = strip0 < nstrips ? strip0 : 0;
+        s_sc[m * NKS + ks] = (m ? p.s1 : p.s0)[(size_t)tile.expert * p.scale_stride + (size_t)(st / 8) * NKS + ks];
+      }
+
+    int xo[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) xo[j] = i * ROWB + (((kc * 4 + j) ^ fp_swz(i)) << 4);
+    v4f acc[NJ][MTL], tmp[NJ][MTL];
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+      for (int t = 0; t < MTL; t++) acc[j][t] = v4f{0.f, 0.f, 0.f, 0.f};
+    v8bf a[2][NJ], b[2][MTL];   // operands of two quarters
+    auto read_b = [&](auto sc, auto qc, int chunk) __attribute__((always_inline)) {
+      constexpr int s = decltype(sc)::value, q = decltype(qc)::value;
+      const uint8_t* xb = smem + (chunk & 1) * XB + s * 256 + xo[q];
+#pragma unroll
+      for (int t = 0; t < MTL; t++) b[q & 1][t] = u4_as_v8bf(*reinterpret_cast<const uint4*>(xb + t * (16 * ROWB)));
+    };
+    auto widen = [&](int d, auto qc) __attribute__((always_inline)) {
+      constexpr int q = decltype(qc)::value;
+#pragma unroll
+      for (int j = 0; j < NJ; j++) {
+        const uint4& w = ring[d][j][q >> 1];
+        const uint2 e0 = fp8x4_to_bf16x4(q & 1 ? w.z : w.x), e1 = fp8x4_to_bf16x4(q & 1 ? w.w : w.y);
+        a[q & 1][j] = u4_as_v8bf(make_uint4(e0.x, e0.y, e1.x, e1.y));
+      }
+    };
+    auto mul = [&](auto qc) __attribute__((always_inline)) {
+      constexpr int q = decltype(qc)::value;
+#pragma unroll
+      for (int t = 0; t < MTL; t++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) tmp[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q & 1][j], b[q & 1][t], q ? tmp[j][t] : v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    };
+    const std::integral_constant<int, 0> q0{};
+    // A k-step in quarters.  Beside a quarter's MFMAs: the reads and the widening of the next one's operands.
+    auto step = [&](auto sc, auto mc, int chunk) __attribute__((always_inline)) {
+      constexpr int s = decltype(sc)::value, d = s % D;
+      constexpr bool more = decltype(mc)::value;
+      static_for<3>([&](auto qc) __attribute__((always_inline)) {
+        constexpr std::integral_constant<int, decltype(qc)::value + 1> next{};
+        read_b(sc, next, chunk);
+        widen(d, next);
+        mul(qc);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if constexpr (more && s < SC / 2)   // the next chunk's rows, in the first half of this one
+#pragma unroll
+        for (int q = s; q < NQ; q += SC / 2) stage(q, chunk + 1);
+      load_w(d, chunk * SC + s + D);
+      if constexpr (s + 1 < SC) read_b(std::integral_constant<int, (s + 1) % SC>{}, q0, chunk);
+      float scale[2];
+#pragma unroll
+      for (int m = 0; m < (GATE_UP ? 2 : 1); m++) scale[m] = s_sc[m * NKS + chunk * SC + s];
+      widen((s + 1) % D, q0);
+      mul(std::integral_constant<int, 3>{});
+#pragma unroll
+      for (int t = 0; t < MTL; t++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[j][t][r] = fmaf(tmp[j][t][r], scale[GATE_UP ? j & 1 : 0], acc[j][t][r]);   // apply_scale_kgroup
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    widen(0, q0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int chunk = 0;
+    for (; (chunk + 1) * SC <= NKS; chunk++) {
+      read_b(q0, q0, chunk);
+      static_for<SC>([&](auto sc) __attribute__((always_inline)) { step(sc, std::true_type{}, chunk); });
+      // the next chunk is in the LDS (what was requested after its rows: SC / 2 + 1 steps of weights), and no one reads this one any more
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SC / 2 + 1) * NJ * 2) : "memory");
+      __syncthreads();
+    }
+    if (chunk * SC < NKS) {
+      read_b(q0, q0, chunk);
+      static_for<SC>([&](auto sc) __attribute__((always_inline)) {
+        if (chunk * SC + decltype(sc)::value < NKS) step(sc, std::false_type{}, chunk);
+      });
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no request may outlive the workgroup's LDS
+
+#pragma unroll
+    for (int u = 0; u < SPW; u++) {
+      const int st = strip0 + u;
+      if (st >= nstrips) continue;
+      const int n0 = st * 16 + kc * 4;
+#pragma unroll
+      for (int t = 0; t < MTL; t++) {
+        const int row = t * 16 + i;
+        if (row < tile.nrows) {
+          bf16_t o[4];
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            // FP8_PERCHANNEL: the whole-K sum times the row's scale; x * 1.0f is exact, so the block-scaled format is untouched
+            const float rs0 = p.r0 ? p.r0[(size_t)tile.expert * p.N + n0 + r] : 1.0f;
+            const bf16_t g = f32_to_bf16(acc[GATE_UP ? 2 * u : u][t][r] * rs0);
+            if constexpr (GATE_UP) {
+              const float rs1 = p.r1 ? p.r1[(size_t)tile.expert * p.N + n0 + r] : 1.0f;
+              const bf16_t up = f32_to_bf16(acc[2 * u + 1][t][r] * rs1);
+              o[r] = f32_to_bf16(act_fn(bf16_to_f32(g), bf16_to_f32(up)));
+            } else {
+              o[r] = g;
+            }
+          }
+          *reinterpret_cast<uint2*>(p.out + (size_t)(tile.row0 + row) * p.N + n0) =
+              make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
+        }
+      }
+    }
+  };
+  if (tile.nrows <= 16) run(std::integral_constant<int, 1>{});
+  else run(std::integral_constant<int, 2>{});
+}
+
+template <bool GATE_UP>
+static int launch_fp8_stream(const FpGemmParams& p, int max_tiles, hipStream_t st) {
+  constexpr int per_wg = 4 * (GATE_UP ? 2 : 4);   // strips
+  const int lds = (int)fp8_stream_lds(p.K);
+  const hipError_t err = ktx_set_max_lds(reinterpret_cast<const void*>(moe_fp8_stream_kernel<GATE_UP>), 160 * 1024);
+  KTX_HIP(err);
+  hipLaunchKernelGGL((moe_fp8_stream_kernel<GATE_UP>), moe_job_grid(max_tiles, (p.N / 16 + per_wg - 1) / per_wg), dim3(256), lds, st, p);
+  KTX_HIP(hipGetLastError());
+  return 0;
+}
+
+int moe_launch_fp8_stream(bool gate_up, const FpGemmParams& p, int max_tiles, hipStream_t st) {
+  return gate_up ? launch_fp8_stream<true>(p, max_tiles, st) : launch_fp8_stream<false>(p, max_tiles, st);
 }

@@ -759,6 +759,31 @@ def test_fp_grouped_edges(oracle, dev, fmt, H, I, rows):
         h.close()
 
 
+@pytest.mark.parametrize("H,I", [(128, 128), (384, 640), (1152, 1664), (2048, 512)])   # 1, 3, 5, 9, 13, 16 and 4 k-steps: chunks of 4, with and without a rest
+@pytest.mark.parametrize("rows", [(1, 16, 17, 0, 32), (33, 0, 65, 48)])
+def test_fp8_streaming_groups(dev, H, I, rows):
+    """moe_fp8_stream_kernel (dev knob 6 = 2) against the chunk-pipelined kernels (1), which test_fp_grouped_edges holds to the oracle: bit for bit."""
+    from helpers import fp8_block_quant
+    from ktransformers_amd import _native
+    E, k, T = len(rows), 1, sum(rows)
+    c = make_case(53, E, k, H, I, T)
+    c["ids"] = np.random.default_rng(T).permutation(np.repeat(np.arange(E), rows)).astype(np.int64)[:, None]
+    h = _native.MoEHandle(E, k, H, I, max_len=T, method="FP8", device=0, group_size=128)
+    try:
+        q = [fp8_block_quant(bf16_to_f32(c[n])) for n in ("gate", "up", "down")]
+        h.load_fp8(*[torch.from_numpy(x[0]).to(dev) for x in q], *[torch.from_numpy(x[1]).to(dev) for x in q])
+        _native.force_generic_path(True)
+        got = []
+        for knob in (1, 2):
+            _native.lib.ktx_debug_set(6, knob)
+            got.append(run(h, c, dev))
+        assert np.array_equal(*got), f"{int((got[0] != got[1]).sum())} outputs differ"
+    finally:
+        _native.lib.ktx_debug_set(6, 0)
+        _native.force_generic_path(False)
+        h.close()
+
+
 @pytest.mark.parametrize("method", ["AMXINT4", "AMXINT8"])
 @pytest.mark.parametrize("H,I", [(1152, 1664), (2048, 512)])   # 9 and 13 k-steps (chunks of 4 and 8, with a rest), 16 and 4; strip groups that are not full
 @pytest.mark.parametrize("rows", [(16, 17, 33, 49, 130), (1, 64, 65, 128)])   # each count of 16-row groups, alone and behind a full tile
