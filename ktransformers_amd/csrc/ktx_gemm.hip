@@ -30,6 +30,8 @@
 
 #include "../../include/ktx_gemm.h"
 
+extern "C" int ktx_debug_get(int idx);   // ktx_moe.hip (include/ktx_moe.h)
+
 namespace {
 
 typedef __bf16 gv8bf __attribute__((ext_vector_type(8)));
@@ -222,8 +224,11 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_nt_kernel(GemmParams p) {   
 //     4-7 (wm = 1, the second wavefront of every SIMD) run one barrier behind wavefronts 0-3: while one half of the workgroup
 //     multiplies, the other reads and issues — the matrix pipe of a SIMD always has exactly one owner;
 //   * LDS rows keep the 128-B row swizzle of the kernels above (applied on the DMA source side); epilogue through LDS as above.
+// NB: 16-column fragments of a wavefront.  4: 256 columns; 3: 192, whose B_b1 is half as long (16 columns of each wavefront, one request a wavefront; phases 1 and 2 of
+// 8 MFMAs): which of them, launch_gemm256 says.
+template <int NB>
 struct Gemm256 {
-  static constexpr int BM = 256, BN = 256, BK = 64, STAGE = 65536, HALF = 16384;
+  static constexpr int BM = 256, BN = NB * 64, WN = NB * 16, BK = 64, STAGE = 65536, HALF = 16384;
   __device__ static __forceinline__ int swz(int R) { return (R & 7) ^ ((R >> 3) & 1); }
 };
 
@@ -238,9 +243,10 @@ __device__ __forceinline__ void gemm_dma_off(const void* base, uint32_t off_lane
 
 // BTILES: B is a dense linear's weights in the decode layout of ktx_linear.hip (16-feature strips x k-steps of 128, p.ldb = k-steps): a
 // 16-byte piece of a row is a 16-byte piece of a tile, so only the DMA's source addresses differ.
-template <bool F32OUT, bool BTILES = false>
+template <bool F32OUT, bool BTILES, int NB>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm256_bf16_nt_kernel(GemmParams p) {
-  using C = Gemm256;
+  using C = Gemm256<NB>;
+  constexpr int NB1 = NB - 2;   // fragments (and requests) of B_b1
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2 stages][A_a0 | A_a1 | B_b0 | B_b1]
   int mt, nt;
   {
@@ -283,10 +289,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const int L = (wave * 2 + i) * 8 + (lane >> 3);
       const int piece = (lane & 7) ^ C::swz(L);
       const int grow = min(row0 + (L >> 6) * 128 + h * 64 + (L & 63), p.M - 1);
-      const int gcol = min(col0 + (L >> 5) * 64 + h * 32 + (L & 31), p.N - 1);
       offA[h][i] = (uint32_t)(((size_t)grow * p.lda) * 2 + piece * 16);
-      offB[h][i] = BTILES ? (uint32_t)(((size_t)(gcol >> 4) * p.ldb * 4 + (piece & 3)) * 1024 + ((piece >> 2) * 16 + (gcol & 15)) * 16)
-                          : (uint32_t)(((size_t)gcol * p.ldb) * 2 + piece * 16);
+      if (h == 1 && i >= NB1) continue;
+      const int Lb = h == 1 && NB1 == 1 ? wave * 8 + (lane >> 3) : L, cols = h == 1 ? NB1 * 16 : 32;   // (an LDS row's 16-byte pieces: as for L, 8 rows further or not)
+      const int pieceb = (lane & 7) ^ C::swz(Lb);
+      const int gcol = min(col0 + Lb / cols * C::WN + h * 32 + Lb % cols, p.N - 1);
+      offB[h][i] = BTILES ? (uint32_t)(((size_t)(gcol >> 4) * p.ldb * 4 + (pieceb & 3)) * 1024 + ((pieceb >> 2) * 16 + (gcol & 15)) * 16)
+                          : (uint32_t)(((size_t)gcol * p.ldb) * 2 + pieceb * 16);
     }
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(const __attribute__((address_space(3))) void*)smem) + wave * 2048;
   // half-tile slots of a stage: 0 = A_a0, 1 = A_a1, 2 = B_b0, 3 = B_b1
@@ -297,43 +306,48 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       gemm_dma_off(A + (size_t)kt * C::BK, offA[slot][1], dst + 1024);
     } else {
       const bf16_t* b = B + (BTILES ? (size_t)(kt >> 1) * 2048 + (kt & 1) * 256 : (size_t)kt * C::BK);
-      gemm_dma_off(b, offB[slot - 2][0], dst);
-      gemm_dma_off(b, offB[slot - 2][1], dst + 1024);
+      if (slot == 3 && NB1 == 1) {
+        gemm_dma_off(b, offB[1][0], dst - wave * 1024);
+      } else {
+        gemm_dma_off(b, offB[slot - 2][0], dst);
+        gemm_dma_off(b, offB[slot - 2][1], dst + 1024);
+      }
     }
   };
 
-  v4f acc[8][4];
+  v4f acc[8][NB];
 #pragma unroll
   for (int i = 0; i < 8; i++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NB; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
   const int r = lane & 15, kq = lane >> 4;
   const int g = C::swz(r);
   // fragment read offsets inside a stage: k-step s = pieces s*4 + kq
   const uint32_t so[2] = {(uint32_t)(((0 + kq) ^ g) * 16), (uint32_t)(((4 + kq) ^ g) * 16)};
-  const uint32_t a_off = (wm * 64 + r) * 128, b_off = 2 * C::HALF + (wn * 32 + r) * 128;
-  uint4 af[4][2], bf0[2][2], bf1[2][2];
+  const uint32_t a_off = (wm * 64 + r) * 128;
+  const uint32_t b_off[2] = {(uint32_t)(2 * C::HALF + (wn * 32 + r) * 128), (uint32_t)(3 * C::HALF + (wn * (NB1 * 16) + r) * 128)};
+  uint4 af[4][2], bf0[2][2], bf1[NB1][2];
   auto read_a = [&](const uint8_t* st, int part) {
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
       for (int s = 0; s < 2; s++) af[i][s] = *reinterpret_cast<const uint4*>(st + part * C::HALF + a_off + i * 2048 + so[s]);
   };
-  auto read_b = [&](const uint8_t* st, int part, uint4 (&bf)[2][2]) {
+  auto read_b = [&](const uint8_t* st, int part, auto& bf) {
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int j = 0; j < (int)(sizeof(bf) / sizeof(bf[0])); j++)
 #pragma unroll
-      for (int s = 0; s < 2; s++) bf[j][s] = *reinterpret_cast<const uint4*>(st + part * C::HALF + b_off + j * 2048 + so[s]);
+      for (int s = 0; s < 2; s++) bf[j][s] = *reinterpret_cast<const uint4*>(st + b_off[part] + j * 2048 + so[s]);
   };
-  auto mma = [&](int ah, int bh, const uint4 (&bf)[2][2]) {
+  auto mma = [&](int ah, int bh, const auto& bf) {
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int s = 0; s < 2; s++)
 #pragma unroll
       for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < (int)(sizeof(bf) / sizeof(bf[0])); j++)
           acc[ah * 4 + i][bh * 2 + j] =
               __builtin_amdgcn_mfma_f32_16x16x32_bf16(g_as_v8bf(af[i][s]), g_as_v8bf(bf[j][s]), acc[ah * 4 + i][bh * 2 + j], 0, 0, 0);
     __builtin_amdgcn_s_setprio(0);
@@ -349,7 +363,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int nk = p.K / C::BK;
   // prologue: k-tile 0 in deadline order, then the first counted wait
   issue(0, 0); issue(0, 2); issue(0, 3); issue(0, 1);
-  asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + NB1) : "memory");   // (B_b1 and A_a1 stay in flight)
   bar();
   if (wm == 1) bar();   // the second wavefront of every SIMD runs one segment behind the first
   for (int kt = 0; kt < nk; kt++) {
@@ -376,30 +390,32 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     mma(1, 1, bf1);
     bar();
     // phase 3: (a1, b0) — operands already in registers
-    if (more) { issue(kt + 1, 1); asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); }
+    if (more) { issue(kt + 1, 1); asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + NB1) : "memory"); }
     bar();
     mma(1, 0, bf0);
     bar();
   }
   if (wm == 0) bar();   // pair the extra barrier of the lagging half
 
-  // ---- epilogue: 16 rows x 64 columns per pass through this wavefront's 8 KiB of LDS (every wavefront is past the last barrier)
+  // ---- epilogue: 16 rows x WN columns per pass through this wavefront's 8 KiB of LDS (every wavefront is past the last barrier)
   constexpr int ES = F32OUT ? 4 : 2;
-  constexpr int RS = 64 * ES + 16;
-  constexpr int PPR = 64 * ES / 16;
-  constexpr int PPL = 16 * PPR / 64;
+  constexpr int RS = C::WN * ES + 16;
+  constexpr int PPR = C::WN * ES / 16;
+  constexpr int PPL = (16 * PPR + 63) / 64;
   constexpr int EPP = 16 / ES;
   uint8_t* ep = smem + wave * 8192;
-  float bv[4] = {0.f, 0.f, 0.f, 0.f};
+  float bv[NB];
+#pragma unroll
+  for (int j = 0; j < NB; j++) bv[j] = 0.f;
   if (p.bias) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) bv[j] = bf16_to_f32(p.bias[min(col0 + wn * 64 + j * 16 + r, p.N - 1)]);
+    for (int j = 0; j < NB; j++) bv[j] = bf16_to_f32(p.bias[min(col0 + wn * C::WN + j * 16 + r, p.N - 1)]);
   }
   uint8_t* Yb = reinterpret_cast<uint8_t*>(p.Y) + (size_t)bz * p.y_bs * ES;
 #pragma unroll
   for (int i = 0; i < 8; i++) {
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < NB; j++)
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         const float v = acc[i][j][q] + bv[j];
@@ -411,21 +427,22 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int u = 0; u < PPL; u++) {
       const int idx = u * 64 + lane;
+      if ((16 * PPR) % 64 != 0 && idx >= 16 * PPR) break;
       const int row = idx / PPR, pc = idx % PPR;
       const uint4 v = *reinterpret_cast<const uint4*>(ep + row * RS + pc * 16);
-      const int grow = row0 + wm * 128 + i * 16 + row, gcol = col0 + wn * 64 + pc * EPP;
+      const int grow = row0 + wm * 128 + i * 16 + row, gcol = col0 + wn * C::WN + pc * EPP;
       if (grow < p.M && gcol < p.N) *reinterpret_cast<uint4*>(Yb + ((size_t)grow * p.ldy + gcol) * ES) = v;
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
 }
 
-template <bool F32OUT, bool BTILES = false>
-int launch_gemm256(GemmParams p, int batch, hipStream_t st) {
-  auto kern = gemm256_bf16_nt_kernel<F32OUT, BTILES>;
-  constexpr int lds = 2 * Gemm256::STAGE;
+template <bool F32OUT, bool BTILES, int NB>
+int launch_gemm256_nb(GemmParams p, int batch, hipStream_t st) {
+  auto kern = gemm256_bf16_nt_kernel<F32OUT, BTILES, NB>;
+  constexpr int lds = 2 * Gemm256<NB>::STAGE;
   p.tm = (p.M + 255) / 256;
-  p.tn = (p.N + 255) / 256;
+  p.tn = (p.N + Gemm256<NB>::BN - 1) / Gemm256<NB>::BN;
   p.xcd_map = (p.tm >= 12 && p.tn >= 8) ? 2 : p.tn >= 8 ? 1 : 0;
   long nblk = p.xcd_map ? (long)p.tm * ((p.tn + 7) / 8 * 8) : (long)p.tm * p.tn;
   if (p.xcd_map == 2) {
@@ -438,6 +455,17 @@ int launch_gemm256(GemmParams p, int batch, hipStream_t st) {
   KTX_HIP(hipGetLastError());
   return 0;
 }
+
+// 192 columns where the CUs take no more rounds of them, one workgroup each, than of 256 (bf16 weights, us, 256 | 192 columns): 1536 -> 24576, 500 rows (1 round) 45.9 |
+// 43.5, 1000 (2) 85.5 | 84.8, 2000 (3 | 4) 128 | 150; 2048 -> 3072, 2048 (1) 48.5 | 44.4; 4096 -> 12000, 700 (1) 113 | 109, 1300 (2) 175 | 168; 1280 -> 9000, 2000 (2) 65.8 | 62.3; 7168 -> 4096, 1000 (64 | 88 tiles a piece of K) 68 | 98.  A k-tile's barriers and reads cost the same for both, so a round of 192 takes 0.95 of one of 256, not 0.75.
+template <bool F32OUT, bool BTILES = false>
+int launch_gemm256(const GemmParams& p, int batch, hipStream_t st) {
+  const long tm = (p.M + 255) / 256 * (long)batch, r4 = (tm * ((p.N + 255) / 256) + 255) / 256, r3 = (tm * ((p.N + 191) / 192) + 255) / 256;
+  const int force = ktx_debug_get(7);   // dev knob 7 (tests): 3 or 4 fragments
+  if (force ? force == 3 : r3 <= r4) return launch_gemm256_nb<F32OUT, BTILES, 3>(p, batch, st);
+  return launch_gemm256_nb<F32OUT, BTILES, 4>(p, batch, st);
+}
+
 
 // fp32 -> three bf16 planes by truncation: w == hi + mid + lo exactly (finite w; 24 mantissa bits = 8 + 8 + 8)
 __global__ __launch_bounds__(256) void split_f32_bf16x3_kernel(const float* __restrict__ w, long n, bf16_t* __restrict__ planes) {

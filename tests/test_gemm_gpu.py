@@ -71,6 +71,43 @@ def test_ping_pong_tile_race_screen(M, N, K):
     assert torch.equal(gemm_bf16_nt(a, b), y_ref)                        # whatever the automatic choice is
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (256, 192, 128), (257, 200, 192), (1000, 1160, 1536), (2048, 6152, 4096)])
+def test_ping_pong_tile_of_192_columns(M, N, K):
+    """Variant 5 with 192 and with 256 columns a workgroup (dev knob 7 = 3 and 4), repeated, with bias and with fp32 output: the bits of variant 2 (the same k order)."""
+    from ktransformers_amd import _native
+    from ktransformers_amd._native import gemm_bf16_nt
+    g = torch.Generator(device="cpu").manual_seed(M + N + K)
+    a = torch.randn((M, K), generator=g).to(torch.bfloat16).to(DEV)
+    b = (torch.randn((N, K), generator=g) * K ** -0.5).to(torch.bfloat16).to(DEV)
+    bias = torch.randn(N, generator=g).to(torch.bfloat16).to(DEV)
+    ref = [gemm_bf16_nt(a, b, variant=2), gemm_bf16_nt(a, b, bias=bias, variant=2), gemm_bf16_nt(a, b, out_f32=True, variant=2)]
+    try:
+        for knob in (3, 4, 3, 3):
+            _native.lib.ktx_debug_set(7, knob)
+            got = [gemm_bf16_nt(a, b, variant=5), gemm_bf16_nt(a, b, bias=bias, variant=5), gemm_bf16_nt(a, b, out_f32=True, variant=5)]
+            assert all(torch.equal(x, y) for x, y in zip(got, ref)), knob
+    finally:
+        _native.lib.ktx_debug_set(7, 0)
+
+
+@pytest.mark.parametrize("T,K,N", [(300, 1536, 24576), (700, 4096, 12000)])
+def test_linear_tiles_of_192_columns(T, K, N):
+    """The same on a bf16 linear's own weights (its tiles are the B operand)."""
+    from ktransformers_amd import _native
+    g = torch.Generator(device="cpu").manual_seed(T + N)
+    h = _native.LinearHandle(K, N, "BF16", 0, T, torch.device(DEV))
+    h.load_bf16((torch.randn((N, K), generator=g) * K ** -0.5).to(torch.bfloat16).to(DEV))
+    x = torch.randn((T, K), generator=g).to(torch.bfloat16).to(DEV)
+    got = []
+    try:
+        for knob in (4, 3):
+            _native.lib.ktx_debug_set(7, knob)
+            got.append(h.forward(x).clone())
+    finally:
+        _native.lib.ktx_debug_set(7, 0)
+    assert torch.equal(*got)
+
+
 def test_bias_strided_rows_and_fp32_output():
     from ktransformers_amd._native import gemm_bf16_nt
     g = torch.Generator(device="cpu").manual_seed(9)
