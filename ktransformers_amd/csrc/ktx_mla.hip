@@ -1148,15 +1148,16 @@ struct MlaPrefillParams {
   int nqb;                       // > 0: 1-D XCD-aware grid of nqb query blocks x H heads (H % 8 == 0); 0: grid (query blocks, heads)
 };
 
-// S of the NEXT tile is computed beside the softmax of this one: 48 MFMAs and ~200 vector instructions that do not wait for each other, in one stream (before,
+// S of the NEXT tile is computed beside the probabilities of this one, and its largest scores are found beside this tile's O: MFMAs and vector instructions that
+// do not wait for each other, in one stream (before,
 // 1280 cycles of MFMAs and ~1450 of vector ALU a tile ran one after the other, and two workgroups a CU hid a third of that).  That takes a second set of scores, 32
 // registers, which the tiles' way through registers left no room for: K, k_pe and V^T come by LDS-DMA, double-buffered, 80 KB a workgroup, two workgroups a CU.
 // A lane's 8 probabilities of a half tile are those of 8 keys that follow each other (which K rows a fragment takes is free), so a V^T fragment is one read.
 // Rows lie unpadded, their 16-byte pieces permuted so that no read has bank conflicts (ds_read_b128 takes lanes 0-3, 12-15, 20-23 and 24-27 together): with i the lane
 // that reads the row, K: piece c in slot c ^ i; k_pe and V^T, 8 pieces a row: c ^ (i >> 1).
-// 128 heads, us, one after the other -> here: 1000 tokens behind 3096 367 -> 317 (788 -> 930 TFLOP/s), 2048 of 8192 1332 -> 1126, 2048 of 2048 260 -> 226, 512 of 512 32 -> 29; 16
-// heads, 300 of 1500: 50 -> 41.  Matrix pipe 44 % busy, vector ALU 42 %, LDS 17 % (58 % with two b64 reads a V^T fragment and padded rows); the clock is 2.0 GHz.  Left to
-// its own order the compiler puts the products first, each fragment's read directly before its use, and the softmax behind them: 325 us.
+// 128 heads, us, one after the other -> here: 1000 tokens behind 3096 367 -> 310 (788 -> 950 TFLOP/s), 2048 of 2048 260 -> 214, 512 of 8192 396 -> 336; 16 heads, 300 of 1500: 50
+// -> 38.  Left to its own order the compiler puts the products first, each fragment's read directly before its use, and the softmax behind them: 325 us; with the
+// largest scores found beside the products as well, 320.  A running maximum moves somewhere in two fifths of the tiles: one branch for both query tiles costs 8 %.
 // DMA false: operands that do not lie on 16 bytes come through registers, into the same places.
 template <bool DMA>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void mla_prefill_kernel(MlaPrefillParams p) {
@@ -1254,7 +1255,39 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   };
 
-  // One key tile of parity par: its scores are in st; MORE: the next tile's go to nx.
+  // The causal mask only exists on a query block's last two key tiles: a tile every query of the wavefront sees whole (wave-uniform test) skips it.
+  // (the empty asm keeps this a wave-uniform BRANCH: speculated into selects, its compares + selects ran on every tile)
+  auto mask = [&](int tile, v4f (&st)[NU][4]) __attribute__((always_inline)) {
+    const int j0 = tile * PF_BN;
+    if (j0 + PF_BN - 1 <= min(pos_off + min(q0, p.T - 1), p.kv_len - 1)) return;
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      const int lim = min(pos_off + tq[u], p.kv_len - 1);       // last visible key of this lane's query
+#pragma unroll
+      for (int kt = 0; kt < 4; kt++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int key = j0 + (kt >> 1) * 32 + g * 8 + (kt & 1) * 4 + r;
+          st[u][kt][r] = key <= lim ? st[u][kt][r] : -__builtin_inff();
+        }
+        asm volatile("" : "+v"(st[u][kt]));
+      }
+    }
+  };
+  float mx[NU];   // the largest score of a tile, over the query's four key-chunk lanes (qi, qi + 16, + 32, + 48)
+  auto largest = [&](const v4f (&st)[NU][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      mx[u] = -__builtin_inff();
+#pragma unroll
+      for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) mx[u] = fmaxf(mx[u], st[u][kt][r]);
+      mx[u] = pf_max_rows(mx[u]);
+    }
+  };
+
+  // One key tile of parity par: its scores are in st, the largest in mx; MORE: the next tile's go to nx.
   const float cexp = p.sm_scale * 1.44269504088896340736f;
   auto step = [&](auto more, int par, int tile, v4f (&st)[NU][4], v4f (&nx)[NU][4]) __attribute__((always_inline)) {
     constexpr bool MORE = decltype(more)::value;
@@ -1262,40 +1295,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (tile + 2 < ntiles) stage_k(tile + 2, par);
       stage_v(tile + 1, par ^ 1);
     }
-    const int j0 = tile * PF_BN;
-    // The causal mask only exists on a query block's last two key tiles: a tile every query of the wavefront sees whole (wave-uniform test) skips it.
-    // (the empty asm keeps this a wave-uniform BRANCH: speculated into selects, its compares + selects ran on every tile)
-    if (!(j0 + PF_BN - 1 <= min(pos_off + min(q0, p.T - 1), p.kv_len - 1))) {
+    // ---- online softmax, per query (lane & 15): where some lane's running maximum moved, O and the sums are scaled to the new one.  It is kept on the RAW scores;
+    // the softmax scale rides in the exponent's multiply: p = exp2(s * c - m * c), c = sm_scale * log2(e).  A lane sums its own keys; the query's four meet at the end.
 #pragma unroll
-      for (int u = 0; u < NU; u++) {
-        const int lim = min(pos_off + tq[u], p.kv_len - 1);       // last visible key of this lane's query
+    for (int u = 0; u < NU; u++)
+      if (!__all(mx[u] <= m_run[u])) {
+        const float m_new = fmaxf(m_run[u], mx[u]);             // finite from tile 0 on: key 0 is visible to every query
+        const float alpha = __builtin_amdgcn_exp2f((m_run[u] - m_new) * cexp);
+        m_run[u] = m_new;
+        l_run[u] *= alpha;
 #pragma unroll
-        for (int kt = 0; kt < 4; kt++) {
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const int key = j0 + (kt >> 1) * 32 + g * 8 + (kt & 1) * 4 + r;
-            st[u][kt][r] = key <= lim ? st[u][kt][r] : -__builtin_inff();
-          }
-          asm volatile("" : "+v"(st[u][kt]));
-        }
+        for (int i = 0; i < 8; i++) o[u][i] *= alpha;
       }
-    }
-    // ---- online softmax, per query (lane & 15; the 4 key-chunk lanes g of a query agree after the two exchanges), beside the next tile's products.
-    // The running maximum is kept on the RAW scores and the softmax scale rides in the exponent's multiply: p = exp2(s * c - m * c), c = sm_scale * log2(e).
+    // ---- the probabilities, beside the next tile's scores
     if constexpr (MORE) qk(par ^ 1, nx);
     uint4 pb[NU][2];
-    float alpha[NU];
 #pragma unroll
     for (int u = 0; u < NU; u++) {
-      float mx = -__builtin_inff();
-#pragma unroll
-      for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) mx = fmaxf(mx, st[u][kt][r]);
-      mx = pf_max_rows(mx);                                     // over the query's four key-chunk lanes (qi, qi + 16, + 32, + 48)
-      const float m_new = fmaxf(m_run[u], mx);                  // finite from tile 0 on: key 0 is visible to every query
-      alpha[u] = __builtin_amdgcn_exp2f((m_run[u] - m_new) * cexp);
-      const float mc = -m_new * cexp;
+      const float mc = -m_run[u] * cexp;
       float sum2[2] = {0.f, 0.f};
       float pv[4][4];
 #pragma unroll
@@ -1305,8 +1322,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           pv[kt][r] = __builtin_amdgcn_exp2f(fmaf(st[u][kt][r], cexp, mc));
           sum2[r & 1] += pv[kt][r];
         }
-      l_run[u] = l_run[u] * alpha[u] + pf_sum_rows(sum2[0] + sum2[1]);
-      m_run[u] = m_new;
+      l_run[u] += sum2[0] + sum2[1];
 #pragma unroll
       for (int ks = 0; ks < 2; ks++)
         pb[u][ks] = make_uint4(ktx_pk_bf16(pv[2 * ks][0], pv[2 * ks][1]), ktx_pk_bf16(pv[2 * ks][2], pv[2 * ks][3]),
@@ -1321,14 +1337,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         __builtin_amdgcn_sched_group_barrier(0x402, 6, 0);
       }
     }
-    // the multiplies of `o *= alpha` are skipped whenever no lane's running maximum moved (alpha == 1 exactly: the common case once the first tiles are past)
+    if constexpr (MORE) {
+      // (here, or the compiler moves them behind the mask's branch, away from the products)
 #pragma unroll
-    for (int u = 0; u < NU; u++)
-      if (!__all(alpha[u] == 1.0f)) {
+      for (int u = 0; u < NU; u++) {
+        asm volatile("" : "+v"(l_run[u]));
 #pragma unroll
-        for (int i = 0; i < 8; i++) o[u][i] *= alpha[u];
+        for (int ks = 0; ks < 2; ks++) asm volatile("" : "+v"(pb[u][ks].x), "+v"(pb[u][ks].y), "+v"(pb[u][ks].z), "+v"(pb[u][ks].w));
       }
-    // ---- O^T += V^T P^T: o[u][i][r] = O[query qi][dim 16*i + 4*g + r] ----------------------------------------------------
+      mask(tile + 1, nx);
+    }
+    // ---- O^T += V^T P^T: o[u][i][r] = O[query qi][dim 16*i + 4*g + r], beside the next tile's largest scores
     const uint8_t* vb = smem + par * PF_VB;
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) {                  // (key half outermost: 8 x NU independent accumulators)
@@ -1339,6 +1358,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int u = 0; u < NU; u++) o[u][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, as_v8bf(pb[u][ks]), o[u][i], 0, 0, 0);
       }
     }
+    if constexpr (MORE) largest(nx);
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 1);
 #pragma unroll
     for (int f = 0; f < 16; f++) {
@@ -1353,6 +1373,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   v4f sa[NU][4], sb[NU][4];
   qk(0, sa);
   __syncthreads();   // (the first step's requests overwrite what this read)
+  mask(0, sa);
+  largest(sa);
   int tile = 0;
   for (; tile + 2 < ntiles; tile += 2) {
     step(std::true_type{}, 0, tile, sa, sb);
@@ -1369,8 +1391,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
   for (int u = 0; u < NU; u++) {
     const int t = q0 + u * 16 + qi;
+    const float l = pf_sum_rows(l_run[u]);
     if (t < p.T) {
-      const float inv = l_run[u] > 0.f ? 1.0f / l_run[u] : 0.f;
+      const float inv = l > 0.f ? 1.0f / l : 0.f;
       bf16_t* op = p.out + ((size_t)t * p.H + h) * 128 + g * 4;
 #pragma unroll
       for (int i = 0; i < 8; i++)
