@@ -2961,7 +2961,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   {
     ProfScope ps(0, st);
     KTX_HIP(moe_launch_prep(pp, false, st));
-    hipLaunchKernelGGL(q8k_quant_kernel<false>, dim3(qlen), dim3(256), 0, st, d_input, H, ws->x_q, ws->x_d, ws->x_bs, x_bsp, x_b256, d_bsz, 1, qlen,
+    hipLaunchKernelGGL(q8k_quant_kernel<false>, q8k_grid(qlen, H), dim3(256), 0, st, d_input, H, ws->x_q, ws->x_d, ws->x_bs, x_bsp, x_b256, d_bsz, 1, qlen,
                        gg_unit_codes(h->gg_type[0]));
   }
   KTX_HIP(hipGetLastError());
@@ -2977,7 +2977,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   if (rc) return rc;
   {
     ProfScope ps(2, st);
-    hipLaunchKernelGGL(q8k_quant_kernel<true>, dim3(npairs), dim3(256), 0, st, (const void*)ws->a_buf, I, ws->a_q, ws->a_d, ws->a_bs,
+    hipLaunchKernelGGL(q8k_quant_kernel<true>, q8k_grid(npairs, I), dim3(256), 0, st, (const void*)ws->a_buf, I, ws->a_q, ws->a_d, ws->a_bs,
                        a_bsp, a_b256, ws->counters, 0, npairs, gg_unit_codes(h->gg_type[2]));
   }
   KTX_HIP(hipGetLastError());

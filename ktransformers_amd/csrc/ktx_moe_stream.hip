@@ -9,8 +9,8 @@
 
 // =====================================================================================================
 // Grouped GEMM of AMXINT4 / AMXINT8 prompts on tiles of 64 rows.  What bounds it is the memory's way in while experts have few rows (256 of 7168 x 2048, gate|up
-// of 31 rows each: 5.2 TB/s) and, with more, the power that MFMAs beside that stream draw: the clock falls to 1.65 GHz of 2.4 as the cycles go down.  So it does
-// no work that no row needs and keeps both units fed:
+// of 31 rows each: 5.2 TB/s) and, with more, the power that MFMAs beside that stream draw: the clock falls as the cycles go down (64 rows each: 1.73 M cycles at 1.87 GHz, with 4
+// wavefronts 1.54 M at 1.65).  So it does no work that no row needs and keeps both units fed:
 //   * a tile multiplies the 16-row groups that hold rows, by an instantiation for each count (a quarter of a 64-row tile is absent at 64 rows an expert);
 //   * each wavefront owns four 16-row weight strips (gate|up: two strips of both; down: four), so a fragment of activations feeds 4 MFMAs; weights stream
 //     through a ring of registers, 4 k-steps deep.  That is 128 KB a CU, as much as its share of the L2 holds; 8 deep is slower (31 rows an expert: 1151 us against 1131);
