@@ -840,6 +840,29 @@ def test_w4_prompts_off_the_gemm_multiply_exact_integers(G, K, N, T, how):
     assert float((y.double() - want).norm() / want.norm()) < 2.0e-3
 
 
+@pytest.mark.parametrize("fmt,group", [("W4", 64), ("W4", 128), ("FP8", 128)])
+@pytest.mark.parametrize("K,N,T", [(4096, 12000, 33), (4096, 10244, 64), (16384, 5130, 48)])   # 188, 164 and 168 workgroups; whole strips, a part of one, rows absent
+def test_tiles_of_64_rows_and_256_features(fmt, group, K, N, T):
+    """The 64 x 256 tiles against the 64 x 128 ones (dev knob 7 = 6): the same pieces of K, the same bits."""
+    from ktransformers_amd import _native
+    g = torch.Generator().manual_seed(K + N + T)
+    dev = torch.device("cuda", 0)
+    h = _native.LinearHandle(K, N, fmt, group, T, dev)
+    if fmt == "FP8":
+        h.load_fp8((torch.randn((N, K), generator=g) * 100).clamp_(-448, 448).to(torch.float8_e4m3fn).to(dev), torch.rand((-(-N // 128), K // 128), generator=g).to(dev))
+    else:
+        h.load_bf16((torch.randn((N, K), generator=g) * K ** -0.5).to(torch.bfloat16).to(dev))
+    x = torch.randn((T, K), generator=g).to(torch.bfloat16).to(dev)
+    got = []
+    try:
+        for knob in (6, 0):
+            _native.lib.ktx_debug_set(7, knob)
+            got.append(h.forward(x).clone())
+    finally:
+        _native.lib.ktx_debug_set(7, 0)
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("N", [24576, 24584])
 def test_bf16_prompts_on_the_gemm_of_decode_tiles(N):
     """520 rows of 2048 -> 24576 (whole strips) and 24584 (half a strip at the end) fill the chip with 256 x 256 tiles over the whole K: the GEMM
