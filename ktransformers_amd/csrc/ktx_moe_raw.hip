@@ -276,6 +276,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       quarter(std::integral_constant<int, 2>{}, st, w);
       quarter(std::integral_constant<int, 3>{}, st, w);
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no request may outlive the workgroup's LDS
 
     if (!wave_ok) return;
     constexpr float unlift = raw_unlift(SCALED);
