@@ -1643,17 +1643,15 @@ __global__ void pack_rawint4_kernel(const uint8_t* __restrict__ src, int N, int 
   out[idx] = v;
 }
 
-// bf16 scales [N][K/32] -> tile order [rg][step][row j][h][8 blocks]; one thread per element.  *outside: set if one is outside raw_scale_fits
-__global__ void pack_rawint4_scales_kernel(const bf16_t* __restrict__ src, int N, int K, bf16_t* __restrict__ out, int* outside) {
+// bf16 scales [N][K/32] -> tile order [rg][step][row j][h][8 blocks]; one thread per element
+__global__ void pack_rawint4_scales_kernel(const bf16_t* __restrict__ src, int N, int K, bf16_t* __restrict__ out) {
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int G = K / 32, NS = K / 512;
   if (idx >= (size_t)N * G) return;
   const int kb8 = (int)(idx % 8), h = (int)((idx / 8) % 2), jrow = (int)((idx / 16) % 4);
   const size_t t = idx / 64;
   const int st = (int)(t % NS), rg = (int)(t / NS);
-  const bf16_t s = src[(size_t)(rg * 4 + jrow) * G + 2 * (8 * st + kb8) + h];
-  out[idx] = s;
-  if (!raw_scale_fits(s)) atomicOr(outside, 1);
+  out[idx] = src[(size_t)(rg * 4 + jrow) * G + 2 * (8 * st + kb8) + h];
 }
 
 #include "ktx_moe_gguf.inc"
@@ -1721,7 +1719,6 @@ struct ktx_moe_s {
   int gg_type[3] = {0, 0, 0};     // GGUF: ggml type of gate / up / down
   size_t gg_stride[3] = {0, 0, 0};
   bool loaded_gguf = false;
-  int* raw_outside = nullptr;     // RAWINT4, [expert]: not 0 where a weight scale does not fit the prompt kernel's operands (raw_scale_fits)
   bool exact = false;             // ktx_moe_set_exact: no path of this handle may re-associate the reference's fp32 sums
 };
 
@@ -1830,7 +1827,7 @@ extern "C" int ktx_moe_create(const ktx_moe_config* cfg, ktx_moe_t* out) {
 extern "C" int ktx_moe_destroy(ktx_moe_t h) {
   if (!h) return 0;
   DeviceGuard _dg(h->cfg.device);
-  void* ptrs[] = {h->gate_w, h->up_w, h->down_w, h->gate_s, h->up_s, h->down_s, h->gate_r, h->up_r, h->down_r, h->mask, h->raw_outside};
+  void* ptrs[] = {h->gate_w, h->up_w, h->down_w, h->gate_s, h->up_s, h->down_s, h->gate_r, h->up_r, h->down_r, h->mask};
   for (void* p : ptrs)
     if (p) hipFree(p);
   delete h;
@@ -2037,8 +2034,6 @@ extern "C" int ktx_moe_load_rawint4(ktx_moe_t h, const void* d_gate, const void*
   KTX_ON_DEVICE(h->cfg.device);
   const int E = h->cfg.expert_num, H = h->cfg.hidden_size, I = h->cfg.intermediate_size;
   const size_t dwords = (size_t)I * H / 8, nsc = (size_t)I * (H / 32);
-  if (!h->raw_outside) KTX_HIP(hipMalloc(&h->raw_outside, E * sizeof(int)));
-  KTX_HIP(hipMemset(h->raw_outside, 0, E * sizeof(int)));
   for (int e = 0; e < E; e++) {
     const uint8_t* src[3] = {(const uint8_t*)d_gate + (size_t)e * I * H / 2, (const uint8_t*)d_up + (size_t)e * I * H / 2,
                              (const uint8_t*)d_down + (size_t)e * H * I / 2};
@@ -2051,7 +2046,7 @@ extern "C" int ktx_moe_load_rawint4(ktx_moe_t h, const void* d_gate, const void*
       hipLaunchKernelGGL(pack_rawint4_kernel, dim3((unsigned)((dwords + 255) / 256)), dim3(256), 0, 0, src[m], Ns[m], Ks[m],
                          reinterpret_cast<uint32_t*>(dst[m]));
       hipLaunchKernelGGL(pack_rawint4_scales_kernel, dim3((unsigned)((nsc + 255) / 256)), dim3(256), 0, 0, ssrc[m], Ns[m],
-                         Ks[m], sdst[m], h->raw_outside + e);
+                         Ks[m], sdst[m]);
     }
   }
   KTX_HIP(hipGetLastError());
@@ -2666,7 +2661,7 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   RawGemmParams g1;
   g1.w0 = h->gate_w; g1.w1 = h->up_w; g1.s0 = (const bf16_t*)h->gate_s; g1.s1 = (const bf16_t*)h->up_s;
   g1.expert_stride = h->gu_stride; g1.scale_stride = nsc_gu; g1.N = I; g1.K = H; g1.act_q = ws->x_q; g1.act_d = ws->x_d;
-  g1.row_src = ws->src_of_row; g1.tiles = ws->tiles; g1.counters = ws->counters; g1.out = ws->a_buf; g1.outside = h->raw_outside;
+  g1.row_src = ws->src_of_row; g1.tiles = ws->tiles; g1.counters = ws->counters; g1.out = ws->a_buf;
   int rc;
   {
     ProfScope ps(1, st);
@@ -2682,7 +2677,7 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   RawGemmParams g2;
   g2.w0 = h->down_w; g2.w1 = nullptr; g2.s0 = (const bf16_t*)h->down_s; g2.s1 = nullptr; g2.expert_stride = h->dn_stride;
   g2.scale_stride = nsc_dn; g2.N = H; g2.K = I; g2.act_q = ws->a_q; g2.act_d = ws->a_d; g2.row_src = nullptr;
-  g2.tiles = ws->tiles; g2.counters = ws->counters; g2.out = ws->dn_buf; g2.outside = h->raw_outside;
+  g2.tiles = ws->tiles; g2.counters = ws->counters; g2.out = ws->dn_buf;
   {
     ProfScope ps(3, st);
     rc = chunk ? moe_launch_rawint4_chunk(false, g2, std::min(npairs, E) + npairs / RAW_ROWS, st) : launch_rawint4<false>(g2, max_tiles, st);

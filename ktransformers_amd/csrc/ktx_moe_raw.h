@@ -23,31 +23,22 @@ struct Tile {
 
 struct RawGemmParams {
   const uint8_t *w0, *w1;      // RAW tiles (gate | down, up)
-  const bf16_t *s0, *s1;       // bf16 scales in the tile order above
+  const bf16_t *s0, *s1;       // bf16 scales, [row group][step][row][half][8 blocks] (pack_rawint4_scales_kernel)
   size_t expert_stride;        // bytes of weights per expert matrix
   size_t scale_stride;         // bf16 elements of scales per expert matrix
   int N, K;
-  const int8_t* act_q;         // [src rows][K]
+  const int8_t* act_q;         // [src rows][K] int8 codes, or f16 ones (prompts: 2 K bytes a row)
   const float* act_d;          // [src rows][K/32]
   const int32_t* row_src;
-  const Tile* tiles;           // <= 4 rows per tile
+  const Tile* tiles;           // rows per tile: 4, of a prompt RAW_ROWS
   const int32_t* counters;
   bf16_t* out;                 // [sorted rows][N]
-  const int* outside;          // [expert]: not 0 if a scale of its matrices is outside raw_scale_fits
 };
 
 typedef _Float16 raw_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 raw_h8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ uint32_t raw_h2_bits(raw_h2 v) { return __builtin_bit_cast(uint32_t, v); }
 
-// What a widened nibble's operand carries: RAW_LIFT (8) times (q - 8) times the group's scale times 2^RAW_LIFT_S; the epilogue takes both back.
-constexpr int RAW_LIFT = 8, RAW_LIFT_S = 6;
-// A scale (bf16) whose operands are exact f16: 0 or magnitudes of 2^-23 .. 4.  2^6 s keeps its 8 significant bits down to f16's last one, 2^-24; 192 * 2^6 s stays
-// below 65504; 8 q 2^6 s is a normal f16.
-__host__ __device__ inline bool raw_scale_fits(bf16_t s) {
-  const unsigned m = s & 0x7fffu;
-  return m == 0 || (m >= (127u - 23u) << 7 && m < (127u + 2u) << 7);
-}
 constexpr int RAW_ROWS = 64;   // rows of a prompt tile
 // One grouped GEMM of a RAWINT4 prompt on tiles of RAW_ROWS rows.
 int moe_launch_rawint4_chunk(bool gate_up, const RawGemmParams& p, int max_tiles, hipStream_t st);

@@ -15,12 +15,11 @@
 // (tests/test_moe_gpu.py::test_rawint4_prompt_chunks).  Decode and short batches (qlen < 64) keep the exact kernels; dev knob 29 = 1
 // forces them for every size.
 //
-// The vector ALU bounds it (busy 70 % of the time at 2048 tokens of Kimi-K2's sizes, 12 instructions an MFMA, the matrix pipe 22 %, rocprofv3 counters), so the
-// operands are what costs it least.  Codes are f16 integers.  A weight's operand is its nibble times its group's scale, which f16 holds exactly
-// (4 and 8 significant bits): the MFMA's sum over a group has at most 23 significant bits, is exact in fp32, and a fragment takes one fma an output (with
-// the activation's scale) where the product of both scales took a multiplication as well.  The term is rounded once, in that fma; before, the product of
-// the scales was, too.  Widening costs 16 instructions per 8 weights of a lane, for all of its row groups.  Scales that f16 does not hold (raw_scale_fits;
-// an expert has one, or it has none) stay outside the operands, in fp32, with the multiplication.
+// The vector ALU bounds it, so the operands are what costs it least: codes and nibbles as f16 integers, whose sum over a group the f16 MFMA gives exactly and in
+// fp32 already (below 2^15), so that a fragment and group takes a scale product and an fma an output, where an int8 MFMA takes a conversion as well: the
+// terms are the reference's, with any scale.
+// (The weight's scale inside the f16 operand is exact for magnitudes of 2^-23 .. 4 and saves the scale products, but the terms are then rounded once where the
+// reference's are twice, the sums reach only 2^119, and experts with another scale need a path of their own.)
 //
 // No second copy of the weights: the RAW tiles are read as they lie in HBM.  MFMA lane (i = lane & 15, kc = lane >> 4) needs
 // row i's eight nibbles k = 64 kb + 32 h + 8 kc + [0, 8) of group (kb, h): those are the pieces (L, j) = (8h + 2kc + o, i & 3),
@@ -30,16 +29,17 @@
 //   multiplies while the other waits: 8 wavefronts on 128 rows are 2 to 20 % slower, though no expert of 65 .. 128 rows is widened twice).  K walks in the RAW
 //   step of 512: its weights go through the LDS into registers (the LDS holds the next step's meanwhile: two steps in registers leave none for
 //   the sums of two rounds), the activations in quarters of it, all by LDS-DMA.
-// At Kimi-K2's sizes, us for the whole forward, scales multiplied behind the MFMAs and weights of two steps in registers -> here: 500 tokens
-// 2015 -> 1905, 2048 4280 -> 3850; 64 experts of 2048 x 1024, top-8: 360 tokens 168 -> 149, 2048 537 -> 474.
+// At Kimi-K2's sizes, us for the whole forward, weights of two steps in registers and each round's sums directly behind its MFMAs -> here (the same bits): 64 tokens 956 ->
+// 931, 500 1988 -> 1968, 2048 4153 -> 4091; 64 experts of 2048 x 1024, top-8: 200 tokens 137 -> 128, 360 169 -> 160, 2048 543 -> 514.
 // =====================================================================================================
-__host__ __device__ constexpr float raw_unlift(bool scaled) { return 1.0f / (float)(scaled ? RAW_LIFT << RAW_LIFT_S : RAW_LIFT); }
-// the pairs (byte 0, byte 2) and (byte 1, byte 3) of the low (par 0) or high nibbles of x, as RAW_LIFT * q * s; x: two's complement nibbles.
-// A nibble (its top bit turned: q + 8) becomes bits 6..9 of an f16 of exponent 2^7: 128 + 8 (q + 8).  s (an f16 with 8 significant bits) times that, less
-// 192 s (= 3 * 64 s: exact), is 8 q s with 11 significant bits at most: exact as well.
+// the pairs (byte 0, byte 2) and (byte 1, byte 3) of the low (par 0) or high nibbles of x as q; x: two's complement nibbles.
+// A nibble (its top bit turned: q + 8) becomes bits 6..9 of an f16 of exponent 2^7: 128 + 8 (q + 8), an eighth of which less 24 is q.
 template <int PAR>
-__device__ __forceinline__ void raw_widen(uint32_t x, uint32_t mask, uint32_t top, raw_h2 s, raw_h2 c, uint32_t& o0, uint32_t& o1) {
-  auto value = [&](uint32_t e) { return raw_h2_bits(__builtin_elementwise_fma(__builtin_bit_cast(raw_h2, (e & mask) ^ top), s, c)); };
+__device__ __forceinline__ void raw_widen(uint32_t x, uint32_t mask, uint32_t top, uint32_t& o0, uint32_t& o1) {
+  auto value = [&](uint32_t e) {
+    const raw_h2 eighth = {(_Float16)0.125f, (_Float16)0.125f}, m24 = {(_Float16)-24.0f, (_Float16)-24.0f};
+    return raw_h2_bits(__builtin_elementwise_fma(__builtin_bit_cast(raw_h2, (e & mask) ^ top), eighth, m24));
+  };
   if constexpr (PAR == 0) { o0 = value(x << 6); o1 = value(x >> 2); }
   else { o0 = value(x << 2); o1 = value(x >> 6); }
 }
@@ -105,21 +105,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     moe_dma(sb + (size_t)st * 128, lds_w + NU * 4096);
   };
   struct WStep { uint4 w[NU][4]; uint4 s[NU][2]; };   // w[u][h * 2 + o]: piece L = 8h + 2kc + o; s[u][h]: 8 bf16 scales (kb = 0..7)
-  auto fetch_w = [&](auto scaled, WStep& d) __attribute__((always_inline)) {
+  auto fetch_w = [&](WStep& d) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < NU; u++) {
 #pragma unroll
       for (int q = 0; q < 4; q++) d.w[u][q] = *reinterpret_cast<const uint4*>(my_w + (u * 4 + q) * 1024 + lane * 16);
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        d.s[u][h] = *reinterpret_cast<const uint4*>(my_w + NU * 4096 + u * 512 + i * 32 + h * 16);
-        // 2^RAW_LIFT_S in both exponents of a pair; a zero becomes 2^-121, which is zero as an f16 (the pack kernel lets no other scale through
-        // whose exponent could overflow or whose f16 would round)
-        if constexpr (decltype(scaled)::value) {
-          constexpr uint32_t up = (uint32_t)RAW_LIFT_S * 0x00800080u;
-          d.s[u][h].x += up; d.s[u][h].y += up; d.s[u][h].z += up; d.s[u][h].w += up;
-        }
-      }
+      for (int h = 0; h < 2; h++) d.s[u][h] = *reinterpret_cast<const uint4*>(my_w + NU * 4096 + u * 512 + i * 32 + h * 16);
     }
     // read before the next step's DMAs may overwrite them
 #pragma unroll
@@ -152,9 +144,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   asm("v_mov_b32 %0, 0x5A005A00" : "=v"(top));      // 128 = 0x5800, and the nibble's top bit (0x0200) turned
 
   // MTL = 16-row groups of the tile that hold rows; one instantiation per count, chosen once per workgroup.
-  auto run = [&](auto mtl, auto scaled) __attribute__((always_inline)) {
+  auto run = [&](auto mtl) __attribute__((always_inline)) {
     constexpr int MTL = decltype(mtl)::value;
-    constexpr bool SCALED = decltype(scaled)::value;
     constexpr int TB = MTL < 2 ? MTL : 2, NP = (MTL + TB - 1) / TB;   // fragments whose sums are in registers at once; rounds of them
     float acc[NU][MTL][4];
 #pragma unroll
@@ -182,10 +173,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const uint4 &w0 = w.w[u][h * 2], &w1 = w.w[u][h * 2 + 1];
         const uint32_t P0 = Q == 0 ? w0.x : Q == 1 ? w0.y : Q == 2 ? w0.z : w0.w;
         const uint32_t P1 = Q == 0 ? w1.x : Q == 1 ? w1.y : Q == 2 ? w1.z : w1.w;
-        const _Float16 s = SCALED ? (_Float16)scale(w, qc, gc, u) : (_Float16)1.0f, c = s * (_Float16)-192.0f;
         uint32_t o[4];
-        raw_widen<par>(P0, mask, top, raw_h2{s, s}, raw_h2{c, c}, o[0], o[1]);
-        raw_widen<par>(P1, mask, top, raw_h2{s, s}, raw_h2{c, c}, o[2], o[3]);
+        raw_widen<par>(P0, mask, top, o[0], o[1]);
+        raw_widen<par>(P1, mask, top, o[2], o[3]);
         bop[g & 1][u] = __builtin_bit_cast(raw_h8, make_uint4(o[0], o[1], o[2], o[3]));
       }
     };
@@ -229,7 +219,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if constexpr (r + 1 == R && Q < 3) widen(w, std::integral_constant<int, (Q + 1) & 3>{}, std::integral_constant<int, 0>{});
         float bsr[NU];
 #pragma unroll
-        for (int u = 0; u < NU; u++) bsr[u] = SCALED ? 1.0f : scale(w, qc, std::integral_constant<int, r / NP>{}, u);
+        for (int u = 0; u < NU; u++) bsr[u] = scale(w, qc, std::integral_constant<int, r / NP>{}, u);
 #pragma unroll
         for (int t = 0; t < TB; t++) {
           if ((r % NP) * TB + t >= MTL) continue;
@@ -240,7 +230,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int e = 0; e < 4; e++) {
               float& o = acc[u][(r % NP) * TB + t][e];
-              o = fmaf(SCALED ? asv[e] : asv[e] * bsr[u], d[r & 1][t][u][e], o);
+              o = fmaf(asv[e] * bsr[u], d[r & 1][t][u][e], o);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -270,7 +260,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();
     for (int st = 0; st < NS; st++) {
       WStep w;
-      fetch_w(scaled, w);
+      fetch_w(w);
       quarter(std::integral_constant<int, 0>{}, st, w);
       quarter(std::integral_constant<int, 1>{}, st, w);
       quarter(std::integral_constant<int, 2>{}, st, w);
@@ -279,7 +269,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no request may outlive the workgroup's LDS
 
     if (!wave_ok) return;
-    constexpr float unlift = raw_unlift(SCALED);
     if constexpr (GATE_UP) {
       const int n = ustrip[0] * 16 + i;
 #pragma unroll
@@ -288,7 +277,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int r = 0; r < 4; r++) {
           const int row = t * 16 + kc * 4 + r;
           if (row < tile.nrows) {
-            const bf16_t gv = f32_to_bf16(acc[0][t][r] * unlift), uv = f32_to_bf16(acc[1][t][r] * unlift);
+            const bf16_t gv = f32_to_bf16(acc[0][t][r]), uv = f32_to_bf16(acc[1][t][r]);
             p.out[(size_t)(tile.row0 + row) * p.N + n] = f32_to_bf16(act_fn(bf16_to_f32(gv), bf16_to_f32(uv)));
           }
         }
@@ -302,17 +291,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
           for (int r = 0; r < 4; r++) {
             const int row = t * 16 + kc * 4 + r;
-            if (row < tile.nrows) p.out[(size_t)(tile.row0 + row) * p.N + n] = f32_to_bf16(acc[u][t][r] * unlift);
+            if (row < tile.nrows) p.out[(size_t)(tile.row0 + row) * p.N + n] = f32_to_bf16(acc[u][t][r]);
           }
       }
     }
   };
-  if (p.outside[tile.expert]) {   // (rare: two instantiations will do; rows that are not there compute on what the LDS holds, and are not stored)
-    if (mt_live <= MT / 2) run(std::integral_constant<int, MT / 2>{}, std::false_type{});
-    else run(std::integral_constant<int, MT>{}, std::false_type{});
-    return;
-  }
-#define KTX_RAW_CASE(m) case m: run(std::integral_constant<int, m>{}, std::true_type{}); break;
+#define KTX_RAW_CASE(m) case m: run(std::integral_constant<int, m>{}); break;
   switch (mt_live) {
     KTX_RAW_CASE(1) KTX_RAW_CASE(2) KTX_RAW_CASE(3) KTX_RAW_CASE(4)
   }

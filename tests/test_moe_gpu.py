@@ -598,7 +598,7 @@ def _memcpy_d2d(dst, src, nbytes):
 @pytest.mark.parametrize("H,I", [(512, 1536), (1536, 512)])
 def test_rawint4_rows_per_tile_and_any_scale(oracle, dev, H, I):
     """Short batches: the exact kernel's work follows a tile's rows (1, 2, 3, 4 and a 4-row tile behind them) and takes any number of 512-k
-    steps, bit for bit.  Prompts take scales of any magnitude (below, at the lower end of and above what f16 holds) like any other: within the
+    steps, bit for bit.  Prompts take scales of any magnitude like any other: within the
     bound of the prompt kernel, and without a change to a bit of what the other experts give."""
     from helpers import rawint4_quantize
     from ktransformers_amd._native import MoEHandle
@@ -635,35 +635,69 @@ def test_rawint4_rows_per_tile_and_any_scale(oracle, dev, H, I):
             h.close()
 
 
+def _rawint4_chain(a, q, s):
+    """bf16 rows a [T][K] times a RAWINT4 matrix (nibbles [N][K/2], bf16 scales [N][K/32]): per 32 k the int8 codes' sum of products, exact, times the fp32 product
+    of both scales, as one fp32 chain of fmas in k order; bf16 bits."""
+    T, K = a.shape
+    g = bf16_to_f32(a).reshape(T, K // 32, 32)
+    d = np.abs(g).max(-1) / np.float32(127)
+    code = np.clip(np.rint(g * np.where(d > 0, 1 / np.where(d > 0, d, 1), 0).astype(np.float32)[..., None]), -128, 127).astype(np.int64)
+    w = np.stack((q & 15, q >> 4), -1).reshape(q.shape[0], K // 32, 32).astype(np.int64) - 8
+    scale = bf16_to_f32(s)
+    acc = np.zeros((T, q.shape[0]), np.float32)
+    for i in range(K // 32):
+        term = (d[:, i, None] * scale[None, :, i]).astype(np.longdouble) * (code[:, i] @ w[:, i].T)   # (39 bits: exact)
+        acc = (term + acc).astype(np.float32)
+    return f32_to_bf16(acc)
+
+
 @pytest.mark.parametrize("H,I", [(512, 1024), (1024, 512)])
-def test_rawint4_prompt_scales_at_the_edges_of_the_operands(dev, H, I):
-    """The prompt kernel's f16 operands carry weight scales of 2^-23 .. 4 and 0; an expert with any other one is multiplied with its scales outside them.
-    Each expert has one scale at or beside an edge (smallest and largest that fit with all their bits, the next outside, zero), in each matrix, and 1, 16,
-    17, 33, 64 or 65 rows (every count of 16-row groups, and a second tile).  Bound: the one of the prompt kernel against this library's exact kernels."""
+@pytest.mark.parametrize("large", [False, True])
+def test_rawint4_prompt_terms_of_any_scale(dev, H, I, large):
+    """The prompt kernel's sums are fmas of the fp32 scale products, bit for bit (down, from the intermediates that the handle holds), for scales of 0, subnormal, tiny
+    and huge ones beside ordinary ones, with 1, 16, 17, 33, 64 and 65 rows of an expert (every count of 16-row groups, and a second tile); large: outputs up to
+    the last magnitudes of fp32."""
+    import ctypes as C
     from helpers import rawint4_quantize
-    from ktransformers_amd._native import MoEHandle
-    rows, edge = (1, 16, 17, 33, 64, 65), (0.0, 2.0 ** -23 * (1 + 127 / 128), 4 * (1 - 1 / 256), 2.0 ** -24, 4.0, 2.0 ** -23)
+    from ktransformers_amd import _native as n
+    rows, edge = (1, 16, 17, 33, 64, 65), (0.0, 2.0 ** -23 * (1 + 127 / 128), 4 * (1 - 1 / 256), 2.0 ** -24, 2.0 ** -130, 2.0 ** 13)
     E, T = len(rows), sum(rows)
     c = make_case(33, E, 1, H, I, T)
     of = np.repeat(np.arange(E), rows)
-    q = [rawint4_quantize(bf16_to_f32(c[n])) for n in ("gate", "up", "down")]
+    q = [rawint4_quantize(bf16_to_f32(c[m])) for m in ("gate", "up", "down")]
     s = [x[1].copy() for x in q]
-    for e in range(E):
-        for m in range(3):
-            s[m][e, 3 + e, (2 * e + m) % s[m].shape[2]] = f32_to_bf16(np.array([edge[(e + m) % E]], np.float32))[0]
-    d = dict(c, ids=of[:, None].astype(np.int64))
-    h = MoEHandle(E, 1, H, I, max_len=T, method="RAWINT4", device=0, group_size=32)
+    if not large:
+        for e in range(E):
+            for m in range(3):
+                s[m][e, 3 + e, (2 * e + m) % s[m].shape[2]] = f32_to_bf16(np.array([edge[(e + m) % E]], np.float32))[0]
+            s[2][e, 11] = f32_to_bf16(np.full(s[2].shape[2], edge[e] * (1 + 3 / 128), np.float32))      # a row of nothing else
+    h = n.MoEHandle(E, 1, H, I, max_len=T, method="RAWINT4", device=0, group_size=32)
     try:
         h.load_rawint4(*[torch.from_numpy(x[0]).to(dev) for x in q], *[torch_bf16(x, dev) for x in s])
-        got = run(h, d, dev)
-        h.set_exact(True)
-        want = run(h, d, dev)
+
+        def taps(x):
+            run(h, dict(c, x=x, ids=of[:, None].astype(np.int64)), dev)
+            p = [C.c_void_p() for _ in range(3)]
+            n.check(n.lib.ktx_moe_debug_ptrs(h._h, *(C.byref(v) for v in p)))
+            torch.cuda.synchronize()
+            out = [torch.empty((T, w), dtype=torch.int16, device=dev) for w in (I, H)]
+            for t, v in zip(out, p):
+                assert _memcpy_d2d(t.data_ptr(), v.value, t.numel() * 2) == 0
+            return [t.cpu().numpy().view(np.uint16) for t in out]      # (of is in expert order: sorted rows are tokens)
+
+        x = c["x"]
+        if large:   # the outputs follow the square of x while gate's are large: up to about 2^125
+            x = f32_to_bf16(bf16_to_f32(x) * np.float32(2.0 ** 20))
+            top = np.abs(bf16_to_f32(taps(x)[1])).max()
+            x = f32_to_bf16(bf16_to_f32(x) * np.float32(2.0 ** int((125 - np.log2(top)) // 2)))
+        act, got = taps(x)
+        for e in range(E):
+            want = _rawint4_chain(act[of == e], q[2][0][e].view(np.uint8).reshape(H, I // 2), s[2][e].reshape(H, I // 32))
+            assert np.array_equal(got[of == e], want), f"{rows[e]} rows: {int((got[of == e] != want).sum())} outputs differ"
+        if large:
+            assert 2.0 ** 121 < np.abs(bf16_to_f32(got)).max() < np.inf
     finally:
         h.close()
-    for e in range(E):
-        large = np.arange(H) == 3 + e      # (the edge scale of down: a column of its own magnitude)
-        _check_fp(got[of == e][:, ~large], want[of == e][:, ~large])
-        _check_fp(got[of == e][:, large], want[of == e][:, large])
 
 
 @pytest.mark.parametrize("method", ["AMXINT4", "FP8", "RAWINT4", "GGUF"])
