@@ -437,35 +437,64 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
+// A grid of tiles of `cols` columns: its mapping and the rounds, one workgroup a CU, that the XCD with the most of them takes
+struct Gemm256Grid {
+  int tm, tn, xcd_map;
+  long nblk, rounds;
+};
+inline Gemm256Grid gemm256_grid(const GemmParams& p, int cols, int batch) {
+  Gemm256Grid g;
+  g.tm = (p.M + 255) / 256;
+  g.tn = (p.N + cols - 1) / cols;
+  const long per = (g.tn + 7) / 8;
+  g.xcd_map = (g.tm >= 12 && g.tn >= 8) ? 2 : g.tn >= 8 ? 1 : 0;
+  if (g.xcd_map == 2) {   // 4 x 8 supertiles, a round of an XCD each, dealt round-robin: every batch entry begins with the first XCD
+    g.rounds = ((g.tm + 3) / 4 * per + 7) / 8;
+    g.nblk = g.rounds * 8 * 32;
+    g.rounds *= batch;
+  } else if (g.xcd_map) {   // columns, dealt round-robin
+    g.nblk = g.tm * per * 8;
+    g.rounds = (batch * g.tm * per + 31) / 32;
+  } else {
+    g.nblk = (long)g.tm * g.tn;
+    g.rounds = (batch * g.nblk + 255) / 256;
+  }
+  return g;
+}
+
 template <bool F32OUT, bool BTILES, int NB>
 int launch_gemm256_nb(GemmParams p, int batch, hipStream_t st) {
+  const Gemm256Grid g = gemm256_grid(p, Gemm256<NB>::BN, batch);
   auto kern = gemm256_bf16_nt_kernel<F32OUT, BTILES, NB>;
   constexpr int lds = 2 * Gemm256<NB>::STAGE;
-  p.tm = (p.M + 255) / 256;
-  p.tn = (p.N + Gemm256<NB>::BN - 1) / Gemm256<NB>::BN;
-  p.xcd_map = (p.tm >= 12 && p.tn >= 8) ? 2 : p.tn >= 8 ? 1 : 0;
-  long nblk = p.xcd_map ? (long)p.tm * ((p.tn + 7) / 8 * 8) : (long)p.tm * p.tn;
-  if (p.xcd_map == 2) {
-    const long ns = (long)((p.tm + 3) / 4) * ((p.tn + 7) / 8);   // 4 x 8 supertiles, dealt to the XCDs round-robin
-    nblk = (ns + 7) / 8 * 8 * 32;
-  }
-  KTX_REQUIRE(nblk < (1L << 31), "ktx_gemm_bf16_nt: too many tiles");
+  p.tm = g.tm; p.tn = g.tn; p.xcd_map = g.xcd_map;
+  KTX_REQUIRE(g.nblk < (1L << 31), "ktx_gemm_bf16_nt: too many tiles");
   KTX_HIP(ktx_set_max_lds(reinterpret_cast<const void*>(kern), lds));
-  hipLaunchKernelGGL(kern, dim3((unsigned)nblk, (unsigned)batch), dim3(512), lds, st, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)g.nblk, (unsigned)batch), dim3(512), lds, st, p);
   KTX_HIP(hipGetLastError());
   return 0;
 }
 
-// 192 columns where the CUs take no more rounds of them, one workgroup each, than of 256 (bf16 weights, us, 256 | 192 columns): 1536 -> 24576, 500 rows (1 round) 45.9 |
-// 43.5, 1000 (2) 85.5 | 84.8, 2000 (3 | 4) 128 | 150; 2048 -> 3072, 2048 (1) 48.5 | 44.4; 4096 -> 12000, 700 (1) 113 | 109, 1300 (2) 175 | 168; 1280 -> 9000, 2000 (2) 65.8 | 62.3; 7168 -> 4096, 1000 (64 | 88 tiles a piece of K) 68 | 98.  A k-tile's barriers and reads cost the same for both, so a round of 192 takes 0.95 of one of 256, not 0.75.
-template <bool F32OUT, bool BTILES = false>
-int launch_gemm256(const GemmParams& p, int batch, hipStream_t st) {
-  const long tm = (p.M + 255) / 256 * (long)batch, r4 = (tm * ((p.N + 255) / 256) + 255) / 256, r3 = (tm * ((p.N + 191) / 192) + 255) / 256;
-  const int force = ktx_debug_get(7);   // dev knob 7 (tests): 3 or 4 fragments
-  if (force ? force == 3 : r3 <= r4) return launch_gemm256_nb<F32OUT, BTILES, 3>(p, batch, st);
-  return launch_gemm256_nb<F32OUT, BTILES, 4>(p, batch, st);
+// Fragments a wavefront: 192 columns where neither the CUs together nor the XCD with the most tiles take more rounds of them than of 256.  A k-tile's
+// barriers and reads cost the same for both, so a round of 192 takes 0.95 of one of 256, not 0.75.  Measured (us, 256 | 192 columns; rounds of that XCD where they differ): bf16
+// weights 1536 -> 24576, 500 rows 45.9 | 43.5, 1000 85.5 | 84.8, 2000 (3 | 4) 128 | 150; 2048 -> 3072, 2048 48.5 | 44.4; 4096 -> 12000, 700 113 | 109, 1300 175 |
+// 168; 1280 -> 9000, 2000 65.8 | 62.3; 7168 -> 4096, 1000 in 4 parts of K (1 | 2) 68 | 98; 2048 -> 18688, 1280 (2 | 3, of the chip 2 | 2) 97 | 135; 2048 -> 20480, 1792 (3 | 4, 3 | 3)
+// 149 | 182.  Plain operands (rows x columns x K): 4096 x 3072 x 2048 51 | 46, fp32 56 | 49; 6000 x 2304 x 2048 90 | 79; 4864 x 4864 x 2048 (2 | 3, 2 | 2) 101 | 125.  Batches: 8 of 1024 x 1536 x 2048
+// 62 | 53; 16 of 512 x 1536 x 1024 36 | 33; 2 of 2048 x 3000 x 2048 52 | 47; 4 of 4096 x 1536 x 1024 (2 | 4, 2 | 2: a batch entry's four supertiles begin with the first XCD) 61 | 92; 4 of
+// 2048 x 1536, K 1024, 2048, 4096: 31.7 | 30.7, 54.2 | 56.6, 98 | 95.  The chip's count beside the XCD's: supertiles at the edge are not full, 2 of 5632 x 2432 x 2048 (4 | 4, of the chip 2 | 3) 139 | 159.
+// Dev knob 7 (tests): 3 or 4 fragments.
+inline int gemm256_fragments(const GemmParams& p, int batch) {
+  if (const int force = ktx_debug_get(7)) return force == 3 ? 3 : 4;
+  const Gemm256Grid g4 = gemm256_grid(p, 256, batch), g3 = gemm256_grid(p, 192, batch);
+  auto of_chip = [&](const Gemm256Grid& g) { return ((long)g.tm * g.tn * batch + 255) / 256; };
+  return g3.rounds <= g4.rounds && of_chip(g3) <= of_chip(g4) ? 3 : 4;
 }
 
+template <bool F32OUT, bool BTILES = false>
+int launch_gemm256(const GemmParams& p, int batch, hipStream_t st) {
+  if (gemm256_fragments(p, batch) == 3) return launch_gemm256_nb<F32OUT, BTILES, 3>(p, batch, st);
+  return launch_gemm256_nb<F32OUT, BTILES, 4>(p, batch, st);
+}
 
 // fp32 -> three bf16 planes by truncation: w == hi + mid + lo exactly (finite w; 24 mantissa bits = 8 + 8 + 8)
 __global__ __launch_bounds__(256) void split_f32_bf16x3_kernel(const float* __restrict__ w, long n, bf16_t* __restrict__ planes) {
@@ -539,7 +568,8 @@ extern "C" int ktx_gemm_bf16_nt(const ktx_gemm_args* a, ktx_stream_t stream) {
   }
   const double na = a->a_bs ? a->batch : 1, nb = a->b_bs ? a->batch : 1;   // a shared operand is counted once
   KTX_TIMED(st, ((double)a->M * a->K * na + (double)a->N * a->K * nb) * 2 + (double)a->M * a->N * a->batch * (a->out_f32 ? 4 : 2),
-            "gemm_bf16_nt_kernel<%d,%s> %dx%dx%d b%d", variant, a->out_f32 ? "f32" : "bf16", a->M, a->N, a->K, a->batch);
+            "gemm_bf16_nt_kernel<%d,%s> %dx%dx%d b%d, %d columns", variant, a->out_f32 ? "f32" : "bf16", a->M, a->N, a->K, a->batch,
+            variant == 5 ? 64 * gemm256_fragments(p, a->batch) : 128);
   const bool f = a->out_f32 != 0;
   if (variant == 5) {
     KTX_REQUIRE((size_t)a->M * a->lda * 2 < ((size_t)1 << 32) && (size_t)a->N * a->ldb * 2 < ((size_t)1 << 32),
@@ -567,7 +597,7 @@ int ktx_gemm256_tiles(int M, int N, int K, int nsplit, const bf16_t* A, long lda
   p.B = reinterpret_cast<const bf16_t*>(tiles); p.ldb = nks; p.b_bs = (long)(p.K / 128) * 2048;
   p.Y = Y; p.ldy = ldy; p.y_bs = y_bs;
   KTX_TIMED(st, (double)nks * ((N + 15) / 16) * 4096.0 + (double)M * K * 2.0 + (double)M * N * nsplit * (out_f32 ? 4 : 2),
-            "gemm256_bf16_nt_kernel<%s,tiles> %dx%dx%d splits %d", out_f32 ? "f32" : "bf16", M, N, K, nsplit);
+            "gemm256_bf16_nt_kernel<%s,tiles> %dx%dx%d splits %d, %d columns", out_f32 ? "f32" : "bf16", M, N, K, nsplit, 64 * gemm256_fragments(p, nsplit));
   return out_f32 ? launch_gemm256<true, true>(p, nsplit, st) : launch_gemm256<false, true>(p, nsplit, st);
 }
 

@@ -90,6 +90,54 @@ def test_ping_pong_tile_of_192_columns(M, N, K):
         _native.lib.ktx_debug_set(7, 0)
 
 
+@pytest.mark.parametrize("B,M,N,K,columns", [
+    (1, 1000, 24576, 1536, 192), (1, 2000, 24576, 1536, 256), (1, 4096, 3072, 2048, 192), (1, 4864, 4864, 1024, 256), (1, 3072, 8064, 1024, 256), (1, 1280, 18688, 1024, 256),
+    (1, 9728, 1664, 1024, 256), (8, 1024, 1536, 1024, 192), (2, 2048, 3000, 1024, 192), (4, 4096, 1536, 1024, 256), (2, 5632, 1792, 1024, 256), (2, 5632, 2432, 1024, 256)])
+def test_columns_follow_the_rounds_of_the_busiest_xcd(B, M, N, K, columns):
+    """192 columns only where neither the CUs together nor the XCD with the most tiles take more rounds of them (up to 1.5 times the time otherwise)."""
+    from ktransformers_amd import _native as n
+    a, b = (torch.zeros((B, r, K), dtype=torch.bfloat16, device=DEV) for r in (M, N))
+    n.timing_enable(2)
+    try:
+        n.gemm_bf16_nt(a, b)
+        labels = [t[0] for t in n.timing_collect()]
+    finally:
+        n.timing_enable(0)
+    assert len(labels) == 1 and labels[0].startswith("gemm_bf16_nt_kernel<5,") and labels[0].endswith(f", {columns} columns"), labels
+
+
+@pytest.mark.parametrize("K,N,T,columns", [(1536, 24576, 1000, 192), (2048, 18688, 1280, 256), (2048, 20480, 1792, 256), (4096, 12000, 700, 192)])
+def test_columns_of_a_linear(K, N, T, columns):
+    """The same on a bf16 linear's tiles."""
+    from ktransformers_amd import _native as n
+    h = n.LinearHandle(K, N, "BF16", 0, T, torch.device(DEV))
+    h.load_bf16(torch.zeros((N, K), dtype=torch.bfloat16, device=DEV))
+    n.timing_enable(2)
+    try:
+        h.forward(torch.zeros((T, K), dtype=torch.bfloat16, device=DEV))
+        labels = [t[0] for t in n.timing_collect() if t[0].startswith("gemm256_bf16_nt_kernel<")]
+    finally:
+        n.timing_enable(0)
+    assert len(labels) == 1 and labels[0].endswith(f", {columns} columns"), labels
+
+
+@pytest.mark.parametrize("B,M,N,K", [(3, 300, 400, 192), (2, 513, 192, 128)])
+def test_ping_pong_tiles_of_batches(B, M, N, K):
+    """192 and 256 columns on batches, bf16 and fp32 output: variant 2's bits."""
+    from ktransformers_amd import _native
+    from ktransformers_amd._native import gemm_bf16_nt
+    g = torch.Generator(device="cpu").manual_seed(M)
+    a = torch.randn((B, M, K), generator=g).to(torch.bfloat16).to(DEV)
+    b = (torch.randn((B, N, K), generator=g) * K ** -0.5).to(torch.bfloat16).to(DEV)
+    ref = [gemm_bf16_nt(a, b, variant=2, out_f32=f) for f in (False, True)]
+    try:
+        for knob in (3, 4):
+            _native.lib.ktx_debug_set(7, knob)
+            assert all(torch.equal(gemm_bf16_nt(a, b, variant=5, out_f32=f), r) for f, r in zip((False, True), ref)), knob
+    finally:
+        _native.lib.ktx_debug_set(7, 0)
+
+
 @pytest.mark.parametrize("T,K,N", [(300, 1536, 24576), (700, 4096, 12000)])
 def test_linear_tiles_of_192_columns(T, K, N):
     """The same on a bf16 linear's own weights (its tiles are the B operand)."""
