@@ -493,7 +493,7 @@ __device__ __forceinline__ MlaWork mla_pick_job(const MlaParams& p, int job, int
 // same bits, and they are the bits the shuffle version produced ((x + shfl16) + shfl32 groups the rows as (r0 + r1) + (r2 + r3) for
 // rows 0 / 1 and likewise here after the 32-swap first: see pf_sum_rows).
 typedef unsigned pf_v2u __attribute__((ext_vector_type(2)));
-typedef float pf_v2f __attribute__((ext_vector_type(2)));
+typedef uint32_t pf_u4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float pf_max_rows(float x) {
   pf_v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
@@ -1158,9 +1158,13 @@ struct MlaPrefillParams {
 // 128 heads, us, one after the other -> here: 1000 tokens behind 3096 367 -> 310 (788 -> 950 TFLOP/s), 2048 of 2048 260 -> 214, 512 of 8192 396 -> 336; 16 heads, 300 of 1500: 50
 // -> 38.  Left to its own order the compiler puts the products first, each fragment's read directly before its use, and the softmax behind them: 325 us; with the
 // largest scores found beside the products as well, 320.  A running maximum moves somewhere in two fifths of the tiles: one branch for both query tiles costs 8 %.
-// DMA false: operands that do not lie on 16 bytes come through registers, into the same places.
-template <bool DMA>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void mla_prefill_kernel(MlaPrefillParams p) {
+// DMA false: operands that do not lie on 16 bytes come through registers, into the same places.  Written where they were requested they stood in the step's way; V^T
+// waits beside S and K beside O, for which the registers suffice but for 11 of them.  ALONE: workgroups that have a CU each (as many as CUs, or fewer) have twice the registers, and both
+// wait for the whole step.  Us, as the tiles' way through registers was before | written at once | now, 8 bytes off: 128 heads, 64 tokens of 4096 125 | 174 | 116 (ALONE; 141 not), 1000 of 4096 370 | 391 |
+// 358 (454 ALONE), 1000 of 1000 96 | 97 | 94; 16 heads, 64 of 2000 63.5 | 60.4 | 60.2; 2 bytes off, where the loads themselves are slow: 167 | - | 156, 391 | - | 415, 105 | - | 110, 80 | - | 76.
+// (4 bytes a request, by LDS-DMA: 174, 413, 111, 88.)
+template <bool DMA, bool ALONE = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 : 2, ALONE ? 1 : 2))) void mla_prefill_kernel(MlaPrefillParams p) {
   constexpr int NU = 2;                              // query tiles of 16 per wavefront: every K fragment read feeds two MFMAs
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][PF_KB] | [2][PF_VB]
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1186,32 +1190,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const bf16_t* kn = p.k_nope + (size_t)h * p.kv_pad * 128;
   const bf16_t* vt = p.v_t + (size_t)h * 128 * p.kv_pad;
 
-  // ---- a tile's requests, 10 a wavefront: 4 rows of K, 8 of k_pe or of V^T each.  Rows of k_pe past kv_len read the last one (their scores are masked).
+  // ---- a tile's requests, 10 a wavefront: 4 rows of K, 8 of k_pe or of V^T each.  Rows of k_pe past kv_len read the last one (their scores are masked).  DMA false: a
+  // lane's 16 bytes wait in registers until put writes them.
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
   const int er = wave * 8 + (lane >> 3), ep = (lane & 7) ^ (wave * 2 + ((lane >> 4) & 1)), vp = (lane & 7) ^ ((wave * 4 + (lane >> 4)) & 7);
   const uint32_t ko_dma = (wave * 4 + (lane >> 4)) * 256 + ((lane & 15) ^ ((wave >> 1) * 4 + (lane >> 4))) * 16, vo_dma = (uint32_t)er * (uint32_t)p.kv_pad * 2u + vp * 16;
-  auto bring = [&](const bf16_t* base, uint32_t lane_bytes, uint32_t at) __attribute__((always_inline)) {   // 16 bytes a lane
+  auto bring = [&](const bf16_t* base, uint32_t lane_bytes, uint32_t at, pf_u4& held) __attribute__((always_inline)) {
     if constexpr (DMA) mla_dma_row_sa(base, lane_bytes, lds0 + at);
-    else *reinterpret_cast<uint4*>(smem + at + lane * 16) = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(base) + lane_bytes);
+    else held = *reinterpret_cast<const pf_u4*>(reinterpret_cast<const uint8_t*>(base) + lane_bytes);
   };
-  auto stage_k = [&](int tile, int buf) __attribute__((always_inline)) {
+  auto put = [&](uint32_t at, const pf_u4& held) __attribute__((always_inline)) {
+    if constexpr (!DMA) *reinterpret_cast<pf_u4*>(smem + at + lane * 16) = held;
+  };
+  auto k_at = [&](int c, int buf) __attribute__((always_inline)) { return (uint32_t)(buf * PF_KB + (c * 4 + wave) * 1024); };   // K: c 0 .. 3, k_pe behind it: 4, 5
+  auto v_at = [&](int c, int buf) __attribute__((always_inline)) { return (uint32_t)(2 * PF_KB + buf * PF_VB + (c * 4 + wave) * 1024); };
+  auto stage_k = [&](int tile, int buf, pf_u4 (&held)[6]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int c = 0; c < 4; c++) bring(kn + (size_t)(tile * PF_BN + c * 16) * 128, ko_dma ^ ((c & 1) * 128), buf * PF_KB + (c * 4 + wave) * 1024);
+    for (int c = 0; c < 4; c++) bring(kn + (size_t)(tile * PF_BN + c * 16) * 128, ko_dma ^ ((c & 1) * 128), k_at(c, buf), held[c]);
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
-      const bf16_t* src = p.k_pe + (size_t)min(tile * PF_BN + c * 32 + er, p.kv_len - 1) * p.kpe_ts + ep * 8;
-      const uint32_t at = buf * PF_KB + PF_KN + (c * 4 + wave) * 1024;
-      if constexpr (DMA) mla_dma_row_a(src, lds0 + at);
-      else *reinterpret_cast<uint4*>(smem + at + lane * 16) = *reinterpret_cast<const uint4*>(src);
+    for (int c = 4; c < 6; c++) {
+      const bf16_t* src = p.k_pe + (size_t)min(tile * PF_BN + (c - 4) * 32 + er, p.kv_len - 1) * p.kpe_ts + ep * 8;
+      if constexpr (DMA) mla_dma_row_a(src, lds0 + k_at(c, buf));
+      else held[c] = *reinterpret_cast<const pf_u4*>(src);
     }
   };
-  auto stage_v = [&](int tile, int buf) __attribute__((always_inline)) {
+  auto stage_v = [&](int tile, int buf, pf_u4 (&held)[4]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int c = 0; c < 4; c++) bring(vt + (size_t)c * 32 * p.kv_pad + tile * PF_BN, vo_dma, 2 * PF_KB + buf * PF_VB + (c * 4 + wave) * 1024);
+    for (int c = 0; c < 4; c++) bring(vt + (size_t)c * 32 * p.kv_pad + tile * PF_BN, vo_dma, v_at(c, buf), held[c]);
   };
-  stage_k(0, 0);
-  stage_v(0, 0);
-  if (ntiles > 1) stage_k(1, 1);
+  auto put_k = [&](int buf, const pf_u4 (&held)[6]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 6; c++) put(k_at(c, buf), held[c]);
+  };
+  auto put_v = [&](int buf, const pf_u4 (&held)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 4; c++) put(v_at(c, buf), held[c]);
+  };
+  {
+    pf_u4 hk[6], hv[4];
+    stage_k(0, 0, hk);
+    stage_v(0, 0, hv);
+    put_k(0, hk);
+    put_v(0, hv);
+    if (ntiles > 1) {
+      stage_k(1, 1, hk);
+      put_k(1, hk);
+    }
+  }
 
   // Q^T fragments: lane (query qi, k-chunk g)
   v8bf qf[NU][6];
@@ -1291,9 +1316,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const float cexp = p.sm_scale * 1.44269504088896340736f;
   auto step = [&](auto more, int par, int tile, v4f (&st)[NU][4], v4f (&nx)[NU][4]) __attribute__((always_inline)) {
     constexpr bool MORE = decltype(more)::value;
+    pf_u4 hk[6], hv[4];
     if constexpr (MORE) {   // (the buffers' last readers were a step ago)
-      if (tile + 2 < ntiles) stage_k(tile + 2, par);
-      stage_v(tile + 1, par ^ 1);
+      if constexpr (DMA) {
+        if (tile + 2 < ntiles) stage_k(tile + 2, par, hk);
+      } else if constexpr (ALONE) {
+        stage_k(min(tile + 2, ntiles - 1), par, hk);
+      }
+      stage_v(tile + 1, par ^ 1, hv);
     }
     // ---- online softmax, per query (lane & 15): where some lane's running maximum moved, O and the sums are scaled to the new one.  It is kept on the RAW scores;
     // the softmax scale rides in the exponent's multiply: p = exp2(s * c - m * c), c = sm_scale * log2(e).  A lane sums its own keys; the query's four meet at the end.
@@ -1346,6 +1376,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int ks = 0; ks < 2; ks++) asm volatile("" : "+v"(pb[u][ks].x), "+v"(pb[u][ks].y), "+v"(pb[u][ks].z), "+v"(pb[u][ks].w));
       }
       mask(tile + 1, nx);
+      if constexpr (!DMA && !ALONE) {   // (V^T waited beside S, K does beside O, where the scores before are gone; the last requests repeat)
+        put_v(par ^ 1, hv);
+        stage_k(min(tile + 2, ntiles - 1), par, hk);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     // ---- O^T += V^T P^T: o[u][i][r] = O[query qi][dim 16*i + 4*g + r], beside the next tile's largest scores
     const uint8_t* vb = smem + par * PF_VB;
@@ -1366,6 +1401,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (f < 12) __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
     }
     if constexpr (MORE) {
+      if constexpr (ALONE) put_v(par ^ 1, hv);
+      put_k(par, hk);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (a step old)
       __syncthreads();
     }
@@ -1420,16 +1457,16 @@ extern "C" int ktx_mla_prefill(int T, int num_heads, int kv_len, int kv_pad, flo
   p.T = T; p.H = num_heads; p.kv_len = kv_len; p.kv_pad = kv_pad; p.sm_scale = sm_scale;
   constexpr int lds = 2 * (PF_KB + PF_VB);
   const bool aligned = ((reinterpret_cast<uintptr_t>(d_k_nope) | reinterpret_cast<uintptr_t>(d_k_pe) | reinterpret_cast<uintptr_t>(d_v_t)) & 15) == 0;
-  KTX_HIP(ktx_set_max_lds(aligned ? reinterpret_cast<const void*>(mla_prefill_kernel<true>) : reinterpret_cast<const void*>(mla_prefill_kernel<false>), lds));
+  const int nqb = (T + 127) / 128;
+  void (*kern)(MlaPrefillParams) = aligned ? mla_prefill_kernel<true> : (long)nqb * num_heads <= 256 ? mla_prefill_kernel<false, true> : mla_prefill_kernel<false>;
+  KTX_HIP(ktx_set_max_lds(reinterpret_cast<const void*>(kern), lds));
   hipStream_t st = (hipStream_t)stream;
   // per (query, key, head): 2*(192 + 128) flop over the causal half
   KTX_TIMED(st, 0.0, "mla_prefill_kernel T=%d Hq=%d kv=%d", T, num_heads, kv_len);
-  const int nqb = (T + 127) / 128;
   const bool xcd = num_heads % 8 == 0;
   p.nqb = xcd ? nqb : 0;
   const dim3 grid = xcd ? dim3((unsigned)(nqb * num_heads)) : dim3(nqb, num_heads);
-  if (aligned) hipLaunchKernelGGL(mla_prefill_kernel<true>, grid, dim3(256), lds, st, p);
-  else hipLaunchKernelGGL(mla_prefill_kernel<false>, grid, dim3(256), lds, st, p);
+  hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p);
   KTX_HIP(hipGetLastError());
   return 0;
 }

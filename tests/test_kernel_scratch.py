@@ -40,7 +40,7 @@ def private_segments(lib, tmp):
     return out
 
 
-@pytest.mark.parametrize("kernel", ["moe_gguf_fold_kernel", "moe_rawint4_chunk_kernel", "mla_decode_wide_kernel", "lin_tile_kernel", "moe_gemm_stream_kernel", "moe_fp8_stream_kernel", "mla_prefill_kernelILb1E"])
+@pytest.mark.parametrize("kernel", ["moe_gguf_fold_kernel", "moe_rawint4_chunk_kernel", "mla_decode_wide_kernel", "lin_tile_kernel", "moe_gemm_stream_kernel", "moe_fp8_stream_kernel", "mla_prefill_kernelILb1E", "mla_prefill_kernelILb0ELb1E"])
 def test_prompt_kernels_keep_their_operands_in_registers(kernel, tmp_path):
     if not os.path.exists(build.LIB) or not os.path.exists(READELF):
         pytest.skip("needs the built library and llvm-readelf")

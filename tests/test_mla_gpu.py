@@ -263,8 +263,8 @@ def test_prefill_expanded_against_fp32_attention(H, T, kv_len, knob22):
     torch.testing.assert_close(out.float(), ref.to(torch.bfloat16).float(), rtol=2.0 ** -7, atol=5e-3)
 
 
-@pytest.mark.parametrize("offset", [0, 4])   # elements: operands on 16 bytes come by LDS-DMA, others through registers
-@pytest.mark.parametrize("H,T,kv_len", [(1, 1, 1), (2, 1, 64), (2, 1, 65), (3, 129, 128 + 129), (8, 33, 320), (2, 256, 4160)])
+@pytest.mark.parametrize("offset", [0, 4, 1])   # elements: operands on 16 bytes come by LDS-DMA, others through registers
+@pytest.mark.parametrize("H,T,kv_len", [(1, 1, 1), (2, 1, 64), (2, 1, 65), (3, 129, 128 + 129), (8, 33, 320), (2, 256, 4160), (130, 130, 321)])   # the last: more workgroups than CUs
 def test_prefill_tiles_of_keys(H, T, kv_len, offset):
     """One key tile, two, odd and even counts of them, against attention in 64 bits.  Probabilities enter the product as bf16 (2^-8 of their size, and they sum to one)
     and the output is rounded to bf16: 2^-8 of the largest value each, at most."""
