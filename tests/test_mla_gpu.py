@@ -8,6 +8,8 @@ import torch
 
 from oracle.mla_ref import mla_paged_ref
 
+from test_mla_prefill_bound import prefill_operands, prefill_scores, prefill_statement
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
@@ -231,14 +233,11 @@ def test_decode_at_128k_context():
 
 
 # ---- non-absorbed prompt attention (ktx_mla_prefill) ----------------------------------------------------------------------
-@pytest.mark.parametrize("knob22", [0, 1])
 @pytest.mark.parametrize("H,T,kv_len", [(4, 130, 130), (3, 70, 201), (16, 128, 128), (2, 257, 1000), (128, 64, 64)])
-def test_prefill_expanded_against_fp32_attention(H, T, kv_len, knob22):
+def test_prefill_expanded_against_fp32_attention(H, T, kv_len):
     """Causal softmax(q k^T) v over qk 192 (128 nope + 64 shared rope) / v 128 in fp32 on the same bf16 operands; the queries are
     the last T keys; the padded key rows are zero as the operator makes them."""
-    from ktransformers_amd import _native
     from ktransformers_amd._native import mla_prefill
-    _native.check(_native.lib.ktx_debug_set(22, knob22))      # 0: the default (<= 256 registers, two workgroups per CU); 1: the unconstrained build
     g = torch.Generator().manual_seed(H * 1000 + T + kv_len)
     kv_pad = (kv_len + 63) // 64 * 64
     q = torch.randn((T, H, 192), generator=g).to(torch.bfloat16).to(DEV)
@@ -250,11 +249,7 @@ def test_prefill_expanded_against_fp32_attention(H, T, kv_len, knob22):
     v[:, :kv_len] = torch.randn((H, kv_len, 128), generator=g).to(torch.bfloat16).to(DEV)
     sm_scale = 192 ** -0.5
     q_pe = q[:, :, 128:].contiguous()
-    try:
-        out = mla_prefill(q[:, :, :128], q_pe, k_nope, cache[:, 512:], v.transpose(1, 2).contiguous(), kv_len, sm_scale)
-        torch.cuda.synchronize()
-    finally:
-        _native.check(_native.lib.ktx_debug_set(22, 0))
+    out = mla_prefill(q[:, :, :128], q_pe, k_nope, cache[:, 512:], v.transpose(1, 2).contiguous(), kv_len, sm_scale)
     k = torch.cat([k_nope[:, :kv_len].float(), cache[:kv_len, 512:].float()[None].expand(H, -1, -1)], dim=-1)    # [H, kv, 192]
     s = torch.einsum("thd,hkd->htk", q.float(), k) * sm_scale
     pos = torch.arange(T, device=DEV)[:, None] + (kv_len - T)
@@ -266,29 +261,20 @@ def test_prefill_expanded_against_fp32_attention(H, T, kv_len, knob22):
 @pytest.mark.parametrize("offset", [0, 4, 1])   # elements: operands on 16 bytes come by LDS-DMA, others through registers
 @pytest.mark.parametrize("H,T,kv_len", [(1, 1, 1), (2, 1, 64), (2, 1, 65), (3, 129, 128 + 129), (8, 33, 320), (2, 256, 4160), (130, 130, 321)])   # the last: more workgroups than CUs
 def test_prefill_tiles_of_keys(H, T, kv_len, offset):
-    """One key tile, two, odd and even counts of them, against attention in 64 bits.  Probabilities enter the product as bf16 (2^-8 of their size, and they sum to one)
-    and the output is rounded to bf16: 2^-8 of the largest value each, at most."""
+    """One key tile, two, odd and even counts of them, against attention in 64 bits, at the bound of its roundings (test_mla_prefill_bound.py: which shows a missing tile)."""
     from ktransformers_amd._native import mla_prefill
-    g = torch.Generator().manual_seed(H * 1000 + T + kv_len)
-    kv_pad = (kv_len + 63) // 64 * 64
+    q, k_nope, cache, v = prefill_operands(H, T, kv_len)
 
     def at_offset(x):
         flat = torch.empty(x.numel() + offset, dtype=torch.bfloat16, device=DEV)
         flat[offset:] = x.reshape(-1).to(DEV)
         return flat[offset:].view(x.shape)
 
-    q = torch.randn((T, H, 192), generator=g).to(torch.bfloat16)
-    k_nope, v = torch.zeros((2, H, kv_pad, 128), dtype=torch.bfloat16)
-    k_nope[:, :kv_len] = torch.randn((H, kv_len, 128), generator=g).to(torch.bfloat16)
-    v[:, :kv_len] = torch.randn((H, kv_len, 128), generator=g).to(torch.bfloat16)
-    cache = torch.randn((kv_len, 576), generator=g).to(torch.bfloat16)
     qd = q.to(DEV)
     out = mla_prefill(qd[:, :, :128], qd[:, :, 128:], at_offset(k_nope), at_offset(cache)[:, 512:], at_offset(v.transpose(1, 2).contiguous()), kv_len, 192 ** -0.5)
-    k = torch.cat([k_nope[:, :kv_len].double(), cache[:, 512:].double()[None].expand(H, -1, -1)], dim=-1)
-    s = torch.matmul(q.double().transpose(0, 1), k.transpose(1, 2)) * 192 ** -0.5
-    s = s.masked_fill(torch.arange(kv_len)[None, :] > torch.arange(T)[:, None] + (kv_len - T), float("-inf"))
-    ref = torch.matmul(torch.softmax(s, dim=-1), v[:, :kv_len].double()).transpose(0, 1)
-    assert float((out.cpu().double() - ref).abs().max()) <= 2.0 ** -7 * float(v.double().abs().max())
+    ref, bound = prefill_statement(prefill_scores(q, k_nope, cache, kv_len), v[:, :kv_len].double())
+    err = (out.cpu().double() - ref).abs()
+    assert bool((err <= bound).all()), f"{int((err > bound).sum())} outputs, up to {float((err / bound).max()):.2f} of the bound"
 
 
 @pytest.mark.parametrize("Hq,kv_len,T", [(128, 4023, 1), (64, 700, 1), (128, 33, 1), (64, 5000, 3)])
