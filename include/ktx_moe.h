@@ -186,24 +186,22 @@ int ktx_profile_enable(int on);
 /* Test hook: non-zero routes every batch through the grouped (bucket + M-tiled GEMM) path, including the small
  * batches that normally take the two-launch decode path, so both implementations can be compared on one input. */
 int ktx_debug_force_generic(int on);
-/* Development knobs for timing experiments and tests (never set by the product path): idx 0 = waves per workgroup of the
- * decode gate/up kernel (0 = auto), idx 1 = ablation bits (bit0: skip the weight stream; results are then meaningless),
- * idx 2 = run only one decode kernel (1 gate/up, 2 down; bench.py's per-kernel timing), idx 4 = prompt (64-row tile) GEMM
- * implementation: 0 auto (streaming kernels for hidden*intermediate >= 4M), 1 chunk-pipelined only, 2 streaming only,
- * 3 the register-tile kernels (256-row tiles; bit-exact in the tests; timed in round 2 with scripts/stream_ab.py: faster
- * only under uniform routing at V2-Lite shapes, slower under skew and at V3 shapes, hence not selected by default),
- * idx 5 = run only one kernel of ktx_mla_decode* (1 the split-KV kernel, 2 the merge; per-kernel timing), idx 6 / 7 = force
- * the MLA workgroup shape (1, 2, 4 head blocks) / the KV split count, idx 8 = force the strips-per-workgroup split of the
- * decode GEMV (tuning sweeps under scripts/), idx 9 = 2 selects the LDS-DMA ring variant of the W4 decode GEMV (measured
- * slower than the default register ring; kept for tuning), idx 10 = 1 turns the k-slices of the AMXINT4 decode gate/up kernel
- * off, idx 11 = 1 selects the first (>= 384 workgroups) split rule of the decode GEMV (both A/B switches of
- * scripts/ab_decode.py), idx 12 = strips per wavefront of the prompt-sized W4 GEMM (1 = the one-strip kernel, 2 / 4 forced;
- * 0 auto), idx 13 = 1 makes ktx_linear_forward_fused_gate issue its two launches instead of the combined kernel (A/B, tests),
- * idx 14 = 1 makes ktx_moe_forward_side run the side linear as a launch of its own (A/B, tests), idx 15 = 1 makes
- * ktx_linear_qb_absorb_eligible answer no (A/B), idx 22 = 1 runs the non-absorbed prompt attention kernel with its
- * unconstrained register allocation (one wavefront per SIMD; A/B of scripts/mla_prefill_bench.py), idx 25 = experts per
- * router workgroup in ktx_linear_forward_fused_gate's combined kernel: 1 -> 8 (rounds 2-3), 2 -> 2, 0 -> 4 where the grid has room
- * (same logits and selection bit for bit). */
+/* Development knobs for timing experiments and tests (never set by the product path): idx 0 = waves per workgroup of the decode gate/up kernel (0 =
+ * auto), idx 1 = ablation bits (bit0: skip the weight stream; results are then meaningless), idx 2 = run only one decode kernel (1 gate/up, 2 down;
+ * bench.py's per-kernel timing), idx 4 = AMXINT4 / AMXINT8 prompt (64-row tile) GEMM implementation: 0 auto (streaming kernels where they were measured
+ * faster), 1 chunk-pipelined only, 2 streaming only, 3 the register-tile kernels (256-row tiles; bit-exact in the tests; timed with
+ * scripts/stream_ab.py: faster only under uniform routing at V2-Lite shapes, slower under skew and at V3 shapes, hence not selected by default), idx 5 =
+ * run only one kernel of ktx_mla_decode* (1 the split-KV kernel, 2 the merge; per-kernel timing), idx 6 / 7 = force the MLA workgroup shape (1, 2, 4
+ * head blocks) / the KV split count, idx 8 = force the strips-per-workgroup split of the decode GEMV (tuning sweeps under scripts/), idx 9 = 2 selects
+ * the LDS-DMA ring variant of the W4 decode GEMV (measured slower than the default register ring; kept for tuning), idx 10 = 1 turns the k-slices of the
+ * AMXINT4 decode gate/up kernel off, idx 11 = 1 selects the first (>= 384 workgroups) split rule of the decode GEMV (both A/B switches of
+ * scripts/ab_decode.py), idx 12 = strips per wavefront of the prompt-sized W4 GEMM (1 = the one-strip kernel, 2 / 4 forced; 0 auto), idx 13 = 1 makes
+ * ktx_linear_forward_fused_gate issue its two launches instead of the combined kernel (A/B, tests), idx 14 = 1 makes ktx_moe_forward_side run the side
+ * linear as a launch of its own (A/B, tests), idx 15 = 1 makes ktx_linear_qb_absorb_eligible answer no (A/B), idx 22 = tile height of the folded K-quant
+ * prompt kernels (1: 64 rows at most, 2: 128), idx 23 = wavefronts of the AMXINT4 / AMXINT8 streaming kernels (1: 4, 2: 8), idx 24 = the FP8 streaming
+ * kernel (1 never, 2 always), idx 25 = experts per router workgroup in ktx_linear_forward_fused_gate's combined kernel: 1 -> 8, 2 -> 2, 0 -> 4 where the
+ * grid has room (same logits and selection bit for bit), idx 31 = 16-column fragments a wavefront of the 256-row bf16 GEMM (3 or 4), idx 32 = 1 keeps W4
+ * FP8 linears off the 64 x 256 tiles. */
 int ktx_debug_set(int idx, int val);
 int ktx_debug_get(int idx);
 /* Per-launch timing of every kernel of the library (bench.py's per-kernel table; ktx_prof.hip).  mode 1: each launch is

@@ -482,9 +482,9 @@ int launch_gemm256_nb(GemmParams p, int batch, hipStream_t st) {
 // 149 | 182.  Plain operands (rows x columns x K): 4096 x 3072 x 2048 51 | 46, fp32 56 | 49; 6000 x 2304 x 2048 90 | 79; 4864 x 4864 x 2048 (2 | 3, 2 | 2) 101 | 125.  Batches: 8 of 1024 x 1536 x 2048
 // 62 | 53; 16 of 512 x 1536 x 1024 36 | 33; 2 of 2048 x 3000 x 2048 52 | 47; 4 of 4096 x 1536 x 1024 (2 | 4, 2 | 2: a batch entry's four supertiles begin with the first XCD) 61 | 92; 4 of
 // 2048 x 1536, K 1024, 2048, 4096: 31.7 | 30.7, 54.2 | 56.6, 98 | 95.  The chip's count beside the XCD's: supertiles at the edge are not full, 2 of 5632 x 2432 x 2048 (4 | 4, of the chip 2 | 3) 139 | 159.
-// Dev knob 7 (tests): 3 or 4 fragments.
+// Dev knob 31 (tests): 3 or 4 fragments.
 inline int gemm256_fragments(const GemmParams& p, int batch) {
-  if (const int force = ktx_debug_get(7)) return force == 3 ? 3 : 4;
+  if (const int force = ktx_debug_get(31)) return force == 3 ? 3 : 4;
   const Gemm256Grid g4 = gemm256_grid(p, 256, batch), g3 = gemm256_grid(p, 192, batch);
   auto of_chip = [&](const Gemm256Grid& g) { return ((long)g.tm * g.tn * batch + 255) / 256; };
   return g3.rounds <= g4.rounds && of_chip(g3) <= of_chip(g4) ? 3 : 4;

@@ -2087,7 +2087,8 @@ static int launch_gemm(const GemmParams& p, int max_tiles, hipStream_t st) {
   return 0;
 }
 
-static int g_dbg[32] = {0};  // dev knobs: [0] waves/workgroup override of the decode gate/up kernel, [1] ablation bits
+constexpr int KTX_DBG = 33;
+static int g_dbg[KTX_DBG] = {0};  // dev knobs (include/ktx_moe.h)
 template <int WBITS, bool GATE_UP>
 static int launch_gemm_rt(const GemmParams& p, int max_tiles, hipStream_t st) {
   const size_t lds = 2 * (8 * 256 * 16 + 16 * 2048) + 256 * 8;
@@ -2141,8 +2142,8 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
 static bool g_prof_on = false;
 static bool g_force_generic = false;  // tests: route small batches through the grouped (prefill) path too
 extern "C" int ktx_debug_force_generic(int on) { g_force_generic = on != 0; return 0; }
-extern "C" int ktx_debug_set(int idx, int val) { if (idx >= 0 && idx < 32) g_dbg[idx] = val; return 0; }
-extern "C" int ktx_debug_get(int idx) { return idx >= 0 && idx < 32 ? g_dbg[idx] : 0; }
+extern "C" int ktx_debug_set(int idx, int val) { if (idx >= 0 && idx < KTX_DBG) g_dbg[idx] = val; return 0; }
+extern "C" int ktx_debug_get(int idx) { return idx >= 0 && idx < KTX_DBG ? g_dbg[idx] : 0; }
 static std::vector<std::pair<hipEvent_t, hipEvent_t>> g_prof_ev[5];
 static std::vector<std::pair<hipEvent_t, hipEvent_t>> g_prof_free;
 
@@ -2390,7 +2391,7 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
   // 2670.  A short K or few workgroups stream no better: 64 of 1536 x 3072, 20 rows 130 | 137.  16 against 32 rows: 3.1 rows 660 | 669, 6.6: 750 | 778, 64 experts of
   // 2048 x 1408, 3: 59 | 63, 9.4: 77 | 77.  32 against 64 rows where nothing streams: 25 rows
   // 134 | 135, 37: 109 | 109, 50: 177 | 169, 75: 152 | 138; with 8 experts 25: 35 | 41, 100: 53 | 58, 125: 60 | 59, 200: 82 | 75 — few tiles leave
-  // CUs idle longer.  Dev knobs (tests) [4]: 1 = never stream, 2 = always at 64 rows; [5]: 1 = 4 wavefronts, 2 = 8.
+  // CUs idle longer.  Dev knobs (tests) [4]: 1 = never stream, 2 = always at 64 rows; [23]: 1 = 4 wavefronts, 2 = 8.
   const auto tiles64 = [&](int strips) { return (std::min(npairs, E) + npairs / 64) * ((I / 16 + strips - 1) / strips); };   // workgroups of gate|up
   const double rows = (double)npairs / std::max(1, E);
   const bool large = (size_t)H * I >= ((size_t)4 << 20), fills8 = std::min(H, I) >= 2048 && tiles64(16) >= 1200;
@@ -2400,7 +2401,7 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
     use_stream = g_dbg[4] != 1 && large && ((rows > 12.0 && fills8) || (rows >= 48.0 && fills4));
     mt = rows <= 8.0 ? 1 : use_stream || (rows > 40.0 && tiles64(4) >= 512) ? 4 : 2;
   }
-  const int stream_nw = g_dbg[5] ? 4 * g_dbg[5] : (fills8 && (H >= 4096 || rows < 48.0)) || (h->wbits == 8 && rows < 56.0) ? 8 : 4;
+  const int stream_nw = g_dbg[23] ? 4 * g_dbg[23] : (fills8 && (H >= 4096 || rows < 48.0)) || (h->wbits == 8 && rows < 56.0) ? 8 : 4;
   const bool use_rt = mt == 4 && g_dbg[4] == 3;   // register-tile kernels (256-row tiles): parity-tested, not yet timed
   if (use_rt) { mt = 16; use_stream = false; }
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
@@ -2475,9 +2476,9 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
   // 19: 1946 | 1903, 31: 2298 | 2185, 47: 2795 | 2641, 64: 3338 | 3012; 64 of 6144 x 3072, 15: 597 | 618, 37: 821 | 798, 94: 1243 | 1175; 128 of 5120 x 2048, 31: 875 | 828; 64 of
   // 2048 x 1408, 28: 148 | 152, 48: 170 | 163, 75: 225 | 197, 192: 408 | 378; 64 of 2560 x 2048, 50: 294 | 276; 128 of 2048 x 512, 128: 289 | 257; with few workgroups either may be
   // ahead: 8 of 4096 x 1536, 70 (300): 69 | 76, 100 (396): 88 | 75; 8 of 6144 x 3072, 100 (792): 200 | 209; 32 of 2560 x 1024, 50 (656): 83 | 89, 125 (1256): 164 | 146.
-  // Dev knob [6] (tests): 1 = never, 2 = always.
+  // Dev knob [24] (tests): 1 = never, 2 = always.
   const bool fills = (std::min(npairs, E) + npairs / 32) * (I / 128) >= 1200 && rows >= ((size_t)H * I >= ((size_t)8 << 20) ? 24.0 : 48.0);
-  const bool stream = fp8 && g_dbg[6] != 1 && (g_dbg[6] == 2 || fills) && fp8_stream_lds(std::max(H, I)) <= 160 * 1024;
+  const bool stream = fp8 && g_dbg[24] != 1 && (g_dbg[24] == 2 || fills) && fp8_stream_lds(std::max(H, I)) <= 160 * 1024;
   const int mt = stream ? 2 : rows <= 8.0 ? 1 : rows <= 60.0 ? 2 : 4;
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
 

@@ -73,7 +73,7 @@ def test_ping_pong_tile_race_screen(M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(1, 8, 64), (256, 192, 128), (257, 200, 192), (1000, 1160, 1536), (2048, 6152, 4096)])
 def test_ping_pong_tile_of_192_columns(M, N, K):
-    """Variant 5 with 192 and with 256 columns a workgroup (dev knob 7 = 3 and 4), repeated, with bias and with fp32 output: the bits of variant 2 (the same k order)."""
+    """Variant 5 with 192 and with 256 columns a workgroup (dev knob 31 = 3 and 4), repeated, with bias and with fp32 output: the bits of variant 2 (the same k order)."""
     from ktransformers_amd import _native
     from ktransformers_amd._native import gemm_bf16_nt
     g = torch.Generator(device="cpu").manual_seed(M + N + K)
@@ -83,11 +83,11 @@ def test_ping_pong_tile_of_192_columns(M, N, K):
     ref = [gemm_bf16_nt(a, b, variant=2), gemm_bf16_nt(a, b, bias=bias, variant=2), gemm_bf16_nt(a, b, out_f32=True, variant=2)]
     try:
         for knob in (3, 4, 3, 3):
-            _native.lib.ktx_debug_set(7, knob)
+            _native.lib.ktx_debug_set(31, knob)
             got = [gemm_bf16_nt(a, b, variant=5), gemm_bf16_nt(a, b, bias=bias, variant=5), gemm_bf16_nt(a, b, out_f32=True, variant=5)]
             assert all(torch.equal(x, y) for x, y in zip(got, ref)), knob
     finally:
-        _native.lib.ktx_debug_set(7, 0)
+        _native.lib.ktx_debug_set(31, 0)
 
 
 @pytest.mark.parametrize("B,M,N,K,columns", [
@@ -108,15 +108,19 @@ def test_columns_follow_the_rounds_of_the_busiest_xcd(B, M, N, K, columns):
 
 @pytest.mark.parametrize("K,N,T,columns", [(1536, 24576, 1000, 192), (2048, 18688, 1280, 256), (2048, 20480, 1792, 256), (4096, 12000, 700, 192)])
 def test_columns_of_a_linear(K, N, T, columns):
-    """The same on a bf16 linear's tiles."""
+    """The same on a bf16 linear's tiles; the knobs of an MLA sweep (workgroup shape, splits) do not move it."""
     from ktransformers_amd import _native as n
     h = n.LinearHandle(K, N, "BF16", 0, T, torch.device(DEV))
     h.load_bf16(torch.zeros((N, K), dtype=torch.bfloat16, device=DEV))
     n.timing_enable(2)
     try:
+        for idx in (6, 7):
+            n.lib.ktx_debug_set(idx, 4 if columns == 192 else 3)
         h.forward(torch.zeros((T, K), dtype=torch.bfloat16, device=DEV))
         labels = [t[0] for t in n.timing_collect() if t[0].startswith("gemm256_bf16_nt_kernel<")]
     finally:
+        for idx in (6, 7):
+            n.lib.ktx_debug_set(idx, 0)
         n.timing_enable(0)
     assert len(labels) == 1 and labels[0].endswith(f", {columns} columns"), labels
 
@@ -132,10 +136,10 @@ def test_ping_pong_tiles_of_batches(B, M, N, K):
     ref = [gemm_bf16_nt(a, b, variant=2, out_f32=f) for f in (False, True)]
     try:
         for knob in (3, 4):
-            _native.lib.ktx_debug_set(7, knob)
+            _native.lib.ktx_debug_set(31, knob)
             assert all(torch.equal(gemm_bf16_nt(a, b, variant=5, out_f32=f), r) for f, r in zip((False, True), ref)), knob
     finally:
-        _native.lib.ktx_debug_set(7, 0)
+        _native.lib.ktx_debug_set(31, 0)
 
 
 @pytest.mark.parametrize("T,K,N", [(300, 1536, 24576), (700, 4096, 12000)])
@@ -149,10 +153,10 @@ def test_linear_tiles_of_192_columns(T, K, N):
     got = []
     try:
         for knob in (4, 3):
-            _native.lib.ktx_debug_set(7, knob)
+            _native.lib.ktx_debug_set(31, knob)
             got.append(h.forward(x).clone())
     finally:
-        _native.lib.ktx_debug_set(7, 0)
+        _native.lib.ktx_debug_set(31, 0)
     assert torch.equal(*got)
 
 

@@ -844,7 +844,7 @@ def test_w4_prompts_off_the_gemm_multiply_exact_integers(G, K, N, T, how):
 @pytest.mark.parametrize("K,N,T", [(4096, 12000, 33), (4096, 10244, 64), (16384, 5130, 48),   # 188, 164 and 168 workgroups; whole strips, a part of one, rows absent
                                    (2176, 32768, 33), (2944, 32641, 64), (2944, 32640, 48)])   # 64 x 128 tiles on all CUs, which add the pieces of K themselves; and on one less
 def test_tiles_of_64_rows_and_256_features(fmt, group, K, N, T):
-    """The 64 x 256 tiles against the 64 x 128 ones (dev knob 7 = 6): the same pieces of K, the same bits."""
+    """The 64 x 256 tiles against the 64 x 128 ones (dev knob 32 = 1): the same pieces of K, the same bits."""
     from ktransformers_amd import _native
     g = torch.Generator().manual_seed(K + N + T)
     dev = torch.device("cuda", 0)
@@ -856,12 +856,12 @@ def test_tiles_of_64_rows_and_256_features(fmt, group, K, N, T):
     x = torch.randn((T, K), generator=g).to(torch.bfloat16).to(dev)
     got = []
     try:
-        for knob in (6, 0):
-            _native.lib.ktx_debug_set(7, knob)
+        for knob in (1, 0):
+            _native.lib.ktx_debug_set(32, knob)
             h._ws_need.clear()
             got.append(h.forward(x).clone())
     finally:
-        _native.lib.ktx_debug_set(7, 0)
+        _native.lib.ktx_debug_set(32, 0)
     assert torch.equal(*got)
 
 

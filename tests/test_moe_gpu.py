@@ -796,7 +796,7 @@ def test_fp_grouped_edges(oracle, dev, fmt, H, I, rows):
 @pytest.mark.parametrize("H,I", [(128, 128), (384, 640), (1152, 1664), (2048, 512)])   # 1, 3, 5, 9, 13, 16 and 4 k-steps: chunks of 4, with and without a rest
 @pytest.mark.parametrize("rows", [(1, 16, 17, 0, 32), (33, 0, 65, 48)])
 def test_fp8_streaming_groups(dev, H, I, rows):
-    """moe_fp8_stream_kernel (dev knob 6 = 2) against the chunk-pipelined kernels (1), which test_fp_grouped_edges holds to the oracle: bit for bit."""
+    """moe_fp8_stream_kernel (dev knob 24 = 2) against the chunk-pipelined kernels (1), which test_fp_grouped_edges holds to the oracle: bit for bit."""
     from helpers import fp8_block_quant
     from ktransformers_amd import _native
     E, k, T = len(rows), 1, sum(rows)
@@ -809,11 +809,11 @@ def test_fp8_streaming_groups(dev, H, I, rows):
         _native.force_generic_path(True)
         got = []
         for knob in (1, 2):
-            _native.lib.ktx_debug_set(6, knob)
+            _native.lib.ktx_debug_set(24, knob)
             got.append(run(h, c, dev))
         assert np.array_equal(*got), f"{int((got[0] != got[1]).sum())} outputs differ"
     finally:
-        _native.lib.ktx_debug_set(6, 0)
+        _native.lib.ktx_debug_set(24, 0)
         _native.force_generic_path(False)
         h.close()
 
@@ -822,7 +822,7 @@ def test_fp8_streaming_groups(dev, H, I, rows):
 @pytest.mark.parametrize("H,I", [(1152, 1664), (2048, 512)])   # 9 and 13 k-steps (chunks of 4 and 8, with a rest), 16 and 4; strip groups that are not full
 @pytest.mark.parametrize("rows", [(16, 17, 33, 49, 130), (1, 64, 65, 128)])   # each count of 16-row groups, alone and behind a full tile
 def test_int_streaming_groups(oracle, dev, method, H, I, rows):
-    """moe_gemm_stream_kernel with 4 and with 8 wavefronts a workgroup (dev knob 5), bit for bit."""
+    """moe_gemm_stream_kernel with 4 and with 8 wavefronts a workgroup (dev knob 23), bit for bit."""
     from ktransformers_amd import _native
     E, k, T = len(rows), 1, sum(rows)
     c = make_case(47, E, k, H, I, T)
@@ -833,12 +833,12 @@ def test_int_streaming_groups(oracle, dev, method, H, I, rows):
         _native.force_generic_path(True)
         _native.lib.ktx_debug_set(4, 2)
         for knob in (1, 2):
-            _native.lib.ktx_debug_set(5, knob)
+            _native.lib.ktx_debug_set(23, knob)
             got = run(h, c, dev)
             assert np.array_equal(got, want), f"{int((got != want).sum())} outputs differ ({4 * knob} wavefronts)"
     finally:
         _native.lib.ktx_debug_set(4, 0)
-        _native.lib.ktx_debug_set(5, 0)
+        _native.lib.ktx_debug_set(23, 0)
         _native.force_generic_path(False)
         h.close()
 
