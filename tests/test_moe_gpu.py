@@ -563,13 +563,13 @@ def test_forward_side_equals_the_separate_launches(dev, method, shape):
 @pytest.mark.parametrize("shape", [(64, 6, 256, 128, 700), (256, 8, 256, 128, 2048), (8, 2, 256, 256, 1500), (16, 4, 256, 128, 100)])
 def test_bucketing_is_the_reference_stable_order(oracle, dev, shape, dup):
     """a5: the (token, slot) -> sorted-row map of the grouped path is the reference's m_local_pos_ (token-major arrival rank
-    inside each expert, experts in ascending order; moe_base.hpp:208-227) — the wavefront-ballot counting sort of
-    moe_prep_kernel is deterministic, so the map can be compared entry by entry with the oracle's bucketing, twice."""
+    inside each expert, experts in ascending order; moe_base.hpp:208-227): moe_prep_kernel ranks an expert's pairs in the
+    table's order, so the map can be compared entry by entry with the oracle's bucketing, twice."""
     import ctypes as C
     from ktransformers_amd import _native as n
     E, k, H, I, T = shape
     c = make_case(7, E, k, H, I, T, invalid_ids=True)
-    if dup:   # a token that names one expert twice: the bitmap scatter hands over to the ballot counting sort
+    if dup:   # a token that names one expert twice
         c["ids"][T // 2, 1] = c["ids"][T // 2, 0]
         c["ids"][T - 2, k - 1] = c["ids"][T - 2, 0]
     h = make_handle("AMXINT4", c, E, k, H, I, T, dev)
@@ -795,17 +795,19 @@ def test_fp_grouped_edges(oracle, dev, fmt, H, I, rows):
 
 @pytest.mark.parametrize("H,I", [(128, 128), (384, 640), (1152, 1664), (2048, 512)])   # 1, 3, 5, 9, 13, 16 and 4 k-steps: chunks of 4, with and without a rest
 @pytest.mark.parametrize("rows", [(1, 16, 17, 0, 32), (33, 0, 65, 48)])
-def test_fp8_streaming_groups(dev, H, I, rows):
-    """moe_fp8_stream_kernel (dev knob 24 = 2) against the chunk-pipelined kernels (1), which test_fp_grouped_edges holds to the oracle: bit for bit."""
-    from helpers import fp8_block_quant
+@pytest.mark.parametrize("method", ["FP8", "FP8_PERCHANNEL"])
+def test_fp8_streaming_groups(dev, method, H, I, rows):
+    """moe_fp8_stream_kernel (dev knob 24 = 2) against the chunk-pipelined kernels (1), which test_fp_grouped_edges holds to the oracle: bit for bit, with scales of blocks
+    and with scales of rows, each its own."""
+    from helpers import fp8_block_quant, fp8_perchannel_quant
     from ktransformers_amd import _native
     E, k, T = len(rows), 1, sum(rows)
     c = make_case(53, E, k, H, I, T)
     c["ids"] = np.random.default_rng(T).permutation(np.repeat(np.arange(E), rows)).astype(np.int64)[:, None]
-    h = _native.MoEHandle(E, k, H, I, max_len=T, method="FP8", device=0, group_size=128)
+    h = _native.MoEHandle(E, k, H, I, max_len=T, method=method, device=0, group_size=128 if method == "FP8" else 0)
     try:
-        q = [fp8_block_quant(bf16_to_f32(c[n])) for n in ("gate", "up", "down")]
-        h.load_fp8(*[torch.from_numpy(x[0]).to(dev) for x in q], *[torch.from_numpy(x[1]).to(dev) for x in q])
+        q = [(fp8_block_quant if method == "FP8" else fp8_perchannel_quant)(bf16_to_f32(c[n])) for n in ("gate", "up", "down")]
+        (h.load_fp8 if method == "FP8" else h.load_fp8_perchannel)(*[torch.from_numpy(x[0]).to(dev) for x in q], *[torch.from_numpy(x[1]).to(dev) for x in q])
         _native.force_generic_path(True)
         got = []
         for knob in (1, 2):
