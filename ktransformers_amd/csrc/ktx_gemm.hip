@@ -482,9 +482,12 @@ int launch_gemm256_nb(GemmParams p, int batch, hipStream_t st) {
 // 149 | 182.  Plain operands (rows x columns x K): 4096 x 3072 x 2048 51 | 46, fp32 56 | 49; 6000 x 2304 x 2048 90 | 79; 4864 x 4864 x 2048 (2 | 3, 2 | 2) 101 | 125.  Batches: 8 of 1024 x 1536 x 2048
 // 62 | 53; 16 of 512 x 1536 x 1024 36 | 33; 2 of 2048 x 3000 x 2048 52 | 47; 4 of 4096 x 1536 x 1024 (2 | 4, 2 | 2: a batch entry's four supertiles begin with the first XCD) 61 | 92; 4 of
 // 2048 x 1536, K 1024, 2048, 4096: 31.7 | 30.7, 54.2 | 56.6, 98 | 95.  The chip's count beside the XCD's: supertiles at the edge are not full, 2 of 5632 x 2432 x 2048 (4 | 4, of the chip 2 | 3) 139 | 159.
+// On a linear's tiles only to 3072 of K, a part's where K is in parts: B comes in pieces from four tiles, and past it 192 columns lose.  1536 -> 12288, 1024 rows 39.4 | 39.4, 3072 -> 12288 70.0 | 70.2, 3456
+// -> 12288 76.9 | 77.9, 7168 -> 12288 151 | 153 (plain operands 91.4 | 85.3 at 4096, 154 | 145 at 7168); 700 in 2 parts: 4096 -> 12288 116 | 112, 5120 -> 11944 138 | 132, 7168 -> 11944 186 | 188.
 // Dev knob 31 (tests): 3 or 4 fragments.
-inline int gemm256_fragments(const GemmParams& p, int batch) {
+inline int gemm256_fragments(const GemmParams& p, int batch, bool tiles) {
   if (const int force = ktx_debug_get(31)) return force == 3 ? 3 : 4;
+  if (tiles && p.K > 3072) return 4;
   const Gemm256Grid g4 = gemm256_grid(p, 256, batch), g3 = gemm256_grid(p, 192, batch);
   auto of_chip = [&](const Gemm256Grid& g) { return ((long)g.tm * g.tn * batch + 255) / 256; };
   return g3.rounds <= g4.rounds && of_chip(g3) <= of_chip(g4) ? 3 : 4;
@@ -492,7 +495,7 @@ inline int gemm256_fragments(const GemmParams& p, int batch) {
 
 template <bool F32OUT, bool BTILES = false>
 int launch_gemm256(const GemmParams& p, int batch, hipStream_t st) {
-  if (gemm256_fragments(p, batch) == 3) return launch_gemm256_nb<F32OUT, BTILES, 3>(p, batch, st);
+  if (gemm256_fragments(p, batch, BTILES) == 3) return launch_gemm256_nb<F32OUT, BTILES, 3>(p, batch, st);
   return launch_gemm256_nb<F32OUT, BTILES, 4>(p, batch, st);
 }
 
@@ -569,7 +572,7 @@ extern "C" int ktx_gemm_bf16_nt(const ktx_gemm_args* a, ktx_stream_t stream) {
   const double na = a->a_bs ? a->batch : 1, nb = a->b_bs ? a->batch : 1;   // a shared operand is counted once
   KTX_TIMED(st, ((double)a->M * a->K * na + (double)a->N * a->K * nb) * 2 + (double)a->M * a->N * a->batch * (a->out_f32 ? 4 : 2),
             "gemm_bf16_nt_kernel<%d,%s> %dx%dx%d b%d, %d columns", variant, a->out_f32 ? "f32" : "bf16", a->M, a->N, a->K, a->batch,
-            variant == 5 ? 64 * gemm256_fragments(p, a->batch) : 128);
+            variant == 5 ? 64 * gemm256_fragments(p, a->batch, false) : 128);
   const bool f = a->out_f32 != 0;
   if (variant == 5) {
     KTX_REQUIRE((size_t)a->M * a->lda * 2 < ((size_t)1 << 32) && (size_t)a->N * a->ldb * 2 < ((size_t)1 << 32),
@@ -597,7 +600,7 @@ int ktx_gemm256_tiles(int M, int N, int K, int nsplit, const bf16_t* A, long lda
   p.B = reinterpret_cast<const bf16_t*>(tiles); p.ldb = nks; p.b_bs = (long)(p.K / 128) * 2048;
   p.Y = Y; p.ldy = ldy; p.y_bs = y_bs;
   KTX_TIMED(st, (double)nks * ((N + 15) / 16) * 4096.0 + (double)M * K * 2.0 + (double)M * N * nsplit * (out_f32 ? 4 : 2),
-            "gemm256_bf16_nt_kernel<%s,tiles> %dx%dx%d splits %d, %d columns", out_f32 ? "f32" : "bf16", M, N, K, nsplit, 64 * gemm256_fragments(p, nsplit));
+            "gemm256_bf16_nt_kernel<%s,tiles> %dx%dx%d splits %d, %d columns", out_f32 ? "f32" : "bf16", M, N, K, nsplit, 64 * gemm256_fragments(p, nsplit, true));
   return out_f32 ? launch_gemm256<true, true>(p, nsplit, st) : launch_gemm256<false, true>(p, nsplit, st);
 }
 

@@ -106,9 +106,9 @@ def test_columns_follow_the_rounds_of_the_busiest_xcd(B, M, N, K, columns):
     assert len(labels) == 1 and labels[0].startswith("gemm_bf16_nt_kernel<5,") and labels[0].endswith(f", {columns} columns"), labels
 
 
-@pytest.mark.parametrize("K,N,T,columns", [(1536, 24576, 1000, 192), (2048, 18688, 1280, 256), (2048, 20480, 1792, 256), (4096, 12000, 700, 192)])
+@pytest.mark.parametrize("K,N,T,columns", [(1536, 24576, 1000, 192), (2048, 18688, 1280, 256), (2048, 20480, 1792, 256), (4096, 12000, 700, 192), (3072, 12288, 1000, 192), (3456, 12288, 1000, 256), (7168, 11944, 700, 256)])
 def test_columns_of_a_linear(K, N, T, columns):
-    """The same on a bf16 linear's tiles; the knobs of an MLA sweep (workgroup shape, splits) do not move it."""
+    """The same on a bf16 linear's tiles, and to 3072 of K (a part's: 4096 and 7168 go in two); the knobs of an MLA sweep (workgroup shape, splits) do not move it."""
     from ktransformers_amd import _native as n
     h = n.LinearHandle(K, N, "BF16", 0, T, torch.device(DEV))
     h.load_bf16(torch.zeros((N, K), dtype=torch.bfloat16, device=DEV))
