@@ -29,19 +29,22 @@
 //   multiplies while the other waits: 8 wavefronts on 128 rows are 2 to 20 % slower, though no expert of 65 .. 128 rows is widened twice).  K walks in the RAW
 //   step of 512: its weights go through the LDS into registers (the LDS holds the next step's meanwhile: two steps in registers leave none for
 //   the sums of two rounds), the activations in quarters of it, all by LDS-DMA.
-// At Kimi-K2's sizes, us for the whole forward, weights of two steps in registers and each round's sums directly behind its MFMAs -> here (the same bits): 64 tokens 956 ->
-// 931, 500 1988 -> 1968, 2048 4153 -> 4091; 64 experts of 2048 x 1024, top-8: 200 tokens 137 -> 128, 360 169 -> 160, 2048 543 -> 514.
+// At Kimi-K2's sizes, us for the whole forward, weights of two steps in registers and each round's sums directly behind its MFMAs -> here (the same bits): 64 tokens 949 ->
+// 883, 500 2027 -> 1910, 2048 4254 -> 3982; 64 experts of 2048 x 1024, top-8: 130 tokens 118 -> 111, 360 170 -> 156, 2048 537 -> 493; 8 of 4096 x 1536, top-2: 64 tokens 74.2 -> 74.4,
+// 300 116 -> 106.  With the nibbles shifted to one place (12 instructions a widened dword, 10 here): 931, 1968, 4091, 115, 160, 514, 76, 110.
 // =====================================================================================================
 // the pairs (byte 0, byte 2) and (byte 1, byte 3) of the low (par 0) or high nibbles of x as q; x: two's complement nibbles.
-// A nibble (its top bit turned: q + 8) becomes bits 6..9 of an f16 of exponent 2^7: 128 + 8 (q + 8), an eighth of which less 24 is q.
+// A nibble (its top bit turned: q + 8) becomes mantissa bits 0..3 or 4..7 of an f16 of exponent 2^10 where it lies, or after a shift by a byte:
+// 1024 + (q + 8), or 1024 + 16 (q + 8).
 template <int PAR>
-__device__ __forceinline__ void raw_widen(uint32_t x, uint32_t mask, uint32_t top, uint32_t& o0, uint32_t& o1) {
+__device__ __forceinline__ void raw_widen(uint32_t x, const uint32_t (&mask)[2], const uint32_t (&top)[2], uint32_t& o0, uint32_t& o1) {
   auto value = [&](uint32_t e) {
-    const raw_h2 eighth = {(_Float16)0.125f, (_Float16)0.125f}, m24 = {(_Float16)-24.0f, (_Float16)-24.0f};
-    return raw_h2_bits(__builtin_elementwise_fma(__builtin_bit_cast(raw_h2, (e & mask) ^ top), eighth, m24));
+    const raw_h2 v = __builtin_bit_cast(raw_h2, (e & mask[PAR]) ^ top[PAR]);
+    if constexpr (PAR == 0) return raw_h2_bits(v + raw_h2{(_Float16)-1032.0f, (_Float16)-1032.0f});
+    else return raw_h2_bits(__builtin_elementwise_fma(v, raw_h2{(_Float16)0.0625f, (_Float16)0.0625f}, raw_h2{(_Float16)-72.0f, (_Float16)-72.0f}));
   };
-  if constexpr (PAR == 0) { o0 = value(x << 6); o1 = value(x >> 2); }
-  else { o0 = value(x << 2); o1 = value(x >> 6); }
+  o0 = value(x);
+  o1 = value(x >> 8);
 }
 
 // 4 wavefronts of one strip (x gate, up; or two strips of down) each, up to RAW_ROWS rows of one expert.
@@ -139,9 +142,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   const uint32_t xo0 = i * 256 + ((kc ^ i) * 16);   // row i's piece kc; piece 4 g + kc: ^ 64 g
   // constants the compiler cannot see through: and + xor become one v_bitop3_b32
-  uint32_t mask, top;
-  asm("s_mov_b32 %0, 0x03C003C0" : "=s"(mask));
-  asm("v_mov_b32 %0, 0x5A005A00" : "=v"(top));      // 128 = 0x5800, and the nibble's top bit (0x0200) turned
+  uint32_t mask[2], top[2];
+  asm("s_mov_b32 %0, 0x000F000F" : "=s"(mask[0]));
+  asm("s_mov_b32 %0, 0x00F000F0" : "=s"(mask[1]));
+  asm("v_mov_b32 %0, 0x64086408" : "=v"(top[0]));   // 1024 = 0x6400, and the nibble's top bit turned
+  asm("v_mov_b32 %0, 0x64806480" : "=v"(top[1]));
 
   // MTL = 16-row groups of the tile that hold rows; one instantiation per count, chosen once per workgroup.
   auto run = [&](auto mtl) __attribute__((always_inline)) {
