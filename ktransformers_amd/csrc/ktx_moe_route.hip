@@ -46,8 +46,9 @@ __device__ __forceinline__ void quant_row_256(bool live, const bf16_t* __restric
 
 // Rows of an expert lie in (token, slot) order — the reference's m_local_pos_ (moe_base.hpp:208-227): the row of a pair depends on the routing table only.
 // A workgroup reads the whole table: it counts all experts' pairs (LDS), which gives its expert's first row and first tile, then ranks its own expert's pairs, a
-// stretch of the table per wavefront, by ballots.  No workgroup waits for another.  One workgroup for all experts took 53 us for 2048 tokens, top-8, 256 experts (a
-// CU's vector ALU and LDS: 16384 pairs, three passes), E of them 22; 1000 tokens 24 -> 14, 32 tokens 12.7 -> 5.5, 500 tokens of 8 experts, top-2, 24 -> 7.
+// stretch of the table per wavefront, by ballots; a stretch of up to 512 pairs is read once.  No workgroup waits for another.  Us, one workgroup for all experts (a CU's vector ALU and
+// LDS, three passes) -> E of them that read the table twice -> here: 256 experts, top-8, 2048 tokens 45 -> 19.6 -> 19.6, 1000 24.1 -> 12.1 -> 10.9, 32 10.5 -> 4.7 -> 4.2; 64, top-6, 300
+// 7.7 -> 7.4 -> 6.2; 8, top-2, 1000 8.0 -> 8.3 -> 7.4, 500 5.9 -> 6.6 -> 6.2, 100 4.6 -> 5.0 -> 4.3 (with the tokens' int8 rows beside).
 __global__ __launch_bounds__(PREP_THREADS) void moe_prep_kernel(PrepParams p) {
   __shared__ int s_cnt[KTX_EMAX];
   __shared__ float s_red[PREP_THREADS / 64];
@@ -69,26 +70,30 @@ __global__ __launch_bounds__(PREP_THREADS) void moe_prep_kernel(PrepParams p) {
     id -= p.expert_begin;
     return (id >= 0 && id < E && !(p.mask && p.mask[id])) ? (int)id : -1;
   };
-  auto for_pairs = [&](auto&& f) {   // f(pair, expert; -1: none, -2: no pair) for the wavefront's stretch, 64 pairs after the other
-    constexpr int U = 8;
-    for (int base = i0; base < i1; base += U * 64) {
-      long long id[U];
+  constexpr int U = 8;
+  int ex[U];   // of 64 pairs each: the expert, -1: none, -2: no pair
+  auto fetch = [&](int base) {
+    long long id[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) id[u] = p.ids[min(base + u * 64 + lane, npairs - 1)];
+    for (int u = 0; u < U; u++) id[u] = p.ids[min(base + u * 64 + lane, npairs - 1)];
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int i = base + u * 64 + lane;
-        if (base + u * 64 < i1) f(i, i < i1 ? expert(id[u]) : -2);
-      }
+    for (int u = 0; u < U; u++) {
+      if (base + u * 64 >= i1) break;
+      ex[u] = base + u * 64 + lane < i1 ? expert(id[u]) : -2;
     }
   };
   for (int e = tid; e < E; e += blockDim.x) s_cnt[e] = 0;
   __syncthreads();
   int mine = 0;   // this wavefront's pairs of this workgroup's expert
-  for_pairs([&](int, int e) {
-    if (e >= 0) atomicAdd(&s_cnt[e], 1);   // (an integer sum: the order of the adds does not matter)
-    mine += __popcll(__ballot(e == me));
-  });
+  for (int base = i0; base < i1; base += U * 64) {
+    fetch(base);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (base + u * 64 >= i1) break;
+      if (ex[u] >= 0) atomicAdd(&s_cnt[ex[u]], 1);   // (an integer sum: the order of the adds does not matter)
+      mine += __popcll(__ballot(ex[u] == me));
+    }
+  }
   __syncthreads();
   auto tiles_of = [&](int c) { return (c + p.rows_per_tile - 1) / p.rows_per_tile; };
   {   // rows and tiles of the experts before this one, and of all
@@ -118,17 +123,23 @@ __global__ __launch_bounds__(PREP_THREADS) void moe_prep_kernel(PrepParams p) {
   if (me == 0 && tid == 0) { p.counters[0] = sum[3]; p.counters[1] = sum[2]; }
   run += row0;
   if (mine || me == 0)
-    for_pairs([&](int i, int e) {
-      const unsigned long long m = __ballot(e == me);
-      if (e == me) {
-        const int r = run + __popcll(m & ((1ull << lane) - 1ull));
-        p.src_of_row[r] = i / p.k;
-        p.row_of_pair[i] = r;
-      } else if (me == 0 && e == -1) {
-        p.row_of_pair[i] = -1;
+    for (int base = i0; base < i1; base += U * 64) {
+      if (per_wave > U * 64) fetch(base);   // (a stretch of one step is still there)
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (base + u * 64 >= i1) break;
+        const int i = base + u * 64 + lane;
+        const unsigned long long m = __ballot(ex[u] == me);
+        if (ex[u] == me) {
+          const int r = run + __popcll(m & ((1ull << lane) - 1ull));
+          p.src_of_row[r] = i / p.k;
+          p.row_of_pair[i] = r;
+        } else if (me == 0 && ex[u] == -1) {
+          p.row_of_pair[i] = -1;
+        }
+        run += __popcll(m);
       }
-      run += __popcll(m);
-    });
+    }
   for (int i = tid; i < ntiles; i += blockDim.x) {
     Tile t;
     t.expert = me; t.row0 = row0 + i * p.rows_per_tile; t.nrows = min(p.rows_per_tile, cnt - i * p.rows_per_tile); t.idx = i; t.cnt = ntiles;
@@ -145,9 +156,9 @@ hipError_t moe_launch_prep(const PrepParams& p, bool quantise, hipStream_t st) {
 // =====================================================================================================
 // K3: weighted combine in slot order (a12) + merge/incremental + bf16 (a4)
 // =====================================================================================================
-// What it costs is the rows' way in, so a thread's loads are V elements wide and all experts of a token (8 at a time) are asked for before the first is
-// used.  2048 rows of 7168, top-8: 60 -> 49 us (5.4 TB/s); 1000: 34 -> 28 (4 elements a thread, one expert after the other, before).
-template <int V, bool F32>
+// What it costs is the rows' way in, so a thread's loads are V elements wide and U experts of a token are asked for before the first is used.  Us, 4 elements a thread, one expert
+// after the other -> here: 2048 rows of 7168, top-8, 52 -> 43 (6.1 TB/s); 1000 23.4 -> 21.9; 2048 of 4096, top-2, 11.6 -> 10.4.
+template <int V, bool F32, int U>
 __global__ __launch_bounds__(128) void moe_combine_kernel(CombineParams p) {
   int T = p.qlen;
   if (p.d_bsz) T = min(max(*p.d_bsz, 0), p.qlen);
@@ -161,18 +172,18 @@ __global__ __launch_bounds__(128) void moe_combine_kernel(CombineParams p) {
   float acc[V];
 #pragma unroll
   for (int e = 0; e < V; e++) acc[e] = 0.f;
-  for (int j0 = 0; j0 < p.k; j0 += 8) {
-    int r[8];
-    float ws[8];
-    uint2 v[8][NQ];
+  for (int j0 = 0; j0 < p.k; j0 += U) {
+    int r[U];
+    float ws[U];
+    uint2 v[U][NQ];
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
+    for (int u = 0; u < U; u++) {
       const int j = min(j0 + u, p.k - 1), row = rows[j];
       ws[u] = weights[j];
       r[u] = j0 + u < p.k ? row : -1;
     }
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
+    for (int u = 0; u < U; u++) {
       if (r[u] < 0) continue;
       const uint8_t* src = reinterpret_cast<const uint8_t*>(p.dn) + ((size_t)r[u] * p.H + h) * (F32 ? 4 : 2);
       if constexpr (NQ >= 2) {
@@ -187,7 +198,7 @@ __global__ __launch_bounds__(128) void moe_combine_kernel(CombineParams p) {
       }
     }
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
+    for (int u = 0; u < U; u++) {
       if (r[u] < 0) continue;
       const float w = ws[u];
 #pragma unroll
@@ -228,13 +239,20 @@ __global__ __launch_bounds__(128) void moe_combine_kernel(CombineParams p) {
   }
 }
 
-// 8 elements a thread where rows lie on 16 bytes (H a multiple of 8 and the rows' address), 4 otherwise; fp32 rows of 4 elements are 16 bytes wide as well
-hipError_t moe_launch_combine(const CombineParams& p, hipStream_t st) {
-  const bool wide = p.H % 8 == 0 && (reinterpret_cast<uintptr_t>(p.dn) & 15) == 0;
-  const dim3 g4((p.H / 4 + 127) / 128, p.qlen), g8((p.H / 8 + 127) / 128, p.qlen);
-  if (p.dn_f32) hipLaunchKernelGGL((moe_combine_kernel<4, true>), g4, dim3(128), 0, st, p);
-  else if (wide) hipLaunchKernelGGL((moe_combine_kernel<8, false>), g8, dim3(128), 0, st, p);
-  else hipLaunchKernelGGL((moe_combine_kernel<4, false>), g4, dim3(128), 0, st, p);
-  return hipGetLastError();
+// U: the experts of a token, as 2, 4 or 8 (what is asked for in vain, and its code, shows in short calls: 500 tokens of 4096, top-2, U 8 4.8 us, 2: 4.4)
+template <int V, bool F32>
+static void launch_combine(const CombineParams& p, hipStream_t st) {
+  const dim3 g((p.H / V + 127) / 128, p.qlen);
+  if (p.k <= 2) hipLaunchKernelGGL((moe_combine_kernel<V, F32, 2>), g, dim3(128), 0, st, p);
+  else if (p.k <= 4) hipLaunchKernelGGL((moe_combine_kernel<V, F32, 4>), g, dim3(128), 0, st, p);
+  else hipLaunchKernelGGL((moe_combine_kernel<V, F32, 8>), g, dim3(128), 0, st, p);
 }
 
+// 8 elements a thread where rows lie on 16 bytes (H a multiple of 8 and the rows' address) and there are enough of them for the CUs, 4 otherwise (100 tokens of 4096, top-2, 8 | 4 elements:
+// 3.6 | 3.2 us, 64 of 2048, top-6: 4.6 | 4.0; 300 of 4096, top-2 about even); fp32 rows of 4 elements are 16 bytes wide as well
+hipError_t moe_launch_combine(const CombineParams& p, hipStream_t st) {
+  if (p.dn_f32) launch_combine<4, true>(p, st);
+  else if ((size_t)p.qlen * p.H >= ((size_t)1 << 20) && p.H % 8 == 0 && (reinterpret_cast<uintptr_t>(p.dn) & 15) == 0) launch_combine<8, false>(p, st);
+  else launch_combine<4, false>(p, st);
+  return hipGetLastError();
+}

@@ -595,6 +595,28 @@ def _memcpy_d2d(dst, src, nbytes):
     return hip.hipMemcpy(dst, src, nbytes, 3)
 
 
+@pytest.mark.parametrize("T,H", [(3, 4), (5, 1032), (300, 4096), (300, 4100)])   # few elements and many, rows on 16 bytes and on 8
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 8, 9, 17])
+def test_combine_of_any_number_of_experts(dev, T, H, k):
+    """ktx_moe_combine is the slot-ordered chain of fp32 fmas, rounded to bf16 once, for every width and count that its kernels are built for; skipped slots, all of them in one
+    token; with and without the output of before."""
+    from ktransformers_amd._native import moe_combine
+    r = np.random.default_rng(T + H + k)
+    rows = f32_to_bf16(r.standard_normal((T * k, H)).astype(np.float32))
+    pair = r.permutation(T * k).astype(np.int32).reshape(T, k)
+    pair[r.random((T, k)) < 0.2] = -1
+    pair[1] = -1
+    w = r.standard_normal((T, k)).astype(np.float32)
+    before = f32_to_bf16(r.standard_normal((T, H)).astype(np.float32))
+    acc = np.zeros((T, H), np.float32)
+    for j in range(k):
+        live = pair[:, j] >= 0
+        acc[live] = (bf16_to_f32(rows[pair[live, j]]).astype(np.longdouble) * w[live, j, None] + acc[live]).astype(np.float32)   # (a product of 32 bits and a sum of 24: exact before the rounding)
+    args = torch_bf16(rows, dev), torch.from_numpy(pair).to(dev), torch.from_numpy(w).to(dev)
+    assert np.array_equal(numpy_u16(moe_combine(*args)), f32_to_bf16(acc))
+    assert np.array_equal(numpy_u16(moe_combine(*args, out=torch_bf16(before, dev), incremental=True)), f32_to_bf16(acc + bf16_to_f32(before)))
+
+
 @pytest.mark.parametrize("H,I", [(512, 1536), (1536, 512)])
 def test_rawint4_rows_per_tile_and_any_scale(oracle, dev, H, I):
     """Short batches: the exact kernel's work follows a tile's rows (1, 2, 3, 4 and a 4-row tile behind them) and takes any number of 512-k
