@@ -2388,7 +2388,9 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
   // 278 | 279 | 264, 62: 307 | 299 | 285; 16 of 6144 x 2048, 62: 111 | 122 | 119, 87: 140 | 132 | 129, 125: 166 | 163 | 153, 250: 260 | 262 | 240; 64 of 3072 x 3072,
   // 125: 465 | 442 | 433; 128 of 4096 x 1536, 50: 382 | 374 | 360; 8 of 4096 x 1536, 100: 51 | 65 | 61, 512: 139 | 153 | 148; 16 of 5120 x 1536, 100: 99 | 103 | 98,
   // 256: 211 | 194 | 199; 64 of 1536 x 3072, 75: 206 | 227 | 216.  AMXINT8: 64 of 2560 x 2048, 50: 260 | 266 | 275, 250: 603 | 620 | 605; 256 of 7168 x 2048, 64: 2650 | 2631 |
-  // 2670.  A short K or few workgroups stream no better: 64 of 1536 x 3072, 20 rows 130 | 137.  16 against 32 rows: 3.1 rows 660 | 669, 6.6: 750 | 778, 64 experts of
+  // 2670; 8 | 4, the workgroups of 8 in brackets: 32 of 6144 x 3072, 88 (900) 478 | 503, 106 (1020) 567 | 546; 64 of 4096 x 2048, 56 (960) 382 | 402; 64 of 3072 x 3072, 75 (1668) 498 | 509; 32 of 5120 x
+  // 2048, 62 (504) 274 | 287; 16 of 6144 x 3072, 75 (408) 278 | 277; 16 of 6144 x 2048, 88 (296) 191 | 187; 128 of 4096 x 1536, 62 (1518) 619 | 637, 94 (1890) 733 | 714; 16 of 5120 x 1536, 62 (186) 133 |
+  // 137.  A short K or few workgroups stream no better: 64 of 1536 x 3072, 20 rows 130 | 137.  16 against 32 rows: 3.1 rows 660 | 669, 6.6: 750 | 778, 64 experts of
   // 2048 x 1408, 3: 59 | 63, 9.4: 77 | 77.  32 against 64 rows where nothing streams: 25 rows
   // 134 | 135, 37: 109 | 109, 50: 177 | 169, 75: 152 | 138; with 8 experts 25: 35 | 41, 100: 53 | 58, 125: 60 | 59, 200: 82 | 75 — few tiles leave
   // CUs idle longer.  Dev knobs (tests) [4]: 1 = never stream, 2 = always at 64 rows; [23]: 1 = 4 wavefronts, 2 = 8.
@@ -2401,7 +2403,7 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
     use_stream = g_dbg[4] != 1 && large && ((rows > 12.0 && fills8) || (rows >= 48.0 && fills4));
     mt = rows <= 8.0 ? 1 : use_stream || (rows > 40.0 && tiles64(4) >= 512) ? 4 : 2;
   }
-  const int stream_nw = g_dbg[23] ? 4 * g_dbg[23] : (fills8 && (H >= 4096 || rows < 48.0)) || (h->wbits == 8 && rows < 56.0) ? 8 : 4;
+  const int stream_nw = g_dbg[23] ? 4 * g_dbg[23] : (fills8 && (H >= 4096 || rows < 48.0)) || (h->wbits == 8 && (rows < 56.0 || (rows < 92.0 && tiles64(16) >= 500))) ? 8 : 4;
   const bool use_rt = mt == 4 && g_dbg[4] == 3;   // register-tile kernels (256-row tiles): parity-tested, not yet timed
   if (use_rt) { mt = 16; use_stream = false; }
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
