@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_nt_kernel(GemmParams p) {   
 //     multiplies, the other reads and issues — the matrix pipe of a SIMD always has exactly one owner;
 //   * LDS rows keep the 128-B row swizzle of the kernels above (applied on the DMA source side); epilogue through LDS as above.
 // NB: 16-column fragments of a wavefront.  4: 256 columns; 3: 192, whose B_b1 is half as long (16 columns of each wavefront, one request a wavefront; phases 1 and 2 of
-// 8 MFMAs): which of them, launch_gemm256 says.
+// 8 MFMAs): which of them, gemm256_fragments says.
 template <int NB>
 struct Gemm256 {
   static constexpr int BM = 256, BN = NB * 64, WN = NB * 16, BK = 64, STAGE = 65536, HALF = 16384;

@@ -1,25 +1,8 @@
 // ktx_moe_raw.h — what ktx_moe.hip (which buckets, quantises and combines) and ktx_moe_raw.hip (the prompt GEMM of RAWINT4 experts) share.
 #ifndef KTX_MOE_RAW_H
 #define KTX_MOE_RAW_H
-#include <type_traits>
-
 #include "ktx_common.h"
-
-template <int N, class F, int I = 0>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, F, I + 1>(static_cast<F&&>(f));
-  }
-}
-
-struct Tile {
-  int expert;  // local expert index
-  int row0;    // first sorted row
-  int nrows;   // <= 16*MT
-  int idx;     // place among its expert's tiles
-  int cnt;     // the expert's tiles
-};
+#include "ktx_moe_tile.h"
 
 struct RawGemmParams {
   const uint8_t *w0, *w1;      // RAW tiles (gate | down, up)

@@ -2,7 +2,7 @@
 #ifndef KTX_MOE_ROUTE_H
 #define KTX_MOE_ROUTE_H
 #include "ktx_common.h"
-#include "ktx_moe_raw.h"
+#include "ktx_moe_tile.h"
 
 #define KTX_EMAX 1024   // experts of a handle
 

@@ -2,7 +2,7 @@
 #ifndef KTX_MOE_STREAM_H
 #define KTX_MOE_STREAM_H
 #include "ktx_common.h"
-#include "ktx_moe_raw.h"
+#include "ktx_moe_tile.h"
 
 // Workgroup -> (tile, strip group) of a grouped GEMM, from a one-dimensional grid: ids are dealt round-robin to the 8 XCDs, so id % 8 is the
 // XCD.  The jobs lie expert after expert, within an expert strip group by strip group, the group's tiles side by side; each XCD takes an

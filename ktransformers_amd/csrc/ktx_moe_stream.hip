@@ -13,7 +13,8 @@
 // wavefronts 1.54 M at 1.65).  So it does no work that no row needs and keeps both units fed:
 //   * a tile multiplies the 16-row groups that hold rows, by an instantiation for each count (a quarter of a 64-row tile is absent at 64 rows an expert);
 //   * each wavefront owns four 16-row weight strips (gate|up: two strips of both; down: four), so a fragment of activations feeds 4 MFMAs; weights stream
-//     through a ring of registers, 4 k-steps deep.  That is 128 KB a CU, as much as its share of the L2 holds; 8 deep is slower (31 rows an expert: 1151 us against 1131);
+//     through a ring of registers, 4 k-steps deep (AMXINT8: 2).  That is 128 KB a CU, as much as its share of the L2 holds; AMXINT4 8 deep is slower (31 rows an expert: 1151 us against
+//     1131; at 94 rows, 64 of 6144 x 3072, it was 1 % faster, 570 against 576);
 //   * activations come by LDS-DMA into one of two buffers of 4 or 8 k-steps while the other is multiplied.  Before, 2048 columns were staged at once, and nothing
 //     multiplied meanwhile: a fifth of the time of a 64-row tile.
 // NW = 8: one workgroup a CU.  NW = 4: two, of half the strips and half the LDS each, so that one starts or ends beside the other's MFMAs, and a job is half as
