@@ -673,7 +673,7 @@ def _rawint4_chain(a, q, s):
     return f32_to_bf16(acc)
 
 
-@pytest.mark.parametrize("H,I", [(512, 1024), (1024, 512)])
+@pytest.mark.parametrize("H,I", [(512, 1024), (1024, 512), (512, 1536)])
 @pytest.mark.parametrize("large", [False, True])
 def test_rawint4_prompt_terms_of_any_scale(dev, H, I, large):
     """The prompt kernel's sums are fmas of the fp32 scale products, bit for bit (down, from the intermediates that the handle holds), for scales of 0, subnormal, tiny
