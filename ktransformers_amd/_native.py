@@ -809,7 +809,7 @@ class LinearHandle:
         T = x2.shape[0]
         n_out = self.N // 2 if glu else self.N
         # (the GEMM behind the prompt paths wants K % 64 == 0, N % 8 == 0 and 16-byte aligned rows: other shapes stay on the strip
-        # kernels, which take any out_features — ADVICE r3)
+        # kernels, which take any out_features)
         gemm_ok = (self.batch == 1 and bsz_tensor is None and self.N % 8 == 0 and self.K % 64 == 0 and x2.data_ptr() % 16 == 0
                    and (x2.stride(0) * 2) % 16 == 0 and not torch.cuda.is_current_stream_capturing())
         if self.fmt == "W4" and gemm_ok and T >= self.PROMPT_MIN_T and not os.environ.get("KTX_W4_PROMPT_KERNEL"):

@@ -1,12 +1,22 @@
 // ktx_common.h — shared device/host helpers for the gfx950 kernels.
 #ifndef KTX_COMMON_H
 #define KTX_COMMON_H
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <mutex>
 #include <string>
 #include <unordered_map>
+
+// a loop over constants: f(integral_constant<int, 0>), .. f(integral_constant<int, N - 1>)
+template <int N, class F, int I = 0>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, F, I + 1>(static_cast<F&&>(f));
+  }
+}
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -90,9 +100,9 @@ __device__ __forceinline__ int quant_rne_sat8(float v) {
 }
 
 // hipFuncSetAttribute acts on the CURRENT device's copy of a kernel, so "set once" is once per (call site, device): a process that
-// splits a model's layers over several GPUs would otherwise launch with the default dynamic-LDS limit on every device but the first
-// (ADVICE r4).  hipFuncAttributeMaxDynamicSharedMemorySize once per (kernel, device); the flag is set only after the call succeeded
-// (ADVICE r5: a failed first attempt must not disable every later one), under a mutex.
+// splits a model's layers over several GPUs would otherwise launch with the default dynamic-LDS limit on every device but the first.
+// hipFuncAttributeMaxDynamicSharedMemorySize once per (kernel, device); the flag is set only after the call succeeded
+// (a failed first attempt must not disable every later one), under a mutex.
 static inline hipError_t ktx_set_max_lds(const void* kernel, int bytes) {
   static std::mutex mu;
   static std::unordered_map<const void*, uint64_t> done;   // kernel -> devices it has been set on

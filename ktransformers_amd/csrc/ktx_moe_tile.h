@@ -1,15 +1,7 @@
-// ktx_moe_tile.h — what every grouped expert kernel takes: the tiles that ktx_moe_route.hip lays out; and a loop over constants.
+// ktx_moe_tile.h — what every grouped expert kernel takes: the tiles that ktx_moe_route.hip lays out.
 #ifndef KTX_MOE_TILE_H
 #define KTX_MOE_TILE_H
-#include <type_traits>
-
-template <int N, class F, int I = 0>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, F, I + 1>(static_cast<F&&>(f));
-  }
-}
+#include "ktx_common.h"
 
 struct Tile {
   int expert;  // local expert index

@@ -865,6 +865,24 @@ def test_tiles_of_64_rows_and_256_features(fmt, group, K, N, T):
     assert torch.equal(*got)
 
 
+@pytest.mark.parametrize("fmt,group", [("W4", 32), ("W4", 64), ("W4", 128), ("FP8", 128), ("BF16", 0)])
+@pytest.mark.parametrize("K,N", [(2816, 577), (4096, 12000), (7168, 264)])     # 64 x 64, 64 x 256 (W4, FP8) and 64 x 64 tiles in more pieces of K
+def test_tiles_of_48_rows(fmt, group, K, N):
+    """33 to 48 rows on tiles of 48: the bits that the same rows have among 49, on tiles of 64 (K is cut by K and T alone, alike up to 256 rows)."""
+    from ktransformers_amd import _native
+    g = torch.Generator().manual_seed(K + N)
+    dev = torch.device("cuda", 0)
+    h = _native.LinearHandle(K, N, fmt, group, 64, dev)
+    if fmt == "FP8":
+        h.load_fp8((torch.randn((N, K), generator=g) * 100).clamp_(-448, 448).to(torch.float8_e4m3fn).to(dev), torch.rand((-(-N // 128), K // 128), generator=g).to(dev))
+    else:
+        h.load_bf16((torch.randn((N, K), generator=g) * K ** -0.5).to(torch.bfloat16).to(dev))
+    x = torch.randn((49, K), generator=g).to(torch.bfloat16).to(dev)
+    want = h.forward(x)
+    for T in (33, 47, 48):
+        assert torch.equal(h.forward(x[:T]), want[:T]), f"{T} rows"
+
+
 @pytest.mark.parametrize("N", [24576, 24584])
 def test_bf16_prompts_on_the_gemm_of_decode_tiles(N):
     """520 rows of 2048 -> 24576 (whole strips) and 24584 (half a strip at the end) fill the chip with 256 x 256 tiles over the whole K: the GEMM
