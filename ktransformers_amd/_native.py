@@ -285,8 +285,16 @@ def check(rc: int) -> None:
         raise KtxError(lib.ktx_last_error().decode("utf-8", "replace"))
 
 
+# The handle of a device's current stream.  torch.cuda.current_stream builds a Stream object around it (2.0 us a call, this 0.1; a linear of one row takes 5 us on the
+# device), so the raw accessor that torch's own code generator uses is taken where this torch has it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_ptr(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index if isinstance(device, torch.device) else None
+    if _raw_stream is None or index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(index)
 
 
 class MoEHandle:
@@ -810,17 +818,14 @@ class LinearHandle:
         n_out = self.N // 2 if glu else self.N
         # (the GEMM behind the prompt paths wants K % 64 == 0, N % 8 == 0 and 16-byte aligned rows: other shapes stay on the strip
         # kernels, which take any out_features)
-        gemm_ok = (self.batch == 1 and bsz_tensor is None and self.N % 8 == 0 and self.K % 64 == 0 and x2.data_ptr() % 16 == 0
-                   and (x2.stride(0) * 2) % 16 == 0 and not torch.cuda.is_current_stream_capturing())
-        if self.fmt == "W4" and gemm_ok and T >= self.PROMPT_MIN_T and not os.environ.get("KTX_W4_PROMPT_KERNEL"):
+        w4_prompt = self.fmt == "W4" and T >= self.PROMPT_MIN_T
+        fp8_prompt = self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and T * self.N > self.FP8_GEMM_OUT[T > 1024 and self.K > 2048]
+        if ((w4_prompt or fp8_prompt) and self.batch == 1 and bsz_tensor is None and self.N % 8 == 0 and self.K % 64 == 0 and x2.data_ptr() % 16 == 0
+                and (x2.stride(0) * 2) % 16 == 0 and not os.environ.get("KTX_W4_PROMPT_KERNEL" if w4_prompt else "KTX_FP8_PROMPT_KERNEL")
+                and not torch.cuda.is_current_stream_capturing()):
             if norm is not None:
                 x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)
-            return self._prompt_forward(x2, out, add1, add2, glu).reshape(*x.shape[:-1], n_out)
-        if (self.fmt == "FP8" and gemm_ok and T >= self.FP8_PROMPT_MIN_T and T * self.N > self.FP8_GEMM_OUT[T > 1024 and self.K > 2048]
-                and not os.environ.get("KTX_FP8_PROMPT_KERNEL")):
-            if norm is not None:
-                x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)
-            return self._prompt_forward_fp8(x2, out, add1, add2, glu).reshape(*x.shape[:-1], n_out)
+            return (self._prompt_forward if w4_prompt else self._prompt_forward_fp8)(x2, out, add1, add2, glu).reshape(*x.shape[:-1], n_out)
         if out is None:
             out = torch.empty((T, n_out), dtype=torch.bfloat16, device=self.device) if bsz_tensor is None else \
                 torch.zeros((T, n_out), dtype=torch.bfloat16, device=self.device)
@@ -835,7 +840,7 @@ class LinearHandle:
                 self._forward_ws(bsz, T, x2, out, None, need)
             else:
                 check(lib.ktx_linear_forward(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), _stream_ptr(self.device)))
-            return out.reshape(*x.shape[:-1], self.N)
+            return out if x.dim() == 2 and out.shape == (T, self.N) else out.reshape(*x.shape[:-1], self.N)
         fu = _LinearFusion(None, 0.0, None, 0, None, 0, x2.stride(0) if strided else 0, 0, 1 if glu else 0)
         keep = []
         if norm is not None:
@@ -1248,6 +1253,7 @@ class MLAWrapper:
         self.max_q_tokens = max_q_tokens or max(256, max_batch_size)
         self.use_cuda_graph = bool(use_cuda_graph)
         self.cfg = None
+        self._sizes, self._need = None, 0   # what cfg was made from, and the workspace that it takes
         self.workspace = None
         if max_batch_size == 1:  # single-request defaults like the reference wrapper (:88-93)
             self.qo_indptr_buf = torch.arange(0, 2, dtype=torch.int32, device=self.device)
@@ -1270,9 +1276,12 @@ class MLAWrapper:
         self.kv_indices = None if identity_pages else (kv_indices if kv_indices is not None else self.kv_indices_buf)
         self.bsz_tensor = bsz_tensor if bsz_tensor is not None else getattr(self, "batch_size_tensor_buf", None)
         self.kv_len_arr = kv_len_arr
-        self.cfg = _MlaConfig(num_heads, head_dim_ckv, head_dim_kpe, page_size, float(sm_scale), self.max_splits,
-                              int(max_kv_len))
-        need = int(lib.ktx_mla_workspace_bytes(C.byref(self.cfg), self.max_q_tokens))
+        sizes = (num_heads, head_dim_ckv, head_dim_kpe, page_size, float(sm_scale), self.max_splits, int(max_kv_len))
+        if self._sizes != (sizes, self.max_q_tokens):   # (a decode loop plans every step with the same ones)
+            self.cfg = _MlaConfig(*sizes)
+            self._need = int(lib.ktx_mla_workspace_bytes(C.byref(self.cfg), self.max_q_tokens))
+            self._sizes = (sizes, self.max_q_tokens)
+        need = self._need
         if self.workspace is None:
             first = need
             if self.use_cuda_graph and self.max_q_tokens <= 4:   # the shared decode wrapper: allocated ONCE, for the largest head count a model on this device may bring (graphs keep its address)

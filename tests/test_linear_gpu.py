@@ -962,3 +962,12 @@ def test_a_batch_without_memory_for_scratch_runs_on_the_strip_kernels(monkeypatc
         monkeypatch.undo()
     assert len(labels) == 1 and labels[0].startswith("lin_gemm"), labels
     close(y, linear_w4_ref(x, *quantize_weights_ref(w.T.contiguous(), 64), 64))
+
+
+def test_calls_go_to_the_current_stream_of_their_device():
+    """The raw accessor of the current stream gives torch's own handle, on the default stream and on others, for devices with and without an index."""
+    n = native()
+    for st in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(st):
+            for dev in (torch.device("cuda", 0), torch.device("cuda")):
+                assert n._stream_ptr(dev) == torch.cuda.current_stream(dev).cuda_stream == st.cuda_stream
