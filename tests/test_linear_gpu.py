@@ -918,7 +918,11 @@ def test_bf16_prompts_on_the_gemm_of_decode_tiles(N):
     ("W8", 2048, 3072, 64, "lin_gemm_kernel"), ("W8", 7168, 2112, 64, "lin_tile_kernel"), ("W8", 7168, 2112, 700, "lin_gemm_kernel"),
     ("W4", 2048, 3072, 16, "lin_gemm"), ("W4", 7168, 2112, 16, "lin_tile_kernel"), ("W4", 1536, 2048, 48, "lin_tile_kernel"),
     ("FP8", 2048, 3072, 16, "lin_gemm_kernel"), ("FP8", 2048, 3072, 48, "lin_tile_kernel"), ("FP8", 5120, 9000, 700, "lin_fp8_gemm_kernel"),
-    ("FP8", 7168, 2112, 1500, "lin_fp8_gemm_kernel"), ("FP8", 2048, 3072, 1025, "lin_tile_kernel")])
+    ("FP8", 7168, 2112, 1500, "lin_fp8_gemm_kernel"), ("FP8", 2048, 3072, 1025, "lin_tile_kernel"),
+    ("W4", 2176, 2112, 16, "lin_tile_kernel"), ("W4", 128, 2112, 17, "lin_tile_kernel"), ("FP8", 2176, 2112, 16, "lin_tile_kernel"), ("FP8", 256, 2112, 32, "lin_gemm_kernel"),
+    ("FP8", 384, 2112, 32, "lin_tile_kernel"), ("FP8", 128, 2112, 33, "lin_tile_kernel"), ("BF16", 2688, 8192, 16, "lin_tile_kernel"), ("BF16", 2688, 8200, 16, "lin_gemm_kernel"),
+    ("BF16", 1664, 2112, 17, "lin_tile_kernel"), ("BF16", 2176, 2112, 32, "lin_gemm_kernel"), ("BF16", 2176, 2112, 33, "lin_tile_kernel"), ("W8", 1664, 2112, 64, "lin_gemm_kernel"),
+    ("W8", 2176, 2112, 33, "lin_tile_kernel")])
 def test_which_kernel_a_batch_takes(fmt, K, N, T, kernel):
     """Strip kernels, tiles or GEMM, where each was measured faster (lin_tile_wins, lin_gemm_parts, LinearHandle.FP8_GEMM_OUT)."""
     n = native()
