@@ -770,18 +770,22 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // merge the KV splits: one 256-thread workgroup per (query token, head, quarter of the 512 output dims) — a workgroup
-// pulls cross-XCD data at only ~65 GB/s (MI355X_MICROARCH.md handoff-payload), so the partials of one head are spread
+// pulls cross-XCD data at only ~65 GB/s, so the partials of one head are spread
 // over four workgroups.  Thread (sl, dg) owns splits sl, sl+16, ... for 8 dims.  EVERY global load of the kernel — the
 // (m, l) pairs, the partial outputs, the bounds — is issued before the first use: right after the kernel boundary each of
 // them is an L2 miss, and a stats -> weights -> addresses -> loads chain would pay that latency three times over.  A dead
 // split's partial may be stale memory, so it is selected away (not multiplied by 0).
-template <int NS, bool JOBS>   // splits per thread and round; JOBS: a token's number of splits is the decode kernel's (njobs)
+// SL < 16 (batches that share out the workgroups; ns, twice the mean of a token's splits, to 8: 4 lanes and all of a head's dims, to 32: 8 and half of them): no lane without a split, more
+// bytes in flight a thread and fewer workgroups, each of which finds the statistics again.  Us, decode and merge, 16 lanes -> here: 128 heads, 32 of 400 tokens 41.2 -> 31.1, 32 of 1000
+// 45.0 -> 35.6, 16 of 2000 36.3 -> 33.8, 8 of 8192 47.5 -> 46.9; 64 heads, 24 of 500 27.3 -> 25.9, 32 of 2000 38.0 -> 35.5; 8 lanes at ns 51 (5 of 8000) lost, 43.6 -> 44.6.
+template <int NS, bool JOBS, int SL = 16>   // splits per thread and round; JOBS: a token's number of splits is the decode kernel's (njobs); split lanes
 __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out, float* lse) {
+  constexpr int DG = 256 / SL, DIMS = DG * 8;
   __shared__ float s_w[1024];
   __shared__ float s_red[8];
-  __shared__ float s_acc[16][128 + 4];
-  const int qt = blockIdx.y, h = blockIdx.x, quarter = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int dg = tid & 15, sl = tid >> 4;   // 16 dim groups of 8 dims x 16 split lanes
+  __shared__ float s_acc[SL][DIMS + 4];
+  const int qt = blockIdx.y, h = blockIdx.x, part = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int dg = tid % DG, sl = tid / DG;   // dim groups of 8 dims x split lanes
   const size_t base = ((size_t)qt * p.Hq + h) * p.nsplit;
   const int nsp = JOBS ? min(max(p.njobs[qt], 1), p.nsplit) : p.nsplit;   // (no request's token: whatever is there, and nothing is stored)
   // ---- all loads
@@ -794,10 +798,10 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out
     ml[i] = s < nsp ? *reinterpret_cast<const float2*>(p.part_ml + (base + s) * 2) : make_float2(0.f, 0.f);
   }
   float4 va[NS], vb[NS];
-  const float* po = p.part_o + base * MLA_DC + quarter * 128 + dg * 8;
+  const float* po = p.part_o + base * MLA_DC + part * DIMS + dg * 8;
 #pragma unroll
   for (int u = 0; u < NS; u++) {
-    const int s = min(sl + 16 * u, nsp - 1);
+    const int s = min(sl + SL * u, nsp - 1);
     va[u] = *reinterpret_cast<const float4*>(po + (size_t)s * MLA_DC);
     vb[u] = *reinterpret_cast<const float4*>(po + (size_t)s * MLA_DC + 4);
   }
@@ -827,20 +831,20 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out
   lsum = (s_red[4] + s_red[5]) + (s_red[6] + s_red[7]);
 
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int c = 0;; c += 16 * NS) {   // (more than one round: a token of the jobs form that holds most of the batch's tiles)
+  for (int c = 0;; c += SL * NS) {   // (more than one round: a token of the jobs form that holds most of the batch's tiles)
 #pragma unroll
   for (int u = 0; u < NS; u++) {
-    const int s = c + sl + 16 * u;
+    const int s = c + sl + SL * u;
     const float w = s < nsp ? s_w[s] : 0.f;
     if (w > 0.f) {
       acc[0] += va[u].x * w; acc[1] += va[u].y * w; acc[2] += va[u].z * w; acc[3] += va[u].w * w;
       acc[4] += vb[u].x * w; acc[5] += vb[u].y * w; acc[6] += vb[u].z * w; acc[7] += vb[u].w * w;
     }
   }
-  if (!JOBS || c + 16 * NS >= nsp) break;
+  if (!JOBS || c + SL * NS >= nsp) break;
 #pragma unroll
   for (int u = 0; u < NS; u++) {
-    const int s = min(c + 16 * NS + sl + 16 * u, nsp - 1);
+    const int s = min(c + SL * NS + sl + SL * u, nsp - 1);
     va[u] = *reinterpret_cast<const float4*>(po + (size_t)s * MLA_DC);
     vb[u] = *reinterpret_cast<const float4*>(po + (size_t)s * MLA_DC + 4);
   }
@@ -848,14 +852,14 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out
 #pragma unroll
   for (int q = 0; q < 8; q++) s_acc[sl][dg * 8 + q] = acc[q];
   __syncthreads();
-  if (tid < 64 && qt < q_total) {   // 128 dims: two per thread
+  if (tid < DIMS / 2 && qt < q_total) {   // two dims per thread
     const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
     float v0 = 0.f, v1 = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; i++) { v0 += s_acc[i][2 * tid]; v1 += s_acc[i][2 * tid + 1]; }
+    for (int i = 0; i < SL; i++) { v0 += s_acc[i][2 * tid]; v1 += s_acc[i][2 * tid + 1]; }
     const uint32_t w = (uint32_t)f32_to_bf16(v0 * inv) | ((uint32_t)f32_to_bf16(v1 * inv) << 16);
-    *reinterpret_cast<uint32_t*>(out + ((size_t)qt * p.Hq + h) * MLA_DC + quarter * 128 + 2 * tid) = w;
-    if (lse && tid == 0 && quarter == 0)
+    *reinterpret_cast<uint32_t*>(out + ((size_t)qt * p.Hq + h) * MLA_DC + part * DIMS + 2 * tid) = w;
+    if (lse && tid == 0 && part == 0)
       lse[(size_t)qt * p.Hq + h] = lsum > 0.f ? (mstar + __logf(lsum)) * 1.44269504089f : -__builtin_inff();
   }
 }
@@ -1108,10 +1112,11 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
   KTX_HIP(hipGetLastError());
   if (only != 1 && !direct) {
     KTX_TIMED(st, (double)total_q_tokens * Hq * MLA_DC * 2.0, "mla_merge_kernel T=%d Hq=%d nsplit=%d", total_q_tokens, Hq, nsplit);
-    const dim3 mg(Hq, total_q_tokens, 4);
     const int ns = p.jobs ? std::min(p.nsplit, 2 * p.jobs / total_q_tokens) : p.nsplit;   // (jobs: twice the mean; the kernel goes on from there)
-    auto merge = [&](auto kern) { hipLaunchKernelGGL(kern, mg, dim3(256), 0, st, p, (bf16_t*)d_out, d_lse); };
-    if (ns <= 32) p.jobs ? merge(mla_merge_kernel<2, true>) : merge(mla_merge_kernel<2, false>);
+    auto merge = [&](auto kern, int parts = 4) { hipLaunchKernelGGL(kern, dim3(Hq, total_q_tokens, parts), dim3(256), 0, st, p, (bf16_t*)d_out, d_lse); };
+    if (p.jobs && ns <= 8) merge(mla_merge_kernel<2, true, 4>, 1);
+    else if (p.jobs && ns <= 16) merge(mla_merge_kernel<2, true, 8>, 2);
+    else if (ns <= 32) p.jobs ? merge(mla_merge_kernel<4, true, 8>, 2) : merge(mla_merge_kernel<2, false>);
     else if (ns <= 64) p.jobs ? merge(mla_merge_kernel<4, true>) : merge(mla_merge_kernel<4, false>);
     else if (ns <= 144) p.jobs ? merge(mla_merge_kernel<9, true>) : merge(mla_merge_kernel<9, false>);
     else p.jobs ? merge(mla_merge_kernel<16, true>) : merge(mla_merge_kernel<16, false>);

@@ -127,7 +127,8 @@ def decode_batch(Hq, lens, page=64, seed=7):
     return (lambda: w.run(q_nope, q_pe, cache[:, :, :512], cache[:, :, 512:])), exact
 
 
-@pytest.mark.parametrize("Hq,lens", [(64, [1000] * 20), (128, [500] * 17 + [130, 64, 1]), (128, [8192, 2100, 5000, 8192, 8000, 7000, 6000, 64]), (64, [64, 33] * 10)])
+@pytest.mark.parametrize("Hq,lens", [(64, [1000] * 20), (128, [500] * 17 + [130, 64, 1]), (128, [8192, 2100, 5000, 8192, 8000, 7000, 6000, 64]), (64, [64, 33] * 10),
+                                     (128, [400] * 31 + [9000]), (128, [100] * 19 + [8000]), (128, [300] * 32)])     # the merge's 4 and 8 split lanes: a token of several rounds; of none
 def test_wide_decode_is_off_by_the_rounding_of_its_outputs(Hq, lens):
     """mla_decode_wide_kernel multiplies P as two bf16 (2^-17 of it is lost) and adds in fp32: against 64-bit sums the result is off by what rounding
     the exact result to bf16 is off by, to 1 %."""
