@@ -701,6 +701,15 @@ class LinearHandle:
         check(lib.ktx_linear_dequant_bf16(self._h, out.data_ptr(), out.stride(0), _stream_ptr(self.device)))
         return out
 
+    def _w4_prompt_on_tiles(self, T: int) -> bool:
+        """Whether the tiles of ktx_linear_forward_ws take a W4 prompt, with Marlin's multiplicand formed in registers, rather than the expansion
+        and the GEMM: the same sums of the same products (in another order where K is cut).  Us, GEMM | tiles: few outputs, 512 rows of 4096 -> 1000 50 | 18, 2048 of them 51 | 39, of
+        2048 -> 576 30 | 21; long K, 512 of 16384 -> 7168 320 | 167, 1000 322 | 278, 800 of 7168 -> 2112 88 | 71, 1000 of 7168 -> 18432 392 | 373, 1400 of 7168 -> 4096 121 | 140; between them
+        640 of 2048 -> 3072 33 | 20, 512 of 1024 -> 4096 23 | 17, 800 equal, 640 of 2048 -> 7168 42 | 48, 512 of 5120 -> 9000 98 | 100."""
+        if not (T <= 2048 if self.N <= 1024 else T <= 1024 if self.K >= 7168 else T <= 640 and self.N <= 4096):
+            return False
+        return self.K % 128 == 0 and self._scratch(T, True) is not None
+
     def _prompt_forward(self, x2: torch.Tensor, out, add1, add2, glu: bool) -> torch.Tensor:
         need = self.N * self.K
         buf = LinearHandle._DEQ_SCRATCH.get(self.device)
@@ -820,12 +829,15 @@ class LinearHandle:
         # kernels, which take any out_features)
         w4_prompt = self.fmt == "W4" and T >= self.PROMPT_MIN_T
         fp8_prompt = self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and T * self.N > self.FP8_GEMM_OUT[T > 1024 and self.K > 2048]
+        rounded = False
         if ((w4_prompt or fp8_prompt) and self.batch == 1 and bsz_tensor is None and self.N % 8 == 0 and self.K % 64 == 0 and x2.data_ptr() % 16 == 0
                 and (x2.stride(0) * 2) % 16 == 0 and not os.environ.get("KTX_W4_PROMPT_KERNEL" if w4_prompt else "KTX_FP8_PROMPT_KERNEL")
                 and not torch.cuda.is_current_stream_capturing()):
-            if norm is not None:
-                x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)
-            return (self._prompt_forward if w4_prompt else self._prompt_forward_fp8)(x2, out, add1, add2, glu).reshape(*x.shape[:-1], n_out)
+            rounded = w4_prompt and not os.environ.get("KTX_VENDOR_GEMM") and self._w4_prompt_on_tiles(T)
+            if not rounded:
+                if norm is not None:
+                    x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)
+                return (self._prompt_forward if w4_prompt else self._prompt_forward_fp8)(x2, out, add1, add2, glu).reshape(*x.shape[:-1], n_out)
         if out is None:
             out = torch.empty((T, n_out), dtype=torch.bfloat16, device=self.device) if bsz_tensor is None else \
                 torch.zeros((T, n_out), dtype=torch.bfloat16, device=self.device)
@@ -837,7 +849,7 @@ class LinearHandle:
         if norm is None and add1 is None and add2 is None and not strided and not glu:
             need = self._scratch(T, bsz is None) if T > 8 else None
             if need is not None:
-                self._forward_ws(bsz, T, x2, out, None, need)
+                self._forward_ws(bsz, T, x2, out, None, need, rounded)
             else:
                 check(lib.ktx_linear_forward(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), _stream_ptr(self.device)))
             return out if x.dim() == 2 and out.shape == (T, self.N) else out.reshape(*x.shape[:-1], self.N)
@@ -861,7 +873,7 @@ class LinearHandle:
                 keep.append(a2)
         need = self._scratch(T, False) if T > 8 else None
         if need is not None:
-            self._forward_ws(bsz, T, x2, out, C.byref(fu), need)
+            self._forward_ws(bsz, T, x2, out, C.byref(fu), need, rounded)
         else:
             check(lib.ktx_linear_forward_fused(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), C.byref(fu), _stream_ptr(self.device)))
         return out.reshape(*x.shape[:-1], n_out)
@@ -874,14 +886,14 @@ class LinearHandle:
             self._ws_need[key] = int(lib.ktx_linear_workspace_bytes(self._h, T, int(plain))) if lib.ktx_linear_tiled(self._h, T) else None
         return self._ws_need[key]
 
-    def _forward_ws(self, bsz, T: int, x2: torch.Tensor, out: torch.Tensor, fu, need: int) -> None:
+    def _forward_ws(self, bsz, T: int, x2: torch.Tensor, out: torch.Tensor, fu, need: int, rounded: bool = False) -> None:
         """ktx_linear_forward_ws with its scratch from torch's allocator (freed to the stream's pool behind the launches).  FP8 prompts take the
         K = 128 MFMA whether the call is eager, captured or has its row count on the device."""
         try:
             ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
         except torch.cuda.OutOfMemoryError:   # (the strip kernels need none)
             ws, need = None, 0
-        prompt = self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")
+        prompt = rounded or self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")
         check(lib.ktx_linear_forward_ws(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), fu, 1 if prompt else 0, ws.data_ptr() if ws is not None else None, need,
                                         _stream_ptr(self.device)))
 

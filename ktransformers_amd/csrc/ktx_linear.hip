@@ -2137,8 +2137,8 @@ extern "C" int ktx_linear_forward_fused(ktx_linear_t h, const int32_t* d_bsz, in
 
 // 9 rows and more with a workspace: ktx_linear_tile.inc.  (dev knob 12, the strips per wavefront of the strip kernels, keeps those)
 static bool tile_eligible(const ktx_linear_s* h, int T) { return T <= h->cfg.max_len && !dec_eligible(h, T) && !ktx_debug_get(12) && !g_lin_force_gemm; }
-static bool tile_plan(const ktx_linear_s* h, int T, LinTilePlan* o) {
-  return lin_tile_plan(h->cfg.format, 128 / std::max(h->cfg.group_size, 1), h->cfg.out_features, h->cfg.in_features, h->NKS, h->batch, T, o);
+static bool tile_plan(const ktx_linear_s* h, int T, LinTilePlan* o, bool rounded = false) {
+  return lin_tile_plan(h->cfg.format, 128 / std::max(h->cfg.group_size, 1), h->cfg.out_features, h->cfg.in_features, h->NKS, h->batch, T, o, rounded);
 }
 static int gemm_parts(const ktx_linear_s* h, int T) {
   return h->cfg.format == KTX_LIN_BF16 ? lin_gemm_parts(h->cfg.out_features, h->cfg.in_features, h->NKS, h->batch, T) : 0;
@@ -2173,7 +2173,7 @@ extern "C" int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T
   int parts = ok && (size_t)T * ldx * 2 < ((size_t)1 << 32) ? gemm_parts(h, T) : 0;
   const bool direct = gemm_direct(h, parts, !d_bsz && (!fu || (!fu->add1 && !fu->add2 && !fu->glu))) && (uintptr_t)d_y % 16 == 0 && (!fu || fu->y_ld % 8 == 0);
   if (!direct && parts && !ws_fits(gemm_ws(h, T, parts))) parts = 0;
-  if (!parts && !(ok && tile_plan(h, T, &o) && ws_fits(o.part_bytes + o.sT_bytes + o.xq_bytes)))
+  if (!parts && !(ok && tile_plan(h, T, &o, prompt != 0) && ws_fits(o.part_bytes + o.sT_bytes + o.xq_bytes)))
     return ktx_linear_forward_fused(h, d_bsz, T, d_x, d_y, fu, stream);
   LinTileParams q{};
   LinParams& p = q.p;
@@ -2206,7 +2206,7 @@ extern "C" int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T
   if (h->cfg.format == KTX_LIN_FP8) {
     const int rc = ktx_fp8_act_quant_padded(d_x, ldx, T, p.Kx, (void*)q.xq, (float*)q.sT, q.s_ld, stream);
     if (rc) return rc;
-    return prompt && o.mt >= 4 ? forward_tile<F_FP8, 128, true>(o, q, st) : forward_tile<F_FP8, 128>(o, q, st);
+    return prompt && o.mt >= 4 ? forward_tile<F_FP8, 128, 1>(o, q, st) : forward_tile<F_FP8, 128>(o, q, st);
   }
   const int g = h->cfg.group_size;
   if (o.sT_bytes) {

@@ -539,6 +539,29 @@ def test_prompt_sized_w4_dequantises_once_and_runs_a_library_gemm(K, N, G):
         assert float((got.float() - ref.float()).norm() / ref.float().norm()) < 5e-3
 
 
+@pytest.mark.parametrize("K,N,T,G", [(2048, 576, 1500, 64), (128, 264, 513, 128), (1536, 24, 600, 32), (7168, 264, 520, 64), (7168, 2112, 777, 128), (4096, 1000, 1030, 32)])
+def test_w4_prompts_on_tiles_multiply_the_rounded_weights(K, N, T, G, monkeypatch):
+    """The tiles with bf16((q - 8) s) formed in registers against the expansion and the GEMM: the same products, so the same bits where K is one chunk (to 16 k-steps, and
+    past 1024 rows); with K cut the fp32 sums are added in another order, which moves a result by a bf16 step now and then (fewer than 1 in 100 here: a rounding error of about
+    2^-22 of the sums against steps of 2^-8)."""
+    n = native()
+    torch.manual_seed(K + N + T)
+    h = n.LinearHandle(K, N, "W4", G, 2048)
+    h.load_bf16((torch.randn(N, K) / 10).to(torch.bfloat16).cuda())
+    x = (torch.randn(T, K) / 10).to(torch.bfloat16).cuda()
+    a1 = torch.randn(T, N).to(torch.bfloat16).cuda()
+    assert h._w4_prompt_on_tiles(T)
+    y, y_add = h.forward(x), h.forward(x, add1=a1)
+    assert torch.equal(y_add, a1 + y)
+    monkeypatch.setattr(n.LinearHandle, "_w4_prompt_on_tiles", lambda self, T: False)
+    want = h.forward(x)
+    if K <= 2048 or T > 1024:
+        assert torch.equal(y, want)
+    else:
+        assert float((y != want).float().mean()) < 0.01
+        torch.testing.assert_close(y.float(), want.float(), rtol=2.0 ** -7, atol=1e-5)
+
+
 # ---- lin_sk_kernel (round 3): the decode GEMV dealt over all CUs ----------------------------------------------------------
 # Shapes: DeepSeek-V3 linears (k-steps 56 / 128 / 144 / 12 / 16 -> ring depths 7 / 8 / 6 / 4), a glu pair, ragged N.
 SK_SHAPES = [(7168, 2112), (16384, 7168), (18432, 1024), (1536, 3072), (2048, 7168), (7168, 4096), (896, 200), (1408, 512)]
