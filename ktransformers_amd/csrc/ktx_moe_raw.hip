@@ -104,8 +104,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int row = (lane >> 1) & 15;
     sb = (lane < 32 ? sbu[0] : sbu[1]) + (size_t)((row >> 2) * NS * 128 + (row & 3) * 32 + (lane & 1) * 16);
   }
-  // the activations' scales of a step: a row's 16 groups lie together, 4 lanes bring them
-  const uint8_t* ga = reinterpret_cast<const uint8_t*>(p.act_d + (size_t)s_src[wave * 16 + (lane >> 2)] * G) + (lane & 3) * 16;
+  // the activations' scales of a step: a row's 16 groups lie together, 4 lanes bring them, group quad q of row r to place q ^ (r >> 2 & 3) (16 rows' reads of one quad:
+  // 16 places of a bank row)
+  const uint8_t* ga = reinterpret_cast<const uint8_t*>(p.act_d + (size_t)s_src[wave * 16 + (lane >> 2)] * G) + ((lane ^ (lane >> 4)) & 3) * 16;
   const uint32_t lds_w = lds0 + XBYTES + ABYTES + wave * WB;
   const uint8_t* my_w = smem + XBYTES + ABYTES + wave * WB;
   constexpr int WDMA = NU * 4 + 2;
@@ -189,7 +190,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const uint8_t* xb = smem + buf * XB;
       float as[SB];   // set: of the lane's row and group
       {
-        const uint8_t* sp = smem + XBYTES + (st & 1) * AB + Q * 16;
+        const uint8_t* sp = smem + XBYTES + (st & 1) * AB + ((Q ^ (i >> 2)) & 3) * 16;   // (r >> 2 & 3 = i >> 2)
         if constexpr (SB == 4) {
           const float4 v = *reinterpret_cast<const float4*>(sp + lane * 64);
           as[0] = v.x; as[1] = v.y; as[2] = v.z; as[3] = v.w;
