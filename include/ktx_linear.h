@@ -120,7 +120,7 @@ int ktx_linear_decode_eligible(ktx_linear_t h, int T);
  * in_features % 128 != 0, rows that are not 16-byte aligned, decode-sized T) or are slower for (short K, a chip that the strips fill) run as
  * ktx_linear_forward_fused.  `fusion` may be NULL.
  * prompt (FP8, T > 32): 1 takes a 128-block in one K = 128 MFMA instead of four of K = 32 (the order of ktx_linear_forward): the same
- * error against 64-bit sums, other last bits.  W4 multiplies exact integers, as ktx_linear_forward does; with prompt = 1 and more than 64 rows the multiplicand of
+ * error against 64-bit sums, other last bits.  W4 multiplies exact integers, as ktx_linear_forward does; with prompt = 2 and more than 64 rows the multiplicand of
  * ktx_linear_dequant_bf16. */
 size_t ktx_linear_workspace_bytes(ktx_linear_t h, int T, int plain);
 int ktx_linear_tiled(ktx_linear_t h, int T);   /* 1: ktx_linear_forward_ws takes T rows on the tiles (or the GEMM), given its scratch */

@@ -706,6 +706,8 @@ class LinearHandle:
         and the GEMM: the same sums of the same products (in another order where K is cut).  Us, GEMM | tiles: few outputs, 512 rows of 4096 -> 1000 50 | 18, 2048 of them 51 | 39, of
         2048 -> 576 30 | 21; long K, 512 of 16384 -> 7168 320 | 167, 1000 322 | 278, 800 of 7168 -> 2112 88 | 71, 1000 of 7168 -> 18432 392 | 373, 1400 of 7168 -> 4096 121 | 140; between them
         640 of 2048 -> 3072 33 | 20, 512 of 1024 -> 4096 23 | 17, 800 equal, 640 of 2048 -> 7168 42 | 48, 512 of 5120 -> 9000 98 | 100."""
+        if getattr(self, "_bias_t", None) is not None:   # (the GEMM adds a bias to the sum, the tiles to the rounded sum)
+            return False
         if not (T <= 2048 if self.N <= 1024 else T <= 1024 if self.K >= 7168 else T <= 640 and self.N <= 4096):
             return False
         return self.K % 128 == 0 and self._scratch(T, True) is not None
@@ -893,8 +895,8 @@ class LinearHandle:
             ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
         except torch.cuda.OutOfMemoryError:   # (the strip kernels need none)
             ws, need = None, 0
-        prompt = rounded or self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")
-        check(lib.ktx_linear_forward_ws(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), fu, 1 if prompt else 0, ws.data_ptr() if ws is not None else None, need,
+        prompt = self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")
+        check(lib.ktx_linear_forward_ws(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), fu, 2 if rounded else 1 if prompt else 0, ws.data_ptr() if ws is not None else None, need,
                                         _stream_ptr(self.device)))
 
     def _forward_glu_in(self, x, bsz_tensor, out, norm, add1, add2, glu):

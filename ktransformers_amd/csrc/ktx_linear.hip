@@ -2173,7 +2173,7 @@ extern "C" int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T
   int parts = ok && (size_t)T * ldx * 2 < ((size_t)1 << 32) ? gemm_parts(h, T) : 0;
   const bool direct = gemm_direct(h, parts, !d_bsz && (!fu || (!fu->add1 && !fu->add2 && !fu->glu))) && (uintptr_t)d_y % 16 == 0 && (!fu || fu->y_ld % 8 == 0);
   if (!direct && parts && !ws_fits(gemm_ws(h, T, parts))) parts = 0;
-  if (!parts && !(ok && tile_plan(h, T, &o, prompt != 0) && ws_fits(o.part_bytes + o.sT_bytes + o.xq_bytes)))
+  if (!parts && !(ok && tile_plan(h, T, &o, prompt == 2) && ws_fits(o.part_bytes + o.sT_bytes + o.xq_bytes)))
     return ktx_linear_forward_fused(h, d_bsz, T, d_x, d_y, fu, stream);
   LinTileParams q{};
   LinParams& p = q.p;

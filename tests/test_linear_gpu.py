@@ -550,7 +550,9 @@ def test_w4_prompts_on_tiles_multiply_the_rounded_weights(K, N, T, G, monkeypatc
     h.load_bf16((torch.randn(N, K) / 10).to(torch.bfloat16).cuda())
     x = (torch.randn(T, K) / 10).to(torch.bfloat16).cuda()
     a1 = torch.randn(T, N).to(torch.bfloat16).cuda()
-    assert h._w4_prompt_on_tiles(T)
+    hb = n.LinearHandle(K, N, "W4", G, 2048)
+    hb.load_bf16((torch.randn(N, K) / 10).to(torch.bfloat16).cuda(), torch.ones(N, dtype=torch.bfloat16, device="cuda"))
+    assert h._w4_prompt_on_tiles(T) and not hb._w4_prompt_on_tiles(T)      # (the GEMM adds a bias before it rounds)
     y, y_add = h.forward(x), h.forward(x, add1=a1)
     assert torch.equal(y_add, a1 + y)
     monkeypatch.setattr(n.LinearHandle, "_w4_prompt_on_tiles", lambda self, T: False)
