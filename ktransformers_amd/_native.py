@@ -644,6 +644,13 @@ def moe_combine(rows: torch.Tensor, row_of_pair: torch.Tensor, weights: torch.Te
 LIN_FMT = {"BF16": 0, "W4": 1, "FP8": 2, "W8": 3}
 
 
+def _share_memory(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether the spans of addresses that two tensors reach over meet (spans, not elements: column slices of one buffer count as shared)."""
+    def end(t):
+        return t.data_ptr() + (sum((n - 1) * s for n, s in zip(t.shape, t.stride())) + 1) * t.element_size()
+    return a.numel() > 0 and b.numel() > 0 and a.data_ptr() < end(b) and b.data_ptr() < end(a)
+
+
 class LinearHandle:
     """Owner of one ktx_linear_t (include/ktx_linear.h): tiled weights of one dense linear on one GPU."""
 
@@ -711,6 +718,15 @@ class LinearHandle:
         if not (T <= 2048 if self.N <= 1024 else T <= 1024 if self.K >= 7168 else T <= 640 and self.N <= 4096):
             return False
         return self.K % 128 == 0 and self._scratch(T, True) is not None
+
+    def _tiles_write(self, x2: torch.Tensor, out: torch.Tensor | None, n_out: int) -> bool:
+        """Whether the tiles may store a W4 prompt's rows, dense bf16, straight into `out`: other workgroups read x2 meanwhile.  Every other `out`
+        (strides, dtype, device or shape of its own, memory shared with x2) is the GEMM's, whose result torch copies or refuses."""
+        if out is None:
+            return True
+        if out.dtype != torch.bfloat16 or out.device != self.device or tuple(out.shape) != (x2.shape[0], n_out) or not out.is_contiguous():
+            return False
+        return not _share_memory(out, x2)
 
     def _prompt_forward(self, x2: torch.Tensor, out, add1, add2, glu: bool) -> torch.Tensor:
         need = self.N * self.K
@@ -835,7 +851,7 @@ class LinearHandle:
         if ((w4_prompt or fp8_prompt) and self.batch == 1 and bsz_tensor is None and self.N % 8 == 0 and self.K % 64 == 0 and x2.data_ptr() % 16 == 0
                 and (x2.stride(0) * 2) % 16 == 0 and not os.environ.get("KTX_W4_PROMPT_KERNEL" if w4_prompt else "KTX_FP8_PROMPT_KERNEL")
                 and not torch.cuda.is_current_stream_capturing()):
-            rounded = w4_prompt and not os.environ.get("KTX_VENDOR_GEMM") and self._w4_prompt_on_tiles(T)
+            rounded = w4_prompt and not os.environ.get("KTX_VENDOR_GEMM") and self._w4_prompt_on_tiles(T) and self._tiles_write(x2, out, n_out)
             if not rounded:
                 if norm is not None:
                     x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)

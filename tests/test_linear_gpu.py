@@ -564,6 +564,51 @@ def test_w4_prompts_on_tiles_multiply_the_rounded_weights(K, N, T, G, monkeypatc
         torch.testing.assert_close(y.float(), want.float(), rtol=2.0 ** -7, atol=1e-5)
 
 
+def w4_prompt_both_ways(K, N, T, G=64, max_len=2048):
+    """A W4 handle whose prompts of T rows the tiles take, rows for it, and a function that makes the same call on the expansion and the GEMM."""
+    n = native()
+    torch.manual_seed(K + N + T)
+    h = n.LinearHandle(K, N, "W4", G, max_len)
+    h.load_bf16((torch.randn(N, K) / 10).to(torch.bfloat16).cuda())
+    assert h._w4_prompt_on_tiles(T)
+
+    def on_the_gemm(*a, **kw):
+        h._w4_prompt_on_tiles = lambda T: False
+        try:
+            return h.forward(*a, **kw)
+        finally:
+            del h._w4_prompt_on_tiles
+    return h, (torch.randn(T, K) / 10).to(torch.bfloat16).cuda(), on_the_gemm
+
+
+@pytest.mark.parametrize("K,N,T", [(2048, 2112, 600), (1024, 1024, 520)])     # (both sides give the same bits: K is one piece)
+def test_a_w4_prompt_fills_any_out(K, N, T):
+    """`out` as torch takes it: dense, a column slice of a wider buffer, rows that lie further apart, fp32, transposed, on the host, over the input (N = K); what
+    has another number of rows is refused before anything is written."""
+    h, x, on_the_gemm = w4_prompt_both_ways(K, N, T)
+    want = on_the_gemm(x)
+    wide = torch.full((T, 2 * N), 7.0, dtype=torch.bfloat16, device="cuda")
+    for out in (torch.empty_like(want), wide[:, :N], wide[:, N:], torch.empty((2 * T, N), dtype=torch.bfloat16, device="cuda")[::2], torch.empty((T, N), device="cuda"),
+                torch.empty((N, T), dtype=torch.bfloat16, device="cuda").t(), torch.empty((1, T, N), dtype=torch.bfloat16, device="cuda"), torch.empty((T, N), dtype=torch.bfloat16),
+                torch.empty(T * N + 1, dtype=torch.bfloat16, device="cuda")[1:].view(T, N)):
+        if out.untyped_storage().data_ptr() == wide.untyped_storage().data_ptr():
+            wide.fill_(7.0)
+        y = h.forward(x, out=out)
+        assert y.data_ptr() == out.data_ptr() and torch.equal(out.view(T, N).to("cuda", torch.bfloat16) if out.is_contiguous() else out.to(torch.bfloat16), want), (out.shape, out.stride(), out.dtype)
+        if out.data_ptr() == wide.data_ptr():
+            assert bool((wide[:, N:] == 7.0).all())
+    assert bool((wide[:, :N] == 7.0).all())
+    # (a dense buffer with room for the rows asked for, so that a kernel that looked at its address alone would stay inside it)
+    room = torch.zeros((T, N), dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(RuntimeError):
+        h.forward(x, out=room[:T - 1])
+    assert not bool(room.any())
+    if K == N:
+        both = x.clone()
+        h.forward(both, out=both)
+        assert torch.equal(both, want)
+
+
 # ---- lin_sk_kernel (round 3): the decode GEMV dealt over all CUs ----------------------------------------------------------
 # Shapes: DeepSeek-V3 linears (k-steps 56 / 128 / 144 / 12 / 16 -> ring depths 7 / 8 / 6 / 4), a glu pair, ragged N.
 SK_SHAPES = [(7168, 2112), (16384, 7168), (18432, 1024), (1536, 3072), (2048, 7168), (7168, 4096), (896, 200), (1408, 512)]
