@@ -719,14 +719,20 @@ class LinearHandle:
             return False
         return self.K % 128 == 0 and self._scratch(T, True) is not None
 
-    def _tiles_write(self, x2: torch.Tensor, out: torch.Tensor | None, n_out: int) -> bool:
-        """Whether the tiles may store a W4 prompt's rows, dense bf16, straight into `out`: other workgroups read x2 meanwhile.  Every other `out`
-        (strides, dtype, device or shape of its own, memory shared with x2) is the GEMM's, whose result torch copies or refuses."""
+    def _tiles_write(self, x2: torch.Tensor, out: torch.Tensor | None, addends: list, glu: bool) -> bool:
+        """Whether the tiles may store a W4 prompt's rows, dense bf16, straight into `out` (other workgroups read x2 and the addends meanwhile) and their epilogue
+        adds what is to be added: bf16 rows, without GLU beside them.  Every other `out` (strides, dtype, device or shape of its own, shared memory) and addend
+        (another dtype, strided columns, the halved rows behind GLU) is the GEMM's, behind which torch adds, and copies or refuses."""
+        T = x2.shape[0]
+        for a in addends:
+            if glu or a.dtype != torch.bfloat16 or a.device != self.device or a.numel() != T * self.N or a.reshape(T, self.N).stride(1) != 1:
+                return False
         if out is None:
             return True
-        if out.dtype != torch.bfloat16 or out.device != self.device or tuple(out.shape) != (x2.shape[0], n_out) or not out.is_contiguous():
+        if out.dtype != torch.bfloat16 or out.device != self.device or tuple(out.shape) != (T, self.N // 2 if glu else self.N) or not out.is_contiguous():
             return False
-        return not _share_memory(out, x2)
+        # (an addend that lies exactly where `out` does is read by the thread that stores there)
+        return not any(_share_memory(out, t) and (t is x2 or t.data_ptr() != out.data_ptr() or not t.is_contiguous()) for t in [x2] + addends)
 
     def _prompt_forward(self, x2: torch.Tensor, out, add1, add2, glu: bool) -> torch.Tensor:
         need = self.N * self.K
@@ -851,7 +857,7 @@ class LinearHandle:
         if ((w4_prompt or fp8_prompt) and self.batch == 1 and bsz_tensor is None and self.N % 8 == 0 and self.K % 64 == 0 and x2.data_ptr() % 16 == 0
                 and (x2.stride(0) * 2) % 16 == 0 and not os.environ.get("KTX_W4_PROMPT_KERNEL" if w4_prompt else "KTX_FP8_PROMPT_KERNEL")
                 and not torch.cuda.is_current_stream_capturing()):
-            rounded = w4_prompt and not os.environ.get("KTX_VENDOR_GEMM") and self._w4_prompt_on_tiles(T) and self._tiles_write(x2, out, n_out)
+            rounded = w4_prompt and not os.environ.get("KTX_VENDOR_GEMM") and self._w4_prompt_on_tiles(T) and self._tiles_write(x2, out, [a for a in (add1, add2) if a is not None], glu)
             if not rounded:
                 if norm is not None:
                     x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)

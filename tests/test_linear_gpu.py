@@ -609,6 +609,28 @@ def test_a_w4_prompt_fills_any_out(K, N, T):
         assert torch.equal(both, want)
 
 
+def test_a_w4_prompt_adds_what_torch_adds():
+    """Addends of bf16 rows go into the tiles' epilogue; of another dtype, with strided columns, as (1, T, N), with rows far apart, and in halves behind GLU
+    they are added as the GEMM's callers always could."""
+    K, N, T = 2048, 2112, 600
+    h, x, on_the_gemm = w4_prompt_both_ways(K, N, T)
+    a = torch.randn((T, N), device="cuda")
+    b = a.to(torch.bfloat16)
+    far = torch.randn((T, N + 24), device="cuda").to(torch.bfloat16)[:, 8:8 + N]
+    half = torch.randn((T, N // 2), device="cuda").to(torch.bfloat16)
+    for kw in (dict(add1=b), dict(add1=a), dict(add1=b, add2=a), dict(add1=b.t().contiguous().t()), dict(add1=b.view(1, T, N), add2=far), dict(add2=far),
+               dict(glu=True), dict(glu=True, add1=half), dict(glu=True, add1=half, add2=half.float())):
+        want, got = on_the_gemm(x, **kw), h.forward(x, **kw)
+        assert got.dtype == want.dtype and torch.equal(got, want), {k: getattr(v, "dtype", v) for k, v in kw.items()}
+    want = on_the_gemm(x, add1=b)
+    here = torch.cat((b, b))
+    assert torch.equal(h.forward(x, add1=here[T:], out=here[T:]), want)                  # the residual in place
+    assert torch.equal(h.forward(x, add1=here[:T], out=here[1:T + 1]), want)             # one row further on in the same buffer
+    for kw in (dict(add1=b[:T - 1]), dict(add1=b[:, :N - 8]), dict(glu=True, add1=b)):
+        with pytest.raises(RuntimeError):
+            h.forward(x, **kw)
+
+
 # ---- lin_sk_kernel (round 3): the decode GEMV dealt over all CUs ----------------------------------------------------------
 # Shapes: DeepSeek-V3 linears (k-steps 56 / 128 / 144 / 12 / 16 -> ring depths 7 / 8 / 6 / 4), a glu pair, ragged N.
 SK_SHAPES = [(7168, 2112), (16384, 7168), (18432, 1024), (1536, 3072), (2048, 7168), (7168, 4096), (896, 200), (1408, 512)]
