@@ -843,7 +843,8 @@ class LinearHandle:
         if x.dtype != torch.bfloat16 or x.shape[-1] != self.K or x.device != self.device:
             raise KtxError(f"forward: expected bf16 [..., {self.K}] on {self.device}, got {x.dtype} {tuple(x.shape)} on {x.device}")
         x2 = x if x.dim() == 2 else x.reshape(-1, self.K)
-        strided = x2.dim() == 2 and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and x2.stride(0) != self.K
+        # (one row expanded to T has stride 0, which a fusion's x_ld reads as dense rows)
+        strided = x2.dim() == 2 and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and x2.stride(0) != self.K and x2.stride(0) != 0
         if not x2.is_contiguous() and not strided:
             x2 = x2.contiguous()
             strided = False
@@ -892,6 +893,8 @@ class LinearHandle:
                 a2 = a.reshape(-1, self.N)
                 if a2.dtype != torch.bfloat16 or a2.shape[0] != T or a2.stride(1) != 1 or a2.device != self.device:
                     raise KtxError(f"forward: {name} must be bf16 [{T}, {self.N}] on {self.device}")
+                if a2.stride(0) == 0:   # (one row expanded to T: a leading dimension of 0 means dense rows)
+                    a2 = a2.contiguous()
                 setattr(fu, name, a2.data_ptr())
                 setattr(fu, name + "_ld", a2.stride(0))
                 keep.append(a2)
@@ -947,6 +950,8 @@ class LinearHandle:
                 a2 = a.reshape(-1, self.N)
                 if a2.dtype != torch.bfloat16 or a2.shape[0] != T or a2.stride(1) != 1 or a2.device != self.device:
                     raise KtxError(f"forward: {name} must be bf16 [{T}, {self.N}] on {self.device}")
+                if a2.stride(0) == 0:   # (one row expanded to T: a leading dimension of 0 means dense rows)
+                    a2 = a2.contiguous()
                 setattr(fu, name, a2.data_ptr())
                 setattr(fu, name + "_ld", a2.stride(0))
                 keep.append(a2)

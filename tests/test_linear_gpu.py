@@ -631,6 +631,24 @@ def test_a_w4_prompt_adds_what_torch_adds():
             h.forward(x, **kw)
 
 
+@pytest.mark.parametrize("fmt,T", [("W4", 600), ("W4", 700), ("W4", 40), ("FP8", 3), ("BF16", 300)])
+def test_one_row_expanded_to_many(fmt, T):
+    """Inputs and addends of stride 0 are the row that they repeat, on the tiles, the GEMM and the decode kernel."""
+    n = native()
+    K, N = 2048, 2112
+    torch.manual_seed(T)
+    h = n.LinearHandle(K, N, fmt, {"W4": 64, "FP8": 128, "BF16": 0}[fmt], 1024)
+    w = (torch.randn(N, K) / 10).to(torch.bfloat16).cuda()
+    if fmt == "FP8":
+        h.load_fp8((w.float() * 4).to(torch.float8_e4m3fn), ((torch.rand((N + 127) // 128, K // 128) + 0.5) / 32).cuda())
+    else:
+        h.load_bf16(w)
+    x, a = (torch.randn(1, K) / 10).to(torch.bfloat16).cuda().expand(T, K), torch.randn(1, N).to(torch.bfloat16).cuda().expand(T, N)
+    xc, ac = x.contiguous(), a.contiguous()
+    assert torch.equal(h.forward(x), h.forward(xc))
+    assert torch.equal(h.forward(x, add1=a, add2=a), h.forward(xc, add1=ac, add2=ac))
+
+
 # ---- lin_sk_kernel (round 3): the decode GEMV dealt over all CUs ----------------------------------------------------------
 # Shapes: DeepSeek-V3 linears (k-steps 56 / 128 / 144 / 12 / 16 -> ring depths 7 / 8 / 6 / 4), a glu pair, ragged N.
 SK_SHAPES = [(7168, 2112), (16384, 7168), (18432, 1024), (1536, 3072), (2048, 7168), (7168, 4096), (896, 200), (1408, 512)]
