@@ -184,24 +184,33 @@ __device__ __forceinline__ void lin_step(const uint4 (&w)[Fmt<FMT, G>::NQ], cons
   }
 }
 
+// TORCH: subnormal results are kept, as torch's cast and the GEMM's epilogue keep them (f32_to_bf16 makes them 0)
+template <bool TORCH = false>
+__device__ __forceinline__ bf16_t lin_round(float v) {
+  if constexpr (TORCH) return (bf16_t)(ktx_pk_bf16(v, 0.f) & 0xffffu);
+  else return f32_to_bf16(v);
+}
+template <bool TORCH = false>
 __device__ __forceinline__ bf16_t lin_out(float v, const bf16_t* bias, int n) {
-  bf16_t o = f32_to_bf16(v);
-  if (bias) o = f32_to_bf16(bf16_to_f32(o) + bf16_to_f32(bias[n]));   // x = gemm(...); x = x + bias (linear.py:709)
+  bf16_t o = lin_round<TORCH>(v);
+  if (bias) o = lin_round<TORCH>(bf16_to_f32(o) + bf16_to_f32(bias[n]));   // x = gemm(...); x = x + bias (linear.py:709)
   return o;
 }
 // bf16 tensor adds that follow the linear in the decoder layer (residual + attn_out; routed + shared; residual + mlp_out:
 // modeling_deepseek_v3.py:1219,1225, :529), each with torch's bf16 rounding, folded into the epilogue
+template <bool TORCH = false>
 __device__ __forceinline__ bf16_t lin_addends(bf16_t o, const LinParams& p, int row, int n) {
-  if (p.add1) o = f32_to_bf16(bf16_to_f32(p.add1[(size_t)row * p.ld1 + n]) + bf16_to_f32(o));
-  if (p.add2) o = f32_to_bf16(bf16_to_f32(p.add2[(size_t)row * p.ld2 + n]) + bf16_to_f32(o));
+  if (p.add1) o = lin_round<TORCH>(bf16_to_f32(p.add1[(size_t)row * p.ld1 + n]) + bf16_to_f32(o));
+  if (p.add2) o = lin_round<TORCH>(bf16_to_f32(p.add2[(size_t)row * p.ld2 + n]) + bf16_to_f32(o));
   return o;
 }
 // DeepseekV3MLP (modeling_deepseek_v3.py:396-398) between the merged gate|up GEMV and down_proj, in bf16 tensor arithmetic:
 // bf16(silu(bf16 g)) * bf16 u -> bf16
+template <bool TORCH = false>
 __device__ __forceinline__ bf16_t lin_glu(float g, float u) {
-  const float gb = bf16_to_f32(f32_to_bf16(g)), ub = bf16_to_f32(f32_to_bf16(u));
-  const float sb = bf16_to_f32(f32_to_bf16(gb / (1.0f + expf(-gb))));
-  return f32_to_bf16(sb * ub);
+  const float gb = bf16_to_f32(lin_round<TORCH>(g)), ub = bf16_to_f32(lin_round<TORCH>(u));
+  const float sb = bf16_to_f32(lin_round<TORCH>(gb / (1.0f + expf(-gb))));
+  return lin_round<TORCH>(sb * ub);
 }
 // 8 bf16 of an input row -> RMSNorm'ed (DeepseekV3RMSNorm.forward: w * bf16(x * r), both roundings as torch's bf16 cast)
 __device__ __forceinline__ uint4 lin_norm8(const uint4& v, float r, const bf16_t* __restrict__ w8) {

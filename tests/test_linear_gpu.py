@@ -649,6 +649,20 @@ def test_one_row_expanded_to_many(fmt, T):
     assert torch.equal(h.forward(x, add1=a, add2=a), h.forward(xc, add1=ac, add2=ac))
 
 
+@pytest.mark.parametrize("K,N,T", [(2048, 272, 520), (7168, 272, 520), (2048, 2112, 600)])      # K in one piece; in pieces that another launch adds
+def test_a_w4_prompt_keeps_subnormal_results(K, N, T):
+    """Outputs under 2^-126, and sums and GLU products of such, are those of the GEMM and of torch.  A row of x is one power of two, so that an output is one product and
+    its bits don't depend on the order of the sums."""
+    h, _, on_the_gemm = w4_prompt_both_ways(K, N, T)
+    x = torch.zeros((T, K), dtype=torch.bfloat16, device="cuda")
+    x[torch.arange(T), torch.randint(0, K, (T,))] = (2.0 ** -torch.randint(40, 132, (T,)).float()).to(torch.bfloat16).cuda()
+    a = (torch.randn((T, N), device="cuda") * 2.0 ** -128).to(torch.bfloat16)
+    for kw in (dict(), dict(add1=a), dict(add1=a, add2=-a), dict(glu=True)):
+        want, got = on_the_gemm(x, **kw), h.forward(x, **kw)
+        small = (want != 0) & (want.float().abs() < 2.0 ** -126)
+        assert float(small.float().mean()) > 0.005 and torch.equal(got, want)
+
+
 # ---- lin_sk_kernel (round 3): the decode GEMV dealt over all CUs ----------------------------------------------------------
 # Shapes: DeepSeek-V3 linears (k-steps 56 / 128 / 144 / 12 / 16 -> ring depths 7 / 8 / 6 / 4), a glu pair, ragged N.
 SK_SHAPES = [(7168, 2112), (16384, 7168), (18432, 1024), (1536, 3072), (2048, 7168), (7168, 4096), (896, 200), (1408, 512)]
