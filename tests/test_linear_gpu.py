@@ -663,6 +663,34 @@ def test_a_w4_prompt_keeps_subnormal_results(K, N, T):
         assert float(small.float().mean()) > 0.005 and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("G", [32, 64, 128])
+@pytest.mark.parametrize("K,N,T", [(2048, 264, 520), (2048, 4096, 512)])      # 64 x 64 tiles, 64 x 128 tiles
+def test_w4_prompts_of_any_scale(G, K, N, T):
+    """Scales of 0, subnormal, tiny, 2^124 and more, infinite and NaN: the tiles' multiplicand is ktx_linear_dequant_bf16's.  A row of x is one power of two, so that an
+    output is one product."""
+    n = native()
+    g = torch.Generator().manual_seed(G + N)
+    q = torch.randint(0, 16, (K, N), generator=g, dtype=torch.uint8)
+    special = torch.tensor([0.0, 2.0 ** -133, 2.0 ** -127, -2.0 ** -120, 1.0, -3.0, 2.0 ** 124, 2.0 ** 125, -2.0 ** 126, 3.3e38, float("inf"), float("-inf"), float("nan")]).to(torch.bfloat16)
+    s = special[torch.randint(0, 10, (K // G, N), generator=g)]
+    s[:, :len(special)] = special          # (an infinite weight makes every output of its column NaN: in these columns, and in the others q - 8 is what s leaves room for)
+    room = (3.38e38 / s.float().abs()).clamp(max=8).floor().repeat_interleave(G, dim=0)[:, len(special):]
+    q[:, len(special):] = torch.minimum(torch.maximum(q[:, len(special):].float(), 8 - room), 8 + room).clamp(0, 15).to(torch.uint8)
+    h = n.LinearHandle(K, N, "W4", G, T)
+    h.load_w4(q.cuda(), s.cuda())
+    assert h._w4_prompt_on_tiles(T)
+    x = torch.zeros((T, K), dtype=torch.bfloat16)
+    x[torch.arange(T), torch.randint(0, K, (T,), generator=g)] = 0.25
+    y = h.forward(x.cuda())
+    h._w4_prompt_on_tiles = lambda T: False
+    want = h.forward(x.cuda())
+    assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y[~y.isnan()], want[~want.isnan()])
+    # (q - 8) s, rounded to bf16, with q - 8 in 64 bits
+    w = ((q.double() - 8.0) * s.double().repeat_interleave(G, dim=0)).float().to(torch.bfloat16)
+    finite = w.float().isfinite().all(0)
+    assert 0.9 < float(finite.float().mean()) < 1 and torch.equal(y.cpu()[:, finite].float(), (x.float() @ w[:, finite].float()).to(torch.bfloat16).float())
+
+
 # ---- lin_sk_kernel (round 3): the decode GEMV dealt over all CUs ----------------------------------------------------------
 # Shapes: DeepSeek-V3 linears (k-steps 56 / 128 / 144 / 12 / 16 -> ring depths 7 / 8 / 6 / 4), a glu pair, ragged N.
 SK_SHAPES = [(7168, 2112), (16384, 7168), (18432, 1024), (1536, 3072), (2048, 7168), (7168, 4096), (896, 200), (1408, 512)]
