@@ -854,11 +854,15 @@ class LinearHandle:
         # kernels, which take any out_features)
         w4_prompt = self.fmt == "W4" and T >= self.PROMPT_MIN_T
         fp8_prompt = self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and T * self.N > self.FP8_GEMM_OUT[T > 1024 and self.K > 2048]
-        rounded = False
+        rounded, ws = False, None
         if ((w4_prompt or fp8_prompt) and self.batch == 1 and bsz_tensor is None and self.N % 8 == 0 and self.K % 64 == 0 and x2.data_ptr() % 16 == 0
                 and (x2.stride(0) * 2) % 16 == 0 and not os.environ.get("KTX_W4_PROMPT_KERNEL" if w4_prompt else "KTX_FP8_PROMPT_KERNEL")
                 and not torch.cuda.is_current_stream_capturing()):
             rounded = w4_prompt and not os.environ.get("KTX_VENDOR_GEMM") and self._w4_prompt_on_tiles(T) and self._tiles_write(x2, out, [a for a in (add1, add2) if a is not None], glu)
+            if rounded:
+                need = self._scratch(T, True)   # (W4: the same with a fusion)
+                ws = self._workspace(need)
+                rounded = ws is not None or not need   # (the strip kernels, which need no scratch, don't round the weights: without memory for it the call is the GEMM's)
             if not rounded:
                 if norm is not None:
                     x2 = rmsnorm(x2.contiguous(), norm[0], norm[1], native_rounding=True)
@@ -874,7 +878,7 @@ class LinearHandle:
         if norm is None and add1 is None and add2 is None and not strided and not glu:
             need = self._scratch(T, bsz is None) if T > 8 else None
             if need is not None:
-                self._forward_ws(bsz, T, x2, out, None, need, rounded)
+                self._forward_ws(bsz, T, x2, out, None, need, rounded, ws)
             else:
                 check(lib.ktx_linear_forward(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), _stream_ptr(self.device)))
             return out if x.dim() == 2 and out.shape == (T, self.N) else out.reshape(*x.shape[:-1], self.N)
@@ -900,7 +904,7 @@ class LinearHandle:
                 keep.append(a2)
         need = self._scratch(T, False) if T > 8 else None
         if need is not None:
-            self._forward_ws(bsz, T, x2, out, C.byref(fu), need, rounded)
+            self._forward_ws(bsz, T, x2, out, C.byref(fu), need, rounded, ws)
         else:
             check(lib.ktx_linear_forward_fused(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), C.byref(fu), _stream_ptr(self.device)))
         return out.reshape(*x.shape[:-1], n_out)
@@ -913,16 +917,21 @@ class LinearHandle:
             self._ws_need[key] = int(lib.ktx_linear_workspace_bytes(self._h, T, int(plain))) if lib.ktx_linear_tiled(self._h, T) else None
         return self._ws_need[key]
 
-    def _forward_ws(self, bsz, T: int, x2: torch.Tensor, out: torch.Tensor, fu, need: int, rounded: bool = False) -> None:
-        """ktx_linear_forward_ws with its scratch from torch's allocator (freed to the stream's pool behind the launches).  FP8 prompts take the
-        K = 128 MFMA whether the call is eager, captured or has its row count on the device."""
+    def _workspace(self, need: int):
+        """`need` bytes of scratch from torch's allocator (freed to the stream's pool behind the launches that take it), or None where there are none."""
         try:
-            ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
-        except torch.cuda.OutOfMemoryError:   # (the strip kernels need none)
-            ws, need = None, 0
+            return torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
+        except torch.cuda.OutOfMemoryError:
+            return None
+
+    def _forward_ws(self, bsz, T: int, x2: torch.Tensor, out: torch.Tensor, fu, need: int, rounded: bool = False, ws: torch.Tensor | None = None) -> None:
+        """ktx_linear_forward_ws with scratch of its own unless `ws` holds it; without memory for it the strip kernels, which need none.  FP8 prompts take
+        the K = 128 MFMA whether the call is eager, captured or has its row count on the device."""
+        if ws is None:
+            ws = self._workspace(need)
         prompt = self.fmt == "FP8" and T >= self.FP8_PROMPT_MIN_T and not os.environ.get("KTX_FP8_PROMPT_KERNEL")
-        check(lib.ktx_linear_forward_ws(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), fu, 2 if rounded else 1 if prompt else 0, ws.data_ptr() if ws is not None else None, need,
-                                        _stream_ptr(self.device)))
+        check(lib.ktx_linear_forward_ws(self._h, bsz, T, x2.data_ptr(), out.data_ptr(), fu, 2 if rounded else 1 if prompt else 0, ws.data_ptr() if ws is not None else None,
+                                        need if ws is not None else 0, _stream_ptr(self.device)))
 
     def _forward_glu_in(self, x, bsz_tensor, out, norm, add1, add2, glu):
         if norm is not None or glu:

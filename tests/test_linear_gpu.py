@@ -1120,6 +1120,25 @@ def test_a_batch_without_memory_for_scratch_runs_on_the_strip_kernels(monkeypatc
     close(y, linear_w4_ref(x, *quantize_weights_ref(w.T.contiguous(), 64), 64))
 
 
+def test_a_w4_prompt_without_memory_for_scratch_multiplies_the_rounded_weights(monkeypatch):
+    """Where the allocator has none left for the tiles' scratch a W4 prompt is the GEMM's, with its multiplicand, not the strip kernels'."""
+    K, N, T = 7168, 264, 520
+    h, x, on_the_gemm = w4_prompt_both_ways(K, N, T)
+    want, nw = on_the_gemm(x), torch.ones(K, dtype=torch.bfloat16, device="cuda")
+    want_norm = on_the_gemm(x, norm=(nw, 1e-6))
+    assert h._scratch(T, True) and not torch.equal(h.forward(x), want)     # (the tiles cut K: other last bits)
+    real = torch.empty
+
+    def empty(*a, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.cuda.OutOfMemoryError("none left")
+        return real(*a, **kw)
+    monkeypatch.setattr(torch, "empty", empty)
+    got, got_norm = h.forward(x), h.forward(x, norm=(nw, 1e-6))
+    monkeypatch.undo()
+    assert torch.equal(got, want) and torch.equal(got_norm, want_norm)
+
+
 def test_calls_go_to_the_current_stream_of_their_device():
     """The raw accessor of the current stream gives torch's own handle, on the default stream and on others, for devices with and without an index."""
     n = native()
