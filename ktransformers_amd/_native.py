@@ -709,15 +709,27 @@ class LinearHandle:
         return out
 
     def _w4_prompt_on_tiles(self, T: int) -> bool:
-        """Whether the tiles of ktx_linear_forward_ws take a W4 prompt, with Marlin's multiplicand formed in registers, rather than the expansion
-        and the GEMM: the same sums of the same products (in another order where K is cut).  Us, GEMM | tiles: few outputs, 512 rows of 4096 -> 1000 50 | 18, 2048 of them 51 | 39, of
-        2048 -> 576 30 | 21; long K, 512 of 16384 -> 7168 320 | 167, 1000 322 | 278, 800 of 7168 -> 2112 88 | 71, 1000 of 7168 -> 18432 392 | 373, 1400 of 7168 -> 4096 121 | 140; between them
-        640 of 2048 -> 3072 33 | 20, 512 of 1024 -> 4096 23 | 17, 800 equal, 640 of 2048 -> 7168 42 | 48, 512 of 5120 -> 9000 98 | 100."""
+        """Whether the tiles of ktx_linear_forward_ws take a W4 prompt, with Marlin's multiplicand formed in registers, rather than the expansion and the GEMM: the same
+        sums of the same products, in another order where K is cut (so that a prompt's last bits depend on out_features as well: alone or merged).  The lines are those
+        of 117 sizes (128 to 18432 inputs, 264 to 32768 outputs) at 10 row counts each, where none of the calls that the tiles take was slower there by more than 1 %.  Us, GEMM | tiles:
+          few outputs: 512 rows of 4096 -> 1000 50 | 18, 2048 of them 51 | 39;
+          short K, few rows: 640 of 2048 -> 4096 35 | 33; no more 64 x 128 tiles than CUs, 512 of 4096 -> 4096 54 | 37 (576 54 | 56);
+          long K: no more tiles than CUs, 800 of 16384 -> 2112 176 | 149 (1000 177 | 185); to 4096 outputs, 1000 of 7168 -> 4096 95 | 77, of 16384 -> 4096 193 | 149; 512 rows, which K's
+          quarters suit, of 16384 -> 7168 325 | 154, of 7168 -> 12000 136 | 125; less than two tiles a CU, 640 of 10240 -> 5120 140 | 123 (800 159 | 177); expanded weights that the 256 MB
+          behind the L2s don't hold, 800 of 16384 -> 9000 358 | 278, 640 of 7168 -> 18432 315 | 249 (640 of 7168 -> 7168 118 | 133, 1000 of 8192 -> 28672 532 | 556)."""
         if getattr(self, "_bias_t", None) is not None:   # (the GEMM adds a bias to the sum, the tiles to the rounded sum)
             return False
-        if not (T <= 2048 if self.N <= 1024 else T <= 1024 if self.K >= 7168 else T <= 640 and self.N <= 4096):
+        if self.K % 128 != 0 or self._scratch(T, True) is None:
             return False
-        return self.K % 128 == 0 and self._scratch(T, True) is not None
+        K, N, tiles = self.K, self.N, -(-T // 64) * -(-self.N // 128)
+        if N <= 1024:
+            return T <= 2048
+        if K < 7168:
+            return T <= 640 and N <= 4096 and (tiles <= 256 or K <= 3072 or K >= 5120)
+        if T > 1024:
+            return False
+        return (tiles <= 256 or T <= 512 or (N <= 4096 and (K < 16384 or N > 3072)) or (tiles <= 448 and K < 16384)
+                or (N * K >= 112 << 20 and (K >= 10240 or T <= 832)))
 
     def _tiles_write(self, x2: torch.Tensor, out: torch.Tensor | None, addends: list, glu: bool) -> bool:
         """Whether the tiles may store a W4 prompt's rows, dense bf16, straight into `out` (other workgroups read x2 and the addends meanwhile) and their epilogue
