@@ -2215,7 +2215,7 @@ extern "C" int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T
   if (h->cfg.format == KTX_LIN_FP8) {
     const int rc = ktx_fp8_act_quant_padded(d_x, ldx, T, p.Kx, (void*)q.xq, (float*)q.sT, q.s_ld, stream);
     if (rc) return rc;
-    return prompt && o.mt >= 4 ? forward_tile<F_FP8, 128, 1>(o, q, st) : forward_tile<F_FP8, 128>(o, q, st);
+    return prompt && o.mt >= 3 ? forward_tile<F_FP8, 128, 1>(o, q, st) : forward_tile<F_FP8, 128>(o, q, st);   // (from 33 rows on)
   }
   const int g = h->cfg.group_size;
   if (o.sT_bytes) {

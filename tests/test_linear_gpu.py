@@ -1035,6 +1035,30 @@ def test_tiles_of_48_rows(fmt, group, K, N):
         assert torch.equal(h.forward(x[:T]), want[:T]), f"{T} rows"
 
 
+@pytest.mark.parametrize("K,N", [(2816, 8200), (4096, 12000), (2176, 32768)])     # tiles of 48 rows and 64, 256 and 128 features
+def test_fp8_prompts_of_33_rows_and_more_take_the_k_128_mfma(K, N):
+    """ktx_linear_forward_ws with prompt = 1, which holds past 32 rows: 33 to 48 have the bits that they have among 49, on tiles of 64 rows.  Magnitudes over many
+    powers of two, half of them cancelling: 8 results in 100000 show the order of the sums (none does with normal weights)."""
+    n = native()
+    g = torch.Generator().manual_seed(K + N)
+    h = n.LinearHandle(K, N, "FP8", 128, 64)
+    w = torch.randn((N, K), generator=g).abs() * torch.exp2(torch.randint(-12, 4, (N, K), generator=g).float())
+    x = torch.randn((49, K), generator=g) * torch.exp2(torch.randint(-12, 8, (49, K), generator=g).float())
+    x[:, 0::2] = -x[:, 1::2]
+    h.load_fp8((w * 100).clamp_(max=448).to(torch.float8_e4m3fn).cuda(), torch.rand((-(-N // 128), K // 128), generator=g).cuda())
+    x = x.to(torch.bfloat16).cuda()
+
+    def forward(T, prompt):
+        y, need = torch.empty((T, N), dtype=torch.bfloat16, device="cuda"), n.lib.ktx_linear_workspace_bytes(h._h, T, 1)
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        n.check(n.lib.ktx_linear_forward_ws(h._h, None, T, x.data_ptr(), y.data_ptr(), None, prompt, ws.data_ptr(), need, n._stream_ptr(x.device)))
+        return y
+    want, other = forward(49, 1), forward(49, 0)
+    for T in (33, 47, 48):
+        assert torch.equal(forward(T, 1), want[:T]), f"{T} rows"
+        assert torch.equal(forward(T, 0), other[:T]) and not torch.equal(other[:T], want[:T])
+
+
 @pytest.mark.parametrize("N", [24576, 24584])
 def test_bf16_prompts_on_the_gemm_of_decode_tiles(N):
     """520 rows of 2048 -> 24576 (whole strips) and 24584 (half a strip at the end) fill the chip with 256 x 256 tiles over the whole K: the GEMM
