@@ -99,3 +99,21 @@ def test_no_request_outlives_its_workgroup(kernel, tmp_path):
                 assert requests and not bad, f"{part.split(chr(10), 1)[0]}: {len(bad)} of {requests} requests may outlive the workgroup"
                 seen += 1
     assert seen, f"{kernel}: not in {build.LIB}"
+
+
+def test_scales_are_read_behind_a_wait_for_them(tmp_path):
+    """lin_tile_kernel's FP8 weight scales come by LDS-DMA, which the compiler doesn't see, and are read back as ordinary memory: a wait for requests lies between in the listing."""
+    if not os.path.exists(build.LIB) or not os.path.exists(OBJDUMP):
+        pytest.skip("needs the built library and llvm-objdump")
+    kernel, seen = "lin_tile_kernelILi2E", 0
+    for code in code_objects(build.LIB):
+        if kernel.encode() not in code:
+            continue
+        (tmp_path / "code.o").write_bytes(code)
+        text = subprocess.run([OBJDUMP, "-d", str(tmp_path / "code.o")], check=True, capture_output=True, text=True).stdout
+        for part in re.split(r"\n(?=[0-9a-f]+ <)", text):
+            if kernel in part.split("\n", 1)[0]:
+                behind = re.split(r"\sglobal_load_lds_dword\s", part)[1:]
+                assert len(behind) >= 2 and all("vmcnt(" in b.split("ds_read_b32")[0] for b in behind), part.split("\n", 1)[0]
+                seen += 1
+    assert seen, f"{kernel}: not in {build.LIB}"
