@@ -496,13 +496,14 @@ def test_qb_absorb_and_prep_in_one_launch(H, T):
 
 
 @pytest.mark.parametrize("K,N,G", [(2048, 576, 64), (7168, 1536, 64), (1536, 208, 128)])
-def test_prompt_sized_w4_dequantises_once_and_runs_a_library_gemm(K, N, G):
-    """T >= LinearHandle.PROMPT_MIN_T: the W4 weights are expanded once with Marlin's in-register rounding bf16((q - 8) * s)
-    (ktx_linear_dequant_bf16: bit-identical to the torch expression on the reference quantiser's q and s) and a plain library
+def test_prompt_sized_w4_dequantises_once_and_runs_a_library_gemm(K, N, G, monkeypatch):
+    """T >= LinearHandle.PROMPT_MIN_T, where the tiles don't take the call (held off here): the W4 weights are expanded once with Marlin's in-register rounding
+    bf16((q - 8) * s) (ktx_linear_dequant_bf16: bit-identical to the torch expression on the reference quantiser's q and s) and a plain library
     GEMM runs on them — against fp64 math on the same rounded weights, against the hand-written W4 GEMM, and with the GLU /
     addend epilogues of the decoder layer."""
     import os
     n = native()
+    monkeypatch.setattr(n.LinearHandle, "_w4_prompt_on_tiles", lambda self, T: False)
     torch.manual_seed(K + N)
     T = n.LinearHandle.PROMPT_MIN_T + 40
     w = (torch.randn(N, K) / 10).to(torch.bfloat16).cuda()
@@ -647,6 +648,32 @@ def test_one_row_expanded_to_many(fmt, T):
     xc, ac = x.contiguous(), a.contiguous()
     assert torch.equal(h.forward(x), h.forward(xc))
     assert torch.equal(h.forward(x, add1=a, add2=a), h.forward(xc, add1=ac, add2=ac))
+
+
+@pytest.mark.parametrize("K,N,T,G", [(4096, 4096, 512, 64), (7168, 18440, 520, 128), (7168, 4096, 1000, 32)])     # K cut, another launch adds; K whole, strips and rows absent; K cut in two
+def test_w4_prompts_on_tiles_of_128_rows(K, N, T, G):
+    """The rounded multiplicand on tiles of 128 rows and 256 features: rows of one power of two give the GEMM's bits (an output is one product), random ones differ in fewer than
+    1 in 100 and by a bf16 step (see above), and RMSNorm in front, rows that lie further apart and a dense `out` change nothing."""
+    n = native()
+    h, x, on_the_gemm = w4_prompt_both_ways(K, N, T, G)
+    ones = torch.zeros_like(x)
+    ones[torch.arange(T), torch.randint(0, K, (T,))] = (2.0 ** torch.randint(-4, 5, (T,)).float()).to(torch.bfloat16).cuda()
+    n.timing_enable(2)
+    try:
+        y = h.forward(ones)
+        labels = [t[0] for t in n.timing_collect()]
+    finally:
+        n.timing_enable(0)
+    assert any(t.startswith("lin_tile_kernel<W4,MT8,NW8,NSW2>") for t in labels), labels
+    assert torch.equal(y, on_the_gemm(ones))
+    y, want = h.forward(x), on_the_gemm(x)
+    assert float((y != want).float().mean()) < 0.01
+    torch.testing.assert_close(y.float(), want.float(), rtol=2.0 ** -7, atol=1e-5)
+    far = torch.zeros((T, K + 64), dtype=torch.bfloat16, device="cuda")[:, :K]
+    far.copy_(x)
+    out, nw = torch.empty_like(y), (1 + torch.randn(K) / 10).to(torch.bfloat16).cuda()
+    assert torch.equal(h.forward(far), y) and h.forward(x, out=out) is out and torch.equal(out, y)
+    assert torch.equal(h.forward(far, norm=(nw, 1e-6)), h.forward(n.rmsnorm(x, nw, 1e-6)))
 
 
 @pytest.mark.parametrize("K,N,T", [(2048, 272, 520), (7168, 272, 520), (2048, 2112, 600)])      # K in one piece; in pieces that another launch adds
@@ -958,8 +985,8 @@ def test_batches_and_short_prompts_on_tiles(fmt, K, N, T):
 @pytest.mark.parametrize("G", [32, 64, 128])
 @pytest.mark.parametrize("K,N,T,how", [(2048, 577, 513, "odd"), (1024, 1000, 512, "rows"), (7168, 264, 640, "capture"), (2048, 12296, 600, "rows"), (384, 33, 1030, "odd")])
 def test_w4_prompts_off_the_gemm_multiply_exact_integers(G, K, N, T, how):
-    """512 rows and more that the expansion GEMM doesn't take (out_features % 8 != 0, a device-side row count, stream capture) multiply
-    (q - 8) exactly and scale in fp32; only the GEMM's multiplicand is rounded to bf16.  Against 64-bit sums an exact product is off by the
+    """512 rows and more that the prompt path doesn't take (out_features % 8 != 0, a device-side row count, stream capture) multiply
+    (q - 8) exactly and scale in fp32; only that path's multiplicand is rounded to bf16.  Against 64-bit sums an exact product is off by the
     outputs' rounding alone: uniform in half an ulp, 2^-8 / sqrt(12) = 1.1e-3 of a power of two and 1.66e-3 in the norm over mantissas; the
     rounded multiplicand adds an independent error to every term whose (q - 8) * s doesn't fit bf16: 2.1e-3 and more.  2.0e-3 parts the two."""
     n = native()
@@ -987,7 +1014,7 @@ def test_w4_prompts_off_the_gemm_multiply_exact_integers(G, K, N, T, how):
             g.replay()
             torch.cuda.synchronize()
             assert float((y.double() - want).norm() / want.norm()) < 2.0e-3
-        assert float((eager.double() - want).norm() / want.norm()) > 2.0e-3     # (the eager call is the GEMM's)
+        assert float((eager.double() - want).norm() / want.norm()) > 2.0e-3     # (the eager call rounds the weights)
     close(y, want.float().cpu())
     assert float((y.double() - want).norm() / want.norm()) < 2.0e-3
 
