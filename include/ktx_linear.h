@@ -121,7 +121,8 @@ int ktx_linear_decode_eligible(ktx_linear_t h, int T);
  * ktx_linear_forward_fused.  `fusion` may be NULL.
  * prompt (FP8, T > 32): 1 takes a 128-block in one K = 128 MFMA instead of four of K = 32 (the order of ktx_linear_forward): the same
  * error against 64-bit sums, other last bits.  W4 multiplies exact integers, as ktx_linear_forward does; with prompt = 2 and more than 64 rows the multiplicand of
- * ktx_linear_dequant_bf16. */
+ * ktx_linear_dequant_bf16, with the GEMM's rounding of the result (subnormals kept) and the bias added to the rounded sum; on the tiles only: without d_ws, or in a call that
+ * they don't cover, exact integers again. */
 size_t ktx_linear_workspace_bytes(ktx_linear_t h, int T, int plain);
 int ktx_linear_tiled(ktx_linear_t h, int T);   /* 1: ktx_linear_forward_ws takes T rows on the tiles (or the GEMM), given its scratch */
 int ktx_linear_forward_ws(ktx_linear_t h, const int32_t* d_bsz, int T, const void* d_x, void* d_y, const ktx_linear_fusion* fusion,

@@ -694,9 +694,10 @@ class LinearHandle:
         self._ws_need.clear()
         return self._bias_t
 
-    # ---- prompt-sized W4 calls: de-quantise once (Marlin's rounding), then the library's own BF16 GEMM (csrc/ktx_gemm.hip;
-    # KTX_VENDOR_GEMM=1 sends the product to torch's F.linear instead — the A/B switch of scripts/gemm_bench.py) ------------
-    PROMPT_MIN_T = 512          # below this, and for calls that the GEMM doesn't take: exact integer weights (ktx_linear_forward_ws)
+    # ---- prompt-sized W4 calls: Marlin's rounded multiplicand, formed in the tiles' registers (ktx_linear_forward_ws, prompt = 2) where _w4_prompt_on_tiles says so,
+    # else de-quantised once for the library's own BF16 GEMM (csrc/ktx_gemm.hip; KTX_VENDOR_GEMM=1 sends the product to torch's F.linear instead — the A/B switch of
+    # scripts/gemm_bench.py) ------------
+    PROMPT_MIN_T = 512          # below this, and for calls that neither takes (out_features % 8, a row count on the device, stream capture): exact integer weights
     _DEQ_SCRATCH: dict = {}
 
     def dequant_bf16(self, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -710,26 +711,24 @@ class LinearHandle:
 
     def _w4_prompt_on_tiles(self, T: int) -> bool:
         """Whether the tiles of ktx_linear_forward_ws take a W4 prompt, with Marlin's multiplicand formed in registers, rather than the expansion and the GEMM: the same
-        sums of the same products, in another order where K is cut (so that a prompt's last bits depend on out_features as well: alone or merged).  The lines are those
-        of 117 sizes (128 to 18432 inputs, 264 to 32768 outputs) at 10 row counts each, where none of the calls that the tiles take was slower there by more than 1 %.  Us, GEMM | tiles:
-          few outputs: 512 rows of 4096 -> 1000 50 | 18, 2048 of them 51 | 39;
-          short K, few rows: 640 of 2048 -> 4096 35 | 33; no more 64 x 128 tiles than CUs, 512 of 4096 -> 4096 54 | 37 (576 54 | 56);
-          long K: no more tiles than CUs, 800 of 16384 -> 2112 176 | 149 (1000 177 | 185); to 4096 outputs, 1000 of 7168 -> 4096 95 | 77, of 16384 -> 4096 193 | 149; 512 rows, which K's
-          quarters suit, of 16384 -> 7168 325 | 154, of 7168 -> 12000 136 | 125; less than two tiles a CU, 640 of 10240 -> 5120 140 | 123 (800 159 | 177); expanded weights that the 256 MB
-          behind the L2s don't hold, 800 of 16384 -> 9000 358 | 278, 640 of 7168 -> 18432 315 | 249 (640 of 7168 -> 7168 118 | 133, 1000 of 8192 -> 28672 532 | 556)."""
+        sums of the same products, in another order where K is cut (so that a prompt's last bits depend on out_features as well: alone or merged).  The lines are those of
+        187 sizes (128 to 18432 inputs, 264 to 32768 outputs) at 9 or 10 row counts each (profiles/w4_prompts_gemm_or_tiles.txt); no call that the tiles take is slower there.
+        Us, GEMM | tiles:
+          few outputs: 512 rows of 4096 -> 1000 50 | 19, 2048 of them 51 | 40; short K, few rows: 640 of 2048 -> 4096 35 | 30;
+          long K: to 4096 outputs, 800 of 16384 -> 2112 177 | 146, 1000 of 7168 -> 4096 95 | 76; 512 rows, which K's quarters suit, of 16384 -> 7168 327 | 154, of 7168 -> 12000 137 | 122;
+          64 x 128 tiles for less than two a CU, 640 of 10240 -> 5120 140 | 115 (800 160 | 174, 640 of 7168 -> 7168 118 | 131); expanded weights that the 256 MB behind the L2s don't
+          hold, 800 of 16384 -> 9000 360 | 275, 640 of 7168 -> 18432 316 | 240 (800 of 7168 -> 12000 207 | 238), past 832 rows to 12288 outputs, where the GEMM hasn't 192 of its
+          largest tiles: 1000 of 16384 -> 7168 324 | 272 (900 of 9472 -> 26136 585 | 614)."""
         if getattr(self, "_bias_t", None) is not None:   # (the GEMM adds a bias to the sum, the tiles to the rounded sum)
             return False
         if self.K % 128 != 0 or self._scratch(T, True) is None:
             return False
-        K, N, tiles = self.K, self.N, -(-T // 64) * -(-self.N // 128)
+        K, N = self.K, self.N
         if N <= 1024:
             return T <= 2048
         if K < 7168:
-            return T <= 640 and N <= 4096 and (tiles <= 256 or K <= 3072 or K >= 5120)
-        if T > 1024:
-            return False
-        return (tiles <= 256 or T <= 512 or (N <= 4096 and (K < 16384 or N > 3072)) or (tiles <= 448 and K < 16384)
-                or (N * K >= 112 << 20 and (K >= 10240 or T <= 832)))
+            return T <= 640 and N <= 4096
+        return T <= 1024 and (N <= 4096 or T <= 512 or -(-T // 64) * -(-N // 128) <= 448 or (N * K >= 112 << 20 and (T <= 832 or N <= 12288)))
 
     def _tiles_write(self, x2: torch.Tensor, out: torch.Tensor | None, addends: list, glu: bool) -> bool:
         """Whether the tiles may store a W4 prompt's rows, dense bf16, straight into `out` (other workgroups read x2 and the addends meanwhile) and their epilogue

@@ -84,12 +84,12 @@ def test_marlin_8bit_multiplicand_matches_the_reference_quantiser(name, G, act):
 
 
 @pytest.mark.parametrize("K,N,T,tiles", [
-    (4096, 1000, 2048, True), (4096, 1000, 2049, False), (4096, 1032, 641, False), (4096, 4096, 512, True), (4096, 4096, 576, False), (3072, 4096, 640, True), (3072, 4096, 641, False),
-    (2048, 4104, 512, False), (5120, 4096, 640, True), (7168, 2112, 1024, True), (7168, 2112, 1025, False), (16384, 2112, 800, True), (16384, 2112, 1000, False), (16384, 4096, 1000, True),
+    (4096, 1000, 2048, True), (4096, 1000, 2049, False), (4096, 1032, 641, False), (3072, 4096, 640, True), (3072, 4096, 641, False),
+    (2048, 4104, 512, False), (7168, 4096, 1024, True), (7168, 4096, 1025, False), (7168, 4104, 1024, False),
     (7168, 5120, 704, True), (7168, 5120, 800, False), (7168, 7168, 512, True), (7168, 7168, 640, False), (7168, 12000, 512, True), (7168, 12000, 800, False), (16384, 7168, 1024, True),
-    (10240, 9000, 1000, False), (7168, 18432, 832, True), (8192, 28672, 1000, False), (4160, 1000, 600, False)])
+    (10240, 9000, 1000, False), (7168, 18432, 832, True), (7168, 18432, 833, False), (10240, 12288, 1024, True), (4160, 1000, 600, False)])
 def test_w4_prompts_that_the_tiles_take(K, N, T, tiles):
-    """LinearHandle._w4_prompt_on_tiles on both sides of its lines, and in calls where the GEMM was measured the faster one by 2 to 23 %."""
+    """LinearHandle._w4_prompt_on_tiles on both sides of its lines, and in calls where the GEMM was measured 7 to 14 % faster."""
     from types import SimpleNamespace
     from ktransformers_amd._native import LinearHandle
     of = lambda scratch, bias: LinearHandle._w4_prompt_on_tiles(SimpleNamespace(K=K, N=N, _bias_t=bias, _scratch=lambda T, plain: scratch), T)
