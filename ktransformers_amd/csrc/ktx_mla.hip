@@ -778,7 +778,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // bytes in flight a thread and fewer workgroups, each of which finds the statistics again.  Us, decode and merge, 16 lanes -> here: 128 heads, 32 of 400 tokens 41.2 -> 31.1, 32 of 1000
 // 45.0 -> 35.6, 16 of 2000 36.3 -> 33.8, 8 of 8192 47.5 -> 46.9; 64 heads, 24 of 500 27.3 -> 25.9, 32 of 2000 38.0 -> 35.5; 8 lanes at ns 51 (5 of 8000) lost, 43.6 -> 44.6.  A token that holds
 // most of an uneven batch's splits goes round more often, and the batch gains all the same: 128 heads, 31 of 400 and one of 9000 49.2 -> 40.4, 19 of 100 and one of 8000 39.6 -> 36.6, 31 of 200
-// and one of 100000 177 -> 169 (profiles/mla_merge_uneven_batches.txt: 26 batches, none slower than its spread).
+// and one of 100000 177 -> 169 (profiles/mla_merge_uneven_batches.txt: 26 batches at 64 and 128 heads, none more than 1.5 % slower).
 template <int NS, bool JOBS, int SL = 16>   // splits per thread and round; JOBS: a token's number of splits is the decode kernel's (njobs); split lanes
 __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p, bf16_t* out, float* lse) {
   constexpr int DG = 256 / SL, DIMS = DG * 8;
