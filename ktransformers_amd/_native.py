@@ -244,6 +244,24 @@ def _register(handle_obj) -> None:
 
 lib = _TracedLib(_load())
 
+
+def _load_host():
+    """csrc/ktx_host.cpp: the shortest calls without an interpreter step per argument.  None where it has not been built: every call is then made from here."""
+    path = os.path.join(_HERE, "lib", "ktx_host.so")
+    if not os.path.exists(path):
+        return None
+    import importlib.machinery
+    import importlib.util
+    loader = importlib.machinery.ExtensionFileLoader("ktx_host", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("ktx_host", loader))
+    loader.exec_module(module)
+    module.bind(KtxError, *(C.cast(getattr(lib._raw, f), C.c_void_p).value
+                            for f in ("ktx_last_error", "ktx_linear_forward", "ktx_moe_forward", "ktx_mla_prefill", "ktx_mla_decode_append")))
+    return module
+
+
+_host = _load_host()   # (its functions return None for what they don't take; calls are recorded here, so TRACE keeps them here)
+
 PROFILE_SLOTS = ("prep", "gate_up_gemm", "act_quant", "down_gemm", "combine")
 
 
@@ -318,12 +336,14 @@ class MoEHandle:
         h = C.c_void_p()
         check(lib.ktx_moe_create(C.byref(cfg), C.byref(h)))
         self._h = h
+        self._host_args = h.value, hidden_size, dev.index
         _register(self)
 
     def close(self) -> None:
         if getattr(self, "_h", None):
             lib.ktx_moe_destroy(self._h)
             self._h = None
+            self._host_args = 0, 0, 0
 
     def __del__(self):
         try:
@@ -437,6 +457,10 @@ class MoEHandle:
     def forward(self, x: torch.Tensor, expert_ids: torch.Tensor, weights: torch.Tensor, out: torch.Tensor | None = None,
                 incremental: bool = False, bsz_tensor: torch.Tensor | None = None) -> torch.Tensor:
         """x bf16 [T,H]; expert_ids int64 [T,k]; weights fp32 [T,k] -> bf16 [T,H].  Enqueues on the current stream."""
+        if out is None and bsz_tensor is None and not incremental and _host is not None and TRACE is None:
+            y = _host.moe(*self._host_args, x, expert_ids, weights)
+            if y is not None:
+                return y
         T, k = expert_ids.shape
         if x.dtype != torch.bfloat16 or x.shape != (T, self.H) or not x.is_contiguous():
             raise KtxError(f"forward: x must be contiguous bf16 [{T},{self.H}]")
@@ -671,12 +695,14 @@ class LinearHandle:
         h = C.c_void_p()
         check(lib.ktx_linear_create(C.byref(cfg), C.byref(h)))
         self._h = h
+        self._host_args = h.value, in_features, out_features, dev.index
         _register(self)
 
     def close(self) -> None:
         if getattr(self, "_h", None):
             lib.ktx_linear_destroy(self._h)
             self._h = None
+            self._host_args = 0, 0, 0, 0
 
     def __del__(self):
         try:
@@ -849,6 +875,10 @@ class LinearHandle:
         ktx_rmsnorm launch where the decode kernel does not run); add1 / add2 = bf16 [..., out] tensors added in that order;
         glu_in: x is bf16 [..., 2 * in] = [gate | up] and the linear reads silu_mul(x) — inside the block-fp8 decode kernel,
         as a separate ktx_silu_mul launch otherwise."""
+        if out is None and bsz_tensor is None and norm is None and add1 is None and add2 is None and not glu and not glu_in and _host is not None and TRACE is None:
+            y = _host.linear(*self._host_args, x)   # (up to 8 dense rows)
+            if y is not None:
+                return y
         if glu_in:
             return self._forward_glu_in(x, bsz_tensor, out, norm, add1, add2, glu)
         if x.dtype != torch.bfloat16 or x.shape[-1] != self.K or x.device != self.device:
@@ -1340,6 +1370,7 @@ class MLAWrapper:
         sizes = (num_heads, head_dim_ckv, head_dim_kpe, page_size, float(sm_scale), self.max_splits, int(max_kv_len))
         if self._sizes != (sizes, self.max_q_tokens):   # (a decode loop plans every step with the same ones)
             self.cfg = _MlaConfig(*sizes)
+            self._cfg_at = C.addressof(self.cfg)
             self._need = int(lib.ktx_mla_workspace_bytes(C.byref(self.cfg), self.max_q_tokens))
             self._sizes = (sizes, self.max_q_tokens)
         need = self._need
@@ -1364,6 +1395,11 @@ class MLAWrapper:
         (the kernel reads position kv_len-1 from these buffers and stores it into the cache pages)."""
         if self.cfg is None:
             raise KtxError("MLAWrapper.run before plan()")
+        if new_ckv is None and new_kpe is None and not return_lse and not partials and _host is not None and TRACE is None:
+            out = _host.mla_decode(self._cfg_at, self.max_q_tokens, self.cfg.page_size, q_nope, q_pe, ckv, k_pe, self.qo_indptr, self.kv_indptr, self.kv_indices,
+                                   self.kv_len_arr, self.bsz_tensor, self.workspace)
+            if out is not None:
+                return out
         T, Hq, dc = q_nope.shape
         if T > self.max_q_tokens:
             raise KtxError(f"MLAWrapper.run: {T} query tokens exceed max_q_tokens={self.max_q_tokens}")
@@ -1430,6 +1466,10 @@ def mla_prefill(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tensor, 
     """Causal non-absorbed prompt attention (include/ktx_mla.h, ktx_mla_prefill).  q_nope [T,H,128] / q_pe [T,H,64] (strided
     views allowed, unit inner stride), k_nope [H,kv_pad,128] contiguous, k_pe [kv_len(+),64] rows with a token stride,
     v_t [H,128,kv_pad] contiguous -> bf16 [T,H,128]; the T queries are the last T of the kv_len keys."""
+    if _host is not None and TRACE is None:
+        out = _host.mla_prefill(q_nope, q_pe, k_nope, k_pe, v_t, kv_len, sm_scale)
+        if out is not None:
+            return out
     T, H, _ = q_nope.shape
     kv_pad = k_nope.shape[1]
     for t, what in ((q_nope, "q_nope"), (q_pe, "q_pe"), (k_nope, "k_nope"), (k_pe, "k_pe"), (v_t, "v_t")):

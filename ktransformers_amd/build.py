@@ -21,6 +21,8 @@ LIB = os.path.join(LIBDIR, "libktx_hip.so")
 # the sequence-mixer, hybrid-decoder, window-attention / scan and decayed-state kernels alone (include/ktx_seq.h, ktx_hyb.h, ktx_swa.h,
 # ktx_gla.h): what the fp32-residual families need, built in about a minute
 SEQ_LIB = os.path.join(LIBDIR, "libktx_seq.so")
+HOST_LIB = os.path.join(LIBDIR, "ktx_host.so")
+HOST_SOURCE = os.path.join(CSRC, "ktx_host.cpp")
 SEQ_SOURCES = ("ktx_seq.hip", "ktx_hyb.hip", "ktx_swa.hip", "ktx_gla.hip", "ktx_err.hip")
 
 # -ffp-contract=off: the parity contract needs every fp32 op rounded exactly as the reference's AVX512 code does;
@@ -95,11 +97,32 @@ def build_seq(force: bool = False, verbose: bool = False) -> str:
     return SEQ_LIB
 
 
+def build_host(force: bool = False, verbose: bool = False) -> str:
+    """The CPython module of the host side (csrc/ktx_host.cpp, against this interpreter's and torch's headers)."""
+    if not force and not _stale(HOST_LIB, [HOST_SOURCE] + _deps(HOST_SOURCE)):
+        return HOST_LIB
+    import sysconfig
+
+    from torch.utils.cpp_extension import include_paths, library_paths
+    os.makedirs(LIBDIR, exist_ok=True)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    tmp = HOST_LIB + f".tmp{os.getpid()}"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           *[f"-I{d}" for d in include_paths() + [os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]], HOST_SOURCE, "-o", tmp,
+           *[f"-L{d}" for d in library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), file=sys.stderr)
+    subprocess.run(cmd, check=True)
+    os.replace(tmp, HOST_LIB)
+    return HOST_LIB
+
+
 def needs_build() -> bool:
     return _stale(LIB, sources() + _headers())
 
 
 def build(force: bool = False, verbose: bool = False) -> str:
+    build_host(force, verbose)
     if not force and not needs_build():
         return LIB
     os.makedirs(OBJDIR, exist_ok=True)
