@@ -2410,7 +2410,7 @@ static int moe_forward_impl(ktx_moe_t h, const int32_t* d_bsz, int qlen, int k, 
 
   PrepParams pp;
   pp.d_bsz = d_bsz; pp.qlen = qlen; pp.k = k; pp.E = E; pp.expert_begin = h->cfg.expert_begin; pp.H = H;
-  pp.rows_per_tile = 16 * mt; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
+  pp.by_size = false; pp.rows_per_tile = 16 * mt; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
   pp.x_q = ws->x_q; pp.x_d = ws->x_d; pp.row_of_pair = ws->row_of_pair; pp.src_of_row = ws->src_of_row;
   pp.tiles = ws->tiles; pp.counters = ws->counters;
   {
@@ -2547,7 +2547,7 @@ static int forward_fp(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, const
 
   PrepParams pp;
   pp.d_bsz = d_bsz; pp.qlen = qlen; pp.k = k; pp.E = E; pp.expert_begin = h->cfg.expert_begin; pp.H = H;
-  pp.rows_per_tile = 16 * mt; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
+  pp.by_size = false; pp.rows_per_tile = 16 * mt; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
   pp.x_q = ws->x_q; pp.x_d = ws->x_d; pp.row_of_pair = ws->row_of_pair; pp.src_of_row = ws->src_of_row;
   pp.tiles = ws->tiles; pp.counters = ws->counters;
   {
@@ -2651,7 +2651,7 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
   const bool chunk = qlen >= 64 && g_dbg[29] != 1 && !h->exact && (size_t)npairs * (std::max(H, I) / 32) * 4 < ((size_t)1 << 32);
   PrepParams pp;
   pp.d_bsz = d_bsz; pp.qlen = qlen; pp.k = k; pp.E = E; pp.expert_begin = h->cfg.expert_begin; pp.H = H;
-  pp.rows_per_tile = chunk ? RAW_ROWS : 4; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
+  pp.by_size = false; pp.rows_per_tile = chunk ? RAW_ROWS : 4; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
   pp.x_q = ws->x_q; pp.x_d = ws->x_d; pp.row_of_pair = ws->row_of_pair; pp.src_of_row = ws->src_of_row;
   pp.tiles = ws->tiles; pp.counters = ws->counters;
   {
@@ -2756,7 +2756,7 @@ static int launch_gguf(const GgGemmParams& p, int max_tiles, hipStream_t st) {
   constexpr int TOK = MT * 16, US = TOK * 16 + 16, NBS = gg_nbs(WT);
   const size_t lds = 2 * 16 * US + 2 * NBS * TOK * 4 + 2 * TOK * 4 + TOK * 4 + (WT == GG_IQ1S ? 4096 * 8 : 0);
   const dim3 grid((p.N / 16 + 3) / 4, max_tiles);
-  const dim3 grid_f = moe_job_grid(max_tiles, (p.N / 16 + 3) / 4);
+  const dim3 grid_f = p.strips ? moe_strip_grid(max_tiles, (p.N / 16 + 3) / 4) : moe_job_grid(max_tiles, (p.N / 16 + 3) / 4);
   if constexpr (gg_foldable(WT)) {   // round 6: the folded-operand kernel; dev knob [21] = 1: gg_block's (the bit-identity test, A/B timing)
     if (g_dbg[21] != 1) {
       const size_t lds_f = 2 * TOK * 256 + 2 * TOK * 4 + TOK * 4 + (WT == GG_Q4K ? 2 * TOK * 32 : WT == GG_IQ1S ? 2 * TOK * 4 + 16384 : 0);
@@ -2815,7 +2815,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
     const int max_tiles = std::min(npairs, E) + npairs / 16;
     PrepParams pp;
     pp.d_bsz = d_bsz; pp.qlen = qlen; pp.k = k; pp.E = E; pp.expert_begin = h->cfg.expert_begin; pp.H = H;
-    pp.rows_per_tile = 16; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
+    pp.by_size = false; pp.rows_per_tile = 16; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
     pp.x_q = ws->x_q; pp.x_d = ws->x_d; pp.row_of_pair = ws->row_of_pair; pp.src_of_row = ws->src_of_row;
     pp.tiles = ws->tiles; pp.counters = ws->counters;
     KTX_HIP(moe_launch_prep(pp, false, st));
@@ -2851,16 +2851,25 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   }
   int mt = std::min(4, pick_mt(qlen, k, E));
   // (IQ1_S keeps to pick_mt: its 16 KiB grid table beside two 32 KiB stages leaves ONE workgroup per CU — measured 1.6x slower)
+  bool strips = false;
   const bool folds = gg_foldable(h->gg_type[0]) && gg_foldable(h->gg_type[2]) && h->gg_type[0] != GG_IQ1S && h->gg_type[2] != GG_IQ1S && g_dbg[21] != 1;
   if (folds) {
     // Rows per tile: a tile's weights are read and folded once, so low tiles cost passes over the weights and high ones work on absent
     // rows.  Measured (Q4_K, 16 | 32 | 64-row tiles, us): 64 experts of 2048 x 1536 with 2.3 rows each 83 | 89 | 95, 4.5: 103 | 109 | 118,
     // 9.4: 123 | 121 | 130, 19: 165 | 145 | 143; 8 experts of 4096 x 14336 with 12 rows 284 | 242 | 264, 25: 353 | 325 | 286, 50: 607 | 469 | 368.
     // 128-row tiles halve the folding's share; below, few tiles fill the last wave worse (same 8 experts, 64 | 128 rows: 125 rows each
-    // 660 | 680, 175: 848 | 793, 200: 948 | 956, 325: 1400 | 1298, 512: 2114 | 1991).  Dev knob [22]: 1 = 64-row tiles, 2 = 128-row ones.
-    const double rows = (double)npairs / std::max(1, E);
-    mt = rows <= 6.0 ? 1 : rows <= 16.0 ? 2 : rows < 144.0 ? 4 : 8;
+    // 660 | 680, 175: 848 | 793, 200: 948 | 956, 325: 1400 | 1298, 512: 2114 | 1991), and so do they in less than two rounds of workgroups (16 of 5632 x 1024, 250 rows, 276 | 284;
+    // on narrow matrices of many rows, see below, they don't: 8 of 1024 x 512, 1500 rows, 107 | 103).  Dev knob [22]: 1 = 64-row tiles, 2 = 128-row ones.
+    const double rows = (double)npairs / std::max(1, E), jobs = ((double)npairs / 128 + 0.5 * E) * std::min(H, I) / 64;
+    strips = rows * 2.0 <= std::min(H, I);
+    mt = rows <= 6.0 ? 1 : rows <= 16.0 ? 2 : rows < 144.0 || (strips && jobs < 1024.0) ? 4 : 8;
     if (g_dbg[22]) mt = g_dbg[22] == 2 ? 8 : std::min(mt, 4);
+    // Strip groups or shares of the experts to the XCDs (moe_pick_strips, moe_pick_job)?  Shares hold as many jobs, not as much work, and end up to a quarter apart; with strip
+    // groups every XCD reads all rows, which counts where an expert has more of them than its matrices have outputs.  Us, shares | strip groups: 8 experts of 4096 x 14336, top-2, 300
+    // tokens 446 | 423, 500 630 | 616, 1696 1669 | 1645; 64 of 2048 x 1536, top-6, 400 162 | 155, 2048 451 | 439; 16 of 5632 x 1024, top-4, 1000 302 | 287; 128 of 1024 x 512, top-8, 900
+    // 101 | 99.4; 8 of 2560 x 1536, top-6, 665 (500 rows) 181 | 181; 8 of 1024 x 512, top-8, 1500 (1500 rows) 103 | 107.  Strip groups with the experts in their own order, which leaves
+    // whole tiles for the end: 500 tokens 630, 1696 1716 (shares 1733 there).
+    strips = strips && mt > 1;
   }
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
 
@@ -2953,7 +2962,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   int32_t* a_b256 = reinterpret_cast<int32_t*>(a_bsp + (size_t)h->max_pairs * (I / 256) * 32);
   PrepParams pp;
   pp.d_bsz = d_bsz; pp.qlen = qlen; pp.k = k; pp.E = E; pp.expert_begin = h->cfg.expert_begin; pp.H = H;
-  pp.rows_per_tile = 16 * mt; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
+  pp.by_size = strips; pp.rows_per_tile = 16 * mt; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
   pp.x_q = ws->x_q; pp.x_d = ws->x_d; pp.row_of_pair = ws->row_of_pair; pp.src_of_row = ws->src_of_row;
   pp.tiles = ws->tiles; pp.counters = ws->counters;
   {
@@ -2966,7 +2975,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   GgGemmParams g1{};
   g1.w0 = h->gate_w; g1.w1 = h->up_w; g1.stride0 = h->gg_stride[0]; g1.stride1 = h->gg_stride[1]; g1.N = I; g1.K = H;
   g1.act_q = ws->x_q; g1.act_d = ws->x_d; g1.act_bs = ws->x_bs; g1.act_bsp = x_bsp; g1.act_b256 = x_b256; g1.row_src = ws->src_of_row; g1.tiles = ws->tiles;
-  g1.counters = ws->counters; g1.out = reinterpret_cast<float*>(ws->a_buf);
+  g1.counters = ws->counters; g1.out = reinterpret_cast<float*>(ws->a_buf); g1.strips = strips;
   int rc;
   {
     ProfScope ps(1, st);
@@ -2982,7 +2991,7 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
   GgGemmParams g2{};
   g2.w0 = h->down_w; g2.w1 = nullptr; g2.stride0 = h->gg_stride[2]; g2.stride1 = 0; g2.N = H; g2.K = I;
   g2.act_q = ws->a_q; g2.act_d = ws->a_d; g2.act_bs = ws->a_bs; g2.act_bsp = a_bsp; g2.act_b256 = a_b256; g2.row_src = nullptr; g2.tiles = ws->tiles;
-  g2.counters = ws->counters; g2.out = reinterpret_cast<float*>(ws->dn_buf);
+  g2.counters = ws->counters; g2.out = reinterpret_cast<float*>(ws->dn_buf); g2.strips = strips;
   {
     ProfScope ps(3, st);
     rc = launch_gguf_type<false>(h->gg_type[2], mt, g2, max_tiles, st);

@@ -10,6 +10,7 @@ struct PrepParams {
   const int32_t* d_bsz;
   int qlen, k, E, expert_begin, H;
   int rows_per_tile;  // 16*MT
+  bool by_size;       // the experts' tiles: from the expert of the most rows on, not in the experts' order (their rows lie in that in any case)
   const int64_t* ids;
   const uint8_t* mask;
   const bf16_t* x;

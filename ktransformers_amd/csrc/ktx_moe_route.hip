@@ -96,12 +96,14 @@ __global__ __launch_bounds__(PREP_THREADS) void moe_prep_kernel(PrepParams p) {
   }
   __syncthreads();
   auto tiles_of = [&](int c) { return (c + p.rows_per_tile - 1) / p.rows_per_tile; };
-  {   // rows and tiles of the experts before this one, and of all
+  const int mine_all = s_cnt[me];
+  {   // rows of the experts before this one, tiles of those whose tiles lie before its own, and rows and tiles of all
     int v[4] = {0, 0, 0, 0};
     for (int e = tid; e < E; e += blockDim.x) {
       const int c = s_cnt[e], tl = tiles_of(c);
       v[2] += c; v[3] += tl;
-      if (e < me) { v[0] += c; v[1] += tl; }
+      if (e < me) v[0] += c;
+      if (p.by_size && c != mine_all ? c > mine_all : e < me) v[1] += tl;
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) {
@@ -119,7 +121,7 @@ __global__ __launch_bounds__(PREP_THREADS) void moe_prep_kernel(PrepParams p) {
     for (int q = 0; q < 4; q++) sum[q] += s_sum[q][w];
     if (w < wave) run += s_mine[w];
   }
-  const int row0 = sum[0], cnt = s_cnt[me], ntiles = tiles_of(cnt);
+  const int row0 = sum[0], cnt = mine_all, ntiles = tiles_of(cnt);
   if (me == 0 && tid == 0) { p.counters[0] = sum[3]; p.counters[1] = sum[2]; }
   run += row0;
   if (mine || me == 0)

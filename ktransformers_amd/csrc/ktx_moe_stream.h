@@ -27,6 +27,27 @@ __device__ __forceinline__ bool moe_pick_job(const Tile* tiles, int ntiles, int 
   if (tile.cnt > 1) tile = tiles[first + ofs % tile.cnt];
   return true;
 }
+// The same by strip groups: an XCD takes every eighth one, of all experts, so that the XCDs end together whatever their experts' tiles hold.  With the experts from the most
+// rows on (PrepParams.by_size) what ends last is small.  The groups past the last eight are dealt job by job, and go first.
+__device__ __forceinline__ bool moe_pick_strips(const Tile* tiles, int ntiles, int nsg, Tile& tile, int& sgroup) {
+  const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3, main = nsg >> 3, rest = nsg & 7;
+  const int dealt = (ntiles * rest + 7 - xcd) >> 3;
+  if (seq < dealt) {
+    const int u = seq * 8 + xcd, t = u / rest;
+    tile = tiles[t];
+    sgroup = main * 8 + u - t * rest;
+    return true;
+  }
+  const int j = seq - dealt;
+  if (j >= ntiles * main) return false;
+  const int t = j / main;
+  tile = tiles[t];
+  const int first = t - tile.idx, ofs = j - first * main;
+  sgroup = ofs / tile.cnt * 8 + xcd;
+  if (tile.cnt > 1) tile = tiles[first + ofs % tile.cnt];
+  return true;
+}
+static dim3 moe_strip_grid(int max_tiles, int nsg) { return dim3((unsigned)((size_t)max_tiles * (nsg >> 3) + ((size_t)max_tiles * (nsg & 7) + 7) / 8) * 8); }
 static dim3 moe_job_grid(int max_tiles, int nsg) { return dim3((unsigned)(((size_t)max_tiles * nsg + 7) / 8 * 8)); }
 
 struct GemmParams {

@@ -247,6 +247,32 @@ def test_folded_q4k_tiles_of_every_row_count(rows):
     assert np.abs(y_ref.view(np.uint16).astype(np.int32)).max() > 0
 
 
+@pytest.mark.parametrize("rows", [(20,), (40, 40, 40), (0, 70, 7, 70, 0, 33, 150), (1, 0, 0, 129), (33,) * 19])
+@pytest.mark.parametrize("H,I", [(256, 512), (512, 768), (1024, 256), (768, 2304)])
+def test_folded_strip_groups_to_the_xcds(rows, H, I):
+    """moe_pick_strips: 4 to 36 strip groups (whole eights, a rest, none of eight) on one expert, equal ones, empty ones, the largest last, at mean rows on both sides of the
+    line to moe_pick_job's shares; the bits are the unfolded kernel's."""
+    from ktransformers_amd import _native as n
+    E, T = len(rows), sum(rows)
+    r0 = np.random.default_rng(T + H)
+    mats = [torch.from_numpy(random_kquant(t, E, a, b, r0)).cuda() for t, a, b in ((Q4, I, H), (Q4, I, H), (Q6, H, I))]
+    x = torch.from_numpy(f32_to_bf16(r0.standard_normal((T, H)).astype(np.float32)).view(np.int16)).view(torch.bfloat16).cuda()
+    ids = torch.from_numpy(r0.permutation(np.repeat(np.arange(E), rows)).astype(np.int64)[:, None]).cuda()
+    w = torch.from_numpy(r0.random((T, 1)).astype(np.float32)).cuda()
+    h = n.MoEHandle(E, 1, H, I, T, "GGUF", 0)
+    h.load_gguf(*mats, Q4, Q4, Q6)
+    n.force_generic_path(True)
+    try:
+        y_fold = h.forward(x, ids, w).view(torch.int16).cpu().numpy()
+        n.lib.ktx_debug_set(21, 1)
+        y_ref = h.forward(x, ids, w).view(torch.int16).cpu().numpy()
+    finally:
+        n.lib.ktx_debug_set(21, 0)
+        n.force_generic_path(False)
+    assert np.array_equal(y_fold, y_ref), f"{int((y_fold != y_ref).sum())} of {y_ref.size} outputs differ"
+    assert np.abs(y_ref.view(np.uint16).astype(np.int32)).max() > 0
+
+
 @pytest.mark.parametrize("T", [1, 4])
 def test_mixtral_8x7b_real_dims(T):
     """BASELINE.json configs[0] (Mixtral-8x7B q4_k_m, kt-kernel/bench/bench_moe.py:166-170): 8 experts, top-2, hidden 4096,
