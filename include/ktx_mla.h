@@ -87,6 +87,14 @@ int ktx_mla_prefill(int T, int num_heads, int kv_len, int kv_pad, float sm_scale
                     int64_t qn_head_stride, const void* d_q_pe, int64_t qp_token_stride, int64_t qp_head_stride,
                     const void* d_k_nope, const void* d_k_pe, int64_t kpe_token_stride, const void* d_v_t, void* d_out,
                     void* stream);
+/* The same with scratch, which lets several workgroups share a query's keys where there are fewer (query block, head) pairs than the chip takes: their results, not
+ * divided, meet in a second launch.  workspace_bytes says how much such a call takes (0: it would not be shared); with less, none or an address off 16 bytes, and for keys or values
+ * off 16 bytes, the call is ktx_mla_prefill's. */
+size_t ktx_mla_prefill_workspace_bytes(int T, int num_heads, int kv_len);
+int ktx_mla_prefill_ws(int T, int num_heads, int kv_len, int kv_pad, float sm_scale, const void* d_q_nope, int64_t qn_token_stride,
+                       int64_t qn_head_stride, const void* d_q_pe, int64_t qp_token_stride, int64_t qp_head_stride,
+                       const void* d_k_nope, const void* d_k_pe, int64_t kpe_token_stride, const void* d_v_t, void* d_out,
+                       void* d_workspace, size_t workspace_bytes, void* stream);
 
 /* Tuning aid (scripts/mla_sweep.py): while a device buffer of >= 16 * workgroups int64 entries is set, every workgroup of the
  * split-KV kernel stamps the wall clock (100 MHz) at its phase boundaries into it; NULL (the default) turns it off. */

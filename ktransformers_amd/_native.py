@@ -116,6 +116,9 @@ def _load() -> C.CDLL:
         C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]
     lib.ktx_mla_prefill.argtypes = [C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p,
                                     C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]
+    lib.ktx_mla_prefill_ws.argtypes = lib.ktx_mla_prefill.argtypes[:-1] + [C.c_void_p, C.c_size_t, C.c_void_p]
+    lib.ktx_mla_prefill_workspace_bytes.argtypes = [C.c_int] * 3
+    lib.ktx_mla_prefill_workspace_bytes.restype = C.c_size_t
     lib.ktx_mla_cache_append.argtypes = [C.POINTER(_MlaConfig), C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p,
                                          C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p]
     lib.ktx_mla_debug_stamps.argtypes = [C.c_void_p]
@@ -206,7 +209,7 @@ def _load() -> C.CDLL:
 # calls of ONE kernel class alone to time that kernel on distinct layers' weights.  Not used by the product path.
 STREAM_CALLS = frozenset((
     "ktx_moe_forward", "ktx_moe_forward_ex", "ktx_moe_combine", "ktx_gate_logits", "ktx_gate_select", "ktx_gate_forward",
-    "ktx_gate_forward_norm", "ktx_mla_decode", "ktx_mla_decode_append", "ktx_mla_cache_append", "ktx_mla_prefill", "ktx_linear_forward",
+    "ktx_gate_forward_norm", "ktx_mla_decode", "ktx_mla_decode_append", "ktx_mla_cache_append", "ktx_mla_prefill", "ktx_mla_prefill_ws", "ktx_linear_forward",
     "ktx_linear_forward_batched", "ktx_linear_forward_batched_prep", "ktx_linear_forward_fused", "ktx_linear_forward_ws", "ktx_rmsnorm", "ktx_fused_add_rmsnorm", "ktx_silu_mul",
     "ktx_mla_prep", "ktx_argmax", "ktx_gemm_bf16_nt", "ktx_attn_decode", "ktx_fp8_act_quant", "ktx_fp8_act_quant_padded", "ktx_linear_gemm_fp8"))   # (not ktx_ep_*: a gather replayed without its reduce would desynchronise the call tags)
 TRACE: list | None = None
@@ -256,7 +259,7 @@ def _load_host():
     module = importlib.util.module_from_spec(importlib.util.spec_from_loader("ktx_host", loader))
     loader.exec_module(module)
     module.bind(KtxError, *(C.cast(getattr(lib._raw, f), C.c_void_p).value
-                            for f in ("ktx_last_error", "ktx_linear_forward", "ktx_moe_forward", "ktx_mla_prefill", "ktx_mla_decode_append")))
+                            for f in ("ktx_last_error", "ktx_linear_forward", "ktx_moe_forward", "ktx_mla_prefill_ws", "ktx_mla_decode_append", "ktx_mla_prefill_workspace_bytes")))
     return module
 
 
@@ -1478,9 +1481,18 @@ def mla_prefill(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tensor, 
             or not k_nope.is_contiguous() or not v_t.is_contiguous() or k_pe.shape[-1] != 64 or k_pe.dim() != 2:
         raise KtxError("mla_prefill: bad operand shapes")
     out = torch.empty((T, H, 128), dtype=torch.bfloat16, device=q_nope.device)
-    check(lib.ktx_mla_prefill(T, H, int(kv_len), kv_pad, float(sm_scale), q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1),
-                              q_pe.data_ptr(), q_pe.stride(0), q_pe.stride(1), k_nope.data_ptr(), k_pe.data_ptr(), k_pe.stride(0),
-                              v_t.data_ptr(), out.data_ptr(), _stream_ptr(q_nope.device)))
+    args = (T, H, int(kv_len), kv_pad, float(sm_scale), q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), q_pe.data_ptr(), q_pe.stride(0), q_pe.stride(1), k_nope.data_ptr(),
+            k_pe.data_ptr(), k_pe.stride(0), v_t.data_ptr(), out.data_ptr())
+    need, ws = int(lib.ktx_mla_prefill_workspace_bytes(T, H, int(kv_len))), None
+    if need:
+        try:
+            ws = torch.empty(need, dtype=torch.uint8, device=q_nope.device)
+        except torch.cuda.OutOfMemoryError:   # (without scratch: one workgroup for all of a query's keys)
+            pass
+    if ws is not None:
+        check(lib.ktx_mla_prefill_ws(*args, ws.data_ptr(), need, _stream_ptr(q_nope.device)))
+    else:
+        check(lib.ktx_mla_prefill(*args, _stream_ptr(q_nope.device)))
     return out
 
 

@@ -19,7 +19,8 @@
 namespace {
 
 typedef int (*mla_prefill_fn)(int, int, int, int, float, const void*, int64_t, int64_t, const void*, int64_t, int64_t, const void*, const void*, int64_t,
-                              const void*, void*, void*);
+                              const void*, void*, void*, size_t, void*);
+typedef size_t (*mla_prefill_bytes_fn)(int, int, int);
 typedef int (*mla_decode_fn)(const ktx_mla_config*, const void*, const void*, void*, void*, int64_t, int64_t, const int32_t*, const int32_t*, const int32_t*,
                              const int32_t*, const int32_t*, int, int, const void*, const void*, void*, float*, void*, size_t, void*);
 typedef int (*linear_fn)(void*, const int32_t*, int, const void*, void*, void*);
@@ -27,6 +28,7 @@ typedef int (*moe_fn)(void*, const int32_t*, int, int, const int64_t*, const flo
 typedef const char* (*error_fn)();
 
 mla_prefill_fn g_prefill;
+mla_prefill_bytes_fn g_prefill_bytes;
 mla_decode_fn g_decode;
 linear_fn g_linear;
 moe_fn g_moe;
@@ -127,9 +129,18 @@ PyObject* mla_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
       v.size(2) != pad || kp.size(1) != 64 || !kn.is_contiguous() || !v.is_contiguous())
     return none();
   const float scale = (float)PyFloat_AS_DOUBLE(a[6]);
+  const size_t need = g_prefill_bytes((int)T, (int)H, (int)kv);
+  at::Tensor ws;
+  if (need) {
+    try {
+      ws = at::empty({(int64_t)need}, qn.options().requires_grad(false).dtype(at::kByte));
+    } catch (const std::exception&) {
+      return none();
+    }
+  }
   return call({T, H, 128}, qn, [&](void* y, void* st) {
     return g_prefill((int)T, (int)H, (int)kv, (int)pad, scale, qn.const_data_ptr(), qn.stride(0), qn.stride(1), qp.const_data_ptr(), qp.stride(0), qp.stride(1),
-                     kn.const_data_ptr(), kp.const_data_ptr(), kp.stride(0), v.const_data_ptr(), y, st);
+                     kn.const_data_ptr(), kp.const_data_ptr(), kp.stride(0), v.const_data_ptr(), y, need ? ws.data_ptr() : nullptr, need, st);
   });
 }
 
@@ -157,16 +168,16 @@ PyObject* mla_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// bind(error type, last_error, linear, moe, mla_prefill, mla_decode): the entry points' addresses
+// bind(error type, last_error, linear, moe, mla_prefill_ws, mla_decode, mla_prefill_workspace_bytes): the entry points' addresses
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  int64_t p[5];
-  if (n != 6) { PyErr_SetString(PyExc_TypeError, "bind: 6 arguments"); return nullptr; }
-  for (int i = 0; i < 5; i++)
+  int64_t p[6];
+  if (n != 7) { PyErr_SetString(PyExc_TypeError, "bind: 7 arguments"); return nullptr; }
+  for (int i = 0; i < 6; i++)
     if (!integer(a[i + 1], p[i])) { PyErr_SetString(PyExc_TypeError, "bind: addresses"); return nullptr; }
   Py_INCREF(a[0]);
   Py_XDECREF(g_error_type);
   g_error_type = a[0];
-  g_error = (error_fn)p[0]; g_linear = (linear_fn)p[1]; g_moe = (moe_fn)p[2]; g_prefill = (mla_prefill_fn)p[3]; g_decode = (mla_decode_fn)p[4];
+  g_error = (error_fn)p[0]; g_linear = (linear_fn)p[1]; g_moe = (moe_fn)p[2]; g_prefill = (mla_prefill_fn)p[3]; g_decode = (mla_decode_fn)p[4]; g_prefill_bytes = (mla_prefill_bytes_fn)p[5];
   Py_RETURN_NONE;
 }
 

@@ -1151,7 +1151,11 @@ struct MlaPrefillParams {
   bf16_t* out;                   // [T][H][128]
   int T, H, kv_len, kv_pad;
   float sm_scale;
-  int nqb;                       // > 0: 1-D XCD-aware grid of nqb query blocks x H heads (H % 8 == 0); 0: grid (query blocks, heads)
+  int nqb;                       // query blocks
+  int xcd;                       // 1-D XCD-aware grid of query blocks x splits x H heads (H % 8 == 0); 0: grid (query blocks, heads, splits)
+  int nsplit;                    // pieces of a query block's keys, of about as many tiles each
+  float* part_o;                 // nsplit > 1: [T][H][nsplit][128] sums, not divided; [T][H][nsplit][2] (largest raw score, sum of the probabilities) behind them
+  float* part_ml;
 };
 
 // S of the NEXT tile is computed beside the probabilities of this one, and its largest scores are found beside this tile's O: MFMAs and vector instructions that
@@ -1169,7 +1173,7 @@ struct MlaPrefillParams {
 // wait for the whole step.  Us, as the tiles' way through registers was before | written at once | now, 8 bytes off: 128 heads, 64 tokens of 4096 125 | 174 | 116 (ALONE; 141 not), 1000 of 4096 370 | 391 |
 // 358 (454 ALONE), 1000 of 1000 96 | 97 | 94; 16 heads, 64 of 2000 63.5 | 60.4 | 60.2; 2 bytes off, where the loads themselves are slow: 167 | - | 156, 391 | - | 415, 105 | - | 110, 80 | - | 76.
 // (4 bytes a request, by LDS-DMA: 174, 413, 111, 88.)
-template <bool DMA, bool ALONE = false>
+template <bool DMA, bool ALONE = false, bool SPLIT = false>   // SPLIT: a workgroup has one of p.nsplit pieces of its queries' keys
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 : 2, ALONE ? 1 : 2))) void mla_prefill_kernel(MlaPrefillParams p) {
   constexpr int NU = 2;                              // query tiles of 16 per wavefront: every K fragment read feeds two MFMAs
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][PF_KB] | [2][PF_VB]
@@ -1179,20 +1183,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 :
   // id % 8 picks the XCD; all query blocks of ONE head go to one XCD (head % 8 == XCD) and run there back to back — the head's K / V^T
   // (1 MB at 2048 keys) is fetched into that XCD's L2 once instead of into all eight.  Within a head: heaviest query blocks first
   // (causal: the last block sees the whole context).
-  int h, qb;
-  if (p.nqb > 0) {
-    const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
-    h = (slot / p.nqb) * 8 + xcd;
-    qb = p.nqb - 1 - slot % p.nqb;
+  int h, qb, split = 0;
+  if (p.xcd) {
+    const int id = blockIdx.x, xcd = id & 7, slot = id >> 3, per_head = SPLIT ? p.nqb * p.nsplit : p.nqb;
+    h = (slot / per_head) * 8 + xcd;
+    qb = slot % per_head;
+    if constexpr (SPLIT) { split = qb % p.nsplit; qb /= p.nsplit; }
+    qb = p.nqb - 1 - qb;
   } else {
     h = blockIdx.y;
     qb = (int)gridDim.x - 1 - (int)blockIdx.x;
+    if constexpr (SPLIT) split = blockIdx.z;
   }
   const int q0 = qb * (64 * NU) + wave * (16 * NU);
   const int qi = lane & 15, g = lane >> 4;
   const int pos_off = p.kv_len - p.T;                // query t sits at position pos_off + t
   const int pos_max = pos_off + min(qb * (64 * NU) + 64 * NU - 1, p.T - 1);
-  const int ntiles = min(pos_max, p.kv_len - 1) / PF_BN + 1;
+  int ntiles = min(pos_max, p.kv_len - 1) / PF_BN + 1, tile0 = 0;   // the keys' tiles: tile0 .. ntiles - 1
+  if constexpr (SPLIT) {
+    const int all = ntiles;
+    tile0 = all * split / p.nsplit;
+    ntiles = all * (split + 1) / p.nsplit;
+    if (tile0 == ntiles) {   // (fewer tiles than pieces)
+      for (int r = tid; r < 64 * NU; r += 256) {
+        const int t = qb * (64 * NU) + r;
+        if (t < p.T) *reinterpret_cast<float2*>(p.part_ml + (((size_t)t * p.H + h) * p.nsplit + split) * 2) = make_float2(-__builtin_inff(), 0.f);
+      }
+      return;
+    }
+  }
   const bf16_t* kn = p.k_nope + (size_t)h * p.kv_pad * 128;
   const bf16_t* vt = p.v_t + (size_t)h * 128 * p.kv_pad;
 
@@ -1234,12 +1253,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 :
   };
   {
     pf_u4 hk[6], hv[4];
-    stage_k(0, 0, hk);
-    stage_v(0, 0, hv);
+    stage_k(tile0, 0, hk);
+    stage_v(tile0, 0, hv);
     put_k(0, hk);
     put_v(0, hv);
-    if (ntiles > 1) {
-      stage_k(1, 1, hk);
+    if (ntiles - tile0 > 1) {
+      stage_k(tile0 + 1, 1, hk);
       put_k(1, hk);
     }
   }
@@ -1336,8 +1355,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 :
 #pragma unroll
     for (int u = 0; u < NU; u++)
       if (!__all(mx[u] <= m_run[u])) {
-        const float m_new = fmaxf(m_run[u], mx[u]);             // finite from tile 0 on: key 0 is visible to every query
-        const float alpha = __builtin_amdgcn_exp2f((m_run[u] - m_new) * cexp);
+        const float m_new = fmaxf(m_run[u], mx[u]);             // finite from tile 0 on: key 0 is visible to every query (SPLIT: or the query has seen no key yet)
+        const float alpha = SPLIT && m_new == m_run[u] ? 1.f : __builtin_amdgcn_exp2f((m_run[u] - m_new) * cexp);
         m_run[u] = m_new;
         l_run[u] *= alpha;
 #pragma unroll
@@ -1348,7 +1367,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 :
     uint4 pb[NU][2];
 #pragma unroll
     for (int u = 0; u < NU; u++) {
-      const float mc = -m_run[u] * cexp;
+      const float mc = SPLIT && m_run[u] == -__builtin_inff() ? 0.f : -m_run[u] * cexp;
       float sum2[2] = {0.f, 0.f};
       float pv[4][4];
 #pragma unroll
@@ -1416,9 +1435,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 :
   v4f sa[NU][4], sb[NU][4];
   qk(0, sa);
   __syncthreads();   // (the first step's requests overwrite what this read)
-  mask(0, sa);
+  mask(tile0, sa);
   largest(sa);
-  int tile = 0;
+  int tile = tile0;
   for (; tile + 2 < ntiles; tile += 2) {
     step(std::true_type{}, 0, tile, sa, sb);
     step(std::true_type{}, 1, tile + 1, sb, sa);
@@ -1430,11 +1449,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 :
 #pragma unroll
       for (int kt = 0; kt < 4; kt++) sa[u][kt] = sb[u][kt];
   }
-  step(std::false_type{}, tile & 1, tile, sa, sb);
+  step(std::false_type{}, (tile - tile0) & 1, tile, sa, sb);
 #pragma unroll
   for (int u = 0; u < NU; u++) {
     const int t = q0 + u * 16 + qi;
     const float l = pf_sum_rows(l_run[u]);
+    if constexpr (SPLIT) {
+      if (t < p.T) {
+        const size_t at = ((size_t)t * p.H + h) * p.nsplit + split;
+        if (g == 0) *reinterpret_cast<float2*>(p.part_ml + at * 2) = make_float2(m_run[u], l);
+        float* po = p.part_o + at * 128 + g * 4;
+#pragma unroll
+        for (int i = 0; i < 8; i++) *reinterpret_cast<float4*>(po + i * 16) = make_float4(o[u][i][0], o[u][i][1], o[u][i][2], o[u][i][3]);
+      }
+      continue;
+    }
     if (t < p.T) {
       const float inv = l > 0.f ? 1.0f / l : 0.f;
       bf16_t* op = p.out + ((size_t)t * p.H + h) * 128 + g * 4;
@@ -1446,10 +1475,76 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 :
   }
 }
 
+// The pieces of a query's keys: out = sum_s w_s O_s / sum_s w_s l_s, w_s = exp2((m_s - max m) c).  Thread = 4 dims of a (token, head), all pieces' loads ahead of the first use.
+template <int NS>
+__global__ __launch_bounds__(256) void mla_prefill_merge_kernel(MlaPrefillParams p) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x, row = i >> 5;
+  if (row >= (long)p.T * p.H) return;
+  const int d = (int)(i & 31) * 4;
+  const float c = p.sm_scale * 1.44269504088896340736f;
+  float2 ml[NS];
+  float4 o[NS];
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    const size_t at = (size_t)row * p.nsplit + min(s, p.nsplit - 1);
+    ml[s] = *reinterpret_cast<const float2*>(p.part_ml + at * 2);
+    o[s] = *reinterpret_cast<const float4*>(p.part_o + at * 128 + d);
+  }
+  float m = -__builtin_inff();
+#pragma unroll
+  for (int s = 0; s < NS; s++) m = fmaxf(m, ml[s].x);
+  float l = 0.f;
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    if (s >= p.nsplit || ml[s].y == 0.f) continue;   // (a piece without a key of the query's: nothing, or old memory)
+    const float w = __builtin_amdgcn_exp2f((ml[s].x - m) * c);
+    l += w * ml[s].y;
+    v.x += w * o[s].x; v.y += w * o[s].y; v.z += w * o[s].z; v.w += w * o[s].w;
+  }
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  *reinterpret_cast<uint2*>(p.out + (size_t)row * 128 + d) = make_uint2(ktx_pk_bf16(v.x * inv, v.y * inv), ktx_pk_bf16(v.z * inv, v.w * inv));
+}
+
+// How many workgroups share a query's keys.  A workgroup of 128 queries and a head alone on its CU takes 1.27 us a key tile, two beside each other 2.0, so that few (query block, head)
+// pairs with long contexts leave most of the chip idle: 64 queries of 16 heads behind 6000 tokens are 16 workgroups of 95 tiles, 128 us.  The pieces cost their sums' way to
+// memory and back and the merge's launch: this estimate, fitted to 66 calls at 1 to 16 pieces, picks one within 4 % of the best everywhere, none slower than whole.  Us, whole | here:
+// 16 heads, 64 queries behind 1000 29 | 15, 6000 128 | 23, 300 behind 1000 36 | 24, 3000 76 | 32, 800 behind 3000 88 | 56; 64 heads, 64 behind 3000 70 | 31, 150 behind 1000 34 | 28; 128
+// heads, 64 behind 3000 72 | 47.  Past 192 pairs, whose workgroups share CUs as it is, 5 to 10 % at most (128 heads, 150 behind 6000 170 | 158) and as often nothing.
+// Dev knob 33 (tests): that many.
+constexpr int PF_SPLITS = 16;
+static int pf_splits(int T, int H, int kv_len) {
+  const int tiles = (kv_len + PF_BN - 1) / PF_BN;
+  if (ktx_debug_get(33) > 0) return std::min(ktx_debug_get(33), PF_SPLITS);
+  const long pairs = (long)((T + 127) / 128) * H;
+  if (pairs > 192) return 1;
+  auto us = [&](int n) {
+    const long each = (pairs * n + 255) / 256;   // workgroups a CU
+    return 6.0 + (tiles + n - 1) / n * 1.27 * (each == 1 ? 1.0 : 0.8 * each) + (n > 1 ? 3.0 + (double)T * H * n * 1040e-6 / 6.0 : 0.0);
+  };
+  int best = 1;
+  for (int n = 2; n <= std::min(PF_SPLITS, tiles); n++)
+    if (us(n) < us(best)) best = n;
+  return us(best) < 0.9 * us(1) ? best : 1;
+}
+static size_t pf_split_bytes(int T, int H, int nsplit) { return nsplit > 1 ? (size_t)T * H * nsplit * 130 * sizeof(float) : 0; }
+
+extern "C" size_t ktx_mla_prefill_workspace_bytes(int T, int num_heads, int kv_len) {
+  return T > 0 && num_heads > 0 && kv_len >= T ? pf_split_bytes(T, num_heads, pf_splits(T, num_heads, kv_len)) : 0;
+}
+
 extern "C" int ktx_mla_prefill(int T, int num_heads, int kv_len, int kv_pad, float sm_scale, const void* d_q_nope,
                                int64_t qn_token_stride, int64_t qn_head_stride, const void* d_q_pe, int64_t qp_token_stride,
                                int64_t qp_head_stride, const void* d_k_nope, const void* d_k_pe, int64_t kpe_token_stride,
                                const void* d_v_t, void* d_out, void* stream) {
+  return ktx_mla_prefill_ws(T, num_heads, kv_len, kv_pad, sm_scale, d_q_nope, qn_token_stride, qn_head_stride, d_q_pe, qp_token_stride, qp_head_stride, d_k_nope, d_k_pe, kpe_token_stride,
+                            d_v_t, d_out, nullptr, 0, stream);
+}
+
+extern "C" int ktx_mla_prefill_ws(int T, int num_heads, int kv_len, int kv_pad, float sm_scale, const void* d_q_nope,
+                                  int64_t qn_token_stride, int64_t qn_head_stride, const void* d_q_pe, int64_t qp_token_stride,
+                                  int64_t qp_head_stride, const void* d_k_nope, const void* d_k_pe, int64_t kpe_token_stride,
+                                  const void* d_v_t, void* d_out, void* d_workspace, size_t workspace_bytes, void* stream) {
   KTX_REQUIRE(d_q_nope && d_q_pe && d_k_nope && d_k_pe && d_v_t && d_out, "ktx_mla_prefill: null pointer");
   KTX_REQUIRE(T > 0 && num_heads > 0 && kv_len >= T, "ktx_mla_prefill: need 0 < T <= kv_len (the new tokens are the last T keys)");
   KTX_REQUIRE(kv_pad >= kv_len && kv_pad % PF_BN == 0, "ktx_mla_prefill: kv_pad must be a multiple of 64 covering kv_len");
@@ -1463,17 +1558,29 @@ extern "C" int ktx_mla_prefill(int T, int num_heads, int kv_len, int kv_pad, flo
   p.T = T; p.H = num_heads; p.kv_len = kv_len; p.kv_pad = kv_pad; p.sm_scale = sm_scale;
   constexpr int lds = 2 * (PF_KB + PF_VB);
   const bool aligned = ((reinterpret_cast<uintptr_t>(d_k_nope) | reinterpret_cast<uintptr_t>(d_k_pe) | reinterpret_cast<uintptr_t>(d_v_t)) & 15) == 0;
-  const int nqb = (T + 127) / 128;
-  void (*kern)(MlaPrefillParams) = aligned ? mla_prefill_kernel<true> : (long)nqb * num_heads <= 256 ? mla_prefill_kernel<false, true> : mla_prefill_kernel<false>;
+  p.nqb = (T + 127) / 128;
+  p.nsplit = aligned && d_workspace && (reinterpret_cast<uintptr_t>(d_workspace) & 15) == 0 ? pf_splits(T, num_heads, kv_len) : 1;
+  if (pf_split_bytes(T, num_heads, p.nsplit) > workspace_bytes) p.nsplit = 1;   // (without scratch: one workgroup for all of a query's keys)
+  p.part_o = (float*)d_workspace;
+  p.part_ml = p.nsplit > 1 ? p.part_o + (size_t)T * num_heads * p.nsplit * 128 : nullptr;
+  void (*kern)(MlaPrefillParams) = p.nsplit > 1 ? mla_prefill_kernel<true, false, true> : aligned ? mla_prefill_kernel<true>
+                                   : (long)p.nqb * num_heads <= 256 ? mla_prefill_kernel<false, true> : mla_prefill_kernel<false>;
   KTX_HIP(ktx_set_max_lds(reinterpret_cast<const void*>(kern), lds));
   hipStream_t st = (hipStream_t)stream;
   // per (query, key, head): 2*(192 + 128) flop over the causal half
-  KTX_TIMED(st, 0.0, "mla_prefill_kernel T=%d Hq=%d kv=%d", T, num_heads, kv_len);
-  const bool xcd = num_heads % 8 == 0;
-  p.nqb = xcd ? nqb : 0;
-  const dim3 grid = xcd ? dim3((unsigned)(nqb * num_heads)) : dim3(nqb, num_heads);
+  KTX_TIMED(st, 0.0, "mla_prefill_kernel T=%d Hq=%d kv=%d splits %d", T, num_heads, kv_len, p.nsplit);
+  p.xcd = num_heads % 8 == 0;
+  const dim3 grid = p.xcd ? dim3((unsigned)((size_t)p.nqb * num_heads * p.nsplit)) : dim3(p.nqb, num_heads, p.nsplit);
   hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p);
   KTX_HIP(hipGetLastError());
+  if (p.nsplit > 1) {
+    const dim3 mgrid((unsigned)(((size_t)T * num_heads + 7) / 8));
+    if (p.nsplit <= 2) hipLaunchKernelGGL(mla_prefill_merge_kernel<2>, mgrid, dim3(256), 0, st, p);
+    else if (p.nsplit <= 4) hipLaunchKernelGGL(mla_prefill_merge_kernel<4>, mgrid, dim3(256), 0, st, p);
+    else if (p.nsplit <= 8) hipLaunchKernelGGL(mla_prefill_merge_kernel<8>, mgrid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL(mla_prefill_merge_kernel<PF_SPLITS>, mgrid, dim3(256), 0, st, p);
+    KTX_HIP(hipGetLastError());
+  }
   return 0;
 }
 

@@ -2087,7 +2087,7 @@ static int launch_gemm(const GemmParams& p, int max_tiles, hipStream_t st) {
   return 0;
 }
 
-constexpr int KTX_DBG = 33;
+constexpr int KTX_DBG = 34;
 static int g_dbg[KTX_DBG] = {0};  // dev knobs (include/ktx_moe.h)
 template <int WBITS, bool GATE_UP>
 static int launch_gemm_rt(const GemmParams& p, int max_tiles, hipStream_t st) {

@@ -278,6 +278,38 @@ def test_prefill_tiles_of_keys(H, T, kv_len, offset):
     assert bool((err <= bound).all()), f"{int((err > bound).sum())} outputs, up to {float((err / bound).max()):.2f} of the bound"
 
 
+@pytest.mark.parametrize("nsplit", [0, 2, 3, 5, 16])   # 0: the library's own choice
+@pytest.mark.parametrize("H,T,kv_len", [(1, 1, 65), (3, 129, 129), (8, 200, 200), (16, 1, 1030), (8, 130, 321), (3, 300, 700), (16, 64, 4160)])
+def test_prefill_keys_shared_by_workgroups(H, T, kv_len, nsplit):
+    """A query's keys in pieces (ktx_mla_prefill_ws): fewer tiles than pieces, queries that see none of a piece's keys, heads of no eight, one, two and more tiles a piece, against
+    attention in 64 bits at the bound of the roundings (the pieces' sums and weights are in 32 bits); without scratch the call is the unshared one's."""
+    from ktransformers_amd import _native as n
+    q, k_nope, cache, v = prefill_operands(H, T, kv_len)
+    k_nope[:, : kv_len // 2] *= 4   # (the largest scores lie in some pieces)
+    qd, args = q.to(DEV), (k_nope.to(DEV), cache.to(DEV)[:, 512:], v.transpose(1, 2).contiguous().to(DEV), kv_len, 192 ** -0.5)
+    whole = None
+    try:
+        n.lib.ktx_debug_set(33, 1)
+        whole = n.mla_prefill(qd[:, :, :128], qd[:, :, 128:], *args)
+        n.lib.ktx_debug_set(33, nsplit)
+        need = n.lib.ktx_mla_prefill_workspace_bytes(T, H, kv_len)
+        out = n.mla_prefill(qd[:, :, :128], qd[:, :, 128:], *args)
+        again = torch.full_like(out, float("nan"))
+        k, kp, vt, kv, scale = args
+        n.check(n.lib.ktx_mla_prefill_ws(T, H, kv, k.shape[1], scale, qd.data_ptr(), qd.stride(0), qd.stride(1), qd.data_ptr() + 256, qd.stride(0), qd.stride(1), k.data_ptr(), kp.data_ptr(),
+                                         kp.stride(0), vt.data_ptr(), again.data_ptr(), torch.empty(max(need, 1), dtype=torch.uint8, device=DEV).data_ptr(), max(need, 1) - 1,
+                                         torch.cuda.current_stream().cuda_stream))
+    finally:
+        n.lib.ktx_debug_set(33, 0)
+    assert torch.equal(again, whole if need else out)
+    if nsplit or kv_len <= 200 or kv_len >= 1030:   # (the library's choice: one tile or a few are not worth it, many of few pairs are)
+        assert (need > 0) == (nsplit > 1 or (not nsplit and kv_len >= 1030))
+    ref, bound = prefill_statement(prefill_scores(q, k_nope, cache, kv_len), v[:, :kv_len].double())
+    for got in (whole, out):
+        err = (got.cpu().double() - ref).abs()
+        assert bool((err <= bound).all()), f"{int((err > bound).sum())} outputs, up to {float((err / bound).max()):.2f} of the bound"
+
+
 @pytest.mark.parametrize("Hq,kv_len,T", [(128, 4023, 1), (64, 700, 1), (128, 33, 1), (64, 5000, 3)])
 def test_merge_riding_the_unabsorb_launch(Hq, kv_len, T):
     """ktx_mla_decode_partials + ktx_linear_forward_batched_merge (the KV-split merge inside the launch of the per-head un-absorb
