@@ -1373,7 +1373,6 @@ class MLAWrapper:
         sizes = (num_heads, head_dim_ckv, head_dim_kpe, page_size, float(sm_scale), self.max_splits, int(max_kv_len))
         if self._sizes != (sizes, self.max_q_tokens):   # (a decode loop plans every step with the same ones)
             self.cfg = _MlaConfig(*sizes)
-            self._cfg_at = C.addressof(self.cfg)
             self._need = int(lib.ktx_mla_workspace_bytes(C.byref(self.cfg), self.max_q_tokens))
             self._sizes = (sizes, self.max_q_tokens)
         need = self._need
@@ -1399,7 +1398,7 @@ class MLAWrapper:
         if self.cfg is None:
             raise KtxError("MLAWrapper.run before plan()")
         if new_ckv is None and new_kpe is None and not return_lse and not partials and _host is not None and TRACE is None:
-            out = _host.mla_decode(self._cfg_at, self.max_q_tokens, self.cfg.page_size, q_nope, q_pe, ckv, k_pe, self.qo_indptr, self.kv_indptr, self.kv_indices,
+            out = _host.mla_decode(self.cfg, self.max_q_tokens, q_nope, q_pe, ckv, k_pe, self.qo_indptr, self.kv_indptr, self.kv_indices,
                                    self.kv_len_arr, self.bsz_tensor, self.workspace)
             if out is not None:
                 return out

@@ -14,6 +14,8 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
+#include <cstring>
+
 #include "../../include/ktx_mla.h"
 
 namespace {
@@ -144,23 +146,32 @@ PyObject* mla_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// mla_decode(config's address, most query tokens, page size, q_nope, q_pe, ckv, k_pe, qo_indptr, kv_indptr, kv_indices | None, kv_len, bsz | None, workspace)
+// mla_decode(config, most query tokens, q_nope, q_pe, ckv, k_pe, qo_indptr, kv_indptr, kv_indices | None, kv_len, bsz | None, workspace)
 PyObject* mla_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  int64_t cfg, most, page;
-  if (n != 13 || !integer(a[0], cfg) || !cfg || !integer(a[1], most) || !integer(a[2], page)) return none();
-  const at::Tensor *qn = plain(a[3], at::kBFloat16), *qp = plain(a[4], at::kBFloat16), *ckv = plain(a[5], at::kBFloat16), *kpe = plain(a[6], at::kBFloat16);
+  int64_t most;
+  ktx_mla_config c;
+  if (n != 12 || !integer(a[1], most)) return none();
+  {   // a copy: another thread's plan may replace the wrapper's while the interpreter is released
+    Py_buffer b;
+    if (PyObject_GetBuffer(a[0], &b, PyBUF_SIMPLE) != 0) { PyErr_Clear(); return none(); }
+    const bool whole = b.len == (Py_ssize_t)sizeof c;
+    if (whole) std::memcpy(&c, b.buf, sizeof c);
+    PyBuffer_Release(&b);
+    if (!whole) return none();
+  }
+  const int64_t page = c.page_size;
+  const at::Tensor *qn = plain(a[2], at::kBFloat16), *qp = plain(a[3], at::kBFloat16), *ckv = plain(a[4], at::kBFloat16), *kpe = plain(a[5], at::kBFloat16);
   const at::Tensor* ix[5];
   for (int i = 0; i < 5; i++) {
-    ix[i] = a[7 + i] == Py_None && (i == 2 || i == 4) ? nullptr : plain(a[7 + i], at::kInt);
-    if (!ix[i] && a[7 + i] != Py_None) return none();
+    ix[i] = a[6 + i] == Py_None && (i == 2 || i == 4) ? nullptr : plain(a[6 + i], at::kInt);
+    if (!ix[i] && a[6 + i] != Py_None) return none();
   }
-  const at::Tensor* ws = plain(a[12], at::kByte);
+  const at::Tensor* ws = plain(a[11], at::kByte);
   if (!qn || !qp || !ckv || !kpe || !ix[0] || !ix[1] || !ix[3] || !ws || qn->dim() != 3 || ckv->dim() < 2 || kpe->dim() < 2 || modes()) return none();
   const int64_t T = qn->size(0), H = qn->size(1), dc = qn->size(2), cs = ckv->stride(-2), ps = kpe->stride(-2), batch = ix[0]->numel() - 1;
   if (T < 1 || T > most || T > INT32_MAX || batch > INT32_MAX || !qn->is_contiguous() || !qp->is_contiguous() || ckv->stride(-1) != 1 || kpe->stride(-1) != 1 || ckv->stride(0) != cs * page ||
       kpe->stride(0) != ps * page)
     return none();
-  const ktx_mla_config c = *(const ktx_mla_config*)cfg;   // (another thread's plan may replace it while the interpreter is released)
   return call({T, H, dc}, *qn, [&](void* y, void* st) {
     return g_decode(&c, qn->const_data_ptr(), qp->const_data_ptr(), (void*)ckv->const_data_ptr(), (void*)kpe->const_data_ptr(), cs, ps, ix[0]->const_data_ptr<int32_t>(),
                     ix[1]->const_data_ptr<int32_t>(), ix[2] ? ix[2]->const_data_ptr<int32_t>() : nullptr, ix[3]->const_data_ptr<int32_t>(),

@@ -1,5 +1,7 @@
 """csrc/ktx_host.cpp makes the shortest calls without an interpreter step per argument: the same kernels on the same arguments as _native.py's own way, which keeps every
 call that the module does not take."""
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -19,7 +21,9 @@ def test_the_module_leaves_what_it_has_not_checked():
     for args in ((), (1, 64, 0, x, ids, w), (1, 64, 0, x, ids, None), (0, 64, 0, x, ids, w)):
         assert n._host.moe(*args) is None
     assert n._host.mla_prefill(*[x] * 5, 1, 1.0) is None and n._host.mla_prefill(x) is None
-    assert n._host.mla_decode(1, 1, 64, x, x, x, x, ids, ids, None, ids, None, x) is None and n._host.mla_decode() is None
+    for cfg in (1, None, b"short", n._MlaConfig(16, 512, 64, 64, 1.0, 1, 0)):
+        assert n._host.mla_decode(cfg, 1, x, x, x, x, ids, ids, None, ids, None, x) is None
+    assert n._host.mla_decode() is None
     with pytest.raises(TypeError):
         n._host.bind(1)
 
@@ -154,6 +158,11 @@ def test_latent_attention(both, pages_of_one):
         return wrapper.run(q, qp, cache[..., :512], cache[..., 512:], **kw)
     for hint in (0, 128):
         assert both(lambda: run(hint)) == 1
+    want, held = run(), copy.deepcopy(wrapper)   # (a copy's run reads the copy's sizes, whatever the first wrapper plans next)
+    run(128)
+    assert both(lambda: held.run(q, qp, cache[..., :512], cache[..., 512:])) == 1 and torch.equal(held.run(q, qp, cache[..., :512], cache[..., 512:]), want)
+    held.cfg.sm_scale = 0.14                     # ... and its present values
+    assert both(lambda: held.run(q, qp, cache[..., :512], cache[..., 512:])) == 1 and not torch.equal(held.run(q, qp, cache[..., :512], cache[..., 512:]), want)
     assert both(lambda: run(new_ckv=rand(B, 512) * 0, new_kpe=rand(B, 64) * 0)) == 0
     out, lse = run(return_lse=True)
     assert torch.equal(out, run()) and lse.shape == (B, H)
