@@ -154,17 +154,6 @@ __device__ __forceinline__ void mla_stage(const MlaParams& p, int req, int kv_en
   }
 }
 
-// Four of them, 8 KiB apart in the LDS, from one scalar base
-__device__ __forceinline__ void mla_dma_4rows(const bf16_t* base, const uint32_t (&off)[4], uint32_t lds_addr) {
-  unsigned keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %5\n\t"
-               "s_add_u32 m0, m0, 0x2000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %5\n\t"
-               "s_add_u32 m0, m0, 0x2000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %5\n\t"
-               "s_add_u32 m0, m0, 0x2000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, %5\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep)
-               : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base), "s"(lds_addr)
-               : "memory", "scc");
-}
 // which request owns query token qt?  Every wavefront resolves it on its own with ONE round of independent loads
 // (lane i looks at request i) — the live-request count *d_bsz is fetched in the same round and applied afterwards, not
 // waited for first: right after a kernel boundary each dependent load is another 1.5-3 us (measured with the phase stamps)
@@ -509,36 +498,38 @@ __device__ __forceinline__ float pf_sum_rows(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Workgroup = 4 head blocks of 16 x 2 wavefronts, one per CU; a step is 64 tokens, staged once for all 64 heads and double-buffered.  A
-// wavefront computes S of 32 of the tokens x 16 heads, takes the other 32 from its partner through the LDS, and after the softmax (which both
-// do) 256 dims of O.  S and O are computed transposed (tokens x heads, dims x heads), so that a lane owns ONE head: the softmax statistics are
+// Workgroup = 4 head blocks of 16, a wavefront each, alone on its SIMD with all its registers (Q 72, O 128); K and V rows in tiles of 32 tokens, staged once for all 64 heads, four
+// of them in the LDS.  S and O are computed transposed (tokens x heads, dims x heads), so that a lane owns ONE head: the softmax statistics are
 // one value a lane, and S^T leaves the MFMA with a lane's tokens where P^T enters the next one — the probabilities never leave the
-// registers (V's rows are read in the order 4 g + (0..3), 16 + 4 g + (0..3) that this gives lane group g).
-// What bounds it: a step's three phases, S, softmax and O, which its two barriers keep one after the other in both wavefronts of a SIMD.  Of a step's
-// 7400 cycles the LDS works 2900 (576 KB read), the matrix pipe 3200 (100 MFMAs a wavefront), the vector ALU 2500 (rocprofv3 counters of
-// the whole launch, 8 requests of 2048 .. 8192 tokens: 13, 18 and 21 % busy, no bank conflicts, two thirds of the waves' time waits).  The rows are
+// registers (V's rows are read in the order 4 g + (0..3), 16 + 4 g + (0..3) that this gives lane group g), and no wavefront waits for another's scores.
+// What bounds it: a tile's 100 MFMAs (1600 cycles) and some 450 other instructions of the same wavefront (96 LDS reads and their waits, the softmax, 9 requests), which one SIMD issues one after
+// the other: 1.45 us a tile at 2.1 GHz; without the LDS reads it would be 1.33, without the requests 1.23, without the second bf16 of P 1.21.  So the tile's parts are laid beside each
+// other: its probabilities and the requests beside the next one's scores, the next one's largest beside this one's O, one instruction of each kind beside an MFMA.
+// Before, two wavefronts a SIMD shared 16 heads in steps of 64 tokens (half of the scores each, exchanged through the LDS, then half of the dims), and two barriers a step kept scores, softmax and O
+// apart in both: 3.1 us for 64 tokens, all of O rescaled in nearly every step, and the last step whole where 32 tokens were left.  Decode and merge, before -> here, us: 128 heads, 8
+// requests of 2048 .. 8192 tokens 44.5 -> 42.0, 32 of 1000 .. 4000 69.9 -> 60.9, 20 of 2000 .. 8000 76 -> 66, 4 of 8192 .. 32768 66 -> 57, 32 of 250 .. 1000 34.0 -> 32.9; 64 heads, 24 of 1250
+// .. 5000 47.4 -> 41.1, 3 of 16384 31.5 -> 29.4, 32 of 500 .. 2000 34.7 -> 32.4; few requests and short contexts (128 heads, 5 of 8000) the same to 1 %.  A call of 8 requests: 1.6 us for the job,
+// 3.6 for pages, Q and the first rows, 0.7 the first scores, 17 the tiles, 3 the partial results' stores.
+// The rows are
 // packed 1 KiB apart with their 16-byte pieces permuted by mla_swz, which keeps both the fragment reads of 16 rows and the transposed reads of
 // 8 rows off each other's banks.
 // P enters the product as two bf16, the second what rounding the first left over.  One bf16 is off by its rounding except where P is exactly 1, a
 // split's largest entry, and here a split is longer than in mla_decode_kernel: the error against 64-bit sums grew by 1 to 4 % (32 requests
-// of 500 tokens, 128 heads 1.77e-3 -> 1.84e-3).  With two it is the outputs' rounding alone, 1.66e-3 at every size.
-// 128 heads, 8 requests, us for 64 tokens (8192 -> 16384 tokens each): mla_decode_kernel<4, 2> 4.2 (scores of half the dims exchanged for every 32
-// tokens, softmax on 4 values a lane and head), this 3.1; with P in one bf16 2.7.  With one bf16 also: no exchange, S computed by both wavefronts
-// + 0.4; a wavefront for itself, 512 dims of O for 32 tokens, + 0.6 (the registers are full, and every MFMA waits for its LDS read); rows
-// padded to 1168 B + 0.5.
+// of 500 tokens, 128 heads 1.77e-3 -> 1.84e-3).  With two it is the outputs' rounding alone, 1.66e-3 at every size, also where P passes 1: sums are rescaled only when a head's
+// largest score has grown by MLA_GROWTH (P to 256) since they last were, for a split's first tile finds most of it and every rescaling is 128 products a lane.
 // distinct for 16 rows, also with rows 4 .. 11 flipped by 1 (ds_read_b128 takes lanes 0-3, 12-15, 20-23, 24-27 together); >> 1 distinct for rows
 // 0-7 and for 8-15 (ds_read_b64_tr_b16 takes 32 lanes together)
 __device__ __forceinline__ uint32_t mla_swz(uint32_t row) { return row & 8 ? ((row & 7) ^ 4) << 1 | 1 : (row & 7) << 1; }
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void mla_decode_wide_kernel(MlaParams p) {
-  constexpr int NWV = 8, NQ = 18, STEP = 2 * MLA_TILE;
-  constexpr uint32_t KT_BYTES = STEP * MLA_DC * 2, KP_BYTES = STEP * MLA_DR * 2;
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];         // [2][64][1024 B] ckv | [2][64][128 B] k_pe | [8 waves][2][64] scores
-  float4* Sx = reinterpret_cast<float4*>(smem + 2 * (KT_BYTES + KP_BYTES));
+constexpr float MLA_GROWTH = 5.5451774f;   // 8 ln 2
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mla_decode_wide_kernel(MlaParams p) {
+  constexpr int NWV = 4, NQ = 18, NBUF = 4, REQ = MLA_TILE / NWV + 1;   // REQ: a wavefront's requests of a tile
+  constexpr int KA = 6, VA = 2;                                          // fragment reads ahead of their MFMAs: k-steps of the scores, groups of 4 dim tiles of O
+  constexpr uint32_t KT_BYTES = MLA_TILE * MLA_DC * 2, KP_BYTES = MLA_TILE * MLA_DR * 2;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];         // [4][32][1024 B] ckv | [4][32][128 B] k_pe
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hb = blockIdx.y;
-  const int ds = wave & 1;
-  const int head = (hb * 4 + (wave >> 1)) * 16 + (lane & 15);
+  const int head = (hb * 4 + wave) * 16 + (lane & 15);
   MLA_TS(0);
 
   MlaWork w;
@@ -556,69 +547,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int nsp = __builtin_amdgcn_readfirstlane(w.nsp);
   MLA_TS(1);
 
-  // the split's run of 32-token tiles: whole steps
+  // the split's run of 32-token tiles: pairs, but for the context's last one
   const int ntiles = (kv_end + MLA_TILE - 1) / MLA_TILE;
-  const int each = 2 * (((kv_end + STEP - 1) / STEP + nsp - 1) / nsp);
+  const int each = 2 * (((kv_end + 2 * MLA_TILE - 1) / (2 * MLA_TILE) + nsp - 1) / nsp);
   const int t_begin = min(split * each, ntiles), t_end = min(t_begin + each, ntiles);
 
-  v4f o[16];     // O^T: dims 256 ds + 16 i + 4 g + (0..3) of the lane's head
+  v4f o[32];     // O^T: dims 16 i + 4 g + (0..3) of the lane's head
 #pragma unroll
-  for (int i = 0; i < 16; i++) o[i] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < 32; i++) o[i] = v4f{0.f, 0.f, 0.f, 0.f};
   float m_run = -__builtin_inff(), l_run = 0.f;
 
   if (t_begin < t_end) {
     if (app_pos >= 0 && hb == 0 && app_pos / MLA_TILE >= t_begin && app_pos / MLA_TILE < t_end) mla_store_appended(p, req, page_base, app_pos, tid);
 
-    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)smem;
-    auto page_of = [&](int tile) -> int {   // looked up a step ahead of its staging (see mla_decode_kernel); clamped: a tile of this request
-      const int t = min(tile, ntiles - 1);
-      const int pidx_ = __builtin_amdgcn_readfirstlane(page_base + (p.tiles_shift >= 0 ? t >> p.tiles_shift : t * MLA_TILE / p.page_size));
+    // lane i holds the page of tile pt0 + i (clamped: a tile of this request): one round of the page table for 64 tiles
+    auto pages_from = [&](int t0) {
+      const int t = min(t0 + lane, ntiles - 1);
+      const int pidx_ = page_base + (p.tiles_shift >= 0 ? t >> p.tiles_shift : t * MLA_TILE / p.page_size);
       return p.kv_indices ? p.kv_indices[pidx_] : pidx_;
     };
-    // Four ckv rows a wavefront and tile, one 1-KiB row per wave-instruction; k_pe: eight rows per wave-instruction, by wavefronts 0-3 for the
-    // first tile of a step and 4-7 for the second.  Rows past the context re-read its last one: finite, weighted with exactly 0.  A tile that is
-    // all context and does not hold the appended row takes the lanes' offsets from registers: address arithmetic on the scalar unit, 250
-    // instructions a step, held a wavefront up for as long as its MFMAs.
-    uint32_t ro[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) ro[c] = (uint32_t)((wave + c * NWV) * p.ckv_ts * 2) + ((uint32_t)lane ^ mla_swz(wave + c * NWV)) * 16u;
-    const int pr = (wave & 3) * 8 + (lane >> 3);
-    const uint32_t po = (uint32_t)(pr * p.kpe_ts * 2) + ((uint32_t)(lane & 7) ^ ((pr >> 1) & 7)) * 16u;
-    auto stage_tile = [&](int tile, int page_v, uint32_t dK, uint32_t dP, int wsel) {
-      const int tok0 = tile * MLA_TILE, last = kv_end - 1 - tok0;
-      const int page0 = __builtin_amdgcn_readfirstlane(page_v);
-      const size_t row0 = (size_t)page0 * p.page_size + (p.tiles_shift >= 0 ? tok0 & (p.page_size - 1) : tok0 % p.page_size);
-      if (last >= MLA_TILE - 1 && (unsigned)(app_pos - tok0) >= (unsigned)MLA_TILE) {
-        mla_dma_4rows(p.ckv + row0 * p.ckv_ts, ro, dK + (uint32_t)wave * (MLA_DC * 2));
-        if ((wave >> 2) == wsel) mla_dma_row_sa(p.k_pe + row0 * p.kpe_ts, po, dP + (uint32_t)(wave & 3) * (8 * MLA_DR * 2));
-        return;
-      }
-      for (int c = 0; c < MLA_TILE / NWV; c++) {
-        const int r = wave + c * NWV, rr = min(r, last);
-        const bf16_t* src = p.ckv + (row0 + rr) * p.ckv_ts;
-        if (tok0 + rr == app_pos) src = p.app_ckv + (size_t)req * MLA_DC;
-        mla_dma_row_sa(src, ((uint32_t)lane ^ mla_swz(r)) * 16u, dK + (uint32_t)r * (MLA_DC * 2));
-      }
-      if ((wave >> 2) == wsel) {
-        const int rr = min(pr, last);
-        const bf16_t* src = p.k_pe + (row0 + rr) * p.kpe_ts;
-        if (tok0 + rr == app_pos) src = p.app_kpe + (size_t)req * MLA_DR;
-        mla_dma_row_a(src + ((lane & 7) ^ ((pr >> 1) & 7)) * 8, dP + (uint32_t)(wave & 3) * (8 * MLA_DR * 2));
-      }
-    };
-    auto stage = [&](int tile, int pg0, int pg1, int buf) {
-      const uint32_t dK = lds0 + (uint32_t)buf * KT_BYTES, dP = lds0 + 2 * KT_BYTES + (uint32_t)buf * KP_BYTES;
-      stage_tile(tile, pg0, dK, dP, 0);
-      stage_tile(min(tile + 1, ntiles - 1), pg1, dK + KT_BYTES / 2, dP + KP_BYTES / 2, 1);   // (behind the context: its last tile again, masked)
-    };
-
-    // fragment addresses within a stage: K rows 16 t + (lane & 15), piece 4 s + g; V rows 4 g + (lane & 15) / 4 (+ 16), piece 2 i + (lane >> 1 & 1)
-    const uint32_t kx = (ds * MLA_TILE + (lane & 15)) * (MLA_DC * 2) + (((uint32_t)g ^ mla_swz(lane & 15)) * 16);
-    const uint32_t px = (ds * MLA_TILE + (lane & 15)) * (MLA_DR * 2) + (((uint32_t)g ^ ((lane >> 1) & 7)) * 16);
-    const uint32_t vr = 4 * g + ((lane & 15) >> 2);
-    const uint32_t vx = vr * (MLA_DC * 2) + ((((lane >> 1) & 1) ^ mla_swz(vr)) * 16) + (lane & 1) * 8 + ds * 512;
-
-    stage(t_begin, page_of(t_begin), page_of(t_begin + 1), 0);
+    int pt0 = t_begin, pages = pages_from(pt0);
+    asm volatile("" ::: "memory");   // (in this order: the pages are waited for first)
     v8bf qf[NQ];   // B[k = (lane >> 4) * 8 .. + 7][n = head] of 16 nope and 2 rope k-steps
     {
       const bf16_t* qn = p.q_nope + ((size_t)qt * p.Hq + head) * MLA_DC + g * 8;
@@ -628,143 +577,260 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int j = 0; j < 2; j++) qf[16 + j] = as_v8bf(*reinterpret_cast<const uint4*>(qr + j * 32));
     }
-    int pn0 = page_of(t_begin + 2), pn1 = page_of(t_begin + 3);
-    MLA_TS(2);
-
-    int cur = 0;
-    for (int tile = t_begin; tile < t_end; tile += 2, cur ^= 1) {
-      // behind this wave's wait and the barrier the step's rows are all there and every wave is done with the other buffer
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      if (tile + 2 < t_end) {
-        stage(tile + 2, pn0, pn1, cur ^ 1);
-        pn0 = page_of(tile + 4); pn1 = page_of(tile + 5);
-      }
-      const uint8_t* kb = smem + cur * KT_BYTES;
-      const uint8_t* pb = smem + 2 * KT_BYTES + cur * KP_BYTES;
-      const int ntok = kv_end - tile * MLA_TILE;
-
-      // ---- S^T = K Q^T: lane holds tokens 16 t + 4 g + r of its head; this wave's half of the tokens, the other's from the LDS
-      v4f st[4], sm[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-      // (a k-step's fragments are read two ahead of the MFMAs: fenced, or the compiler reads one fragment ahead and waits for it)
-      v8bf kf[3][2];
-      auto load_k = [&](int s) __attribute__((always_inline)) {
-        const uint8_t* a = s < 16 ? kb + (kx ^ ((s & 3) * 64)) + (s >> 2) * 256 : pb + (px ^ ((s - 16) * 64));
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)smem;
+    // Eight ckv rows a wavefront and tile, one 1-KiB row per wave-instruction; k_pe: eight rows in one.  Rows past the context re-read its last one: finite, weighted
+    // with exactly 0.  A tile that is all context and does not hold the appended row takes the lanes' offsets from registers: address arithmetic on the scalar
+    // unit, 250 instructions for 64 tokens, held a wavefront up for as long as its MFMAs.
+    uint32_t ro[MLA_TILE / NWV];
 #pragma unroll
-        for (int t = 0; t < 2; t++) kf[s % 3][t] = as_v8bf(*reinterpret_cast<const uint4*>(a + t * (s < 16 ? 16 * MLA_DC * 2 : 16 * MLA_DR * 2)));
-      };
-      load_k(0);
-      load_k(1);
+    for (int c = 0; c < MLA_TILE / NWV; c++) ro[c] = (uint32_t)((wave + c * NWV) * p.ckv_ts * 2) + ((uint32_t)lane ^ mla_swz(wave + c * NWV)) * 16u;
+    const int pr = wave * 8 + (lane >> 3);
+    const uint32_t po = (uint32_t)(pr * p.kpe_ts * 2) + ((uint32_t)(lane & 7) ^ ((pr >> 1) & 7)) * 16u;
+    uint32_t dK, dP;
+    const bf16_t *base_k, *base_p;
+    // where tile lies and goes; true: whole rows of the context's cache, which request(0 .. 8) bring
+    auto locate = [&](int tile) __attribute__((always_inline)) {
+      if (tile - pt0 >= 64) {
+        pt0 = tile;
+        pages = pages_from(pt0);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(pages)::"memory");
+      }
+      const int buf = (tile - t_begin) & (NBUF - 1);
+      dK = lds0 + buf * KT_BYTES; dP = lds0 + NBUF * KT_BYTES + buf * KP_BYTES + wave * (8 * MLA_DR * 2);
+      const int tok0 = tile * MLA_TILE;
+      const int page0 = __builtin_amdgcn_readlane(pages, tile - pt0);
+      const size_t row0 = (size_t)page0 * p.page_size + (p.tiles_shift >= 0 ? tok0 & (p.page_size - 1) : tok0 % p.page_size);
+      base_k = p.ckv + row0 * p.ckv_ts;
+      base_p = p.k_pe + row0 * p.kpe_ts;
+      return kv_end - 1 - tok0 >= MLA_TILE - 1 && (unsigned)(app_pos - tok0) >= (unsigned)MLA_TILE;
+    };
+    auto request = [&](int i) __attribute__((always_inline)) {
+      if (i < MLA_TILE / NWV) mla_dma_row_sa(base_k, ro[i], dK + (wave + i * NWV) * (MLA_DC * 2));
+      else mla_dma_row_sa(base_p, po, dP);
+    };
+    auto request_any = [&](int tile) {   // as many requests, of a located tile that ends the context or holds the appended row
+      const int tok0 = tile * MLA_TILE, last = kv_end - 1 - tok0;
+      for (int c = 0; c < MLA_TILE / NWV; c++) {
+        const int r = wave + c * NWV, rr = min(r, last);
+        const bf16_t* src = base_k + rr * p.ckv_ts;
+        if (tok0 + rr == app_pos) src = p.app_ckv + (size_t)req * MLA_DC;
+        mla_dma_row_sa(src, ((uint32_t)lane ^ mla_swz(r)) * 16u, dK + (uint32_t)r * (MLA_DC * 2));
+      }
+      const int rr = min(pr, last);
+      const bf16_t* src = base_p + rr * p.kpe_ts;
+      if (tok0 + rr == app_pos) src = p.app_kpe + (size_t)req * MLA_DR;
+      mla_dma_row_a(src + ((lane & 7) ^ ((pr >> 1) & 7)) * 8, dP);
+    };
+#pragma unroll
+    for (int c = 0; c < NBUF - 1; c++)
+      if (t_begin + c < t_end) {
+        if (!locate(t_begin + c)) {
+          request_any(t_begin + c);
+        } else {
+#pragma unroll
+          for (int i = 0; i < REQ; i++) request(i);
+        }
+        if (c == 0) {   // the compiler does not see the requests, so that its wait for these is one for those as well: the first tile comes beside them
+#pragma unroll
+          for (int j = 0; j < NQ; j++) asm volatile("" : "+a"(qf[j]));
+        }
+      }
+    MLA_TS(2);
+    // tile's rows are there for all wavefronts, and all are done with the tile whose buffer the next request takes: what is requested behind it stays in flight
+    auto arrived = [&](int tile) __attribute__((always_inline)) {
+      if (tile == t_begin && tile + 2 < t_end) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * REQ) : "memory");
+      else if (tile + 1 < t_end) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(REQ) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // fragment addresses within a tile: K rows 16 t + (lane & 15), piece 4 s + g; V rows 4 g + (lane & 15) / 4 (+ 16), piece 2 i + (lane >> 1 & 1)
+    const uint32_t kx = (lane & 15) * (MLA_DC * 2) + (((uint32_t)g ^ mla_swz(lane & 15)) * 16);
+    const uint32_t px = (lane & 15) * (MLA_DR * 2) + (((uint32_t)g ^ ((lane >> 1) & 7)) * 16);
+    const uint32_t vr = 4 * g + ((lane & 15) >> 2);
+    const uint32_t vx = vr * (MLA_DC * 2) + ((((lane >> 1) & 1) ^ mla_swz(vr)) * 16) + (lane & 1) * 8;
+
+    // ---- S^T = K Q^T: lane holds tokens 16 t + 4 g + r of its head.  Fragments are read KA k-steps ahead of the MFMAs: fenced, or the compiler reads one
+    // fragment ahead and waits for it; between(s): what goes beside k-step s
+    v8bf kf[KA + 1][2];
+    auto load_k = [&](int tile, int s) __attribute__((always_inline)) {
+      const int buf = (tile - t_begin) & (NBUF - 1);
+      const uint8_t* a = s < 16 ? smem + buf * KT_BYTES + (kx ^ ((s & 3) * 64)) + (s >> 2) * 256 : smem + NBUF * KT_BYTES + buf * KP_BYTES + (px ^ ((s - 16) * 64));
+#pragma unroll
+      for (int t = 0; t < 2; t++) kf[s % (KA + 1)][t] = as_v8bf(*reinterpret_cast<const uint4*>(a + t * (s < 16 ? 16 * MLA_DC * 2 : 16 * MLA_DR * 2)));
+    };
+    auto scores = [&](int tile, v4f (&s2)[2], auto between) __attribute__((always_inline)) {
+      s2[0] = s2[1] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < NQ; s++) {
-        if (s + 2 < NQ) load_k(s + 2);
+        if (s + KA < NQ) load_k(tile, s + KA);
 #pragma unroll
-        for (int t = 0; t < 2; t++) sm[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s % 3][t], qf[s], sm[t], 0, 0, 0);
+        for (int t = 0; t < 2; t++) s2[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s % (KA + 1)][t], qf[s], s2[t], 0, 0, 0);
+        between(s);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // in pieces, beside the products of O: 0 the scale, 1 what lies past the context, 2 and 3 the largest
+    float mx = 0.f;
+    auto prepare = [&](int piece, int tile, v4f (&s2)[2]) __attribute__((always_inline)) {
+      if (piece == 0) {
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) s2[t][r] *= p.sm_scale;
+      } else if (piece == 1) {
+        const int ntok = kv_end - tile * MLA_TILE;
+        if (ntok < MLA_TILE) {
+#pragma unroll
+          for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+              if (16 * t + 4 * g + r >= ntok) s2[t][r] = -__builtin_inff();
+        }
+      } else if (piece == 2) {
+        mx = fmaxf(fmaxf(fmaxf(s2[0][0], s2[0][1]), fmaxf(s2[0][2], s2[0][3])), fmaxf(fmaxf(s2[1][0], s2[1][1]), fmaxf(s2[1][2], s2[1][3])));
+      } else {
+        mx = pf_max_rows(mx);   // finite: a tile has >= 1 visible token
+      }
+    };
+
+    typedef __attribute__((address_space(3))) v4s16 lds_v4;
+    union VFrag { v4s16 h[2]; v8bf v; };
+    VFrag vf[VA + 1][4];
+    auto load_v = [&](int tile, int j, int i) __attribute__((always_inline)) {   // the rows' transposed reads, dims 128 i + 16 j
+      const uint8_t* a = smem + ((tile - t_begin) & (NBUF - 1)) * KT_BYTES + (vx ^ (j * 32)) + i * 256;
+      vf[j % (VA + 1)][i].h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)a);
+      vf[j % (VA + 1)][i].h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(a + 16 * MLA_DC * 2));
+    };
+    // A tile: its probabilities beside the next one's scores, its share of O beside their largest.
+    // MORE: there is a next one.  One instruction of each kind beside an MFMA: a
+    // wavefront alone on its SIMD has nobody to fill the matrix pipe while it issues a row of reads.
+    auto step = [&](auto more, int tile, v4f (&st)[2], v4f (&sn)[2]) __attribute__((always_inline)) {
+      constexpr bool MORE = decltype(more)::value;
+      if constexpr (MORE) {
+        arrived(tile + 1);
+#pragma unroll
+        for (int s = 0; s < KA; s++) load_k(tile + 1, s);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int t = 0; t < 2; t++) Sx[(wave * 2 + t) * 64 + lane] = make_float4(sm[t][0], sm[t][1], sm[t][2], sm[t][3]);
-      __syncthreads();
+      for (int i = 0; i < 32; i++) asm volatile("" : "+a"(o[i]));
+      if (__builtin_amdgcn_ballot_w64(mx > m_run + MLA_GROWTH) != 0ull) {
+        const float m_new = fmaxf(m_run, mx), alpha = __expf(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
 #pragma unroll
-      for (int t = 0; t < 2; t++) {
-        const float4 v = Sx[((wave ^ 1) * 2 + t) * 64 + lane];
-        const v4f other = {v.x, v.y, v.z, v.w};
-        st[t] = ds ? other : sm[t];
-        st[2 + t] = ds ? sm[t] : other;
-      }
-#pragma unroll
-      for (int t = 0; t < 4; t++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) st[t][r] *= p.sm_scale;
-      if (ntok < STEP) {
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-          for (int r = 0; r < 4; r++)
-            if (16 * t + 4 * g + r >= ntok) st[t][r] = -__builtin_inff();
-      }
-      float mt[4];
-#pragma unroll
-      for (int t = 0; t < 4; t++) mt[t] = fmaxf(fmaxf(st[t][0], st[t][1]), fmaxf(st[t][2], st[t][3]));
-      const float m_new = fmaxf(m_run, pf_max_rows(fmaxf(fmaxf(mt[0], mt[1]), fmaxf(mt[2], mt[3]))));   // finite: a step has >= 1 visible token
-#pragma unroll
-      for (int t = 0; t < 4; t++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) st[t][r] = __expf(st[t][r] - m_new);
-      uint32_t pk[8];
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        mt[t] = (st[t][0] + st[t][1]) + (st[t][2] + st[t][3]);
-        pk[2 * t] = ktx_pk_bf16(st[t][0], st[t][1]);
-        pk[2 * t + 1] = ktx_pk_bf16(st[t][2], st[t][3]);
-      }
-      const float sum = pf_sum_rows((mt[0] + mt[1]) + (mt[2] + mt[3]));
-      const float alpha = __expf(m_run - m_new);
-      l_run = l_run * alpha + sum;
-      m_run = m_new;
-      const v8bf pf[2] = {as_v8bf(make_uint4(pk[0], pk[1], pk[2], pk[3])), as_v8bf(make_uint4(pk[4], pk[5], pk[6], pk[7]))};
-      // what the rounding left over
-#pragma unroll
-      for (int t = 0; t < 4; t++)
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-          pk[2 * t + h] = ktx_pk_bf16(st[t][2 * h] - __uint_as_float(pk[2 * t + h] << 16), st[t][2 * h + 1] - __uint_as_float(pk[2 * t + h] & 0xffff0000u));
-      const v8bf pl[2] = {as_v8bf(make_uint4(pk[0], pk[1], pk[2], pk[3])), as_v8bf(make_uint4(pk[4], pk[5], pk[6], pk[7]))};
-      // the rescale only where some head's running maximum moved (alpha == 1 exactly otherwise)
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0ull) {
-#pragma unroll
-        for (int i = 0; i < 16; i++)
+        for (int i = 0; i < 32; i++) {
 #pragma unroll
           for (int r = 0; r < 4; r++) o[i][r] *= alpha;
+          asm volatile("" : "+a"(o[i]));   // (in the MFMAs' registers on both sides of the branch, or the compiler moves all of them there and back in every tile)
+        }
       }
-      // ---- O^T += V^T P^T: transposed reads of the same rows
-      typedef __attribute__((address_space(3))) v4s16 lds_v4;
-      union VFrag { v4s16 h[2]; v8bf v; };
-      VFrag vf[2][4];
-      auto load_v = [&](int j) __attribute__((always_inline)) {
-        const uint8_t* a = kb + (vx ^ (j * 32));
 #pragma unroll
-        for (int q = 0; q < 4; q++) {   // (i, u) = (q >> 1, q & 1)
-          vf[j & 1][q].h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(a + (q >> 1) * 256 + (q & 1) * (32 * MLA_DC * 2)));
-          vf[j & 1][q].h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(a + (q >> 1) * 256 + (q & 1) * (32 * MLA_DC * 2) + 16 * MLA_DC * 2));
+      for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) st[t][r] = __expf(st[t][r] - m_run);
+      bool bring = false;
+      if constexpr (MORE)
+        if (tile + NBUF - 1 < t_end) {
+          bring = locate(tile + NBUF - 1);
+          if (!bring) request_any(tile + NBUF - 1);
+        }
+      uint32_t hi[4], lo[4];
+      float sum = 0.f;
+      auto probabilities = [&](int piece) __attribute__((always_inline)) {
+        if (piece < 4) {
+          const int t = piece >> 1, h = piece & 1;
+          hi[piece] = ktx_pk_bf16(st[t][2 * h], st[t][2 * h + 1]);
+        } else if (piece < 8) {   // what the rounding left over
+          const int t = (piece >> 1) & 1, h = piece & 1;
+          lo[piece - 4] = ktx_pk_bf16(st[t][2 * h] - __uint_as_float(hi[piece - 4] << 16), st[t][2 * h + 1] - __uint_as_float(hi[piece - 4] & 0xffff0000u));
+        } else if (piece == 8) {
+          sum = ((st[0][0] + st[0][1]) + (st[0][2] + st[0][3])) + ((st[1][0] + st[1][1]) + (st[1][2] + st[1][3]));
+        } else if (piece == 9) {
+          l_run += pf_sum_rows(sum);
         }
       };
-      load_v(0);
+      if constexpr (MORE) {
+        scores(tile + 1, sn, [&](int s) __attribute__((always_inline)) {
+          probabilities(s);
+          if (s >= NQ - 4 * VA) load_v(tile, (s - NQ + 4 * VA) / 4, (s - NQ + 4 * VA) % 4);
+          if (s >= 1 && s < 1 + REQ && bring) request(s - 1);
+        });
+      } else {
+#pragma unroll
+        for (int i = 0; i < 10; i++) probabilities(i);
+#pragma unroll
+        for (int j = 0; j < 4 * VA; j++) load_v(tile, j / 4, j % 4);
+      }
+      const v8bf pf = as_v8bf(make_uint4(hi[0], hi[1], hi[2], hi[3])), pl = as_v8bf(make_uint4(lo[0], lo[1], lo[2], lo[3]));
+      // ---- O^T += V^T P^T
 #pragma unroll
       for (int j = 0; j < 8; j++) {
-        if (j + 1 < 8) load_v(j + 1);
 #pragma unroll
-        for (int u = 0; u < 2; u++)
+        for (int i = 0; i < 4; i++)
+          if (j + VA < 8) load_v(tile, j + VA, i);
 #pragma unroll
-          for (int i = 0; i < 2; i++) o[i * 8 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j & 1][i * 2 + u].v, pf[u], o[i * 8 + j], 0, 0, 0);
+        for (int i = 0; i < 4; i++) o[i * 8 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j % (VA + 1)][i].v, pf, o[i * 8 + j], 0, 0, 0);
 #pragma unroll
-        for (int u = 0; u < 2; u++)
+        for (int i = 0; i < 4; i++) o[i * 8 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j % (VA + 1)][i].v, pl, o[i * 8 + j], 0, 0, 0);
+        if constexpr (MORE)
+          if (j >= 1 && j < 5) prepare(j - 1, tile + 1, sn);
 #pragma unroll
-          for (int i = 0; i < 2; i++) o[i * 8 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j & 1][i * 2 + u].v, pl[u], o[i * 8 + j], 0, 0, 0);
+        for (int i = 0; i < 8; i++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
+    };
+
+    v4f sa[2], sb[2];
+    arrived(t_begin);
+#pragma unroll
+    for (int s = 0; s < KA; s++) load_k(t_begin, s);
+    scores(t_begin, sa, [](int) {});
+#pragma unroll
+    for (int i = 0; i < 4; i++) prepare(i, t_begin, sa);
+    MLA_TS(3);
+    int tile = t_begin;
+    for (; tile + 1 < t_end; tile++) {
+      step(std::true_type{}, tile, sa, sb);
+      sa[0] = sb[0];
+      sa[1] = sb[1];
     }
+    step(std::false_type{}, tile, sa, sb);
   }
   MLA_TS(6);
 
-  const int dim0 = ds * 256 + 4 * g;   // + 16 i
+  const int dim0 = 4 * g;   // + 16 i
   if (p.out1) {   // one split holds the whole row: the merge kernel's arithmetic for a single partial (weight 1), in place
     const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
     bf16_t* po = p.out1 + ((size_t)qt * p.Hq + head) * MLA_DC + dim0;
 #pragma unroll
-    for (int i = 0; i < 16; i++)
+    for (int i = 0; i < 32; i++)
       *reinterpret_cast<uint2*>(po + i * 16) = make_uint2(ktx_pk_bf16(o[i][0] * inv, o[i][1] * inv), ktx_pk_bf16(o[i][2] * inv, o[i][3] * inv));
-    if (p.lse1 && g == 0 && ds == 0)
+    if (p.lse1 && g == 0)
       p.lse1[(size_t)qt * p.Hq + head] = l_run > 0.f ? (m_run + __logf(l_run)) * 1.44269504089f : -__builtin_inff();
     return;
   }
   // ---- partial results: un-normalised O plus (m, l) per head
   const size_t pidx = ((size_t)qt * p.Hq + head) * p.nsplit + split;
-  if (g == 0 && ds == 0) *reinterpret_cast<float2*>(p.part_ml + pidx * 2) = make_float2(m_run, l_run);
+  if (g == 0) *reinterpret_cast<float2*>(p.part_ml + pidx * 2) = make_float2(m_run, l_run);
   if (t_begin < t_end) {
     float* po = p.part_o + pidx * MLA_DC + dim0;
 #pragma unroll
-    for (int i = 0; i < 16; i++) *reinterpret_cast<float4*>(po + i * 16) = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
+    for (int i = 0; i < 32; i++) *reinterpret_cast<float4*>(po + i * 16) = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
   }
   MLA_TS(7);
 }
@@ -1100,9 +1166,9 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
   } else if (wide) {
     KTX_TIMED(st, kv_bytes + (double)total_q_tokens * Hq * (MLA_DC + MLA_DR + MLA_DC) * 2.0,
               "mla_decode_wide_kernel T=%d Hq=%d nsplit=%d", total_q_tokens, Hq, p.nsplit);
-    constexpr size_t lds4 = 2 * 2 * MLA_TILE * (MLA_DC + MLA_DR) * sizeof(bf16_t) + 8 * 2 * 64 * sizeof(float4);   // all of a CU's
-    KTX_HIP(ktx_set_max_lds(reinterpret_cast<const void*>(mla_decode_wide_kernel), 160 * 1024));
-    hipLaunchKernelGGL(mla_decode_wide_kernel, p.jobs ? dim3(p.jobs, hblocks) : grid, dim3(512), lds4, st, p);
+    constexpr size_t lds4 = 4 * MLA_TILE * (MLA_DC + MLA_DR) * sizeof(bf16_t);
+    KTX_HIP(ktx_set_max_lds(reinterpret_cast<const void*>(mla_decode_wide_kernel), (int)lds4));
+    hipLaunchKernelGGL(mla_decode_wide_kernel, p.jobs ? dim3(p.jobs, hblocks) : grid, dim3(256), lds4, st, p);
   } else {
     KTX_TIMED(st, kv_bytes + (double)total_q_tokens * Hq * (MLA_DC + MLA_DR + MLA_DC) * 2.0,
               "mla_decode_kernel<1,4> T=%d Hq=%d nsplit=%d", total_q_tokens, Hq, nsplit);

@@ -138,6 +138,42 @@ def test_wide_decode_is_off_by_the_rounding_of_its_outputs(Hq, lens):
     assert float((run().double() - want).norm()) <= 1.01 * floor
 
 
+@pytest.mark.parametrize("Hq,lens,ramp", [(128, [32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 31, 1, 512, 700, 1024, 3] * 2, 0.0),   # 1 to 5 tiles a workgroup and more, whole and not
+                                          (64, [9000] * 60 + [1, 40, 8999, 9000], 0.0),                                          # more than 64 tiles: the page table again
+                                          (128, [2000] * 8 + [4000] * 12, 2.5), (128, [2000] * 8 + [4000] * 12, -2.5),            # scores that grow a tile by less than what rescales the sums ...
+                                          (64, [4000] * 20, 7.0), (64, [4000] * 20, 0.4)])                                        # ... by more, and by little for long
+def test_wide_decode_tiles_and_growing_scores(Hq, lens, ramp):
+    """mla_decode_wide_kernel at the edges of its tiles, and where a head's largest score moves on in every tile of 32 (by `ramp`): off by the rounding of its outputs."""
+    from ktransformers_amd import _native as n
+    g = torch.Generator(device=DEV).manual_seed(11)
+    B, page, pages = len(lens), 64, [(m + 63) // 64 for m in lens]
+    first = [0] + [int(v) for v in np.cumsum(pages)]
+    table = torch.randperm(first[-1], device=DEV, generator=g).to(torch.int32)
+    cache, q_nope, q_pe = (torch.randn(s, device=DEV, generator=g).to(torch.bfloat16) for s in ((first[-1], page, 576), (B, Hq, 512), (B, Hq, 64)))
+    scale = 192 ** -0.5
+    if ramp:   # the last rotated dim, which O has no part of: q 16 there, a token's key its tile's share
+        q_pe[..., -1] = 16
+        for b in range(B):
+            at = (torch.arange(pages[b] * 64, device=DEV) // 32 % 64).float() * (ramp / 16 / scale)
+            cache[table[first[b]:first[b + 1]].long(), :, -1] = at.view(-1, 64).to(torch.bfloat16)
+    w = n.MLAWrapper(B, first[-1], use_cuda_graph=False, device=DEV, max_q_tokens=B)
+    dev = [torch.tensor(a, dtype=torch.int32, device=DEV) for a in (range(B + 1), first, lens, [B])]
+    w.plan(dev[0], dev[1], table, dev[2], dev[3], Hq, 512, 64, page, scale, max_kv_len=max(lens))
+    n.timing_enable(2)
+    try:
+        out = w.run(q_nope, q_pe, cache[:, :, :512], cache[:, :, 512:])
+        assert any("mla_decode_wide_kernel" in t[0] for t in n.timing_collect())
+    finally:
+        n.timing_enable(0)
+    want = []
+    for b, m in enumerate(lens):
+        rows = cache[table[first[b]:first[b + 1]].long()].view(-1, 576)[:m].double()
+        want.append(torch.softmax(torch.cat((q_nope[b], q_pe[b]), dim=1).double() @ rows.T * scale, dim=1) @ rows[:, :512])
+    want = torch.stack(want)
+    floor = float((want.to(torch.bfloat16).double() - want).norm())
+    assert float((out.double() - want).norm()) <= 1.01 * floor
+
+
 @pytest.mark.parametrize("Hq,lens,wide", [(64, [600] * 20, False), (64, [300] * 24, False), (128, [200] * 16, False), (64, [16384] * 2, False), (128, [2000] * 8, False),
                                           (64, [50] * 20, True), (64, [1000] * 20, True), (128, [1000] * 12, True), (128, [8192] * 8, True), (64, [8192] * 3, True)])
 def test_which_decode_kernel_a_batch_takes(Hq, lens, wide):
