@@ -205,6 +205,29 @@ def test_fp8_act_quant_writes_its_rows_only(T):
         assert not bool(sT[:, T:zeros].any()) and bool((sT[:, zeros:] == 7.0).all())
 
 
+@pytest.mark.parametrize("exponent", [-133, -126, -90, -82, -81, 0, 9, 98, 99, 100, 126])   # of a block's largest: subnormal scales, both ends of the reciprocal's range, large ones
+def test_fp8_act_quant_rounds_as_a_division(exponent):
+    """quant8_fp8 multiplies by the scale's reciprocal and corrects the product once: the bytes of x / s in e4m3, zeros' signs included, for every pair of bf16
+    mantissas of an element and of its block's largest magnitude."""
+    n = native()
+    top = torch.ldexp(torch.arange(128, 256, dtype=torch.float64) / 128, torch.tensor(exponent)).to(torch.bfloat16)   # one block a row
+    x = torch.ldexp(torch.arange(128, 256, dtype=torch.float64) / 128, torch.tensor(exponent)).expand(128, 128)
+    g = torch.Generator().manual_seed(exponent + 200)
+    x = torch.ldexp(x, -torch.randint(1, 12, (8, 128, 128), generator=g)) * (1 - 2 * torch.randint(0, 2, (8, 128, 128), generator=g))   # eight sets of exponents and signs
+    x[:, :, 5], x[:, :, 6] = 0.0, -0.0
+    x = x.to(torch.bfloat16)
+    x[..., 0] = top
+    x = x.view(1024, 128)
+    amax = x.float().abs().amax(1, keepdim=True)
+    s = amax / 448.0
+    want = torch.where(s > 0, x.float() / s, torch.zeros(())).to(torch.float8_e4m3fn)
+    q, sT = torch.empty((1024, 128), dtype=torch.uint8, device="cuda"), torch.empty((1, 1024), device="cuda")
+    xc = x.cuda()
+    n.check(n.lib.ktx_fp8_act_quant(xc.data_ptr(), 128, 1024, 128, q.data_ptr(), sT.data_ptr(), 1024, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(sT.cpu().view(-1), s.view(-1))
+    assert torch.equal(q.cpu(), want.view(torch.uint8))
+
+
 @pytest.mark.parametrize("K,N,G", [(2048, 576, 64), (1536, 200, 32), (7168, 2112, 128), (1024, 64, -1), (384, 48, 128)])
 def test_w8_format_is_the_bf16_kernel_on_marlins_multiplicand_bit_for_bit(K, N, G):
     """The W8 format (include/ktx_linear.h: KTX_LIN_W8, round 4): one byte per weight in HBM, bf16((q - 128) * s) formed in registers
