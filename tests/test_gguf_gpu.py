@@ -108,6 +108,34 @@ def test_small(types, T):
     run_case(4, 2, 256, 512, T, types, seed=T)
 
 
+@pytest.mark.parametrize("types", [(Q4, Q4, Q4), (IQ1, IQ1, Q6), (Q5, Q5, Q2)])
+@pytest.mark.parametrize("H,I", [(256, 256), (768, 4352)])
+def test_q8_k_of_ties_signs_and_empty_blocks(types, H, I):
+    """q8k_quant_kernel (16 lanes a block) against the decode kernels' quantisation (a wavefront a block), the same chain behind both: rows whose largest magnitude comes
+    several times with both signs, in either order, blocks of zeros, negative zeros and single elements, and counts of blocks that end inside a workgroup."""
+    from ktransformers_amd import _native as n
+    rng = np.random.default_rng(H + I)
+    x = rng.choice(np.array([1.0, -1.0, 0.5, -0.5, 0.25, 0.0, -0.0], np.float32), (8, H))
+    x[1] = 0.0
+    x[2], x[3] = np.abs(x[2]), -np.abs(x[3])
+    x[4] = np.where(np.arange(H) % 256 == 77, -3.0, -0.0)
+    x[5, :] = np.where(np.arange(H) % 128 == 5, 2.0, 0.1)
+    x[5, 133::256] = -2.0
+    ids, w = torch.arange(8).view(8, 1).cuda() % 2, torch.ones((8, 1)).cuda()
+    h = n.MoEHandle(2, 1, H, I, 16, "GGUF", 0)
+    h.load_gguf(*(torch.from_numpy(random_kquant(t, 2, r, c, rng)).cuda() for t, r, c in ((types[0], I, H), (types[1], I, H), (types[2], H, I))), *types)
+    xb = torch.from_numpy(x).to(torch.bfloat16).cuda()
+    n.check(n.lib.ktx_debug_set(20, 1))      # (one k-slice: the grouped kernels' chain)
+    try:
+        want = h.forward(xb, ids, w)
+        n.force_generic_path(True)
+        got = h.forward(xb, ids, w)
+    finally:
+        n.force_generic_path(False)
+        n.check(n.lib.ktx_debug_set(20, 0))
+    assert bool(want.float().abs().sum(1)[[0, 2, 3, 4, 5]].gt(0).all()) and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("types", [(Q5, Q5, Q6), (Q5, Q5, Q5), (Q2, Q2, Q3), (Q3, Q3, Q2), (Q2, Q2, Q2), (Q3, Q3, Q3), (IQ4, IQ4, IQ4),
                                    (IQ4, IQ4, Q5), (Q4, Q4, Q2)])
 @pytest.mark.parametrize("T", [1, 3, 19])
