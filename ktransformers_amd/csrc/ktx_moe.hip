@@ -2648,10 +2648,15 @@ static int forward_rawint4(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, 
 
   // prompt chunks: 64-row tiles through the group-scaled 16x16x32 kernel (moe_rawint4_chunk_kernel: same terms, one fp32 chain per
   // output instead of the reference's sixteen); short batches and dev knob 29 = 1 keep the exact 4-row kernel
+  // Their tiles lie from the expert of the most rows on: what takes a workgroup longest starts first, what ends last is small.  Us, experts in their own order | so: 64 experts of 2048 x 1024, top-8, 64
+  // tokens 79.6 | 72.1, 100 97.1 | 78.0, 200 116 | 101, 500 167 | 154, 1901 424 | 411; 64 of 3072 x 1024, top-4, 942 224 | 208; 32 of 4096 x 2048, top-8, 400 346 | 333; 384 of 7168 x 2048, top-8, 500 1763 |
+  // 1732, 1000 2425 | 2394, 2048 3609 | 3562; where every expert has hundreds of rows the same (8 of 6144 x 3072, top-8, 2000 2787 | 2790), 28 calls none more than 2 % slower (16 of 6144 x 512, top-6, 256 109.7
+  // | 111.7).  Tiles of fp8 and AMXINT4 experts stay in the experts' order: there full tiles wait for the matrix pipe and short ones for the weights, which by size are no longer on the chip together (256
+  // of 7168 x 2048, top-8: fp8, 1000 tokens 2125 | 2305, AMXINT4, 2048 1514 | 1566).
   const bool chunk = qlen >= 64 && g_dbg[29] != 1 && !h->exact && (size_t)npairs * (std::max(H, I) / 32) * 4 < ((size_t)1 << 32);
   PrepParams pp;
   pp.d_bsz = d_bsz; pp.qlen = qlen; pp.k = k; pp.E = E; pp.expert_begin = h->cfg.expert_begin; pp.H = H;
-  pp.by_size = false; pp.rows_per_tile = chunk ? RAW_ROWS : 4; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
+  pp.by_size = chunk; pp.rows_per_tile = chunk ? RAW_ROWS : 4; pp.ids = d_expert_ids; pp.mask = h->mask; pp.x = (const bf16_t*)d_input;
   pp.x_q = ws->x_q; pp.x_d = ws->x_d; pp.row_of_pair = ws->row_of_pair; pp.src_of_row = ws->src_of_row;
   pp.tiles = ws->tiles; pp.counters = ws->counters;
   {
