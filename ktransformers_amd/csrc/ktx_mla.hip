@@ -1003,13 +1003,13 @@ extern "C" int ktx_mla_decode_partials(const ktx_mla_config* cfg, const void* d_
 }
 
 // mla_decode_wide_kernel or mla_decode_kernel<4, 2> for a call of the 64-head shape?  narrow: the splits that the latter would take.  The wide one
-// walks 64 tokens in 3.1 us against 4.2 and shares out what the requests hold, but its first step ends 3 us later, and its shares
+// walks 64 tokens in 2.9 us against 4.2 and shares out what the requests hold, but its first step ends 3 us later, and its shares
 // write 256 workgroups' partials.  Measured with the merge (us, <4, 2> | wide, requests of equal length; of unequal ones the wide one gains 5-20 % more):
 //   one step of 64 tokens: 24 of 40, 64 heads 19 | 14 (nothing to merge);
 //   more workgroups of <4, 2> than CUs, a second round: 16 of 1000, 128 heads 38 | 32; 3 of 8192, 64 heads 34 | 29; 32 of 400, 64 heads (W = 224) 31 | 28;
 //     of 200 tokens at most lost: 20 of 200, 128 heads (W = 160) 32 | 32, unequal 27 | 31;
-//   one round: as <4, 2>'s splits deepen (in tiles of 32): 128 heads, 8 of 3000 (6) 31 | 33, of 4096 (8) 35 | 36, unequal 34 | 32, of 8192 (16) 52 | 49; 64 heads,
-//     where a split's partials weigh twice as much against its tokens, 8 of 4096 (8) 32 | 33, of 6000 (12) 40 | 37, 20 of 600 (2) 22 | 27.
+//   one round: as <4, 2>'s splits deepen (in tiles of 32): 128 heads, 8 of 2000 (4) 27 | 29, of 3000 (6) 32 | 32, unequal 30 | 29, of 4500 (9) 38 | 37, unequal 36 | 31, of 7000 (14) 48 | 43; 64
+//     heads, 8 of 2000 (4) 25 | 25, 10 24 | 27, 8 of 3000 (6) 27 | 27, 16 32 | 33, unequal 30 | 30, 8 of 4500 (9) 34 | 30, 16 39 | 37, unequal 37 | 32, 20 of 600 (2) 22 | 27.
 // Without a hint of the contexts' length: past 16 tokens.
 static bool mla_wide_steps(const ktx_mla_config* cfg, int total_q_tokens, int narrow) {
   if (total_q_tokens > 64) return false;
@@ -1018,7 +1018,7 @@ static bool mla_wide_steps(const ktx_mla_config* cfg, int total_q_tokens, int na
   if (steps == 1) return true;
   if (narrow * total_q_tokens * hblocks > 256) return steps * total_q_tokens * hblocks >= 192;
   const int tiles = (cfg->kv_len_hint + MLA_TILE - 1) / MLA_TILE;
-  return (tiles + narrow - 1) / narrow >= (hblocks == 1 ? 10 : 8);
+  return (tiles + narrow - 1) / narrow >= 8;
 }
 
 // Workgroup shape and KV split count of a decode call — one place, because the one-launch decode step (ktx_attn.hip) must
@@ -1038,7 +1038,16 @@ static void mla_pick_shape(const ktx_mla_config* cfg, int total_q_tokens, size_t
   // a decode BATCH (>= 8 query tokens, each with its own context): every head block of a token re-reads that token's latent rows, so
   // 64 heads per workgroup halve the KV traffic (V3 dims, 8 x 4096 tokens: 150 -> 75 MB per layer; batch-of-8 step 14.47 -> 13.91 ms,
   // profiles/r06_zz_bs8_mla_shape.txt)
-  const bool batched = decode_sized && total_q_tokens >= 8 && Hq % 64 == 0 && !one_launch;
+  // Fewer (5 and more: what the one-launch step and its companions take stays as it is) where the 2x4 shape's workgroups would take a second round of the CUs. Us, 2x4 | these, 128 heads: 5 of 800
+  // (260 workgroups) 20.8 | 20.8, 6 (312) 23.4 | 21.4; 5 of 2000 (320) 32 | 26, unequal 27 | 26, of 3000 39 | 29, unequal 30 | 30, of 6000 58 | 33, unequal 42 | 30; 7 of 1200 (364) 27 | 23, of 7500 71 | 42; one
+  // call of 45 lost much, 6 unequal ones of 3000 26.5 | 29.9.  64 heads take one round to 7 requests: 5 of 2000 18 | 22, of 7500 30 | 31.
+  auto second_round = [&]() {
+    if (cfg->kv_len_hint <= 0) return false;   // (contexts of unknown length: as before)
+    const int tiles = (cfg->kv_len_hint + MLA_TILE - 1) / MLA_TILE, pairs = Hq / 32 * total_q_tokens, most = std::min(std::max(16, 256 / pairs), std::max(1, cfg->max_splits));
+    const int depth = (tiles + most - 1) / most;
+    return pairs * ((tiles + depth - 1) / depth) >= 300;
+  };
+  const bool batched = decode_sized && Hq % 64 == 0 && !one_launch && (total_q_tokens >= 8 || (total_q_tokens >= 5 && second_round()));
   int shape = (Hq % 32 == 0 && Hq >= 64 && decode_sized && !long_ctx && !batched) ? 2 : (Hq % 64 == 0) ? 4 : 1;
   {   // tuning knobs (scripts/mla_sweep.py): 6 = force the workgroup shape, 7 = force the split count
     const int fs = ktx_debug_get(6);

@@ -192,6 +192,24 @@ def test_which_decode_kernel_a_batch_takes(Hq, lens, wide):
     assert float((out.double() - want).norm() / want.norm()) < 2.4e-3      # (sqrt(2) of 1.66e-3: outputs and probabilities in bf16)
 
 
+@pytest.mark.parametrize("Hq,lens,kernel", [(128, [3000] * 4, "mla_decode_kernel<2,4>"), (128, [400] * 5, "mla_decode_kernel<2,4>"), (128, [2000, 500, 777, 1999, 1], "mla_decode_kernel<4,2>"),
+                                            (128, [1000] * 6, "mla_decode_kernel<4,2>"), (128, [4500] * 5, "mla_decode_wide_kernel"), (128, [6000, 33, 1500, 6000, 64, 4000, 31], "mla_decode_wide_kernel"),
+                                            (64, [7000] * 7, "mla_decode_kernel<2,4>"), (64, [4200] * 8, "mla_decode_wide_kernel"), (64, [3000] * 8, "mla_decode_kernel<4,2>")])
+def test_which_decode_kernel_a_few_requests_take(Hq, lens, kernel):
+    """5 to 7 requests of 128 heads leave the 2x4 shape where its workgroups would take a second round; the 64-token kernel from splits of 8 tiles on at 64 heads too."""
+    from ktransformers_amd import _native as n
+    run, exact = decode_batch(Hq, lens)
+    n.timing_enable(2)
+    try:
+        out = run()
+        labels = [t[0] for t in n.timing_collect()]
+    finally:
+        n.timing_enable(0)
+    assert labels[0].startswith(kernel), labels
+    want = exact()
+    assert float((out.double() - want).norm() / want.norm()) < 2.4e-3      # (sqrt(2) of 1.66e-3: outputs and probabilities in bf16)
+
+
 def test_single_split_equals_many():
     run_case(16, 64, [3000], [1], seed=4, max_splits=1)
 
