@@ -1279,10 +1279,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 :
     const int all = ntiles;
     tile0 = all * split / p.nsplit;
     ntiles = all * (split + 1) / p.nsplit;
-    if (tile0 == ntiles) {   // (fewer tiles than pieces)
+    if (tile0 == ntiles) {   // (fewer tiles than pieces: a sum of -1 says that no O is there)
       for (int r = tid; r < 64 * NU; r += 256) {
         const int t = qb * (64 * NU) + r;
-        if (t < p.T) *reinterpret_cast<float2*>(p.part_ml + (((size_t)t * p.H + h) * p.nsplit + split) * 2) = make_float2(-__builtin_inff(), 0.f);
+        if (t < p.T) *reinterpret_cast<float2*>(p.part_ml + (((size_t)t * p.H + h) * p.nsplit + split) * 2) = make_float2(-__builtin_inff(), -1.f);
       }
       return;
     }
@@ -1430,7 +1430,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 :
 #pragma unroll
     for (int u = 0; u < NU; u++)
       if (!__all(mx[u] <= m_run[u])) {
-        const float m_new = fmaxf(m_run[u], mx[u]);             // finite from tile 0 on: key 0 is visible to every query (SPLIT: or the query has seen no key yet)
+        const float m_new = fmaxf(m_run[u], mx[u]);             // finite from tile 0 on: key 0 is visible to every query (SPLIT, tile0 > 0: or the query has seen no key yet)
         const float alpha = SPLIT && m_new == m_run[u] ? 1.f : __builtin_amdgcn_exp2f((m_run[u] - m_new) * cexp);
         m_run[u] = m_new;
         l_run[u] *= alpha;
@@ -1442,7 +1442,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ALONE ? 1 :
     uint4 pb[NU][2];
 #pragma unroll
     for (int u = 0; u < NU; u++) {
-      const float mc = SPLIT && m_run[u] == -__builtin_inff() ? 0.f : -m_run[u] * cexp;
+      // (SPLIT: no key seen yet, so that the tile's weigh nothing.  A first tile of scores of -inf gives NaN, shared or not.)
+      const float mc = SPLIT && tile0 > 0 && m_run[u] == -__builtin_inff() ? 0.f : -m_run[u] * cexp;
       float sum2[2] = {0.f, 0.f};
       float pv[4][4];
 #pragma unroll
@@ -1572,7 +1573,7 @@ __global__ __launch_bounds__(256) void mla_prefill_merge_kernel(MlaPrefillParams
   float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int s = 0; s < NS; s++) {
-    if (s >= p.nsplit || ml[s].y == 0.f) continue;   // (a piece without a key of the query's: nothing, or old memory)
+    if (s >= p.nsplit || ml[s].y < 0.f) continue;   // (a piece without a tile: old memory.  One without a key of the query's weighs 0, which an infinite value makes NaN as in an unshared tile.)
     const float w = __builtin_amdgcn_exp2f((ml[s].x - m) * c);
     l += w * ml[s].y;
     v.x += w * o[s].x; v.y += w * o[s].y; v.z += w * o[s].z; v.w += w * o[s].w;

@@ -364,6 +364,45 @@ def test_prefill_keys_shared_by_workgroups(H, T, kv_len, nsplit):
         assert bool((err <= bound).all()), f"{int((err > bound).sum())} outputs, up to {float((err / bound).max()):.2f} of the bound"
 
 
+@pytest.mark.parametrize("nsplit", [2, 3, 5, 16])
+@pytest.mark.parametrize("what", ["scores", "values", "nan"])
+def test_prefill_infinities_shared_or_not(what, nsplit):
+    """Infinities and NaN come out of a shared query as out of an unshared one: a query whose visible scores are all -inf (head 0), whose first tile's are (head 1), a later run of
+    tiles (head 2); an infinite value, which queries before it multiply with 0; a NaN in a key."""
+    from ktransformers_amd import _native as n
+    H, T, kv_len = 3, 130, 1030
+    q, k_nope, cache, v = prefill_operands(H, T, kv_len)
+    q[:, :, 0] = 0
+    s = prefill_scores(q, k_nope, cache, kv_len)
+    ref, bound = prefill_statement(s, v[:, :kv_len].double())
+    if what == "scores":
+        q[[7, 100], :, 0] = 3e38
+        k_nope[:, :, 0] = 0
+        for h, keys in enumerate((slice(None), slice(0, 64), slice(192, 384))):
+            k_nope[h, keys, 0] = -4
+            s[h, [7, 100], keys] = float("-inf")
+        ref, bound = prefill_statement(s, v[:, :kv_len].double())
+    elif what == "values":
+        v[:, 950, 5], v[:, 64, 9], v[:, 1029, 11] = float("inf"), float("-inf"), float("inf")
+    else:
+        k_nope[1, 970, 3], v[2, 20, 2] = float("nan"), float("nan")
+    qd, args = q.to(DEV), (k_nope.to(DEV), cache.to(DEV)[:, 512:], v.transpose(1, 2).contiguous().to(DEV), kv_len, 192 ** -0.5)
+    try:
+        n.lib.ktx_debug_set(33, 1)
+        whole = n.mla_prefill(qd[:, :, :128], qd[:, :, 128:], *args).cpu().double()
+        n.lib.ktx_debug_set(33, nsplit)
+        shared = n.mla_prefill(qd[:, :, :128], qd[:, :, 128:], *args).cpu().double()
+    finally:
+        n.lib.ktx_debug_set(33, 0)
+    finite = torch.isfinite(whole)
+    assert bool((~finite).any()) and bool(finite.any())
+    if what == "scores":
+        assert bool(torch.isnan(whole[[7, 100], 0]).all()) and bool(finite[:, 2].all())
+    assert torch.equal(torch.isnan(whole), torch.isnan(shared)) and torch.equal(whole[torch.isinf(whole)], shared[torch.isinf(whole)])
+    for got in (whole, shared):
+        assert bool(((got - ref).abs() <= bound)[finite].all())
+
+
 @pytest.mark.parametrize("Hq,kv_len,T", [(128, 4023, 1), (64, 700, 1), (128, 33, 1), (64, 5000, 3)])
 def test_merge_riding_the_unabsorb_launch(Hq, kv_len, T):
     """ktx_mla_decode_partials + ktx_linear_forward_batched_merge (the KV-split merge inside the launch of the per-head un-absorb
