@@ -555,7 +555,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   v4f o[32];     // O^T: dims 16 i + 4 g + (0..3) of the lane's head
 #pragma unroll
   for (int i = 0; i < 32; i++) o[i] = v4f{0.f, 0.f, 0.f, 0.f};
-  float m_run = -__builtin_inff(), l_run = 0.f;
+  float m_run = -__FLT_MAX__, l_run = 0.f;   // (lowest, not -inf: scores of -inf then weigh 0 also where a split begins with a whole tile of them)
 
   if (t_begin < t_end) {
     if (app_pos >= 0 && hb == 0 && app_pos / MLA_TILE >= t_begin && app_pos / MLA_TILE < t_end) mla_store_appended(p, req, page_base, app_pos, tid);
@@ -815,7 +815,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
   const int dim0 = 4 * g;   // + 16 i
   if (p.out1) {   // one split holds the whole row: the merge kernel's arithmetic for a single partial (weight 1), in place
-    const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+    const float inv = t_begin < t_end ? 1.0f / l_run : 0.f;   // (scores of -inf alone: NaN)
     bf16_t* po = p.out1 + ((size_t)qt * p.Hq + head) * MLA_DC + dim0;
 #pragma unroll
     for (int i = 0; i < 32; i++)

@@ -174,6 +174,32 @@ def test_wide_decode_tiles_and_growing_scores(Hq, lens, ramp):
     assert float((out.double() - want).norm()) <= 1.01 * floor
 
 
+@pytest.mark.parametrize("lens", [[2000] * 20, [40] * 24])   # several splits a request; one, whose result the kernel stores itself
+def test_wide_decode_of_infinite_scores(lens):
+    """Scores of -inf weigh nothing, wherever a split begins: every even tile of 32 tokens is -inf to every third head."""
+    from ktransformers_amd import _native as n
+    g = torch.Generator(device=DEV).manual_seed(5)
+    B, Hq, page, m = len(lens), 128, 64, lens[0]
+    pages = (m + 63) // 64
+    cache, q_nope, q_pe = (torch.randn(s, device=DEV, generator=g).to(torch.bfloat16) for s in ((B * pages, page, 576), (B, Hq, 512), (B, Hq, 64)))
+    q_pe[..., -1] = 0
+    q_pe[:, ::3, -1] = 3e38
+    cache[..., -1] = torch.where(torch.arange(64, device=DEV) < 32, -4.0, 0.0).to(torch.bfloat16)
+    w = n.MLAWrapper(B, B * pages, use_cuda_graph=False, device=DEV, max_q_tokens=B)
+    dev = [torch.tensor(a, dtype=torch.int32, device=DEV) for a in (range(B + 1), range(0, B * pages + 1, pages), lens, [B])]
+    w.plan(dev[0], dev[1], None, dev[2], dev[3], Hq, 512, 64, page, 192 ** -0.5, max_kv_len=m, identity_pages=True)
+    n.timing_enable(2)
+    try:
+        out = w.run(q_nope, q_pe, cache[:, :, :512], cache[:, :, 512:])
+        assert "mla_decode_wide_kernel" in n.timing_collect()[0][0]
+    finally:
+        n.timing_enable(0)
+    rows = cache.view(B, pages * 64, 576)[:, :m].double()
+    want = torch.matmul(torch.softmax(torch.matmul(torch.cat((q_nope, q_pe), dim=2).double(), rows.transpose(1, 2).contiguous()) * 192 ** -0.5, dim=2), rows[..., :512].contiguous())
+    floor = float((want.to(torch.bfloat16).double() - want).norm())
+    assert float((out.double() - want).norm()) <= 1.01 * floor
+
+
 @pytest.mark.parametrize("Hq,lens,wide", [(64, [600] * 20, False), (64, [300] * 24, False), (128, [200] * 16, False), (64, [16384] * 2, False), (128, [2000] * 8, False),
                                           (64, [50] * 20, True), (64, [1000] * 20, True), (128, [1000] * 12, True), (128, [8192] * 8, True), (64, [8192] * 3, True)])
 def test_which_decode_kernel_a_batch_takes(Hq, lens, wide):
