@@ -515,8 +515,9 @@ __device__ __forceinline__ float pf_sum_rows(float x) {
 // 8 rows off each other's banks.
 // P enters the product as two bf16, the second what rounding the first left over.  One bf16 is off by its rounding except where P is exactly 1, a
 // split's largest entry, and here a split is longer than in mla_decode_kernel: the error against 64-bit sums grew by 1 to 4 % (32 requests
-// of 500 tokens, 128 heads 1.77e-3 -> 1.84e-3).  With two it is the outputs' rounding alone, 1.66e-3 at every size, also where P passes 1: sums are rescaled only when a head's
-// largest score has grown by MLA_GROWTH (P to 256) since they last were, for a split's first tile finds most of it and every rescaling is 128 products a lane.
+// of 500 tokens, 128 heads 1.77e-3 -> 1.84e-3).  With two it is the outputs' rounding alone, 1.66e-3 at every size, also where P is far below 1: sums are rescaled only when a head's
+// largest score has grown by MLA_GROWTH since they last were, for a split's first tile finds most of it and every rescaling is 128 products a lane.  What P is relative to lies that much
+// above the largest score then, so that P ends at 1 and sums of it overflow where they did with every maximum followed, not at a 256th of that.
 // distinct for 16 rows, also with rows 4 .. 11 flipped by 1 (ds_read_b128 takes lanes 0-3, 12-15, 20-23, 24-27 together); >> 1 distinct for rows
 // 0-7 and for 8-15 (ds_read_b64_tr_b16 takes 32 lanes together)
 __device__ __forceinline__ uint32_t mla_swz(uint32_t row) { return row & 8 ? ((row & 7) ^ 4) << 1 | 1 : (row & 7) << 1; }
@@ -724,8 +725,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       }
 #pragma unroll
       for (int i = 0; i < 32; i++) asm volatile("" : "+a"(o[i]));
-      if (__builtin_amdgcn_ballot_w64(mx > m_run + MLA_GROWTH) != 0ull) {
-        const float m_new = fmaxf(m_run, mx), alpha = __expf(m_run - m_new);
+      if (__builtin_amdgcn_ballot_w64(mx > m_run) != 0ull) {
+        const float m_new = fmaxf(m_run, mx + MLA_GROWTH), alpha = __expf(m_run - m_new);
         m_run = m_new;
         l_run *= alpha;
 #pragma unroll

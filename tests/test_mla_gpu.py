@@ -143,7 +143,8 @@ def test_wide_decode_is_off_by_the_rounding_of_its_outputs(Hq, lens):
                                           (128, [2000] * 8 + [4000] * 12, 2.5), (128, [2000] * 8 + [4000] * 12, -2.5),            # scores that grow a tile by less than what rescales the sums ...
                                           (64, [4000] * 20, 7.0), (64, [4000] * 20, 0.4)])                                        # ... by more, and by little for long
 def test_wide_decode_tiles_and_growing_scores(Hq, lens, ramp):
-    """mla_decode_wide_kernel at the edges of its tiles, and where a head's largest score moves on in every tile of 32 (by `ramp`): off by the rounding of its outputs."""
+    """mla_decode_wide_kernel at the edges of its tiles, and where a head's largest score moves on in every tile of 32 (by `ramp`): off by the rounding of its outputs.  One dim,
+    which the scores have no part of, holds 2e36: probabilities past 1 would take its sums out of fp32."""
     from ktransformers_amd import _native as n
     g = torch.Generator(device=DEV).manual_seed(11)
     B, page, pages = len(lens), 64, [(m + 63) // 64 for m in lens]
@@ -151,6 +152,7 @@ def test_wide_decode_tiles_and_growing_scores(Hq, lens, ramp):
     table = torch.randperm(first[-1], device=DEV, generator=g).to(torch.int32)
     cache, q_nope, q_pe = (torch.randn(s, device=DEV, generator=g).to(torch.bfloat16) for s in ((first[-1], page, 576), (B, Hq, 512), (B, Hq, 64)))
     scale = 192 ** -0.5
+    q_nope[..., 7], cache[..., 7] = 0, 2e36
     if ramp:   # the last rotated dim, which O has no part of: q 16 there, a token's key its tile's share
         q_pe[..., -1] = 16
         for b in range(B):
@@ -170,6 +172,8 @@ def test_wide_decode_tiles_and_growing_scores(Hq, lens, ramp):
         rows = cache[table[first[b]:first[b + 1]].long()].view(-1, 576)[:m].double()
         want.append(torch.softmax(torch.cat((q_nope[b], q_pe[b]), dim=1).double() @ rows.T * scale, dim=1) @ rows[:, :512])
     want = torch.stack(want)
+    assert bool(((out[..., 7].double() - want[..., 7]).abs() <= 2.0 ** -8 * 1.01 * want[..., 7]).all())
+    out, want = (torch.cat((t[..., :7], t[..., 8:]), dim=-1) for t in (out, want))
     floor = float((want.to(torch.bfloat16).double() - want).norm())
     assert float((out.double() - want).norm()) <= 1.01 * floor
 
