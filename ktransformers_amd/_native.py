@@ -249,15 +249,22 @@ lib = _TracedLib(_load())
 
 
 def _load_host():
-    """csrc/ktx_host.cpp: the shortest calls without an interpreter step per argument.  None where it has not been built: every call is then made from here."""
-    path = os.path.join(_HERE, "lib", "ktx_host.so")
+    """csrc/ktx_host.cpp: the shortest calls without an interpreter step per argument.  None where it has not been built for this torch and this interpreter, or does not load
+    (with a warning): every call is then made from here."""
+    from .build import host_lib
+    path = host_lib()
     if not os.path.exists(path):
         return None
     import importlib.machinery
     import importlib.util
     loader = importlib.machinery.ExtensionFileLoader("ktx_host", path)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("ktx_host", loader))
-    loader.exec_module(module)
+    try:
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("ktx_host", loader))
+        loader.exec_module(module)
+    except ImportError as e:
+        import warnings
+        warnings.warn(f"{path} does not load, so that short calls take the host longer: {e}", RuntimeWarning, stacklevel=2)
+        return None
     module.bind(KtxError, *(C.cast(getattr(lib._raw, f), C.c_void_p).value
                             for f in ("ktx_last_error", "ktx_linear_forward", "ktx_moe_forward", "ktx_mla_prefill_ws", "ktx_mla_decode_append", "ktx_mla_prefill_workspace_bytes")))
     return module

@@ -21,7 +21,6 @@ LIB = os.path.join(LIBDIR, "libktx_hip.so")
 # the sequence-mixer, hybrid-decoder, window-attention / scan and decayed-state kernels alone (include/ktx_seq.h, ktx_hyb.h, ktx_swa.h,
 # ktx_gla.h): what the fp32-residual families need, built in about a minute
 SEQ_LIB = os.path.join(LIBDIR, "libktx_seq.so")
-HOST_LIB = os.path.join(LIBDIR, "ktx_host.so")
 HOST_SOURCE = os.path.join(CSRC, "ktx_host.cpp")
 SEQ_SOURCES = ("ktx_seq.hip", "ktx_hyb.hip", "ktx_swa.hip", "ktx_gla.hip", "ktx_err.hip")
 
@@ -97,24 +96,33 @@ def build_seq(force: bool = False, verbose: bool = False) -> str:
     return SEQ_LIB
 
 
+def host_lib() -> str:
+    """Where the host module of this interpreter and this torch lies: it has both's layouts compiled in, so that another one's is not found."""
+    import sysconfig
+
+    import torch
+    return os.path.join(LIBDIR, f"ktx_host-{torch.__version__}{sysconfig.get_config_var('EXT_SUFFIX')}")
+
+
 def build_host(force: bool = False, verbose: bool = False) -> str:
     """The CPython module of the host side (csrc/ktx_host.cpp, against this interpreter's and torch's headers)."""
-    if not force and not _stale(HOST_LIB, [HOST_SOURCE] + _deps(HOST_SOURCE)):
-        return HOST_LIB
+    target = host_lib()
+    if not force and not _stale(target, [HOST_SOURCE, __file__] + _deps(HOST_SOURCE)):
+        return target
     import sysconfig
 
     from torch.utils.cpp_extension import include_paths, library_paths
     os.makedirs(LIBDIR, exist_ok=True)
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
-    tmp = HOST_LIB + f".tmp{os.getpid()}"
+    tmp = target + f".tmp{os.getpid()}"
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
            *[f"-I{d}" for d in include_paths() + [os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]], HOST_SOURCE, "-o", tmp,
            *[f"-L{d}" for d in library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
     if verbose:
         print(" ".join(cmd), file=sys.stderr)
     subprocess.run(cmd, check=True)
-    os.replace(tmp, HOST_LIB)
-    return HOST_LIB
+    os.replace(tmp, target)
+    return target
 
 
 def needs_build() -> bool:
@@ -122,7 +130,16 @@ def needs_build() -> bool:
 
 
 def build(force: bool = False, verbose: bool = False) -> str:
-    build_host(force, verbose)
+    """libktx_hip.so, and the host module beside it where there are a compiler and headers for it: without it every call is made from Python."""
+    lib = _build_lib(force, verbose)
+    try:
+        build_host(force, verbose)
+    except (OSError, ImportError, subprocess.CalledProcessError) as e:
+        print(f"ktransformers_amd: {os.path.basename(HOST_SOURCE)} was not built ({e}); short calls take the host longer without it", file=sys.stderr)
+    return lib
+
+
+def _build_lib(force: bool, verbose: bool) -> str:
     if not force and not needs_build():
         return LIB
     os.makedirs(OBJDIR, exist_ok=True)

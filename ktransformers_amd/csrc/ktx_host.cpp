@@ -1,4 +1,4 @@
-// ktx_host.cpp — the host side of the shortest calls (a CPython module, built as lib/ktx_host.so): checks, the result's allocation and the call into
+// ktx_host.cpp — the host side of the shortest calls (a CPython module, built as lib/ktx_host-<torch><interpreter>.so): checks, the result's allocation and the call into
 // libktx_hip.so without an interpreter step per argument.
 //
 // A decode step makes these calls by the hundred, and their kernels take 4 to 12 us: in Python (ctypes converts 10 to 20 arguments, a tensor's sizes and
