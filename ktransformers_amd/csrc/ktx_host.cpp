@@ -11,10 +11,12 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <cstring>
+#include <string>
 
 #include "../../include/ktx_mla.h"
 
@@ -47,7 +49,10 @@ inline const at::Tensor* plain(PyObject* o, at::ScalarType type) {
   if ((ks != usual && ks != inference) || t.scalar_type() != type) return nullptr;
   return &t;
 }
-inline bool modes() { return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled(); }
+inline bool modes() {   // (or a transform of torch.func, inside which new tensors are wrapped)
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
 inline void* stream_of(const at::Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 inline PyObject* none() { Py_RETURN_NONE; }
 inline bool integer(PyObject* o, int64_t& v) {
@@ -57,32 +62,33 @@ inline bool integer(PyObject* o, int64_t& v) {
   return true;
 }
 
-struct Released {   // the interpreter, while a launch may wait for the queue
+struct Released {   // the interpreter, while a launch may wait for the queue, or memory for the allocator or the device
   PyThreadState* state = PyEval_SaveThread();
   ~Released() { PyEval_RestoreThread(state); }
 };
 
-// f(out, stream) into a tensor of `sizes` beside x.  None where the memory for it is not there: Python's way says so.
+// f(out, scratch, stream) into a tensor of `sizes` beside x, with `need` bytes of scratch.  None where there is no memory for them: Python's way says so, or does without.
 template <class F>
-PyObject* call(at::IntArrayRef sizes, const at::Tensor& x, F&& f) {
+PyObject* call(at::IntArrayRef sizes, const at::Tensor& x, F&& f, size_t need = 0) {
   at::Tensor out;
-  void* stream;
-  try {
-    out = at::empty(sizes, x.options().requires_grad(false));
-    stream = stream_of(x);
-  } catch (const std::exception&) {
-    return none();
-  }
-  int rc;
+  int rc = 0;
+  bool allocated = false;
+  std::string what;
   try {
     const Released r;
-    rc = f(out.data_ptr(), stream);
+    at::Tensor ws;   // (given back before the interpreter is waited for)
+    out = at::empty(sizes, x.options().requires_grad(false));
+    if (need) ws = at::empty({(int64_t)need}, x.options().requires_grad(false).dtype(at::kByte));
+    void* stream = stream_of(x);
+    allocated = true;
+    rc = f(out.data_ptr(), need ? ws.data_ptr() : nullptr, stream);
   } catch (const std::exception& e) {
-    PyErr_SetString(g_error_type, e.what());
-    return nullptr;
+    if (!allocated) return none();
+    what = e.what();
+    rc = -1;
   }
   if (rc != 0) {
-    PyErr_SetString(g_error_type, g_error());
+    PyErr_SetString(g_error_type, what.empty() ? g_error() : what.c_str());
     return nullptr;
   }
   return THPVariable_Wrap(std::move(out));
@@ -96,7 +102,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!x || x->dim() != 2 || x->size(1) != K || x->size(0) < 1 || x->size(0) > 8 || x->get_device() != dev || !x->is_contiguous() || modes()) return none();
   const int T = (int)x->size(0);
   const void* xp = x->const_data_ptr();
-  return call({T, N}, *x, [&](void* y, void* st) { return g_linear((void*)h, nullptr, T, xp, y, st); });
+  return call({T, N}, *x, [&](void* y, void*, void* st) { return g_linear((void*)h, nullptr, T, xp, y, st); });
 }
 
 // moe(handle, H, device index, x, ids, weights)
@@ -112,7 +118,7 @@ PyObject* moe(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const void* xp = x->const_data_ptr();
   const int64_t* ip = ids->const_data_ptr<int64_t>();
   const float* wp = w->const_data_ptr<float>();
-  return call({T, H}, *x, [&](void* y, void* st) { return g_moe((void*)h, nullptr, (int)T, (int)k, ip, wp, xp, y, 0, st); });
+  return call({T, H}, *x, [&](void* y, void*, void* st) { return g_moe((void*)h, nullptr, (int)T, (int)k, ip, wp, xp, y, 0, st); });
 }
 
 // mla_prefill(q_nope, q_pe, k_nope, k_pe, v_t, kv_len, sm_scale)
@@ -132,18 +138,10 @@ PyObject* mla_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   const float scale = (float)PyFloat_AS_DOUBLE(a[6]);
   const size_t need = g_prefill_bytes((int)T, (int)H, (int)kv);
-  at::Tensor ws;
-  if (need) {
-    try {
-      ws = at::empty({(int64_t)need}, qn.options().requires_grad(false).dtype(at::kByte));
-    } catch (const std::exception&) {
-      return none();
-    }
-  }
-  return call({T, H, 128}, qn, [&](void* y, void* st) {
+  return call({T, H, 128}, qn, [&](void* y, void* ws, void* st) {
     return g_prefill((int)T, (int)H, (int)kv, (int)pad, scale, qn.const_data_ptr(), qn.stride(0), qn.stride(1), qp.const_data_ptr(), qp.stride(0), qp.stride(1),
-                     kn.const_data_ptr(), kp.const_data_ptr(), kp.stride(0), v.const_data_ptr(), y, need ? ws.data_ptr() : nullptr, need, st);
-  });
+                     kn.const_data_ptr(), kp.const_data_ptr(), kp.stride(0), v.const_data_ptr(), y, ws, need, st);
+  }, need);
 }
 
 // mla_decode(config, most query tokens, q_nope, q_pe, ckv, k_pe, qo_indptr, kv_indptr, kv_indices | None, kv_len, bsz | None, workspace)
@@ -172,7 +170,7 @@ PyObject* mla_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (T < 1 || T > most || T > INT32_MAX || batch > INT32_MAX || !qn->is_contiguous() || !qp->is_contiguous() || ckv->stride(-1) != 1 || kpe->stride(-1) != 1 || ckv->stride(0) != cs * page ||
       kpe->stride(0) != ps * page)
     return none();
-  return call({T, H, dc}, *qn, [&](void* y, void* st) {
+  return call({T, H, dc}, *qn, [&](void* y, void*, void* st) {
     return g_decode(&c, qn->const_data_ptr(), qp->const_data_ptr(), (void*)ckv->const_data_ptr(), (void*)kpe->const_data_ptr(), cs, ps, ix[0]->const_data_ptr<int32_t>(),
                     ix[1]->const_data_ptr<int32_t>(), ix[2] ? ix[2]->const_data_ptr<int32_t>() : nullptr, ix[3]->const_data_ptr<int32_t>(),
                     ix[4] ? ix[4]->const_data_ptr<int32_t>() : nullptr, (int)batch, (int)T, nullptr, nullptr, y, nullptr, (void*)ws->const_data_ptr(), (size_t)ws->numel(), st);

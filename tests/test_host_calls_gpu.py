@@ -1,6 +1,8 @@
 """csrc/ktx_host.cpp makes the shortest calls without an interpreter step per argument: the same kernels on the same arguments as _native.py's own way, which keeps every
 call that the module does not take."""
 import copy
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -84,7 +86,7 @@ def test_linears(both, fmt):
     assert both(lambda: h.forward(torch.nn.Parameter(x[:2]))) == 1
     with torch.inference_mode():
         assert both(lambda: h.forward(x[:2])) == 1
-    wide = torch.cat((x, x), dim=1)
+    wide, two = torch.cat((x, x), dim=1), x[:2]
     for call in (lambda: h.forward(x[:9]), lambda: h.forward(x[:4].view(2, 2, -1)), lambda: h.forward(wide[:3, :512]), lambda: h.forward(x[:1].expand(4, -1)),
                  lambda: h.forward(x[:2], out=torch.empty((2, 272), dtype=torch.bfloat16, device="cuda")), lambda: h.forward(x[:2], add1=torch.ones((2, 272), dtype=torch.bfloat16, device="cuda")),
                  lambda: h.forward(x[:4], bsz_tensor=torch.tensor([4], dtype=torch.int32, device="cuda"))):
@@ -92,6 +94,7 @@ def test_linears(both, fmt):
     for bad in (x[:2].float(), x[:2, :256].contiguous(), x[:2].cpu()):
         with pytest.raises(n.KtxError):
             h.forward(bad)
+    assert both(lambda: torch.vmap(lambda v: h.forward(two), out_dims=None)(torch.zeros(3))) == 0   # (a tensor of none of its levels, but what is made inside may be wrapped)
     want = h.forward(x[:3])
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
@@ -179,3 +182,47 @@ def test_latent_attention(both, pages_of_one):
     for bad in ((q[..., :64], q[..., 128:], kn, kp[:, 512:], v), (q[..., :128], q[..., 128:], kn.transpose(0, 1), kp[:, 512:], v), (q[..., :128].float(), q[..., 128:], kn, kp[:, 512:], v)):
         with pytest.raises((n.KtxError, RuntimeError)):
             n.mla_prefill(*bad, kv, 0.07)
+
+
+@gpu
+def test_other_threads_run_while_a_call_waits_for_memory():
+    """A call's memory comes without the interpreter's lock: another thread holds the allocator (it gives cached memory back, which waits for the device) while a third one counts."""
+    if n._host is None:
+        pytest.skip("needs the built module")
+    h, x = _linear("BF16")
+    a = torch.randn((4096, 4096), device="cuda").to(torch.bfloat16)
+    b = torch.empty_like(a)
+    for _ in range(3):
+        torch.mm(a, a, out=b)
+        h.forward(x[:2])
+    torch.cuda.synchronize()
+    at = {}
+
+    def give_back():
+        at["held"] = time.perf_counter()
+        torch.cuda.empty_cache()
+        at["given"] = time.perf_counter()
+
+    def call():
+        at["called"] = time.perf_counter()
+        h.forward(x[:2])
+        at["returned"] = time.perf_counter()
+    cached = torch.empty(512 << 20, dtype=torch.uint8, device="cuda")
+    del cached
+    for _ in range(3000):
+        torch.mm(a, a, out=b)
+    threads = [threading.Thread(target=give_back), threading.Thread(target=call)]
+    threads[0].start()
+    time.sleep(0.03)
+    longest, last = 0.0, time.perf_counter()   # (a thread's start() waits for it)
+    threads[1].start()
+    while threads[1].is_alive():
+        time.sleep(0.001)
+        longest, last = max(longest, time.perf_counter() - last), time.perf_counter()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    waited = at["returned"] - at["called"]
+    if at["called"] >= at["given"] or waited < 0.1:
+        pytest.skip(f"the device was done before the call (the allocator was held for {at['given'] - at['held']:.3f} s, the call took {waited:.3f})")
+    assert longest < 0.5 * waited, (longest, waited)
