@@ -1022,10 +1022,19 @@ static bool mla_wide_steps(const ktx_mla_config* cfg, int total_q_tokens, int na
   return (tiles + narrow - 1) / narrow >= 8;
 }
 
+// The jobs form of mla_decode_wide_kernel (see mla_decode_impl): its jobs, and the splits that a token has at most (0: not in this form).
+static int mla_jobs(int hblocks, int total_q_tokens) { return std::max(2 * total_q_tokens, 256 / hblocks); }
+static int mla_jobs_cap(const ktx_mla_config* cfg, int total_q_tokens, int batch, size_t workspace_bytes) {
+  const size_t counts = (size_t)total_q_tokens * 4, rec = (size_t)total_q_tokens * cfg->num_heads * (MLA_DC + 2) * sizeof(float);   // a count, and one split, of every token
+  if (cfg->num_heads % 64 != 0 || total_q_tokens < 2 || total_q_tokens > 64 || batch > 64 || workspace_bytes <= counts || ktx_debug_get(7) > 0) return 0;
+  return (int)std::min<size_t>(std::min(std::min(256, mla_jobs(cfg->num_heads / 64, total_q_tokens)), std::max(1, cfg->max_splits)), (workspace_bytes - counts) / rec);
+}
+
 // Workgroup shape and KV split count of a decode call — one place, because the one-launch decode step (ktx_attn.hip) must
 // split the context exactly as the stand-alone kernel does to reproduce its partials bit for bit.
+// jobs_cap: mla_jobs_cap's for this call, 0 where it cannot take the jobs form.
 static void mla_pick_shape(const ktx_mla_config* cfg, int total_q_tokens, size_t workspace_bytes, int* shape_out, int* nsplit_out,
-                           bool* wide_out, bool one_launch = false) {
+                           bool* wide_out, int jobs_cap, bool one_launch = false) {
   const int Hq = cfg->num_heads;
   // workgroup shape (head blocks x dim slices): decode-sized calls of many-headed models take 2x4 (32 heads share one staged
   // KV tile, 128 output dims per wave), prompts of those models 4x2, everything else 1x4
@@ -1039,16 +1048,14 @@ static void mla_pick_shape(const ktx_mla_config* cfg, int total_q_tokens, size_t
   // a decode BATCH (>= 8 query tokens, each with its own context): every head block of a token re-reads that token's latent rows, so
   // 64 heads per workgroup halve the KV traffic (V3 dims, 8 x 4096 tokens: 150 -> 75 MB per layer; batch-of-8 step 14.47 -> 13.91 ms,
   // profiles/r06_zz_bs8_mla_shape.txt)
-  // Fewer (5 and more: what the one-launch step and its companions take stays as it is) where the 2x4 shape's workgroups would take a second round of the CUs. Us, 2x4 | these, 128 heads: 5 of 800
-  // (260 workgroups) 20.8 | 20.8, 6 (312) 23.4 | 21.4; 5 of 2000 (320) 32 | 26, unequal 27 | 26, of 3000 39 | 29, unequal 30 | 30, of 6000 58 | 33, unequal 42 | 30; 7 of 1200 (364) 27 | 23, of 7500 71 | 42; one
-  // call of 45 lost much, 6 unequal ones of 3000 26.5 | 29.9.  64 heads take one round to 7 requests: 5 of 2000 18 | 22, of 7500 30 | 31.
-  auto second_round = [&]() {
-    if (cfg->kv_len_hint <= 0) return false;   // (contexts of unknown length: as before)
-    const int tiles = (cfg->kv_len_hint + MLA_TILE - 1) / MLA_TILE, pairs = Hq / 32 * total_q_tokens, most = std::min(std::max(16, 256 / pairs), std::max(1, cfg->max_splits));
-    const int depth = (tiles + most - 1) / most;
-    return pairs * ((tiles + depth - 1) / depth) >= 300;
-  };
-  const bool batched = decode_sized && Hq % 64 == 0 && !one_launch && (total_q_tokens >= 8 || (total_q_tokens >= 5 && second_round()));
+  // Fewer (5 and more: what the one-launch step and its companions take stays as it is) of long contexts go to mla_decode_wide_kernel's shares of the batch: the 2x4 shape's workgroups take more
+  // than one round of the CUs there, in equal splits that wait for the longest request.  The line is the one of mla_wide_steps, splits (16 of them) of 8 tiles at 128 heads, and lower for more: us,
+  // 2x4 | shares, 5 requests of 3600 42 | 29, unequal (a quarter to all, four batches) 26 .. 30 | 25 .. 29, one of 3600 and four of 450 27.4 | 27.4; 7 of 4500 50 | 34, unequal 39 | 30, one and six 31 | 28; 5 of
+  // 8000 72 | 36, 56 | 34, 41 | 28; 192 heads, 5 of 3000 40 | 30; 256, 5 of 2600 51 | 32.  Slower from there on: two long requests and three short ones, 1.11 at 3600, 1.05 at 4100, 0.99 at 4500.  Below the
+  // line 2x4 stays, also where the 64-head shapes are faster for equal requests (5 of 2000 32 | 26): 6 unequal ones of 3000 take 26.7 | 28.6 (<4, 2>: 29.9), one of 2000 and four of 250 21.4 | 24.4.
+  // With a hint far above all contexts the shares are slower, as past 8 requests: hint 6400, 5 of 800 25.2 | 26.8, one of 800 and four of 100 18.3 | 21.7.  (profiles/mla_decode_few_requests.txt)
+  const bool few = !one_launch && !long_ctx && total_q_tokens >= 5 && total_q_tokens < 8 && Hq % 64 == 0 && jobs_cap >= 32 && (long)cfg->kv_len_hint * (Hq / 64) > 7168;
+  const bool batched = decode_sized && Hq % 64 == 0 && !one_launch && (total_q_tokens >= 8 || few);
   int shape = (Hq % 32 == 0 && Hq >= 64 && decode_sized && !long_ctx && !batched) ? 2 : (Hq % 64 == 0) ? 4 : 1;
   {   // tuning knobs (scripts/mla_sweep.py): 6 = force the workgroup shape, 7 = force the split count
     const int fs = ktx_debug_get(6);
@@ -1075,7 +1082,7 @@ static void mla_pick_shape(const ktx_mla_config* cfg, int total_q_tokens, size_t
     return ktx_debug_get(7) <= 0 ? (tiles + depth - 1) / depth : n;
   };
   const int narrow = splits_of(MLA_TILE);
-  const bool wide = shape == 4 && mla_wide_steps(cfg, total_q_tokens, narrow);
+  const bool wide = shape == 4 && (few || mla_wide_steps(cfg, total_q_tokens, narrow));
   nsplit = wide ? splits_of(2 * MLA_TILE) : narrow;   // (mla_decode_wide_kernel's steps)
   // <= 256 splits: the merge kernel keeps splits/16 partial rows per thread in registers (NS = 16 is its largest, spill-free
   // instantiation); longer contexts simply put more 32-token tiles into each split
@@ -1095,7 +1102,7 @@ extern "C" int ktx_mla_decode_nsplit(const ktx_mla_config* cfg, int total_q_toke
   // before the launch lost 7 us to section 4.1.6).
   const int bound_k = ktx_debug_get(1);   // dev knob 1: the bound in K tokens (scripts/attn_fused_bench.py, ATTN_BOUND_K)
   if (cfg->kv_len_hint >= (bound_k > 0 ? bound_k * 1024 : 40960)) return 0;
-  mla_pick_shape(cfg, total_q_tokens, workspace_bytes, &shape, &nsplit, &wide, true);
+  mla_pick_shape(cfg, total_q_tokens, workspace_bytes, &shape, &nsplit, &wide, 0, true);
   return shape == 2 ? nsplit : 0;   // the one-launch step is built on the 2x4 workgroup shape only
 }
 
@@ -1117,7 +1124,8 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
   const int Hq = cfg->num_heads;
   int shape = 0, nsplit = 0;
   bool wide = false;
-  mla_pick_shape(cfg, total_q_tokens, workspace_bytes, &shape, &nsplit, &wide);
+  const int jobs_cap = partials_nsplit ? 0 : mla_jobs_cap(cfg, total_q_tokens, batch, workspace_bytes);
+  mla_pick_shape(cfg, total_q_tokens, workspace_bytes, &shape, &nsplit, &wide, jobs_cap);
   const int hbw = shape, nwv = shape == 1 ? 4 : 8;
   const int hblocks = Hq / (16 * hbw);
   KTX_REQUIRE(nsplit >= 1, "ktx_mla_decode: workspace too small");
@@ -1143,15 +1151,10 @@ static int mla_decode_impl(const ktx_mla_config* cfg, const void* d_q_nope, cons
   // the form before, 40 so).
   p.jobs = 0;
   p.njobs = nullptr;
-  if (wide && !partials_nsplit && nsplit > 1 && total_q_tokens > 1 && total_q_tokens <= 64 && batch <= 64 && ktx_debug_get(7) <= 0) {
-    const size_t rec = (size_t)total_q_tokens * Hq * (MLA_DC + 2) * sizeof(float);   // one split of every token
-    const int jobs = std::max(2 * total_q_tokens, 256 / hblocks);
-    const int cap = (int)std::min<size_t>(std::min(std::min(256, jobs), std::max(1, cfg->max_splits)), (workspace_bytes - (size_t)total_q_tokens * 4) / rec);
-    if (workspace_bytes > (size_t)total_q_tokens * 4 && cap > 1) {
-      p.jobs = jobs; p.nsplit = cap;
-      p.part_ml = p.part_o + (size_t)total_q_tokens * Hq * cap * MLA_DC;
-      p.njobs = reinterpret_cast<int*>(p.part_ml + (size_t)total_q_tokens * Hq * cap * 2);
-    }
+  if (wide && nsplit > 1 && jobs_cap > 1) {
+    p.jobs = mla_jobs(hblocks, total_q_tokens); p.nsplit = jobs_cap;
+    p.part_ml = p.part_o + (size_t)total_q_tokens * Hq * jobs_cap * MLA_DC;
+    p.njobs = reinterpret_cast<int*>(p.part_ml + (size_t)total_q_tokens * Hq * jobs_cap * 2);
   }
   p.out1 = direct ? (bf16_t*)d_out : nullptr;
   p.lse1 = direct ? d_lse : nullptr;

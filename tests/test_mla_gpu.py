@@ -222,11 +222,12 @@ def test_which_decode_kernel_a_batch_takes(Hq, lens, wide):
     assert float((out.double() - want).norm() / want.norm()) < 2.4e-3      # (sqrt(2) of 1.66e-3: outputs and probabilities in bf16)
 
 
-@pytest.mark.parametrize("Hq,lens,kernel", [(128, [3000] * 4, "mla_decode_kernel<2,4>"), (128, [400] * 5, "mla_decode_kernel<2,4>"), (128, [2000, 500, 777, 1999, 1], "mla_decode_kernel<4,2>"),
-                                            (128, [1000] * 6, "mla_decode_kernel<4,2>"), (128, [4500] * 5, "mla_decode_wide_kernel"), (128, [6000, 33, 1500, 6000, 64, 4000, 31], "mla_decode_wide_kernel"),
+@pytest.mark.parametrize("Hq,lens,kernel", [(128, [3000] * 4, "mla_decode_kernel<2,4>"), (128, [400] * 5, "mla_decode_kernel<2,4>"), (128, [2000, 500, 777, 1999, 1], "mla_decode_kernel<2,4>"),
+                                            (128, [1000] * 6, "mla_decode_kernel<2,4>"), (128, [3000, 900, 2100, 2999, 1500, 800], "mla_decode_kernel<2,4>"), (128, [3584] * 7, "mla_decode_kernel<2,4>"),
+                                            (128, [3585] * 7, "mla_decode_wide_kernel"), (128, [4500] * 5, "mla_decode_wide_kernel"), (192, [3000] * 5, "mla_decode_wide_kernel"), (128, [6000, 33, 1500, 6000, 64, 4000, 31], "mla_decode_wide_kernel"),
                                             (64, [7000] * 7, "mla_decode_kernel<2,4>"), (64, [4200] * 8, "mla_decode_wide_kernel"), (64, [3000] * 8, "mla_decode_kernel<4,2>")])
 def test_which_decode_kernel_a_few_requests_take(Hq, lens, kernel):
-    """5 to 7 requests of 128 heads leave the 2x4 shape where its workgroups would take a second round; the 64-token kernel from splits of 8 tiles on at 64 heads too."""
+    """5 to 7 requests of 128 heads and more leave the 2x4 shape from splits of 8 tiles on, for the kernel that shares out what they hold; the 64-head kernel from there on at 64 heads too."""
     from ktransformers_amd import _native as n
     run, exact = decode_batch(Hq, lens)
     n.timing_enable(2)
@@ -238,6 +239,30 @@ def test_which_decode_kernel_a_few_requests_take(Hq, lens, kernel):
     assert labels[0].startswith(kernel), labels
     want = exact()
     assert float((out.double() - want).norm() / want.norm()) < 2.4e-3      # (sqrt(2) of 1.66e-3: outputs and probabilities in bf16)
+
+
+@pytest.mark.parametrize("bytes_of_splits,max_splits,partials", [(31, 256, False), (256, 16, False), (256, 256, True)])
+def test_few_requests_without_room_for_shares(bytes_of_splits, max_splits, partials):
+    """5 requests of long contexts whose workspace, split limit or way of merging leaves no shares of the batch: the 2x4 shape, as for short ones."""
+    from ktransformers_amd import _native as n
+    lens, Hq = [4500] * 5, 128
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q_nope, q_pe, cache = (torch.randn(s, device=DEV, generator=g).to(torch.bfloat16) for s in ((5, Hq, 512), (5, Hq, 64), (71, 64, 576)))
+    w = n.MLAWrapper(5, 71 * 5, use_cuda_graph=False, device=DEV, max_q_tokens=5, max_splits=max_splits)
+    dev = [torch.tensor(a, dtype=torch.int32, device=DEV) for a in (range(6), range(0, 71 * 6, 71), list(range(71)) * 5, lens, [5])]
+    w.plan(*dev, Hq, 512, 64, 64, 192 ** -0.5, max_kv_len=4500)
+    if bytes_of_splits < 256:
+        w.workspace = w.workspace[:bytes_of_splits * 5 * Hq * 514 * 4 + 20]
+    n.timing_enable(2)
+    try:
+        out = w.run(q_nope, q_pe, cache[:, :, :512], cache[:, :, 512:], partials=partials)
+        assert n.timing_collect()[0][0].startswith("mla_decode_kernel<2,4>")
+    finally:
+        n.timing_enable(0)
+    if not partials:
+        rows = cache.view(-1, 576)[:4500].double()
+        want = torch.softmax(torch.cat((q_nope, q_pe), dim=2).double().view(-1, 576) @ rows.T.contiguous() * 192 ** -0.5, dim=1) @ rows[:, :512].contiguous()
+        assert float((out.double().view(-1, 512) - want).norm() / want.norm()) < 2.4e-3      # (sqrt(2) of 1.66e-3: outputs and probabilities in bf16)
 
 
 def test_single_split_equals_many():
