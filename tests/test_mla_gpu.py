@@ -178,6 +178,41 @@ def test_wide_decode_tiles_and_growing_scores(Hq, lens, ramp):
     assert float((out.double() - want).norm()) <= 1.01 * floor
 
 
+@pytest.mark.parametrize("page", [64, 96, 256])   # 96: no power of two, so that a tile's page is divided out
+def test_wide_decode_appends_in_long_contexts(page):
+    """The appended row's tile comes by its own requests (request_any) into the run of tiles that a workgroup already has in flight: contexts of dozens of tiles a workgroup, lengths that are
+    whole tiles, so that only the new row makes the difference, and others.  Results, and the cache afterwards."""
+    from ktransformers_amd import _native as n
+    lens = [4000, 4032, 3072, 2560, 3999, 4001, 96, 2049, 33, 3584, 1, 4000]
+    g = torch.Generator(device=DEV).manual_seed(page)
+    B, Hq, pages = len(lens), 128, [(m + page - 1) // page for m in lens]
+    first = [0] + [int(v) for v in np.cumsum(pages)]
+    table = torch.randperm(first[-1], device=DEV, generator=g).to(torch.int32)
+    cache, q_nope, q_pe, new = (torch.randn(s, device=DEV, generator=g).to(torch.bfloat16) for s in ((first[-1], page, 576), (B, Hq, 512), (B, Hq, 64), (B, 576)))
+    new *= 3   # (a stale row's score and values are others by much)
+    after = cache.clone()
+    for b, m in enumerate(lens):
+        after[int(table[first[b] + (m - 1) // page]), (m - 1) % page] = new[b]
+    w = n.MLAWrapper(B, first[-1], use_cuda_graph=False, device=DEV, max_q_tokens=B)
+    dev = [torch.tensor(a, dtype=torch.int32, device=DEV) for a in (range(B + 1), first, lens, [B])]
+    w.plan(dev[0], dev[1], table, dev[2], dev[3], Hq, 512, 64, page, 192 ** -0.5, max_kv_len=max(lens))
+    n.timing_enable(2)
+    try:
+        out = w.run(q_nope, q_pe, cache[:, :, :512], cache[:, :, 512:], new_ckv=new[:, :512].contiguous(), new_kpe=new[:, 512:].contiguous())
+        assert "mla_decode_wide_kernel" in n.timing_collect()[0][0]
+    finally:
+        n.timing_enable(0)
+    assert torch.equal(cache, after)
+    want = []
+    for b, m in enumerate(lens):
+        rows = after[table[first[b]:first[b + 1]].long()].view(-1, 576)[:m].double()
+        want.append(torch.softmax(torch.cat((q_nope[b], q_pe[b]), dim=1).double() @ rows.T * 192 ** -0.5, dim=1) @ rows[:, :512])
+    want = torch.stack(want)
+    floor = (want.to(torch.bfloat16).double() - want).norm(dim=(1, 2))
+    err = (out.double() - want).norm(dim=(1, 2))
+    assert bool((err <= 1.02 * floor).all()), (err / floor).tolist()   # (the outputs' rounding, each request by itself; of one token the result is the row)
+
+
 @pytest.mark.parametrize("lens", [[2000] * 20, [40] * 24])   # several splits a request; one, whose result the kernel stores itself
 def test_wide_decode_of_infinite_scores(lens):
     """Scores of -inf weigh nothing, wherever a split begins: every even tile of 32 tokens is -inf to every third head."""
