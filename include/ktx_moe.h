@@ -201,7 +201,7 @@ int ktx_debug_force_generic(int on);
  * prompt kernels (1: 64 rows at most, 2: 128), idx 23 = wavefronts of the AMXINT4 / AMXINT8 streaming kernels (1: 4, 2: 8), idx 24 = the FP8 streaming
  * kernel (1 never, 2 always), idx 25 = experts per router workgroup in ktx_linear_forward_fused_gate's combined kernel: 1 -> 8, 2 -> 2, 0 -> 4 where the
  * grid has room (same logits and selection bit for bit), idx 31 = 16-column fragments a wavefront of the 256-row bf16 GEMM (3 or 4), idx 32 = 1 keeps W4 and
- * FP8 linears off the 64 x 256 tiles. */
+ * FP8 linears off the 64 x 256 tiles, idx 33 = pieces of a query's keys in ktx_mla_prefill_ws (1 to 16; 0 auto). */
 int ktx_debug_set(int idx, int val);
 int ktx_debug_get(int idx);
 /* Per-launch timing of every kernel of the library (bench.py's per-kernel table; ktx_prof.hip).  mode 1: each launch is

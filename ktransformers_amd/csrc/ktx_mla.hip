@@ -508,8 +508,9 @@ __device__ __forceinline__ float pf_sum_rows(float x) {
 // Before, two wavefronts a SIMD shared 16 heads in steps of 64 tokens (half of the scores each, exchanged through the LDS, then half of the dims), and two barriers a step kept scores, softmax and O
 // apart in both: 3.1 us for 64 tokens, all of O rescaled in nearly every step, and the last step whole where 32 tokens were left.  Decode and merge, before -> here, us: 128 heads, 8
 // requests of 2048 .. 8192 tokens 44.5 -> 42.0, 32 of 1000 .. 4000 69.9 -> 60.9, 20 of 2000 .. 8000 76 -> 66, 4 of 8192 .. 32768 66 -> 57, 32 of 250 .. 1000 34.0 -> 32.9; 64 heads, 24 of 1250
-// .. 5000 47.4 -> 41.1, 3 of 16384 31.5 -> 29.4, 32 of 500 .. 2000 34.7 -> 32.4; few requests and short contexts (128 heads, 5 of 8000) the same to 1 %.  A call of 8 requests: 1.6 us for the job,
-// 3.6 for pages, Q and the first rows, 0.7 the first scores, 17 the tiles, 3 the partial results' stores.
+// .. 5000 47.4 -> 41.1, 3 of 16384 31.5 -> 29.4, 32 of 500 .. 2000 34.7 -> 32.4.  A call of 8 requests: 1.6 us for the job,
+// 3.6 for pages, Q and the first rows, 0.7 the first scores, 17 the tiles, 3 the partial results' stores; over the whole launch the matrix pipe is busy 24 %, the vector ALU 20, the LDS 17, without a
+// bank conflict (profiles/expert_prompt_counters.txt).
 // The rows are
 // packed 1 KiB apart with their 16-byte pieces permuted by mla_swz, which keeps both the fragment reads of 16 rows and the transposed reads of
 // 8 rows off each other's banks.
@@ -1588,7 +1589,9 @@ __global__ __launch_bounds__(256) void mla_prefill_merge_kernel(MlaPrefillParams
 
 // How many workgroups share a query's keys.  A workgroup of 128 queries and a head alone on its CU takes 1.27 us a key tile, two beside each other 2.0, so that few (query block, head)
 // pairs with long contexts leave most of the chip idle: 64 queries of 16 heads behind 6000 tokens are 16 workgroups of 95 tiles, 128 us.  The pieces cost their sums' way to
-// memory and back and the merge's launch: this estimate, fitted to 66 calls at 1 to 16 pieces, picks one within 4 % of the best everywhere, none slower than whole.  Us, whole | here:
+// memory and back and the merge's launch: this estimate, fitted to 66 calls at 1 to 16 pieces (profiles/mla_prefill_pieces.txt), picks
+// a count within 9 % of the best one where it shares, within 6 in all but one, and shares only where it sees a tenth to gain: up to 16 % is left there (16 heads, 1500 queries behind 1000 59.7,
+// three pieces 51.5).  Us, whole | here:
 // 16 heads, 64 queries behind 1000 29 | 15, 6000 128 | 23, 300 behind 1000 36 | 24, 3000 76 | 32, 800 behind 3000 88 | 56; 64 heads, 64 behind 3000 70 | 31, 150 behind 1000 34 | 28; 128
 // heads, 64 behind 3000 72 | 47.  Past 192 pairs, whose workgroups share CUs as it is, 5 to 10 % at most (128 heads, 150 behind 6000 170 | 158) and as often nothing.
 // Dev knob 33 (tests): that many.

@@ -2870,10 +2870,12 @@ static int forward_gguf(ktx_moe_s* h, const int32_t* d_bsz, int qlen, int k, con
     mt = rows <= 6.0 ? 1 : rows <= 16.0 ? 2 : rows < 144.0 || (strips && jobs < 1024.0) ? 4 : 8;
     if (g_dbg[22]) mt = g_dbg[22] == 2 ? 8 : std::min(mt, 4);
     // Strip groups or shares of the experts to the XCDs (moe_pick_strips, moe_pick_job)?  Shares hold as many jobs, not as much work, and end up to a quarter apart; with strip
-    // groups every XCD reads all rows, which counts where an expert has more of them than its matrices have outputs.  Us, shares | strip groups: 8 experts of 4096 x 14336, top-2, 300
+    // groups every XCD reads all rows, which counts where an expert has many of them beside its matrices' outputs (the line: half
+    // as many).  Us, shares | strip groups: 8 experts of 4096 x 14336, top-2, 300
     // tokens 446 | 423, 500 630 | 616, 1696 1669 | 1645; 64 of 2048 x 1536, top-6, 400 162 | 155, 2048 451 | 439; 16 of 5632 x 1024, top-4, 1000 302 | 287; 128 of 1024 x 512, top-8, 900
     // 101 | 99.4; 8 of 2560 x 1536, top-6, 665 (500 rows) 181 | 181; 8 of 1024 x 512, top-8, 1500 (1500 rows) 103 | 107.  Strip groups with the experts in their own order, which leaves
-    // whole tiles for the end: 500 tokens 630, 1696 1716 (shares 1733 there).
+    // whole tiles for the end: 500 tokens 630, 1696 1716 (shares 1733 there).  235 calls about this line and the one of 1024 jobs above: profiles/q4k_prompts_strip_groups.txt; 5 % less on the whole, the
+    // worst 3.6 % more (16 of 5632 x 1024, 200 rows 212 | 220).
     strips = strips && mt > 1;
   }
   const int max_tiles = std::min(npairs, E) + npairs / (16 * mt);
