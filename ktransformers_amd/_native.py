@@ -1367,7 +1367,7 @@ class MLAWrapper:
              page_size, sm_scale, q_data_type=torch.bfloat16, kv_data_type=torch.bfloat16, max_kv_len: int = 0,
              identity_pages: bool = False):
         """max_kv_len: the longest context that the plan's runs may meet (the cache's capacity will do, but the nearer the better: a batch all of whose contexts are far below it takes
-        up to a fifth longer).  It picks kernel and splits: without it batches of up to 16 query tokens stay on the 32-token kernel.
+        2 to 6 us longer).  It picks kernel and splits: without it batches of up to 16 query tokens stay on the 32-token kernel.
         identity_pages: the page table is the identity (request r owns pages kv_indptr[r] .. kv_indptr[r+1]-1 in order, as
         in the single-request StaticCache): the kernel then skips the page-table load (include/ktx_mla.h)."""
         if q_data_type != torch.bfloat16 or kv_data_type != torch.bfloat16:
